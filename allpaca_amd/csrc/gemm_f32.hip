@@ -1,0 +1,244 @@
+// Matrix product  C[M,N] = A[M,K] . W[N,K]^T  of float32 operands on the matrix cores (v_mfma_f32_16x16x4_f32: float32
+// products and sums, no reduced mode).
+//
+// Every output is  s0 + s1 + .. + s7  added in this order; slice i is the chain over k in [i L, (i+1) L), L the
+// multiple of 32 that eight of cover K, four k an instruction, sixteen k in the order 0 4 8 12, 1 5 9 13, .. .  That
+// depends on K alone, not on M, N, the tile or the grid: a row of a batch equals that row computed alone bit for bit.
+//
+// The eight slices are the eight waves of a block.  Each computes the block's whole tile over its own k and meets the
+// others in LDS at the end, so a product with few tiles (decoded rows; 2,048 outputs and a few hundred rows) still has
+// eight waves a compute unit at work, no wave waits for another inside the loop, and there are no partial sums in
+// memory.  A wave brings 32 k of its rows into registers as eight lanes a row (128 consecutive bytes; the instruction's
+// own operand order would have every lane in another row), D of such stages ahead, and turns them into operands in a
+// piece of LDS of its own.
+//
+// What bounds it: with few rows the bytes of W, else the matrix cores' float32 rate (157 TFLOP/s, of which a library
+// product of 8,192^3 reaches 151).  Measured, microseconds (in brackets the kernel of one fma chain an output on the
+// vector units, which takes the other types): 4 rows x 2,048 outputs x K 2,048 9.4; x 128,256 outputs 149 (7.1 TB/s);
+// 330 rows x 16,384 outputs 206 (about 1,600; 107 TFLOP/s); 2,048 rows x 2,048 outputs x K 8,192 531 (129 TFLOP/s).  The
+// 65 products of a step of a 1B model in float32: 4 rows 1.12 ms (40.3), 340 rows 6.6 ms (38.9).
+#include "mfma.h"
+#include <math.h>
+
+namespace {
+
+constexpr int SLICES = 8, STAGE = 32;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <bool ONCE>
+__device__ __forceinline__ f32x4 load_f32x4(BufferRsrc rsrc, int lane_bytes, int scalar_bytes) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(f32x4, (u32x4)__builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_bytes, scalar_bytes, ONCE ? 2 : 0));
+}
+template <int N>
+struct Count { static constexpr int value = N; };
+template <int N, typename F>
+__device__ __forceinline__ void each_count(F f) {        // f(1), .. f(N), known when compiling
+  if constexpr (N > 1) each_count<N - 1>(f);
+  f(Count<N>{});
+}
+
+// MT x NT tiles of 16 rows x 16 outputs a block, D stages of loads ahead.
+template <int MT, int NT, int D, bool ONCE, int MIN_WAVES>
+__global__ __launch_bounds__(64 * SLICES, MIN_WAVES) void gemm_f32_kernel(
+    const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, void* __restrict__ C, int c_dtype,
+    int ldc, int M, int N, int K, int mode, int tiles_m, int tiles) {
+  constexpr int BANDS = MT + NT;
+  constexpr int STAGE_F4 = BANDS * 128, SUM_F4 = MT * NT * 64;       // float4 a wave: its stage, its sums
+  __shared__ f32x4 lds[SLICES * (STAGE_F4 > SUM_F4 ? STAGE_F4 : SUM_F4)];
+  // The block ids that one XCD gets (every eighth) are a run of tiles, row tiles of the same outputs next to each other:
+  // they share W in that XCD's L2.
+  const int per = (tiles + 7) / 8;
+  const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (t >= tiles || (int)(blockIdx.x / 8) >= per) return;
+  const int m0 = (t % tiles_m) * (16 * MT), n0 = (t / tiles_m) * (16 * NT);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+
+  const int slice = STAGE * ((K + STAGE * SLICES - 1) / (STAGE * SLICES));
+  const int k0 = wave * slice;
+  const int steps = (min(K, k0 + slice) - k0 + STAGE - 1) / STAGE;   // <= 0: no k left for this wave
+
+  // What this lane loads of a stage: rows lane/8 and lane/8 + 8 of every band, 4 k at (lane%8)*4.  Rows past the end are
+  // the last row again (their sums are not stored); for k past the end it loads the stage's first k, and 0 goes into LDS.
+  const int lr = lane / 8, lk = (lane % 8) * 4;
+  const int rows_w = min(N - n0, 16 * NT), rows_a = min(M - m0, 16 * MT);
+  const BufferRsrc from_w = make_rsrc(W + (size_t)n0 * ldw), from_a = make_rsrc(A + (size_t)m0 * lda);
+  int off[BANDS][2];
+#pragma unroll
+  for (int b = 0; b < BANDS; ++b)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      off[b][h] = 4 * (lk + (b < NT ? min(16 * b + lr + 8 * h, rows_w - 1) * ldw : min(16 * (b - NT) + lr + 8 * h, rows_a - 1) * lda));
+  f32x4 reg[D][BANDS][2];
+  auto load = [&](int slot, int s) __attribute__((always_inline)) {
+    const int at = 4 * (k0 + s * STAGE);
+    const int back = k0 + s * STAGE + lk >= K ? 4 * lk : 0;
+#pragma unroll
+    for (int b = 0; b < BANDS; ++b)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        reg[slot][b][h] = b < NT ? load_f32x4<ONCE>(from_w, off[b][h] - back, at) : load_f32x4<false>(from_a, off[b][h] - back, at);
+  };
+
+  // the wave's stage in LDS: row r of a band is 8 pieces of 16 bytes, piece c at place c ^ (r % 8) (reads of one piece
+  // over eight rows then fall on different banks)
+  f32x4* mine = lds + wave * STAGE_F4;
+  const int put_at = lr * 8 + ((lane % 8) ^ lr);
+  const int row = lane % 16, quarter = lane / 16;
+  const int get_at[2] = {row * 8 + (quarter ^ (row % 8)), row * 8 + ((quarter + 4) ^ (row % 8))};
+  auto put = [&](int slot, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < BANDS; ++b)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) mine[b * 128 + h * 64 + put_at] = reg[slot][b][h];
+    if (k0 + (s + 1) * STAGE > K && k0 + s * STAGE + lk >= K) {
+#pragma unroll
+      for (int b = 0; b < 2 * BANDS; ++b) mine[b * 64 + put_at] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    wave_lds_order();
+  };
+  f32x4 f[2][BANDS];                                    // operands of a stage's first and second 16 k
+  auto get = [&](int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < BANDS; ++b) f[half][b] = mine[b * 128 + get_at[half]];
+    wave_lds_order();
+  };
+  floatx4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[half][j][e], f[half][NT + i][e], acc[i][j], 0, 0, 0);
+  };
+  // A stage: its second operands come out of LDS under the first products; then the next stage goes in, the loads that
+  // take its registers go out, and its first operands come back under the second products.
+  auto stage = [&](int s, int next_slot, bool next, bool more) __attribute__((always_inline)) {
+    get(1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (next) {
+      put(next_slot, s + 1);
+      __builtin_amdgcn_sched_barrier(0);                // (the loads take the registers that have just been written out)
+      if (more) load(next_slot, s + 1 + D);
+      __builtin_amdgcn_sched_barrier(0);
+      get(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+  };
+  auto begin = [&](auto count) __attribute__((always_inline)) {                        // stages there are, at least (what is known when compiling)
+    constexpr int R = decltype(count)::value;
+#pragma unroll
+    for (int u = 0; u < D && u < R; ++u) load(u, u);
+    put(0, 0);
+    if (R > D) load(0, D);
+    get(0);
+  };
+  auto finish = [&](int s0, auto count) __attribute__((always_inline)) {               // the last stages, without a condition between the loads
+    constexpr int R = decltype(count)::value;
+#pragma unroll
+    for (int i = 0; i < R; ++i) stage(s0 + i, (i + 1) % D, i + 1 < R, i + 1 + D < R);
+  };
+  // Straight code for the last 2 D stages: behind a branch that may have loaded the compiler waits for more than it needs.
+  if (steps > 2 * D) {
+    begin(Count<2 * D + 1>{});
+    int s0 = 0;
+    for (; steps - s0 > 2 * D; s0 += D)
+#pragma unroll
+      for (int u = 0; u < D; ++u) stage(s0 + u, (u + 1) % D, true, true);
+    each_count<2 * D>([&](auto r) __attribute__((always_inline)) {
+      if (steps - s0 == decltype(r)::value) finish(s0, r);
+    });
+  } else {
+    each_count<2 * D>([&](auto r) __attribute__((always_inline)) {
+      if (steps == decltype(r)::value) begin(r), finish(0, r);
+    });
+  }
+
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) lds[wave * SUM_F4 + (i * NT + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  for (int p = threadIdx.x; p < SUM_F4; p += 64 * SLICES) {
+    f32x4 v = lds[p];
+#pragma unroll
+    for (int w = 1; w < SLICES; ++w) v += lds[w * SUM_F4 + p];
+    const int tile = p / 64, l = p % 64;
+    const int m = m0 + (tile / NT) * 16 + l % 16, n = n0 + (tile % NT) * 16 + (l / 16) * 4;
+    if (m >= M) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (n + e >= N) continue;
+      const size_t o = (size_t)m * ldc + n + e;
+      if (mode == 1) ((float*)C)[o] += v[e];
+      else store_f(C, c_dtype, o, v[e]);
+    }
+  }
+}
+
+template <int MT, int NT, int D, bool ONCE, int MIN_WAVES>
+int launch(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
+           hipStream_t stream) {
+  const int tiles_m = ceil_div(M, 16 * MT);
+  const long long tiles = (long long)tiles_m * ceil_div(N, 16 * NT);
+  if (tiles > (1 << 27)) return APC_ERR_BAD_ARG;
+  hipLaunchKernelGGL((gemm_f32_kernel<MT, NT, D, ONCE, MIN_WAVES>), dim3(ceil_div((int)tiles, 8) * 8), dim3(64 * SLICES), 0,
+                     stream, A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, tiles_m, (int)tiles);
+  APC_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // namespace
+
+// Whether the kernel takes these operands: 16-byte loads along k.
+bool gemm_f32_takes(const void* A, int lda, const void* W, int ldw, int K) {
+  return K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15u) == 0 && lda < (1 << 22) &&
+         ldw < (1 << 22);            // (64 rows fit a descriptor's 32-bit offsets)
+}
+
+// The tile: the least of these times (microseconds at K = 2,048; K stretches them alike) over the tiles' shapes.  A
+// block of the small tiles shares its compute unit with others, so their time grows with the blocks; the large ones have
+// a unit to themselves and go in whole rounds of 256.  Measured on 24 to 2,048 rows x 2,048 to 16,384 outputs, where the
+// choice is within a tenth of the best of the six: 2,048 outputs take 9.4 us up to 48 rows, 18 at 160 rows (48 x 32
+// tiles; 16 x 16: 25, 64 x 64: 41), 31 at 330 (48 x 64; 16 x 16: 43).
+int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
+             hipStream_t stream) {
+  struct Shape { int mt, nt; bool shares; double start, round; };
+  constexpr Shape shapes[] = {{1, 1, true, 4.5, 5.0},   {2, 1, true, 4.0, 5.8},   {2, 2, false, 1.5, 13.0},
+                              {3, 2, false, 1.5, 15.5}, {3, 4, false, 1.5, 28.7}, {4, 4, false, 1.5, 39.0}};
+  int best = 0;
+  double best_cost = 1e30;
+  for (int i = 0; i < 6; ++i) {
+    const Shape& s = shapes[i];
+    double rounds = (double)ceil_div(M, 16 * s.mt) * ceil_div(N, 16 * s.nt) / 256;
+    if (!s.shares) rounds = ceil(rounds);
+    const double cost = s.start + s.round * (rounds > 1.0 ? rounds : 1.0);
+    if (cost < best_cost) best = i, best_cost = cost;
+  }
+#define GO(...) return launch<__VA_ARGS__>(A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
+  // (one row tile: W is read once, past the caches)
+  switch (best) {
+    case 0:
+      if (M <= 16) GO(1, 1, 4, true, 4);
+      GO(1, 1, 4, false, 4);
+    case 1:
+      if (M <= 32) GO(2, 1, 2, true, 2);
+      GO(2, 1, 2, false, 2);
+    case 2: GO(2, 2, 1, false, 2);
+    case 3: GO(3, 2, 1, false, 2);
+    case 4: GO(3, 4, 1, false, 2);
+    default: GO(4, 4, 1, false, 2);
+  }
+#undef GO
+}

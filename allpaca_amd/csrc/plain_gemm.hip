@@ -1,4 +1,6 @@
-// Plain matrix product  C[M,N] = A[M,K] . W[N,K]^T  in true 32-bit arithmetic.
+// Plain matrix product  C[M,N] = A[M,K] . W[N,K]^T  in true 32-bit arithmetic: other types than float32, widths that are
+// no multiple of 4, heads with matrices of their own (float32 products otherwise: gemm_f32.hip, which adds in another
+// fixed order).
 //
 // Every output element is one chain  acc = fma(a[k], w[k], acc)  over k = 0..K-1
 // in order, whatever M, N or the tile a row falls into: a row of a batch equals
@@ -10,6 +12,11 @@
 #include "common.h"
 
 constexpr int TM = 64, TN = 64, TK = 16;
+
+// gemm_f32.hip: the same product of float32 operands on the matrix cores
+bool gemm_f32_takes(const void* A, int lda, const void* W, int ldw, int K);
+int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
+             hipStream_t stream);
 
 // mode 0: C = acc (C of c_dtype)   mode 1: C += acc (C float32)
 // blockIdx.z: one of several products of the same sizes, whose operands lie these many elements apart.
@@ -90,6 +97,10 @@ APC_EXPORT int apc_gemm_plain(const void* A, int a_dtype, int lda, const void* W
   if (mode == 1 && c_dtype != APC_F32) return APC_ERR_BAD_ARG;
   const int gy = ceil_div(M, TM);
   if (gy > 65535) return APC_ERR_BAD_ARG;
+  // float32 with rows of whole 16-byte pieces goes to the matrix cores, whatever M is (the two kernels add in different
+  // orders, and a row alone must equal the row in a batch)
+  if (a_dtype == APC_F32 && w_dtype == APC_F32 && gemm_f32_takes(A, lda, W, ldw, K))
+    return gemm_f32((const float*)A, lda, (const float*)W, ldw, C, c_dtype, ldc, M, N, K, mode, stream);
   hipLaunchKernelGGL(gemm_plain_kernel, dim3(ceil_div(N, TN), gy), dim3(256), 0, stream, A, a_dtype, lda, W, w_dtype,
                      ldw, C, c_dtype, ldc, M, N, K, mode, HeadStrides{});
   APC_LAUNCH_CHECK();

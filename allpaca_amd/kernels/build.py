@@ -23,7 +23,7 @@ from typing import Dict, List
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
 
 LIBS: Dict[str, List[str]] = {
-    "plain": ["plain_ops.hip", "plain_gemm.hip", "plain_attention.hip", "plain_mixers.hip", "plain_heads.hip", "plain_recurrent.hip", "plain_routed.hip",
+    "plain": ["plain_ops.hip", "plain_gemm.hip", "gemm_f32.hip", "plain_attention.hip", "plain_mixers.hip", "plain_heads.hip", "plain_recurrent.hip", "plain_routed.hip",
               "plain_scan.hip", "plain_latent.hip", "plain_delta.hip", "sampling.hip"],
     "tuned": ["gemm_bf16.hip", "gemm_wide_bf16.hip", "gemm_direct_bf16.hip", "skinny_gemm_bf16.hip", "attention_bf16.hip", "attention_wide_bf16.hip", "attention_masked_bf16.hip", "conv_heads_bf16.hip", "rope_bf16.hip", "rotary_pages_bf16.hip",
               "linear_attention_bf16.hip", "routed_bf16.hip", "selective_scan_bf16.hip", "latent_heads_bf16.hip", "attention_latent_bf16.hip",
