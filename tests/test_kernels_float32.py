@@ -72,3 +72,54 @@ def test_product_lets_infinities_and_nan_through():
     o.gemm_plain(a, w, out)
     want = a.double() @ w.double().T
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+
+
+def paged(lengths, Hk, d, P, seed):
+    """A cache with the keys and values of several sequences on shuffled pages, NaN in every slot without a key."""
+    g = torch.Generator().manual_seed(seed)
+    blocks = [-(-n // P) for n in lengths]
+    order = torch.randperm(sum(blocks) + 2, generator=g)
+    cache = torch.full((len(order), 2, Hk, P, d), math.nan, device=DEV)
+    values = cache[:, 1].view(-1, Hk, d, P)
+    table = torch.zeros(len(lengths), max(blocks), dtype=torch.int32)
+    kv, at = [], 0
+    for i, n in enumerate(lengths):
+        k, v = gen(n, Hk, d, seed=seed + 2 * i), gen(n, Hk, d, seed=seed + 2 * i + 1)
+        for b in range(blocks[i]):
+            page, m = int(order[at + b]), min(P, n - b * P)
+            table[i, b] = page
+            cache[page, 0, :, :m] = k[b * P:b * P + m].transpose(0, 1)
+            values[page, :, :, :m] = v[b * P:b * P + m].permute(1, 2, 0)
+        at += blocks[i]
+        kv.append((k.double(), v.double()))
+    return cache, table.to(DEV), kv
+
+
+# groups of 4, 2, 1 heads on a kv head (and 3, taken one by one); heads up to 64 and up to 128; pages under, at and over
+# a chunk of 64 keys; lengths around a chunk and around eight of them
+@pytest.mark.parametrize("H,Hk,d,P", [(8, 2, 64, 16), (6, 2, 32, 4), (4, 2, 128, 16), (3, 1, 100, 8), (4, 1, 80, 128)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_attention_against_64_bits_and_rows_alone(H, Hk, d, P, window):
+    o = ops()
+    lengths = [577, 1, 63, 64, 65]
+    cache, table, kv = paged(lengths, Hk, d, P, seed=11)
+    pos = torch.tensor([p for n in lengths for p in range(n)], dtype=torch.int32, device=DEV)
+    seg = torch.tensor([i for i, n in enumerate(lengths) for _ in range(n)], dtype=torch.int32, device=DEV)
+    q = gen(len(pos), 8 + H * d, seed=5)
+    out = torch.empty(len(pos), H * d, device=DEV)                    # (enough rows for the form of a row a wave)
+    o.paged_attention_plain(q, 8, out, H, Hk, d, cache, P, table, pos, seg, window=window)
+    for r in [0, 62, 63, 64, 69, 70, 511, 512, 576, 577, 578, 640, 641, 704, 705, len(pos) - 1]:
+        alone = torch.empty(1, H * d, device=DEV)                     # (a block a row)
+        o.paged_attention_plain(q[r:r + 1], 8, alone, H, Hk, d, cache, P, table, pos[r:r + 1], seg[r:r + 1], window=window)
+        assert torch.equal(alone[0], out[r])
+        p, (k, v) = int(pos[r]), kv[int(seg[r])]
+        first = max(0, p - window + 1) if window else 0
+        k, v = (x[first:p + 1].repeat_interleave(H // Hk, 1) for x in (k, v))
+        qr = q[r, 8:].double().view(H, d)
+        s = torch.einsum("hd,thd->ht", qr, k) / math.sqrt(d)
+        want = torch.einsum("ht,thd->hd", s.softmax(-1), v)
+        # a score is off by at most (d + 2) U of the sum of its products' magnitudes, a weight by twice that relatively
+        # and by the exponential's few U, a sum of n weights and products by n + 16 U
+        most = float((torch.einsum("hd,thd->ht", qr.abs(), k.abs()) / math.sqrt(d)).max())
+        bound = (2 * (d + 2) * most + 2 * (p + 1 - first + 16) + 16) * U * float(v.abs().max())
+        assert float((out[r].double().view(H, d) - want).abs().max()) <= bound
