@@ -990,6 +990,348 @@ __global__ __launch_bounds__(SNT) void sample_end_kernel(const float* __restrict
   sample_row_one_block(sh.one, logits + (size_t)row * sz.ldl, sz.V, temperature[row], top_k[row], tp, r, out + row);
 }
 
+// ---- Rows that all keep at most SMALL_MAX candidates (0 < top-k <= 1,024), in two launches ----
+// The k largest of a row are among the k largest of its pieces: every block leaves its piece's (and up to FEW_SPARE more,
+// so that a coarse threshold will do), one block a row selects the row's k from those exactly, sorts them and does the
+// reference's sequential arithmetic.  A threshold is found by radix descent over the same 64-bit sort key as below, 11
+// bits a pass, with the histogram in LDS.  What bounds it is latency: each launch is a handful of passes over values that
+// are in L2 after the first, each with two or three barriers; the descents above make five launches of it, each of which
+// begins with where the one before it left off.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 10 + 20 us (the descents:
+// 73 us in seven launches).  Of the 20 us, by clock readings inside the kernel: the pieces' results 2, their candidates 4,
+// the selection 5, sorting and exponentials 3, the sums in order 5.
+constexpr int FEW_SPARE = 128, FEW_STRIDE = SMALL_MAX + FEW_SPARE;
+constexpr int FEW_BITS = 11, FEW_BINS = 1 << FEW_BITS;
+
+struct FewSpace {
+  float* piece_best;       // [row][pieces] ...
+  int* piece_arg;
+  uint32_t* piece_finite;
+  uint32_t* piece_count;   // candidates left
+  uint32_t* key;           // [row][pieces][FEW_STRIDE]
+  int* id;
+  size_t bytes;
+};
+
+int most_pieces(int R) {
+  const int want = ceil_div(512, R);
+  return want > MAX_PIECES ? MAX_PIECES : want;
+}
+
+FewSpace carve_few(void* base, int R) {
+  FewSpace s;
+  size_t at = 0;
+  auto take = [&](size_t bytes) { char* q = (char*)((uintptr_t)base + at); at += round16(bytes); return q; };
+  const size_t n = (size_t)R * most_pieces(R);
+  s.piece_best = (float*)take(n * 4);
+  s.piece_arg = (int*)take(n * 4);
+  s.piece_finite = (uint32_t*)take(n * 4);
+  s.piece_count = (uint32_t*)take(n * 4);
+  s.key = (uint32_t*)take(n * FEW_STRIDE * 4);
+  s.id = (int*)take(n * FEW_STRIDE * 4);
+  s.bytes = at;
+  return s;
+}
+
+struct alignas(8) FewShared {
+  uint32_t hist[FEW_BINS];
+  uint32_t wave_sum[PNT / WAVE];
+  uint32_t bin, above, at_bin, count;
+  float bv[PNT / WAVE];
+  int bi[PNT / WAVE];
+  uint32_t nv[PNT / WAVE];
+};
+
+// The largest threshold c (a sort key with zeros below some digit) at which at least k and at most `most` >= k of the
+// values stand at or above it; `each(f)` calls f(sort key) for the values of the block's NT threads.  Fewer than k values:
+// 0.  With most == k the answer is exact: sort keys are all different.
+template <int NT, typename Each>
+__device__ __forceinline__ u64 few_threshold(FewShared& sh, uint32_t k, uint32_t most, int key_bits, Each&& each) {
+  constexpr int PER = FEW_BINS / NT;
+  u64 prefix = 0;
+  uint32_t above = 0;                                   // values above the prefix's range
+  for (int hi = 64;;) {
+    const int lo = hi - FEW_BITS;                       // (ends at 9 or before: an id has at most 22 bits, see apc_sample_rows)
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < PER; ++g) sh.hist[threadIdx.x + g * NT] = 0;
+    if (threadIdx.x == 0) sh.bin = 0xffffffffu;
+    __syncthreads();
+    each([&](u64 c) {
+      if (hi < 64 && (c >> hi) != (prefix >> hi)) return;
+      atomicAdd(&sh.hist[(uint32_t)(c >> lo) & (FEW_BINS - 1)], 1u);
+    });
+    __syncthreads();
+    // threads in descending order of the bins
+    const int top = FEW_BINS - 1 - PER * (int)threadIdx.x, lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    uint32_t h[PER], own = 0;
+#pragma unroll
+    for (int g = 0; g < PER; ++g) own += h[g] = sh.hist[top - g];
+    uint32_t v = own;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+      const uint32_t up = __shfl_up(v, o, WAVE);
+      if (lane >= o) v += up;
+    }
+    if (lane == WAVE - 1) sh.wave_sum[wave] = v;
+    __syncthreads();
+    uint32_t before = above + v - own;
+#pragma unroll
+    for (int w = 0; w < NT / WAVE; ++w)
+      if (w < wave) before += sh.wave_sum[w];
+#pragma unroll
+    for (int g = 0; g < PER; ++g) {
+      if (before < k && k <= before + h[g]) sh.bin = top - g, sh.above = before, sh.at_bin = h[g];
+      before += h[g];
+    }
+    __syncthreads();
+    if (sh.bin == 0xffffffffu) return 0;                // (the first pass only: fewer than k values)
+    prefix |= (u64)sh.bin << lo;
+    above = sh.above;
+    if (above + sh.at_bin <= most || lo <= 64 - key_bits) return prefix;
+    hi = lo;
+  }
+}
+
+__device__ __forceinline__ void first_max(float& best, int& best_i, float ov, int oi) {
+  if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
+}
+
+__global__ __launch_bounds__(PNT) void sample_few_pieces_kernel(const float* __restrict__ logits, SampleShape sz,
+                                                                const float* __restrict__ temperature,
+                                                                const int* __restrict__ top_k, FewSpace sp) {
+  __shared__ FewShared sh;
+  const int row = blockIdx.y, piece = blockIdx.x;
+  const float* lg = logits + (size_t)row * sz.ldl;
+  const float t = fmaxf(temperature[row], 1e-5f);
+  const int tk = top_k[row];
+  const int i0 = piece * sz.chunk, i1 = min(sz.V, i0 + sz.chunk);
+  float best = -INFINITY;
+  int best_i = 0x7fffffff;
+  uint32_t nfin = 0;
+  for_piece(lg, sz.vec, i0, i1, [&](int i, float v) {
+    if (v > best) { best = v; best_i = i; }
+    nfin += finite_f(v) ? 1u : 0u;
+  });
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) {
+    first_max(best, best_i, __shfl_xor(best, o, WAVE), __shfl_xor(best_i, o, WAVE));
+    nfin += __shfl_xor(nfin, o, WAVE);
+  }
+  if (threadIdx.x % WAVE == 0) {
+    sh.bv[threadIdx.x / WAVE] = best;
+    sh.bi[threadIdx.x / WAVE] = best_i;
+    sh.nv[threadIdx.x / WAVE] = nfin;
+  }
+  if (threadIdx.x == 0) sh.count = 0;
+  __syncthreads();
+  nfin = 0;
+  for (int w = 0; w < PNT / WAVE; ++w) {
+    first_max(best, best_i, sh.bv[w], sh.bi[w]);
+    nfin += sh.nv[w];
+  }
+  const size_t at = (size_t)row * sz.pieces + piece;
+  if (threadIdx.x == 0) {
+    sp.piece_best[at] = best;
+    sp.piece_arg[at] = best_i;
+    sp.piece_finite[at] = nfin;
+  }
+  if (tk <= 0 || tk > SMALL_MAX || temperature[row] <= 1e-5f) return;   // the last launch knows what to do with the row
+  auto each = [&](auto f) {
+    for_piece(lg, sz.vec, i0, i1, [&](int i, float x) {
+      if (finite_f(x)) f(sort_key(key_of(x / t), i, sz.id_bits, 0));
+    });
+  };
+  const u64 from = nfin <= (uint32_t)(tk + FEW_SPARE) ? 0 : few_threshold<PNT>(sh, tk, tk + FEW_SPARE, 32 + sz.id_bits, each);
+  each([&](u64 c) {
+    if (c < from) return;
+    const uint32_t j = atomicAdd(&sh.count, 1u);        // (at most tk + FEW_SPARE of them)
+    sp.key[at * FEW_STRIDE + j] = (uint32_t)(c >> 32);
+    sp.id[at * FEW_STRIDE + j] = id_of_sort_key(c, sz.id_bits, 0);
+  });
+  __syncthreads();
+  if (threadIdx.x == 0) sp.piece_count[at] = sh.count;
+}
+
+// a[0] + a[1] + .. of the first n values, one after the other (the order of the reference's sums), by one wave; `each`
+// gets lane i's running sum for value i.  (Loops of a few instructions: a block alone pays for every line of code it
+// brings in, and written out 64 times these sums took longer than all else.)
+template <typename Each>
+__device__ __forceinline__ float sum_in_order(const float* a, int n, Each&& each) {
+  const int lane = threadIdx.x % WAVE;
+  float acc = 0.f;
+  for (int i0 = 0; i0 < n; i0 += WAVE) {
+    const float mine = i0 + lane < n ? a[i0 + lane] : 0.f;
+    float run = 0.f;
+    const int m = min(WAVE, n - i0);
+#pragma unroll 1
+    for (int l = 0; l < m; ++l) {
+      acc += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), l));
+      run = lane == l ? acc : run;
+    }
+    if (each(i0 + lane, run)) break;
+  }
+  return acc;
+}
+
+constexpr int FEW_HELD = 6144;           // candidates of a row that are held in LDS (all of them up to top-k 64)
+struct FewEnd {
+  FewShared select;
+  SampleShared one;
+  u64 held[FEW_HELD];
+  uint32_t from[MAX_PIECES + 1];         // where the candidates of a piece begin
+};
+
+__global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __restrict__ logits, SampleShape sz,
+                                                             const float* __restrict__ temperature,
+                                                             const int* __restrict__ top_k, const float* __restrict__ top_p,
+                                                             const float* __restrict__ uniform, FewSpace sp, int* __restrict__ out) {
+  __shared__ FewEnd sh;
+  const int row = blockIdx.x, tk = top_k[row];
+  const float T = temperature[row], tp = top_p[row];
+  float best = -INFINITY;
+  int best_i = 0x7fffffff;
+  uint32_t n = 0;
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  if (lane < sz.pieces) {                               // every wave for itself, a piece a lane
+    const size_t at = (size_t)row * sz.pieces + lane;
+    best = sp.piece_best[at];
+    best_i = sp.piece_arg[at];
+    n = sp.piece_finite[at];
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) {
+    first_max(best, best_i, __shfl_xor(best, o, WAVE), __shfl_xor(best_i, o, WAVE));
+    n += __shfl_xor(n, o, WAVE);
+  }
+  if (n == 0u || T <= 1e-5f) {
+    if (threadIdx.x == 0) out[row] = n == 0u || best_i == 0x7fffffff ? 0 : best_i;
+    return;
+  }
+  const bool cut = tk > 0 && n > (uint32_t)tk;
+  const uint32_t keep = cut ? (uint32_t)tk : n;
+  const bool use_top_p = tp >= 0.0f && tp < 1.0f && keep > 1u;
+  if (tk <= 0 || tk > SMALL_MAX || !(cut || use_top_p)) {
+    // the caller's word on the row was wrong, or fewer candidates than top-k keeps and no top-p: drawn in id order
+    sample_row_one_block(sh.one, logits + (size_t)row * sz.ldl, sz.V, T, tk, tp, uniform[row], out + row);
+    return;
+  }
+  if (wave == 0) {
+    uint32_t v = lane < sz.pieces ? sp.piece_count[(size_t)row * sz.pieces + lane] : 0u;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+      const uint32_t up = __shfl_up(v, o, WAVE);
+      if (lane >= o) v += up;
+    }
+    if (lane == 0) sh.from[0] = 0;
+    if (lane < MAX_PIECES) sh.from[lane + 1] = v;
+  }
+  __syncthreads();
+  const uint32_t total = sh.from[MAX_PIECES];
+  const bool held = total <= (uint32_t)FEW_HELD;
+  auto candidate = [&](int p, int j) {
+    const size_t at = ((size_t)row * sz.pieces + p) * FEW_STRIDE + j;
+    return sort_key(sp.key[at], sp.id[at], sz.id_bits, 0);
+  };
+  if (held) {                                           // the first 128 of all of a wave's pieces are asked for together
+    constexpr int MINE = MAX_PIECES / (SNT / WAVE);
+    u64 c[MINE][2];
+#pragma unroll
+    for (int g = 0; g < MINE; ++g)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        // (places that hold no candidate are read too: there is room for FEW_STRIDE in every piece)
+        c[g][u] = candidate(min(wave + g * (SNT / WAVE), sz.pieces - 1), lane + u * WAVE);
+      }
+#pragma unroll
+    for (int g = 0; g < MINE; ++g) {
+      const int p = wave + g * (SNT / WAVE), count = (int)(sh.from[p + 1] - sh.from[p]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (lane + u * WAVE < count) sh.held[sh.from[p] + lane + u * WAVE] = c[g][u];
+      for (int j = lane + 2 * WAVE; j < count; j += WAVE) sh.held[sh.from[p] + j] = candidate(p, j);
+    }
+    __syncthreads();
+  }
+  auto each = [&](auto f) {                             // every candidate of the row's pieces
+    if (held) {
+      for (int i = threadIdx.x; i < (int)total; i += SNT) f(sh.held[i]);
+    } else {
+      for (int p = wave; p < sz.pieces; p += SNT / WAVE)
+        for (int j = lane; j < (int)(sh.from[p + 1] - sh.from[p]); j += WAVE) f(candidate(p, j));
+    }
+  };
+  u64* picked = reinterpret_cast<u64*>(sh.select.hist);  // (the histogram is done with by then)
+  static_assert(sizeof(sh.select.hist) >= SMALL_MAX * sizeof(u64), "the candidates that are kept fit the histogram's room");
+  if (threadIdx.x == 0) sh.select.count = 0;
+  const u64 from = cut ? few_threshold<SNT>(sh.select, keep, keep, 32 + sz.id_bits, each) : 0;
+  __syncthreads();
+  each([&](u64 c) {
+    if (c < from) return;
+    const uint32_t j = atomicAdd(&sh.select.count, 1u);
+    if (j < (uint32_t)SMALL_MAX) picked[j] = c;
+  });
+  __syncthreads();
+  // as `sample_few`, with the exponentials and quotients by all threads and the sums in order by one wave
+  const int cnt = (int)keep;
+  for (int e = threadIdx.x; e < cnt; e += SNT) {
+    const u64 mine = picked[e];
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < cnt; ++j) rank += picked[j] > mine ? 1 : 0;
+    sh.one.s_key2[rank] = (uint32_t)(mine >> 32);
+    sh.one.s_id2[rank] = id_of_sort_key(mine, sz.id_bits, 0);
+  }
+  __syncthreads();
+  float* e = reinterpret_cast<float*>(sh.one.s_key);
+  const float vmax = value_of(sh.one.s_key2[0]);
+  for (int i = threadIdx.x; i < cnt; i += SNT) e[i] = expf(value_of(sh.one.s_key2[i]) - vmax);
+  __syncthreads();
+  if (wave != 0) return;
+  auto all = [](int, float) { return false; };
+  int m = cnt;
+  if (use_top_p) {
+    const float sum = sum_in_order(e, m, all);
+    if (sum == 0.f || !finite_f(sum)) {
+      const int some = (int)ceilf(tp * (float)m);
+      m = some < 1 ? 1 : (some > m ? m : some);
+    } else {
+      float* share = reinterpret_cast<float*>(sh.one.s_id);
+      for (int i = lane; i < cnt; i += WAVE) share[i] = e[i] / sum;
+      __builtin_amdgcn_wave_barrier();
+      int first = m - 1;
+      sum_in_order(share, cnt, [&](int i, float run) {
+        const unsigned long long hit = __ballot(i < cnt && run >= tp);
+        if (hit) first = i - lane + __ffsll(hit) - 1;
+        return hit != 0;
+      });
+      m = first + 1;
+    }
+  }
+  const float sum = sum_in_order(e, m, all);
+  float* share = reinterpret_cast<float*>(sh.one.s_id);
+  for (int i = lane; i < m; i += WAVE) share[i] = sum == 0.f ? 1.0f / (float)m : e[i] / sum;
+  __builtin_amdgcn_wave_barrier();
+  // r - p[0] - p[1] - ..: the first candidate at which nothing is left
+  int pick = m - 1;
+  float left = uniform[row];
+  for (int i0 = 0; i0 < m; i0 += WAVE) {
+    const float mine = i0 + lane < m ? share[i0 + lane] : 0.f;
+    float run = 0.f;
+    const int here = min(WAVE, m - i0);
+#pragma unroll 1
+    for (int l = 0; l < here; ++l) {
+      left -= __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), l));
+      run = lane == l ? left : run;
+    }
+    const unsigned long long hit = __ballot(i0 + lane < m && run <= 0.f);
+    if (hit) {
+      pick = i0 + __ffsll(hit) - 1;
+      break;
+    }
+  }
+  if (lane == 0) out[row] = sh.one.s_id2[pick];
+}
+
 std::mutex pass_attr_lock;
 bool pass_attr_set[64];
 
@@ -998,7 +1340,8 @@ bool pass_attr_set[64];
 // KiB of working memory that apc_sample_rows wants for n_rows rows (it takes the one-block way without)
 APC_EXPORT int apc_sample_rows_scratch_kib(int n_rows) {
   if (n_rows <= 0 || n_rows > 65535) return 0;
-  return (int)((carve(nullptr, n_rows).bytes + 1023) / 1024);
+  const size_t bytes = carve(nullptr, n_rows).bytes, few = carve_few(nullptr, n_rows).bytes;
+  return (int)(((bytes > few ? bytes : few) + 1023) / 1024);
 }
 
 // `cuts`: bit 0 set if some row may have top-k > 0, bit 1 if some row may have 0 <= top-p < 1, bit 2 if every row that
@@ -1022,8 +1365,10 @@ APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, 
     APC_LAUNCH_CHECK();
     return 0;
   }
-  if (((uintptr_t)scratch & 15u) || scratch_bytes < carve(nullptr, n_rows).bytes) return APC_ERR_BAD_ARG;
-  {
+  const bool few = (cuts & 5) == 5;
+  if (((uintptr_t)scratch & 15u) || scratch_bytes < (few ? carve_few(nullptr, n_rows).bytes : carve(nullptr, n_rows).bytes))
+    return APC_ERR_BAD_ARG;
+  if (!few) {
     std::lock_guard<std::mutex> hold(pass_attr_lock);
     if (!pass_attr_set[dev]) {
       const hipError_t e = hipFuncSetAttribute((const void*)sample_pass_kernel,
@@ -1032,7 +1377,6 @@ APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, 
       pass_attr_set[dev] = true;
     }
   }
-  const SampleSpace sp = carve(scratch, n_rows);
   SampleShape sz;
   sz.ldl = ldl;
   sz.V = V;
@@ -1044,15 +1388,23 @@ APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, 
   sz.key_digits = ceil_div(32 + sz.id_bits, DIGIT_BITS);
   sz.id_digits = ceil_div(sz.id_bits, DIGIT_BITS);
   const dim3 grid(sz.pieces, n_rows);
+  if (few) {
+    const FewSpace fs = carve_few(scratch, n_rows);
+    hipLaunchKernelGGL(sample_few_pieces_kernel, grid, dim3(PNT), 0, stream, logits, sz, temperature, top_k, fs);
+    APC_LAUNCH_CHECK();
+    hipLaunchKernelGGL(sample_few_end_kernel, dim3(n_rows), dim3(SNT), 0, stream, logits, sz, temperature, top_k, top_p, uniform, fs, out);
+    APC_LAUNCH_CHECK();
+    return 0;
+  }
+  const SampleSpace sp = carve(scratch, n_rows);
   hipLaunchKernelGGL(sample_max_kernel, grid, dim3(PNT), 0, stream, logits, sz, sp);
   APC_LAUNCH_CHECK();
-  const bool few = (cuts & 5) == 5;
   int q = 0, prev_stage = -1, prev_digit = -1;
   for (int stage = 0; stage < N_SELECTS; ++stage) {
     int digits = sz.key_digits;
     if (stage == ST_TOPK && !(cuts & 1)) continue;
-    if (stage == ST_TOPP && (!(cuts & 2) || few)) continue;
-    if (stage == ST_DRAW) digits = few ? 1 : ((cuts & 3) ? sz.key_digits : sz.id_digits);
+    if (stage == ST_TOPP && !(cuts & 2)) continue;
+    if (stage == ST_DRAW) digits = (cuts & 3) ? sz.key_digits : sz.id_digits;
     for (int digit = 0; digit < digits; ++digit) {
       hipLaunchKernelGGL(sample_pass_kernel, grid, dim3(PNT), sizeof(PassShared), stream, logits, sz, temperature,
                          top_k, top_p, uniform, sp, q, stage, digit, prev_stage, prev_digit);

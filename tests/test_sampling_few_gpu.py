@@ -1,0 +1,66 @@
+"""Rows whose top-k keeps at most 1,024 candidates, chosen in two launches: every token is the one that the kernel of one
+block a row gives, which walks the same candidates in the same order with the same float32 sums."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def both_ways(logits, temperature, top_k, top_p, uniform):
+    from allpaca_amd.kernels import ops
+    R = logits.shape[0]
+    f = lambda x, dt: torch.tensor(np.broadcast_to(np.asarray(x), R).copy(), dtype=dt, device=DEV)  # noqa: E731
+    args = (f(temperature, torch.float32), f(top_k, torch.int32), f(top_p, torch.float32), f(uniform, torch.float32))
+    got, want = (torch.full((R,), -7, dtype=torch.int32, device=DEV) for _ in range(2))
+    ops.sample_rows(logits, *args, got, few_after_top_k=True)
+    ops.sample_rows(logits, *args, want, one_block=True)
+    return got.tolist(), want.tolist()
+
+
+# vocabularies of one piece, of ragged pieces, of rows that start off 16 bytes; rows with many and with few pieces
+@pytest.mark.parametrize("V,R", [(7, 3), (1003, 5), (4099, 9), (32001, 70), (128256, 8), (60000, 600)])
+def test_random_rows(V, R):
+    g = torch.Generator(device=DEV).manual_seed(V)
+    rng = np.random.default_rng(V)
+    logits = torch.randn(R, V, generator=g, device=DEV) * 3
+    for top_k in (1, 40, 63, 64, 65, 1024):
+        for top_p in (0.0, 0.5, 0.95, 1.0):
+            if V >= 32001 and (top_k, top_p) not in ((1, 0.95), (40, 0.95), (64, 0.5), (65, 1.0), (1024, 0.95)):
+                continue                                     # (a row of one block takes milliseconds there)
+            got, want = both_ways(logits, 0.8, top_k, top_p, rng.random(R))
+            assert got == want, (top_k, top_p)
+
+
+@pytest.mark.parametrize("V", [513, 9001])
+def test_equal_values_infinities_and_masked_rows(V):
+    rng = np.random.default_rng(1)
+    rows = [np.full(V, 1.5), np.round(rng.normal(size=V)), np.full(V, -np.inf), np.full(V, np.nan), rng.normal(size=V),
+            rng.normal(size=V), rng.normal(size=V), np.where(np.arange(V) % 2, 0.0, -0.0), rng.normal(size=V) * 1e-30,
+            rng.normal(size=V) * 1e30]
+    rows[1][::3] = -0.0
+    rows[4][rng.random(V) < 0.98] = -np.inf                  # fewer candidates than top-k keeps
+    rows[5][[3, 77]] = np.inf
+    rows[6][:] = -np.inf
+    rows[6][[5, 500]] = 2.0, 2.0
+    logits = torch.tensor(np.stack(rows), dtype=torch.float32, device=DEV)
+    for top_k in (1, 40, 300, 1024):
+        for top_p in (0.3, 0.95, 1.0):
+            for u in (0.0, 0.37, 0.999999):
+                got, want = both_ways(logits, 0.7, top_k, top_p, u)
+                assert got == want, (top_k, top_p, u)
+
+
+def test_greedy_rows_and_rows_the_callers_word_was_wrong_about():
+    g = torch.Generator(device=DEV).manual_seed(5)
+    logits = torch.randn(6, 20000, generator=g, device=DEV)
+    logits[1, 19999] = logits[1, 44] = 50.0                  # greedy: the first of two maxima
+    rng = np.random.default_rng(2)
+    got, want = both_ways(logits, [0.8, 0.0, 1.3, 1e-6, 0.5, 0.9], [40, 0, 0, 7, 3000, 40], [0.9, 0.9, 0.9, 1.0, 0.9, 1.0], rng.random(6))
+    assert got == want and got[1] == 44
+    # a view of a wider matrix whose rows start off 16 bytes
+    wide = torch.randn(6, 20003, generator=g, device=DEV)
+    got, want = both_ways(wide[:, 1:20002], 0.8, 40, 0.95, rng.random(6))
+    assert got == want
