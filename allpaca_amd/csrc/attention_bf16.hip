@@ -23,6 +23,7 @@
 // cores): attention_qtile_kernel hip/src/kernels.cpp:2203, attention_split_gqa_kernel 2276, merges 2479-2516.
 #include "attention_wide.h"
 #include "mfma.h"
+#include <algorithm>
 #include <math.h>
 
 constexpr int KT = 64;            // keys per tile in the prefill kernel
@@ -537,7 +538,7 @@ struct KVRegs {
   Frag v[DP / 16];     // 32 positions of 16 value elements per tile
 };
 
-// Three ways to the finished heads of a (row, kv head):
+// Ways to the finished heads of a (row, kv head):
 //  DEC_PARTS  a block is 4 parts (ranges of KW keys) of the pair; its waves leave their results in `parts` and
 //             attn_merge_kernel, a second launch, finishes.  Kept for the sizes the other two do not take.
 //  DEC_LAST   the same split over blocks, but a block first adds its 4 waves' results in LDS, leaves ONE partial
@@ -555,10 +556,19 @@ struct KVRegs {
 //             which pays once the pairs alone fill the chip (8B shapes, 2,048 keys a row: 32 rows 52.9 -> 49.1 us, 64
 //             rows 98.2 -> 91.6 us, 128 rows 196 -> 181 us; with 16 rows 30.2 -> 34.7 us.  Blocks of 8 waves were 2 %
 //             faster at one block a compute unit and 8-15 % slower at two).
-// The order of additions for a row depends on its position, KW and the number of parts only.
+//  DEC_EVEN   rows of very different lengths, where a block a pair leaves the chip waiting for the longest row's block (64
+//             rows of 90 to 2,100 keys: 63 us of which the bytes are 23).  Each kv head's work, the steps of 32 keys of
+//             all its rows one after the other (a row counts two steps more for what it costs beside its keys), goes in
+//             equal shares to the waves of one round of blocks; every wave finds its share and the rows it falls into
+//             from the rows' positions, so a recorded graph fits whatever lengths they reach.  A row inside one share is
+//             finished by its wave; the pieces of a row that lies in several go through memory as in DEC_LAST, and the
+//             wave that leaves the last of them adds them in order.  37 us there, and no slower where rows are equal
+//             (64 rows of 2,048: 90 and 88 us).  What is left over the bytes is a wave's chain of rows: about 4 us each.
+// The order of additions for a row depends on its position, KW and the number of parts only (DEC_EVEN: on the lengths of
+// the rows in front of it too).
 constexpr int NW = 4;  // waves of a block of the decode kernel
 constexpr int LAST_DIRECT = 8;  // up to so many blocks a pair the last one reads the others' results in one go
-enum { DEC_PARTS = 0, DEC_WHOLE = 1, DEC_LAST = 2 };
+enum { DEC_PARTS = 0, DEC_WHOLE = 1, DEC_LAST = 2, DEC_EVEN = 3 };
 // Keys a part of a row takes when the launch gives the number of parts and not their length (KW == 0): the row's
 // `span` keys in n_parts equal ranges, in whole steps of 32 keys and no fewer than 64.  Rows of different lengths in
 // one launch then all use every block of their pair, and a launch's shape (blocks a pair) does not change with the
@@ -584,35 +594,76 @@ __device__ __forceinline__ void st_coh(float* p, float v) {
 __device__ __forceinline__ float ld_coh(const float* p) {
   return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// The same accesses (sc1, as the two above compile to), 16 and 8 bytes at a time; places in floats.
+constexpr int COHERENT = 16;
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void st_coh4(BufferRsrc to, int place, floatx4 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), to, 4 * place, 0, COHERENT);
+}
+__device__ __forceinline__ floatx4 ld_coh4(BufferRsrc from, int place) {
+  return __builtin_bit_cast(floatx4, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(from, 4 * place, 0, COHERENT));
+}
+__device__ __forceinline__ floatx2 ld_coh2(BufferRsrc from, int place) {
+  return __builtin_bit_cast(floatx2, (u32x2_t)__builtin_amdgcn_raw_buffer_load_b64(from, 4 * place, 0, COHERENT));
+}
+__device__ __forceinline__ int wave_sum_int(int v) {
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+  return v;
+}
+__device__ __forceinline__ int wave_scan_int(int v) {  // the sum of this lane's and all earlier lanes' values
+#pragma unroll
+  for (int o = 1; o < WAVE; o <<= 1) {
+    const int up = __shfl_up(v, o, WAVE);
+    if ((int)(threadIdx.x % WAVE) >= o) v += up;
+  }
+  return v;
+}
+// DEC_EVEN: what a row costs beside its steps of 32 keys (page ids, query, the first loads' way, its result), in steps,
+// and the least that a wave is given.
+// EVEN_BLOCKS: a block a compute unit (two, where registers allow them, were slower: 64 ragged rows 37 -> 48 us, more
+// pieces and as many bytes in flight).  EVEN_BATCH: pieces of a row that the last wave asks for together.
+constexpr int EVEN_ROW_COST = 2, EVEN_MIN_SHARE = 8, EVEN_BLOCKS = 256, EVEN_BATCH = 4;
 template <int DP, int MODE>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
     const bf16_t* __restrict__ q, int ldq, int q_off, int H, int Hk, int d, const bf16_t* __restrict__ cache, int P,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ positions,
     const int* __restrict__ row_seg, const int* __restrict__ rows, int window, float scale, int KW, int n_parts,
     float* __restrict__ parts, bf16_t* __restrict__ out, int ldo, int* __restrict__ counters) {
-  constexpr bool WHOLE = MODE == DEC_WHOLE, LAST = MODE == DEC_LAST;
+  constexpr bool WHOLE = MODE == DEC_WHOLE, LAST = MODE == DEC_LAST, EVEN = MODE == DEC_EVEN;
   __shared__ __attribute__((aligned(16))) bf16_t Ps[NW * 16 * (32 + KPAD)];
   extern __shared__ __attribute__((aligned(16))) float meet[];  // WHOLE, LAST: [NW][heads of the tile][d + 2]
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   const int li = lane % 16, lc = lane / 16;
   const int G = H / Hk, gtiles = (G + 15) / 16;
   const int ri = blockIdx.x;
-  const int row = rows ? rows[ri] : ri;
   const int kvh = blockIdx.y / gtiles, gt = blockIdx.y % gtiles;
   const int part = blockIdx.z * NW + wave;
-  const int pos = positions[row];
-  const int first = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
-  const int seen0 = (first / 32) * 32;  // the first position that is loaded
-  // KW == 0: the row's own keys, from the first one it sees, in n_parts equal ranges (see row_keys_per_part); else
-  // ranges of KW keys counted from position 0
-  const int base = KW > 0 ? 0 : seen0;
-  KW = row_keys_per_part(KW, pos + 1 - seen0, n_parts);
-  // nothing to see for this part: the wave leaves (DEC_PARTS), or stays with an empty result (DEC_LAST: the block's
-  // waves meet)
-  const bool empty =
-      !WHOLE && (part >= n_parts || max(base + part * KW, seen0) >= min(base + (part + 1) * KW, pos + 1));
-  if (MODE == DEC_PARTS && empty) return;
-  const int* bt = block_table + (size_t)row_seg[row] * max_blocks;
+  int row = 0, pos = 0, first = 0, seen0 = 0;  // the row in work; seen0: the first position that is loaded
+  const int* bt = nullptr;
+  auto take_row = [&](int r, int position, int seg) {
+    row = r;
+    pos = position;
+    first = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+    seen0 = (first / 32) * 32;
+    bt = block_table + (size_t)seg * max_blocks;
+  };
+  bool empty = false;
+  int base = 0;
+  if constexpr (!EVEN) {
+    const int r = rows ? rows[ri] : ri;
+    take_row(r, positions[r], row_seg[r]);
+    // KW == 0: the row's own keys, from the first one it sees, in n_parts equal ranges (see row_keys_per_part); else
+    // ranges of KW keys counted from position 0
+    base = KW > 0 ? 0 : seen0;
+    KW = row_keys_per_part(KW, pos + 1 - seen0, n_parts);
+    // nothing to see for this part: the wave leaves (DEC_PARTS), or stays with an empty result (DEC_LAST: the block's
+    // waves meet)
+    empty = !WHOLE && (part >= n_parts || max(base + part * KW, seen0) >= min(base + (part + 1) * KW, pos + 1));
+    if (MODE == DEC_PARTS && empty) return;
+  }
   const size_t page_stride = (size_t)2 * Hk * P * d;
   const size_t head_off = (size_t)kvh * P * d, v_off = (size_t)Hk * P * d;
   // the page ids of a range of keys, one per lane, fetched once per range: the loads of keys and values then
@@ -620,7 +671,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
   int page0 = 0, my_page = 0;
 
   Frag qf[DP / 32];
-  {
+  floatx4 o[DP / 16];
+  float m_run, l_run;
+  auto begin_row = [&]() {
     const int g = gt * 16 + li;
     const bf16_t* qrow = q + (size_t)row * ldq + q_off + (size_t)(kvh * G + min(g, G - 1)) * d;
 #pragma unroll
@@ -628,11 +681,12 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
       const int e = ks * 32 + lc * 8;
       qf[ks] = (g < G && e < d) ? load_frag(qrow + e) : zero_frag();
     }
-  }
-  floatx4 o[DP / 16];
 #pragma unroll
-  for (int dt = 0; dt < DP / 16; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+    for (int dt = 0; dt < DP / 16; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    m_run = -INFINITY;
+    l_run = 0.f;
+  };
+  if constexpr (!EVEN) begin_row();
   bf16_t* pw = Ps + wave * 16 * (32 + KPAD);
 
   // Operands of 32 keys straight from the pages, with loads that the caches do not keep (a decoded row reads its keys
@@ -744,6 +798,146 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
   // a range in pieces of no more keys than a wave keeps page ids for (one piece, but for rows far longer than the
   // launch's parts were counted for, and for the one range a wave of DEC_WHOLE has of a long row)
   const int piece = max(32, (62 * P) / 32 * 32);
+  if constexpr (EVEN) {
+    // This wave's share of its kv head's work, and the rows it falls into.  Rows are looked at 64 at a time, one a lane.
+    const int waves = gridDim.x * NW, me = blockIdx.x * NW + wave;
+    int r_l = 0, pos_l = 0, seg_l = 0, cost_l = 0;
+    auto look_at = [&](int i0) {
+      cost_l = 0;
+      const int i = i0 + lane;
+      if (i >= n_parts) return;
+      r_l = rows ? rows[i] : i;
+      pos_l = positions[r_l];
+      seg_l = row_seg[r_l];
+      const int f = (window > 0 && pos_l - window + 1 > 0) ? pos_l - window + 1 : 0;
+      cost_l = (pos_l - f / 32 * 32) / 32 + 1 + EVEN_ROW_COST;
+    };
+    look_at(0);
+    int end_l = wave_scan_int(cost_l), total = __builtin_amdgcn_readlane(end_l, WAVE - 1);
+    if (n_parts > WAVE) {
+      for (int i0 = WAVE; i0 < n_parts; i0 += WAVE) {
+        look_at(i0);
+        total += wave_sum_int(cost_l);
+      }
+      look_at(0);
+    }
+    const int share = max(EVEN_MIN_SHARE, (total + waves - 1) / waves);
+    const int lo = me * share, hi = min(lo + share, total);
+    const int tile_heads = min(G - gt * 16, 16), stride = d + 4;     // (a piece of a head: its sums, maximum, sum, room)
+    const BufferRsrc pieces = make_rsrc(parts + (size_t)blockIdx.y * waves * 2 * tile_heads * stride);
+    for (int i0 = 0;;) {
+      const int start_l = end_l - cost_l;
+      unsigned long long todo = __ballot(cost_l > 0 && end_l > lo && start_l < hi);
+      const int before = __builtin_amdgcn_readlane(end_l, WAVE - 1);
+      for (; todo; todo &= todo - 1) {
+        const int l = __ffsll(todo) - 1;
+        const int steps0 = __builtin_amdgcn_readlane(start_l, l) + EVEN_ROW_COST;   // where the row's steps begin
+        const int steps = __builtin_amdgcn_readlane(end_l, l) - steps0;
+        const int s_lo = max(lo - steps0, 0), s_hi = min(hi - steps0, steps);
+        if (s_lo >= s_hi) continue;
+        take_row(__builtin_amdgcn_readlane(r_l, l), __builtin_amdgcn_readlane(pos_l, l), __builtin_amdgcn_readlane(seg_l, l));
+        begin_row();
+        const int k_hi = min(seen0 + 32 * s_hi, pos + 1);
+        for (int k = seen0 + 32 * s_lo; k < k_hi; k += piece) run_range(k, min(k + piece, k_hi));
+        const int g = gt * 16 + li;
+        const int w0 = steps0 / share, n_pieces = (steps0 + steps - 1) / share - w0 + 1;
+        bf16_t* heads = out + (size_t)row * ldo + (size_t)(kvh * G + gt * 16) * d;
+        if (n_pieces == 1) {
+          if (g < G) {
+#pragma unroll
+            for (int dt = 0; dt < DP / 16; ++dt) {
+              const int e = dt * 16 + lc * 4;
+              if (e < d) {
+                uint2 pk;
+                pk.x = bf16_pair(o[dt][0] / l_run, o[dt][1] / l_run);
+                pk.y = bf16_pair(o[dt][2] / l_run, o[dt][3] / l_run);
+                *reinterpret_cast<uint2*>(heads + (size_t)li * d + e) = pk;
+              }
+            }
+          }
+          continue;
+        }
+        // one of several pieces: the row's first piece is its wave's last, in place 1; the others are their wave's first
+        if (g < G) {
+          const int at = ((2 * me + (s_lo == 0 ? 1 : 0)) * tile_heads + li) * stride;
+#pragma unroll
+          for (int dt = 0; dt < DP / 16; ++dt) {
+            const int e = dt * 16 + lc * 4;
+            if (e < d) st_coh4(pieces, at + e, o[dt]);
+          }
+          if (lc == 0) st_coh4(pieces, at + d, floatx4{m_run, l_run, 0.f, 0.f});
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's stores have reached memory
+        int* counter = counters + (size_t)(i0 + l) * gridDim.y + blockIdx.y;
+        int done = 0;
+        if (lane == 0) done = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane(done) != n_pieces - 1) continue;
+        // the last of the row's waves: all pieces in order, some at a time
+        asm volatile("" ::: "memory");
+        if (lane == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+        const int quads = tile_heads * d / 4;
+        for (int x0 = 0; x0 < quads; x0 += 2 * WAVE) {   // two quads of elements a lane
+          floatx4 acc[2];
+          float m[2], sum[2];
+          int at[2], last[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int x = min(x0 + u * WAVE + lane, quads - 1), hg = 4 * x / d;
+            at[u] = (2 * w0 * tile_heads + hg) * stride + 4 * x - hg * d;
+            last[u] = (2 * w0 * tile_heads + hg) * stride + d;
+            acc[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+            m[u] = -INFINITY;
+            sum[u] = 0.f;
+          }
+          for (int p0 = 0; p0 < n_pieces; p0 += EVEN_BATCH) {
+            floatx4 po[2][EVEN_BATCH];
+            floatx2 ml[2][EVEN_BATCH];
+#pragma unroll
+            for (int p = 0; p < EVEN_BATCH; ++p)
+#pragma unroll
+              for (int u = 0; u < 2; ++u) {
+                const int pp = min(p0 + p, n_pieces - 1), off = (2 * pp + (pp == 0 ? 1 : 0)) * tile_heads * stride;
+                ml[u][p] = ld_coh2(pieces, last[u] + off);
+                po[u][p] = ld_coh4(pieces, at[u] + off);
+              }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              float m_new = m[u];
+#pragma unroll
+              for (int p = 0; p < EVEN_BATCH; ++p)
+                if (p0 + p < n_pieces) m_new = fmaxf(m_new, ml[u][p][0]);
+              const float m_safe = m_new == -INFINITY ? 0.f : m_new, old = exp2_neg(m[u] - m_safe);
+              m[u] = m_new;
+              sum[u] *= old;
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[u][r] *= old;
+#pragma unroll
+              for (int p = 0; p < EVEN_BATCH; ++p)
+                if (p0 + p < n_pieces) {
+                  const float wgt = exp2_neg(ml[u][p][0] - m_safe);
+                  sum[u] = fmaf(ml[u][p][1], wgt, sum[u]);
+#pragma unroll
+                  for (int r = 0; r < 4; ++r) acc[u][r] = fmaf(po[u][p][r], wgt, acc[u][r]);
+                }
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int x = x0 + u * WAVE + lane;
+            if (x >= quads) continue;
+            uint2 pk;
+            pk.x = bf16_pair(acc[u][0] / sum[u], acc[u][1] / sum[u]);
+            pk.y = bf16_pair(acc[u][2] / sum[u], acc[u][3] / sum[u]);
+            *reinterpret_cast<uint2*>(heads + 4 * x) = pk;
+          }
+        }
+      }
+      i0 += WAVE;
+      if (i0 >= n_parts || before >= hi) return;
+      look_at(i0);
+      end_l = before + wave_scan_int(cost_l);
+    }
+  }
   if constexpr (WHOLE) {
     // ranges wave, wave + NW, ..: with the row's own ranges (the launch gave no length) that is one range a wave
     for (int r = wave; base + r * KW <= pos; r += NW) {
@@ -1065,11 +1259,44 @@ APC_EXPORT int apc_attention_decode_bf16(const void* q, int ldq, int q_off, void
     return 0;
   }
   DEC_BY_HEAD(DEC_PARTS, grid, 0, n_parts, workspace, (int*)nullptr);
-#undef DEC_BY_HEAD
-#undef DEC_LAUNCH
   APC_LAUNCH_CHECK();
   hipLaunchKernelGGL(attn_merge_kernel, dim3(n_rows, H), dim3(MERGE_NT), 0, stream,
                      workspace, n_parts, keys_per_part, H, d, positions, rows, window, (bf16_t*)out, ldo);
+  APC_LAUNCH_CHECK();
+  return 0;
+}
+
+// Blocks of a launch of DEC_EVEN for every kv head (and tile of 16 of its heads).
+static int even_blocks(int H, int Hk) {
+  const int tiles = Hk * ((H / Hk + 15) / 16);
+  return std::max(1, EVEN_BLOCKS / tiles);
+}
+// Floats of the workspace below, 0 if the kernel does not take these sizes.
+APC_EXPORT int apc_attention_decode_even_workspace(int H, int Hk, int d) {
+  if (H <= 0 || Hk <= 0 || H % Hk || d <= 0 || d > 256 || d % 16) return 0;
+  const int G = H / Hk, tiles = Hk * ((G + 15) / 16);
+  return tiles * even_blocks(H, Hk) * NW * 2 * (G < 16 ? G : 16) * (d + 4);
+}
+// Decoded rows of any lengths, the work of all rows dealt out evenly (see DEC_EVEN).  workspace: as many
+// floats as apc_attention_decode_even_workspace says; counters: n_rows * Hk * ceil(H / Hk / 16) ints, zero before the
+// first call and zero again after every call.  Calls that share either must not overlap (one stream).
+APC_EXPORT int apc_attention_decode_even_bf16(const void* q, int ldq, int q_off, void* out, int ldo, int n_rows, int H,
+                                              int Hk, int d, const void* cache, int page_tokens, const int* block_table,
+                                              int max_blocks, const int* positions, const int* row_seg, const int* rows,
+                                              int window, float scale, float* workspace, int* counters,
+                                              hipStream_t stream) {
+  if (n_rows <= 0) return 0;
+  const int e = check_common(q, ldq, q_off, cache, H, Hk, d, page_tokens);
+  if (e) return e;
+  if (max_blocks <= 0 || window < 0 || !out || !workspace || !counters) return APC_ERR_BAD_ARG;
+  const int tiles = Hk * ((H / Hk + 15) / 16);
+  if (tiles > 65535) return APC_ERR_BAD_ARG;
+  if (ldo % 4 || ((uintptr_t)out & 7u)) return APC_ERR_UNSUPPORTED;  // outputs are stored 8 bytes at a time
+  const int keys_per_part = 0;
+  dim3 grid(even_blocks(H, Hk), tiles);
+  DEC_BY_HEAD(DEC_EVEN, grid, 0, n_rows, workspace, counters);
+#undef DEC_BY_HEAD
+#undef DEC_LAUNCH
   APC_LAUNCH_CHECK();
   return 0;
 }

@@ -49,7 +49,7 @@ struct Program {
   float final_norm_eps = 0.f;
   std::vector<ApcLayer> layers;
   std::vector<ApcPlanEntry> plan;
-  ApcTunables tun{256, 1, 1, 8, 2048, 0};
+  ApcTunables tun{256, 1, 1, 8, 2048, 0, 256, 1024};
   int* pair_counters = nullptr;
   int pair_capacity = 0;
   // ---- the step in work
@@ -415,6 +415,14 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
     const int* rows = s.all_rows_decode ? nullptr : s.decode_rows;
     const long pairs = (long)n * Hk * cdiv(H / Hk, 16);
     const int n_parts = decode_parts(pairs, span);
+    if (decode_even(pairs, span, P.tun.even_min_pairs, P.tun.even_min_span) && pairs <= P.pair_capacity && out.ld % 4 == 0 &&
+        ((uintptr_t)out.p & 7u) == 0) {
+      float* ws = P.floats((size_t)apc_attention_decode_even_workspace(H, Hk, d));
+      LAUNCH(P, "attention_decode_bf16 (even shares)",
+             apc_attention_decode_even_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width, s.positions,
+                                            s.row_seg, rows, window, sc, ws, P.pair_counters, P.stream));
+      return 1;
+    }
     // (rows so short that one block's waves take a pair's ranges need no partial results either)
     if ((pairs >= P.tun.whole_min_pairs || n_parts <= WHOLE_WAVES) && apc_attention_decode_whole_fits(H, Hk, d)) {
       // no length of the ranges: every row's own keys, one range a wave of its block
@@ -704,6 +712,9 @@ APC_HOST_EXPORT const char* apc_host_timing_report(void* prog) {
 APC_HOST_EXPORT int apc_host_rule_tiled_k_split(int M, int N, int K) { return apc_rules::tiled_k_split(M, N, K); }
 APC_HOST_EXPORT int apc_host_rule_decode_parts(long long pairs, int span) {
   return apc_rules::decode_parts((long)pairs, span);
+}
+APC_HOST_EXPORT int apc_host_rule_decode_even(long long pairs, int span, int min_pairs, int min_span) {
+  return apc_rules::decode_even((long)pairs, span, min_pairs, min_span);
 }
 APC_HOST_EXPORT int apc_host_rule_key_splits(int n_tiles, int n_heads, int keys, int window, int splits_max,
                                              int range_min) {

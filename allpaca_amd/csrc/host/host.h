@@ -74,7 +74,7 @@ struct ApcStep {
 
 // Rules that tests and measurements move; the defaults are the kernels' wrappers' own.
 struct ApcTunables {
-  int whole_min_pairs, last_block_merges, wide_tiles, key_splits_max, key_range_min, force_plain;
+  int whole_min_pairs, last_block_merges, wide_tiles, key_splits_max, key_range_min, force_plain, even_min_pairs, even_min_span;
 };
 
 }  // extern "C"

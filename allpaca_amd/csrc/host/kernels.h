@@ -72,6 +72,11 @@ int apc_attention_decode_bf16(const void* q, int ldq, int q_off, void* out, int 
                               const void* cache, int page_tokens, const int* block_table, int max_blocks,
                               const int* positions, const int* row_seg, const int* rows, int window, float scale,
                               int keys_per_part, int n_parts, float* workspace, int* counters, hipStream_t stream);
+int apc_attention_decode_even_bf16(const void* q, int ldq, int q_off, void* out, int ldo, int n_rows, int H, int Hk, int d,
+                                   const void* cache, int page_tokens, const int* block_table, int max_blocks,
+                                   const int* positions, const int* row_seg, const int* rows, int window, float scale,
+                                   float* workspace, int* counters, hipStream_t stream);
+int apc_attention_decode_even_workspace(int H, int Hk, int d);
 int apc_attention_decode_last_fits(int H, int Hk, int d, int n_parts);
 int apc_attention_decode_whole_fits(int H, int Hk, int d);
 int apc_attention_prefill_tile_rows();

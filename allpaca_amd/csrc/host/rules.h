@@ -43,6 +43,10 @@ inline int decode_parts(long pairs, int span) {
   return (int)std::max(1L, std::min((long)WHOLE_WAVES * per_pair, cdiv(span, 64)));
 }
 
+// whether a decode step's rows share out their work over all waves (rows of very different lengths): enough pairs that
+// no pair would be cut for its own sake, and a longest row that could be far longer than the others
+inline bool decode_even(long pairs, int span, int min_pairs, int min_span) { return pairs >= min_pairs && span > min_span; }
+
 // ranges of keys that the 128-row attention kernel cuts every tile of a step into; `keys`: of the longest prompt
 inline int key_splits(int n_tiles, int n_heads, int keys, int window, int splits_max, int range_min) {
   const long blocks = (long)n_tiles * n_heads;

@@ -99,8 +99,8 @@ class NativeProgram:
                                    1 if v.writes else 0)
             if L.apc_host_program_add_entry(self.handle, ctypes.byref(entry)) < 0:
                 return self._give_up()
-        self.counters = tuned._pair_counters(self.device, 4096)
-        self.counters.zero_()      # a count that a failed launch left would hold up every later step
+        # (this program's own: the steps of one engine never overlap, those of two may)
+        self.counters = torch.zeros(4096, dtype=torch.int32, device=self.device)
         self._set_tunables()
         self.arenas: List[torch.Tensor] = []
         self.arena: Optional[torch.Tensor] = None
@@ -127,12 +127,12 @@ class NativeProgram:
     def _rules() -> tuple:
         """The numbers the kernels' wrappers keep as module constants (tests and measurements move them)."""
         return (tuned.WHOLE_MIN_PAIRS, tuned.LAST_BLOCK_MERGES, tuned.WIDE_TILES, tuned.KEY_SPLITS_MAX,
-                tuned.KEY_RANGE_MIN, ops.FORCE_PLAIN)
+                tuned.KEY_RANGE_MIN, ops.FORCE_PLAIN, tuned.EVEN_MIN_PAIRS, tuned.EVEN_MIN_SPAN)
 
     def _set_tunables(self) -> None:
         t = H.ApcTunables(int(min(tuned.WHOLE_MIN_PAIRS, 1 << 30)), int(bool(tuned.LAST_BLOCK_MERGES)),
                           int(bool(tuned.WIDE_TILES)), int(tuned.KEY_SPLITS_MAX), int(tuned.KEY_RANGE_MIN),
-                          int(bool(ops.FORCE_PLAIN)))
+                          int(bool(ops.FORCE_PLAIN)), int(min(tuned.EVEN_MIN_PAIRS, 1 << 30)), int(tuned.EVEN_MIN_SPAN))
         self._tunables = self._rules()
         self.lib.apc_host_program_tunables(self.handle, ctypes.byref(t), self.counters.data_ptr(),
                                            self.counters.numel())

@@ -52,7 +52,8 @@ class ApcPacked(Structure):
 
 class ApcTunables(Structure):
     _fields_ = [("whole_min_pairs", c_int), ("last_block_merges", c_int), ("wide_tiles", c_int),
-                ("key_splits_max", c_int), ("key_range_min", c_int), ("force_plain", c_int)]
+                ("key_splits_max", c_int), ("key_range_min", c_int), ("force_plain", c_int),
+                ("even_min_pairs", c_int), ("even_min_span", c_int)]
 
 
 P, I = c_void_p, c_int
@@ -72,6 +73,7 @@ _lib.SIGNATURES["host"].update({
     "apc_host_timing_report": [P],
     "apc_host_rule_tiled_k_split": [I, I, I],
     "apc_host_rule_decode_parts": [c_longlong, I],
+    "apc_host_rule_decode_even": [c_longlong, I, I, I],
     "apc_host_rule_key_splits": [I, I, I, I, I, I],
     # ---- the cache manager's books
     "apc_pool_new": [I], "apc_pool_free": [P], "apc_pool_alloc": [P], "apc_pool_give_back": [P, I],

@@ -347,6 +347,20 @@ WHOLE_MIN_PAIRS = 256
 WHOLE_WAVES = 4   # waves of such a block (NW in attention_bf16.hip)
 
 
+# From so many pairs on, in steps whose longest row may have more keys than this, the rows' work is dealt out evenly over
+# all waves of one round of blocks (DEC_EVEN in attention_bf16.hip) instead of a block a pair, whose longest row sets the
+# launch's time.  Microseconds a layer, block a pair / even: 64 rows of 90 to 2,100 keys (24 heads of 128 on 8) 63.2 / 37.0,
+# 64 rows of 2,048 89.6 / 88, 32 rows of 328 to 4,296 65.8 / 40.2, one row of 4,096 beside 63 of 128 71 / 25, 64 rows of 90
+# to 2,100 with heads of 64 33.6 / 22.3; short rows pay more for the shares than they gain: 64 rows of 300 18.5 / 22.1, 200
+# rows of 30 to 700 with heads of 64 24.0 / 28.  With fewer pairs the way below, which cuts every pair for itself, is
+# faster (16 rows of 2,048 26.8 / 30, 8 rows 17.6 / 26).
+EVEN_MIN_PAIRS, EVEN_MIN_SPAN = 256, 1024
+
+
+def _decode_even(pairs: int, span: int) -> bool:
+    return pairs >= EVEN_MIN_PAIRS and span > EVEN_MIN_SPAN
+
+
 # With fewer pairs: the blocks of a pair leave one partial result each and the one that finishes last adds them (no
 # second kernel), where the sizes allow; False: partial results per wave and a kernel that merges them.
 LAST_BLOCK_MERGES = True
@@ -382,8 +396,9 @@ def _key_splits(step, n_heads: int, window: int) -> int:
 
 def _pair_counters(device: torch.device, pairs: int) -> torch.Tensor:
     """Zeroed int32 counters, one per (row, kv head tile), that live as long as the process: a call leaves them zero
-    again, and a replayed graph keeps pointing at them.  Grown by allocating anew; the old ones stay (graphs)."""
-    key = (device.type, device.index if device.index is not None else torch.cuda.current_device())
+    again, and a replayed graph keeps pointing at them.  Grown by allocating anew; the old ones stay (graphs).  Every
+    stream has its own: launches that share them must not overlap."""
+    key = (device.type, device.index if device.index is not None else torch.cuda.current_device(), _ops._stream())
     have = _counters.setdefault(key, [])
     if not have or have[-1].numel() < pairs:
         have.append(torch.zeros(max(1024, pairs), dtype=torch.int32, device=device))
@@ -433,6 +448,15 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
         rows = step.decode_rows.data_ptr() if step.decode_rows is not None else 0
         pairs = n * n_kv_heads * -(-(n_heads // n_kv_heads) // 16)
         n_parts = -(-step.max_decode_context // KEYS_PER_PART) if KEYS_PER_PART else _decode_parts(pairs, span)
+        if _decode_even(pairs, span) and not KEYS_PER_PART and ldo % 4 == 0 and out.data_ptr() % 8 == 0:
+            ws = torch.empty(L.apc_attention_decode_even_workspace(n_heads, n_kv_heads, head_dim), dtype=torch.float32,
+                             device=q.device)
+            _lib.check(L.apc_attention_decode_even_bf16(
+                q.data_ptr(), ldq, q_off, out.data_ptr(), ldo, n, n_heads, n_kv_heads, head_dim, cache.data_ptr(),
+                page_tokens, block_table.data_ptr(), block_table.shape[1], step.positions.data_ptr(),
+                step.row_seg.data_ptr(), rows, int(window), sc, ws.data_ptr(),
+                _pair_counters(q.device, pairs).data_ptr(), stream), "attention_decode_bf16 (even shares)")
+            return True
         # (rows so short that one block's waves take a pair's ranges need no partial results either)
         if ((pairs >= WHOLE_MIN_PAIRS or n_parts <= WHOLE_WAVES)
                 and L.apc_attention_decode_whole_fits(n_heads, n_kv_heads, head_dim)):

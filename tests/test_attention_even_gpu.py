@@ -1,0 +1,51 @@
+"""Decoded rows whose work is dealt out evenly over all waves of the launch, against the plain attention: rows inside one
+wave's share, rows in two and in many pieces, shares that end at a row's first and last step, more than 64 rows, groups
+wider than a tile of 16 heads, windows, pages of 8, and slots that hold NaN."""
+import pytest
+import torch
+
+from test_kernels_tuned import run_attention, tuned
+
+RAGGED = [1 + (i * 977) % 2100 for i in range(70)]
+
+
+@pytest.fixture
+def even(monkeypatch):
+    monkeypatch.setattr(tuned(), "EVEN_MIN_PAIRS", 1)
+    monkeypatch.setattr(tuned(), "EVEN_MIN_SPAN", 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Hk,d,P_,lens,rows,window", [
+    (32, 8, 128, 16, [2048, 1, 17, 700, 2047], [1] * 5, 0),
+    (6, 2, 64, 16, RAGGED, [1] * 70, 0),                          # rows looked at in two goes
+    (6, 2, 64, 16, RAGGED, [1] * 70, 300),
+    (8, 8, 128, 16, [256] * 32, [1] * 32, 0),                     # shares that end where rows do
+    (2, 1, 128, 16, [9000, 31, 32, 33, 1], [1] * 5, 0),           # one row over most of the waves
+    (6, 2, 48, 8, [4000, 129, 64, 1], [1] * 4, 0),                # a wave's keys in several pieces (pages of 8)
+    (20, 1, 32, 24, [100, 2600, 64], [1] * 3, 0),                 # a group wider than one tile of heads
+    (34, 2, 80, 16, [100, 2600], [1] * 2, 0),
+    (16, 1, 256, 32, [500, 90], [1] * 2, 0),
+    (4, 2, 32, 16, [300, 200, 90, 2500], [1] * 4, 100),
+    (4, 4, 16, 16, [300, 200, 90, 1200], [1] * 4, 1000),
+    (8, 2, 128, 16, [900, 133, 400], [1, 40, 1], 5),              # decoded rows beside a portion
+])
+def test_rows_of_any_lengths(even, H, Hk, d, P_, lens, rows, window):
+    run_attention(H=H, Hk=Hk, d=d, P_=P_, lens=lens, rows_per_seg=rows, window=window, seed=H + d)
+    run_attention(H=H, Hk=Hk, d=d, P_=P_, lens=lens, rows_per_seg=rows, window=window, seed=H + d, stale=float("nan"))
+
+
+@pytest.mark.gpu
+def test_chosen_by_itself_and_the_counters_are_zero_again():
+    t = tuned()
+    run_attention(H=16, Hk=8, d=64, P_=16, lens=RAGGED[:40], rows_per_seg=[1] * 40, seed=3)
+    used = [c for have in t._counters.values() for c in have]
+    assert used and all(int(c.abs().sum()) == 0 for c in used)
+
+
+def test_the_executors_rule_is_the_wrappers_rule():
+    from allpaca_amd.kernels import host, tuned as t
+    L = host.load()
+    for pairs in (1, 64, 255, 256, 512, 4096):
+        for span in (1, 1024, 1025, 2048, 131072):
+            assert bool(L.apc_host_rule_decode_even(pairs, span, t.EVEN_MIN_PAIRS, t.EVEN_MIN_SPAN)) == t._decode_even(pairs, span)
