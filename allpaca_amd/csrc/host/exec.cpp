@@ -398,10 +398,11 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
   const int width = s.table_width[E.group];
   if (s.n_tiles) {
     const bool wide = P.tun.wide_tiles && apc_attention_prefill_wide_takes(d, page, s.n_tiles, T - s.n_decode);
-    const int splits = wide
-                           ? key_splits(s.n_tiles, H, s.max_prompt_keys, window, P.tun.key_splits_max,
-                                        std::max(1, P.tun.key_range_min))
-                           : 1;
+    const int splits = !wide ? 1
+                       : d <= 64 || (long)s.n_tiles * H > CHIP_UNITS
+                           ? key_splits_by_time(s.n_tiles, T - s.n_decode, H, d, s.prompt_passes, window, P.tun.key_splits_max)
+                           : key_splits(s.n_tiles, H, s.max_prompt_keys, window, P.tun.key_splits_max,
+                                        std::max(1, P.tun.key_range_min));
     float* parts = splits > 1 ? P.floats((size_t)splits * T * H * (d + 2)) : nullptr;
     LAUNCH(P, "attention_prefill_bf16",
            apc_attention_prefill_bf16(q.p, q.ld, 0, out.p, out.ld, H, Hk, d, E.kv, page, table, width,
@@ -712,6 +713,10 @@ APC_HOST_EXPORT const char* apc_host_timing_report(void* prog) {
 APC_HOST_EXPORT int apc_host_rule_tiled_k_split(int M, int N, int K) { return apc_rules::tiled_k_split(M, N, K); }
 APC_HOST_EXPORT int apc_host_rule_decode_parts(long long pairs, int span) {
   return apc_rules::decode_parts((long)pairs, span);
+}
+APC_HOST_EXPORT int apc_host_rule_key_splits_by_time(int n_tiles, int rows, int n_heads, int d, long long passes, int window,
+                                                     int splits_max) {
+  return apc_rules::key_splits_by_time(n_tiles, rows, n_heads, d, passes, window, splits_max);
 }
 APC_HOST_EXPORT int apc_host_rule_decode_even(long long pairs, int span, int min_pairs, int min_span) {
   return apc_rules::decode_even((long)pairs, span, min_pairs, min_span);

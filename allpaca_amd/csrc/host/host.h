@@ -70,6 +70,7 @@ struct ApcStep {
   int max_decode_context;     // largest position + 1 among the single-row segments
   int all_rows_decode;        // every row is a single-row segment (decode_rows is then not read)
   int max_prompt_keys;        // largest position + rows among the longer segments (how attention cuts their keys)
+  long long prompt_passes;    // passes of 64 keys over all tiles of 128 rows of the longer segments
 };
 
 // Rules that tests and measurements move; the defaults are the kernels' wrappers' own.

@@ -57,4 +57,23 @@ inline int key_splits(int n_tiles, int n_heads, int keys, int window, int splits
   return (int)std::max(1L, s);
 }
 
+// the same from a model of the launch's time (tuned._key_splits_by_time says what it rests on).  passes: of 64 keys, over
+// all tiles; rows: of the step
+inline int key_splits_by_time(int n_tiles, int rows, int n_heads, int d, long long passes, int window, int splits_max) {
+  const long blocks = (long)n_tiles * n_heads;
+  double mean = (double)passes / n_tiles;
+  if (window) mean = std::min(mean, (double)(cdiv(window, 64) + 2));
+  int best = 1;
+  double best_us = 1e30;
+  for (int s = 1; s <= std::max(1, splits_max); ++s) {
+    const long unit = cdiv(blocks * s, CHIP_UNITS);   // blocks of the busiest compute unit
+    const double q = mean / s;
+    double us = d <= 64 ? (unit / 2) * (6.0 + 1.15 * q) + (unit % 2) * (6.0 + 0.66 * q) : unit * (12.5 + 0.8 * q);
+    if (s > 1) us += (d <= 64 ? 5.0 : 12.0) + (double)s * rows * n_heads * (d + 2) * 8.0 / 6e6;
+    if (s == 1) best_us = 0.97 * us;                  // (cut only where it is worth something)
+    else if (us < best_us) best = s, best_us = us;
+  }
+  return best;
+}
+
 }  // namespace apc_rules

@@ -993,7 +993,7 @@ __global__ __launch_bounds__(SNT) void sample_end_kernel(const float* __restrict
 // ---- Rows that all keep at most SMALL_MAX candidates (0 < top-k <= 1,024), in two launches ----
 // The k largest of a row are among the k largest of its pieces: every block leaves its piece's (and up to FEW_SPARE more,
 // so that a coarse threshold will do), one block a row selects the row's k from those exactly, sorts them and does the
-// reference's sequential arithmetic.  A threshold is found by radix descent over the same 64-bit sort key as below, 11
+// reference's sequential arithmetic.  A threshold is found by radix descent over the same 64-bit sort key, 11
 // bits a pass, with the histogram in LDS.  What bounds it is latency: each launch is a handful of passes over values that
 // are in L2 after the first, each with two or three barriers; the descents above make five launches of it, each of which
 // begins with where the one before it left off.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 10 + 20 us (the descents:

@@ -151,6 +151,7 @@ class NativeProgram:
         s.max_decode_context = info.max_decode_context
         s.all_rows_decode = 1 if info.decode_rows is None else 0
         s.max_prompt_keys = max([p + n for p, n in zip(info.host_pos0, info.host_rows) if n > 1] or [0])
+        s.prompt_passes = tuned._prompt_passes(info.host_pos0, info.host_rows) if info.n_tiles else 0
         return s
 
     def room_for(self, s: H.ApcStep) -> torch.Tensor:

@@ -36,7 +36,8 @@ class ApcStep(Structure):
     _fields_ = ([("T", c_int), ("S", c_int), ("R", c_int), ("n_decode", c_int), ("n_tiles", c_int)]
                 + [(name, c_void_p) for name in STEP_ARRAYS]
                 + [("n_groups", c_int), ("table", c_void_p * MAX_PAGED_GROUPS), ("table_width", c_int * MAX_PAGED_GROUPS),
-                   ("max_decode_context", c_int), ("all_rows_decode", c_int), ("max_prompt_keys", c_int)])
+                   ("max_decode_context", c_int), ("all_rows_decode", c_int), ("max_prompt_keys", c_int),
+                   ("prompt_passes", c_longlong)])
 
 
 class ApcStepFinding(Structure):
@@ -75,6 +76,7 @@ _lib.SIGNATURES["host"].update({
     "apc_host_rule_decode_parts": [c_longlong, I],
     "apc_host_rule_decode_even": [c_longlong, I, I, I],
     "apc_host_rule_key_splits": [I, I, I, I, I, I],
+    "apc_host_rule_key_splits_by_time": [I, I, I, I, c_longlong, I, I],
     # ---- the cache manager's books
     "apc_pool_new": [I], "apc_pool_free": [P], "apc_pool_alloc": [P], "apc_pool_give_back": [P, I],
     "apc_pool_free_count": [P], "apc_pool_pages": [P], "apc_pool_allocations": [P],

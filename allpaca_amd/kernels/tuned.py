@@ -394,6 +394,41 @@ def _key_splits(step, n_heads: int, window: int) -> int:
     return max(1, min(KEY_SPLITS_MAX, 256 // blocks, max(keys // KEY_RANGE_MIN, few)))
 
 
+def _prompt_passes(pos0, rows) -> int:
+    """Passes of 64 keys that the 128-row attention kernel makes over the tiles of all segments of several rows."""
+    return sum((p + min(i + 128, n) - 1) // 64 + 1 for p, n in zip(pos0, rows) if n > 1 for i in range(0, n, 128))
+
+
+def _key_splits_by_time(n_tiles: int, rows: int, n_heads: int, head_dim: int, passes: int, window: int) -> int:
+    """The ranges of keys with the least time by this model (microseconds): a compute unit's blocks one after the other, a
+    block 12.5 + 0.8 a pass of 64 keys; with heads of 64, where two share a unit, two together 6 + 1.15 a pass and one by
+    itself 6 + 0.66; and for the kernel that adds the ranges 12 (heads of 64: 5) and its bytes at 6 TB/s.  It takes
+    launches of more blocks than units, whose last round may be nearly empty, and all with heads of 64: 1,500 rows over
+    24,000 keys at 32 heads of 64 (384 blocks, one and a half a unit) 459 us whole, 402, 389, 355, 367 us in 2 to 5 ranges
+    (chosen: 4); over 4,000 keys 100, 96, 105, 105 (1); 700 rows over 8,000 95, 88, 92, 79, 84 (4); 300 rows over 16,000
+    166, 94, 100, 82, 73 (5); 1,024 rows over 16,000 186, 172, 172, 173 (2); 1,500 rows over 16,000 at 24 heads of 128 (288
+    blocks) 468, 396, 379, 376, 379 (3), over 3,000 119, 127, 135 (1); 2,048 rows over 8,000 at 32 heads 309, 346 (1)."""
+    blocks = n_tiles * n_heads
+    mean = passes / n_tiles
+    if window:
+        mean = min(mean, float(-(-window // 64) + 2))
+    best, best_us = 1, 1e30
+    for s in range(1, max(1, KEY_SPLITS_MAX) + 1):
+        unit = -(-blocks * s // CHIP_UNITS)     # blocks of the busiest compute unit
+        q = mean / s
+        if head_dim <= 64:
+            us = (unit // 2) * (6.0 + 1.15 * q) + (unit % 2) * (6.0 + 0.66 * q)
+        else:
+            us = unit * (12.5 + 0.8 * q)
+        if s > 1:
+            us += (5.0 if head_dim <= 64 else 12.0) + s * rows * n_heads * (head_dim + 2) * 8.0 / 6e6
+        if s == 1:
+            best_us = 0.97 * us                 # (cut only where it is worth something)
+        elif us < best_us:
+            best, best_us = s, us
+    return best
+
+
 def _pair_counters(device: torch.device, pairs: int) -> torch.Tensor:
     """Zeroed int32 counters, one per (row, kv head tile), that live as long as the process: a call leaves them zero
     again, and a replayed graph keeps pointing at them.  Grown by allocating anew; the old ones stay (graphs).  Every
@@ -433,7 +468,13 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
     if step.n_tiles:
         # (only the kernel of 128-row blocks cuts keys into ranges: no room is taken for the others)
         wide = WIDE_TILES and L.apc_attention_prefill_wide_takes(head_dim, page_tokens, step.n_tiles, T - step.n_decode_rows)
-        splits = _key_splits(step, n_heads, window) if wide else 1
+        if not wide:
+            splits = 1
+        elif head_dim <= 64 or step.n_tiles * n_heads > CHIP_UNITS:
+            splits = _key_splits_by_time(step.n_tiles, T - step.n_decode_rows, n_heads, head_dim,
+                                         _prompt_passes(step.host_pos0, step.host_rows), int(window))
+        else:
+            splits = _key_splits(step, n_heads, window)
         parts = (torch.empty(splits * T * n_heads * (head_dim + 2), dtype=torch.float32, device=q.device)
                  if splits > 1 else None)
         _lib.check(L.apc_attention_prefill_bf16(

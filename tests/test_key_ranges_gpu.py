@@ -1,0 +1,47 @@
+"""Ranges of keys of a prompt's tiles by the time they are expected to take: what is chosen, the executor's rule beside the
+wrapper's, and the attention with every number of ranges."""
+import numpy as np
+import pytest
+import torch
+
+
+def test_chosen_ranges():
+    from allpaca_amd.kernels import tuned as t
+
+    def chosen(rows, before, heads, d, window=0):
+        tiles = -(-rows // 128)
+        return t._key_splits_by_time(tiles, rows, heads, d, t._prompt_passes([before, 9], [rows, 1]), window)
+
+    assert [chosen(1500, n, 32, 64) for n in (24001, 4000, 1000, 0)] == [4, 1, 1, 1]
+    assert (chosen(700, 8000, 32, 64), chosen(300, 16000, 32, 64), chosen(1024, 16384, 32, 64)) == (4, 5, 2)
+    assert [chosen(1500, n, 24, 128) for n in (16000, 3000, 0)] == [3, 1, 1]
+    # whole rounds of blocks stay whole; a window is what a tile sees
+    assert chosen(2048, 16384, 32, 64) == 1 and chosen(2048, 30720, 32, 128) == 1
+    assert chosen(1500, 24001, 32, 64, window=1000) == 1
+    assert t._prompt_passes([0, 100, 5], [129, 1, 2]) == 2 + 3 + 1
+
+
+def test_the_executors_rule_is_the_wrappers_rule(monkeypatch):
+    from allpaca_amd.kernels import host, tuned as t
+    L = host.load()
+    for most in (8, 3, 0):
+        monkeypatch.setattr(t, "KEY_SPLITS_MAX", most)
+        for rows in (64, 300, 700, 1024, 1500, 2048):
+            for before in (0, 900, 4000, 24001, 130000):
+                for heads, d in ((32, 64), (24, 128), (64, 128), (4, 64)):
+                    for window in (0, 1000):
+                        tiles, passes = -(-rows // 128), t._prompt_passes([before], [rows])
+                        want = t._key_splits_by_time(tiles, rows, heads, d, passes, window)
+                        assert L.apc_host_rule_key_splits_by_time(tiles, rows, heads, d, passes, window, most) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("window", [0, 200])
+def test_every_number_of_ranges(monkeypatch, d, window):
+    """Portions whose tiles see very different numbers of keys, some fewer than there are ranges."""
+    from test_kernels_tuned import run_attention, tuned
+    for s in range(1, 9):
+        monkeypatch.setattr(tuned(), "_key_splits_by_time", lambda *a, s=s: s)
+        monkeypatch.setattr(tuned(), "_key_splits", lambda *a, s=s: s)
+        run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500, 130, 77], rows_per_seg=[300, 129, 1], window=window, seed=s)
