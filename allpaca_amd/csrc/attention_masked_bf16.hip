@@ -339,13 +339,24 @@ constexpr int NW = DT / WAVE;
 // 64 keys: scores with all heads of the group as S = K Q^T (keys as the rows of 4 tiles, straight from the pages into
 // the operand), maxima and sums with a key a lane, weights to LDS in bfloat16, then O^T += V^T P^T over the 64 keys for
 // every 16 value elements (8 slots of an element a lane, straight from the pages).
+// With one range of keys a row the block writes the finished heads itself.  Short rows are bound by the chain of waits
+// from the row's position over its pages to the output: all keys and values of a pass are asked for together and four
+// heads' maxima and sums are taken side by side.  8 rows of up to 81 keys, 8 kv heads of 64 elements: 8.0 us, against
+// 12.7 with values asked for behind the scores and a head after the other, and 4.5 of a launch that added one part up.
+struct MaskedEnd {
+  void* out;
+  int ldo, out_f32, sink;
+  const float *sinks, *gate;
+  int ldg;
+  float out_scale;
+};
 template <int KS, int ET>  // 32-element steps over a key; tiles of 16 value elements
 __global__ __launch_bounds__(DT) void attn_masked_decode_kernel(
     const bf16_t* __restrict__ q, int ldq, int H, int G, int dk, int dv, const bf16_t* __restrict__ cache, int P,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ positions,
     const int* __restrict__ row_seg, const int* __restrict__ rows, int mask, int mask_size, int keep, float scale, int n_splits,
     float* __restrict__ parts, int key_parts, float softcap, const float* __restrict__ r1,
-    const float* __restrict__ r2) {
+    const float* __restrict__ r2, MaskedEnd end) {
   __shared__ __attribute__((aligned(16))) float sc_all[NW][HGMAX * SROW];
   __shared__ __attribute__((aligned(16))) bf16_t ps_all[NW][HGMAX * PROW];
   __shared__ float ml_all[NW][HGMAX][3];        // running maximum, running sum, the last pass's factor
@@ -363,6 +374,7 @@ __global__ __launch_bounds__(DT) void attn_masked_decode_kernel(
   const int* bt = block_table + (size_t)row_seg[r] * max_blocks;
   const size_t page_stride = (size_t)G * P * (dk + dv);
   const bf16_t* head = cache + (size_t)g * P * (dk + dv);
+  const int page_bits = __builtin_ctz(P);
 
   // the heads' queries as the second operand: column li = head, 8 elements from (ks * 32 + lc * 8) on
   Frag qf[KS];
@@ -375,7 +387,8 @@ __global__ __launch_bounds__(DT) void attn_masked_decode_kernel(
   }
   const bool shaped = softcap > 0.f || r1 != nullptr;
   const ScoreShape shape = score_shape(scale, softcap, r1, r2, g * per + (li < per ? li : 0), 1.0f);
-  for (int idx = lane; idx < HGMAX * PROW; idx += WAVE) ps[idx] = 0;    // rows of heads that do not exist stay 0
+  for (int idx = lane; idx < HGMAX * PROW / 8; idx += WAVE)            // rows of heads that do not exist stay 0
+    *reinterpret_cast<uint4*>(ps + idx * 8) = uint4{0, 0, 0, 0};
   if (lane < HGMAX) { ml[lane][0] = -INFINITY; ml[lane][1] = 0.f; ml[lane][2] = 1.f; }
   floatx4 o[ET];
 #pragma unroll
@@ -392,20 +405,41 @@ __global__ __launch_bounds__(DT) void attn_masked_decode_kernel(
   for (int pass = split * per_split; pass < pass_end; ++pass) {
     const int t0 = (pass < kept_passes ? pass * DT : a0 + (pass - kept_passes) * DT) + wave * WAVE;
     if (t0 > pos || (t0 + WAVE <= first && t0 >= keep)) continue;           // no key the row sees
+    // All loads of the 64 keys and values are asked for with no condition on the way, the pages first: a lane whose key
+    // the row does not see reads the row's own key again (its score is not used, and its value is taken out below).
+    const bf16_t *kp[4], *vp[2];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) {
+      const int tu = t0 + tt * 16 + li, t = (tu >= first || tu < keep) && tu <= pos ? tu : pos;
+      kp[tt] = head + (size_t)bt[t >> page_bits] * page_stride + (size_t)(t & (P - 1)) * dk;
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int tu = t0 + kk * 32 + lc * 8, tp = (tu + 8 > first || tu < keep) && tu <= pos ? tu : pos & ~7;
+      vp[kk] = head + (size_t)bt[tp >> page_bits] * page_stride + (size_t)P * dk + (tp & (P - 1));
+    }
+    Frag vf[ET][2];
+    auto ask_for_values = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < ET; ++i) {
+        const int e = min(i * 16 + li, dv - 1);   // (an element beyond the last is not written)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) vf[i][kk] = load_frag_once(vp[kk] + (size_t)e * P);
+      }
+    };
     // ---- scores of keys t0 .. t0 + 63: 4 tiles of 16 keys
     {
       Frag kf[4][KS];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
-        const int t = t0 + tt * 16 + li;
-        const bool seen = (t >= first || t < keep) && t <= pos;
-        const bf16_t* kp = head + (size_t)(seen ? bt[t / P] : 0) * page_stride + (size_t)(t % P) * dk;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           const int c = ks * 32 + lc * 8;
-          kf[tt][ks] = (seen && c < dk) ? load_frag_once(kp + c) : zero_frag();
+          kf[tt][ks] = c < dk ? load_frag_once(kp[tt] + c) : zero_frag();
         }
       }
+      // (the values beside the keys where registers allow it: nothing waits for the scores but the weights)
+      if constexpr (KS <= 4 && ET <= 8) ask_for_values();
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
         floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -423,36 +457,44 @@ __global__ __launch_bounds__(DT) void attn_masked_decode_kernel(
         *reinterpret_cast<float4*>(sc + li * SROW + tt * 16 + lc * 4) = sv;
       }
     }
-    // ---- the value pieces are asked for now: they do not wait for the weights
-    Frag vf[ET][2];
+    if constexpr (!(KS <= 4 && ET <= 8)) ask_for_values();
 #pragma unroll
-    for (int i = 0; i < ET; ++i) {
-      const int e = i * 16 + li;
+    for (int i = 0; i < ET; ++i)
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         const int tp = t0 + kk * 32 + lc * 8;
-        if (e < dv && tp <= pos && (tp + 8 > first || tp < keep)) {
-          vf[i][kk] = load_frag_once(head + (size_t)bt[tp / P] * page_stride + (size_t)P * dk + (size_t)e * P + tp % P);
-          if (tp < first || tp + 8 > pos + 1) keep_positions(vf[i][kk], first - tp, pos - tp + 1, keep - tp);
-        } else {
-          vf[i][kk] = zero_frag();
-        }
+        if (tp < first || tp + 8 > pos + 1) keep_positions(vf[i][kk], first - tp, pos - tp + 1, keep - tp);
       }
-    }
     wave_lds_order();
-    // ---- softmax, a key a lane
+    // ---- softmax, a key a lane, four heads side by side (their exchanges between lanes do not wait for each other)
     const int t = t0 + lane;
     const bool valid = (t >= first || t < keep) && t <= pos;
-    for (int j = 0; j < per; ++j) {
-      const float s = valid ? sc[j * SROW + lane] : -INFINITY;
-      const float m_old = ml[j][0], l_old = ml[j][1];
-      const float m_new = fmaxf(m_old, wave_max(s));   // finite: the 64 keys hold one the row sees
-      const float alpha = __expf(m_old - m_new);
-      const float p = valid ? __expf(s - m_new) : 0.f;
-      ps[j * PROW + lane] = float_to_bf16(p);
-      const float l_new = l_old * alpha + wave_sum(p);
+    constexpr int HS = 4;
+    for (int j0 = 0; j0 < per; j0 += HS) {
+      float s[HS], m_old[HS], l_old[HS], m_new[HS], alpha[HS], p[HS], l_new[HS];
+#pragma unroll
+      for (int u = 0; u < HS; ++u) {
+        const int j = min(j0 + u, per - 1);
+        s[u] = valid ? sc[j * SROW + lane] : -INFINITY;
+        m_old[u] = ml[j][0];
+        l_old[u] = ml[j][1];
+      }
+#pragma unroll
+      for (int u = 0; u < HS; ++u) m_new[u] = fmaxf(m_old[u], wave_max(s[u]));   // finite: the 64 keys hold one the row sees
+#pragma unroll
+      for (int u = 0; u < HS; ++u) {
+        alpha[u] = __expf(m_old[u] - m_new[u]);
+        p[u] = valid ? __expf(s[u] - m_new[u]) : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < HS; ++u) l_new[u] = l_old[u] * alpha[u] + wave_sum(p[u]);
       wave_lds_order();                           // every lane has read the old values
-      if (lane == 0) { ml[j][0] = m_new; ml[j][1] = l_new; ml[j][2] = alpha; }
+#pragma unroll
+      for (int u = 0; u < HS; ++u) {
+        if (j0 + u >= per) continue;
+        ps[(j0 + u) * PROW + lane] = float_to_bf16(p[u]);
+        if (lane == 0) { ml[j0 + u][0] = m_new[u]; ml[j0 + u][1] = l_new[u]; ml[j0 + u][2] = alpha[u]; }
+      }
     }
     wave_lds_order();
     // ---- values
@@ -493,6 +535,15 @@ __global__ __launch_bounds__(DT) void attn_masked_decode_kernel(
         const float f = m == -INFINITY ? 0.f : __expf(m - M);
         a = fmaf(f, ox[w][jj][e], a);
         l = fmaf(f, ml_all[w][j][1], l);
+      }
+      if (n_splits == 1) {                        // nothing to add: as attn_masked_merge_kernel does it with one part
+        const int h = g * per + j;
+        const float z = end.sinks ? end.sinks[h] : 0.f, top = end.sink ? fmaxf(M, z) : M;
+        const float w = M == -INFINITY ? 0.f : __expf(M - top), L = w * l + (end.sink ? __expf(z - top) : 0.f);
+        float inv = end.out_scale / L;
+        if (end.gate) inv *= 1.0f / (1.0f + __expf(-end.gate[(size_t)r * end.ldg + h]));
+        store_f(end.out, end.out_f32 ? APC_F32 : APC_BF16, (size_t)r * end.ldo + (size_t)h * dv + e, w * a * inv);
+        continue;
       }
       float* p = parts + (((size_t)ri * H + g * per + j) * n_splits + split) * (dv + 2);
       p[2 + e] = a;
@@ -617,10 +668,11 @@ APC_EXPORT int apc_attention_masked_decode_bf16(const void* q, int ldq, void* ou
       (long)n_rows * G * n_splits > 0x7fffffffL || H > 65535)
     return APC_ERR_BAD_ARG;
   dim3 grid(n_rows * G * n_splits), block(DT);
+  const MaskedEnd end{out, ldo, out_f32, sink, sinks, gate, ldg, out_scale};
 #define MD_LAUNCH(KS_, ET_)                                                                                       \
   hipLaunchKernelGGL((attn_masked_decode_kernel<KS_, ET_>), grid, block, 0, stream, (const bf16_t*)q, ldq, H, G, dk, \
                      dv, (const bf16_t*)cache, page_tokens, block_table, max_blocks, positions, row_seg, rows, mask,  \
-                     mask_size, keep, scale, n_splits, parts, key_parts, softcap, r1, r2)
+                     mask_size, keep, scale, n_splits, parts, key_parts, softcap, r1, r2, end)
 #define MD_VALUES(KS_)                     \
   do {                                     \
     if (dv <= 64) MD_LAUNCH(KS_, 4);       \
@@ -633,6 +685,7 @@ APC_EXPORT int apc_attention_masked_decode_bf16(const void* q, int ldq, void* ou
 #undef MD_VALUES
 #undef MD_LAUNCH
   APC_LAUNCH_CHECK();
+  if (n_splits == 1) return 0;
   hipLaunchKernelGGL(attn_masked_merge_kernel, dim3(n_rows, H), dim3(64), 0, stream, parts, n_splits, H, dv, rows, sink,
                      sinks, gate, ldg, out, ldo, out_f32, out_scale);
   APC_LAUNCH_CHECK();

@@ -576,6 +576,9 @@ def masked_attention_bf16(q, out, n_heads, n_kv_heads, key_dim, value_dim, cache
         keys = min(step.max_decode_context, mask_size) if code else step.max_decode_context
         # a row's first pass starts at a multiple of 256 at or below its first key; kept first keys are passes of their own
         passes = -(-(keys + 255) // 256) + -(-min(keep, step.max_decode_context) // 256)
+        # (every row sees its keys from 0 on: no such passes, and contexts up to 256 take one launch, 8 us for 17)
+        if not code or step.max_decode_context <= mask_size:
+            passes = -(-step.max_decode_context // 256)
         splits = max(1, min(passes, MASKED_DECODE_SPLITS, MASKED_DECODE_BLOCKS // max(1, n * n_kv_heads)))
         parts = torch.empty(n * n_heads * splits * (value_dim + 2), dtype=torch.float32, device=q.device)
         _lib.check(L.apc_attention_masked_decode_bf16(
