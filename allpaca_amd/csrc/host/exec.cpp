@@ -292,6 +292,12 @@ int swiglu(Program& P, const Buf& h, const ApcLayer& L, const Buf& out) {
              apc_gemm_swiglu_bf16(h.p, h.ld, L.w_gate.data, L.w_up.data, out.p, out.ld, M, F, K, P.stream));
     return 0;
   }
+  if (h.dtype == APC_DT_F32 && out.dtype == APC_DT_F32 && L.w_gate.dtype == APC_DT_F32 && L.w_gate.K == K &&
+      L.w_gate.N == 2 * F && out.rows == M && apc_swiglu_f32_takes(h.p, h.ld, L.w_gate.data, L.w_gate.ld, F, K)) {
+    LAUNCH(P, "swiglu_f32",
+           apc_swiglu_f32(h.p, h.ld, L.w_gate.data, L.w_gate.ld, out.p, out.ld, M, F, K, P.stream));
+    return 0;
+  }
   Buf gu = P.rows(M, 2 * F, h.dtype == APC_DT_F32 ? APC_DT_F32 : out.dtype);
   int rc = gemm_plain(P, h, L.w_gate, gu, false);
   if (rc) return rc;

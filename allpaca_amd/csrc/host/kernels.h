@@ -17,6 +17,9 @@ int apc_silu_mul(const void* gu, int in_dtype, int ldg, void* out, int out_dtype
 int apc_rope_kv_write(void* qkv, int dtype, int ld, int q_off, int k_off, int v_off, int n_tok, int H, int Hk, int d,
                       int rot, const float* cos_sin, const int* positions, const int* row_seg, const int* block_table,
                       int max_blocks, void* cache, int cache_dtype, int page_tokens, hipStream_t stream);
+int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int ldw, int F, int K);
+int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, void* out, int ldo, int M, int F, int K,
+                   hipStream_t stream);
 int apc_gemm_plain(const void* A, int a_dtype, int lda, const void* W, int w_dtype, int ldw, void* C, int c_dtype,
                    int ldc, int M, int N, int K, int mode, hipStream_t stream);
 int apc_paged_attention_plain(const void* q, int q_dtype, int ldq, int q_off, void* out, int out_dtype, int ldo,

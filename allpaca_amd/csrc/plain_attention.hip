@@ -1,5 +1,6 @@
-// Plain attention over the paged cache: one wave per (query row, head), keys in
-// order in chunks of 64 anchored at key 0, online softmax in float32.
+// Plain attention over the paged cache.  This first kernel takes any types and sizes: one wave per (query row, head),
+// keys in order in chunks of 64 anchored at key 0, online softmax in float32.  (float32 queries and pages in pieces of
+// 16 bytes: paged_attention_f32_kernel below, which adds in another fixed order.)
 //
 // For the row at position `pos` of its request:  keys t in [first, pos],
 // first = 0 or pos - window + 1;  s_t = (q . K[t]) * scale;  m = max s;

@@ -33,6 +33,8 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
         "apc_rope_kv_write": [P, I, I, I, I, I, I, I, I, I, I, P, P, P, P, I, P, I, I, P],
         "apc_cast": [P, I, P, I, Z, P],
         "apc_gemm_plain": [P, I, I, P, I, I, P, I, I, I, I, I, I, P],
+        "apc_swiglu_f32_takes": [P, I, P, I, I, I],
+        "apc_swiglu_f32": [P, I, P, I, P, I, I, I, I, P],
         "apc_paged_attention_plain": [P, I, I, I, P, I, I, I, I, I, I, P, I, I, P, I, P, P, I, F, P],
         "apc_conv_heads": [P, I, I, I, I, I, I, I, I, I, I, I, P, P, I, P, I, P, P, P, P, P, I, F, I, P, P, I, F, I, P, I, I, P, I, P, I, I, P],
         "apc_conv_state": [P, I, I, P, I, P, I, I, P, P, P, P],

@@ -301,9 +301,25 @@ def swiglu(h: torch.Tensor, w_gate_up, out: torch.Tensor) -> None:
         tuned.swiglu_bf16(h, w_gate_up[0], w_gate_up[1], out)
         return
     T, F = out.shape
+    if h.dtype == out.dtype == w_gate_up.dtype == torch.float32 and _swiglu_f32(h, w_gate_up, out):
+        return
     gu = torch.empty((T, 2 * F), dtype=torch.float32 if h.dtype == torch.float32 else out.dtype, device=h.device)
     gemm_plain(h, w_gate_up, gu)
     silu_mul(gu, out)
+
+
+def _swiglu_f32(h: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """Both products and the activation in one float32 kernel; False (nothing done) for rows it does not take."""
+    _gpu(h, w, out)
+    ldh, ldw, ldo = _rows(h, "swiglu h"), _rows(w, "swiglu w"), _rows(out, "swiglu out")
+    T, F = out.shape
+    L = _lib.load("plain")
+    if (h.shape[0] != T or w.shape != (2 * F, h.shape[1])
+            or not L.apc_swiglu_f32_takes(h.data_ptr(), ldh, w.data_ptr(), ldw, F, h.shape[1])):
+        return False
+    _lib.check(L.apc_swiglu_f32(h.data_ptr(), ldh, w.data_ptr(), ldw, out.data_ptr(), ldo, T, F, h.shape[1], _stream()),
+               "swiglu_f32")
+    return True
 
 
 def linear_pre(raw: torch.Tensor, ss: torch.Tensor, eps: float, w, out: torch.Tensor) -> bool:
