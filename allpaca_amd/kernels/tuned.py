@@ -396,7 +396,7 @@ def _key_splits(step, n_heads: int, window: int) -> int:
 
 def _prompt_passes(pos0, rows) -> int:
     """Passes of 64 keys that the 128-row attention kernel makes over the tiles of all segments of several rows."""
-    return sum((p + min(i + 128, n) - 1) // 64 + 1 for p, n in zip(pos0, rows) if n > 1 for i in range(0, n, 128))
+    return sum((p + min(i + 128, n) - 1) // 64 + 1 for p, n in zip(pos0 or (), rows or ()) if n > 1 for i in range(0, n, 128))
 
 
 def _key_splits_by_time(n_tiles: int, rows: int, n_heads: int, head_dim: int, passes: int, window: int) -> int:
@@ -432,12 +432,22 @@ def _key_splits_by_time(n_tiles: int, rows: int, n_heads: int, head_dim: int, pa
 def _pair_counters(device: torch.device, pairs: int) -> torch.Tensor:
     """Zeroed int32 counters, one per (row, kv head tile), that live as long as the process: a call leaves them zero
     again, and a replayed graph keeps pointing at them.  Grown by allocating anew; the old ones stay (graphs).  Every
-    stream has its own: launches that share them must not overlap."""
-    key = (device.type, device.index if device.index is not None else torch.cuda.current_device(), _ops._stream())
-    have = _counters.setdefault(key, [])
-    if not have or have[-1].numel() < pairs:
-        have.append(torch.zeros(max(1024, pairs), dtype=torch.int32, device=device))
-    return have[-1]
+    stream has its own: launches that share them must not overlap.  The graphs recorded on a device share one set, made
+    by the calls outside of recordings (an allocation while recording would be cleared by that one graph alone); where
+    that is too small yet, a recording clears counters of its own at every replay."""
+    where = (device.type, device.index if device.index is not None else torch.cuda.current_device())
+
+    def kept(who):
+        have = _counters.setdefault(where + (who,), [])
+        if not have or have[-1].numel() < pairs:
+            have.append(torch.zeros(max(1024, pairs), dtype=torch.int32, device=device))
+        return have[-1]
+
+    if torch.cuda.is_current_stream_capturing():
+        have = _counters.get(where + ("graphs",))
+        return have[-1] if have and have[-1].numel() >= pairs else torch.zeros(pairs, dtype=torch.int32, device=device)
+    kept("graphs")
+    return kept(_ops._stream())
 
 
 def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int,
@@ -472,7 +482,8 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
             splits = 1
         elif head_dim <= 64 or step.n_tiles * n_heads > CHIP_UNITS:
             splits = _key_splits_by_time(step.n_tiles, T - step.n_decode_rows, n_heads, head_dim,
-                                         _prompt_passes(step.host_pos0, step.host_rows), int(window))
+                                         _prompt_passes(getattr(step, "host_pos0", None), getattr(step, "host_rows", None)),
+                                         int(window))
         else:
             splits = _key_splits(step, n_heads, window)
         parts = (torch.empty(splits * T * n_heads * (head_dim + 2), dtype=torch.float32, device=q.device)

@@ -49,3 +49,32 @@ def test_the_executors_rule_is_the_wrappers_rule():
     for pairs in (1, 64, 255, 256, 512, 4096):
         for span in (1, 1024, 1025, 2048, 131072):
             assert bool(L.apc_host_rule_decode_even(pairs, span, t.EVEN_MIN_PAIRS, t.EVEN_MIN_SPAN)) == t._decode_even(pairs, span)
+
+
+def test_counters_are_never_first_made_while_a_graph_records(monkeypatch):
+    """A buffer that a recording allocates is cleared by that graph's replays alone: it must not be kept for others."""
+    from allpaca_amd.kernels import tuned as t
+    stream, recording = [1], [False]
+    monkeypatch.setattr(t, "_counters", {})
+    monkeypatch.setattr(t._ops, "_stream", lambda: stream[0])
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: recording[0])
+    cpu = torch.device("cpu")
+    kept = lambda: {c.data_ptr() for have in t._counters.values() for c in have}
+    recording[0] = True
+    assert t._pair_counters(cpu, 8).data_ptr() not in kept()             # nothing was made before: its own
+    stream[0], recording[0] = 2, False
+    eager = t._pair_counters(cpu, 8)
+    before = kept()
+    stream[0], recording[0] = 3, True
+    of_graph = t._pair_counters(cpu, 8)
+    assert kept() == before and of_graph.data_ptr() in before and of_graph.data_ptr() != eager.data_ptr()
+    assert t._pair_counters(cpu, 5000).numel() >= 5000 and kept() == before
+    stream[0], recording[0] = 4, False
+    assert t._pair_counters(cpu, 8).data_ptr() not in (eager.data_ptr(), of_graph.data_ptr())
+
+
+def test_a_step_that_does_not_say_where_its_prompts_start_is_not_cut():
+    from allpaca_amd.kernels import tuned as t
+    assert t._prompt_passes(None, None) == 0
+    assert t._key_splits_by_time(12, 1500, 32, 64, 0, 0) == 1
