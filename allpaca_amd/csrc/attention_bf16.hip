@@ -626,6 +626,18 @@ __device__ __forceinline__ int wave_scan_int(int v) {  // the sum of this lane's
 // EVEN_BLOCKS: a block a compute unit (two, where registers allow them, were slower: 64 ragged rows 37 -> 48 us, more
 // pieces and as many bytes in flight).  EVEN_BATCH: pieces of a row that the last wave asks for together.
 constexpr int EVEN_ROW_COST = 2, EVEN_MIN_SHARE = 8, EVEN_BLOCKS = 256, EVEN_BATCH = 4;
+// Where the pieces of kv head tile `tile` lie in the workspace, in floats: a region for every tile, two places a wave.
+// All regions have the room of a full tile: blocks of all tiles run side by side, and the last tile of a group may have
+// fewer heads than the others.
+struct EvenRoom {
+  int tile_heads, stride;  // heads of the tile; a head of a piece: its sums, maximum, sum, room
+  long long first, end;
+};
+__host__ __device__ inline EvenRoom even_room(int G, int d, int waves, int tile) {
+  const int left = G - tile % ((G + 15) / 16) * 16, heads = left < 16 ? left : 16;
+  const long long place = (long long)waves * 2 * (d + 4), first = tile * place * (G < 16 ? G : 16);
+  return {heads, d + 4, first, first + place * heads};
+}
 template <int DP, int MODE>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
     const bf16_t* __restrict__ q, int ldq, int q_off, int H, int Hk, int d, const bf16_t* __restrict__ cache, int P,
@@ -823,8 +835,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
     }
     const int share = max(EVEN_MIN_SHARE, (total + waves - 1) / waves);
     const int lo = me * share, hi = min(lo + share, total);
-    const int tile_heads = min(G - gt * 16, 16), stride = d + 4;     // (a piece of a head: its sums, maximum, sum, room)
-    const BufferRsrc pieces = make_rsrc(parts + (size_t)blockIdx.y * waves * 2 * tile_heads * stride);
+    const EvenRoom room = even_room(G, d, waves, blockIdx.y);
+    const int tile_heads = room.tile_heads, stride = room.stride;
+    const BufferRsrc pieces = make_rsrc(parts + room.first);
     for (int i0 = 0;;) {
       const int start_l = end_l - cost_l;
       unsigned long long todo = __ballot(cost_l > 0 && end_l > lo && start_l < hi);
@@ -1275,7 +1288,15 @@ static int even_blocks(int H, int Hk) {
 APC_EXPORT int apc_attention_decode_even_workspace(int H, int Hk, int d) {
   if (H <= 0 || Hk <= 0 || H % Hk || d <= 0 || d > 256 || d % 16) return 0;
   const int G = H / Hk, tiles = Hk * ((G + 15) / 16);
-  return tiles * even_blocks(H, Hk) * NW * 2 * (G < 16 ? G : 16) * (d + 4);
+  return (int)even_room(G, d, even_blocks(H, Hk) * NW, tiles).first;
+}
+// The floats of it that the blocks of a kv head tile use: [first, end).
+APC_EXPORT int apc_attention_decode_even_region(int H, int Hk, int d, int tile, long long* first, long long* end) {
+  if (apc_attention_decode_even_workspace(H, Hk, d) <= 0 || tile < 0 || tile >= Hk * ((H / Hk + 15) / 16)) return APC_ERR_BAD_ARG;
+  const EvenRoom room = even_room(H / Hk, d, even_blocks(H, Hk) * NW, tile);
+  *first = room.first;
+  *end = room.end;
+  return 0;
 }
 // Decoded rows of any lengths, the work of all rows dealt out evenly (see DEC_EVEN).  workspace: as many
 // floats as apc_attention_decode_even_workspace says; counters: n_rows * Hk * ceil(H / Hk / 16) ints, zero before the

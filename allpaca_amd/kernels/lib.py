@@ -119,6 +119,7 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
                                   P, I, I, P, P, F, P],
         "apc_attention_decode_even_bf16": [P, I, I, P, I, I, I, I, I, P, I, P, I, P, P, P, I, F, P, P, P],
         "apc_attention_decode_even_workspace": [I, I, I],
+        "apc_attention_decode_even_region": [I, I, I, I, P, P],
         "apc_attention_decode_last_fits": [I, I, I, I],
         "apc_attention_decode_whole_fits": [I, I, I],
         "apc_attention_prefill_tile_rows": [],
@@ -166,7 +167,7 @@ class KernelTimer:
 _timer = None
 # entry points that launch nothing (questions about sizes): never timed
 NOT_KERNELS = {"apc_delta_rule_bf16_takes", "apc_delta_rule_fact_size", "apc_delta_rule_coef_size",
-               "apc_gated_recurrence_bf16_takes", "apc_latent_attention_takes", "apc_latent_rows_bf16_takes", "apc_selective_scan_bf16_takes", "apc_attention_masked_takes", "apc_rotary_pages_bf16_takes", "apc_routed_bf16_takes", "apc_routed_max_tiles", "apc_linear_attention_bf16_takes", "apc_conv_heads_bf16_takes", "apc_attention_decode_whole_fits", "apc_attention_decode_last_fits", "apc_attention_decode_even_workspace", "apc_attention_prefill_tile_rows",
+               "apc_gated_recurrence_bf16_takes", "apc_latent_attention_takes", "apc_latent_rows_bf16_takes", "apc_selective_scan_bf16_takes", "apc_attention_masked_takes", "apc_rotary_pages_bf16_takes", "apc_routed_bf16_takes", "apc_routed_max_tiles", "apc_linear_attention_bf16_takes", "apc_conv_heads_bf16_takes", "apc_attention_decode_whole_fits", "apc_attention_decode_last_fits", "apc_attention_decode_even_workspace", "apc_attention_decode_even_region", "apc_attention_prefill_tile_rows",
                "apc_attention_prefill_wide_takes",
                "apc_gemm_direct_k_split", "apc_gemm_direct_emit_parts", "apc_sample_rows_scratch_kib"}
 

@@ -1,6 +1,8 @@
 """Decoded rows whose work is dealt out evenly over all waves of the launch, against the plain attention: rows inside one
 wave's share, rows in two and in many pieces, shares that end at a row's first and last step, more than 64 rows, groups
 wider than a tile of 16 heads, windows, pages of 8, and slots that hold NaN."""
+import ctypes
+
 import pytest
 import torch
 
@@ -33,6 +35,36 @@ def even(monkeypatch):
 def test_rows_of_any_lengths(even, H, Hk, d, P_, lens, rows, window):
     run_attention(H=H, Hk=Hk, d=d, P_=P_, lens=lens, rows_per_seg=rows, window=window, seed=H + d)
     run_attention(H=H, Hk=Hk, d=d, P_=P_, lens=lens, rows_per_seg=rows, window=window, seed=H + d, stale=float("nan"))
+
+
+@pytest.mark.parametrize("H,Hk,d", [(20, 1, 32), (24, 1, 64), (34, 2, 80), (48, 2, 128), (71, 1, 256), (32, 8, 128),
+                                    (32, 32, 64), (16, 1, 16), (64, 2, 128)])
+def test_the_tiles_pieces_lie_apart(H, Hk, d):
+    """The places of all kv head tiles, also of a group's last one with fewer than 16 heads, in the workspace and apart."""
+    from allpaca_amd.kernels import lib
+    L = lib.load("tuned")
+    tiles, at = Hk * -(-(H // Hk) // 16), 0
+    for tile in range(tiles):
+        first, end = ctypes.c_longlong(), ctypes.c_longlong()
+        assert L.apc_attention_decode_even_region(H, Hk, d, tile, ctypes.byref(first), ctypes.byref(end)) == 0
+        heads = min(16, H // Hk - tile % (tiles // Hk) * 16)
+        waves = max(1, 256 // tiles) * 4
+        assert first.value >= at and end.value - first.value == waves * 2 * heads * (d + 4)
+        at = end.value
+    assert at <= L.apc_attention_decode_even_workspace(H, Hk, d)
+    assert L.apc_attention_decode_even_region(H, Hk, d, tiles, ctypes.byref(first), ctypes.byref(end)) < 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Hk,d,n", [(20, 1, 32, 128), (34, 2, 64, 64), (24, 1, 128, 128)])
+def test_wide_groups_with_work_for_nearly_all_waves(H, Hk, d, n):
+    """Groups of several tiles of heads, the last one short, in the rule's own range: pieces of every tile in most places."""
+    t = tuned()
+    lens = [1100 + (i * 977) % 400 for i in range(n)]
+    assert t._decode_even(n * Hk * -(-(H // Hk) // 16), max(lens))
+    waves, steps = 4 * (256 // (Hk * -(-(H // Hk) // 16))), sum(-(-x // 32) + 2 for x in lens)
+    assert steps / max(8, -(-steps // waves)) > 0.9 * waves          # (a wave's share, 8 at least)
+    run_attention(H=H, Hk=Hk, d=d, P_=16, lens=lens, rows_per_seg=[1] * n, seed=n)
 
 
 @pytest.mark.gpu
