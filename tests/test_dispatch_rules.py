@@ -71,6 +71,14 @@ def test_what_the_sampler_tells_the_kernels(monkeypatch, rules, want):
     assert (seen["any_top_k"], seen["any_top_p"], seen["few_after_top_k"]) == want
 
 
+def test_entry_points_that_launch_nothing_are_not_timed_as_kernels():
+    """A kernel's last argument is its stream; what has none answers a question about sizes."""
+    from allpaca_amd.kernels import lib
+    asked = {n for group, entries in lib.SIGNATURES.items() if group != "host"
+             for n, args in entries.items() if not args or args[-1] is not lib.P}
+    assert "apc_swiglu_f32_takes" in asked and asked <= lib.NOT_KERNELS
+
+
 def test_ranges_the_decode_attention_cuts_a_rows_keys_into():
     """Four ranges a block, as many blocks a (row, kv head) pair as keep the launch within the chip's compute units,
     and no range under 64 keys."""
