@@ -66,6 +66,8 @@ class StepInfo:
     tile_row0: Optional[torch.Tensor] = None     # int32 [n_tiles]
     tile_rows: Optional[torch.Tensor] = None     # int32 [n_tiles]
     n_tiles: int = 0
+    # counters of the decode attention that belong to the engine of a step that is recorded (see tuned._pair_counters)
+    pair_counters: Optional[list] = None
 
 
 # the arrays of the buffer, in order; block tables follow, one per paged group

@@ -61,6 +61,7 @@ class ModelRunner:
         self.tile_rows = ops.attention_tile_rows(self.rt.dtype)          # how the attention kernel wants longer segments cut
         self.position_axes = int(getattr(model.spec, "position_axes", 1))
         self.graphs: Dict[Tuple[int, int], "DecodeGraph"] = {}
+        self.pair_counters: list = []       # of the decode attention in its graphs (made when one is first recorded)
         self.graph_replays = 0
         self.steps = 0
         # The C++ side of a step (csrc/host/pack.cpp): entries checked against the cache's books, pages taken, the
@@ -394,6 +395,7 @@ class DecodeGraph:
             lay.part(self.np, name)[:] = value
         self.info = lay.info(self.dev, list(range(rows)), [1] * rows, [0] * rows, [0] * rows, span, True)
         self.info.max_context = span
+        self.info.pair_counters = runner.pair_counters
         self.copied = torch.cuda.Event()
         # what the pinned block tables hold: the request of every row and how many of its pages (per group), so that
         # a step writes only what is new (`CacheManager.table_version` changes when pages were taken away)

@@ -429,25 +429,23 @@ def _key_splits_by_time(n_tiles: int, rows: int, n_heads: int, head_dim: int, pa
     return best
 
 
-def _pair_counters(device: torch.device, pairs: int) -> torch.Tensor:
-    """Zeroed int32 counters, one per (row, kv head tile), that live as long as the process: a call leaves them zero
-    again, and a replayed graph keeps pointing at them.  Grown by allocating anew; the old ones stay (graphs).  Every
-    stream has its own: launches that share them must not overlap.  The graphs recorded on a device share one set, made
-    by the calls outside of recordings (an allocation while recording would be cleared by that one graph alone); where
-    that is too small yet, a recording clears counters of its own at every replay."""
-    where = (device.type, device.index if device.index is not None else torch.cuda.current_device())
-
-    def kept(who):
-        have = _counters.setdefault(where + (who,), [])
-        if not have or have[-1].numel() < pairs:
-            have.append(torch.zeros(max(1024, pairs), dtype=torch.int32, device=device))
-        return have[-1]
-
-    if torch.cuda.is_current_stream_capturing():
-        have = _counters.get(where + ("graphs",))
-        return have[-1] if have and have[-1].numel() >= pairs else torch.zeros(pairs, dtype=torch.int32, device=device)
-    kept("graphs")
-    return kept(_ops._stream())
+def _pair_counters(device: torch.device, pairs: int, own: Optional[list] = None) -> torch.Tensor:
+    """Zeroed int32 counters, one per (row, kv head tile): a call leaves them zero again, so launches that share them must
+    not overlap.  `own`: the list of an engine that records its steps (`StepInfo.pair_counters`); its steps never overlap,
+    and a replayed graph keeps pointing at what its recording found there.  Without it every stream has a set that lives
+    as long as the process.  Grown by allocating anew; the old ones stay (graphs).  A recording that finds none large
+    enough takes counters of its own, which every replay clears: what is allocated while recording is cleared by that one
+    graph alone, and must not be kept for others."""
+    recording = torch.cuda.is_current_stream_capturing()
+    if own is None and not recording:
+        own = _counters.setdefault((device.type, device.index if device.index is not None else torch.cuda.current_device(),
+                                    _ops._stream()), [])
+    if own and own[-1].numel() >= pairs:
+        return own[-1]
+    if recording:
+        return torch.zeros(pairs, dtype=torch.int32, device=device)
+    own.append(torch.zeros(max(1024, pairs), dtype=torch.int32, device=device))
+    return own[-1]
 
 
 def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int,
@@ -499,6 +497,7 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
         span = min(step.max_decode_context, window) if window else step.max_decode_context
         rows = step.decode_rows.data_ptr() if step.decode_rows is not None else 0
         pairs = n * n_kv_heads * -(-(n_heads // n_kv_heads) // 16)
+        counters = lambda: _pair_counters(q.device, pairs, getattr(step, "pair_counters", None))  # noqa: E731
         n_parts = -(-step.max_decode_context // KEYS_PER_PART) if KEYS_PER_PART else _decode_parts(pairs, span)
         if _decode_even(pairs, span) and not KEYS_PER_PART and ldo % 4 == 0 and out.data_ptr() % 8 == 0:
             ws = torch.empty(L.apc_attention_decode_even_workspace(n_heads, n_kv_heads, head_dim), dtype=torch.float32,
@@ -507,7 +506,7 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
                 q.data_ptr(), ldq, q_off, out.data_ptr(), ldo, n, n_heads, n_kv_heads, head_dim, cache.data_ptr(),
                 page_tokens, block_table.data_ptr(), block_table.shape[1], step.positions.data_ptr(),
                 step.row_seg.data_ptr(), rows, int(window), sc, ws.data_ptr(),
-                _pair_counters(q.device, pairs).data_ptr(), stream), "attention_decode_bf16 (even shares)")
+                counters().data_ptr(), stream), "attention_decode_bf16 (even shares)")
             return True
         # (rows so short that one block's waves take a pair's ranges need no partial results either)
         if ((pairs >= WHOLE_MIN_PAIRS or n_parts <= WHOLE_WAVES)
@@ -526,7 +525,7 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
                 q.data_ptr(), ldq, q_off, out.data_ptr(), ldo, n, n_heads, n_kv_heads, head_dim, cache.data_ptr(),
                 page_tokens, block_table.data_ptr(), block_table.shape[1], step.positions.data_ptr(),
                 step.row_seg.data_ptr(), rows, int(window), sc, kw, n_parts, ws.data_ptr(),
-                _pair_counters(q.device, pairs).data_ptr(), stream), "attention_decode_bf16 (last block merges)")
+                counters().data_ptr(), stream), "attention_decode_bf16 (last block merges)")
             return True
         ws = torch.empty(n * n_heads * n_parts * (head_dim + 2), dtype=torch.float32, device=q.device)
         _lib.check(L.apc_attention_decode_bf16(

@@ -83,8 +83,9 @@ def test_the_executors_rule_is_the_wrappers_rule():
             assert bool(L.apc_host_rule_decode_even(pairs, span, t.EVEN_MIN_PAIRS, t.EVEN_MIN_SPAN)) == t._decode_even(pairs, span)
 
 
-def test_counters_are_never_first_made_while_a_graph_records(monkeypatch):
-    """A buffer that a recording allocates is cleared by that graph's replays alone: it must not be kept for others."""
+def test_recordings_share_counters_within_an_engine_only(monkeypatch):
+    """Graphs of two engines may be replayed side by side on two streams, and calls outside of graphs on a third.  A buffer
+    that a recording allocates is cleared by that graph's replays alone: it must not be kept for others."""
     from allpaca_amd.kernels import tuned as t
     stream, recording = [1], [False]
     monkeypatch.setattr(t, "_counters", {})
@@ -92,18 +93,23 @@ def test_counters_are_never_first_made_while_a_graph_records(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: recording[0])
     cpu = torch.device("cpu")
-    kept = lambda: {c.data_ptr() for have in t._counters.values() for c in have}
+    one, two = [], []
     recording[0] = True
-    assert t._pair_counters(cpu, 8).data_ptr() not in kept()             # nothing was made before: its own
-    stream[0], recording[0] = 2, False
+    assert t._pair_counters(cpu, 8, one).numel() >= 8 and not one        # nothing was made before: the recording's own
+    assert t._pair_counters(cpu, 8).numel() >= 8 and not t._counters
+    recording[0] = False
+    first, other = t._pair_counters(cpu, 8, one), t._pair_counters(cpu, 8, two)
     eager = t._pair_counters(cpu, 8)
-    before = kept()
-    stream[0], recording[0] = 3, True
-    of_graph = t._pair_counters(cpu, 8)
-    assert kept() == before and of_graph.data_ptr() in before and of_graph.data_ptr() != eager.data_ptr()
-    assert t._pair_counters(cpu, 5000).numel() >= 5000 and kept() == before
-    stream[0], recording[0] = 4, False
-    assert t._pair_counters(cpu, 8).data_ptr() not in (eager.data_ptr(), of_graph.data_ptr())
+    stream[0] = 2
+    places = [x.data_ptr() for x in (first, other, eager, t._pair_counters(cpu, 8))]
+    assert len(set(places)) == 4 and t._pair_counters(cpu, 8, one) is first
+    recording[0], stream[0] = True, 3
+    assert t._pair_counters(cpu, 8, one) is first and t._pair_counters(cpu, 8, two) is other
+    alone = t._pair_counters(cpu, 8)                                     # a caller's own graph
+    assert alone.data_ptr() not in places and (cpu.type, 0, 3) not in t._counters
+    assert t._pair_counters(cpu, 5000, one).numel() >= 5000 and len(one) == 1
+    recording[0] = False
+    assert t._pair_counters(cpu, 5000, one).numel() >= 5000 and one[0] is first
 
 
 def test_a_step_that_does_not_say_where_its_prompts_start_is_not_cut():
