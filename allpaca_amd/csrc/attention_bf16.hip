@@ -562,8 +562,12 @@ struct KVRegs {
 //             equal shares to the waves of one round of blocks; every wave finds its share and the rows it falls into
 //             from the rows' positions, so a recorded graph fits whatever lengths they reach.  A row inside one share is
 //             finished by its wave; the pieces of a row that lies in several go through memory as in DEC_LAST, and the
-//             wave that leaves the last of them adds them in order.  37 us there, and no slower where rows are equal
-//             (64 rows of 2,048: 90 and 88 us).  What is left over the bytes is a wave's chain of rows: about 4 us each.
+//             wave that leaves the last of them adds them in order.  37 us there.  What is left over the bytes is a
+//             wave's chain of rows, about 4 us each, and the way of the pieces through memory, so rows of about one
+//             length are better off with DEC_WHOLE (32 rows of 1,100 keys on 8 kv heads of 128: 26.1 and 31.8 us): the
+//             caller chooses by the lengths.  Choosing inside the kernel was slower both ways: the registers of either
+//             path cost the other a wave a SIMD at heads of 64 (96 rows 53.8 -> 61.8 us), and a look at all rows
+//             1 to 4 us.
 // The order of additions for a row depends on its position, KW and the number of parts only (DEC_EVEN: on the lengths of
 // the rows in front of it too).
 constexpr int NW = 4;  // waves of a block of the decode kernel

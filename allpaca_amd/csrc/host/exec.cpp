@@ -422,8 +422,10 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
     const int* rows = s.all_rows_decode ? nullptr : s.decode_rows;
     const long pairs = (long)n * Hk * cdiv(H / Hk, 16);
     const int n_parts = decode_parts(pairs, span);
-    if (decode_even(pairs, span, P.tun.even_min_pairs, P.tun.even_min_span) && pairs <= P.pair_capacity && out.ld % 4 == 0 &&
-        ((uintptr_t)out.p & 7u) == 0) {
+    const bool pair_fits = apc_attention_decode_whole_fits(H, Hk, d);
+    if (decode_even(pairs, span, pair_fits, P.tun.even_min_pairs, P.tun.even_min_span) &&
+        (!pair_fits || even_pays(s.decode_steps, s.decode_longest, n, (int)(pairs / n), window)) && pairs <= P.pair_capacity &&
+        out.ld % 4 == 0 && ((uintptr_t)out.p & 7u) == 0) {
       float* ws = P.floats((size_t)apc_attention_decode_even_workspace(H, Hk, d));
       LAUNCH(P, "attention_decode_bf16 (even shares)",
              apc_attention_decode_even_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width, s.positions,
@@ -431,7 +433,7 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
       return 1;
     }
     // (rows so short that one block's waves take a pair's ranges need no partial results either)
-    if ((pairs >= P.tun.whole_min_pairs || n_parts <= WHOLE_WAVES) && apc_attention_decode_whole_fits(H, Hk, d)) {
+    if ((pairs >= P.tun.whole_min_pairs || n_parts <= WHOLE_WAVES) && pair_fits) {
       // no length of the ranges: every row's own keys, one range a wave of its block
       LAUNCH(P, "attention_decode_bf16 (whole)",
              apc_attention_decode_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width,
@@ -724,8 +726,11 @@ APC_HOST_EXPORT int apc_host_rule_key_splits_by_time(int n_tiles, int rows, int 
                                                      int splits_max) {
   return apc_rules::key_splits_by_time(n_tiles, rows, n_heads, d, passes, window, splits_max);
 }
-APC_HOST_EXPORT int apc_host_rule_decode_even(long long pairs, int span, int min_pairs, int min_span) {
-  return apc_rules::decode_even((long)pairs, span, min_pairs, min_span);
+APC_HOST_EXPORT int apc_host_rule_even_pays(long long steps, int longest, int n_rows, int tiles, int window) {
+  return apc_rules::even_pays(steps, longest, n_rows, tiles, window);
+}
+APC_HOST_EXPORT int apc_host_rule_decode_even(long long pairs, int span, int pair_fits, int min_pairs, int min_span) {
+  return apc_rules::decode_even((long)pairs, span, pair_fits != 0, min_pairs, min_span);
 }
 APC_HOST_EXPORT int apc_host_rule_key_splits(int n_tiles, int n_heads, int keys, int window, int splits_max,
                                              int range_min) {

@@ -70,6 +70,9 @@ struct ApcStep {
   int max_decode_context;     // largest position + 1 among the single-row segments
   int all_rows_decode;        // every row is a single-row segment (decode_rows is then not read)
   int max_prompt_keys;        // largest position + rows among the longer segments (how attention cuts their keys)
+  // the single-row segments' keys in steps of 32: over all of them, and of the longest one (0: not known)
+  long long decode_steps;
+  int decode_longest;
   long long prompt_passes;    // passes of 64 keys over all tiles of 128 rows of the longer segments
 };
 

@@ -43,9 +43,27 @@ inline int decode_parts(long pairs, int span) {
   return (int)std::max(1L, std::min((long)WHOLE_WAVES * per_pair, cdiv(span, 64)));
 }
 
-// whether a decode step's rows share out their work over all waves (rows of very different lengths): enough pairs that
-// no pair would be cut for its own sake, and a longest row that could be far longer than the others
-inline bool decode_even(long pairs, int span, int min_pairs, int min_span) { return pairs >= min_pairs && span > min_span; }
+// whether a decode step's rows go to the kernel that may share out their work over all waves: enough pairs that no pair
+// would be cut for its own sake (where a block has no room for a pair of its own: so many that shares are sure to pay), no
+// more than there are counters for, and a longest row that could be far longer than the others
+constexpr int EVEN_MAX_PAIRS = 4096, EVEN_ALONE_MIN_PAIRS = 1024;
+inline bool decode_even(long pairs, int span, bool pair_fits, int min_pairs, int min_span) {
+  return pairs >= (pair_fits ? min_pairs : std::max(min_pairs, EVEN_ALONE_MIN_PAIRS)) && pairs <= EVEN_MAX_PAIRS && span > min_span;
+}
+
+// Whether shares beat a block a pair for the lengths at hand (tuned._even_pays says what it rests on).  steps: of 32 keys,
+// over all rows; longest: of the longest row
+inline bool even_pays(long long steps, int longest, int n_rows, int tiles, int window) {
+  if (window) {
+    const int most = window / 32 + 1;
+    longest = std::min(longest, most);
+    steps = std::min(steps, (long long)n_rows * most);
+  }
+  const int waves = std::max(1, CHIP_UNITS / tiles) * WHOLE_WAVES;
+  const double units = (double)n_rows * WHOLE_WAVES / waves, share = (double)(steps + 2LL * n_rows) / waves;
+  const double whole = std::max(1.03 * share + 2.5 + 1.1 * units, 4.1 + 0.245 * longest * std::min(std::ceil(units), 2.8));
+  return 7.3 + std::max(share, 8.3) + 0.05 * (n_rows / 64.0) < whole;
+}
 
 // ranges of keys that the 128-row attention kernel cuts every tile of a step into; `keys`: of the longest prompt
 inline int key_splits(int n_tiles, int n_heads, int keys, int window, int splits_max, int range_min) {

@@ -66,6 +66,10 @@ class StepInfo:
     tile_row0: Optional[torch.Tensor] = None     # int32 [n_tiles]
     tile_rows: Optional[torch.Tensor] = None     # int32 [n_tiles]
     n_tiles: int = 0
+    # the decode rows' keys in steps of 32: over all of them, and of the longest one (how attention divides the rows)
+    decode_work: Tuple[int, int] = (0, 0)
+    # where attention leaves the shapes it is asked for (`tuned.decode_shape`), by which an engine tells its graphs apart
+    decode_shapes: Optional[set] = None
     # counters of the decode attention that belong to the engine of a step that is recorded (see tuned._pair_counters)
     pair_counters: Optional[list] = None
 
@@ -73,6 +77,14 @@ class StepInfo:
 # the arrays of the buffer, in order; block tables follow, one per paged group
 ARRAYS = ("tokens", "positions", "row_seg", "seg_row0", "seg_rows", "seg_pos0", "state_slots", "logit_rows",
           "decode_rows", "tile_row0", "tile_rows", "position_axes")
+
+
+def decode_work(lengths: Sequence[int], rows: int = 0) -> Tuple[int, int]:
+    """`StepInfo.decode_work` of decode rows that see so many keys, padded to `rows` by rows that see one."""
+    if not lengths:
+        return max(0, rows), min(1, max(0, rows))
+    steps = [(n + 31) >> 5 for n in lengths]
+    return sum(steps) + max(0, rows - len(steps)), max(steps)
 
 
 class StepLayout:
@@ -121,7 +133,8 @@ class StepLayout:
             n_tiles=self.n_tiles, host_row0=list(host_row0), host_rows=list(host_rows), host_pos0=list(host_pos0),
             host_slots=list(host_slots),
             max_context=max([p + n for p, n in zip(host_pos0, host_rows)] or [0]), max_rows=max(list(host_rows) or [0]),
-            decode_only=all(n == 1 for n in host_rows))
+            decode_only=all(n == 1 for n in host_rows),
+            decode_work=decode_work([p + 1 for p, n in zip(host_pos0, host_rows) if n == 1]))
 
 
 def pack_step(entries: Sequence[Entry], pos0: Sequence[int], slots: Sequence[int],

@@ -90,8 +90,11 @@ class NativeProgram:
             layer.w_down, layer.F = _matrix(f["w_down"], self.keep), int(f["F"])
             if L.apc_host_program_add_layer(self.handle, ctypes.byref(layer)) < 0:
                 return self._give_up()
+        self.decode_shapes = set()      # see StepInfo.decode_shapes
         for e, v in zip(spec.plan, views):
             a = blocks[e.block]["mixer"]
+            if rt.dtype == v.kv.dtype == torch.bfloat16:
+                self.decode_shapes.add(tuned.decode_shape(a["H"], a["Hk"], a["d"], int(a["window"])))
             if tuple(v.kv.shape[1:]) != (2, a["Hk"], v.page_tokens, a["d"]) or (v.window or 0) != a["window"]:
                 return self._give_up()
             self.keep.append(v.kv)
@@ -151,6 +154,7 @@ class NativeProgram:
         s.max_decode_context = info.max_decode_context
         s.all_rows_decode = 1 if info.decode_rows is None else 0
         s.max_prompt_keys = max([p + n for p, n in zip(info.host_pos0, info.host_rows) if n > 1] or [0])
+        s.decode_steps, s.decode_longest = info.decode_work
         s.prompt_passes = tuned._prompt_passes(info.host_pos0, info.host_rows) if info.n_tiles else 0
         return s
 

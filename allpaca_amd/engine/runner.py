@@ -19,7 +19,8 @@ import torch
 
 from ..cache import CacheManager, CacheStorage, OutOfPages, PagedView, StateView
 from ..models.decoder import DecoderModel
-from .batch import Entry, StepInfo, StepLayout, pack_step
+from ..kernels import tuned
+from .batch import Entry, StepInfo, StepLayout, decode_work, pack_step
 
 
 class StepError(ValueError):
@@ -56,12 +57,14 @@ class ModelRunner:
         self.use_graphs = bool(use_graphs) and all(getattr(p, "graph_safe", False) for p in parts)
         from ..kernels import ops
         if self.rt.dtype == torch.bfloat16 and not ops.FORCE_PLAIN:
-            from ..kernels import tuned
             tuned.check_chip(self.rt.device)
         self.tile_rows = ops.attention_tile_rows(self.rt.dtype)          # how the attention kernel wants longer segments cut
         self.position_axes = int(getattr(model.spec, "position_axes", 1))
         self.graphs: Dict[Tuple[int, int], "DecodeGraph"] = {}
         self.pair_counters: list = []       # of the decode attention in its graphs (made when one is first recorded)
+        # of its attention: what tells the graphs of a bucket apart (a model that is walked in Python tells them in its
+        # first step)
+        self.decode_shapes: set = self.native.decode_shapes if self.native is not None else set()
         self.graph_replays = 0
         self.steps = 0
         # The C++ side of a step (csrc/host/pack.cpp): entries checked against the cache's books, pages taken, the
@@ -251,6 +254,7 @@ class ModelRunner:
         """The model on a packed step: logits at the wanted rows."""
         if self.native is not None:
             return self.native.forward(info)
+        info.decode_shapes = self.decode_shapes
         return self.model.forward(info, self.bind_views(info))
 
     def bind_views(self, info: StepInfo) -> list:
@@ -290,12 +294,26 @@ class ModelRunner:
             return (n + 1) // 2 * 2
         return 1 << max(0, (n - 1).bit_length())
 
+    def _graph_key(self, rows: int, span: int, lengths: Sequence[int]) -> tuple:
+        """(rows, span), and how attention divides the rows where that depends on their lengths: graphs of one bucket that
+        differ in it are different graphs.  Padding rows see one key."""
+        if not tuned.decode_routes_differ(rows, span, self.decode_shapes):
+            return rows, span
+        return (rows, span) + tuned.decode_routes(rows, span, decode_work(lengths, rows), self.decode_shapes)
+
+    def _graph(self, rows: int, span: int, lengths: Sequence[int]) -> Tuple["DecodeGraph", bool]:
+        """The graph for these contexts, and whether it was recorded now."""
+        g = self.graphs.get(self._graph_key(rows, span, lengths))
+        if g is not None:
+            return g, False
+        g = DecodeGraph(self, rows, span, decode_work(lengths, rows))
+        self.graphs[self._graph_key(rows, span, lengths)] = g    # (its recording may have told the shapes)
+        return g, True
+
     def _graph_for(self, seqs: Sequence[Hashable]) -> "DecodeGraph":
-        key = self._bucket(len(seqs), max(self.cache.length(s) for s in seqs) + 1)
-        g = self.graphs.get(key)
-        if g is None:
-            g = self.graphs[key] = DecodeGraph(self, *key)
-        return g
+        lengths = [self.cache.length(s) + 1 for s in seqs]
+        rows, span = self._bucket(len(seqs), max(lengths))
+        return self._graph(rows, span, lengths)[0]
 
     def capture_decode_graphs(self, max_rows: int, max_context: Optional[int] = None) -> int:
         """Captures now, instead of at its first use (some tens of milliseconds in the middle of serving), the
@@ -313,10 +331,10 @@ class ModelRunner:
                     break
                 longest *= 2
         made = 0
-        for key in sorted(keys):
-            if key not in self.graphs:
-                self.graphs[key] = DecodeGraph(self, *key)
-                made += 1
+        for rows, span in sorted(keys):
+            # contexts of one length, the longest and the shortest of the bucket, and one long context beside short ones
+            for lengths in ([span] * rows, [span // 2 + 1] * rows, [span]):
+                made += self._graph(rows, span, lengths)[1]
         return made
 
     def _launch(self, g: "DecodeGraph", tokens: Sequence[int]) -> torch.Tensor:
@@ -379,7 +397,8 @@ class DecodeGraph:
     """The launches of one decode step for `rows` single-token requests whose contexts fit `span` positions.
     Rows beyond the live requests are padding: token 0 at position 0 of the spare page and the spare slot."""
 
-    def __init__(self, runner: ModelRunner, rows: int, span: int):
+    def __init__(self, runner: ModelRunner, rows: int, span: int, work: Tuple[int, int] = (0, 0)):
+        """`work`: contexts to record for (`StepInfo.decode_work`)."""
         self.runner, self.rows, self.span = runner, rows, span
         cache = runner.cache
         self.widths = [-(-span // cache.page_tokens) for _ in cache.paged_groups]
@@ -396,6 +415,8 @@ class DecodeGraph:
         self.info = lay.info(self.dev, list(range(rows)), [1] * rows, [0] * rows, [0] * rows, span, True)
         self.info.max_context = span
         self.info.pair_counters = runner.pair_counters
+        self.info.decode_work = work
+        self.info.decode_shapes = runner.decode_shapes
         self.copied = torch.cuda.Event()
         # what the pinned block tables hold: the request of every row and how many of its pages (per group), so that
         # a step writes only what is new (`CacheManager.table_version` changes when pages were taken away)

@@ -37,7 +37,7 @@ class ApcStep(Structure):
                 + [(name, c_void_p) for name in STEP_ARRAYS]
                 + [("n_groups", c_int), ("table", c_void_p * MAX_PAGED_GROUPS), ("table_width", c_int * MAX_PAGED_GROUPS),
                    ("max_decode_context", c_int), ("all_rows_decode", c_int), ("max_prompt_keys", c_int),
-                   ("prompt_passes", c_longlong)])
+                   ("decode_steps", c_longlong), ("decode_longest", c_int), ("prompt_passes", c_longlong)])
 
 
 class ApcStepFinding(Structure):
@@ -74,7 +74,8 @@ _lib.SIGNATURES["host"].update({
     "apc_host_timing_report": [P],
     "apc_host_rule_tiled_k_split": [I, I, I],
     "apc_host_rule_decode_parts": [c_longlong, I],
-    "apc_host_rule_decode_even": [c_longlong, I, I, I],
+    "apc_host_rule_even_pays": [c_longlong, I, I, I, I],
+    "apc_host_rule_decode_even": [c_longlong, I, I, I, I],
     "apc_host_rule_key_splits": [I, I, I, I, I, I],
     "apc_host_rule_key_splits_by_time": [I, I, I, I, c_longlong, I, I],
     # ---- the cache manager's books

@@ -347,18 +347,63 @@ WHOLE_MIN_PAIRS = 256
 WHOLE_WAVES = 4   # waves of such a block (NW in attention_bf16.hip)
 
 
-# From so many pairs on, in steps whose longest row may have more keys than this, the rows' work is dealt out evenly over
+# From so many pairs on, in steps whose longest row may have more keys than this, the rows' work may be dealt out evenly over
 # all waves of one round of blocks (DEC_EVEN in attention_bf16.hip) instead of a block a pair, whose longest row sets the
-# launch's time.  Microseconds a layer, block a pair / even: 64 rows of 90 to 2,100 keys (24 heads of 128 on 8) 63.2 / 37.0,
-# 64 rows of 2,048 89.6 / 88, 32 rows of 328 to 4,296 65.8 / 40.2, one row of 4,096 beside 63 of 128 71 / 25, 64 rows of 90
-# to 2,100 with heads of 64 33.6 / 22.3; short rows pay more for the shares than they gain: 64 rows of 300 18.5 / 22.1, 200
-# rows of 30 to 700 with heads of 64 24.0 / 28.  With fewer pairs the way below, which cuts every pair for itself, is
-# faster (16 rows of 2,048 26.8 / 30, 8 rows 17.6 / 26).
+# launch's time; whether it is, the rows' lengths say (`_even_pays`).  With fewer pairs the way below, which cuts every pair
+# for itself, is faster (16 rows of 2,048 26.8 / 30 us, 8 rows 17.6 / 26).  Where a block has no room for a pair (16 heads of
+# 256 on a kv head) a pair's keys go to parts in memory: from 1,024 pairs on shares are faster whatever the lengths (1,024
+# rows of 1,100 250 / 205, of 30 to 1,100 125 / 115), with 256 pairs not (61 / 92, 47 / 62).  More pairs than the compiled
+# executor has counters for keep a block each.
 EVEN_MIN_PAIRS, EVEN_MIN_SPAN = 256, 1024
+EVEN_MAX_PAIRS, EVEN_ALONE_MIN_PAIRS = 4096, 1024
 
 
-def _decode_even(pairs: int, span: int) -> bool:
-    return pairs >= EVEN_MIN_PAIRS and span > EVEN_MIN_SPAN
+def _decode_even(pairs: int, span: int, pair_fits: bool = True) -> bool:
+    least = EVEN_MIN_PAIRS if pair_fits else max(EVEN_MIN_PAIRS, EVEN_ALONE_MIN_PAIRS)
+    return least <= pairs <= EVEN_MAX_PAIRS and span > EVEN_MIN_SPAN
+
+
+def _even_pays(steps: int, longest: int, n_rows: int, tiles: int, window: int) -> bool:
+    """Whether shares beat a block a pair for the lengths at hand (`StepInfo.decode_work`, which a window cuts), by the time
+    of either in units of a wave's step of 32 keys.  Shares: a wave's share, a few units for the pieces' way through memory,
+    and a look at all rows.  A block a pair: the same work, or the longest row's chain over four waves, slowed by the blocks
+    that share its compute unit.  Fitted to 774 launches (1 to 32 kv heads of 64 to 256, 8 to 512 rows of equal, spread and
+    single long lengths), where the choice is on average 0.5 % over the better of the two; shares alone are 2.1 %, a block a
+    pair alone 50 %.  Microseconds a layer, block a pair / shares, 8 kv heads of 128: 32 rows of 1,100 keys 26.1 / 31.8, of
+    2,048 44.2 / 50.2, of 1,000 to 2,048 39.9 / 40.1, of 90 to 2,100 33.2 / 25.6; 64 rows of 1,100 49.1 / 53.8, of 2,048
+    85.7 / 87.5, of 1,000 to 2,048 75.1 / 71.4, of 90 to 2,100 63.5 / 37.9, one of 8,000 beside 63 of 100 120 / 30; 128 rows of
+    2,048 169 / 166.  32 kv heads of 128: 8 rows of 2,048 43.2 / 47.9, of 90 to 2,100 24.7 / 25.6, 16 rows of those 57 / 30."""
+    if window:
+        most = window // 32 + 1
+        longest, steps = min(longest, most), min(steps, n_rows * most)
+    waves = max(1, CHIP_UNITS // tiles) * WHOLE_WAVES
+    units, share = n_rows * WHOLE_WAVES / waves, (steps + 2 * n_rows) / waves
+    whole = max(1.03 * share + 2.5 + 1.1 * units, 4.1 + 0.245 * longest * min(math.ceil(units), 2.8))
+    return 7.3 + max(share, 8.3) + 0.05 * (n_rows / 64) < whole
+
+
+def decode_shape(n_heads: int, n_kv_heads: int, head_dim: int, window: int) -> tuple:
+    """What the way of a layer's decoded rows depends on beside the rows: (tiles of heads a row, whether a block has room
+    for a (row, kv head) pair, window)."""
+    fits = bool(_lib.load("tuned").apc_attention_decode_whole_fits(n_heads, n_kv_heads, head_dim))
+    return n_kv_heads * -(-(n_heads // n_kv_heads) // 16), fits, int(window)
+
+
+def _decode_shares(rows: int, span: int, work, shape) -> bool:
+    """Whether the rows of such a layer share out their work; `work`: `StepInfo.decode_work`."""
+    tiles, fits, window = shape
+    return (_decode_even(rows * tiles, min(span, window) if window else span, fits)
+            and (not fits or _even_pays(work[0], work[1], rows, tiles, window)))
+
+
+def decode_routes_differ(rows: int, span: int, shapes) -> bool:
+    """Whether the rows' lengths say how some layer of these shapes divides its decoded rows."""
+    return any(f and _decode_even(rows * t, min(span, w) if w else span) for t, f, w in shapes)
+
+
+def decode_routes(rows: int, span: int, work, shapes) -> tuple:
+    """How every one of the layers' shapes divides decoded rows of such lengths."""
+    return tuple(_decode_shares(rows, span, work, s) for s in sorted(shapes))
 
 
 # With fewer pairs: the blocks of a pair leave one partial result each and the one that finishes last adds them (no
@@ -473,6 +518,9 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
     sc = (1.0 / math.sqrt(head_dim)) if scale is None else float(scale)
     L = _lib.load("tuned")
     stream = _ops._stream()
+    shape = decode_shape(n_heads, n_kv_heads, head_dim, window)
+    if getattr(step, "decode_shapes", None) is not None:
+        step.decode_shapes.add(shape)
     if step.n_tiles:
         # (only the kernel of 128-row blocks cuts keys into ranges: no room is taken for the others)
         wide = WIDE_TILES and L.apc_attention_prefill_wide_takes(head_dim, page_tokens, step.n_tiles, T - step.n_decode_rows)
@@ -499,7 +547,8 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
         pairs = n * n_kv_heads * -(-(n_heads // n_kv_heads) // 16)
         counters = lambda: _pair_counters(q.device, pairs, getattr(step, "pair_counters", None))  # noqa: E731
         n_parts = -(-step.max_decode_context // KEYS_PER_PART) if KEYS_PER_PART else _decode_parts(pairs, span)
-        if _decode_even(pairs, span) and not KEYS_PER_PART and ldo % 4 == 0 and out.data_ptr() % 8 == 0:
+        pair_fits = shape[1]
+        if _decode_shares(n, step.max_decode_context, getattr(step, "decode_work", (0, 0)), shape) and not KEYS_PER_PART and ldo % 4 == 0 and out.data_ptr() % 8 == 0:
             ws = torch.empty(L.apc_attention_decode_even_workspace(n_heads, n_kv_heads, head_dim), dtype=torch.float32,
                              device=q.device)
             _lib.check(L.apc_attention_decode_even_bf16(
@@ -509,8 +558,7 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
                 counters().data_ptr(), stream), "attention_decode_bf16 (even shares)")
             return True
         # (rows so short that one block's waves take a pair's ranges need no partial results either)
-        if ((pairs >= WHOLE_MIN_PAIRS or n_parts <= WHOLE_WAVES)
-                and L.apc_attention_decode_whole_fits(n_heads, n_kv_heads, head_dim)):
+        if (pairs >= WHOLE_MIN_PAIRS or n_parts <= WHOLE_WAVES) and pair_fits:
             _lib.check(L.apc_attention_decode_bf16(
                 q.data_ptr(), ldq, q_off, out.data_ptr(), ldo, n, n_heads, n_kv_heads, head_dim, cache.data_ptr(),
                 page_tokens, block_table.data_ptr(), block_table.shape[1], step.positions.data_ptr(),
