@@ -43,13 +43,13 @@ __device__ __forceinline__ void each_count(F f) {        // f(1), .. f(N), known
 // GLU: W is [2 N][K], rows of gates and then rows of values; a block's bands of W are NT / 2 of gates and the NT / 2 of
 // values that belong to them, and it writes silu(gate) * value.  A product is the same sum as without, so the result is
 // the bits of the product of 2 N outputs and the activation's own pass.
-template <int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU>
-__global__ __launch_bounds__(64 * SLICES, MIN_WAVES) void gemm_f32_kernel(
+template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU>
+__global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
     const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, void* __restrict__ C, int c_dtype,
     int ldc, int M, int N, int K, int mode, int tiles_m, int tiles) {
   constexpr int BANDS = MT + NT;
   constexpr int STAGE_F4 = BANDS * 128, SUM_F4 = MT * NT * 64;       // float4 a wave: its stage, its sums
-  __shared__ f32x4 lds[SLICES * (STAGE_F4 > SUM_F4 ? STAGE_F4 : SUM_F4)];
+  __shared__ f32x4 lds[SL * (STAGE_F4 > SUM_F4 ? STAGE_F4 : SUM_F4)];
   // The block ids that one XCD gets (every eighth) are a run of tiles, row tiles of the same outputs next to each other:
   // they share W in that XCD's L2.
   const int per = (tiles + 7) / 8;
@@ -174,13 +174,14 @@ __global__ __launch_bounds__(64 * SLICES, MIN_WAVES) void gemm_f32_kernel(
 #pragma unroll
     for (int j = 0; j < NT; ++j) lds[wave * SUM_F4 + (i * NT + j) * 64 + lane] = acc[i][j];
   __syncthreads();
-  for (int p = threadIdx.x; p < MT * NO * 64; p += 64 * SLICES) {
+  const bool wide = mode == 0 && c_dtype == APC_F32 && ldc % 4 == 0 && ((uintptr_t)C & 15u) == 0;   // 16-byte stores
+  for (int p = threadIdx.x; p < MT * NO * 64; p += 64 * SL) {
     const int i = p / (NO * 64), j = p / 64 % NO, l = p % 64;
     auto sum = [&](int band) __attribute__((always_inline)) {
       const int at = (i * NT + band) * 64 + l;
       f32x4 v = lds[at];
 #pragma unroll
-      for (int w = 1; w < SLICES; ++w) v += lds[w * SUM_F4 + at];
+      for (int w = 1; w < SL; ++w) v += lds[w * SUM_F4 + at];
       return v;
     };
     f32x4 v = sum(j);
@@ -191,6 +192,10 @@ __global__ __launch_bounds__(64 * SLICES, MIN_WAVES) void gemm_f32_kernel(
     }
     const int m = m0 + i * 16 + l % 16, n = n0 + j * 16 + (l / 16) * 4;
     if (m >= M) continue;
+    if (wide && n + 4 <= N) {
+      *(f32x4*)((float*)C + (size_t)m * ldc + n) = v;
+      continue;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if (n + e >= N) continue;
@@ -201,16 +206,32 @@ __global__ __launch_bounds__(64 * SLICES, MIN_WAVES) void gemm_f32_kernel(
   }
 }
 
-template <int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU = false>
-int launch(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
+// Slices without k are left out: with all eight, a block of a large tile keeps its unit for 6 us whatever K is, most of
+// its waves idle and 128 KiB of LDS taken.  2,048 rows x 16,384 outputs at K = 32, 64, 128: 200, 203, 216 us with eight
+// slices and stores of 4 bytes, 84, 101, 147 with the two or four there are, 53, 69, 125 with 16-byte stores beside (one
+// fma chain an output on the vector units: 70, 98, 150).
+template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU>
+int launch_slices(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
            hipStream_t stream) {
   const int tiles_m = ceil_div(M, 16 * MT);
   const long long tiles = (long long)tiles_m * ceil_div(N, 16 * (GLU ? NT / 2 : NT));
   if (tiles > (1 << 27)) return APC_ERR_BAD_ARG;
-  hipLaunchKernelGGL((gemm_f32_kernel<MT, NT, D, ONCE, MIN_WAVES, GLU>), dim3(ceil_div((int)tiles, 8) * 8), dim3(64 * SLICES), 0,
+  hipLaunchKernelGGL((gemm_f32_kernel<SL, MT, NT, D, ONCE, MIN_WAVES, GLU>), dim3(ceil_div((int)tiles, 8) * 8), dim3(64 * SL), 0,
                      stream, A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, tiles_m, (int)tiles);
   APC_LAUNCH_CHECK();
   return 0;
+}
+
+template <int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU = false>
+int launch(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
+           hipStream_t stream) {
+#define SL_GO(SL_) return launch_slices<SL_, MT, NT, D, ONCE, MIN_WAVES, GLU>(A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
+  if constexpr (MT * NT >= 4 && MT * NT <= 6) {         // (smaller tiles share their units with eight too; larger ones are not chosen)
+    if (K <= 2 * STAGE) SL_GO(2);
+    if (K <= 4 * STAGE) SL_GO(4);
+  }
+  SL_GO(SLICES);
+#undef SL_GO
 }
 
 }  // namespace
@@ -221,28 +242,47 @@ bool gemm_f32_takes(const void* A, int lda, const void* W, int ldw, int K) {
          ldw < (1 << 22);            // (64 rows fit a descriptor's 32-bit offsets)
 }
 
-// The tile: the least of these times (microseconds at K = 2,048; K stretches them alike) over the tiles' shapes.  A
-// block of the small tiles shares its compute unit with others, so their time grows with the blocks; the large ones have
-// a unit to themselves and go in whole rounds of 256.  Measured on 24 to 2,048 rows x 2,048 to 16,384 outputs, where the
-// choice is within a tenth of the best of the six: 2,048 outputs take 9.4 us up to 48 rows, 18 at 160 rows (48 x 32
-// tiles; 16 x 16: 25, 64 x 64: 41), 31 at 330 (48 x 64; 16 x 16: 43).
-int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
-             hipStream_t stream) {
-  struct Shape { int mt, nt; bool shares; double start, round; };
-  constexpr Shape shapes[] = {{1, 1, true, 4.5, 5.0},   {2, 1, true, 4.0, 5.8},   {2, 2, false, 1.5, 13.0},
-                              {3, 2, false, 1.5, 15.5}, {3, 4, false, 1.5, 28.7}, {4, 4, false, 1.5, 39.0}};
+// A tile of 16 mt x 16 nt and what a launch of its blocks costs: start and, for every 256 of them, round.
+struct TileCost { int mt, nt; bool shares; double start, round; };
+template <int COUNT>
+static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, int outputs) {   // outputs: of 16 nt columns
   int best = 0;
   double best_cost = 1e30;
-  for (int i = 0; i < 6; ++i) {
-    const Shape& s = shapes[i];
-    double rounds = (double)ceil_div(M, 16 * s.mt) * ceil_div(N, 16 * s.nt) / 256;
+  for (int i = 0; i < COUNT; ++i) {
+    const TileCost& s = shapes[i];
+    double rounds = (double)ceil_div(M, 16 * s.mt) * ceil_div(N, outputs * s.nt) / 256;
     if (!s.shares) rounds = ceil(rounds);
     const double cost = s.start + s.round * (rounds > 1.0 ? rounds : 1.0);
     if (cost < best_cost) best = i, best_cost = cost;
   }
+  return best;
+}
+
+// The tile: the least of these times (microseconds at K = 2,048; K stretches them alike) over the tiles' shapes.  A
+// block of the small tiles shares its compute unit with others, so their time grows with the blocks; the large ones have
+// a unit to themselves and go in whole rounds of 256.  Measured on 24 to 2,048 rows x 2,048 to 16,384 outputs, where the
+// choice is within a tenth of the best of the six: 2,048 outputs take 9.4 us up to 48 rows, 18 at 160 rows (48 x 32
+// tiles; 16 x 16: 25, 64 x 64: 41), 31 at 330 (48 x 64; 16 x 16: 43).  (The 64 x 64 tile keeps 48 registers of loads in
+// scratch memory and is the best from 512 rows x 2,048 outputs on all the same: 43 us against 50 and 53 of the next two,
+// 1,024 rows x 8,192 311 against 317.)
+// Up to K = 128 (see launch_slices) blocks of all tiles share their units.
+constexpr TileCost TILES[] = {{1, 1, true, 4.5, 5.0},   {2, 1, true, 4.0, 5.8},   {2, 2, false, 1.5, 13.0},
+                              {3, 2, false, 1.5, 15.5}, {3, 4, false, 1.5, 28.7}, {4, 4, false, 1.5, 39.0}};
+constexpr TileCost TILES_SHORT[] = {{1, 1, true, 3.6, 0.75}, {2, 1, true, 3.6, 0.95}, {2, 2, true, 4.1, 0.69},
+                                    {3, 2, true, 4.4, 0.93}};        // (48 x 64 and 64 x 64 are never the least)
+static int tile_of(int M, int N, int K) { return K <= 4 * STAGE ? least_cost(TILES_SHORT, M, N, 16) : least_cost(TILES, M, N, 16); }
+
+// Rows of the tile, times 1,000, and its outputs.
+APC_EXPORT int apc_gemm_f32_tile(int M, int N, int K) {
+  const TileCost& t = TILES[tile_of(M, N, K)];
+  return 16 * t.mt * 1000 + 16 * t.nt;
+}
+
+int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
+             hipStream_t stream) {
 #define GO(...) return launch<__VA_ARGS__>(A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
   // (one row tile: W is read once, past the caches)
-  switch (best) {
+  switch (tile_of(M, N, K)) {
     case 0:
       if (M <= 16) GO(1, 1, 4, true, 4);
       GO(1, 1, 4, false, 4);
@@ -264,25 +304,24 @@ APC_EXPORT int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int l
   return gemm_f32_takes(A, lda, W, ldw, K) && ((long long)F + 64) * ldw < (1LL << 29);   // byte offsets of 32 bits
 }
 
+constexpr TileCost GLU_TILES[] = {{1, 2, true, 4.5, 8.5}, {2, 2, false, 1.5, 13.0}, {3, 2, false, 1.5, 15.5},
+                                  {3, 4, false, 1.5, 28.7}, {4, 4, false, 1.5, 39.0}};
+constexpr TileCost GLU_TILES_SHORT[] = {{1, 2, true, 3.6, 0.95}, {2, 2, true, 4.1, 0.69}, {3, 2, true, 4.4, 0.93}};
+static int glu_tile_of(int M, int F, int K) { return K <= 4 * STAGE ? least_cost(GLU_TILES_SHORT, M, F, 8) : least_cost(GLU_TILES, M, F, 8); }
+
+// Rows of the tile, times 1,000, and its outputs (half of the columns it computes).
+APC_EXPORT int apc_swiglu_f32_tile(int M, int F, int K) {
+  const TileCost& t = GLU_TILES[glu_tile_of(M, F, K)];
+  return 16 * t.mt * 1000 + 8 * t.nt;
+}
+
 APC_EXPORT int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, void* out, int ldo, int M, int F, int K,
                               hipStream_t stream) {
   if (M <= 0 || F <= 0) return 0;
   if (K <= 0 || lda < K || ldw < K || ldo < F) return APC_ERR_BAD_ARG;
   if (!apc_swiglu_f32_takes(A, lda, W, ldw, F, K)) return APC_ERR_UNSUPPORTED;
-  struct Shape { int mt, nt; bool shares; double start, round; };
-  constexpr Shape shapes[] = {{1, 2, true, 4.5, 8.5}, {2, 2, false, 1.5, 13.0}, {3, 2, false, 1.5, 15.5},
-                              {3, 4, false, 1.5, 28.7}, {4, 4, false, 1.5, 39.0}};
-  int best = 0;
-  double best_cost = 1e30;
-  for (int i = 0; i < 5; ++i) {
-    const Shape& s = shapes[i];
-    double rounds = (double)ceil_div(M, 16 * s.mt) * ceil_div(F, 8 * s.nt) / 256;
-    if (!s.shares) rounds = ceil(rounds);
-    const double cost = s.start + s.round * (rounds > 1.0 ? rounds : 1.0);
-    if (cost < best_cost) best = i, best_cost = cost;
-  }
 #define GO(...) return launch<__VA_ARGS__, true>((const float*)A, lda, (const float*)W, ldw, out, APC_F32, ldo, M, F, K, 0, stream)
-  switch (best) {
+  switch (glu_tile_of(M, F, K)) {
     case 0:
       if (M <= 16) GO(1, 2, 2, true, 4);
       GO(1, 2, 2, false, 4);

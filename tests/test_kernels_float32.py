@@ -6,8 +6,6 @@ import numpy as np
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
-
 DEV = "cuda:0"
 U = 2.0 ** -24
 
@@ -28,9 +26,23 @@ def product_bound(a, w):
 
 
 # rows and outputs of every tile's range (16 x 16, 32 x 16, 32 x 32, 48 x 32, 48 x 64, 64 x 64) and their remainders;
-# widths with whole and ragged stages of 32 and slices with 0, 1, 2, several of them
-@pytest.mark.parametrize("M,N,K", [(1, 16, 4), (3, 70, 36), (16, 515, 256), (17, 33, 260), (8, 2048, 2048), (24, 16384, 96),
-                                   (100, 2041, 388), (160, 2048, 1028), (331, 2045, 516), (480, 2050, 320), (33, 100, 8192)])
+# widths with whole and ragged stages of 32 and slices with 0, 1, 2, several of them; widths of two, of four and of eight
+# slices at the tiles that leave the empty ones out
+SIZES = [(1, 16, 4), (3, 70, 36), (16, 515, 256), (17, 33, 260), (8, 2048, 2048), (24, 16384, 96), (100, 2041, 388),
+         (160, 2048, 1028), (331, 2045, 516), (480, 2050, 320), (33, 100, 8192), (509, 2045, 324), (509, 2045, 4), (331, 2047, 32),
+         (509, 4101, 36), (331, 2045, 64), (500, 4090, 68), (331, 2045, 128), (700, 4099, 128), (331, 2045, 132), (20, 130, 100)]
+
+
+def test_the_sizes_reach_every_tile():
+    from allpaca_amd.kernels import lib
+    L = lib.load("plain")
+    for slices, tiles in ((lambda k: k > 128, {16016, 32016, 32032, 48032, 48064, 64064}),
+                          (lambda k: 64 < k <= 128, {16016, 32032, 48032}), (lambda k: k <= 64, {16016, 32032, 48032})):
+        assert {L.apc_gemm_f32_tile(*s) for s in SIZES if slices(s[2])} >= tiles
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SIZES)
 def test_product_against_64_bits_and_rows_alone(M, N, K):
     o = ops()
     a, w = gen(M, K, seed=1), gen(N, K, seed=2)
@@ -48,6 +60,7 @@ def test_product_against_64_bits_and_rows_alone(M, N, K):
     assert torch.equal(both, add + out)
 
 
+@pytest.mark.gpu
 def test_product_of_views_reads_nothing_past_their_width():
     """Rows of a wider matrix whose other columns hold NaN, outputs into a wider matrix, bfloat16 outputs."""
     o = ops()
@@ -64,6 +77,7 @@ def test_product_of_views_reads_nothing_past_their_width():
         assert torch.equal(half, wide[:, :90].to(torch.bfloat16))
 
 
+@pytest.mark.gpu
 def test_product_lets_infinities_and_nan_through():
     o = ops()
     a, w = gen(5, 36, seed=6), gen(20, 36, seed=7)
@@ -97,6 +111,7 @@ def paged(lengths, Hk, d, P, seed):
 
 # groups of 4, 2, 1 heads on a kv head (and 3, taken one by one); heads up to 64 and up to 128; pages under, at and over
 # a chunk of 64 keys; lengths around a chunk and around eight of them
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,Hk,d,P", [(8, 2, 64, 16), (6, 2, 32, 4), (4, 2, 128, 16), (3, 1, 100, 8), (4, 1, 80, 128)])
 @pytest.mark.parametrize("window", [0, 70])
 def test_attention_against_64_bits_and_rows_alone(H, Hk, d, P, window):

@@ -6,11 +6,21 @@ import torch
 
 from test_kernels_tuned import DEV, gen
 
-pytestmark = pytest.mark.gpu
+SIZES = [(1, 1, 4), (1, 16, 32), (4, 1000, 260), (4, 8192, 2048), (16, 17, 512), (17, 8200, 64), (40, 2048, 1028), (49, 4095, 96),
+         (130, 1024, 288), (340, 8192, 512), (700, 9000, 36), (509, 2045, 132), (49, 4095, 132), (49, 100, 36), (700, 9000, 100),
+         (30, 3000, 132), (1, 40, 100)]
 
 
-@pytest.mark.parametrize("M,F,K", [(1, 1, 4), (1, 16, 32), (4, 1000, 260), (4, 8192, 2048), (16, 17, 512), (17, 8200, 64),
-                                   (40, 2048, 1028), (49, 4095, 96), (130, 1024, 288), (340, 8192, 512), (700, 9000, 36)])
+def test_the_sizes_reach_every_tile():
+    from allpaca_amd.kernels import lib
+    L = lib.load("plain")
+    for slices, tiles in ((lambda k: k > 128, {16016, 32016, 48016, 48032, 64032}),
+                          (lambda k: 64 < k <= 128, {16016, 32016, 48016}), (lambda k: k <= 64, {16016, 32016, 48016})):
+        assert {L.apc_swiglu_f32_tile(*s) for s in SIZES if slices(s[2])} >= tiles
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,F,K", SIZES)
 @pytest.mark.parametrize("pad", [0, 4])
 def test_both_products_and_the_activation(M, F, K, pad):
     from allpaca_amd.kernels import ops
@@ -24,6 +34,7 @@ def test_both_products_and_the_activation(M, F, K, pad):
     assert bool((out[:, F:] == 7.0).all())
 
 
+@pytest.mark.gpu
 def test_rows_that_are_no_pieces_of_16_bytes_are_left_alone():
     from allpaca_amd.kernels import ops
     h, w = gen(4, 63).to(DEV), gen(48, 63).to(DEV)
