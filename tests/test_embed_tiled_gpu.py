@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dim", [8, 24, 32, 41, 1016, 1024, 1032, 4104])
 @pytest.mark.parametrize("dtype", [torch.float32, BF])
-@pytest.mark.parametrize("pad", [0, 2, 4])
+@pytest.mark.parametrize("pad", [0, 2, 4, 8])
 def test_rows_of_the_table(dim, dtype, pad):
     from allpaca_amd.kernels import ops
     table = gen(37, dim, seed=dim, dtype=BF).to(DEV)
