@@ -36,12 +36,20 @@ APC_EXPORT int apc_embed_rows(const void* table, int table_dtype, const int* tok
 constexpr int EMBED_NT = 128;
 __global__ __launch_bounds__(EMBED_NT) void embed_rows_tiled_kernel(
     const bf16_t* __restrict__ table, int chunks, const int* __restrict__ tokens, void* __restrict__ out, int out_dtype,
-    int dim, int ldo, int wide) {
+    int dim, int ldo, int wide, int pieces) {
   const int t = blockIdx.x, k = (blockIdx.y * EMBED_NT + threadIdx.x) * 8;
   if (k >= dim) return;
   const int n = tokens[t];
   const bf16_t* piece = table + (size_t)(n / 16) * chunks * 512 + (n % 16) * 8 + (size_t)(k / 32) * 512 + ((k % 32) / 8) * 128;
-  const uint4 v = *reinterpret_cast<const uint4*>(piece);
+  uint4 v;
+  if (pieces) {
+    v = *reinterpret_cast<const uint4*>(piece);
+  } else {                                     // a table that begins off 16 bytes
+    uint32_t e[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) e[i] = piece[i];
+    v = uint4{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
+  }
   const uint32_t p[4] = {v.x, v.y, v.z, v.w};
   const size_t at = (size_t)t * ldo + k;
   if (wide && out_dtype == APC_BF16) {
@@ -68,8 +76,9 @@ APC_EXPORT int apc_embed_rows_tiled(const void* table, int chunks, const int* to
   if (dim <= 0 || ldo < dim || chunks * 32 < dim) return APC_ERR_BAD_ARG;
   // whole pieces on 16-byte stores
   const int wide = dim % 8 == 0 && ldo % (out_dtype == APC_BF16 ? 8 : 4) == 0 && !((uintptr_t)out & 15u);
+  const int pieces = !((uintptr_t)table & 15u);
   hipLaunchKernelGGL(embed_rows_tiled_kernel, dim3(n_tok, ceil_div(dim, EMBED_NT * 8)), dim3(EMBED_NT), 0, stream,
-                     (const bf16_t*)table, chunks, tokens, out, out_dtype, dim, ldo, wide);
+                     (const bf16_t*)table, chunks, tokens, out, out_dtype, dim, ldo, wide, pieces);
   APC_LAUNCH_CHECK();
   return 0;
 }

@@ -19,3 +19,18 @@ def test_rows_of_the_table(dim, dtype, pad):
     ops.embed_rows(pack(table), toks, rows[:, :dim])
     assert torch.equal(rows[:, :dim].float().cpu(), table.float().cpu()[toks.cpu().long()])
     assert bool((rows[:, dim:] == 5.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, BF])
+def test_a_table_that_begins_off_16_bytes(dtype):
+    from allpaca_amd.kernels import ops
+    from allpaca_amd.kernels.packing import PackedWeight
+    table = gen(37, 264, seed=3, dtype=BF).to(DEV)
+    tiles = pack(table)
+    room = torch.zeros(tiles.data.numel() + 8, dtype=BF, device=DEV)
+    moved = room[1:1 + tiles.data.numel()].view(tiles.data.shape)
+    moved.copy_(tiles.data)
+    toks = torch.tensor([36, 0, 15, 16, 31, 36, 5], dtype=torch.int32, device=DEV)
+    rows = torch.empty(7, 264, dtype=dtype, device=DEV)
+    ops.embed_rows(PackedWeight(moved, *[getattr(tiles, n) for n in ("N", "K")]), toks, rows)
+    assert torch.equal(rows.float().cpu(), table.float().cpu()[toks.cpu().long()])
