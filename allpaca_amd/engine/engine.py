@@ -103,7 +103,7 @@ class Engine:
         widest = max([sum(ps.shape[0] for ps in b.param_specs().values() if len(ps.shape) == 2 and ps.store == "compute")
                       for b in model.blocks] or [0])
         step = cfg.max_batch_tokens * (4 * spec.hidden_size + 4 * widest) * 2
-        out = cfg.max_active_requests * (3 * 4 * spec.vocab_size + (256 << 10))
+        out = cfg.max_active_requests * (3 * 4 * spec.vocab_size + (320 << 10))
         return step + out + (1 << 30)
 
     @classmethod

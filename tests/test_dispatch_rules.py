@@ -79,6 +79,16 @@ def test_entry_points_that_launch_nothing_are_not_timed_as_kernels():
     assert "apc_swiglu_f32_takes" in asked and asked <= lib.NOT_KERNELS
 
 
+def test_the_room_kept_out_of_the_cache_holds_the_samplers_scratch():
+    from allpaca_amd.engine import Engine
+    from allpaca_amd.kernels import lib
+    L = lib.load("plain")
+    model = SimpleNamespace(spec=SimpleNamespace(hidden_size=64, vocab_size=0), blocks=[])
+    room = lambda n: Engine.reserve_bytes(model, SimpleNamespace(max_batch_tokens=8, max_active_requests=n))  # noqa: E731
+    for rows in (1, 2, 7, 16, 17, 64, 300, 1024):
+        assert room(rows) - room(0) >= 1024 * L.apc_sample_rows_scratch_kib(rows), rows
+
+
 def test_ranges_the_decode_attention_cuts_a_rows_keys_into():
     """Four ranges a block, as many blocks a (row, kv head) pair as keep the launch within the chip's compute units,
     and no range under 64 keys."""
