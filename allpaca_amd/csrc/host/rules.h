@@ -77,6 +77,7 @@ inline int key_splits(int n_tiles, int n_heads, int keys, int window, int splits
 
 // the same from a model of the launch's time (tuned._key_splits_by_time says what it rests on).  passes: of 64 keys, over
 // all tiles; rows: of the step
+constexpr double KEY_PARTS_MAX = 268435456.0;   // bytes of partial results
 inline int key_splits_by_time(int n_tiles, int rows, int n_heads, int d, long long passes, int window, int splits_max) {
   const long blocks = (long)n_tiles * n_heads;
   double mean = (double)passes / n_tiles;
@@ -84,6 +85,7 @@ inline int key_splits_by_time(int n_tiles, int rows, int n_heads, int d, long lo
   int best = 1;
   double best_us = 1e30;
   for (int s = 1; s <= std::max(1, splits_max); ++s) {
+    if (s > 1 && (double)s * rows * n_heads * (d + 2) * 4.0 > KEY_PARTS_MAX) break;
     const long unit = cdiv(blocks * s, CHIP_UNITS);   // blocks of the busiest compute unit
     const double q = mean / s;
     double us = d <= 64 ? (unit / 2) * (6.0 + 1.15 * q) + (unit % 2) * (6.0 + 0.66 * q) : unit * (12.5 + 0.8 * q);

@@ -439,6 +439,11 @@ def _key_splits(step, n_heads: int, window: int) -> int:
     return max(1, min(KEY_SPLITS_MAX, 256 // blocks, max(keys // KEY_RANGE_MIN, few)))
 
 
+# Bytes that partial results of such ranges may take (the engine keeps 1 GiB beside its cache for what a step needs over
+# its activations); a step of many rows has blocks enough.
+KEY_PARTS_MAX = 256 << 20
+
+
 def _prompt_passes(pos0, rows) -> int:
     """Passes of 64 keys that the 128-row attention kernel makes over the tiles of all segments of several rows."""
     return sum((p + min(i + 128, n) - 1) // 64 + 1 for p, n in zip(pos0 or (), rows or ()) if n > 1 for i in range(0, n, 128))
@@ -452,13 +457,16 @@ def _key_splits_by_time(n_tiles: int, rows: int, n_heads: int, head_dim: int, pa
     24,000 keys at 32 heads of 64 (384 blocks, one and a half a unit) 459 us whole, 402, 389, 355, 367 us in 2 to 5 ranges
     (chosen: 4); over 4,000 keys 100, 96, 105, 105 (1); 700 rows over 8,000 95, 88, 92, 79, 84 (4); 300 rows over 16,000
     166, 94, 100, 82, 73 (5); 1,024 rows over 16,000 186, 172, 172, 173 (2); 1,500 rows over 16,000 at 24 heads of 128 (288
-    blocks) 468, 396, 379, 376, 379 (3), over 3,000 119, 127, 135 (1); 2,048 rows over 8,000 at 32 heads 309, 346 (1)."""
+    blocks) 468, 396, 379, 376, 379 (3), over 3,000 119, 127, 135 (1); 2,048 rows over 8,000 at 32 heads 309, 346 (1).
+    The ranges' partial results stay within KEY_PARTS_MAX bytes."""
     blocks = n_tiles * n_heads
     mean = passes / n_tiles
     if window:
         mean = min(mean, float(-(-window // 64) + 2))
     best, best_us = 1, 1e30
     for s in range(1, max(1, KEY_SPLITS_MAX) + 1):
+        if s > 1 and s * rows * n_heads * (head_dim + 2) * 4.0 > KEY_PARTS_MAX:
+            break
         unit = -(-blocks * s // CHIP_UNITS)     # blocks of the busiest compute unit
         q = mean / s
         if head_dim <= 64:

@@ -21,12 +21,24 @@ def test_chosen_ranges():
     assert t._prompt_passes([0, 100, 5], [129, 1, 2]) == 2 + 3 + 1
 
 
+def test_partial_results_are_bounded():
+    """Steps of more rows than the default: their ranges' partial results would take up to 8 times the rows' outputs."""
+    from allpaca_amd.kernels import tuned as t
+    most = 0
+    for rows in range(1000, 40000, 371):
+        for heads, d in ((32, 64), (24, 128), (64, 128)):
+            s = t._key_splits_by_time(-(-rows // 128), rows, heads, d, t._prompt_passes([900000], [rows]), 0)
+            if s > 1:
+                most = max(most, s * rows * heads * (d + 2) * 4)
+    assert 0 < most <= t.KEY_PARTS_MAX
+
+
 def test_the_executors_rule_is_the_wrappers_rule(monkeypatch):
     from allpaca_amd.kernels import host, tuned as t
     L = host.load()
     for most in (8, 3, 0):
         monkeypatch.setattr(t, "KEY_SPLITS_MAX", most)
-        for rows in (64, 300, 700, 1024, 1500, 2048):
+        for rows in (64, 300, 700, 1024, 1500, 2048, 4000, 9000, 33000):
             for before in (0, 900, 4000, 24001, 130000):
                 for heads, d in ((32, 64), (24, 128), (64, 128), (4, 64)):
                     for window in (0, 1000):
