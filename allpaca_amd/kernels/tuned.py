@@ -482,6 +482,14 @@ def _key_splits_by_time(n_tiles: int, rows: int, n_heads: int, head_dim: int, pa
     return best
 
 
+def _prompt_ranges(step, rows: int, n_heads: int, head_dim: int, window: int) -> int:
+    """Ranges that the kernel of 128-row blocks cuts the keys of a step's tiles (`rows` rows in all) into."""
+    if head_dim <= 64 or step.n_tiles * n_heads > CHIP_UNITS:
+        passes = _prompt_passes(getattr(step, "host_pos0", None), getattr(step, "host_rows", None))
+        return _key_splits_by_time(step.n_tiles, rows, n_heads, head_dim, passes, window)
+    return _key_splits(step, n_heads, window)
+
+
 def _pair_counters(device: torch.device, pairs: int, own: Optional[list] = None) -> torch.Tensor:
     """Zeroed int32 counters, one per (row, kv head tile): a call leaves them zero again, so launches that share them must
     not overlap.  `own`: the list of an engine that records its steps (`StepInfo.pair_counters`); its steps never overlap,
@@ -532,14 +540,7 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
     if step.n_tiles:
         # (only the kernel of 128-row blocks cuts keys into ranges: no room is taken for the others)
         wide = WIDE_TILES and L.apc_attention_prefill_wide_takes(head_dim, page_tokens, step.n_tiles, T - step.n_decode_rows)
-        if not wide:
-            splits = 1
-        elif head_dim <= 64 or step.n_tiles * n_heads > CHIP_UNITS:
-            splits = _key_splits_by_time(step.n_tiles, T - step.n_decode_rows, n_heads, head_dim,
-                                         _prompt_passes(getattr(step, "host_pos0", None), getattr(step, "host_rows", None)),
-                                         int(window))
-        else:
-            splits = _key_splits(step, n_heads, window)
+        splits = _prompt_ranges(step, T - step.n_decode_rows, n_heads, head_dim, int(window)) if wide else 1
         parts = (torch.empty(splits * T * n_heads * (head_dim + 2), dtype=torch.float32, device=q.device)
                  if splits > 1 else None)
         _lib.check(L.apc_attention_prefill_bf16(

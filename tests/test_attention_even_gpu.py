@@ -35,8 +35,9 @@ def even(monkeypatch):
     (8, 2, 128, 16, [900, 133, 400], [1, 40, 1], 5),              # decoded rows beside a portion
 ])
 def test_rows_of_any_lengths(even, H, Hk, d, P_, lens, rows, window):
-    run_attention(H=H, Hk=Hk, d=d, P_=P_, lens=lens, rows_per_seg=rows, window=window, seed=H + d)
-    run_attention(H=H, Hk=Hk, d=d, P_=P_, lens=lens, rows_per_seg=rows, window=window, seed=H + d, stale=float("nan"))
+    for stale in (0.0, float("nan")):
+        run_attention(H=H, Hk=Hk, d=d, P_=P_, lens=lens, rows_per_seg=rows, window=window, seed=H + d, stale=stale,
+                      entry="apc_attention_decode_even_bf16")
 
 
 @pytest.mark.parametrize("H,Hk,d", [(20, 1, 32), (24, 1, 64), (34, 2, 80), (48, 2, 128), (71, 1, 256), (32, 8, 128),
@@ -59,26 +60,21 @@ def test_the_tiles_pieces_lie_apart(H, Hk, d):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,Hk,d,n", [(20, 1, 32, 128), (34, 2, 64, 64), (24, 1, 128, 128)])
-def test_wide_groups_with_work_for_nearly_all_waves(H, Hk, d, n):
-    """Groups of several tiles of heads, the last one short, in the rule's own range: pieces of every tile in most places."""
-    t = tuned()
+def test_wide_groups_with_work_for_nearly_all_waves(even, H, Hk, d, n):
+    """Groups of several tiles of heads, the last one short: pieces of every tile in most of its places."""
     lens = [1100 + (i * 977) % 400 for i in range(n)]
-    assert t._decode_even(n * Hk * -(-(H // Hk) // 16), max(lens))
     waves, steps = 4 * (256 // (Hk * -(-(H // Hk) // 16))), sum(-(-x // 32) + 2 for x in lens)
     assert steps / max(8, -(-steps // waves)) > 0.9 * waves          # (a wave's share, 8 at least)
-    run_attention(H=H, Hk=Hk, d=d, P_=16, lens=lens, rows_per_seg=[1] * n, seed=n)
+    run_attention(H=H, Hk=Hk, d=d, P_=16, lens=lens, rows_per_seg=[1] * n, seed=n, entry="apc_attention_decode_even_bf16")
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("lens,chosen", [(RAGGED[:40], True), ([1100] * 32, False)])
 def test_chosen_by_itself_and_the_counters_are_zero_again(monkeypatch, lens, chosen):
-    from allpaca_amd.kernels import lib
     t = tuned()
     monkeypatch.setattr(t, "_counters", {})
-    with lib.timing() as launched:
-        run_attention(H=16, Hk=8, d=64, P_=16, lens=lens, rows_per_seg=[1] * len(lens), seed=3)
-    names = set(launched.totals())
-    assert ("apc_attention_decode_even_bf16" in names) == chosen and ("apc_attention_decode_bf16" in names) != chosen
+    run_attention(H=16, Hk=8, d=64, P_=16, lens=lens, rows_per_seg=[1] * len(lens), seed=3,
+                  entry="apc_attention_decode_even_bf16" if chosen else "apc_attention_decode_bf16")
     used = [c for have in t._counters.values() for c in have]
     assert bool(used) == chosen and all(int(c.abs().sum()) == 0 for c in used)
 

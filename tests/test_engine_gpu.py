@@ -353,14 +353,14 @@ def test_a_long_prompt_at_the_widths_of_a_real_model_in_portions_of_512_and_128(
 
     toks = H.random_tokens(V, T, seed=11)
     asked = [4100, 4223, 4351, T - 1]          # positions whose logits are compared
-    n_heads = cfg_json["num_attention_heads"]
+    n_heads, head_dim = cfg_json["num_attention_heads"], cfg_json["head_dim"]
 
     def run(dtype, portion, seen):
         r = runner(dtype)
         forward = r.forward
-        # into how many ranges the attention kernel cuts the keys of this step's tiles (the executor's rule is the
-        # wrappers' own: tests/test_dispatch_rules.py)
-        r.forward = lambda info: seen.append(tuned._key_splits(info, n_heads, 0)) or forward(info)
+        # into how many ranges the attention kernel cuts the keys of this step's tiles (the executor's rules are the
+        # wrappers' own: tests/test_dispatch_rules.py, tests/test_key_ranges_gpu.py)
+        r.forward = lambda info: seen.append(tuned._prompt_ranges(info, info.n_rows, n_heads, head_dim, 0)) or forward(info)
         r.admit("p")
         got, at = {}, 0
         while at < T:

@@ -494,9 +494,10 @@ def test_product_for_q_k_v_that_rotates_declines_what_it_does_not_take():
                                   torch.zeros(17, dtype=torch.int32, device=DEV), bt, cache2, P_)
 
 
-def run_attention(H, Hk, d, P_, lens, rows_per_seg, window=0, seed=0, stale=0.0, loud=None, ranges=None, relocate=None):
+def run_attention(H, Hk, d, P_, lens, rows_per_seg, window=0, seed=0, stale=0.0, loud=None, ranges=None, relocate=None, entry=None):
     """Sequences of `lens` keys in the cache; the last `rows_per_seg[s]` positions of sequence s are the step's rows.
-    `ranges`: into how many ranges the kernel for tiles of 128 rows is expected to cut the keys of this step.
+    `ranges`: into how many ranges the launch for tiles of 128 rows is expected to cut the keys of this step.
+    `entry`: the entry point that is expected to take the step's single rows.
     `stale`: what lies in the slots beyond a sequence's last key and in the spare page; with a window, the pages that
     every row of the step has passed are marked as given back in the block table (the spare page stands in).
     `loud`: (sequence, position, factor) of a key whose scores dwarf all others.
@@ -519,12 +520,17 @@ def run_attention(H, Hk, d, P_, lens, rows_per_seg, window=0, seed=0, stale=0.0,
     step = pack_step(entries, pos0, [0] * len(lens), tables, torch.device(DEV), [spare],
                      tile_rows=kernel_ops.attention_tile_rows(BF))
     T = sum(rows_per_seg)
-    if ranges is not None:
-        assert t._key_splits(step, H, window) == ranges
     # queries scaled up: scores of deviation ~2.5, so a few keys carry each row and a wrong or missing one shows
     q = gen(T, H * d + 16, seed=seed + 7, scale=2.5, dtype=BF).to(DEV)
     out = torch.zeros(T, H * d, dtype=BF, device=DEV)
-    assert t.attention_bf16(q, 16, out, H, Hk, d, cache, P_, step.block_tables[0], step, window=window)
+    with t._lib.timing() as launched:
+        assert t.attention_bf16(q, 16, out, H, Hk, d, cache, P_, step.block_tables[0], step, window=window)
+    launched = launched.totals()
+    if ranges is not None:
+        ints = launched["apc_attention_prefill_bf16"]["args"][0]     # (.., number of ranges, rows of their results)
+        assert ints[-2:] == (ranges, T) and step.n_tiles == ints[8]
+    if entry is not None:
+        assert {n for n in launched if "decode" in n} == {entry}
     got = f64(out).reshape(T, H, d)
     q64 = f64(q)[:, 16:].reshape(T, H, d)
     at = 0
@@ -629,6 +635,8 @@ def test_attention_of_whole_tiles_with_the_keys_cut_into_ranges(monkeypatch, ran
     (rows that see no key of a range), a key that dwarfs the others in the first and in a later range, 8 ranges."""
     nan = float("nan")
     monkeypatch.setattr(tuned(), "KEY_RANGE_MIN", range_min)
+    # (heads of 64 take their ranges by another rule: here the same numbers)
+    monkeypatch.setattr(tuned(), "_prompt_ranges", lambda step, rows, H, d, window: tuned()._key_splits(step, H, window))
     n = lambda keys, blocks: max(1, min(8, 256 // blocks, max(keys // range_min, min(keys // (range_min // 2), 128 // blocks))))
     run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500, 200, 128], rows_per_seg=[300, 200, 100], seed=range_min, stale=nan,
                   ranges=n(1500, 6 * 4))
@@ -645,12 +653,14 @@ def test_attention_of_whole_tiles_with_the_keys_cut_into_ranges(monkeypatch, ran
 @pytest.mark.parametrize("d", [128, 64])
 def test_attention_of_whole_tiles_with_the_keys_cut_into_ranges_at_the_size_from_which_it_is_done(d):
     # 1,024 keys a range while the cut leaves the chip at most half full: 4,500 keys in 4 ranges, 17,000 in 8, 1,000 whole;
-    # 2,048 keys a range where it fills the chip: 32 heads x 4 tiles over 4,200 keys in 2 ranges, over 4,000 whole
-    run_attention(H=4, Hk=2, d=d, P_=16, lens=[4500], rows_per_seg=[100], seed=1, ranges=4)
-    run_attention(H=2, Hk=1, d=d, P_=64, lens=[17000], rows_per_seg=[129], seed=2, ranges=8)
-    run_attention(H=4, Hk=2, d=d, P_=16, lens=[1000], rows_per_seg=[100], seed=3, ranges=1)
-    run_attention(H=32, Hk=8, d=d, P_=16, lens=[4200], rows_per_seg=[512], seed=4, ranges=2)
-    run_attention(H=32, Hk=8, d=d, P_=16, lens=[4000], rows_per_seg=[512], seed=5, ranges=1)
+    # 2,048 keys a range where it fills the chip: 32 heads x 4 tiles over 4,200 keys in 2 ranges, over 4,000 whole.  Heads
+    # of 64 go by the expected time: a launch of few blocks is cut as far as it goes, one that half fills the chip in two
+    few, long, short, full, less = (4, 8, 1, 2, 1) if d > 64 else (8, 8, 8, 2, 2)
+    run_attention(H=4, Hk=2, d=d, P_=16, lens=[4500], rows_per_seg=[100], seed=1, ranges=few)
+    run_attention(H=2, Hk=1, d=d, P_=64, lens=[17000], rows_per_seg=[129], seed=2, ranges=long)
+    run_attention(H=4, Hk=2, d=d, P_=16, lens=[1000], rows_per_seg=[100], seed=3, ranges=short)
+    run_attention(H=32, Hk=8, d=d, P_=16, lens=[4200], rows_per_seg=[512], seed=4, ranges=full)
+    run_attention(H=32, Hk=8, d=d, P_=16, lens=[4000], rows_per_seg=[512], seed=5, ranges=less)
 
 
 @pytest.mark.parametrize("d", [128, 64])
@@ -721,9 +731,10 @@ def test_attention_decode_by_one_block_a_row_and_kv_head(monkeypatch, H, Hk, d, 
 
 
 def test_attention_decode_of_many_rows_takes_the_one_block_kernel_by_itself():
-    # 40 rows x 8 kv heads: above the threshold without forcing; contexts from 1 to 2,100 keys
-    lens = [1 + (i * 211) % 2100 for i in range(40)]
-    run_attention(H=16, Hk=8, d=64, P_=16, lens=lens, rows_per_seg=[1] * 40, seed=3)
+    # 40 rows x 8 kv heads: above the threshold without forcing; contexts from 1 to 1,024 keys, and longer ones of about
+    # one length (beyond: tests/test_attention_even_gpu.py)
+    for lens in ([1 + (i * 211) % 1024 for i in range(40)], [1800 + i for i in range(32)]):
+        run_attention(H=16, Hk=8, d=64, P_=16, lens=lens, rows_per_seg=[1] * len(lens), seed=3, entry="apc_attention_decode_bf16")
 
 
 def test_attention_finds_a_far_key_in_every_path(monkeypatch):

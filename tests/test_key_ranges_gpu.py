@@ -54,6 +54,8 @@ def test_every_number_of_ranges(monkeypatch, d, window):
     """Portions whose tiles see very different numbers of keys, some fewer than there are ranges."""
     from test_kernels_tuned import run_attention, tuned
     for s in range(1, 9):
-        monkeypatch.setattr(tuned(), "_key_splits_by_time", lambda *a, s=s: s)
-        monkeypatch.setattr(tuned(), "_key_splits", lambda *a, s=s: s)
-        run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500, 130, 77], rows_per_seg=[300, 129, 1], window=window, seed=s)
+        monkeypatch.setattr(tuned(), "_prompt_ranges", lambda *a, s=s: s)
+        run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500, 130, 77], rows_per_seg=[300, 129, 1], window=window, seed=s, ranges=s)
+        run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500, 130, 77], rows_per_seg=[300, 129, 1], window=window, seed=s, ranges=s,
+                      stale=float("nan"))
+        run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500], rows_per_seg=[256], window=window, seed=s, ranges=s, loud=(0, 1460, 40.0))
