@@ -92,7 +92,9 @@ __global__ __launch_bounds__(64) void paged_attention_plain_kernel(
 //   else     a block of four waves, a row each, one list after the other: many rows (prompts), where the number of
 //            loads is; waves that have no chunk would stand idle in the other form.
 // Measured, 32 heads of 64 on 8 kv heads, microseconds a layer (the kernel above): 4 rows at 101 to 907 keys 15 (259),
-// 340 rows of three prompts 33 (205).  Prompts on the SPREAD form: 73.
+// 340 rows of three prompts 33 (205).  Prompts on the SPREAD form: 73.  With heads over 64 in groups of 4 the SPREAD form
+// is 6 registers short and keeps them in scratch memory (32 heads of 128 on 8 kv heads, 4 rows at 100 to 900
+// keys: 33 us, 523 in the kernel above).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int LISTS = 8, ROWS_A_BLOCK = 4;
 

@@ -1345,9 +1345,10 @@ APC_EXPORT int apc_sample_rows_scratch_kib(int n_rows) {
 }
 
 // `cuts`: bit 0 set if some row may have top-k > 0, bit 1 if some row may have 0 <= top-p < 1, bit 2 if every row that
-// samples has 0 < top-k <= 1,024 (its survivors are then few, and the launches of top-p and of the draw fall away).
-// A caller that does not know its rows passes 3.  A row for which the caller's word is wrong still gets its token,
-// the slow way.
+// samples has 0 < top-k <= 1,024.  Bits 0 and 2 together take the two launches of sample_few_pieces_kernel and
+// sample_few_end_kernel, with or without top-p, and the working memory in carve_few's layout; everything else the
+// descents, in carve's.  A caller that does not know its rows passes 3.  A row for which the caller's word is wrong
+// still gets its token, the slow way.
 APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, const float* temperature,
                                const int* top_k, const float* top_p, const float* uniform, int* out, void* scratch,
                                size_t scratch_bytes, int cuts, hipStream_t stream) {
