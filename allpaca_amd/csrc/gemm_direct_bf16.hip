@@ -5,13 +5,14 @@
 // into a ring of registers, three steps of 32 columns ahead of their use.  The four waves of a block stand side by
 // side along N: each owns NF bands of 16 outputs and all 128 rows of the block, so no weight byte is loaded twice and
 // none crosses LDS.  The activations are shared by the four waves: they go from global memory into LDS with direct
-// loads (no registers in between), already in fragment order (a 16 x 32 fragment = one load instruction = 1 KiB
-// that a later ds_read_b128 returns lane by lane, free of bank conflicts), in four stages of 64 columns.
-// Per 64 columns a block moves 16 KiB of A and 8 NF KiB of W through the load path and reads 64 KiB from LDS, where
-// the 128 x 128 tile of gemm_bf16.hip moves 32 KiB and 96 KiB for half as many MFMAs (NF = 8).  At the shapes of a
-// 2,048-row step it waits for its loads: every block streams (128 + 64 NF) K 2 bytes through the L2, which the
-// counters show busy three quarters of the time or more; 60 % fewer requests to the L2 (four waves made to load
-// the same bands, timing only) bought 13 %, and the vendor library's products take about the same time.
+// loads (no registers in between), 8 rows x 64 columns an instruction, in four stages of 64 columns.  Such a load asks for
+// eight whole lines of 128 bytes; one that fetches an MFMA fragment as it is used (16 rows x 64 bytes) asks for sixteen
+// half lines, and those come out of L2 at 38 GB/s a compute unit where whole lines come at 131 (measured with loads alone,
+// 256 blocks over the same 2 MiB).  A lane takes the 16 bytes lane % 8 ^ row of its row, so that the later ds_read_b128 of
+// a fragment finds its rows in different banks.  With whole lines instead of fragments 2,048 rows x 4,096 columns of K into
+// 3,072 / 4,096 / 6,144 / 8,192 bfloat16 outputs (NF 3, 4, 6, 8) went from 60 / 68 / 89 / 112 to 50 / 59 / 81 / 102 us.
+// What bounds it now: with every load in the first-level cache (timing only) the four take 41 / 51 / 72 / 92 us; loads
+// further ahead (7 steps of W, 6 stages of A), fragments read 7 groups ahead or not read at all change nothing.
 //
 // The accumulators (8 row groups x NF bands x 4 registers) live in the accumulation registers; the MFMA is written as
 // an instruction with that register class, because left to itself the compiler moved accumulators between the two
@@ -130,10 +131,12 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
   int woff[NF];  // SwiGLU: NOUT gate bands, then the same bands of up
 #pragma unroll
   for (int f = 0; f < NF; ++f) woff[f] = (min(band0 + f % NOUT, bands - 1) - base_band) * chunks * 1024 + lane * 16;
-  int aoff[NP / 2];  // this wave's row groups wave * NP / 2 + j: lane -> (row lane % 16, 8 columns lane / 16)
+  // This wave's pieces of A in a stage, 8 rows x 64 columns each: lane -> (row lane / 8, 16 bytes lane % 8 ^ row), so that
+  // an instruction asks for eight whole lines of 128 bytes
+  int aoff[NP];
 #pragma unroll
-  for (int j = 0; j < NP / 2; ++j)
-    aoff[j] = (min(m0 + (wave * (NP / 2) + j) * 16 + lane % 16, M - 1) - m0) * lda * 2 + (lane / 16) * 16;
+  for (int p = 0; p < NP; ++p)
+    aoff[p] = (min(m0 + (wave * NP + p) * 8 + lane / 8, M - 1) - m0) * lda * 2 + ((lane % 8) ^ (lane / 8)) * 16;
 
   floatx4 acc[BMG][NF];
 #pragma unroll
@@ -143,9 +146,13 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
 
   const int ktiles = K / 64;
   auto a_piece = [&](int kt, int p) {  // piece p (0..NP-1) of this wave's share of stage kt
-    const int j = p / 2, c = p % 2;
-    load_to_lds(abuf, &As[kt % S][(wave * (NP / 2) + j) * 2 + c][0], aoff[j], min(kt, ktiles - 1) * 128 + c * 64);
+    load_to_lds(abuf, &As[kt % S][wave * NP + p][0], aoff[p], min(kt, ktiles - 1) * 128);
   };
+  // where a lane finds row lane % 16, columns c * 32 + (lane / 16) * 8 .. + 7 of a row group
+  int roff[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    roff[c] = (lane % 16) * 128 + (((c * 4 + lane / 16) ^ (lane % 8)) * 16);
   Frag ring[R][NF];
   auto w_piece = [&](int slot, int q, int f) {  // band f of step q (32 columns)
     ring[slot][f] = load_frag_buffer((is_swiglu(MODE) && f >= NOUT) ? ubuf : wbuf, woff[f],
@@ -177,10 +184,10 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
       wait_loads_but<NVM>();             // this wave's pieces of the stage are in LDS ...
       __builtin_amdgcn_s_barrier();      // ... and so are the other waves'; all have left the stage before
       __builtin_amdgcn_sched_barrier(0);
-      const unsigned char* abase = &As[stage % S][0][lane * 16];
+      const unsigned char* abase = &As[stage % S][0][0];
       Frag fa[PA + 1];  // group g reads fragment (row group g % BMG, chunk g / BMG)
 #pragma unroll
-      for (int g = 0; g < PA; ++g) fa[g] = *reinterpret_cast<const Frag*>(abase + g * 2048);
+      for (int g = 0; g < PA; ++g) fa[g] = *reinterpret_cast<const Frag*>(abase + roff[0] + g * 2048);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -189,7 +196,7 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
         const int into = (2 * u + c + LEAD) % R;   // slot of the step LEAD ahead: the step before this one has left it
         if (g + PA < G)
           fa[(g + PA) % (PA + 1)] =
-              *reinterpret_cast<const Frag*>(abase + ((g + PA) % BMG) * 2048 + ((g + PA) / BMG) * 1024);
+              *reinterpret_cast<const Frag*>(abase + roff[(g + PA) / BMG] + ((g + PA) % BMG) * 2048);
         if (g < NP) a_piece(stage + S - 1, g);     // into the stage that every wave left at the barrier above
 #pragma unroll
         for (int f = 0; f < NF; ++f)
@@ -368,13 +375,13 @@ __global__ __launch_bounds__(256, 1) void gemm_direct_slices_kernel(const bf16_t
 }
 
 // Which NF takes a shape: a launch runs ceil(blocks / 256) rounds of one block a compute unit, and a round of blocks
-// with NF bands a wave takes about 27 + 10.8 NF time units (measured at 2,048 rows with weights from HBM: 58, 74, 86, 92
-// and 112 us a round of 4,096 columns of K for NF = 3, 4, 5, 6, 8); 3 and 5 bands give the 3,072 and 5,120 columns of
+// with NF bands a wave takes about 19 + 10.4 NF time units (measured at 2,048 rows with weights from HBM: 50, 59, 81 and
+// 102 us a round of 4,096 columns of K for NF = 3, 4, 6, 8); 3 and 5 bands give the 3,072 and 5,120 columns of
 // a 3B model one full round.
 // (Tried and taken out: one launch in which the columns of a nearly empty last round go to tiles of 64 rows.  With
 // 2,048 rows x 14,336 SwiGLU outputs, 3.5 rounds of 128-row tiles, it took 589 us against 453 us: a 64-row tile moves
 // 72 KiB through the load path per 64 columns of K for half the MFMAs.)
-constexpr double round_cost(int nf) { return 27.0 + 10.8 * nf; }
+constexpr double round_cost(int nf) { return 19.0 + 10.4 * nf; }
 int pick_bands(int M, int N, bool swiglu, int k_split = 1, double* cost_out = nullptr) {
   const int mt = ceil_div(M, 128);
   int best = 0;
