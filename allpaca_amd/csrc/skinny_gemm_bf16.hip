@@ -7,8 +7,13 @@
 //  * a block owns NB bands (16 NB output columns) and all of K; each of its WPB waves takes a contiguous
 //    range of K and reads it in steps of 4 tiles per band: every load of W is 1 KiB of consecutive bytes and a
 //    wave walks forward through one region of memory;
-//  * the activations are the other operand (row m = lane % 16, 16 bytes of k per lane), loaded once per step
-//    for all NB bands: D[n][m], so a lane ends with 4 consecutive n of one row m (SwiGLU: steps of 2 tiles);
+//  * the activations are the other operand, D[n][m], loaded once per step for all NB bands, so a lane ends with 4
+//    consecutive n of one row m (SwiGLU: steps of 2 tiles).  One load takes 8 rows x 64 columns, whole lines of 128 bytes,
+//    for a pair of tiles: lanes 0-7 of 16 hold the rows' part of the first tile, lanes 8-15 of the second.  Both tiles
+//    are multiplied with it; the first one's sums count in columns 0-7 of the result, the second one's in 8-15, and
+//    they are added at the end (9-16 rows: two groups of 8, the same sums).  Operands of 16 rows x 32 columns, as the
+//    instruction takes them, are half lines, which come out of L2 at a third of the rate, and with up to 8 rows half of
+//    them repeat a row: a step of one row at 1B shapes 743 -> 727 us, of 8 rows at 8B shapes 3.39 -> 3.32 ms;
 //  * the loads of the next step are in flight while the current one is multiplied (two register sets that
 //    swap roles; no branch around a load in the steady state);
 //  * the waves' partial sums are added in wave order through LDS, then the epilogue runs: store (bfloat16 or
@@ -31,11 +36,22 @@ constexpr int TILE_ELEMS = 16 * 32;  // elements of a tile
 
 enum { SK_STORE_BF16 = 0, SK_STORE_F32 = 1, SK_ACC_F32 = 2, SK_SWIGLU = 3, SK_QKV_ROPE = 4, SK_ACT = 5 };
 
-template <int MT, int NB, int U>
+template <int MG, int NB, int U>
 struct SkRegs {
   Frag w[NB][U];
-  Frag a[MT][U];
+  Frag a[MG][U / 2];
 };
+
+// what lane l ^ 8 holds
+__device__ __forceinline__ floatx4 eight_lanes_on(const floatx4& v) {
+  floatx4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float x = v[r];  // (a bit cast of the element itself takes element 0)
+    o[r] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x128, 0xf, 0xf, true));  // row_ror:8
+  }
+  return o;
+}
 
 // NB: weight bands per block (for SwiGLU: 2 = one gate band and the up band of the same outputs)
 // What the folded norm needs.  ss: sums of x^2 per row and band, [16 rows][ld_ss] floats, ld_ss = n_ss rounded up
@@ -77,7 +93,7 @@ struct SkRope {
 constexpr int sk_step(int mode) { return mode == SK_SWIGLU ? 2 : SK_U; }
 constexpr int sk_blocks(int mode, int wpb) { return (mode == SK_SWIGLU && wpb == 8) ? 2 : 1; }
 
-template <int MT, int MODE, int NB, int WPB, bool PRE, bool EMIT>
+template <int MG, int MODE, int NB, int WPB, bool PRE, bool EMIT>
 __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda,
                                                                const bf16_t* __restrict__ W,
                                                                const bf16_t* __restrict__ W2, int chunks,
@@ -87,10 +103,11 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
   static_assert(!EMIT || MODE == SK_ACC_F32, "only a product that adds into the residual emits the next norm's row");
   static_assert(!PRE || MODE != SK_ACC_F32, "a product that reads a normalised row stores its result");
   constexpr int U = sk_step(MODE);
-  static_assert(MT == 1, "written for one tile of rows (the finishing wave's early loads, the folded norm)");
-  __shared__ float red[WPB * NB * MT * 256];
-  __shared__ float row_ss[WPB * MT * 16];
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  static_assert(MG == 1 || MG == 2, "one or two groups of 8 rows");
+  static_assert(U % 2 == 0, "activations come two tiles at a time");
+  __shared__ float red[WPB * NB * 256];
+  __shared__ float row_ss[WPB * 16];
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int i = lane % 16, c = lane / 16;
   constexpr int OUT_BANDS = (MODE == SK_SWIGLU || MODE == SK_QKV_ROPE) ? 1 : NB;
   const int band0 = blockIdx.x * OUT_BANDS;
@@ -117,31 +134,35 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
       wb[b] = W + (size_t)(qkv_head * (rope.d / 16) + blockIdx.x % (rope.d / 32) + b * (rope.d / 32)) * chunks * TILE_ELEMS + lane * 8;
     else wb[b] = W + (size_t)min(band0 + b, bands - 1) * chunks * TILE_ELEMS + lane * 8;
   }
-  const bf16_t* arow[MT];
+  // row group g: lanes i < 8 take row g * 8 + i of a pair's first tile, lanes i >= 8 row g * 8 + i - 8 of its second
+  uint32_t arow[MG];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) arow[mt] = A + (size_t)min(mt * 16 + i, M - 1) * lda + c * 8;
+  for (int g = 0; g < MG; ++g) arow[g] = (uint32_t)min(g * 8 + i % 8, M - 1) * (uint32_t)lda + (i / 8) * 32 + c * 8;
 
-  floatx4 acc[NB][MT];
+  // acc[b][g][t]: the tiles t of the pairs; of its 16 columns the group's rows are those of the lanes i / 8 == t
+  floatx4 acc[NB][MG][2];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[b][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  auto load_step = [&](SkRegs<MT, NB, U>& r, int ch) {  // tiles ch .. ch+3, all inside K
+    for (int g = 0; g < MG; ++g) acc[b][g][0] = acc[b][g][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto load_step = [&](SkRegs<MG, NB, U>& r, int ch) {  // tiles ch .. ch + U - 1, all inside K
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int b = 0; b < NB; ++b) r.w[b][u] = load_frag_once(wb[b] + (size_t)(ch + u) * TILE_ELEMS);
+      if (u % 2 == 0) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) r.a[mt][u] = load_frag(arow[mt] + (ch + u) * 32);
+        for (int g = 0; g < MG; ++g) r.a[g][u / 2] = load_frag(A + (ch + u) * 32 + arow[g]);
+      }
     }
   };
-  auto compute = [&](const SkRegs<MT, NB, U>& r) {
+  auto compute = [&](const SkRegs<MG, NB, U>& r) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int g = 0; g < MG; ++g)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b][mt] = mfma16(r.w[b][u], r.a[mt][u], acc[b][mt]);
+        for (int b = 0; b < NB; ++b) acc[b][g][u % 2] = mfma16(r.w[b][u], r.a[g][u / 2], acc[b][g][u % 2]);
   };
 
   // this wave's range of tiles along K: [c_lo, c_hi); steps of 4 whole tiles, then single tiles
@@ -152,7 +173,7 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
   const int nsteps = c_full_hi > c_lo ? (c_full_hi - c_lo) / U : 0;
   // Steps are loaded two ahead (register sets r0, r1 take turns); no branch lies around a load in the steady loop,
   // so the waits for one set never wait for the other.
-  SkRegs<MT, NB, U> r0, r1;
+  SkRegs<MG, NB, U> r0, r1;
   if (nsteps > 0) load_step(r0, c_lo);
   if (nsteps > 1) load_step(r1, c_lo + U);
   // Behind the first loads of the stream, and needed only at the end: the sums of x^2 that the emitting product
@@ -161,22 +182,26 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
   float ss_piece = 0.f;
   if constexpr (PRE) {
     const int groups = norm.ld_ss / 4;
-    floatx4 v[SS_LOADS];
+    constexpr int AT_ONCE = MG == 1 ? SS_LOADS : SS_LOADS / 4;   // (two groups' steps leave registers for few)
 #pragma unroll
-    for (int j = 0; j < SS_LOADS; ++j) {
-      const int q = wave * 4 + c + j * WPB * 4;
-      v[j] = q < groups ? *reinterpret_cast<const floatx4*>(norm.ss + (size_t)i * norm.ld_ss + q * 4)
-                        : floatx4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int j0 = 0; j0 < SS_LOADS; j0 += AT_ONCE) {
+      floatx4 v[AT_ONCE];
 #pragma unroll
-    for (int j = 0; j < SS_LOADS; ++j) {
-      const int q = wave * 4 + c + j * WPB * 4;
+      for (int j = 0; j < AT_ONCE; ++j) {
+        const int q = wave * 4 + c + (j0 + j) * WPB * 4;
+        v[j] = q < groups ? *reinterpret_cast<const floatx4*>(norm.ss + (size_t)i * norm.ld_ss + q * 4)
+                          : floatx4{0.f, 0.f, 0.f, 0.f};
+      }
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (q * 4 + e < norm.n_ss) ss_piece += v[j][e];
+      for (int j = 0; j < AT_ONCE; ++j) {
+        const int q = wave * 4 + c + (j0 + j) * WPB * 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (q * 4 + e < norm.n_ss) ss_piece += v[j][e];
+      }
     }
   }
-  constexpr int ITEMS = OUT_BANDS * MT;  // (band, m-tile) pairs to finish: wave w finishes pair w
+  constexpr int ITEMS = OUT_BANDS;  // bands to finish: wave w finishes band w
   const int fin_n = (band0 + wave) * 16 + c * 4;  // first of this lane's 4 columns if this wave finishes a band
   const bool fin_vec = vec_c && wave < ITEMS && i < M && fin_n + 3 < N;
   floatx4 c_old = floatx4{0.f, 0.f, 0.f, 0.f}, g_next = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -212,15 +237,24 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
     if (rem >= 2) compute(r1);
     if (rem == 3) compute(r0);
   }
-  // what is left of the range: single tiles; the last one may be cut by K (K is a multiple of 8, so a lane's
-  // 16 bytes of activations are inside or outside as a whole; W is zero beyond K)
-  for (int ch = c_lo + nsteps * U; ch < c_hi; ++ch) {
-    const bool in = ch * 32 + c * 8 < K;
+  // Both tiles' sums of a row, in the lane i of the row
+  floatx4 row[NB];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const Frag af = in ? load_frag(arow[mt] + ch * 32) : zero_frag();
+  for (int b = 0; b < NB; ++b) {
+    row[b] = acc[b][0][0] + eight_lanes_on(acc[b][0][1]);
+    if constexpr (MG == 2) {
+      const floatx4 second = eight_lanes_on(acc[b][1][0]) + acc[b][1][1];
+      if (i >= 8) row[b] = second;
+    }
+  }
+  // what is left of the range: single tiles, row i in the lanes i; the last one may be cut by K (K is a multiple of 8, so
+  // a lane's 16 bytes of activations are inside or outside as a whole; W is zero beyond K)
+  if (c_lo + nsteps * U < c_hi) {
+    const bf16_t* rest = A + (size_t)min(i, M - 1) * lda + c * 8;
+    for (int ch = c_lo + nsteps * U; ch < c_hi; ++ch) {
+      const Frag af = ch * 32 + c * 8 < K ? load_frag(rest + ch * 32) : zero_frag();
 #pragma unroll
-      for (int b = 0; b < NB; ++b) acc[b][mt] = mfma16(load_frag_once(wb[b] + (size_t)ch * TILE_ELEMS), af, acc[b][mt]);
+      for (int b = 0; b < NB; ++b) row[b] = mfma16(load_frag_once(wb[b] + (size_t)ch * TILE_ELEMS), af, row[b]);
     }
   }
 
@@ -230,11 +264,9 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
     if (c == 0) row_ss[wave * 16 + i] = ss_piece;
   }
   // partial sums of the waves, added in wave order
-  float* mine = red + wave * (NB * MT * 256);
+  float* mine = red + wave * (NB * 256);
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) *reinterpret_cast<floatx4*>(&mine[((b * MT + mt) * 64 + lane) * 4]) = acc[b][mt];
+  for (int b = 0; b < NB; ++b) *reinterpret_cast<floatx4*>(&mine[(b * 64 + lane) * 4]) = row[b];
   __syncthreads();
 
   constexpr int NSUM = (MODE == SK_SWIGLU || MODE == SK_QKV_ROPE) ? 2 : 1;
@@ -247,7 +279,7 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
       sum[s] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < WPB; ++w)
-        sum[s] += *reinterpret_cast<const floatx4*>(&red[w * (NB * MT * 256) + (bb * MT * 64 + lane) * 4]);
+        sum[s] += *reinterpret_cast<const floatx4*>(&red[w * (NB * 256) + (bb * 64 + lane) * 4]);
     }
     const int m = i;  // D[n][m]: this lane holds row m = lane % 16 of the tile and columns fin_n .. fin_n + 3
     if constexpr (PRE) {
@@ -381,7 +413,8 @@ static int launch_skinny(const bf16_t* A, int lda, const bf16_t* W, const bf16_t
   int vec_c = ldc % 4 == 0 && ((uintptr_t)C % (4 * elem)) == 0;
   if (EMIT) vec_c = vec_c && norm.ld_raw % 4 == 0 && ((uintptr_t)norm.raw % 8) == 0 && aligned16(norm.g);
 #define SK_LAUNCH(NB_, WPB_)                                                                                  \
-  hipLaunchKernelGGL((skinny_gemm_kernel<1, MODE, NB_, WPB_, PRE, EMIT>),                                     \
+  hipLaunchKernelGGL((M <= 8 ? skinny_gemm_kernel<1, MODE, NB_, WPB_, PRE, EMIT>                              \
+                             : skinny_gemm_kernel<2, MODE, NB_, WPB_, PRE, EMIT>),                            \
                      dim3(ceil_div(bands, MODE == SK_SWIGLU ? 1 : NB_)), dim3(WPB_ * WAVE), 0, stream, A, lda, W, \
                      W2, chunks, C, ldc, M, N, K, norm, vec_c, rope)
   if constexpr (MODE == SK_SWIGLU || MODE == SK_QKV_ROPE) {
@@ -403,7 +436,7 @@ static int launch_skinny(const bf16_t* A, int lda, const bf16_t* W, const bf16_t
 }
 
 static bool operands_ok(const void* A, int lda, const void* W, int M, int K) {
-  return M <= 16 && K % 8 == 0 && lda % 8 == 0 && aligned16(A) && aligned16(W);
+  return M <= 16 && K % 8 == 0 && lda % 8 == 0 && lda < (1 << 28) && aligned16(A) && aligned16(W);  // (32-bit offsets of 16 rows)
 }
 
 // W: tiled layout of an [N, K] matrix.  mode: 0 store bfloat16, 1 store float32, 2 add into float32, 17 .. 19: an
