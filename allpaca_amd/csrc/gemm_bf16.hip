@@ -396,47 +396,125 @@ struct FinishNorm {
   int act = 0;      // mode G_ACT: the activation
 };
 
+// How the finishing kernels below go over a row: a wave takes 256 columns of it, a lane four of them, in one piece of 16
+// bytes (VEC: N and the row strides multiples of 4, everything aligned) or, otherwise, 64 columns apart.  Nothing crosses a
+// wave, so there is no barrier, and up to four slices' loads are in flight.  Bound by the slices' bytes: 512 rows x 4,096
+// columns in four slices, added into the residual with the norm's row left, 54 MB in 10.1 us (a thread a column and a
+// block 256 columns of a row: two slices, 38 MB, in 11.5).
+constexpr int FIN_COLS = 256;
+template <bool VEC, int LANES = WAVE>
+__device__ __forceinline__ int fin_column(int first, int lane, int j) { return VEC ? first + lane * 4 + j : first + j * LANES + lane; }
+
+// A lane's four sums over the slices, in slice order; 0 beyond N.  LANES: lanes that share the row's piece
+template <bool VEC, int LANES = WAVE>
+__device__ __forceinline__ floatx4 fin_sum(const float* __restrict__ row, size_t plane, int k_split, int first, int lane, int N) {
+  floatx4 g = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < k_split; s0 += 4) {
+    floatx4 v[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      v[s] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (s0 + s < k_split) {
+        const float* src = row + (size_t)(s0 + s) * plane;
+        if constexpr (VEC) {
+          if (first + lane * 4 < N) v[s] = *reinterpret_cast<const floatx4*>(src + first + lane * 4);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (fin_column<VEC, LANES>(first, lane, j) < N) v[s][j] = src[fin_column<VEC, LANES>(first, lane, j)];
+        }
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s0 + s < k_split) g += v[s];
+  }
+  return g;
+}
+
+// 1 / sqrt(mean of x^2 + eps) of row m, from up to 256 sums of x^2
+__device__ __forceinline__ float fin_rstd(const FinishNorm& norm, int m, int lane, int K) {
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int p = j * WAVE + lane;
+    if (p < norm.pre_parts) sum += norm.pre_ss[(size_t)m * norm.pre_parts + p];
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o /= 2) sum += __shfl_xor(sum, o, WAVE);
+  return 1.0f / sqrtf(sum / (float)K + norm.eps);
+}
+
+template <bool VEC>
+__device__ __forceinline__ void fin_store_bf16(bf16_t* row, int first, int lane, int N, const floatx4& y) {
+  if constexpr (VEC) {
+    if (first + lane * 4 < N) {
+      uint2 o;
+      o.x = pack_bf16x2(y[0], y[1]);
+      o.y = pack_bf16x2(y[2], y[3]);
+      *reinterpret_cast<uint2*>(row + first + lane * 4) = o;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (fin_column<VEC>(first, lane, j) < N) row[fin_column<VEC>(first, lane, j)] = float_to_bf16(y[j]);
+  }
+}
+template <bool VEC>
+__device__ __forceinline__ void fin_store_f32(float* row, int first, int lane, int N, const floatx4& y) {
+  if constexpr (VEC) {
+    if (first + lane * 4 < N) *reinterpret_cast<floatx4*>(row + first + lane * 4) = y;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (fin_column<VEC>(first, lane, j) < N) row[fin_column<VEC>(first, lane, j)] = y[j];
+  }
+}
+
 // Sums the float32 sums that G_PARTIAL blocks left ([which][slice][M][N], slices in order) and finishes:
-// store bfloat16 / float32, add into a float32 residual, or SwiGLU of the two matrices' sums.
-template <bool PRE, bool EMIT>
+// store bfloat16 / float32, add into a float32 residual, an activation, or SwiGLU of the two matrices' sums.
+template <bool PRE, bool EMIT, bool VEC>
 __global__ __launch_bounds__(256) void gemm_finish_kernel(const float* __restrict__ partials, int k_split, int M, int N,
                                                           int K, int mode, void* __restrict__ C, int ldc,
                                                           FinishNorm norm) {
-  __shared__ float red[4];
-  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
-  const bool on = n < N;
-  float rstd = 1.f;
-  if constexpr (PRE) {  // pre_parts <= 256: one value a thread, added in a fixed order
-    const float v = threadIdx.x < norm.pre_parts ? norm.pre_ss[(size_t)m * norm.pre_parts + threadIdx.x] : 0.f;
-    rstd = 1.0f / sqrtf(block_sum<256>(v, red) / (float)K + norm.eps);
-  }
+  const int parts = ceil_div(N, FIN_COLS);
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int m = blockIdx.y, part = blockIdx.x * 4 + wave, first = part * FIN_COLS;
+  if (part >= parts) return;
   const size_t plane = (size_t)M * N;
-  const float* src = partials + (size_t)m * N + (on ? n : 0);
-  float g = 0.f;
-  for (int s = 0; s < k_split; ++s) g += src[s * plane];
-  g *= rstd;
-  const size_t o = (size_t)m * ldc + n;
-  float sq = 0.f;
-  if (on) {
-    if (mode == G_STORE_BF16) ((bf16_t*)C)[o] = float_to_bf16(g);
-    else if (mode == G_ACT) ((bf16_t*)C)[o] = float_to_bf16(activation_f(g, norm.act));
-    else if (mode == G_STORE_F32) ((float*)C)[o] = g;
-    else if (mode == G_ACC_F32) {
-      const float x = ((float*)C)[o] + g;
-      ((float*)C)[o] = x;
-      if constexpr (EMIT) {
-        norm.raw[(size_t)m * norm.ld_raw + n] = float_to_bf16(x * norm.g[n]);
-        sq = x * x;
-      }
-    } else {
-      float u = 0.f;
-      for (int s = 0; s < k_split; ++s) u += src[(k_split + s) * plane];
-      ((bf16_t*)C)[o] = float_to_bf16(silu_f(g) * (u * rstd));
+  const float* src = partials + (size_t)m * N;
+  floatx4 old = floatx4{0.f, 0.f, 0.f, 0.f}, gv = floatx4{0.f, 0.f, 0.f, 0.f};  // the residual, the next norm's weight
+  if (mode == G_ACC_F32) old = fin_sum<VEC>((const float*)C + (size_t)m * ldc, 0, 1, first, lane, N);
+  if constexpr (EMIT) gv = fin_sum<VEC>(norm.g, 0, 1, first, lane, N);
+  floatx4 g = fin_sum<VEC>(src, plane, k_split, first, lane, N);
+  const float rstd = PRE ? fin_rstd(norm, m, lane, K) : 1.f;
+  if constexpr (PRE) g *= rstd;
+  bf16_t* out16 = (bf16_t*)C + (size_t)m * ldc;
+  float* out32 = (float*)C + (size_t)m * ldc;
+  if (mode == G_STORE_BF16) {
+    fin_store_bf16<VEC>(out16, first, lane, N, g);
+  } else if (mode == G_ACT) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) g[j] = activation_f(g[j], norm.act);
+    fin_store_bf16<VEC>(out16, first, lane, N, g);
+  } else if (mode == G_STORE_F32) {
+    fin_store_f32<VEC>(out32, first, lane, N, g);
+  } else if (mode == G_ACC_F32) {
+    const floatx4 x = old + g;
+    fin_store_f32<VEC>(out32, first, lane, N, x);
+    if constexpr (EMIT) {
+      fin_store_bf16<VEC>(norm.raw + (size_t)m * norm.ld_raw, first, lane, N, x * gv);
+      float sq = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];   // (0 beyond N)
+#pragma unroll
+      for (int o = WAVE / 2; o > 0; o /= 2) sq += __shfl_xor(sq, o, WAVE);
+      if (lane == 0) norm.emit_ss[(size_t)m * parts + part] = sq;
     }
-  }
-  if constexpr (EMIT) {
-    const float total = block_sum<256>(sq, red);
-    if (threadIdx.x == 0) norm.emit_ss[(size_t)m * gridDim.x + blockIdx.x] = total;
+  } else {
+    floatx4 u = fin_sum<VEC>(src + (size_t)k_split * plane, plane, k_split, first, lane, N);
+    if constexpr (PRE) u *= rstd;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) g[j] = silu_f(g[j]) * u[j];
+    fin_store_bf16<VEC>(out16, first, lane, N, g);
   }
 }
 
@@ -472,35 +550,6 @@ static int launch_partials(const void* A, int lda, const void* W, const void* Wu
   return 0;
 }
 
-// The plain finishing steps (no folded norm, no SwiGLU) four outputs a thread: the slices added in order, then stored
-// or added into the residual.  N and ldc multiples of 4, 16-byte aligned rows.  (One output a thread takes 34 us for
-// 2,048 x 4,096 outputs in two slices, this 13.)
-__global__ __launch_bounds__(256) void gemm_finish4_kernel(const float* __restrict__ partials, int k_split, int M, int N,
-                                                           int mode, void* __restrict__ C, int ldc, int act) {
-  const int n4 = N / 4;
-  const size_t total = (size_t)M * n4, plane = (size_t)M * N;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-    const int m = (int)(i / n4), n = (int)(i % n4) * 4;
-    const float* src = partials + (size_t)m * N + n;
-    floatx4 g = *reinterpret_cast<const floatx4*>(src);
-    for (int s = 1; s < k_split; ++s) g += *reinterpret_cast<const floatx4*>(src + s * plane);
-    const size_t o = (size_t)m * ldc + n;
-    if (mode == G_ACT)
-      for (int k = 0; k < 4; ++k) g[k] = activation_f(g[k], act);
-    if (mode == G_STORE_BF16 || mode == G_ACT) {
-      uint2 pk;
-      pk.x = pack_bf16x2(g[0], g[1]);
-      pk.y = pack_bf16x2(g[2], g[3]);
-      *reinterpret_cast<uint2*>((bf16_t*)C + o) = pk;
-    } else if (mode == G_STORE_F32) {
-      *reinterpret_cast<floatx4*>((float*)C + o) = g;
-    } else {
-      floatx4* dst = reinterpret_cast<floatx4*>((float*)C + o);
-      *dst = *dst + g;
-    }
-  }
-}
-
 static int launch_splitk(const void* A, int lda, const void* W, const void* Wu, void* C, int ldc, int M, int N, int K,
                          int mode, int k_split, float* workspace, int pre, int emit, FinishNorm norm,
                          hipStream_t stream) {
@@ -516,21 +565,20 @@ static int launch_splitk(const void* A, int lda, const void* W, const void* Wu, 
   if ((mode == G_SWIGLU) != (Wu != nullptr)) return APC_ERR_BAD_ARG;
   const int e = launch_partials(A, lda, W, Wu, M, N, K, k_split, workspace, stream);
   if (e) return e;
-  if (!pre && !emit && mode != G_SWIGLU && N % 4 == 0 && ldc % 4 == 0 && aligned16(C) && (long)M * N >= (1L << 20)) {
-    const long want = ((long)M * (N / 4) + 255) / 256;
-    hipLaunchKernelGGL(gemm_finish4_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, stream, workspace,
-                       k_split, M, N, mode, C, ldc, norm.act);
-    APC_LAUNCH_CHECK();
-    return 0;
-  }
-  const dim3 grid(ceil_div(N, 256), M);
-#define FINISH(PRE_, EMIT_)                                                                                     \
-  hipLaunchKernelGGL((gemm_finish_kernel<PRE_, EMIT_>), grid, dim3(256), 0, stream, workspace, k_split, M, N, K, mode, \
-                     C, ldc, norm)
-  if (pre) FINISH(true, false);
-  else if (emit) FINISH(false, true);
-  else FINISH(false, false);
+  const bool out16 = mode == G_STORE_BF16 || mode == G_SWIGLU || mode == G_ACT;
+  bool vec = N % 4 == 0 && ldc % 4 == 0 && aligned16(workspace) && ((uintptr_t)C & (out16 ? 7u : 15u)) == 0;
+  if (emit) vec = vec && aligned16(norm.g) && norm.ld_raw % 4 == 0 && ((uintptr_t)norm.raw & 7u) == 0;
+#define FINISH_AS(PRE_, EMIT_, VEC_)                                                                                 \
+  hipLaunchKernelGGL((gemm_finish_kernel<PRE_, EMIT_, VEC_>), dim3(ceil_div(N, 4 * FIN_COLS), M), dim3(256), 0, stream, \
+                     workspace, k_split, M, N, K, mode, C, ldc, norm)
+#define FINISH(PRE_, EMIT_)                \
+  if (vec) FINISH_AS(PRE_, EMIT_, true);   \
+  else FINISH_AS(PRE_, EMIT_, false)
+  if (pre) { FINISH(true, false); }
+  else if (emit) { FINISH(false, true); }
+  else { FINISH(false, false); }
 #undef FINISH
+#undef FINISH_AS
   APC_LAUNCH_CHECK();
   return 0;
 }
@@ -538,8 +586,11 @@ static int launch_splitk(const void* A, int lda, const void* W, const void* Wu, 
 // Finishing kernel of the product for q, k and v (K in slices): it adds the slices, scales them if the row came from
 // a product that left the norm's row (PRE), rounds to bfloat16 as a stored result would be, rotates q and k by the
 // row's position (whole heads, pairs (e, e + d/2)) and writes k and v into the paged cache: what the product's
-// finishing kernel and the kernel for rotation and cache write would do one after the other.  A block has 256
-// columns of one row, which are whole heads (256 is a multiple of d): a value meets its partner through LDS.
+// finishing kernel and the kernel for rotation and cache write would do one after the other.  The first blocks take q and
+// k, a wave 256 columns of one row, which are whole heads (256 is a multiple of d): a value meets its partner through LDS.
+// The others take v, 16 rows x 64 columns a block: the cache has a column's values of consecutive positions side by side,
+// and 16 lanes with one column of the 16 rows write them as 32 bytes in one or two pages.  (With one row a wave the bytes of a
+// sector come from different waves: 512 rows of 6,144 columns in two slices 17.5 us, so 12.5.)
 struct FinishRope {
   const float* cos_sin;    // [positions][2][d / 2]
   const int* positions;    // [M]
@@ -550,46 +601,93 @@ struct FinishRope {
   int P, H, Hk, d;
 };
 
-template <bool PRE>
+constexpr int FIN_V_ROWS = 16, FIN_V_COLS = 64;
+
+template <bool PRE, bool VEC>
 __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* __restrict__ partials, int k_split, int M,
                                                                    int N, int K, bf16_t* __restrict__ q_out, int ldq,
-                                                                   FinishNorm norm, FinishRope rope) {
-  __shared__ float red[4];
-  __shared__ float vals[256];
-  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
-  const bool on = n < N;
-  float rstd = 1.f;
-  if constexpr (PRE) {
-    const float v = threadIdx.x < norm.pre_parts ? norm.pre_ss[(size_t)m * norm.pre_parts + threadIdx.x] : 0.f;
-    rstd = 1.0f / sqrtf(block_sum<256>(v, red) / (float)K + norm.eps);
-  }
-  const size_t plane = (size_t)M * N;
-  const float* src = partials + (size_t)m * N + (on ? n : 0);
-  float g = 0.f;
-  for (int s = 0; s < k_split; ++s) g += src[s * plane];
-  const float x = bf16_to_float(float_to_bf16(g * rstd));
-  vals[threadIdx.x] = x;
-  __syncthreads();
-  if (!on) return;
-  const int d = rope.d, half = d / 2, head = n / d, e = n % d;
-  const int pos = rope.positions[m];
-  bf16_t* page = rope.cache + (size_t)rope.block_table[(size_t)rope.row_seg[m] * rope.max_blocks + pos / rope.P] *
-                                  ((size_t)2 * rope.Hk * rope.P * d);
-  const int slot = pos % rope.P;
-  if (head < rope.H + rope.Hk) {
-    const float* cs = rope.cos_sin + (size_t)pos * d;
-    float y;
-    if (e < half) {
-      const float av = x, bv = vals[threadIdx.x + half], c = cs[e], sn = cs[half + e];
-      y = av * c - bv * sn;
-    } else {
-      const float av = vals[threadIdx.x - half], bv = x, c = cs[e - half], sn = cs[e];
-      y = av * sn + bv * c;
+                                                                   FinishNorm norm, FinishRope rope, int qk_blocks) {
+  __shared__ __attribute__((aligned(16))) float vals[4][FIN_COLS];
+  static_assert(FIN_V_ROWS * FIN_V_COLS == 4 * FIN_COLS, "both kinds of block hold 1,024 values");
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int d = rope.d, half = d / 2, qk = (rope.H + rope.Hk) * d;  // columns of q and k
+  const size_t plane = (size_t)M * N, page_elems = (size_t)2 * rope.Hk * rope.P * d;
+  if ((int)blockIdx.x >= qk_blocks) {
+    const int b = blockIdx.x - qk_blocks, tiles = ceil_div(N - qk, FIN_V_COLS);
+    const int row0 = b / tiles * FIN_V_ROWS, col0 = qk + b % tiles * FIN_V_COLS;
+    // 16 lanes a row, four columns a lane
+    const int r = threadIdx.x / 16, m = row0 + r, l16 = threadIdx.x % 16;
+    const int sr = threadIdx.x % 16, sm = row0 + sr;                   // the row that this lane stores
+    int pos = 0, seg = 0;
+    if (sm < M) pos = rope.positions[sm], seg = rope.row_seg[sm];
+    floatx4 g = floatx4{0.f, 0.f, 0.f, 0.f};
+    float sum = 0.f;
+    if (m < M) {
+      g = fin_sum<VEC, 16>(partials + (size_t)m * N, plane, k_split, col0, l16, N);
+      if constexpr (PRE)
+        for (int p = l16; p < norm.pre_parts; p += 16) sum += norm.pre_ss[(size_t)m * norm.pre_parts + p];
     }
-    if (head < rope.H) q_out[(size_t)m * ldq + n] = float_to_bf16(y);
-    else page[((size_t)(head - rope.H) * rope.P + slot) * d + e] = float_to_bf16(y);
+    if constexpr (PRE) {
+#pragma unroll
+      for (int o = 8; o > 0; o /= 2) sum += __shfl_xor(sum, o, WAVE);
+      g *= 1.0f / sqrtf(sum / (float)K + norm.eps);
+    }
+    bf16_t* page = rope.cache;
+    if (sm < M) page += (size_t)rope.block_table[(size_t)seg * rope.max_blocks + pos / rope.P] * page_elems;
+    bf16_t* tile = reinterpret_cast<bf16_t*>(&vals[0][0]);             // [column][16 rows + 2]
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tile[fin_column<VEC, 16>(0, l16, j) * (FIN_V_ROWS + 2) + r] = float_to_bf16(g[j]);
+    __syncthreads();
+    if (sm >= M) return;
+    bf16_t* out = page + (size_t)rope.Hk * rope.P * d + pos % rope.P;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = j * 16 + threadIdx.x / 16;
+      if (col0 + c < N) out[(size_t)(col0 - qk + c) * rope.P] = tile[c * (FIN_V_ROWS + 2) + sr];
+    }
+    return;
+  }
+  const int across = ceil_div(qk, 4 * FIN_COLS);
+  const int m = blockIdx.x / across, first = (blockIdx.x % across * 4 + wave) * FIN_COLS;
+  if (first >= qk) return;
+  const int pos = rope.positions[m], seg = rope.row_seg[m];
+  floatx4 g = fin_sum<VEC>(partials + (size_t)m * N, plane, k_split, first, lane, N);
+  const float rstd = PRE ? fin_rstd(norm, m, lane, K) : 1.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) g[j] = bf16_to_float(float_to_bf16(PRE ? g[j] * rstd : g[j]));
+  bf16_t* page = rope.cache + (size_t)rope.block_table[(size_t)seg * rope.max_blocks + pos / rope.P] * page_elems;
+  const float* cs = rope.cos_sin + (size_t)pos * d;
+  floatx4 cosv, sinv, partner;  // partner: the value `half` columns on or back (d is a power of two)
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = fin_column<VEC>(first, lane, j) % half;
+    cosv[j] = cs[r], sinv[j] = cs[half + r];
+    vals[wave][fin_column<VEC>(0, lane, j)] = g[j];
+  }
+  wave_lds_order();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) partner[j] = vals[wave][fin_column<VEC>(0, lane, j) ^ half];
+  floatx4 y;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    y[j] = fin_column<VEC>(first, lane, j) % d < half ? g[j] * cosv[j] - partner[j] * sinv[j] : partner[j] * sinv[j] + g[j] * cosv[j];
+  bf16_t* keys = page + (size_t)(pos % rope.P) * d;
+  if constexpr (VEC) {  // four columns of one head
+    const int n = first + lane * 4, head = n / d;
+    if (n >= qk) return;
+    uint2 o;
+    o.x = pack_bf16x2(y[0], y[1]);
+    o.y = pack_bf16x2(y[2], y[3]);
+    *reinterpret_cast<uint2*>(head < rope.H ? q_out + (size_t)m * ldq + n
+                                            : keys + (size_t)(head - rope.H) * rope.P * d + n % d) = o;
   } else {
-    page[(size_t)rope.Hk * rope.P * d + ((size_t)(head - rope.H - rope.Hk) * d + e) * rope.P + slot] = float_to_bf16(x);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = fin_column<VEC>(first, lane, j), head = n / d;
+      if (n >= qk) continue;
+      if (head < rope.H) q_out[(size_t)m * ldq + n] = float_to_bf16(y[j]);
+      else keys[(size_t)(head - rope.H) * rope.P * d + n % d] = float_to_bf16(y[j]);
+    }
   }
 }
 
@@ -744,13 +842,19 @@ APC_EXPORT int apc_gemm_splitk_qkv_rope_bf16(const void* A, int lda, const float
   if (e) return e;
   const FinishNorm norm{ss, ss_parts, eps, nullptr, nullptr, 0, nullptr};
   const FinishRope rope{cos_sin, positions, row_seg, block_table, max_blocks, (bf16_t*)cache, page_tokens, H, Hk, d};
-  const dim3 grid(ceil_div(N, 256), M);
-  if (ss)
-    hipLaunchKernelGGL((gemm_finish_qkv_rope_kernel<true>), grid, dim3(256), 0, stream, workspace, k_split, M, N, K,
-                       (bf16_t*)q_out, ldq, norm, rope);
-  else
-    hipLaunchKernelGGL((gemm_finish_qkv_rope_kernel<false>), grid, dim3(256), 0, stream, workspace, k_split, M, N, K,
-                       (bf16_t*)q_out, ldq, norm, rope);
+  const bool vec = d % 8 == 0 && ldq % 4 == 0 && aligned16(workspace) && ((uintptr_t)q_out & 7u) == 0 && ((uintptr_t)cache & 7u) == 0;
+  const int qk = (H + Hk) * d;
+  const long qk_blocks = (long)M * ceil_div(qk, 4 * FIN_COLS);
+  const long blocks = qk_blocks + (long)ceil_div(M, FIN_V_ROWS) * ceil_div(N - qk, FIN_V_COLS);
+  if (blocks > 0x7fffffffL) return APC_ERR_BAD_ARG;
+#define FINISH_ROPE(PRE_, VEC_)                                                                                         \
+  hipLaunchKernelGGL((gemm_finish_qkv_rope_kernel<PRE_, VEC_>), dim3((unsigned)blocks), dim3(256), 0, stream, workspace, \
+                     k_split, M, N, K, (bf16_t*)q_out, ldq, norm, rope, (int)qk_blocks)
+  if (ss && vec) FINISH_ROPE(true, true);
+  else if (ss) FINISH_ROPE(true, false);
+  else if (vec) FINISH_ROPE(false, true);
+  else FINISH_ROPE(false, false);
+#undef FINISH_ROPE
   APC_LAUNCH_CHECK();
   return 0;
 }

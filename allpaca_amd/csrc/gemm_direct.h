@@ -3,8 +3,18 @@
 #pragma once
 #include "common.h"
 
-// Fewer rows than this stay with the 128 x 128 tile and its K slices (too few blocks of 128 rows for the chip).
+// From so many rows on whatever the columns.
 constexpr int GEMM_DIRECT_MIN_ROWS = 1024;
+// Fewer rows, K in one piece: where the 128 x 128 tile (64 outputs wide for SwiGLU) would not get by with one tile a
+// compute unit.  Microseconds, that tile / this kernel, K 4,096: 768 rows x 6,144 outputs (288 tiles) 63 / 50, 1,000 x
+// 4,096 (256 tiles) 43 / 48, 512 x 6,144 (192) 42 / 49; K 3,072: 896 x 5,120 (280) 49 / 38, 768 x 5,120 (240) 34 / 38;
+// SwiGLU of 14,336 outputs, K 4,096: 128 rows (224) 53 / 67, 130 (448) 75 / 59, 256 (448) 79 / 67; of 8,192 outputs, K 3,072:
+// 256 rows (256) 37 / 48, 384 (384) 54 / 49.
+constexpr int GEMM_DIRECT_FEW_ROWS = 129;
+// K in slices (the adding kernel is the same): from so many rows on.  As above with the best number of slices for either:
+// down of an 8B model (4,096 x 14,336) at 256 rows 47 / 48, 384 rows 66 / 67, 512 78 / 70, 768 116 / 110, 1,000 137 / 112;
+// of a 3B model (3,072 x 8,192) 256 rows 29 / 28, 384 37 / 37, 512 46 / 38, 768 59 / 53.
+constexpr int GEMM_DIRECT_SLICES_MIN_ROWS = 257;
 
 // mode: 0 store bfloat16, 1 store float32, 2 add into float32, 3 SwiGLU (W = gate, W2 = up, N = the width of each).
 // True if launch_gemm_direct runs this shape (K a multiple of 128, N and ldc of 4, 16-byte aligned A and C, ...).
@@ -17,10 +27,7 @@ int launch_gemm_direct_act(int act, const bf16_t* A, int lda, const bf16_t* W, v
                            hipStream_t stream);
 // Products on rows that a product into the residual left for the RMS norm (A = the rows times the norm's weight, ss =
 // [M][ss_parts] sums of x^2): the sums are scaled by 1 / sqrt(sum(ss[m]) / K + eps), before the activation where there
-// is one.  mode 0 (store bfloat16) or 3 (SwiGLU).  SwiGLU from GEMM_DIRECT_PRE_MIN_ROWS rows on: the 28,672 weight
-// rows of an 8B model's gate and up give 128-row tiles a full round of blocks already at 512 rows, where the 128 x 128
-// tile takes 153 us and this 117; the others from GEMM_DIRECT_MIN_ROWS on.
-constexpr int GEMM_DIRECT_PRE_MIN_ROWS = 384;
+// is one.  mode 0 (store bfloat16) or 3 (SwiGLU).
 bool gemm_direct_pre_takes(int mode, const void* A, int lda, const void* C, int ldc, int M, int N, int K, int ss_parts);
 int launch_gemm_direct_pre(int mode, const bf16_t* A, int lda, const float* ss, int ss_parts, float eps, const bf16_t* W,
                            const bf16_t* W2, void* C, int ldc, int M, int N, int K, hipStream_t stream);

@@ -421,6 +421,14 @@ int launch_mode(int nf, const bf16_t* A, int lda, const bf16_t* W, const bf16_t*
   return launch<8, MODE>(A, lda, W, W2, C, ldc, M, N, K, stream, pre);
 }
 
+bool direct_takes(int mode, const void* A, int lda, const void* C, int ldc, int M, int N, int K) {
+  if (mode < 0 || mode > D_STORE_ACT || M <= 0 || K < 128 || K % 128 || N % 4 || ldc % 4) return false;
+  if (((uintptr_t)A & 15u) || ((uintptr_t)C & 15u) || lda % 8) return false;
+  // the lanes' byte offsets into the block's rows of A and the wave's bands of W are 32-bit
+  if ((long)128 * lda * 2 >= 0x7fffffffL || (long)8 * ceil_div(K, 32) * 1024 >= 0x7fffffffL) return false;
+  return true;
+}
+
 }  // namespace
 
 // A product with few output columns fills one round of blocks only with narrow tiles (4 bands a wave for the 4,096
@@ -442,7 +450,8 @@ int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* 
                               int k_split, hipStream_t stream) {
   if (k_split < 1 || k_split > 65535 || K % k_split) return APC_ERR_UNSUPPORTED;
   const int k_slice = K / k_split;
-  if (!gemm_direct_takes(D_STORE_F32, A, lda, partials, N, M, N, k_slice)) return APC_ERR_UNSUPPORTED;
+  if (M < GEMM_DIRECT_SLICES_MIN_ROWS || !direct_takes(D_STORE_F32, A, lda, partials, N, M, N, k_slice))
+    return APC_ERR_UNSUPPORTED;
   const int nf = pick_bands(M, N, false, k_split);
   const int nb = 4 * nf * 16;
   const long blocks = 8L * ceil_div((long)ceil_div(N, nb) * ceil_div(M, 128), 8L);
@@ -462,12 +471,10 @@ int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* 
 }
 
 namespace {
-bool direct_takes(int mode, int min_rows, const void* A, int lda, const void* C, int ldc, int M, int N, int K) {
-  if (mode < 0 || mode > D_STORE_ACT || M < min_rows || K < 128 || K % 128 || N % 4 || ldc % 4) return false;
-  if (((uintptr_t)A & 15u) || ((uintptr_t)C & 15u) || lda % 8) return false;
-  // the lanes' byte offsets into the block's rows of A and the wave's bands of W are 32-bit
-  if ((long)128 * lda * 2 >= 0x7fffffffL || (long)8 * ceil_div(K, 32) * 1024 >= 0x7fffffffL) return false;
-  return true;
+// whether these rows and columns are enough for this kernel with K in one piece (gemm_direct.h has both sides' times)
+bool enough_tiles(int M, int N, bool swiglu) {
+  if (M >= GEMM_DIRECT_MIN_ROWS) return true;
+  return M >= GEMM_DIRECT_FEW_ROWS && (long)ceil_div(M, 128) * ceil_div(N, swiglu ? 64 : 128) > 256;
 }
 
 int launch_columns(int nf, int mode, const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C, int ldc, int M,
@@ -538,7 +545,7 @@ int launch_direct(int mode, const bf16_t* A, int lda, const bf16_t* W, const bf1
 }  // namespace
 
 bool gemm_direct_takes(int mode, const void* A, int lda, const void* C, int ldc, int M, int N, int K) {
-  return mode <= D_SWIGLU && direct_takes(mode, GEMM_DIRECT_MIN_ROWS, A, lda, C, ldc, M, N, K);
+  return mode <= D_SWIGLU && enough_tiles(M, N, mode == D_SWIGLU) && direct_takes(mode, A, lda, C, ldc, M, N, K);
 }
 
 int launch_gemm_direct(int mode, const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C, int ldc, int M,
@@ -557,10 +564,7 @@ int launch_gemm_direct_act(int act, const bf16_t* A, int lda, const bf16_t* W, v
 
 bool gemm_direct_pre_takes(int mode, const void* A, int lda, const void* C, int ldc, int M, int N, int K, int ss_parts) {
   if (ss_parts <= 0 || (mode != D_STORE_BF16 && mode != D_SWIGLU)) return false;
-  // SwiGLU's many outputs fill a round of 128-row tiles from 384 rows on; other products only where the direct kernel
-  // takes them without a folded norm too
-  const int min_rows = mode == D_SWIGLU ? GEMM_DIRECT_PRE_MIN_ROWS : GEMM_DIRECT_MIN_ROWS;
-  return direct_takes(mode, min_rows, A, lda, C, ldc, M, N, K);
+  return gemm_direct_takes(mode, A, lda, C, ldc, M, N, K);
 }
 
 int launch_gemm_direct_pre(int mode, const bf16_t* A, int lda, const float* ss, int ss_parts, float eps, const bf16_t* W,
@@ -575,7 +579,7 @@ int launch_gemm_direct_pre(int mode, const bf16_t* A, int lda, const float* ss, 
 }
 
 int gemm_direct_emit_parts(const void* A, int lda, const void* C, int ldc, int M, int N, int K) {
-  if (!direct_takes(D_ACC_EMIT, GEMM_DIRECT_MIN_ROWS, A, lda, C, ldc, M, N, K) || M > 65535) return 0;
+  if (M < GEMM_DIRECT_MIN_ROWS || !direct_takes(D_ACC_EMIT, A, lda, C, ldc, M, N, K) || M > 65535) return 0;
   if (gemm_direct_k_split(M, N, K) > 1) return ceil_div(N, 1024);
   return column_tiles(plan_columns(M, N, false), N, false);
 }

@@ -234,7 +234,7 @@ int pre_tiled(Program& P, const Emit& e, const ApcMatrix& w, const ApcMatrix* wu
   const int M = e.raw.rows, K = e.raw.cols;
   if (!(M > SKINNY_MAX_ROWS && act_ok(e.raw) && e.ss_rows == M && e.ss_cols >= 1 && e.ss_cols <= 256)) return 0;
   const int n_mats = wu ? 2 : 1;
-  const int ks = tiled_k_split(M, n_cols * n_mats, K);
+  const int ks = tiled_k_split(M, n_cols * n_mats, K, wu != nullptr);
   if (ks == 1) {
     LAUNCH(P, "gemm_pre_bf16",
            apc_gemm_pre_bf16(e.raw.p, e.raw.ld, e.ss, e.ss_cols, e.eps, w.data, wu ? wu->data : nullptr, out.p, out.ld, M,
@@ -277,7 +277,7 @@ int swiglu(Program& P, const Buf& h, const ApcLayer& L, const Buf& out) {
   const int M = h.rows, K = h.cols, F = out.cols;
   if (L.w_gate.packed) {
     if (!act_ok(h) || out.dtype != APC_DT_BF16 || L.w_gate.K != K || L.w_gate.N != F) return -1;
-    const int ks = M > SKINNY_MAX_ROWS ? tiled_k_split(M, 2 * F, K) : 1;
+    const int ks = M > SKINNY_MAX_ROWS ? tiled_k_split(M, 2 * F, K, true) : 1;
     if (ks > 1) {
       float* ws = P.floats((size_t)2 * ks * M * F);
       LAUNCH(P, "gemm_splitk_bf16 (swiglu)",

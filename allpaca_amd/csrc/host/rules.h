@@ -32,9 +32,28 @@ inline int k_split_many_rows(int M, int N, int K) {  // 129..1024 rows
   return std::max(1, std::min(s, K / 256));
 }
 
-inline int tiled_k_split(int M, int N, int K) {
+// 257..1024 rows, by the expected time (tuned._k_split_direct says what it rests on)
+constexpr int DIRECT_SLICES_MIN_ROWS = 257;
+inline int k_split_direct(int M, int N, int K) {
+  const long tiles = cdiv(M, 128);
+  int best = 1;
+  double least = 0.0;
+  for (int s : {1, 2, 3, 4, 6, 8}) {
+    if (s > 1 && K % (128 * s)) continue;
+    double us = 1e30;
+    for (int nf : {3, 4, 5, 6, 8}) us = std::min(us, (double)cdiv(tiles * cdiv(N, 64 * nf) * s, CHIP_UNITS) * (19.0 + 10.4 * nf));
+    if (s == 1 && tiles * cdiv(N, 128) <= CHIP_UNITS) us = 41.0;
+    us = us * (K / (4096.0 * s)) + (s == 1 ? 7.0 : 4.5 + s * ((double)M * N) * (1.38 / 1048576.0));
+    if (s == 1 || us < least) best = s, least = us;
+  }
+  return best;
+}
+
+inline int tiled_k_split(int M, int N, int K, bool gated = false) {
   if (M <= SPLITK_MAX_ROWS) return k_split(M, N, K);
-  return M <= MANY_ROWS_SPLIT_MAX ? k_split_many_rows(M, N, K) : 1;
+  if (M > MANY_ROWS_SPLIT_MAX) return 1;
+  if (M >= DIRECT_SLICES_MIN_ROWS && !gated && K % 256 == 0 && N % 4 == 0) return k_split_direct(M, N, K);
+  return k_split_many_rows(M, N, K);
 }
 
 // ranges that the decode kernel cuts every row's keys into (the kernel sizes them from the row's own length)

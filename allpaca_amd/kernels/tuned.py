@@ -15,6 +15,7 @@ from . import lib as _lib
 from . import ops as _ops
 from .packing import PackedWeight
 
+CHIP_UNITS = 256   # compute units the rules below were measured on
 MANY_ROWS_SPLIT_MAX = 1024   # up to here the tiled kernel may cut K into slices to get enough blocks
 SKINNY_MAX_ROWS = 16     # the streaming kernel: up to one 16-row tile of activations
 SPLITK_MAX_ROWS = 128    # the tiled kernel with K cut into slices: 17..128 rows
@@ -29,7 +30,7 @@ def _k_split(M: int, N: int, K: int) -> int:
 
 
 def _k_split_many_rows(M: int, N: int, K: int) -> int:
-    """Slices of K for 129..1024 rows: a matrix with few output columns gives the 128 x 128 tiles too few blocks
+    """Slices of K on 128 x 128 tiles for 129..1024 rows: a matrix with few output columns gives the 128 x 128 tiles too few blocks
     for 256 compute units (o_proj and down of an 8B model at 512 rows: 128), and slicing K, at the price of writing
     and adding float32 partial sums, was measured faster up to about 200 blocks (down, 4096 x 14336, 256 rows: 150
     us whole, 52 us in 4 slices); with more outputs than K and 150 blocks or more it was not."""
@@ -47,16 +48,42 @@ def _k_split_many_rows(M: int, N: int, K: int) -> int:
     return max(1, min(s, K // 256))
 
 
-def _tiled_k_split(M: int, N: int, K: int) -> int:
-    """Slices of K on the tiled kernel for M rows (1: K in one piece)."""
+DIRECT_SLICES_MIN_ROWS = 257   # the kernel that keeps the weights out of LDS takes slices from here on
+
+
+def _k_split_direct(M: int, N: int, K: int) -> int:
+    """Slices of K for 257..1024 rows, by the expected microseconds: rounds of 256 blocks of 128 rows x 64 nf columns at
+    19 + 10.4 nf a round and 4,096 columns of K (`gemm_direct_bf16.hip`); the slices' way through memory, 4.5 and 1.38 a slice
+    and 2^20 outputs; K whole on 128 x 128 tiles 41 (more than 256 of them: the rounds above), and 7 for what the adding
+    kernel would have done on the way, the norm's row or the rotation.  Against 9 matrices of 1B to 8B models at 384 to 1,000
+    rows the times are off by up to 4 us (512 rows, 4,096 x 14,336: 2 / 4 / 8 slices 93.6 / 70.4 / 73.9, expected 98 / 69 / 72)."""
+    tiles = -(-M // 128)
+    best, least = 1, 0.0
+    for s in (1, 2, 3, 4, 6, 8):
+        if s > 1 and K % (128 * s):
+            continue
+        us = min(-(-(tiles * -(-N // (64 * nf)) * s) // CHIP_UNITS) * (19.0 + 10.4 * nf) for nf in (3, 4, 5, 6, 8))
+        if s == 1 and tiles * -(-N // 128) <= CHIP_UNITS:
+            us = 41.0
+        us = us * (K / (4096.0 * s)) + (7.0 if s == 1 else 4.5 + s * (M * N) * (1.38 / 1048576.0))
+        if s == 1 or us < least:
+            best, least = s, us
+    return best
+
+
+def _tiled_k_split(M: int, N: int, K: int, gated: bool = False) -> int:
+    """Slices of K on the tiled kernels for M rows (1: K in one piece).  gated: gate and up in one product, N columns in all."""
     if M <= SPLITK_MAX_ROWS:
         return _k_split(M, N, K)
-    return _k_split_many_rows(M, N, K) if M <= MANY_ROWS_SPLIT_MAX else 1
+    if M > MANY_ROWS_SPLIT_MAX:
+        return 1
+    if M >= DIRECT_SLICES_MIN_ROWS and not gated and K % 256 == 0 and N % 4 == 0:
+        return _k_split_direct(M, N, K)
+    return _k_split_many_rows(M, N, K)
 
 
 # The chip these rules and the kernels' launch plans were measured on (`csrc/host/rules.h`, `gemm_direct_bf16.hip`:
 # rounds of 256 blocks over 8 XCDs; `attention_wide_bf16.hip`: 160 KiB of LDS a compute unit).
-CHIP_UNITS = 256
 CHIP_LDS_BYTES = 160 * 1024
 _chips_checked: set = set()
 
@@ -135,7 +162,7 @@ def swiglu_bf16(h: torch.Tensor, wg: PackedWeight, wu: PackedWeight, out: torch.
                          "of 8, 16-byte aligned")
     lda, ldc = _ops._rows(h, "h"), _ops._rows(out, "out")
     L = _lib.load("tuned")
-    ks = _tiled_k_split(M, 2 * F, K) if M > SKINNY_MAX_ROWS else 1
+    ks = _tiled_k_split(M, 2 * F, K, True) if M > SKINNY_MAX_ROWS else 1
     if ks > 1:
         ws = torch.empty(2 * ks * M * F, dtype=torch.float32, device=h.device)
         _lib.check(L.apc_gemm_splitk_bf16(h.data_ptr(), lda, wg.data.data_ptr(), wu.data.data_ptr(), out.data_ptr(), ldc,
@@ -211,7 +238,7 @@ def _pre_tiled(raw: torch.Tensor, ss: torch.Tensor, eps: float, w, wu, out: torc
             and ss.dim() == 2 and ss.shape[0] == M and 1 <= ss.shape[1] <= 256):
         return False
     n_mats = 2 if wu is not None else 1
-    ks = _tiled_k_split(M, n_cols * n_mats, K)
+    ks = _tiled_k_split(M, n_cols * n_mats, K, wu is not None)
     L = _lib.load("tuned")
     wu_ptr = wu.data.data_ptr() if wu is not None else 0
     if ks == 1:

@@ -320,6 +320,33 @@ def test_product_of_the_normalised_row_from_what_was_left_with_17_to_1024_rows(M
         check(f64(out), P.silu(raw64 @ f64(w[:F]).T * rstd) * (raw64 @ f64(w[F:2 * F]).T * rstd), BF)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # the kernel without weights in LDS, K in slices (its first row count, a last row tile of 1, of 44 and of 128 rows; one
+    # to eight slices) and the row before it; a K that has no slices of its own (1,088)
+    (256, 520, 2048), (257, 520, 2048), (300, 132, 1536), (1000, 264, 6144), (1024, 2048, 512), (640, 96, 1088),
+    # K in one piece with more than 256 tiles of 128 x 128, and with 256
+    (129, 16516, 128), (130, 16384, 256),
+    # the adding kernel without whole pieces (columns no multiple of 4), and two rows of it at 128 rows
+    (140, 130, 2048), (257, 1022, 1024), (128, 516, 1024)])
+def test_products_of_some_hundred_rows(M, N, K):
+    t = tuned()
+    a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=2, dtype=BF).to(DEV)
+    want = f64(a) @ f64(w).T
+    pw = pack(w)
+    for out_dtype in (BF, torch.float32):
+        out = torch.full((M, N), 7.0, dtype=out_dtype, device=DEV)
+        t.gemm_bf16(a, pw, out)
+        check(f64(out), want, out_dtype)
+    res = gen(M, N, seed=3).to(DEV)
+    x = f64(res) + want
+    t.gemm_bf16(a, pw, res, accumulate=True)
+    check(f64(res), x, torch.float32)
+    wide = torch.full((M, N + 5), 7.0, dtype=torch.float32, device=DEV)      # rows that begin off 16 bytes
+    t.gemm_bf16(a, pw, wide[:, 1:N + 1])
+    check(f64(wide[:, 1:N + 1]), want, torch.float32)
+    assert (wide[:, 0] == 7).all() and (wide[:, N + 1:] == 7).all()
+
+
 def test_folded_norm_refuses_what_it_does_not_take():
     t = tuned()
     w = pack(gen(32, 64, dtype=BF).to(DEV))
