@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "gemm_direct.h"
+#include "gemm_rows.h"
 #include "gemm_wide.h"
 #include "mfma.h"
 
@@ -39,9 +40,9 @@ struct GemmRegs {
 // ss[m][parts] are its sums of x^2 per row and block of columns; the sums of this product are scaled by
 // 1 / sqrt(sum(ss[m]) / K + eps): the product of the normalised row without a kernel for the norm.
 struct TiledPre {
-  const float* ss;
-  int parts;
-  float eps;
+  const float* ss = nullptr;
+  int parts = 0;
+  float eps = 0.f;
 };
 
 // Rows in runs that each multiply with a matrix of their own (routed experts: the rows that chose an expert lie side by
@@ -229,19 +230,11 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(const bf16_t* __restrict
       for (int j = 0; j < PIECES; ++j) load_piece(s[dd], min(kt0 + dd, last), j);
 #pragma unroll
     for (int j = 0; j < PIECES; ++j) store_piece(s[0], 0, j);
-    if constexpr (PRE) {  // behind the first loads of the tiles: one row a thread, its parts added in order, 8 loads
-      if (tid < BM) {     // at a time; read after the barriers of the K loop
-        const float* row = pre.ss + (size_t)min(m0 + tid, M - 1) * pre.parts;
-        float sum = 0.f;
-        for (int p0 = 0; p0 < pre.parts; p0 += 8) {
-          float v[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = p0 + j < pre.parts ? row[p0 + j] : 0.f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) sum += v[j];
-        }
-        rstd_s[tid] = 1.0f / sqrtf(sum / (float)K + pre.eps);
-      }
+    if constexpr (PRE) {  // behind the first loads of the tiles; read after the barriers of the K loop
+      constexpr int LANES = 256 / BM;
+      const int r = tid / LANES;
+      const float sum = row_parts_sum<LANES>(pre.ss + (size_t)min(m0 + r, M - 1) * pre.parts, pre.parts, tid % LANES);
+      if (tid % LANES == 0) rstd_s[r] = 1.0f / sqrtf(sum / (float)K + pre.eps);
     }
     __syncthreads();
     int kt = 0;
@@ -330,6 +323,8 @@ template <int MODE, bool PRE = false>
 static int launch_gemm(const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C, int ldc, int M, int N,
                        int K, hipStream_t stream, TiledPre pre = TiledPre{}, int act = 0) {
   constexpr int NB = MODE == G_SWIGLU ? BN / 2 : BN;
+  if (gemm_rows_takes(MODE, A, lda, W, W2, C, ldc, M, N, K))
+    return launch_gemm_rows(MODE, A, lda, W, W2, C, ldc, M, N, K, RowsNorm{const_cast<float*>(pre.ss), pre.parts, pre.eps, nullptr, nullptr, 0, act}, stream);
   if constexpr (MODE == G_ACT) {
     if (gemm_direct_takes(G_STORE_BF16, A, lda, C, ldc, M, N, K)) return launch_gemm_direct_act(act, A, lda, W, C, ldc, M, N, K, stream);
   } else if constexpr (!PRE) {
@@ -432,16 +427,9 @@ __device__ __forceinline__ floatx4 fin_sum(const float* __restrict__ row, size_t
   return g;
 }
 
-// 1 / sqrt(mean of x^2 + eps) of row m, from up to 256 sums of x^2
+// 1 / sqrt(mean of x^2 + eps) of row m, from its sums of x^2
 __device__ __forceinline__ float fin_rstd(const FinishNorm& norm, int m, int lane, int K) {
-  float sum = 0.f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int p = j * WAVE + lane;
-    if (p < norm.pre_parts) sum += norm.pre_ss[(size_t)m * norm.pre_parts + p];
-  }
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o /= 2) sum += __shfl_xor(sum, o, WAVE);
+  const float sum = row_parts_sum<WAVE>(norm.pre_ss + (size_t)m * norm.pre_parts, norm.pre_parts, lane);
   return 1.0f / sqrtf(sum / (float)K + norm.eps);
 }
 
@@ -563,6 +551,9 @@ static int launch_splitk(const void* A, int lda, const void* W, const void* Wu, 
     return APC_ERR_BAD_ARG;
   }
   if ((mode == G_SWIGLU) != (Wu != nullptr)) return APC_ERR_BAD_ARG;
+  if (!emit && lda >= K && gemm_rows_takes(mode, A, lda, W, Wu, C, ldc, M, N, K))   // no slices: the workspace stays as it is
+    return launch_gemm_rows(mode, (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)Wu, C, ldc, M, N, K,
+                            RowsNorm{const_cast<float*>(norm.pre_ss), norm.pre_parts, norm.eps, nullptr, nullptr, 0, norm.act}, stream);
   const int e = launch_partials(A, lda, W, Wu, M, N, K, k_split, workspace, stream);
   if (e) return e;
   const bool out16 = mode == G_STORE_BF16 || mode == G_SWIGLU || mode == G_ACT;
@@ -621,15 +612,9 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
     int pos = 0, seg = 0;
     if (sm < M) pos = rope.positions[sm], seg = rope.row_seg[sm];
     floatx4 g = floatx4{0.f, 0.f, 0.f, 0.f};
-    float sum = 0.f;
-    if (m < M) {
-      g = fin_sum<VEC, 16>(partials + (size_t)m * N, plane, k_split, col0, l16, N);
-      if constexpr (PRE)
-        for (int p = l16; p < norm.pre_parts; p += 16) sum += norm.pre_ss[(size_t)m * norm.pre_parts + p];
-    }
+    if (m < M) g = fin_sum<VEC, 16>(partials + (size_t)m * N, plane, k_split, col0, l16, N);
     if constexpr (PRE) {
-#pragma unroll
-      for (int o = 8; o > 0; o /= 2) sum += __shfl_xor(sum, o, WAVE);
+      const float sum = row_parts_sum<16>(norm.pre_ss + (size_t)min(m, M - 1) * norm.pre_parts, norm.pre_parts, l16);
       g *= 1.0f / sqrtf(sum / (float)K + norm.eps);
     }
     bf16_t* page = rope.cache;
@@ -713,6 +698,22 @@ APC_EXPORT int apc_gemm_direct_emit_bf16(const void* A, int lda, const void* W, 
                                  parts, workspace, stream);
 }
 
+// Products of 17 to 64 rows that need no slices of K (gemm_rows_bf16.hip): whether the entry points below hand one to that
+// kernel (mode as theirs, 4 for q, k and v with C the output of q), and then need no workspace.
+APC_EXPORT int apc_gemm_rows_takes(int mode, const void* A, int lda, const void* W, const void* Wu, const void* C, int ldc,
+                                   int M, int N, int K) {
+  return gemm_rows_takes(mode_is_act(mode) ? G_ACT : mode, A, lda, W, Wu, C, ldc, M, N, K);
+}
+// residual += A . W^T on that kernel, with raw as in apc_gemm_splitk_emit_bf16 and ss [M][N / 16] sums of residual^2 per row
+// and band of 16 columns
+APC_EXPORT int apc_gemm_rows_emit_bf16(const void* A, int lda, const void* W, float* residual, int ldc, int M, int N, int K,
+                                       const float* g, void* raw, int ldr, float* ss, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (lda < K || ldc < N || !g || !raw || !ss || ldr < N) return APC_ERR_BAD_ARG;
+  return launch_gemm_rows(G_ACC_F32, (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, residual, ldc, M, N, K,
+                          RowsNorm{ss, N / 16, 0.f, g, (bf16_t*)raw, ldr}, stream);
+}
+
 APC_EXPORT int apc_gemm_splitk_bf16(const void* A, int lda, const void* W, const void* Wu, void* C, int ldc, int M,
                                     int N, int K, int mode, int k_split, float* workspace, hipStream_t stream) {
   return launch_splitk(A, lda, W, Wu, C, ldc, M, N, K, mode, k_split, workspace, 0, 0, FinishNorm{}, stream);
@@ -729,12 +730,12 @@ APC_EXPORT int apc_gemm_splitk_emit_bf16(const void* A, int lda, const void* W, 
 }
 
 // The storing products (mode 0, 1 or 3) on a row that apc_gemm_splitk_emit_bf16 left: A = raw [M, K],
-// ss = [M][ss_parts] sums of x^2 (ss_parts <= 256); the sums are scaled by 1 / sqrt(sum(ss[m]) / K + eps).
+// ss = [M][ss_parts] sums of x^2 (ss_parts <= 1,024); the sums are scaled by 1 / sqrt(sum(ss[m]) / K + eps).
 APC_EXPORT int apc_gemm_splitk_pre_bf16(const void* A, int lda, const float* ss, int ss_parts, float eps,
                                         const void* W, const void* Wu, void* C, int ldc, int M, int N, int K, int mode,
                                         int k_split, float* workspace, hipStream_t stream) {
   if (!ss || ss_parts <= 0 || mode == G_ACC_F32) return APC_ERR_BAD_ARG;
-  if (ss_parts > 256) return APC_ERR_UNSUPPORTED;
+  if (ss_parts > 1024) return APC_ERR_UNSUPPORTED;
   const FinishNorm norm{ss, ss_parts, eps, nullptr, nullptr, 0, nullptr};
   return launch_splitk(A, lda, W, Wu, C, ldc, M, N, K, mode, k_split, workspace, 1, 0, norm, stream);
 }
@@ -836,8 +837,13 @@ APC_EXPORT int apc_gemm_splitk_qkv_rope_bf16(const void* A, int lda, const float
   if (H <= 0 || Hk <= 0 || d <= 0 || ldq < H * d || !cos_sin || !positions || !row_seg || !block_table ||
       max_blocks <= 0 || !cache || page_tokens <= 0 || !q_out || (ss && ss_parts <= 0))
     return APC_ERR_BAD_ARG;
-  if (d % 2 || 256 % d || (ss && ss_parts > 256)) return APC_ERR_UNSUPPORTED;
+  if (d % 2 || 256 % d || (ss && ss_parts > 1024)) return APC_ERR_UNSUPPORTED;
   const int N = (H + 2 * Hk) * d;
+  if (lda >= K && gemm_rows_qkv_takes(A, lda, W, q_out, ldq, M, K, H, Hk, d, cos_sin, cache)) {
+    const RowsNorm rows{const_cast<float*>(ss), ss_parts, eps};
+    const RowsRope to{cos_sin, positions, row_seg, block_table, max_blocks, (bf16_t*)cache, page_tokens, H, Hk, d};
+    return launch_gemm_rows_qkv((const bf16_t*)A, lda, (const bf16_t*)W, (bf16_t*)q_out, ldq, M, K, rows, to, stream);
+  }
   const int e = launch_partials(A, lda, W, nullptr, M, N, K, k_split, workspace, stream);
   if (e) return e;
   const FinishNorm norm{ss, ss_parts, eps, nullptr, nullptr, 0, nullptr};

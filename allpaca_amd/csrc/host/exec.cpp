@@ -142,7 +142,7 @@ int gemm_bf16(Program& P, const Buf& a, const ApcMatrix& w, const Buf& out, bool
   const int mode = accumulate ? 2 : (out.dtype == APC_DT_BF16 ? 0 : 1);
   if (M > SKINNY_MAX_ROWS) {
     const int ks = M <= MANY_ROWS_SPLIT_MAX ? tiled_k_split(M, N, K) : apc_gemm_direct_k_split(M, N, K);
-    if (ks > 1) {
+    if (ks > 1 && !apc_gemm_rows_takes(mode, a.p, a.ld, w.data, nullptr, out.p, out.ld, M, N, K)) {
       float* ws = P.floats((size_t)ks * M * N);
       LAUNCH(P, "gemm_splitk_bf16",
              apc_gemm_splitk_bf16(a.p, a.ld, w.data, nullptr, out.p, out.ld, M, N, K, mode, ks, ws, P.stream));
@@ -189,6 +189,17 @@ int gemm_emit_bf16(Program& P, const Buf& a, const ApcMatrix& w, const Buf& resi
     emit.filled = true;
     return 1;
   }
+  if (M > SKINNY_MAX_ROWS && N / 16 <= ss_parts_max(M) && apc_gemm_rows_takes(2, a.p, a.ld, w.data, nullptr, residual.p, residual.ld, M, N, K)) {
+    emit.raw = P.emit_rows(emit, M, N);
+    emit.ss_rows = M;
+    emit.ss_cols = N / 16;
+    emit.ss = (float*)P.emit_take(emit, sizeof(float) * (size_t)M * emit.ss_cols);
+    LAUNCH(P, "gemm_rows_emit_bf16",
+           apc_gemm_rows_emit_bf16(a.p, a.ld, w.data, (float*)residual.p, residual.ld, M, N, K, emit.g, emit.raw.p, N, emit.ss,
+                                   P.stream));
+    emit.filled = true;
+    return 1;
+  }
   if (M > SKINNY_MAX_ROWS) {
     const int ks = tiled_k_split(M, N, K);
     if (ks == 1) return 0;
@@ -232,10 +243,10 @@ bool pre_ok_skinny(const Emit& e, int K) {
 // the storing products on a row that a product into the residual left, more than 16 rows; 1 done, 0 not taken
 int pre_tiled(Program& P, const Emit& e, const ApcMatrix& w, const ApcMatrix* wu, const Buf& out, int n_cols, int mode) {
   const int M = e.raw.rows, K = e.raw.cols;
-  if (!(M > SKINNY_MAX_ROWS && act_ok(e.raw) && e.ss_rows == M && e.ss_cols >= 1 && e.ss_cols <= 256)) return 0;
+  if (!(M > SKINNY_MAX_ROWS && act_ok(e.raw) && e.ss_rows == M && e.ss_cols >= 1 && e.ss_cols <= ss_parts_max(M))) return 0;
   const int n_mats = wu ? 2 : 1;
   const int ks = tiled_k_split(M, n_cols * n_mats, K, wu != nullptr);
-  if (ks == 1) {
+  if (ks == 1 || apc_gemm_rows_takes(mode, e.raw.p, e.raw.ld, w.data, wu ? wu->data : nullptr, out.p, out.ld, M, n_cols, K)) {
     LAUNCH(P, "gemm_pre_bf16",
            apc_gemm_pre_bf16(e.raw.p, e.raw.ld, e.ss, e.ss_cols, e.eps, w.data, wu ? wu->data : nullptr, out.p, out.ld, M,
                              n_cols, K, mode, P.stream));
@@ -278,7 +289,7 @@ int swiglu(Program& P, const Buf& h, const ApcLayer& L, const Buf& out) {
   if (L.w_gate.packed) {
     if (!act_ok(h) || out.dtype != APC_DT_BF16 || L.w_gate.K != K || L.w_gate.N != F) return -1;
     const int ks = M > SKINNY_MAX_ROWS ? tiled_k_split(M, 2 * F, K, true) : 1;
-    if (ks > 1) {
+    if (ks > 1 && !apc_gemm_rows_takes(3, h.p, h.ld, L.w_gate.data, L.w_up.data, out.p, out.ld, M, F, K)) {
       float* ws = P.floats((size_t)2 * ks * M * F);
       LAUNCH(P, "gemm_splitk_bf16 (swiglu)",
              apc_gemm_splitk_bf16(h.p, h.ld, L.w_gate.data, L.w_up.data, out.p, out.ld, M, F, K, 3, ks, ws, P.stream));
@@ -349,10 +360,11 @@ int qkv_rope(Program& P, const Buf& a, const Emit* pre, const ApcLayer& L, const
   if (!(act_ok(a) && qkv.dtype == APC_DT_BF16 && E.kv_dtype == APC_DT_BF16)) return 0;
   if (few && !(d % 32 == 0 && qkv.ld % 4 == 0 && ((uintptr_t)qkv.p & 7u) == 0)) return 0;
   const int ks = few ? 1 : tiled_k_split(M, N, K);
-  if (!few && (ks == 1 || 256 % d || d % 2)) return 0;
+  const bool rows = !few && d % 32 == 0 && apc_gemm_rows_takes(4, a.p, a.ld, L.w_qkv.data, nullptr, qkv.p, qkv.ld, M, N, K);
+  if (!few && ((ks == 1 && !rows) || 256 % d || d % 2)) return 0;
   if (pre) {
     if (few && !pre_ok_skinny(*pre, K)) return 0;
-    if (!few && !(pre->ss_rows == M && pre->ss_cols >= 1 && pre->ss_cols <= 256)) return 0;
+    if (!few && !(pre->ss_rows == M && pre->ss_cols >= 1 && pre->ss_cols <= ss_parts_max(M))) return 0;
   }
   if (L.w_qkv.K != K || L.w_qkv.N != N || qkv.rows != M || qkv.cols < H * d) return -1;
   const ApcStep& s = P.step;

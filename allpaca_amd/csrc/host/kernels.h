@@ -44,6 +44,10 @@ int apc_gemm_splitk_qkv_rope_bf16(const void* A, int lda, const float* ss, int s
                                   void* q_out, int ldq, int M, int K, int H, int Hk, int d, const float* cos_sin,
                                   const int* positions, const int* row_seg, const int* block_table, int max_blocks,
                                   void* cache, int page_tokens, int k_split, float* workspace, hipStream_t stream);
+int apc_gemm_rows_takes(int mode, const void* A, int lda, const void* W, const void* Wu, const void* C, int ldc, int M, int N,
+                        int K);
+int apc_gemm_rows_emit_bf16(const void* A, int lda, const void* W, float* residual, int ldc, int M, int N, int K,
+                            const float* g, void* raw, int ldr, float* ss, hipStream_t stream);
 int apc_gemm_direct_k_split(int M, int N, int K);
 int apc_gemm_direct_emit_parts(const void* A, int lda, const void* residual, int ldc, int M, int N, int K);
 int apc_gemm_direct_emit_bf16(const void* A, int lda, const void* W, float* residual, int ldc, int M, int N, int K,

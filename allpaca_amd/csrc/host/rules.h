@@ -8,6 +8,7 @@
 namespace apc_rules {
 
 constexpr int SKINNY_MAX_ROWS = 16;
+constexpr int ROWS_MAX = 64;        // the kernel that finishes in one launch
 constexpr int SPLITK_MAX_ROWS = 128;
 constexpr int MANY_ROWS_SPLIT_MAX = 1024;
 constexpr int WHOLE_WAVES = 4;
@@ -55,6 +56,9 @@ inline int tiled_k_split(int M, int N, int K, bool gated = false) {
   if (M >= DIRECT_SLICES_MIN_ROWS && !gated && K % 256 == 0 && N % 4 == 0) return k_split_direct(M, N, K);
   return k_split_many_rows(M, N, K);
 }
+
+// sums of x^2 a row that the products behind a norm take
+inline int ss_parts_max(int M) { return M <= ROWS_MAX ? 1024 : 256; }
 
 // ranges that the decode kernel cuts every row's keys into (the kernel sizes them from the row's own length)
 inline int decode_parts(long pairs, int span) {

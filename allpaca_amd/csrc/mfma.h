@@ -54,6 +54,37 @@ __device__ __forceinline__ floatx16 mfma32(const Frag& a, const Frag& b, floatx1
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
 }
 
+// The sum of a row's `parts` sums of x^2 over the LANES lanes side by side that share the row (every lane gets it; `j`: which
+// of them this is).  Eight loads of four values a lane are in flight: 256 parts of 64 rows read 8 values at a time by a
+// thread a row held the tiled product's first step up by 9 us, and one value at a time by eight lanes by 2-3.
+template <int LANES>
+__device__ __forceinline__ float row_parts_sum(const float* __restrict__ row, int parts, int j) {
+  float sum = 0.f;
+  if (parts % 4 == 0 && ((uintptr_t)row & 15u) == 0) {
+    for (int p0 = j * 4; p0 < parts; p0 += LANES * 32) {
+      floatx4 v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        v[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if (p0 + k * LANES * 4 < parts) v[k] = *reinterpret_cast<const floatx4*>(row + p0 + k * LANES * 4);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+    }
+  } else {
+    for (int p0 = j; p0 < parts; p0 += LANES * 8) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = p0 + k * LANES < parts ? row[p0 + k * LANES] : 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum += v[k];
+    }
+  }
+#pragma unroll
+  for (int o = LANES / 2; o > 0; o /= 2) sum += __shfl_xor(sum, o, WAVE);
+  return sum;
+}
+
 __device__ __forceinline__ float silu_f(float g) { return g / (1.0f + __expf(-g)); }
 // An activation by code: 1 silu, 2 the square of max(z, 0), 3 gelu in its tanh form (tanh by one exponential, off by
 // about 1e-7), else z itself.

@@ -25,14 +25,14 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 LIBS: Dict[str, List[str]] = {
     "plain": ["plain_ops.hip", "plain_gemm.hip", "gemm_f32.hip", "plain_attention.hip", "plain_mixers.hip", "plain_heads.hip", "plain_recurrent.hip", "plain_routed.hip",
               "plain_scan.hip", "plain_latent.hip", "plain_delta.hip", "sampling.hip"],
-    "tuned": ["gemm_bf16.hip", "gemm_wide_bf16.hip", "gemm_direct_bf16.hip", "skinny_gemm_bf16.hip", "attention_bf16.hip", "attention_wide_bf16.hip", "attention_masked_bf16.hip", "conv_heads_bf16.hip", "rope_bf16.hip", "rotary_pages_bf16.hip",
+    "tuned": ["gemm_bf16.hip", "gemm_wide_bf16.hip", "gemm_direct_bf16.hip", "gemm_rows_bf16.hip", "skinny_gemm_bf16.hip", "attention_bf16.hip", "attention_wide_bf16.hip", "attention_masked_bf16.hip", "conv_heads_bf16.hip", "rope_bf16.hip", "rotary_pages_bf16.hip",
               "linear_attention_bf16.hip", "routed_bf16.hip", "selective_scan_bf16.hip", "latent_heads_bf16.hip", "attention_latent_bf16.hip",
               "delta_rule_bf16.hip", "gated_recurrence_bf16.hip"],
     # what measurements need and the engine does not (what a streaming read and a loop of MFMAs reach on this card)
     "bench": ["probe.hip"],
     "host": ["host/exec.cpp", "host/cache.cpp", "host/pack.cpp", "host/sched.cpp"],
 }
-HEADERS = ["common.h", "mfma.h", "gemm_wide.h", "gemm_direct.h", "attention_wide.h", "no_alloc.h",
+HEADERS = ["common.h", "mfma.h", "gemm_wide.h", "gemm_direct.h", "gemm_rows.h", "attention_wide.h", "no_alloc.h",
            "host/host.h", "host/kernels.h", "host/rules.h", "host/cache.h"]
 # libraries a library is linked against (built first; found at run time beside it)
 NEEDS: Dict[str, List[str]] = {"host": ["plain", "tuned"]}

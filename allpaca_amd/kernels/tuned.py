@@ -18,6 +18,7 @@ from .packing import PackedWeight
 CHIP_UNITS = 256   # compute units the rules below were measured on
 MANY_ROWS_SPLIT_MAX = 1024   # up to here the tiled kernel may cut K into slices to get enough blocks
 SKINNY_MAX_ROWS = 16     # the streaming kernel: up to one 16-row tile of activations
+ROWS_MAX = 64            # the kernel that finishes a product of 17 rows or more in one launch (`gemm_rows_bf16.hip`)
 SPLITK_MAX_ROWS = 128    # the tiled kernel with K cut into slices: 17..128 rows
 
 
@@ -82,6 +83,19 @@ def _tiled_k_split(M: int, N: int, K: int, gated: bool = False) -> int:
     return _k_split_many_rows(M, N, K)
 
 
+def _rows_take(a: torch.Tensor, w: PackedWeight, wu: Optional[PackedWeight], out: torch.Tensor, N: int, mode: int) -> bool:
+    """Whether such a product of 17 to 64 rows runs in one launch, without slices (N: columns of the product)."""
+    M, K = a.shape
+    return bool(SKINNY_MAX_ROWS < M <= ROWS_MAX and _lib.load("tuned").apc_gemm_rows_takes(
+        mode, a.data_ptr(), a.stride(0), w.data.data_ptr(), wu.data.data_ptr() if wu is not None else 0, out.data_ptr(),
+        out.stride(0), M, N, K))
+
+
+def _ss_parts_max(M: int) -> int:
+    """Sums of x^2 a row that the products behind a norm take."""
+    return 1024 if M <= ROWS_MAX else 256
+
+
 # The chip these rules and the kernels' launch plans were measured on (`csrc/host/rules.h`, `gemm_direct_bf16.hip`:
 # rounds of 256 blocks over 8 XCDs; `attention_wide_bf16.hip`: 160 KiB of LDS a compute unit).
 CHIP_LDS_BYTES = 160 * 1024
@@ -139,7 +153,7 @@ def gemm_bf16(a: torch.Tensor, w: PackedWeight, out: torch.Tensor, accumulate: b
     if M > SKINNY_MAX_ROWS:
         # more than 1,024 rows: the product of many rows says itself whether it wants K in two slices
         ks = _tiled_k_split(M, N, K) if M <= MANY_ROWS_SPLIT_MAX else L.apc_gemm_direct_k_split(M, N, K)
-        if ks > 1:
+        if ks > 1 and not _rows_take(a, w, None, out, N, mode):
             ws = torch.empty(ks * M * N, dtype=torch.float32, device=a.device)
             _lib.check(L.apc_gemm_splitk_bf16(a.data_ptr(), lda, w.data.data_ptr(), 0, out.data_ptr(), ldc, M, N, K,
                                               mode, ks, ws.data_ptr(), _ops._stream()), "gemm_splitk_bf16")
@@ -163,7 +177,7 @@ def swiglu_bf16(h: torch.Tensor, wg: PackedWeight, wu: PackedWeight, out: torch.
     lda, ldc = _ops._rows(h, "h"), _ops._rows(out, "out")
     L = _lib.load("tuned")
     ks = _tiled_k_split(M, 2 * F, K, True) if M > SKINNY_MAX_ROWS else 1
-    if ks > 1:
+    if ks > 1 and not _rows_take(h, wg, wu, out, F, 3):
         ws = torch.empty(2 * ks * M * F, dtype=torch.float32, device=h.device)
         _lib.check(L.apc_gemm_splitk_bf16(h.data_ptr(), lda, wg.data.data_ptr(), wu.data.data_ptr(), out.data_ptr(), ldc,
                                           M, F, K, 3, ks, ws.data_ptr(), _ops._stream()), "gemm_splitk_bf16")
@@ -177,8 +191,8 @@ def gemm_emit_bf16(a: torch.Tensor, w: PackedWeight, residual: torch.Tensor, g: 
     """residual += a . w^T, and for the RMS norm with weight g that reads the residual next: the row
     bfloat16(residual * g) and sums of residual^2 per row and group of columns.  Returns (raw [M, N], ss) or None,
     with nothing done, for sizes no kernel takes.  ss is [16, ceil(N/16) rounded up to 4] from the streaming kernel
-    (up to 16 rows) and [M, ceil(N/256)] from the tiled kernel with K in slices; the products below take what the
-    same number of rows gives."""
+    (up to 16 rows), [M, N/16] from the kernel of up to 64 rows and [M, ceil(N/256)] from the tiled kernel with K in
+    slices; the products below take what the same number of rows gives."""
     _ops._gpu(a, w.data, residual, g)
     M, K = a.shape
     N = w.N
@@ -203,6 +217,13 @@ def gemm_emit_bf16(a: torch.Tensor, w: PackedWeight, residual: torch.Tensor, g: 
                                                g.data_ptr(), raw.data_ptr(), N, ss.data_ptr(), parts,
                                                ws.data_ptr() if ws is not None else 0, _ops._stream()),
                    "gemm_direct_emit_bf16")
+        return raw, ss
+    if N // 16 <= _ss_parts_max(M) and _rows_take(a, w, None, residual, N, 2):
+        raw = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+        ss = torch.empty((M, N // 16), dtype=torch.float32, device=a.device)
+        _lib.check(L.apc_gemm_rows_emit_bf16(a.data_ptr(), lda, w.data.data_ptr(), residual.data_ptr(), ldc, M, N, K,
+                                             g.data_ptr(), raw.data_ptr(), N, ss.data_ptr(), _ops._stream()),
+                   "gemm_rows_emit_bf16")
         return raw, ss
     if M > SKINNY_MAX_ROWS:   # the tiled kernel: only where K is cut into slices (the finishing kernel leaves the row)
         ks = _tiled_k_split(M, N, K)
@@ -235,13 +256,13 @@ def _pre_tiled(raw: torch.Tensor, ss: torch.Tensor, eps: float, w, wu, out: torc
     256 sums of squares a row (what the tiled kernels leave: a part per 256 or per 128 columns)."""
     M, K = raw.shape
     if not (M > SKINNY_MAX_ROWS and _act_ok(raw) and ss.dtype == torch.float32 and ss.is_contiguous()
-            and ss.dim() == 2 and ss.shape[0] == M and 1 <= ss.shape[1] <= 256):
+            and ss.dim() == 2 and ss.shape[0] == M and 1 <= ss.shape[1] <= _ss_parts_max(M)):
         return False
     n_mats = 2 if wu is not None else 1
     ks = _tiled_k_split(M, n_cols * n_mats, K, wu is not None)
     L = _lib.load("tuned")
     wu_ptr = wu.data.data_ptr() if wu is not None else 0
-    if ks == 1:
+    if ks == 1 or _rows_take(raw, w, wu, out, n_cols, mode):
         _lib.check(L.apc_gemm_pre_bf16(raw.data_ptr(), _ops._rows(raw, "raw"), ss.data_ptr(), ss.shape[1], float(eps),
                                        w.data.data_ptr(), wu_ptr, out.data_ptr(), _ops._rows(out, "out"), M, n_cols, K,
                                        mode, _ops._stream()), "gemm_pre_bf16")
@@ -292,7 +313,8 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
     if few and not (d % 32 == 0 and q_out.stride(0) % 4 == 0 and q_out.data_ptr() % 8 == 0):
         return False
     ks = 1 if few else _tiled_k_split(M, N, K)
-    if not few and (ks == 1 or 256 % d or d % 2):
+    rows = not few and d % 32 == 0 and _rows_take(a, w, None, q_out, N, 4)
+    if not few and ((ks == 1 and not rows) or 256 % d or d % 2):
         return False
     ss, eps = None, 0.0
     if pre is not None:
@@ -300,7 +322,7 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
         if few and not _pre_ok(a, ss, K):
             return False
         if not few and not (ss.dtype == torch.float32 and ss.is_contiguous() and ss.dim() == 2 and ss.shape[0] == M
-                            and 1 <= ss.shape[1] <= 256):
+                            and 1 <= ss.shape[1] <= _ss_parts_max(M)):
             return False
     if not (w.K == K and w.N == N and q_out.shape[0] == M and q_out.shape[1] >= H * d):
         raise ValueError(f"qkv: a [{M}, {K}], w {w.shape}, {H}+2*{Hk} heads of {d}, q_out {tuple(q_out.shape)}")

@@ -347,6 +347,59 @@ def test_products_of_some_hundred_rows(M, N, K):
     assert (wide[:, 0] == 7).all() and (wide[:, N + 1:] == 7).all()
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # the kernel that finishes a product of 17 to 64 rows in one launch: one, two and four bands a block (the last block's
+    # bands beyond the matrix among them), 2 and 4 groups of 16 rows, waves with 2 to 9 steps of K; the rows around it
+    (17, 48, 1024), (32, 4112, 1088), (33, 4096, 1024), (64, 8240, 1536), (50, 16, 4160), (20, 5136, 1024), (64, 5120, 1024),
+    (64, 272, 4608), (65, 272, 2048), (16, 272, 2048), (40, 264, 1024), (40, 272, 1032)])
+def test_products_of_17_to_64_rows(M, N, K):
+    t = tuned()
+    a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=2, dtype=BF).to(DEV)
+    want = f64(a) @ f64(w).T
+    pw = pack(w)
+    for out_dtype in (BF, torch.float32):
+        out = torch.full((M + 1, N + 4), 7.0, dtype=out_dtype, device=DEV)
+        t.gemm_bf16(a, pw, out[:M, :N])
+        check(f64(out[:M, :N]), want, out_dtype)
+        assert (out[M] == 7).all() and (out[:, N:] == 7).all()
+    out = torch.empty(M, N, dtype=BF, device=DEV)
+    t.gemm_bf16(a, pw, out, activation=2)
+    check(f64(out), np.maximum(want, 0.0) ** 2, BF)
+    base = gen(M, N, seed=3, scale=2.0).to(DEV)
+    res = base.clone()
+    t.gemm_bf16(a, pw, res, accumulate=True)
+    check(f64(res), f64(base) + want, torch.float32)
+    # with the next norm's row left, and the products behind the norm
+    g = (1 + 0.2 * gen(N, seed=4)).to(DEV)
+    res = base.clone()
+    left = t.gemm_emit_bf16(a, pw, res, g)
+    if left is not None:
+        raw, ss = left
+        x = f64(base) + want
+        check(f64(res), x, torch.float32)
+        parts = min(ss.shape[1], -(-N // 16))              # (the streaming kernel's rows end in up to three unused places)
+        assert np.allclose(f64(ss)[:M, :parts].sum(axis=1), (x ** 2).sum(axis=1), rtol=1e-5)
+        d = np.abs(f64(raw) - bf16_round(x * f64(g)))
+        assert (d <= 2.0 ** -7 * np.abs(x * f64(g)) + 1.5e-5 * np.abs(x).max()).all() and (d > 0).mean() < 0.01
+        if N >= 1024:
+            eps, N2 = 1e-5, 176
+            rstd = 1.0 / np.sqrt((x ** 2).mean(axis=1, keepdims=True) + eps)
+            w2 = gen(2 * N2, N, seed=5, dtype=BF).to(DEV)
+            y = f64(raw) @ f64(w2).T * rstd
+            for out_dtype in (BF, torch.float32):
+                out = torch.empty(M, 2 * N2, dtype=out_dtype, device=DEV)
+                assert t.gemm_pre_bf16(raw, ss, eps, pack(w2), out)
+                check(f64(out), y, out_dtype)
+            out = torch.empty(M, N2, dtype=BF, device=DEV)
+            assert t.swiglu_pre_bf16(raw, ss, eps, pack(w2[:N2].contiguous()), pack(w2[N2:].contiguous()), out)
+            check(f64(out), P.silu(y[:, :N2]) * y[:, N2:], BF)
+    F = N // 2 // 16 * 16
+    if F:
+        out = torch.empty(M, F, dtype=BF, device=DEV)
+        t.swiglu_bf16(a, pack(w[:F].contiguous()), pack(w[F:2 * F].contiguous()), out)
+        check(f64(out), P.silu(want[:, :F]) * want[:, F:2 * F], BF)
+
+
 def test_folded_norm_refuses_what_it_does_not_take():
     t = tuned()
     w = pack(gen(32, 64, dtype=BF).to(DEV))
