@@ -19,7 +19,7 @@ CHIP_UNITS = 256   # compute units the rules below were measured on
 MANY_ROWS_SPLIT_MAX = 1024   # up to here the tiled kernel may cut K into slices to get enough blocks
 SKINNY_MAX_ROWS = 16     # the streaming kernel: up to one 16-row tile of activations
 ROWS_MAX = 64            # the kernel that finishes a product of 17 rows or more in one launch (`gemm_rows_bf16.hip`)
-SPLITK_MAX_ROWS = 128    # the tiled kernel with K cut into slices: 17..128 rows
+SPLITK_MAX_ROWS = 128    # the tiled kernel with K cut into slices: 17..128 rows, where the one above does not take them
 
 
 def _k_split(M: int, N: int, K: int) -> int:
