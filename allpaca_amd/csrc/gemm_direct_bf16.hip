@@ -25,6 +25,7 @@
 // K must be a multiple of 128, N of 4.
 // Reference counterpart: gemm_nt_bf16_tiled_kernel, hip/src/kernels.cpp:634 (no matrix cores there).
 #include "gemm_direct.h"
+#include "host/rules.h"
 #include "mfma.h"
 
 namespace {
@@ -452,7 +453,7 @@ int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* 
   const int k_slice = K / k_split;
   if (M < GEMM_DIRECT_SLICES_MIN_ROWS || !direct_takes(D_STORE_F32, A, lda, partials, N, M, N, k_slice))
     return APC_ERR_UNSUPPORTED;
-  const int nf = pick_bands(M, N, false, k_split);
+  const int nf = M <= apc_rules::MANY_ROWS_SPLIT_MAX ? apc_rules::direct_slices(M, N, k_split).bands : pick_bands(M, N, false, k_split);
   const int nb = 4 * nf * 16;
   const long blocks = 8L * ceil_div((long)ceil_div(N, nb) * ceil_div(M, 128), 8L);
   if (blocks > 0x7fffffffL) return APC_ERR_BAD_ARG;

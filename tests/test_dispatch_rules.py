@@ -126,3 +126,14 @@ def test_the_executors_rules_are_the_wrappers_rules():
                     got = L.apc_host_rule_key_splits(step.n_tiles, heads, pos0 + rows, window, tuned.KEY_SPLITS_MAX,
                                                      tuned.KEY_RANGE_MIN)
                     assert got == want, (rows, pos0, heads, window)
+
+
+@pytest.mark.parametrize("M,N,slices", [(896, 6144, 3), (384, 5120, 6), (300, 5120, 3), (300, 5120, 6), (896, 2048, 6), (512, 4096, 4),
+                                        (512, 6144, 2), (1024, 8192, 4)])
+def test_slices_without_weights_in_lds_fill_their_rounds_by_the_busiest_xcd(M, N, slices):
+    """The tiles of a launch are dealt out to 8 XCDs of 32 compute units by eighths, all slices of a tile to one XCD: the
+    bands a wave takes are not such that a round beyond the first serves a few blocks of one XCD."""
+    from allpaca_amd.kernels import host
+    bands = host.load().apc_host_rule_direct_bands(M, N, slices)
+    busiest = -(-(-(-M // 128) * -(-N // (64 * bands))) // 8) * slices
+    assert busiest / (32 * -(-busiest // 32)) >= 0.7, (bands, busiest)
