@@ -11,10 +11,6 @@ constexpr int GEMM_DIRECT_MIN_ROWS = 1024;
 // SwiGLU of 14,336 outputs, K 4,096: 128 rows (224) 53 / 67, 130 (448) 75 / 59, 256 (448) 79 / 67; of 8,192 outputs, K 3,072:
 // 256 rows (256) 37 / 48, 384 (384) 54 / 49.
 constexpr int GEMM_DIRECT_FEW_ROWS = 129;
-// K in slices (the adding kernel is the same): from so many rows on.  As above with the best number of slices for either:
-// down of an 8B model (4,096 x 14,336) at 256 rows 47 / 48, 384 rows 66 / 67, 512 78 / 70, 768 116 / 110, 1,000 137 / 112;
-// of a 3B model (3,072 x 8,192) 256 rows 29 / 28, 384 37 / 37, 512 46 / 38, 768 59 / 53.
-constexpr int GEMM_DIRECT_SLICES_MIN_ROWS = 257;
 
 // mode: 0 store bfloat16, 1 store float32, 2 add into float32, 3 SwiGLU (W = gate, W2 = up, N = the width of each).
 // True if launch_gemm_direct runs this shape (K a multiple of 128, N and ldc of 4, 16-byte aligned A and C, ...).

@@ -451,7 +451,11 @@ int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* 
                               int k_split, hipStream_t stream) {
   if (k_split < 1 || k_split > 65535 || K % k_split) return APC_ERR_UNSUPPORTED;
   const int k_slice = K / k_split;
-  if (M < GEMM_DIRECT_SLICES_MIN_ROWS || !direct_takes(D_STORE_F32, A, lda, partials, N, M, N, k_slice))
+  if (M <= apc_rules::MANY_ROWS_SPLIT_MAX) {   // the slices that the rule means for this kernel and not for the 128 x 128 tile
+    const apc_rules::Slices rule = apc_rules::slices_many_rows(M, N, K);
+    if (!rule.direct || rule.k_split != k_split) return APC_ERR_UNSUPPORTED;
+  }
+  if (!direct_takes(D_STORE_F32, A, lda, partials, N, M, N, k_slice))
     return APC_ERR_UNSUPPORTED;
   const int nf = M <= apc_rules::MANY_ROWS_SPLIT_MAX ? apc_rules::direct_slices(M, N, k_split).bands : pick_bands(M, N, false, k_split);
   const int nb = 4 * nf * 16;

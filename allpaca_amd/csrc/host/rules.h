@@ -52,19 +52,38 @@ inline DirectSlices direct_slices(int M, int N, int k_split) {
   return best;
 }
 
-// 257..1024 rows, by the expected time (tuned._k_split_direct says what it rests on)
-constexpr int DIRECT_SLICES_MIN_ROWS = 257;
-inline int k_split_direct(int M, int N, int K) {
-  const long tiles = cdiv(M, 128);
-  int best = 1;
-  double least = 0.0;
-  for (int s : {1, 2, 3, 4, 6, 8}) {
-    if (s > 1 && K % (128 * s)) continue;
-    double us = 1e30;
-    for (int nf : {3, 4, 5, 6, 8}) us = std::min(us, (double)cdiv(tiles * cdiv(N, 64 * nf) * s, CHIP_UNITS) * (19.0 + 10.4 * nf));
-    if (s == 1 && tiles * cdiv(N, 128) <= CHIP_UNITS) us = 41.0;
-    us = us * (K / (4096.0 * s)) + (s == 1 ? 7.0 : 4.5 + s * ((double)M * N) * (1.38 / 1048576.0));
-    if (s == 1 || us < least) best = s, least = us;
+// 129..1024 rows: slices of K, and whether the kernel without weights in LDS takes them (tuned._slices_many_rows says what
+// it rests on).  Expected microseconds:
+struct Slices {
+  int k_split;
+  bool direct;
+};
+constexpr int DIRECT_SLICES_MIN_ROWS = 257, DIRECT_MIN_ROWS = 1024;
+inline double outputs_us(int M, int N) { return (double)M * N / 1048576.0; }
+inline double direct_slices_us(int M, int N, int K, int s) {
+  return direct_slices(M, N, s).us * (K / (4096.0 * s)) + 8.0 + (1.5 * s + 0.7) * outputs_us(M, N);
+}
+inline double tiled_slices_us(int M, int N, int K, int s) {
+  const long columns = cdiv(N, 128), blocks = cdiv(M, 128) * columns * s, full = (blocks - 1) / 512, rest = blocks - 512 * full;
+  const double first = (double)std::min(rest, (long)CHIP_UNITS) / CHIP_UNITS;
+  double us = 64.5 * full + (rest > CHIP_UNITS ? 48.7 : 27.3) + 12.6 * first;
+  if (columns % 8) us *= 1.0 + 0.23 * std::min(blocks, (long)CHIP_UNITS) / CHIP_UNITS;
+  return us * (K / (4096.0 * s)) + 8.6 + (1.6 * s + 0.3) * outputs_us(M, N);
+}
+inline double whole_us(int M, int N, int K) {
+  const long tiles = cdiv(M, 128) * cdiv(N, 128);
+  if (M < DIRECT_MIN_ROWS && tiles <= CHIP_UNITS) return 11.0 + (30.5 + 9.0 * tiles / CHIP_UNITS) * (K / 4096.0);
+  return 12.0 + direct_slices(M, N, 1).us * (K / 4096.0);
+}
+inline Slices slices_many_rows(int M, int N, int K) {
+  Slices best{k_split_many_rows(M, N, K), false};
+  if (M < DIRECT_SLICES_MIN_ROWS || M > MANY_ROWS_SPLIT_MAX || K % 128 || N % 4) return best;
+  double least = 0.96 * (best.k_split == 1 ? whole_us(M, N, K) : tiled_slices_us(M, N, K, best.k_split));
+  if (best.k_split > 1 && whole_us(M, N, K) < least) best = {1, false}, least = whole_us(M, N, K);
+  for (int s : {2, 3, 4, 6, 8}) {
+    if (K % (128 * s) || K < 256 * s) continue;
+    const double us = direct_slices_us(M, N, K, s);
+    if (us < least) best = {s, true}, least = us;
   }
   return best;
 }
@@ -72,8 +91,7 @@ inline int k_split_direct(int M, int N, int K) {
 inline int tiled_k_split(int M, int N, int K, bool gated = false) {
   if (M <= SPLITK_MAX_ROWS) return k_split(M, N, K);
   if (M > MANY_ROWS_SPLIT_MAX) return 1;
-  if (M >= DIRECT_SLICES_MIN_ROWS && !gated && K % 256 == 0 && N % 4 == 0) return k_split_direct(M, N, K);
-  return k_split_many_rows(M, N, K);
+  return gated ? k_split_many_rows(M, N, K) : slices_many_rows(M, N, K).k_split;
 }
 
 // sums of x^2 a row that the products behind a norm take

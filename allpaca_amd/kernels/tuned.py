@@ -50,26 +50,57 @@ def _k_split_many_rows(M: int, N: int, K: int) -> int:
 
 
 DIRECT_SLICES_MIN_ROWS = 257   # the kernel that keeps the weights out of LDS takes slices from here on
+DIRECT_MIN_ROWS = 1024         # and K in one piece whatever the columns
 
 
-def _k_split_direct(M: int, N: int, K: int) -> int:
-    """Slices of K for 257..1024 rows, by the expected microseconds: rounds of 256 blocks of 128 rows x 64 nf columns at
-    19 + 10.4 nf a round and 4,096 columns of K (`gemm_direct_bf16.hip`); the slices' way through memory, 4.5 and 1.38 a slice
-    and 2^20 outputs; K whole on 128 x 128 tiles 41 (more than 256 of them: the rounds above), and 7 for what the adding
-    kernel would have done on the way, the norm's row or the rotation.  Against 9 matrices of 1B to 8B models at 384 to 1,000
-    rows the times are off by up to 4 us (512 rows, 4,096 x 14,336: 2 / 4 / 8 slices 93.6 / 70.4 / 73.9, expected 98 / 69 / 72)."""
-    tiles = -(-M // 128)
-    best, least = 1, 0.0
-    for s in (1, 2, 3, 4, 6, 8):
-        if s > 1 and K % (128 * s):
+def _direct_slices_us(M: int, N: int, s: int) -> float:
+    """Microseconds of that kernel for 4,096 columns of K a slice (`direct_slices` in `csrc/host/rules.h`)."""
+    us = []
+    for nf in (3, 4, 5, 6, 8):
+        tiles = -(-M // 128) * -(-N // (64 * nf))
+        rounds = -(-(-(-tiles // 8) * s) // (CHIP_UNITS // 8))
+        us.append(rounds * (12.0 + nf * (7.5 + 3.8 * (tiles * s) / (rounds * CHIP_UNITS))))
+    return min(us)
+
+
+def _slices_many_rows(M: int, N: int, K: int):
+    """(slices of K, whether the kernel without weights in LDS takes them) for 129..1024 rows.  From 257 rows on that
+    kernel's slices, which have to be of one length in pieces of 128 columns, are held against what the 128 x 128 tile
+    does (its slices or K whole, `_k_split_many_rows`) by the expected microseconds: `_direct_slices_us`; two blocks of the
+    tile share a unit, 27 to 40 for 256 of them and 64 for 512, up to 1.23 times that where the column tiles are no multiple of
+    the 8 XCDs, which then all fetch all of W; the adding kernel 9 and 1.6 a slice and 2^20 outputs; K whole 6 more for
+    what the adding kernel would have done on the way, the norm's row or the rotation.  Against 8,500 products of 257 to 1,024
+    rows (K 768 to 14,336 into 640 to 11,008 columns, 900 sizes in 1 to 8 slices on either kernel) the times are off by 5 %
+    (root mean square), and what is chosen takes 0.94 of the tile's time in the mean, 1.08 at worst.  K without many
+    divisors stays with the tile, whose slices need none: 384 rows, K 15,104 into 640 columns 84 us in the two slices that
+    the other kernel has, 33 in five.  512 rows, 4,096 x 14,336: 78 in three slices on the tile, 70 in four on the other."""
+    s = _k_split_many_rows(M, N, K)
+    if not (DIRECT_SLICES_MIN_ROWS <= M <= MANY_ROWS_SPLIT_MAX) or K % 128 or N % 4:
+        return s, False
+    outputs = M * N / 1048576.0
+    tiles = -(-M // 128) * -(-N // 128)
+    if M < DIRECT_MIN_ROWS and tiles <= CHIP_UNITS:
+        whole = 11.0 + (30.5 + 9.0 * tiles / CHIP_UNITS) * (K / 4096.0)
+    else:
+        whole = 12.0 + _direct_slices_us(M, N, 1) * (K / 4096.0)
+    best, direct, least = s, False, 0.96 * whole
+    if s > 1:
+        blocks = tiles * s
+        full = (blocks - 1) // 512
+        rest = blocks - 512 * full
+        us = 64.5 * full + (48.7 if rest > CHIP_UNITS else 27.3) + 12.6 * (min(rest, CHIP_UNITS) / CHIP_UNITS)
+        if -(-N // 128) % 8:
+            us *= 1.0 + 0.23 * min(blocks, CHIP_UNITS) / CHIP_UNITS
+        least = 0.96 * (us * (K / (4096.0 * s)) + 8.6 + (1.6 * s + 0.3) * outputs)
+        if whole < least:
+            best, least = 1, whole
+    for s in (2, 3, 4, 6, 8):
+        if K % (128 * s) or K < 256 * s:
             continue
-        us = min(-(-(tiles * -(-N // (64 * nf)) * s) // CHIP_UNITS) * (19.0 + 10.4 * nf) for nf in (3, 4, 5, 6, 8))
-        if s == 1 and tiles * -(-N // 128) <= CHIP_UNITS:
-            us = 41.0
-        us = us * (K / (4096.0 * s)) + (7.0 if s == 1 else 4.5 + s * (M * N) * (1.38 / 1048576.0))
-        if s == 1 or us < least:
-            best, least = s, us
-    return best
+        us = _direct_slices_us(M, N, s) * (K / (4096.0 * s)) + 8.0 + (1.5 * s + 0.7) * outputs
+        if us < least:
+            best, direct, least = s, True, us
+    return best, direct
 
 
 def _tiled_k_split(M: int, N: int, K: int, gated: bool = False) -> int:
@@ -78,9 +109,7 @@ def _tiled_k_split(M: int, N: int, K: int, gated: bool = False) -> int:
         return _k_split(M, N, K)
     if M > MANY_ROWS_SPLIT_MAX:
         return 1
-    if M >= DIRECT_SLICES_MIN_ROWS and not gated and K % 256 == 0 and N % 4 == 0:
-        return _k_split_direct(M, N, K)
-    return _k_split_many_rows(M, N, K)
+    return _k_split_many_rows(M, N, K) if gated else _slices_many_rows(M, N, K)[0]
 
 
 def _rows_take(a: torch.Tensor, w: PackedWeight, wu: Optional[PackedWeight], out: torch.Tensor, N: int, mode: int) -> bool:

@@ -137,3 +137,29 @@ def test_slices_without_weights_in_lds_fill_their_rounds_by_the_busiest_xcd(M, N
     bands = host.load().apc_host_rule_direct_bands(M, N, slices)
     busiest = -(-(-(-M // 128) * -(-N // (64 * bands))) // 8) * slices
     assert busiest / (32 * -(-busiest // 32)) >= 0.7, (bands, busiest)
+
+
+@pytest.mark.parametrize("M,N,K,slices,direct", [
+    # K without many divisors: as many slices as the 128 x 128 tile wants (measured: 33, 40, 48, 64 and 37 us; in the two
+    # slices that the kernel without weights in LDS has 84, 68, 67, 72 and 67)
+    (384, 640, 15104, 5, False), (500, 2048, 11008, 4, False), (384, 3072, 11008, 3, False), (384, 4096, 11008, 2, False), (384, 1280, 11008, 5, False),
+    # slices on the kernel without weights in LDS
+    (512, 4096, 14336, 4, True), (512, 6144, 4096, 2, True), (384, 3072, 8192, 4, True),
+    # at 1,024 rows K in one piece is that kernel's too, and its time counts, not the tile's
+    (1024, 5120, 3072, 1, False), (1024, 4096, 14336, 2, True),
+    # below 257 rows, K no multiple of 128
+    (256, 4096, 14336, 4, False), (300, 640, 1288, 5, False)])
+def test_slices_of_k_for_some_hundred_rows(M, N, K, slices, direct):
+    from allpaca_amd.kernels import tuned
+    assert tuned._slices_many_rows(M, N, K) == (slices, direct)
+
+
+def test_the_kernel_library_takes_the_slices_that_the_wrappers_mean_for_it():
+    from allpaca_amd.kernels import host, tuned
+    L = host.load()
+    for M in (129, 200, 256, 257, 300, 384, 500, 512, 640, 768, 896, 1000, 1023, 1024):
+        for N in (192, 640, 1000, 1002, 1920, 2048, 3072, 4096, 5120, 6144, 8192, 11008, 28672):
+            for K in (128, 192, 512, 768, 1152, 1288, 2048, 3072, 4096, 5376, 8192, 11008, 14336, 15104):
+                s, direct = tuned._slices_many_rows(M, N, K)
+                assert (L.apc_host_rule_tiled_k_split(M, N, K), bool(L.apc_host_rule_slices_direct(M, N, K))) == (s, direct), (M, N, K)
+                assert not direct or (s > 1 and K % (128 * s) == 0)
