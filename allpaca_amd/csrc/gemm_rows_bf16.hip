@@ -5,7 +5,7 @@
 // MFMA operands, each read once by one wave, and a block's eight waves take an eighth of K each and meet in LDS, so no sums
 // go through memory and no second kernel adds them.  What is new with more rows is the activations: every block reads all
 // M x K of them, and they come out of L2 at 131 GB/s a compute unit in whole lines of 128 bytes.  That is why a block takes
-// up to four bands of 16 outputs where there are bands enough (pick_bands_of).
+// up to four bands of 16 outputs where there are bands enough.
 //  * A step is 64 columns of K: of NB bands two tiles each, and of every 16 rows two loads of 8 rows x 128 bytes, eight
 //    lanes side by side a line.  (Loads whose lanes sit where the operands want them, eight rows in eight lanes, come at
 //    35 GB/s a compute unit: 64 rows x 4,096 columns of K into 4,096 outputs 20.4 us, so 14.4.)  They go
@@ -14,11 +14,12 @@
 //  * DEPTH register sets of a step: what a compute unit has in flight is 8 waves x DEPTH x NB x 2 KiB of weights.
 //  * Operands as in skinny_gemm_bf16.hip (weights first): a lane ends with four consecutive outputs of a row.
 // Bound by a fixed part of some 5 us (first loads, the waves' meeting, the store) and the activations' way: with the weights
-// beside them a compute unit gets 50-60 GB/s in all.  Times, and where the tiled kernel is the better one: gemm_rows_takes.
+// beside them a compute unit gets 33-60 GB/s in all.  Times, and where the tiled kernel is the better one: gemm_rows_takes.
 // K must be a multiple of 64, from 1,024 on; N of 16.
 // The order of additions for an output depends on K alone.
 // Reference counterpart: gemm_nt_bf16_tiled_kernel, hip/src/kernels.cpp:634 (no matrix cores there).
 #include "gemm_rows.h"
+#include "host/rules.h"
 #include "mfma.h"
 
 namespace {
@@ -238,18 +239,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rows_gemm_kernel(const bf16_t* 
   }
 }
 
-// Bands of weights a block: blocks of one compute unit each, in rounds of 256; a band costs what 64 rows of activations do
-// (weights come from memory, activations from L2 at a multiple of the rate).
-long rounds_of(int bands, int nb, bool pairs) { return ceil_div((long)ceil_div(bands, pairs ? nb / 2 : nb), 256L); }
-int pick_bands_of(int bands, bool pairs, int row_tiles) {
-  int best = 0;
-  long least = 0;
-  for (int nb : {1, 2, 4}) {
-    if (pairs && nb == 1) continue;
-    const long cost = rounds_of(bands, nb, pairs) * (nb * 4 + row_tiles);
-    if (!best || cost < least) best = nb, least = cost;
-  }
-  return best;
+int kind_of(int mode) {
+  return mode == R_SWIGLU ? apc_rules::ROWS_GATED : mode == R_QKV_ROPE ? apc_rules::ROWS_QKV : apc_rules::ROWS_PLAIN;
 }
 
 template <int MODE, bool PRE, bool EMIT>
@@ -266,7 +257,7 @@ int launch(const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C,
   if constexpr (MODE == R_QKV_ROPE) {
     ROWS_BY_M(2, bands / 2);
   } else {
-    const int nb = pick_bands_of(bands, MODE == R_SWIGLU, mt);
+    const int nb = apc_rules::rows_bands(M, N, K, kind_of(MODE));
     if (nb == 4) { ROWS_BY_M(4, ceil_div(bands, out_bands(MODE, 4))); }
     else if (nb == 2) { ROWS_BY_M(2, ceil_div(bands, out_bands(MODE, 2))); }
     else if constexpr (MODE != R_SWIGLU) { ROWS_BY_M(1, bands); }
@@ -280,20 +271,16 @@ int launch(const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C,
 bool aligned(const void* p, unsigned n) { return ((uintptr_t)p & (n - 1)) == 0; }
 }  // namespace
 
-// The activations that a compute unit reads decide against the tiled kernel, which reads a slice of them: rows x columns
-// of K x rounds of blocks up to 2^18, half of it where there is more than one round.  Microseconds in a step of 64 rows at
-// 3B shapes, tiled kernel and adding kernel / this: q, k, v with rotation and cache 18.9 / 16.5, o_proj with the norm's row
-// 14.4 / 12.0, SwiGLU of 8,192 27.1 / 24.4.  In a loop: 32 rows, K 2,048 into 3,072 outputs 13 / 6.1, K 4,096 into 4,096
-// 16.6 / 10.7, K 8,192 into 3,072 21 / 16.6; 64 rows, K 4,096 into 4,096 17.7 / 14.2; beyond: 64 rows, K 8,192 into 3,072
-// 18.4 / 23.6, 32 rows, K 14,336 into 4,096 27.4 / 32.9, SwiGLU of 14,336 (two rounds) 41.8 / 44.4.
+// Where the tiled kernel is the better one: apc_rules::rows_bands.  Microseconds in a step of 64 rows at 3B shapes, tiled kernel
+// and adding kernel / this: q, k, v with rotation and cache 18.9 / 16.8, o_proj with the norm's row 14.4 / 12.2, SwiGLU of
+// 8,192 27.1 / 23.7.  In a loop: 32 rows, K 2,048 into 3,072 outputs 13 / 6.1, K 4,096 into 4,096 16.6 / 10.7; 64 rows, K 4,096
+// into 4,096 17.7 / 14.2; the other way: 64 rows, K 8,192 into 3,072 18.4 / 23.6, 32 rows, K 14,336 into 4,096 27.4 / 32.9.
 bool gemm_rows_takes(int mode, const void* A, int lda, const void* W, const void* W2, const void* C, int ldc, int M, int N, int K) {
   const bool out32 = mode == R_STORE_F32 || mode == R_ACC_F32;
   if (M <= 16 || M > GEMM_ROWS_MAX || K < GEMM_ROWS_MIN_K || K % 64 || N <= 0 || N % 16 || lda % 8 || lda >= (1 << 24) || ldc % 4 ||
       !aligned(A, 16) || !aligned(W, 16) || !aligned(W2, 16) || !aligned(C, out32 ? 16 : 8))
     return false;
-  const int bands = N / 16, mt = ceil_div(M, 16);
-  const long rounds = mode == R_QKV_ROPE ? rounds_of(bands, 2, false) : rounds_of(bands, pick_bands_of(bands, mode == R_SWIGLU, mt), mode == R_SWIGLU);
-  return rounds * mt * 16 * K <= (rounds > 1 ? 1L << 17 : 1L << 18);
+  return apc_rules::rows_bands(M, N, K, kind_of(mode)) > 0;
 }
 
 int launch_gemm_rows(int mode, const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C, int ldc, int M, int N, int K,

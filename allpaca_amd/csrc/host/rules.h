@@ -94,6 +94,45 @@ inline int tiled_k_split(int M, int N, int K, bool gated = false) {
   return gated ? k_split_many_rows(M, N, K) : slices_many_rows(M, N, K).k_split;
 }
 
+// Products of 17 to 64 rows: bands of 16 outputs a block of gemm_rows_bf16.hip takes, or 0 where the tiled kernel is expected
+// to be faster.  Microseconds, N the width of each matrix of a gated product.  Fitted to 6,134 products (17 to 64 rows, K 1,024
+// to 14,336, 320 to 32,000 columns; off by 6 to 8 %, root mean square): of 1,988 sizes what is chosen takes 0.86 of the tiled
+// kernel's time in the mean and 1.07 at worst.
+//  * gemm_rows_bf16.hip: every block reads its bands' weights and all activations, and a round has a fixed part.  32 rows,
+//    K 8,192, q, k and v of 640 columns are 20 blocks that each read a megabyte: 22 us, and 13 in slices on the tiled kernel.
+//  * The tiled kernel: steps of 64 columns, two blocks a unit, the slices through memory and a second kernel.  With columns
+//    enough it needs neither slices nor that kernel: 64 rows, K 1,024, SwiGLU of 14,336 15 us there, 19 in two rounds here.
+enum RowsKind : int { ROWS_PLAIN = 0, ROWS_GATED = 1, ROWS_QKV = 2 };
+inline double rows_us(int M, int N, int K, int bands, int kind, long* rounds) {
+  const long blocks = cdiv(N / 16, kind == ROWS_GATED ? bands / 2 : bands), r = cdiv(blocks, CHIP_UNITS);
+  const double fill = (double)blocks / (double)(r * CHIP_UNITS), tiles = M / 16.0;
+  *rounds = r;
+  return 3.8 + 3.0 * (r - 1) + r * (K / 1024.0) * (bands * (0.56 + 0.58 * fill) + 0.5 * tiles - (bands == 1 ? 0.37 : 0.25)) +
+         (kind == ROWS_QKV ? 0.58 : 0.1) * tiles;
+}
+inline double tiled_rows_us(int M, int N, int K, int kind) {
+  const int columns = kind == ROWS_GATED ? 2 * N : N, s = k_split(M, columns, K);
+  const double steps = (double)cdiv(K / 64, s), full = (double)(cdiv(columns, 128) * s) / CHIP_UNITS;
+  double us = 4.5 + steps * (0.33 + 0.32 * full + (full > 1.0 ? 0.33 : 0.0));
+  if (s > 1) us += 3.2 + 2.0e-6 * s * M * (double)columns;
+  if (kind == ROWS_GATED) us += 0.5;
+  if (kind == ROWS_QKV) us += s > 1 ? 0.4 : 9.0;   // K whole: rotation and cache write in a kernel of their own
+  return us;
+}
+inline int rows_bands(int M, int N, int K, int kind) {
+  if (cdiv(M, 16) * 16 * (long)K > 1L << 18) return 0;   // beyond, 17 rows, K 11,008 into 320 to 1,280 columns: up to 1.27 of the tiled kernel's time
+  int best = 0;
+  double least = tiled_rows_us(M, N, K, kind);
+  for (int bands : {1, 2, 4}) {
+    if ((kind == ROWS_GATED && bands == 1) || (kind == ROWS_QKV && bands != 2)) continue;
+    long rounds;
+    const double us = rows_us(M, N, K, bands, kind, &rounds);
+    // rounds further on overlap less than expected: 17 rows, K 4,096 into 32,000 columns 53 us, tiled 47
+    if (us < least && (rounds == 1 || rounds * K <= (kind == ROWS_PLAIN ? 4096 : 2048))) best = bands, least = us;
+  }
+  return best;
+}
+
 // sums of x^2 a row that the products behind a norm take
 inline int ss_parts_max(int M) { return M <= ROWS_MAX ? 1024 : 256; }
 

@@ -163,3 +163,17 @@ def test_the_kernel_library_takes_the_slices_that_the_wrappers_mean_for_it():
                 s, direct = tuned._slices_many_rows(M, N, K)
                 assert (L.apc_host_rule_tiled_k_split(M, N, K), bool(L.apc_host_rule_slices_direct(M, N, K))) == (s, direct), (M, N, K)
                 assert not direct or (s > 1 and K % (128 * s) == 0)
+
+
+@pytest.mark.parametrize("kind,M,N,K,bands", [
+    # few columns and a long K (0: plain, 1: gated, 2: q, k and v): a few blocks read everything, in slices many share it
+    (2, 32, 640, 8192, 0), (2, 48, 640, 5440, 0), (2, 32, 1280, 8192, 0), (2, 64, 640, 4096, 0), (1, 32, 320, 8192, 0), (0, 48, 320, 5440, 0),
+    # more than a round of blocks, where the tiled kernel needs no slices
+    (1, 64, 14336, 1024, 0), (1, 17, 32000, 1024, 0), (0, 64, 32000, 1024, 0),
+    # what one launch is for
+    (0, 64, 4096, 4096, 1), (0, 64, 3072, 3072, 1), (2, 64, 5120, 3072, 2), (1, 64, 8192, 3072, 4), (0, 32, 3072, 2048, 1), (0, 32, 3072, 8192, 1), (2, 17, 3072, 2048, 2),
+    # (the tiled kernel with a few blocks more than compute units)
+    (0, 17, 10240, 2048, 4), (0, 37, 8320, 4032, 4)])
+def test_products_of_17_to_64_rows_in_one_launch_where_that_is_faster(kind, M, N, K, bands):
+    from allpaca_amd.kernels import host
+    assert host.load().apc_host_rule_rows_bands(M, N, K, kind) == bands
