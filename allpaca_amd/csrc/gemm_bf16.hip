@@ -705,7 +705,11 @@ APC_EXPORT int apc_gemm_rows_takes(int mode, const void* A, int lda, const void*
   return gemm_rows_takes(mode_is_act(mode) ? G_ACT : mode, A, lda, W, Wu, C, ldc, M, N, K);
 }
 // residual += A . W^T on that kernel, with raw as in apc_gemm_splitk_emit_bf16 and ss [M][N / 16] sums of residual^2 per row
-// and band of 16 columns
+// and band of 16 columns; for what apc_gemm_rows_emit_takes (raw 8-byte aligned, its row stride a multiple of 4)
+APC_EXPORT int apc_gemm_rows_emit_takes(const void* A, int lda, const void* W, const float* residual, int ldc, int M, int N,
+                                        int K, const float* g) {
+  return aligned16(g) && gemm_rows_takes(G_ACC_F32, A, lda, W, nullptr, residual, ldc, M, N, K);
+}
 APC_EXPORT int apc_gemm_rows_emit_bf16(const void* A, int lda, const void* W, float* residual, int ldc, int M, int N, int K,
                                        const float* g, void* raw, int ldr, float* ss, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;

@@ -189,7 +189,8 @@ int gemm_emit_bf16(Program& P, const Buf& a, const ApcMatrix& w, const Buf& resi
     emit.filled = true;
     return 1;
   }
-  if (M > SKINNY_MAX_ROWS && N / 16 <= ss_parts_max(M) && apc_gemm_rows_takes(2, a.p, a.ld, w.data, nullptr, residual.p, residual.ld, M, N, K)) {
+  if (M > SKINNY_MAX_ROWS && N / 16 <= ss_parts_max(M) &&
+      apc_gemm_rows_emit_takes(a.p, a.ld, w.data, (const float*)residual.p, residual.ld, M, N, K, emit.g)) {
     emit.raw = P.emit_rows(emit, M, N);
     emit.ss_rows = M;
     emit.ss_cols = N / 16;

@@ -247,7 +247,8 @@ def gemm_emit_bf16(a: torch.Tensor, w: PackedWeight, residual: torch.Tensor, g: 
                                                ws.data_ptr() if ws is not None else 0, _ops._stream()),
                    "gemm_direct_emit_bf16")
         return raw, ss
-    if N // 16 <= _ss_parts_max(M) and _rows_take(a, w, None, residual, N, 2):
+    if SKINNY_MAX_ROWS < M <= ROWS_MAX and N // 16 <= _ss_parts_max(M) and L.apc_gemm_rows_emit_takes(
+            a.data_ptr(), lda, w.data.data_ptr(), residual.data_ptr(), ldc, M, N, K, g.data_ptr()):
         raw = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
         ss = torch.empty((M, N // 16), dtype=torch.float32, device=a.device)
         _lib.check(L.apc_gemm_rows_emit_bf16(a.data_ptr(), lda, w.data.data_ptr(), residual.data_ptr(), ldc, M, N, K,

@@ -400,6 +400,26 @@ def test_products_of_17_to_64_rows(M, N, K):
         check(f64(out), P.silu(want[:, :F]) * want[:, F:2 * F], BF)
 
 
+@pytest.mark.parametrize("M", [8, 40, 100, 300])
+def test_product_into_the_residual_takes_a_norm_weight_off_16_bytes(M):
+    t = tuned()
+    N, K = 272, 1024
+    a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=2, dtype=BF).to(DEV)
+    base, g = gen(M, N, seed=3).to(DEV), (1 + 0.2 * gen(N + 1, seed=4)).to(DEV)[1:]
+    assert g.data_ptr() % 16 == 4
+    res = base.clone()
+    raw, ss = t.gemm_emit_bf16(a, pack(w), res, g)
+    x = f64(base) + f64(a) @ f64(w).T
+    check(f64(res), x, torch.float32)
+    d = np.abs(f64(raw) - bf16_round(x * f64(g)))
+    assert (d <= 2.0 ** -7 * np.abs(x * f64(g)) + 1.5e-5 * np.abs(x).max()).all() and (d > 0).mean() < 0.01
+    rstd = 1.0 / np.sqrt((x ** 2).mean(axis=1, keepdims=True) + 1e-5)
+    w2 = gen(64, N, seed=5, dtype=BF).to(DEV)
+    out = torch.empty(M, 64, dtype=BF, device=DEV)
+    assert t.gemm_pre_bf16(raw, ss, 1e-5, pack(w2), out)
+    check(f64(out), f64(raw) @ f64(w2).T * rstd, BF)
+
+
 def test_folded_norm_refuses_what_it_does_not_take():
     t = tuned()
     w = pack(gen(32, 64, dtype=BF).to(DEV))
