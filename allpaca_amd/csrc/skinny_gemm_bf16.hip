@@ -135,9 +135,10 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
     else wb[b] = W + (size_t)min(band0 + b, bands - 1) * chunks * TILE_ELEMS + lane * 8;
   }
   // row group g: lanes i < 8 take row g * 8 + i of a pair's first tile, lanes i >= 8 row g * 8 + i - 8 of its second
+  // (in pieces of 8 elements: 15 rows of any stride an int holds fit 32 bits)
   uint32_t arow[MG];
 #pragma unroll
-  for (int g = 0; g < MG; ++g) arow[g] = (uint32_t)min(g * 8 + i % 8, M - 1) * (uint32_t)lda + (i / 8) * 32 + c * 8;
+  for (int g = 0; g < MG; ++g) arow[g] = (uint32_t)min(g * 8 + i % 8, M - 1) * (uint32_t)(lda / 8) + (i / 8) * 4 + c;
 
   // acc[b][g][t]: the tiles t of the pairs; of its 16 columns the group's rows are those of the lanes i / 8 == t
   floatx4 acc[NB][MG][2];
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
       for (int b = 0; b < NB; ++b) r.w[b][u] = load_frag_once(wb[b] + (size_t)(ch + u) * TILE_ELEMS);
       if (u % 2 == 0) {
 #pragma unroll
-        for (int g = 0; g < MG; ++g) r.a[g][u / 2] = load_frag(A + (ch + u) * 32 + arow[g]);
+        for (int g = 0; g < MG; ++g) r.a[g][u / 2] = load_frag(A + (ch + u) * 32 + (size_t)arow[g] * 8);
       }
     }
   };
@@ -436,7 +437,7 @@ static int launch_skinny(const bf16_t* A, int lda, const bf16_t* W, const bf16_t
 }
 
 static bool operands_ok(const void* A, int lda, const void* W, int M, int K) {
-  return M <= 16 && K % 8 == 0 && lda % 8 == 0 && lda < (1 << 28) && aligned16(A) && aligned16(W);  // (32-bit offsets of 16 rows)
+  return M <= 16 && K % 8 == 0 && lda % 8 == 0 && aligned16(A) && aligned16(W);
 }
 
 // W: tiled layout of an [N, K] matrix.  mode: 0 store bfloat16, 1 store float32, 2 add into float32, 17 .. 19: an

@@ -95,6 +95,29 @@ def test_gemm_bf16_strided_views_and_padding_rows_untouched():
     assert (wide[:, :8] == 3.0).all() and (wide[:, 58:] == 3.0).all()
 
 
+@pytest.mark.parametrize("M", [1, 2, 9, 16])
+def test_few_rows_a_long_way_apart(M):
+    """A row stride of 2^28 elements and more (for one row it means nothing): offsets beyond 32 bits."""
+    t = tuned()
+    N, K, stride = 48, 264, (1 << 28) + 8
+    a0, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=2, dtype=BF).to(DEV)
+    a = torch.empty((M - 1) * stride + K, dtype=BF, device=DEV).as_strided((M, K), (stride, 1))
+    a.copy_(a0)
+    assert a.stride(0) == stride
+    want = f64(a0) @ f64(w).T
+    out = torch.empty(M, N, dtype=BF, device=DEV)
+    t.gemm_bf16(a, pack(w), out)
+    check(f64(out), want, BF)
+    res, g = gen(M, N, seed=3).to(DEV), torch.ones(N, device=DEV)
+    x = f64(res) + want
+    raw, _ = t.gemm_emit_bf16(a, pack(w), res, g)
+    check(f64(res), x, torch.float32)
+    check(f64(raw), x, BF)
+    out = torch.empty(M, 16, dtype=BF, device=DEV)
+    t.swiglu_bf16(a, pack(w[:16].contiguous()), pack(w[16:32].contiguous()), out)
+    check(f64(out), P.silu(want[:, :16]) * want[:, 16:32], BF)
+
+
 def test_widths_the_mfma_kernels_do_not_take_stay_row_major_and_run_on_the_plain_kernel():
     from allpaca_amd.kernels import ops
     a, w = gen(5, 13, seed=1, dtype=BF).to(DEV), gen(7, 13, seed=2, dtype=BF).to(DEV)   # K = 13
