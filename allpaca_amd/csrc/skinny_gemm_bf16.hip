@@ -86,15 +86,21 @@ struct SkRope {
   int P, H, Hk, d;
 };
 
-// Tiles per band and step, and blocks that share a compute unit.  SwiGLU on a wide layer has more blocks than
-// compute units and each block streams 2 bands: with steps of 2 tiles a block of 8 waves needs under 128 registers
-// a lane, two blocks share a unit, and one block's first loads and final reduction hide behind the other's stream
-// (8B shapes, 8 rows: 48.0 -> 44.4 us; the bytes in flight per unit stay the same).
+// Tiles per band and step, and the waves a SIMD that the compiler is asked to leave registers for (512 a lane in all).
+// SwiGLU on a wide layer has more blocks than compute units and each block streams 2 bands: with steps of 2 tiles a wave
+// needs no more than 128 registers, two blocks of 8 waves share a unit, and one block's first loads and final reduction
+// hide behind the other's stream (8B shapes, 8 rows: 48.0 -> 44.4 us; the bytes in flight per unit stay the same).  For 9-16
+// rows this has to be asked for: left to itself the compiler took 134 registers with a folded norm, one block a unit (with
+// it, and the norm's sums added behind the stream, 9 rows at 8B shapes 42.2 -> 38.9 us, 16 rows 44.3 -> 40.9; q, k and v of
+// 16 rows stored 18.0 -> 16.4).
 constexpr int sk_step(int mode) { return mode == SK_SWIGLU ? 2 : SK_U; }
-constexpr int sk_blocks(int mode, int wpb) { return (mode == SK_SWIGLU && wpb == 8) ? 2 : 1; }
+constexpr int sk_waves(int mg, int mode, int nb, int wpb, bool pre) {
+  if (mode == SK_SWIGLU || nb == 1) return pre || mg == 2 ? 4 : mode == SK_ACC_F32 ? 5 : 6;
+  return mg == 2 && wpb == 4 && !(mode == SK_QKV_ROPE && pre) ? 3 : 1;
+}
 
 template <int MG, int MODE, int NB, int WPB, bool PRE, bool EMIT>
-__global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda,
+__global__ __launch_bounds__(WPB * 64, sk_waves(MG, MODE, NB, WPB, PRE)) void skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda,
                                                                const bf16_t* __restrict__ W,
                                                                const bf16_t* __restrict__ W2, int chunks,
                                                                void* __restrict__ C, int ldc, int M, int N, int K,
@@ -180,26 +186,27 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
   // Behind the first loads of the stream, and needed only at the end: the sums of x^2 that the emitting product
   // left (PRE; the 4 * WPB (wave, c) pairs of the block take groups of 4 bands in turn, the pieces meet in LDS with
   // the partial sums of the product), and what the finishing wave of an output band adds to (residual, EMIT: g).
+  // Two row groups' steps leave registers for two of these loads, which wait for their sum until the stream is through.
+  constexpr int AT_ONCE = MG == 1 ? SS_LOADS : 2;
   float ss_piece = 0.f;
+  floatx4 ss_v[AT_ONCE];
+  auto ss_load = [&](int j) {
+    const int q = wave * 4 + c + j * WPB * 4;
+    return q * 4 < norm.ld_ss ? *reinterpret_cast<const floatx4*>(norm.ss + (size_t)i * norm.ld_ss + q * 4)
+                              : floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto ss_add = [&](const floatx4& v, int j) {
+    const int q = wave * 4 + c + j * WPB * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (q * 4 + e < norm.n_ss) ss_piece += v[e];
+  };
   if constexpr (PRE) {
-    const int groups = norm.ld_ss / 4;
-    constexpr int AT_ONCE = MG == 1 ? SS_LOADS : SS_LOADS / 4;   // (two groups' steps leave registers for few)
 #pragma unroll
-    for (int j0 = 0; j0 < SS_LOADS; j0 += AT_ONCE) {
-      floatx4 v[AT_ONCE];
+    for (int j = 0; j < AT_ONCE; ++j) ss_v[j] = ss_load(j);
+    if constexpr (MG == 1) {
 #pragma unroll
-      for (int j = 0; j < AT_ONCE; ++j) {
-        const int q = wave * 4 + c + (j0 + j) * WPB * 4;
-        v[j] = q < groups ? *reinterpret_cast<const floatx4*>(norm.ss + (size_t)i * norm.ld_ss + q * 4)
-                          : floatx4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int j = 0; j < AT_ONCE; ++j) {
-        const int q = wave * 4 + c + (j0 + j) * WPB * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (q * 4 + e < norm.n_ss) ss_piece += v[j][e];
-      }
+      for (int j = 0; j < AT_ONCE; ++j) ss_add(ss_v[j], j);
     }
   }
   constexpr int ITEMS = OUT_BANDS;  // bands to finish: wave w finishes band w
@@ -260,6 +267,12 @@ __global__ __launch_bounds__(WPB * 64, sk_blocks(MODE, WPB)) void skinny_gemm_ke
   }
 
   if constexpr (PRE) {
+    if constexpr (MG == 2) {
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j) ss_add(ss_v[j], j);
+#pragma unroll 1
+      for (int j = AT_ONCE; j * WPB * 16 < norm.ld_ss; ++j) ss_add(ss_load(j), j);   // more bands than 32 a wave
+    }
     ss_piece += __shfl_xor(ss_piece, 16);
     ss_piece += __shfl_xor(ss_piece, 32);
     if (c == 0) row_ss[wave * 16 + i] = ss_piece;

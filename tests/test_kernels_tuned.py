@@ -208,6 +208,33 @@ def test_product_of_the_normalised_row_from_what_was_left(M, N, K):
     assert np.abs(f64(out) - exact).max() <= 2.0 ** -8 * np.abs(x * rstd * g).max() * np.abs(f64(w)).sum(axis=1).max()
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # sums of x^2 a lane: within the two loads of 9 to 16 rows, one and more behind them (8 waves from 4,112 on, 16 from
+    # 8,208, 4 waves from 2,064), and 8 rows beside them
+    (9, 40, 4096), (12, 40, 4112), (16, 72, 8320), (16, 16400, 2080), (9, 16400, 4104), (8, 16400, 4104)])
+def test_products_behind_a_norm_with_many_sums_a_row(M, N, K):
+    t = tuned()
+    x = f64(gen(M, K, seed=1, scale=3.0))
+    x[0, : K // 2] *= 40.0
+    w = gen(N, K, seed=3, dtype=BF).to(DEV)
+    raw = torch.from_numpy(bf16_round(x)).to(BF).to(DEV)
+    bands = -(-K // 16)
+    xp = np.zeros((M, bands * 16)); xp[:, :K] = x
+    ss = torch.full((16, -(-bands // 4) * 4), 1e9)
+    ss[:M, :bands] = torch.from_numpy((xp.reshape(M, bands, 16) ** 2).sum(axis=2)).float()
+    ss = ss.to(DEV)
+    rstd = 1.0 / np.sqrt((x ** 2).mean(axis=1, keepdims=True) + 3e-4)
+    y = f64(raw) @ f64(w).T * rstd
+    for out_dtype in (BF, torch.float32):
+        out = torch.empty(M, N, dtype=out_dtype, device=DEV)
+        assert t.gemm_pre_bf16(raw, ss, 3e-4, pack(w), out)
+        check(f64(out), y, out_dtype)
+    F = N // 2 // 8 * 8
+    out = torch.empty(M, F, dtype=BF, device=DEV)
+    assert t.swiglu_pre_bf16(raw, ss, 3e-4, pack(w[:F].contiguous()), pack(w[F:2 * F].contiguous()), out)
+    check(f64(out), P.silu(y[:, :F]) * y[:, F:2 * F], BF)
+
+
 @pytest.mark.parametrize("M,F,K", [(1, 24, 64), (8, 176, 512), (16, 200, 112), (4, 14336 // 8, 1024), (8, 14336, 512),
                                    (11, 9000, 256)])
 def test_swiglu_of_the_normalised_row_from_what_was_left(M, F, K):
