@@ -126,6 +126,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rows_gemm_kernel(const bf16_t* 
     }
   }
   constexpr int ITEMS = OUT * MT, ROUNDS = (ITEMS + WAVES - 1) / WAVES;  // (band, 16 rows) to finish, dealt out to the waves
+  // (64 rows and four bands leave no registers for the norm's weight: it is asked for at the end)
+  constexpr bool G_EARLY = MT * NB < 16;
   floatx4 old[ROUNDS], gv[ROUNDS];
   if constexpr (MODE == R_ACC_F32) {
 #pragma unroll
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rows_gemm_kernel(const bf16_t* 
       old[q] = gv[q] = floatx4{0.f, 0.f, 0.f, 0.f};
       if (item < ITEMS && m < M && nn < N) {
         old[q] = *reinterpret_cast<const floatx4*>((const float*)C + (size_t)m * ldc + nn);
-        if constexpr (EMIT) gv[q] = *reinterpret_cast<const floatx4*>(norm.g + nn);
+        if constexpr (EMIT && G_EARLY) gv[q] = *reinterpret_cast<const floatx4*>(norm.g + nn);
       }
     }
   }
@@ -213,6 +215,9 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rows_gemm_kernel(const bf16_t* 
     const bool on = m < M && nn < N;
     if constexpr (MODE == R_ACC_F32) {
       const floatx4 x = old[q] + sum[0];
+      if constexpr (EMIT && !G_EARLY) {
+        if (on) gv[q] = *reinterpret_cast<const floatx4*>(norm.g + nn);
+      }
       if (on) *reinterpret_cast<floatx4*>((float*)C + (size_t)m * ldc + nn) = x;
       if constexpr (EMIT) {
         if (on)

@@ -66,3 +66,12 @@ def test_products_of_few_rows_keep_their_registers():
         if waves == 8 and (mode == 3 or (bands == 1 and pre)):   # 3: SwiGLU.  Two blocks of 8 waves a unit
             assert k[".vgpr_count"] <= 128, args
     assert seen >= 80
+
+
+def test_products_of_17_to_64_rows_keep_nothing_in_memory():
+    pytest.importorskip("msgpack")
+    found = [(arguments(name, "rows_gemm_kernel"), k) for name, k in kernels("tuned")]
+    found = [(args, k) for args, k in found if args]
+    assert len(found) >= 80
+    for args, k in found:
+        assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, args
