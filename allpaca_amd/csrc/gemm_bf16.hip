@@ -699,10 +699,15 @@ APC_EXPORT int apc_gemm_direct_emit_bf16(const void* A, int lda, const void* W, 
 }
 
 // Products of 17 to 64 rows that need no slices of K (gemm_rows_bf16.hip): whether the entry points below hand one to that
-// kernel (mode as theirs, 4 for q, k and v with C the output of q), and then need no workspace.
+// kernel (mode as theirs), and then need no workspace.  For q, k and v: apc_gemm_rows_qkv_takes.
 APC_EXPORT int apc_gemm_rows_takes(int mode, const void* A, int lda, const void* W, const void* Wu, const void* C, int ldc,
                                    int M, int N, int K) {
+  if (mode > G_SWIGLU && !mode_is_act(mode)) return 0;
   return gemm_rows_takes(mode_is_act(mode) ? G_ACT : mode, A, lda, W, Wu, C, ldc, M, N, K);
+}
+APC_EXPORT int apc_gemm_rows_qkv_takes(const void* A, int lda, const void* W, const void* q_out, int ldq, int M, int K, int H,
+                                       int Hk, int d, const float* cos_sin, const void* cache) {
+  return gemm_rows_qkv_takes(A, lda, W, q_out, ldq, M, K, H, Hk, d, cos_sin, cache);
 }
 // residual += A . W^T on that kernel, with raw as in apc_gemm_splitk_emit_bf16 and ss [M][N / 16] sums of residual^2 per row
 // and band of 16 columns; for what apc_gemm_rows_emit_takes (raw 8-byte aligned, its row stride a multiple of 4)
@@ -831,7 +836,8 @@ APC_EXPORT int apc_gemm_pre_bf16(const void* A, int lda, const float* ss, int ss
 // q, k and v of 17 or more rows with K in slices, q and k rotated, k and v written into the paged cache (see
 // gemm_finish_qkv_rope_kernel).  W: tiled layout of [(H + 2 Hk) d, K]; q_out [M, ldq] takes the rotated q heads in its
 // first H d columns; 256 must be a multiple of d.  With ss: A is a row that a product into the residual left and the
-// sums are scaled as in apc_gemm_splitk_pre_bf16.  workspace: k_split * M * (H + 2 Hk) d floats.
+// sums are scaled as in apc_gemm_splitk_pre_bf16.  workspace: k_split * M * (H + 2 Hk) d floats, none for what
+// apc_gemm_rows_qkv_takes.
 APC_EXPORT int apc_gemm_splitk_qkv_rope_bf16(const void* A, int lda, const float* ss, int ss_parts, float eps,
                                              const void* W, void* q_out, int ldq, int M, int K, int H, int Hk, int d,
                                              const float* cos_sin, const int* positions, const int* row_seg,

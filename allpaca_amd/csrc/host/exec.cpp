@@ -361,7 +361,7 @@ int qkv_rope(Program& P, const Buf& a, const Emit* pre, const ApcLayer& L, const
   if (!(act_ok(a) && qkv.dtype == APC_DT_BF16 && E.kv_dtype == APC_DT_BF16)) return 0;
   if (few && !(d % 32 == 0 && qkv.ld % 4 == 0 && ((uintptr_t)qkv.p & 7u) == 0)) return 0;
   const int ks = few ? 1 : tiled_k_split(M, N, K);
-  const bool rows = !few && d % 32 == 0 && apc_gemm_rows_takes(4, a.p, a.ld, L.w_qkv.data, nullptr, qkv.p, qkv.ld, M, N, K);
+  const bool rows = !few && apc_gemm_rows_qkv_takes(a.p, a.ld, L.w_qkv.data, qkv.p, qkv.ld, M, K, H, Hk, d, L.cos_sin, E.kv);
   if (!few && ((ks == 1 && !rows) || 256 % d || d % 2)) return 0;
   if (pre) {
     if (few && !pre_ok_skinny(*pre, K)) return 0;
@@ -378,7 +378,7 @@ int qkv_rope(Program& P, const Buf& a, const Emit* pre, const ApcLayer& L, const
                                     s.row_seg, table, width, E.kv, E.page_tokens, P.stream));
     return 1;
   }
-  float* ws = P.floats((size_t)ks * M * N);
+  float* ws = rows ? nullptr : P.floats((size_t)ks * M * N);
   LAUNCH(P, "gemm_splitk_qkv_rope_bf16",
          apc_gemm_splitk_qkv_rope_bf16(a.p, a.ld, pre ? pre->ss : nullptr, pre ? pre->ss_cols : 0, pre ? pre->eps : 0.f,
                                        L.w_qkv.data, qkv.p, qkv.ld, M, K, H, Hk, d, L.cos_sin, s.positions,

@@ -46,6 +46,8 @@ int apc_gemm_splitk_qkv_rope_bf16(const void* A, int lda, const float* ss, int s
                                   void* cache, int page_tokens, int k_split, float* workspace, hipStream_t stream);
 int apc_gemm_rows_takes(int mode, const void* A, int lda, const void* W, const void* Wu, const void* C, int ldc, int M, int N,
                         int K);
+int apc_gemm_rows_qkv_takes(const void* A, int lda, const void* W, const void* q_out, int ldq, int M, int K, int H, int Hk, int d,
+                            const float* cos_sin, const void* cache);
 int apc_gemm_rows_emit_takes(const void* A, int lda, const void* W, const float* residual, int ldc, int M, int N, int K,
                              const float* g);
 int apc_gemm_rows_emit_bf16(const void* A, int lda, const void* W, float* residual, int ldc, int M, int N, int K,

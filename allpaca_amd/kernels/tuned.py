@@ -113,7 +113,7 @@ def _tiled_k_split(M: int, N: int, K: int, gated: bool = False) -> int:
 
 
 def _rows_take(a: torch.Tensor, w: PackedWeight, wu: Optional[PackedWeight], out: torch.Tensor, N: int, mode: int) -> bool:
-    """Whether such a product of 17 to 64 rows runs in one launch, without slices (N: columns of the product)."""
+    """Whether such a product of 17 to 64 rows runs in one launch, without slices (N: columns of each matrix)."""
     M, K = a.shape
     return bool(SKINNY_MAX_ROWS < M <= ROWS_MAX and _lib.load("tuned").apc_gemm_rows_takes(
         mode, a.data_ptr(), a.stride(0), w.data.data_ptr(), wu.data.data_ptr() if wu is not None else 0, out.data_ptr(),
@@ -282,8 +282,9 @@ def _pre_ok(raw: torch.Tensor, ss: torch.Tensor, K: int) -> bool:
 
 
 def _pre_tiled(raw: torch.Tensor, ss: torch.Tensor, eps: float, w, wu, out: torch.Tensor, n_cols: int, mode: int) -> bool:
-    """The same on the tiled kernel (more than 16 rows), K in slices or in one piece: ss is [M, parts] with up to
-    256 sums of squares a row (what the tiled kernels leave: a part per 256 or per 128 columns)."""
+    """The same with more than 16 rows, in one launch or on the tiled kernel, K in slices or in one piece: ss is [M,
+    parts] with up to 256 sums of squares a row (what the tiled kernels leave: a part per 256 or per 128 columns), up to 64
+    rows 1,024 (a part per 16 columns)."""
     M, K = raw.shape
     if not (M > SKINNY_MAX_ROWS and _act_ok(raw) and ss.dtype == torch.float32 and ss.is_contiguous()
             and ss.dim() == 2 and ss.shape[0] == M and 1 <= ss.shape[1] <= _ss_parts_max(M)):
@@ -330,8 +331,8 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
                   block_table: torch.Tensor, cache: torch.Tensor, page_tokens: int) -> bool:
     """q, k, v in one product that also rotates q and k (whole heads) and writes k and v into the pages; rotated q
     goes to the first n_heads * head_dim columns of q_out.  Up to 16 rows: the streaming kernel (head size a
-    multiple of 32); more rows: the tiled kernel where it cuts K into slices, in its finishing kernel (256 a
-    multiple of the head size).  `a`: the normalised rows, or with `pre` = (ss, eps) the row that
+    multiple of 32); up to 64 the kernel that finishes in one launch, where that is faster; more rows: the tiled kernel
+    where it cuts K into slices, in its finishing kernel (256 a multiple of the head size).  `a`: the normalised rows, or with `pre` = (ss, eps) the row that
     `gemm_emit_bf16` left.  False, with nothing done, for sizes neither takes."""
     _ops._gpu(a, w.data, q_out, cos_sin, positions, row_seg, block_table, cache)
     M, K = a.shape
@@ -343,7 +344,9 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
     if few and not (d % 32 == 0 and q_out.stride(0) % 4 == 0 and q_out.data_ptr() % 8 == 0):
         return False
     ks = 1 if few else _tiled_k_split(M, N, K)
-    rows = not few and d % 32 == 0 and _rows_take(a, w, None, q_out, N, 4)
+    rows = SKINNY_MAX_ROWS < M <= ROWS_MAX and _lib.load("tuned").apc_gemm_rows_qkv_takes(
+        a.data_ptr(), a.stride(0), w.data.data_ptr(), q_out.data_ptr(), q_out.stride(0), M, K, H, Hk, d, cos_sin.data_ptr(),
+        cache.data_ptr())
     if not few and ((ks == 1 and not rows) or 256 % d or d % 2):
         return False
     ss, eps = None, 0.0
@@ -371,12 +374,12 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
             _ops._i32(positions, M, "positions"), _ops._i32(row_seg, M, "row_seg"), block_table.data_ptr(),
             block_table.shape[1], cache.data_ptr(), page_tokens, _ops._stream()), "skinny_qkv_rope_bf16")
         return True
-    ws = torch.empty(ks * M * N, dtype=torch.float32, device=a.device)
+    ws = None if rows else torch.empty(ks * M * N, dtype=torch.float32, device=a.device)
     _lib.check(L.apc_gemm_splitk_qkv_rope_bf16(
         a.data_ptr(), _ops._rows(a, "a"), ss_ptr, ss.shape[1] if ss is not None else 0, float(eps), w.data.data_ptr(),
         q_out.data_ptr(), _ops._rows(q_out, "q_out"), M, K, H, Hk, d, cos_sin.data_ptr(),
         _ops._i32(positions, M, "positions"), _ops._i32(row_seg, M, "row_seg"), block_table.data_ptr(),
-        block_table.shape[1], cache.data_ptr(), page_tokens, ks, ws.data_ptr(), _ops._stream()),
+        block_table.shape[1], cache.data_ptr(), page_tokens, ks, ws.data_ptr() if ws is not None else 0, _ops._stream()),
         "gemm_splitk_qkv_rope_bf16")
     return True
 

@@ -624,6 +624,35 @@ def test_product_for_q_k_v_that_rotates_and_fills_the_pages_equals_the_kernels_o
     assert (results[0][1] != 0).sum() + (results[0][2] != 0).sum() == M * 2 * Hk * d   # every row wrote its k and v, once
 
 
+def test_product_for_q_k_v_in_one_launch_takes_no_workspace():
+    from allpaca_amd.kernels import lib, ops
+    M, H, Hk, d, K, P_ = 50, 6, 2, 64, 1024, 16
+    w = pack(gen((H + 2 * Hk) * d, K, seed=3, dtype=BF).to(DEV))
+    a = gen(M, K, seed=1, dtype=BF).to(DEV)
+    table = gen(M * 2 * (d // 2), seed=2).view(M, 2, d // 2).to(DEV)
+    pos = torch.arange(M, dtype=torch.int32, device=DEV)
+    seg = torch.zeros(M, dtype=torch.int32, device=DEV)
+    bt = torch.arange(-(-M // P_), dtype=torch.int32, device=DEV).view(1, -1)
+    cache = torch.zeros(bt.numel(), 2, Hk, P_, d, dtype=BF, device=DEV)
+    qkv = torch.empty(M, (H + 2 * Hk) * d, dtype=BF, device=DEV)
+    L = lib.load("tuned")
+    assert L.apc_gemm_rows_qkv_takes(a.data_ptr(), K, w.data.data_ptr(), qkv.data_ptr(), qkv.stride(0), M, K, H, Hk, d,
+                                     table.data_ptr(), cache.data_ptr())
+    results = []
+    # the second table begins off 16 bytes: the sliced product and its workspace
+    off = torch.empty(table.numel() + 1, device=DEV)[1:].view(table.shape)
+    for cos_sin, room in ((table, False), (off.copy_(table), True)):
+        cache.zero_()
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        assert ops.qkv_rope_write(a, None, w, qkv, H, Hk, d, cos_sin, pos, seg, bt, cache, P_)
+        assert (torch.cuda.max_memory_allocated() > before) == room
+        results.append((f64(qkv)[:, :H * d], f64(cache)))
+    for got, want in zip(*results):
+        assert np.abs(got - want).max() <= 2.0 ** -6 * np.abs(want).max() and (got != want).mean() < 0.02
+
+
 def test_product_for_q_k_v_that_rotates_declines_what_it_does_not_take():
     from allpaca_amd.kernels import ops
     H, Hk, d, K, P_ = 2, 1, 48, 64, 16                                          # head size no multiple of 32
