@@ -732,6 +732,8 @@ APC_HOST_EXPORT const char* apc_host_timing_report(void* prog) {
 
 // ---- the rules, for tests that hold them against the Python wrappers' own
 APC_HOST_EXPORT int apc_host_rule_tiled_k_split(int M, int N, int K) { return apc_rules::tiled_k_split(M, N, K); }
+APC_HOST_EXPORT int apc_host_rule_gated_k_split(int M, int N, int K) { return apc_rules::tiled_k_split(M, N, K, true); }
+APC_HOST_EXPORT int apc_host_rule_ss_parts_max(int M) { return apc_rules::ss_parts_max(M); }
 APC_HOST_EXPORT int apc_host_rule_rows_bands(int M, int N, int K, int kind) { return apc_rules::rows_bands(M, N, K, kind); }
 APC_HOST_EXPORT int apc_host_rule_slices_direct(int M, int N, int K) { return apc_rules::slices_many_rows(M, N, K).direct; }
 APC_HOST_EXPORT int apc_host_rule_direct_bands(int M, int N, int k_split) { return apc_rules::direct_slices(M, N, k_split).bands; }

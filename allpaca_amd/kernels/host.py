@@ -73,6 +73,8 @@ _lib.SIGNATURES["host"].update({
     "apc_host_timing": [P, I],
     "apc_host_timing_report": [P],
     "apc_host_rule_tiled_k_split": [I, I, I],
+    "apc_host_rule_gated_k_split": [I, I, I],
+    "apc_host_rule_ss_parts_max": [I],
     "apc_host_rule_rows_bands": [I, I, I, I],
     "apc_host_rule_slices_direct": [I, I, I],
     "apc_host_rule_direct_bands": [I, I, I],

@@ -177,3 +177,14 @@ def test_the_kernel_library_takes_the_slices_that_the_wrappers_mean_for_it():
 def test_products_of_17_to_64_rows_in_one_launch_where_that_is_faster(kind, M, N, K, bands):
     from allpaca_amd.kernels import host
     assert host.load().apc_host_rule_rows_bands(M, N, K, kind) == bands
+
+
+def test_gated_products_and_the_sums_behind_a_norm_by_the_executors_rules():
+    from allpaca_amd.kernels import host, tuned
+    L = host.load()
+    for M in (17, 64, 65, 128, 129, 200, 256, 257, 384, 512, 640, 1000, 1024, 1025, 2048):
+        assert L.apc_host_rule_ss_parts_max(M) == tuned._ss_parts_max(M)
+        for N in (192, 640, 1000, 2048, 4096, 8192, 16384, 28672):
+            for K in (120, 512, 1088, 2048, 4096, 11008, 14336):
+                assert L.apc_host_rule_gated_k_split(M, N, K) == tuned._tiled_k_split(M, N, K, True), (M, N, K)
+                assert 128 < M <= 1024 or tuned._tiled_k_split(M, N, K, True) == tuned._tiled_k_split(M, N, K)

@@ -338,8 +338,8 @@ def test_product_into_the_residual_leaves_the_next_norms_row_with_more_than_1024
                                    (64, 28672, 520), (300, 8192, 264), (300, 2048, 1288),
                                    # SwiGLU on the 256-row tile with the norm's scale in its epilogue
                                    (1024, 2 * 16640, 128),
-                                   # SwiGLU from 384 rows on: the kernel that loads its weights straight into registers,
-                                   # the norm's scale in its epilogue (a last row tile of 116, of 128 and of 0 rows)
+                                   # K in one piece with up to 256 tiles (128 x 64 for SwiGLU): the 128 x 128 tile (a
+                                   # last row tile of 116 and of 128 rows)
                                    (500, 2 * 1200, 384), (384, 2 * 264, 128), (640, 2 * 2056, 256)])
 def test_product_of_the_normalised_row_from_what_was_left_with_17_to_1024_rows(M, N, K):
     """On the tiled kernel, with K in slices (the finishing kernel scales) or whole (the product's epilogue does)."""
@@ -371,15 +371,17 @@ def test_product_of_the_normalised_row_from_what_was_left_with_17_to_1024_rows(M
 
 
 @pytest.mark.parametrize("M,N,K", [
-    # the kernel without weights in LDS, K in slices (its first row count, a last row tile of 1, of 44 and of 128 rows; one
-    # to eight slices) and the row before it; a K that has no slices of its own (1,088)
-    (256, 520, 2048), (257, 520, 2048), (300, 132, 1536), (1000, 264, 6144), (1024, 2048, 512), (640, 96, 1088),
+    # the kernel without weights in LDS, K in slices (its first row count, a last row tile of 1, of 44 and of 104 rows; two
+    # to eight slices), the row before it, and K of 512 and 1,088, which the tile has whole and in its own slices
+    (256, 520, 2048), (257, 520, 2048), (300, 132, 1536), (1000, 264, 6144), (1024, 4096, 4096), (385, 6144, 2048), (1024, 2048, 512), (640, 96, 1088),
     # K in one piece with more than 256 tiles of 128 x 128, and with 256
     (129, 16516, 128), (130, 16384, 256),
     # the adding kernel without whole pieces (columns no multiple of 4), and two rows of it at 128 rows
     (140, 130, 2048), (257, 1022, 1024), (128, 516, 1024)])
 def test_products_of_some_hundred_rows(M, N, K):
     t = tuned()
+    assert t._slices_many_rows(M, N, K)[1] == ((M, N, K) in [(257, 520, 2048), (300, 132, 1536), (1000, 264, 6144), (1024, 4096, 4096),
+                                                            (385, 6144, 2048)])
     a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=2, dtype=BF).to(DEV)
     want = f64(a) @ f64(w).T
     pw = pack(w)
@@ -397,16 +399,52 @@ def test_products_of_some_hundred_rows(M, N, K):
     assert (wide[:, 0] == 7).all() and (wide[:, N + 1:] == 7).all()
 
 
-@pytest.mark.parametrize("M,N,K", [
-    # the kernel that finishes a product of 17 to 64 rows in one launch: one, two and four bands a block (the last block's
-    # bands beyond the matrix among them), 2 and 4 groups of 16 rows, waves with 2 to 9 steps of K; the rows around it
-    (17, 48, 1024), (32, 4112, 1088), (33, 4096, 1024), (64, 8240, 1536), (50, 16, 4160), (20, 5136, 1024), (64, 5120, 1024),
-    (64, 272, 4608), (65, 272, 2048), (16, 272, 2048), (40, 264, 1024), (40, 272, 1032)])
-def test_products_of_17_to_64_rows(M, N, K):
+@pytest.mark.parametrize("M,N,K,direct", [
+    # the kernel without weights in LDS with K in one piece below 1,024 rows: more than 256 tiles (columns N: two of 130 and
+    # four of 66, a last row tile of 1, 2 and 116 rows, last bands of 4 and 8 columns), 256 tiles, and a K of no whole stages
+    (129, 16516, 128, True), (130, 16640, 384, True), (500, 8328, 256, True), (600, 6664, 128, True), (130, 16384, 256, False), (300, 11008, 192, False)])
+def test_products_of_some_hundred_rows_with_tiles_for_every_compute_unit(M, N, K, direct):
+    """Plain and behind a norm, stored and gated (N // 2 columns of 64 a tile, so as many tiles)."""
+    t = tuned()
+    F = N // 2 // 8 * 8
+    a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=3, dtype=BF, scale=0.3).to(DEV)
+    assert t._tiled_k_split(M, N, K) == 1 and t._tiled_k_split(M, 2 * F, K, True) == 1
+    assert (-(-M // 128) * -(-N // 128) > 256 and -(-M // 128) * -(-F // 64) > 256 and K % 128 == 0) == direct
+    pw, pg, pu = pack(w), pack(w[:F].contiguous()), pack(w[F:2 * F].contiguous())
+    parts = -(-K // 128)
+    ss = torch.from_numpy(np.random.default_rng(4).uniform(0.5, 40.0, (M, parts)).astype(np.float32)).to(DEV)
+    rstd = 1.0 / np.sqrt(f64(ss).sum(axis=1, keepdims=True) / K + 1e-5)
+    y = f64(a) @ f64(w).T
+    for out_dtype in (BF, torch.float32):
+        out = torch.empty(M, N, dtype=out_dtype, device=DEV)
+        t.gemm_bf16(a, pw, out)
+        check(f64(out), y, out_dtype)
+        assert t.gemm_pre_bf16(a, ss, 1e-5, pw, out)
+        check(f64(out), y * rstd, out_dtype)
+    out = torch.empty(M, F, dtype=BF, device=DEV)
+    t.swiglu_bf16(a, pg, pu, out)
+    check(f64(out), P.silu(y[:, :F]) * y[:, F:2 * F], BF)
+    assert t.swiglu_pre_bf16(a, ss, 1e-5, pg, pu, out)
+    check(f64(out), P.silu(y[:, :F] * rstd) * (y[:, F:2 * F] * rstd), BF)
+
+
+@pytest.mark.parametrize("M,N,K,bands", [
+    # the kernel that finishes a product of 17 to 64 rows in one launch, by the bands a block takes (the last block's bands
+    # beyond the matrix among them): 2 to 4 groups of 16 rows, waves with 2 to 16 steps of K, so that the loop over the
+    # register sets runs as well as what is in front of it and behind it
+    (17, 48, 1024, 1), (33, 4096, 1024, 1), (17, 64, 4160, 1), (33, 512, 3136, 1), (64, 4096, 2048, 1), (64, 4096, 4096, 1), (20, 272, 8192, 1),
+    (32, 4112, 1088, 2), (20, 5136, 1024, 2), (64, 5120, 1024, 2), (48, 4112, 2112, 2), (64, 5120, 3072, 2), (32, 4112, 4160, 2),
+    (64, 8240, 1536, 4), (50, 8208, 2048, 4), (17, 8208, 4096, 4),
+    # where the tiled kernel is faster, rows around it, columns and K that it does not take
+    (50, 16, 4160, 0), (64, 272, 4608, 0), (65, 272, 2048, 0), (16, 272, 2048, 0), (40, 264, 1024, 0), (40, 272, 1032, 0)])
+def test_products_of_17_to_64_rows(M, N, K, bands):
+    from allpaca_amd.kernels import host, lib
     t = tuned()
     a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=2, dtype=BF).to(DEV)
     want = f64(a) @ f64(w).T
     pw = pack(w)
+    assert bool(bands) == bool(lib.load("tuned").apc_gemm_rows_takes(0, a.data_ptr(), K, pw.data.data_ptr(), 0, a.data_ptr(), N, M, N, K))
+    assert not bands or host.load().apc_host_rule_rows_bands(M, N, K, 0) == bands
     for out_dtype in (BF, torch.float32):
         out = torch.full((M + 1, N + 4), 7.0, dtype=out_dtype, device=DEV)
         t.gemm_bf16(a, pw, out[:M, :N])
@@ -624,6 +662,62 @@ def test_product_for_q_k_v_that_rotates_and_fills_the_pages_equals_the_kernels_o
     assert (results[0][1] != 0).sum() + (results[0][2] != 0).sum() == M * 2 * Hk * d   # every row wrote its k and v, once
 
 
+@pytest.mark.parametrize("M,H,Hk,d,K,P_,pre,off,rows", [
+    # in one launch: two to four row groups, whole and not, heads of 32 to 256, 2 to 6 steps of K a wave
+    (17, 6, 2, 64, 1088, 8, True, 0, True), (33, 3, 1, 32, 1024, 16, False, 0, True), (64, 4, 2, 256, 1024, 32, True, 0, True),
+    (48, 2, 1, 256, 1024, 16, False, 0, True), (50, 5, 1, 64, 1536, 16, True, 0, True), (17, 24, 8, 128, 3072, 16, False, 0, True),
+    (64, 24, 8, 128, 3072, 16, True, 0, True),
+    # the adding kernel, four columns a lane: 16 rows of v at a time, the last ones beyond the step's
+    (50, 6, 2, 64, 4160, 16, True, 0, False), (100, 3, 1, 32, 1032, 24, False, 0, False), (257, 4, 2, 128, 2048, 16, True, 0, False),
+    # column by column: heads of 2 and 4, q off 8 bytes
+    (40, 5, 3, 4, 520, 8, True, 0, False), (100, 7, 1, 2, 1032, 16, False, 0, False), (30, 6, 2, 64, 1088, 16, True, 1, False),
+    (129, 4, 2, 256, 2048, 16, False, 2, False)])
+def test_product_for_q_k_v_rotated_and_in_the_pages_against_float64(M, H, Hk, d, K, P_, pre, off, rows):
+    """off: elements in front of q_out's first column, whose row stride is no multiple of 4 then."""
+    from allpaca_amd.kernels import lib, ops
+    rng = np.random.default_rng(M + d)
+    N, half = (H + 2 * Hk) * d, d // 2
+    w, a = gen(N, K, seed=3, dtype=BF).to(DEV), gen(M, K, seed=1, dtype=BF, scale=2.0).to(DEV)
+    pw, eps = pack(w), 2e-5
+    ss = torch.from_numpy(rng.uniform(0.5, 40.0, (M, K // 16 if rows else -(-K // 256))).astype(np.float32)).to(DEV) if pre else None
+    blocks = max(5, -(-M // P_) + 2)
+    places = rng.permutation(3 * blocks * P_)[:M]
+    seg, pos = places // (blocks * P_), places % (blocks * P_)
+    bt = rng.permutation(3 * blocks).reshape(3, blocks)
+    ang = np.arange(blocks * P_)[:, None] * (1.0 / 300.0 ** (np.arange(half) / half))[None, :]
+    table = torch.from_numpy(np.stack([np.cos(ang), np.sin(ang)], 1).astype(np.float32)).to(DEV)
+    i32 = lambda v: torch.from_numpy(np.ascontiguousarray(v).astype(np.int32)).to(DEV)  # noqa: E731
+    cache = torch.full((3 * blocks, 2, Hk, P_, d), 5.0, dtype=BF, device=DEV)
+    q = torch.full((M, N + off), 7.0, dtype=BF, device=DEV)[:, off:]
+    assert rows == bool(lib.load("tuned").apc_gemm_rows_qkv_takes(a.data_ptr(), K, pw.data.data_ptr(), q.data_ptr(), q.stride(0), M, K, H, Hk,
+                                                                  d, table.data_ptr(), cache.data_ptr()))
+    assert ops.qkv_rope_write(a, (ss, eps) if pre else None, pw, q, H, Hk, d, table, i32(pos), i32(seg), i32(bt), cache, P_)
+    y = f64(a) @ f64(w).T
+    if pre:
+        y = y / np.sqrt(f64(ss).sum(axis=1, keepdims=True) / K + eps)
+    noise = 1e-5 * np.abs(y).max()                       # of a float32 sum, as `check` allows
+    heads = y.reshape(M, H + 2 * Hk, d)
+    cos, sin = f64(table)[pos][:, None, 0], f64(table)[pos][:, None, 1]
+    lo, hi = heads[:, :H + Hk, :half], heads[:, :H + Hk, half:]
+    turned = np.concatenate([lo * cos - hi * sin, lo * sin + hi * cos], axis=2)
+    pair = np.concatenate([np.hypot(lo, hi)] * 2, axis=2)
+    # the sums rounded to bfloat16 (both of a pair: 2^-8 of its length, which the rotation keeps, or less), the result once more
+
+    def near(got, want, by):
+        assert (np.abs(got - want) <= 1.01 * by + 2.0 * noise).all(), np.abs(got - want).max()
+
+    near(f64(q)[:, :H * d].reshape(M, H, d), turned[:, :H], 2.0 ** -8 * (pair[:, :H] + np.abs(turned[:, :H])))
+    assert (f64(q)[:, H * d:] == 7.0).all()
+    kept = f64(cache)
+    page, slot = bt[seg, pos // P_], pos % P_
+    near(kept[page, 0, :, slot], turned[:, H:], 2.0 ** -8 * (pair[:, H:] + np.abs(turned[:, H:])))
+    values = kept[:, 1].reshape(3 * blocks, Hk, d, P_)
+    near(values[page, :, :, slot], heads[:, H + Hk:], 2.0 ** -8 * np.abs(heads[:, H + Hk:]))
+    kept[page, 0, :, slot] = 5.0
+    values[page, :, :, slot] = 5.0
+    assert (kept[:, 0] == 5.0).all() and (values == 5.0).all()   # nothing beside the rows' places
+
+
 def test_product_for_q_k_v_in_one_launch_takes_no_workspace():
     from allpaca_amd.kernels import lib, ops
     M, H, Hk, d, K, P_ = 50, 6, 2, 64, 1024, 16
@@ -634,7 +728,7 @@ def test_product_for_q_k_v_in_one_launch_takes_no_workspace():
     seg = torch.zeros(M, dtype=torch.int32, device=DEV)
     bt = torch.arange(-(-M // P_), dtype=torch.int32, device=DEV).view(1, -1)
     cache = torch.zeros(bt.numel(), 2, Hk, P_, d, dtype=BF, device=DEV)
-    qkv = torch.empty(M, (H + 2 * Hk) * d, dtype=BF, device=DEV)
+    qkv = torch.zeros(M, (H + 2 * Hk) * d, dtype=BF, device=DEV)
     L = lib.load("tuned")
     assert L.apc_gemm_rows_qkv_takes(a.data_ptr(), K, w.data.data_ptr(), qkv.data_ptr(), qkv.stride(0), M, K, H, Hk, d,
                                      table.data_ptr(), cache.data_ptr())
