@@ -6,6 +6,7 @@ no multiple of 8, a head size that is no multiple of 16 or above 256) and the ca
 kernel: never a wrong result."""
 from __future__ import annotations
 
+import functools
 import math
 from typing import Optional
 
@@ -63,6 +64,7 @@ def _direct_slices_us(M: int, N: int, s: int) -> float:
     return min(us)
 
 
+@functools.lru_cache(maxsize=4096)   # (8 us of Python a product otherwise)
 def _slices_many_rows(M: int, N: int, K: int):
     """(slices of K, whether the kernel without weights in LDS takes them) for 129..1024 rows.  From 257 rows on that
     kernel's slices, which have to be of one length in pieces of 128 columns, are held against what the 128 x 128 tile

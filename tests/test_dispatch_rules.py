@@ -188,3 +188,11 @@ def test_gated_products_and_the_sums_behind_a_norm_by_the_executors_rules():
             for K in (120, 512, 1088, 2048, 4096, 11008, 14336):
                 assert L.apc_host_rule_gated_k_split(M, N, K) == tuned._tiled_k_split(M, N, K, True), (M, N, K)
                 assert 128 < M <= 1024 or tuned._tiled_k_split(M, N, K, True) == tuned._tiled_k_split(M, N, K)
+
+
+def test_the_expected_times_of_a_size_are_worked_out_once(monkeypatch):
+    """A step's products come in the same few sizes, and the rule is 8 us of Python a product."""
+    from allpaca_amd.kernels import tuned
+    want = tuned._tiled_k_split(517, 4100, 4224)
+    monkeypatch.setattr(tuned, "_direct_slices_us", lambda *a: pytest.fail("worked out again"))
+    assert tuned._tiled_k_split(517, 4100, 4224) == want
