@@ -12,8 +12,8 @@
 // Epilogues: store bfloat16 / float32, add into a float32 residual, an activation on the sums (bfloat16 out), or SwiGLU: then the W tile is
 // 64 gate rows and the matching 64 up rows, each wave computes gate and up of the same 64 x 32 outputs,
 // and the block writes a 128 x 64 tile of silu(gate) * up.
-// With up to 1,024 rows K may be cut into slices for different blocks (from 257 rows on by gemm_direct_bf16.hip's kernel)
-// and a second kernel adds the slices in order; products of 17 to 64 rows that gemm_rows_bf16.hip takes need none.  The
+// With up to 1,024 rows K may be cut into slices for different blocks (from 257 rows on by gemm_direct_bf16.hip's kernel
+// where that is faster) and a second kernel adds the slices in order; products of 17 to 64 rows that gemm_rows_bf16.hip takes need none.  The
 // order of additions for an output depends on N, K and the number of the step's rows, never on which they are.
 // Reference counterpart: gemm_nt_bf16_tiled_kernel, hip/src/kernels.cpp:634 (no matrix cores there).
 #include <type_traits>
