@@ -391,38 +391,41 @@ struct FinishNorm {
   int act = 0;      // mode G_ACT: the activation
 };
 
-// How the finishing kernels below go over a row: a wave takes 256 columns of it, a lane four of them, in one piece of 16
-// bytes (VEC: N and the row strides multiples of 4, everything aligned) or, otherwise, 64 columns apart.  Nothing crosses a
-// wave, so there is no barrier, and up to four slices' loads are in flight.  Bound by the slices' bytes: 512 rows x 4,096
-// columns in four slices, added into the residual with the norm's row left, 54 MB in 10.1 us (a thread a column and a
-// block 256 columns of a row: two slices, 38 MB, in 11.5).
+// How the finishing kernels below go over a row: a wave takes 256 columns of it, a lane four of them in one piece, whatever
+// the row begins on (the hardware takes pieces off 16 bytes; the last lane's is moved back into the row and turned).  Nothing
+// crosses a wave, so there is no barrier, and up to four slices' loads are in flight.  Bound by the slices' bytes: 512 rows x
+// 4,096 columns in four slices, added into the residual with the norm's row left, 54 MB in 10.1 us (a thread a column and
+// a block 256 columns of a row: two slices, 38 MB, in 11.5).  Rows off 16 bytes and columns no multiple of 4, product and adding
+// kernel: 24 rows, K 4,104 into 3,001 columns 16.1 us, 512 rows, K 4,096 32.5 (in pieces of 4 bytes, four columns a lane 21.4 and
+// 38.0, one column a lane 16.9 and 35.0).
 constexpr int FIN_COLS = 256;
-template <bool VEC, int LANES = WAVE>
-__device__ __forceinline__ int fin_column(int first, int lane, int j) { return VEC ? first + lane * 4 + j : first + j * LANES + lane; }
+typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uint2_any __attribute__((ext_vector_type(2), aligned(2)));
 
-// A lane's four sums over the slices, in slice order; 0 beyond N.  LANES: lanes that share the row's piece
-template <bool VEC, int LANES = WAVE>
-__device__ __forceinline__ floatx4 fin_sum(const float* __restrict__ row, size_t plane, int k_split, int first, int lane, int N) {
+// The sums of the columns col .. col + 3 over the slices, in slice order; 0 beyond N
+__device__ __forceinline__ floatx4 fin_sum(const float* __restrict__ row, size_t plane, int k_split, int col, int N) {
   floatx4 g = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (N < 4) {
+    for (int s = 0; s < k_split; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (col + j < N) g[j] += row[(size_t)s * plane + col + j];
+    return g;
+  }
+  const int from = min(col, N - 4), back = col - from;
   for (int s0 = 0; s0 < k_split; s0 += 4) {
     floatx4 v[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      v[s] = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (s0 + s < k_split) {
-        const float* src = row + (size_t)(s0 + s) * plane;
-        if constexpr (VEC) {
-          if (first + lane * 4 < N) v[s] = *reinterpret_cast<const floatx4*>(src + first + lane * 4);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (fin_column<VEC, LANES>(first, lane, j) < N) v[s][j] = src[fin_column<VEC, LANES>(first, lane, j)];
-        }
-      }
-    }
+    for (int s = 0; s < 4; ++s)
+      if (s0 + s < k_split) v[s] = *reinterpret_cast<const floatx4_any*>(row + (size_t)(s0 + s) * plane + from);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
       if (s0 + s < k_split) g += v[s];
+  }
+  if (back > 0) {
+    if (back & 1) g = floatx4{g[1], g[2], g[3], 0.f};
+    if (back & 2) g = floatx4{g[2], g[3], 0.f, 0.f};
+    if (back >= 4) g = floatx4{0.f, 0.f, 0.f, 0.f};
   }
   return g;
 }
@@ -433,76 +436,69 @@ __device__ __forceinline__ float fin_rstd(const FinishNorm& norm, int m, int lan
   return 1.0f / sqrtf(sum / (float)K + norm.eps);
 }
 
-template <bool VEC>
-__device__ __forceinline__ void fin_store_bf16(bf16_t* row, int first, int lane, int N, const floatx4& y) {
-  if constexpr (VEC) {
-    if (first + lane * 4 < N) {
-      uint2 o;
-      o.x = pack_bf16x2(y[0], y[1]);
-      o.y = pack_bf16x2(y[2], y[3]);
-      *reinterpret_cast<uint2*>(row + first + lane * 4) = o;
-    }
+__device__ __forceinline__ void fin_store_bf16(bf16_t* row, int col, int N, const floatx4& y) {
+  if (col + 3 < N) {
+    *reinterpret_cast<uint2_any*>(row + col) = uint2_any{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
   } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (fin_column<VEC>(first, lane, j) < N) row[fin_column<VEC>(first, lane, j)] = float_to_bf16(y[j]);
+    for (int j = 0; j < 3; ++j)
+      if (col + j < N) row[col + j] = float_to_bf16(y[j]);
   }
 }
-template <bool VEC>
-__device__ __forceinline__ void fin_store_f32(float* row, int first, int lane, int N, const floatx4& y) {
-  if constexpr (VEC) {
-    if (first + lane * 4 < N) *reinterpret_cast<floatx4*>(row + first + lane * 4) = y;
+__device__ __forceinline__ void fin_store_f32(float* row, int col, int N, const floatx4& y) {
+  if (col + 3 < N) {
+    *reinterpret_cast<floatx4_any*>(row + col) = y;
   } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (fin_column<VEC>(first, lane, j) < N) row[fin_column<VEC>(first, lane, j)] = y[j];
+    for (int j = 0; j < 3; ++j)
+      if (col + j < N) row[col + j] = y[j];
   }
 }
 
 // Sums the float32 sums that G_PARTIAL blocks left ([which][slice][M][N], slices in order) and finishes:
 // store bfloat16 / float32, add into a float32 residual, an activation, or SwiGLU of the two matrices' sums.
-template <bool PRE, bool EMIT, bool VEC>
+template <bool PRE, bool EMIT>
 __global__ __launch_bounds__(256) void gemm_finish_kernel(const float* __restrict__ partials, int k_split, int M, int N,
                                                           int K, int mode, void* __restrict__ C, int ldc,
                                                           FinishNorm norm) {
   const int parts = ceil_div(N, FIN_COLS);
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int m = blockIdx.y, part = blockIdx.x * 4 + wave, first = part * FIN_COLS;
+  const int m = blockIdx.y, part = blockIdx.x * 4 + wave, col = part * FIN_COLS + lane * 4;
   if (part >= parts) return;
   const size_t plane = (size_t)M * N;
   const float* src = partials + (size_t)m * N;
   floatx4 old = floatx4{0.f, 0.f, 0.f, 0.f}, gv = floatx4{0.f, 0.f, 0.f, 0.f};  // the residual, the next norm's weight
-  if (mode == G_ACC_F32) old = fin_sum<VEC>((const float*)C + (size_t)m * ldc, 0, 1, first, lane, N);
-  if constexpr (EMIT) gv = fin_sum<VEC>(norm.g, 0, 1, first, lane, N);
-  floatx4 g = fin_sum<VEC>(src, plane, k_split, first, lane, N);
+  if (mode == G_ACC_F32) old = fin_sum((const float*)C + (size_t)m * ldc, 0, 1, col, N);
+  if constexpr (EMIT) gv = fin_sum(norm.g, 0, 1, col, N);
+  floatx4 g = fin_sum(src, plane, k_split, col, N);
   const float rstd = PRE ? fin_rstd(norm, m, lane, K) : 1.f;
   if constexpr (PRE) g *= rstd;
   bf16_t* out16 = (bf16_t*)C + (size_t)m * ldc;
   float* out32 = (float*)C + (size_t)m * ldc;
   if (mode == G_STORE_BF16) {
-    fin_store_bf16<VEC>(out16, first, lane, N, g);
+    fin_store_bf16(out16, col, N, g);
   } else if (mode == G_ACT) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) g[j] = activation_f(g[j], norm.act);
-    fin_store_bf16<VEC>(out16, first, lane, N, g);
+    fin_store_bf16(out16, col, N, g);
   } else if (mode == G_STORE_F32) {
-    fin_store_f32<VEC>(out32, first, lane, N, g);
+    fin_store_f32(out32, col, N, g);
   } else if (mode == G_ACC_F32) {
     const floatx4 x = old + g;
-    fin_store_f32<VEC>(out32, first, lane, N, x);
+    fin_store_f32(out32, col, N, x);
     if constexpr (EMIT) {
-      fin_store_bf16<VEC>(norm.raw + (size_t)m * norm.ld_raw, first, lane, N, x * gv);
+      fin_store_bf16(norm.raw + (size_t)m * norm.ld_raw, col, N, x * gv);
       float sq = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];   // (0 beyond N)
 #pragma unroll
       for (int o = WAVE / 2; o > 0; o /= 2) sq += __shfl_xor(sq, o, WAVE);
       if (lane == 0) norm.emit_ss[(size_t)m * parts + part] = sq;
     }
   } else {
-    floatx4 u = fin_sum<VEC>(src + (size_t)k_split * plane, plane, k_split, first, lane, N);
+    floatx4 u = fin_sum(src + (size_t)k_split * plane, plane, k_split, col, N);
     if constexpr (PRE) u *= rstd;
 #pragma unroll
     for (int j = 0; j < 4; ++j) g[j] = silu_f(g[j]) * u[j];
-    fin_store_bf16<VEC>(out16, first, lane, N, g);
+    fin_store_bf16(out16, col, N, g);
   }
 }
 
@@ -556,20 +552,13 @@ static int launch_splitk(const void* A, int lda, const void* W, const void* Wu, 
                             RowsNorm{const_cast<float*>(norm.pre_ss), norm.pre_parts, norm.eps, nullptr, nullptr, 0, norm.act}, stream);
   const int e = launch_partials(A, lda, W, Wu, M, N, K, k_split, workspace, stream);
   if (e) return e;
-  const bool out16 = mode == G_STORE_BF16 || mode == G_SWIGLU || mode == G_ACT;
-  bool vec = N % 4 == 0 && ldc % 4 == 0 && aligned16(workspace) && ((uintptr_t)C & (out16 ? 7u : 15u)) == 0;
-  if (emit) vec = vec && aligned16(norm.g) && norm.ld_raw % 4 == 0 && ((uintptr_t)norm.raw & 7u) == 0;
-#define FINISH_AS(PRE_, EMIT_, VEC_)                                                                                 \
-  hipLaunchKernelGGL((gemm_finish_kernel<PRE_, EMIT_, VEC_>), dim3(ceil_div(N, 4 * FIN_COLS), M), dim3(256), 0, stream, \
-                     workspace, k_split, M, N, K, mode, C, ldc, norm)
-#define FINISH(PRE_, EMIT_)                \
-  if (vec) FINISH_AS(PRE_, EMIT_, true);   \
-  else FINISH_AS(PRE_, EMIT_, false)
-  if (pre) { FINISH(true, false); }
-  else if (emit) { FINISH(false, true); }
-  else { FINISH(false, false); }
+#define FINISH(PRE_, EMIT_)                                                                                                \
+  hipLaunchKernelGGL((gemm_finish_kernel<PRE_, EMIT_>), dim3(ceil_div(N, 4 * FIN_COLS), M), dim3(256), 0, stream, workspace, \
+                     k_split, M, N, K, mode, C, ldc, norm)
+  if (pre) FINISH(true, false);
+  else if (emit) FINISH(false, true);
+  else FINISH(false, false);
 #undef FINISH
-#undef FINISH_AS
   APC_LAUNCH_CHECK();
   return 0;
 }
@@ -594,7 +583,7 @@ struct FinishRope {
 
 constexpr int FIN_V_ROWS = 16, FIN_V_COLS = 64;
 
-template <bool PRE, bool VEC>
+template <bool PRE>
 __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* __restrict__ partials, int k_split, int M,
                                                                    int N, int K, bf16_t* __restrict__ q_out, int ldq,
                                                                    FinishNorm norm, FinishRope rope, int qk_blocks) {
@@ -612,7 +601,7 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
     int pos = 0, seg = 0;
     if (sm < M) pos = rope.positions[sm], seg = rope.row_seg[sm];
     floatx4 g = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (m < M) g = fin_sum<VEC, 16>(partials + (size_t)m * N, plane, k_split, col0, l16, N);
+    if (m < M) g = fin_sum(partials + (size_t)m * N, plane, k_split, col0 + l16 * 4, N);
     if constexpr (PRE) {
       const float sum = row_parts_sum<16>(norm.pre_ss + (size_t)min(m, M - 1) * norm.pre_parts, norm.pre_parts, l16);
       g *= 1.0f / sqrtf(sum / (float)K + norm.eps);
@@ -621,7 +610,7 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
     if (sm < M) page += (size_t)rope.block_table[(size_t)seg * rope.max_blocks + pos / rope.P] * page_elems;
     bf16_t* tile = reinterpret_cast<bf16_t*>(&vals[0][0]);             // [column][16 rows + 2]
 #pragma unroll
-    for (int j = 0; j < 4; ++j) tile[fin_column<VEC, 16>(0, l16, j) * (FIN_V_ROWS + 2) + r] = float_to_bf16(g[j]);
+    for (int j = 0; j < 4; ++j) tile[(l16 * 4 + j) * (FIN_V_ROWS + 2) + r] = float_to_bf16(g[j]);
     __syncthreads();
     if (sm >= M) return;
     bf16_t* out = page + (size_t)rope.Hk * rope.P * d + pos % rope.P;
@@ -633,46 +622,43 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
     return;
   }
   const int across = ceil_div(qk, 4 * FIN_COLS);
-  const int m = blockIdx.x / across, first = (blockIdx.x % across * 4 + wave) * FIN_COLS;
+  const int m = blockIdx.x / across, first = (blockIdx.x % across * 4 + wave) * FIN_COLS, n = first + lane * 4;
   if (first >= qk) return;
   const int pos = rope.positions[m], seg = rope.row_seg[m];
-  floatx4 g = fin_sum<VEC>(partials + (size_t)m * N, plane, k_split, first, lane, N);
+  floatx4 g = fin_sum(partials + (size_t)m * N, plane, k_split, n, N);
   const float rstd = PRE ? fin_rstd(norm, m, lane, K) : 1.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) g[j] = bf16_to_float(float_to_bf16(PRE ? g[j] * rstd : g[j]));
   bf16_t* page = rope.cache + (size_t)rope.block_table[(size_t)seg * rope.max_blocks + pos / rope.P] * page_elems;
   const float* cs = rope.cos_sin + (size_t)pos * d;
   floatx4 cosv, sinv, partner;  // partner: the value `half` columns on or back (d is a power of two)
+  *reinterpret_cast<floatx4*>(&vals[wave][lane * 4]) = g;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int r = fin_column<VEC>(first, lane, j) % half;
+    const int r = (n + j) % half;
     cosv[j] = cs[r], sinv[j] = cs[half + r];
-    vals[wave][fin_column<VEC>(0, lane, j)] = g[j];
   }
   wave_lds_order();
 #pragma unroll
-  for (int j = 0; j < 4; ++j) partner[j] = vals[wave][fin_column<VEC>(0, lane, j) ^ half];
+  for (int j = 0; j < 4; ++j) partner[j] = vals[wave][(lane * 4 + j) ^ half];
   floatx4 y;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    y[j] = fin_column<VEC>(first, lane, j) % d < half ? g[j] * cosv[j] - partner[j] * sinv[j] : partner[j] * sinv[j] + g[j] * cosv[j];
+    y[j] = (n + j) % d < half ? g[j] * cosv[j] - partner[j] * sinv[j] : partner[j] * sinv[j] + g[j] * cosv[j];
   bf16_t* keys = page + (size_t)(pos % rope.P) * d;
-  if constexpr (VEC) {  // four columns of one head
-    const int n = first + lane * 4, head = n / d;
-    if (n >= qk) return;
-    uint2 o;
-    o.x = pack_bf16x2(y[0], y[1]);
-    o.y = pack_bf16x2(y[2], y[3]);
-    *reinterpret_cast<uint2*>(head < rope.H ? q_out + (size_t)m * ldq + n
-                                            : keys + (size_t)(head - rope.H) * rope.P * d + n % d) = o;
-  } else {
+  if (d % 4 == 0) {  // four columns of one head
+    const int head = n / d;
+    if (n < qk)
+      *reinterpret_cast<uint2_any*>(head < rope.H ? q_out + (size_t)m * ldq + n : keys + (size_t)(head - rope.H) * rope.P * d + n % d) =
+          uint2_any{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+    return;
+  }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = fin_column<VEC>(first, lane, j), head = n / d;
-      if (n >= qk) continue;
-      if (head < rope.H) q_out[(size_t)m * ldq + n] = float_to_bf16(y[j]);
-      else keys[(size_t)(head - rope.H) * rope.P * d + n % d] = float_to_bf16(y[j]);
-    }
+  for (int j = 0; j < 4; ++j) {  // heads of 2
+    const int head = (n + j) / d;
+    if (n + j >= qk) continue;
+    if (head < rope.H) q_out[(size_t)m * ldq + n + j] = float_to_bf16(y[j]);
+    else keys[(size_t)(head - rope.H) * rope.P * d + (n + j) % d] = float_to_bf16(y[j]);
   }
 }
 
@@ -858,18 +844,15 @@ APC_EXPORT int apc_gemm_splitk_qkv_rope_bf16(const void* A, int lda, const float
   if (e) return e;
   const FinishNorm norm{ss, ss_parts, eps, nullptr, nullptr, 0, nullptr};
   const FinishRope rope{cos_sin, positions, row_seg, block_table, max_blocks, (bf16_t*)cache, page_tokens, H, Hk, d};
-  const bool vec = d % 8 == 0 && ldq % 4 == 0 && aligned16(workspace) && ((uintptr_t)q_out & 7u) == 0 && ((uintptr_t)cache & 7u) == 0;
   const int qk = (H + Hk) * d;
   const long qk_blocks = (long)M * ceil_div(qk, 4 * FIN_COLS);
   const long blocks = qk_blocks + (long)ceil_div(M, FIN_V_ROWS) * ceil_div(N - qk, FIN_V_COLS);
   if (blocks > 0x7fffffffL) return APC_ERR_BAD_ARG;
-#define FINISH_ROPE(PRE_, VEC_)                                                                                         \
-  hipLaunchKernelGGL((gemm_finish_qkv_rope_kernel<PRE_, VEC_>), dim3((unsigned)blocks), dim3(256), 0, stream, workspace, \
-                     k_split, M, N, K, (bf16_t*)q_out, ldq, norm, rope, (int)qk_blocks)
-  if (ss && vec) FINISH_ROPE(true, true);
-  else if (ss) FINISH_ROPE(true, false);
-  else if (vec) FINISH_ROPE(false, true);
-  else FINISH_ROPE(false, false);
+#define FINISH_ROPE(PRE_)                                                                                                \
+  hipLaunchKernelGGL((gemm_finish_qkv_rope_kernel<PRE_>), dim3((unsigned)blocks), dim3(256), 0, stream, workspace, k_split, M, \
+                     N, K, (bf16_t*)q_out, ldq, norm, rope, (int)qk_blocks)
+  if (ss) FINISH_ROPE(true);
+  else FINISH_ROPE(false);
 #undef FINISH_ROPE
   APC_LAUNCH_CHECK();
   return 0;

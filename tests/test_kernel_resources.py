@@ -75,3 +75,13 @@ def test_products_of_17_to_64_rows_keep_nothing_in_memory():
     assert len(found) >= 80
     for args, k in found:
         assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, args
+
+
+def test_adding_kernels_leave_room_for_eight_waves_a_simd():
+    """They are bound by loads in flight, of which a lane that takes its columns one by one has few."""
+    pytest.importorskip("msgpack")
+    found = [(arguments(name, kernel), k) for name, k in kernels("tuned")
+             for kernel in ("gemm_finish_kernel", "gemm_finish_qkv_rope_kernel") if arguments(name, kernel)]
+    assert len(found) >= 4
+    for args, k in found:
+        assert k[".vgpr_count"] <= 64 and k[".private_segment_fixed_size"] == 0, args
