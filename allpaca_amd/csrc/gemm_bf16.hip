@@ -591,6 +591,7 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
   static_assert(FIN_V_ROWS * FIN_V_COLS == 4 * FIN_COLS, "both kinds of block hold 1,024 values");
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int d = rope.d, half = d / 2, qk = (rope.H + rope.Hk) * d;  // columns of q and k
+  const int log_d = __builtin_ctz((unsigned)d);                      // (256 is a multiple of d)
   const size_t plane = (size_t)M * N, page_elems = (size_t)2 * rope.Hk * rope.P * d;
   if ((int)blockIdx.x >= qk_blocks) {
     const int b = blockIdx.x - qk_blocks, tiles = ceil_div(N - qk, FIN_V_COLS);
@@ -635,7 +636,7 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
   *reinterpret_cast<floatx4*>(&vals[wave][lane * 4]) = g;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int r = (n + j) % half;
+    const int r = (n + j) & (half - 1);
     cosv[j] = cs[r], sinv[j] = cs[half + r];
   }
   wave_lds_order();
@@ -644,21 +645,21 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
   floatx4 y;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    y[j] = (n + j) % d < half ? g[j] * cosv[j] - partner[j] * sinv[j] : partner[j] * sinv[j] + g[j] * cosv[j];
+    y[j] = ((n + j) & half) == 0 ? g[j] * cosv[j] - partner[j] * sinv[j] : partner[j] * sinv[j] + g[j] * cosv[j];
   bf16_t* keys = page + (size_t)(pos % rope.P) * d;
   if (d % 4 == 0) {  // four columns of one head
-    const int head = n / d;
+    const int head = n >> log_d;
     if (n < qk)
-      *reinterpret_cast<uint2_any*>(head < rope.H ? q_out + (size_t)m * ldq + n : keys + (size_t)(head - rope.H) * rope.P * d + n % d) =
+      *reinterpret_cast<uint2_any*>(head < rope.H ? q_out + (size_t)m * ldq + n : keys + (size_t)(head - rope.H) * rope.P * d + (n & (d - 1))) =
           uint2_any{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
     return;
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {  // heads of 2
-    const int head = (n + j) / d;
+    const int head = (n + j) >> log_d;
     if (n + j >= qk) continue;
     if (head < rope.H) q_out[(size_t)m * ldq + n + j] = float_to_bf16(y[j]);
-    else keys[(size_t)(head - rope.H) * rope.P * d + (n + j) % d] = float_to_bf16(y[j]);
+    else keys[(size_t)(head - rope.H) * rope.P * d + ((n + j) & (d - 1))] = float_to_bf16(y[j]);
   }
 }
 
