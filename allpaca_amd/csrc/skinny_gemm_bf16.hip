@@ -187,13 +187,13 @@ __global__ __launch_bounds__(WPB * 64, sk_waves(MG, MODE, NB, WPB, PRE)) void sk
   // left (PRE; the 4 * WPB (wave, c) pairs of the block take groups of 4 bands in turn, the pieces meet in LDS with
   // the partial sums of the product), and what the finishing wave of an output band adds to (residual, EMIT: g).
   // Two row groups' steps leave registers for two of these loads, which wait for their sum until the stream is through.
-  constexpr int AT_ONCE = MG == 1 ? SS_LOADS : 2;
   float ss_piece = 0.f;
-  floatx4 ss_v[AT_ONCE];
+  floatx4 ss_v[2];
+  const int ss_groups = PRE ? norm.ld_ss / 4 : 0;
   auto ss_load = [&](int j) {
     const int q = wave * 4 + c + j * WPB * 4;
-    return q * 4 < norm.ld_ss ? *reinterpret_cast<const floatx4*>(norm.ss + (size_t)i * norm.ld_ss + q * 4)
-                              : floatx4{0.f, 0.f, 0.f, 0.f};
+    return q < ss_groups ? *reinterpret_cast<const floatx4*>(norm.ss + (size_t)i * norm.ld_ss + q * 4)
+                         : floatx4{0.f, 0.f, 0.f, 0.f};
   };
   auto ss_add = [&](const floatx4& v, int j) {
     const int q = wave * 4 + c + j * WPB * 4;
@@ -201,13 +201,14 @@ __global__ __launch_bounds__(WPB * 64, sk_waves(MG, MODE, NB, WPB, PRE)) void sk
     for (int e = 0; e < 4; ++e)
       if (q * 4 + e < norm.n_ss) ss_piece += v[e];
   };
-  if constexpr (PRE) {
+  if constexpr (PRE && MG == 1) {
+    floatx4 v[SS_LOADS];
 #pragma unroll
-    for (int j = 0; j < AT_ONCE; ++j) ss_v[j] = ss_load(j);
-    if constexpr (MG == 1) {
+    for (int j = 0; j < SS_LOADS; ++j) v[j] = ss_load(j);
 #pragma unroll
-      for (int j = 0; j < AT_ONCE; ++j) ss_add(ss_v[j], j);
-    }
+    for (int j = 0; j < SS_LOADS; ++j) ss_add(v[j], j);
+  } else if constexpr (PRE) {
+    ss_v[0] = ss_load(0), ss_v[1] = ss_load(1);
   }
   constexpr int ITEMS = OUT_BANDS;  // bands to finish: wave w finishes band w
   const int fin_n = (band0 + wave) * 16 + c * 4;  // first of this lane's 4 columns if this wave finishes a band
@@ -268,10 +269,9 @@ __global__ __launch_bounds__(WPB * 64, sk_waves(MG, MODE, NB, WPB, PRE)) void sk
 
   if constexpr (PRE) {
     if constexpr (MG == 2) {
-#pragma unroll
-      for (int j = 0; j < AT_ONCE; ++j) ss_add(ss_v[j], j);
+      ss_add(ss_v[0], 0), ss_add(ss_v[1], 1);
 #pragma unroll 1
-      for (int j = AT_ONCE; j * WPB * 16 < norm.ld_ss; ++j) ss_add(ss_load(j), j);   // more bands than 32 a wave
+      for (int j = 2; j * WPB * 4 < ss_groups; ++j) ss_add(ss_load(j), j);   // more bands than 32 a wave
     }
     ss_piece += __shfl_xor(ss_piece, 16);
     ss_piece += __shfl_xor(ss_piece, 32);
