@@ -13,10 +13,14 @@
 // piece of LDS of its own.
 //
 // What bounds it: with few rows the bytes of W, else the matrix cores' float32 rate (157 TFLOP/s, of which a library
-// product of 8,192^3 reaches 151).  Measured, microseconds (in brackets the kernel of one fma chain an output on the
-// vector units, which takes the other types): 4 rows x 2,048 outputs x K 2,048 9.4; x 128,256 outputs 149 (7.1 TB/s);
-// 330 rows x 16,384 outputs 206 (about 1,600; 107 TFLOP/s); 2,048 rows x 2,048 outputs x K 8,192 531 (129 TFLOP/s).  The
-// 65 products of a step of a 1B model in float32: 4 rows 1.12 ms (40.3), 340 rows 6.6 ms (38.9).
+// product of 8,192^3 reaches 151 and a loop of these instructions 156).  Blocks of the large tiles go on to further tiles
+// with the next one's first loads on their way while the eight waves meet, and a stage's LDS stores and loads stand between
+// its first half's products: 325 rows x 8,192 outputs of SwiGLU 200 -> 187 us, x 2,048 outputs x K 2,048 32.2 -> 29.6, K
+// 8,192 104.9 -> 101 (108 TFLOP/s).  What is left there: the loads (without them, timing only, 14 % less: their way into the
+// registers beside the products) and, for every tile, 3 us in which the waves meet.  Measured, microseconds (in brackets
+// the kernel of one fma chain an output on the vector units, which takes the other types): 4 rows x 2,048 outputs x K
+// 2,048 7.8; x 128,256 outputs 149 (7.1 TB/s); 325 rows x 16,384 outputs and SwiGLU 187 (about 1,600; 117 TFLOP/s); 2,048
+// rows x 2,048 outputs x K 8,192 519 (132 TFLOP/s).
 #include "mfma.h"
 #include <math.h>
 
@@ -48,15 +52,16 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
     const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, void* __restrict__ C, int c_dtype,
     int ldc, int M, int N, int K, int mode, int tiles_m, int tiles) {
   constexpr int BANDS = MT + NT;
-  constexpr int STAGE_F4 = BANDS * 128, SUM_F4 = MT * NT * 64;       // float4 a wave: its stage, its sums
-  __shared__ f32x4 lds[SL * (STAGE_F4 > SUM_F4 ? STAGE_F4 : SUM_F4)];
-  // The block ids that one XCD gets (every eighth) are a run of tiles, row tiles of the same outputs next to each other:
-  // they share W in that XCD's L2.
-  const int per = (tiles + 7) / 8;
-  const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (t >= tiles || (int)(blockIdx.x / 8) >= per) return;
+  constexpr bool ON = SL == SLICES && D == 1;                         // tile after tile (large tiles, a long K)
+  constexpr int STAGE_F4 = BANDS * 128, SUM_F4 = MT * NT * 64;       // float4 a wave: its stage, and at the end its sums
+  constexpr int WAVE_F4 = STAGE_F4 > SUM_F4 ? STAGE_F4 : SUM_F4;
+  __shared__ f32x4 lds[SL * WAVE_F4];
+  // The block ids that one XCD gets (every eighth) take a run of tiles, row tiles of the same outputs next to each other:
+  // they share W in that XCD's L2.  A block goes on to the tile gridDim.x / 8 further in its run.
+  const int per = (tiles + 7) / 8, first = (blockIdx.x % 8) * per, last = min(tiles, first + per), stride = gridDim.x / 8;
+  int t = first + blockIdx.x / 8;
+  if (t >= last) return;
   constexpr int NO = GLU ? NT / 2 : NT;                              // bands of outputs
-  const int m0 = (t % tiles_m) * (16 * MT), n0 = (t / tiles_m) * (16 * NO);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
 
   const int slice = STAGE * ((K + STAGE * SLICES - 1) / (STAGE * SLICES));
@@ -66,41 +71,51 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
   // What this lane loads of a stage: rows lane/8 and lane/8 + 8 of every band, 4 k at (lane%8)*4.  Rows past the end are
   // the last row again (their sums are not stored); for k past the end it loads the stage's first k, and 0 goes into LDS.
   const int lr = lane / 8, lk = (lane % 8) * 4;
-  const int rows_w = min(N - n0, 16 * NO), rows_a = min(M - m0, 16 * MT);
-  const BufferRsrc from_w = make_rsrc(W + (size_t)n0 * ldw), from_a = make_rsrc(A + (size_t)m0 * lda);
-  int off[BANDS][2];
-#pragma unroll
-  for (int b = 0; b < BANDS; ++b)
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      off[b][h] = 4 * (lk + (b < NT ? ((b < NO ? 0 : N) + min(16 * (b % NO) + lr + 8 * h, rows_w - 1)) * ldw : min(16 * (b - NT) + lr + 8 * h, rows_a - 1) * lda));
-  f32x4 reg[D][BANDS][2];
-  auto load = [&](int slot, int s) __attribute__((always_inline)) {
-    const int at = 4 * (k0 + s * STAGE);
-    const int back = k0 + s * STAGE + lk >= K ? 4 * lk : 0;
+  BufferRsrc from_w, from_a;
+  int off[BANDS][2], m0, n0;
+  auto aim = [&](int tile) __attribute__((always_inline)) {          // the loads that follow are of this tile
+    m0 = (tile % tiles_m) * (16 * MT), n0 = (tile / tiles_m) * (16 * NO);
+    const int rows_w = min(N - n0, 16 * NO), rows_a = min(M - m0, 16 * MT);
+    from_w = make_rsrc(W + (size_t)n0 * ldw), from_a = make_rsrc(A + (size_t)m0 * lda);
 #pragma unroll
     for (int b = 0; b < BANDS; ++b)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        reg[slot][b][h] = b < NT ? load_f32x4<ONCE>(from_w, off[b][h] - back, at) : load_f32x4<false>(from_a, off[b][h] - back, at);
+        off[b][h] = 4 * (lk + (b < NT ? ((b < NO ? 0 : N) + min(16 * (b % NO) + lr + 8 * h, rows_w - 1)) * ldw : min(16 * (b - NT) + lr + 8 * h, rows_a - 1) * lda));
+  };
+  f32x4 reg[D][BANDS][2];
+  auto load_one = [&](int slot, int s, int b, int h) __attribute__((always_inline)) {
+    const int at = 4 * (k0 + s * STAGE);
+    const int back = k0 + s * STAGE + lk >= K ? 4 * lk : 0;
+    reg[slot][b][h] = b < NT ? load_f32x4<ONCE>(from_w, off[b][h] - back, at) : load_f32x4<false>(from_a, off[b][h] - back, at);
+  };
+  auto load = [&](int slot, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < BANDS; ++b)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) load_one(slot, s, b, h);
   };
 
   // the wave's stage in LDS: row r of a band is 8 pieces of 16 bytes, piece c at place c ^ (r % 8) (reads of one piece
   // over eight rows then fall on different banks)
-  f32x4* mine = lds + wave * STAGE_F4;
+  f32x4* mine = lds + wave * WAVE_F4;
   const int put_at = lr * 8 + ((lane % 8) ^ lr);
   const int row = lane % 16, quarter = lane / 16;
   const int get_at[2] = {row * 8 + (quarter ^ (row % 8)), row * 8 + ((quarter + 4) ^ (row % 8))};
-  auto put = [&](int slot, int s) __attribute__((always_inline)) {
-#pragma unroll
-    for (int b = 0; b < BANDS; ++b)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) mine[b * 128 + h * 64 + put_at] = reg[slot][b][h];
+  auto put_one = [&](int slot, int b, int h) __attribute__((always_inline)) { mine[b * 128 + h * 64 + put_at] = reg[slot][b][h]; };
+  auto put_end = [&](int s) __attribute__((always_inline)) {
     if (k0 + (s + 1) * STAGE > K && k0 + s * STAGE + lk >= K) {
 #pragma unroll
       for (int b = 0; b < 2 * BANDS; ++b) mine[b * 64 + put_at] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     wave_lds_order();
+  };
+  auto put = [&](int slot, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < BANDS; ++b)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) put_one(slot, b, h);
+    put_end(s);
   };
   f32x4 f[2][BANDS];                                    // operands of a stage's first and second 16 k
   auto get = [&](int half) __attribute__((always_inline)) {
@@ -109,100 +124,179 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
     wave_lds_order();
   };
   floatx4 acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto multiply_one = [&](int half, int u) __attribute__((always_inline)) {            // the u-th product of a half
+    const int e = u / (MT * NT), i = u / NT % MT, j = u % NT;
+    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[half][j][e], f[half][NT + i][e], acc[i][j], 0, 0, 0);
+  };
+  constexpr int PRODUCTS = 4 * MT * NT;
   auto multiply = [&](int half) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[half][j][e], f[half][NT + i][e], acc[i][j], 0, 0, 0);
+    for (int u = 0; u < PRODUCTS; ++u) multiply_one(half, u);
   };
+  // The sums of a tile's eight slices, of what this thread stores: its q-th piece of four outputs.
+  constexpr int PIECES = (MT * NO + SL - 1) / SL;
+  auto meet = [&](f32x4 (&v)[PIECES]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) lds[wave * WAVE_F4 + (i * NT + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PIECES; ++q) {
+      const int p = threadIdx.x + q * 64 * SL;
+      if (p >= MT * NO * 64) continue;
+      const int i = p / (NO * 64), j = p / 64 % NO, l = p % 64;
+      auto sum = [&](int band) __attribute__((always_inline)) {
+        const int at = (i * NT + band) * 64 + l;
+        f32x4 u = lds[at];
+#pragma unroll
+        for (int w = 1; w < SL; ++w) u += lds[w * WAVE_F4 + at];
+        return u;
+      };
+      v[q] = sum(j);
+      if constexpr (GLU) {
+        const f32x4 u = sum(NO + j);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[q][e] = (v[q][e] / (1.0f + expf(-v[q][e]))) * u[e];
+      }
+    }
+  };
+  const bool wide = mode == 0 && c_dtype == APC_F32 && ldc % 4 == 0 && ((uintptr_t)C & 15u) == 0;   // 16-byte stores
+  auto leave = [&](const f32x4 (&v)[PIECES], int row0, int out0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < PIECES; ++q) {
+      const int p = threadIdx.x + q * 64 * SL;
+      const int m = row0 + p / (NO * 64) * 16 + p % 16, n = out0 + p / 64 % NO * 16 + (p % 64 / 16) * 4;
+      if (p >= MT * NO * 64 || m >= M) continue;
+      if (wide && n + 4 <= N) {
+        *(f32x4*)((float*)C + (size_t)m * ldc + n) = v[q];
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) continue;
+        const size_t o = (size_t)m * ldc + n + e;
+        if (mode == 1) ((float*)C)[o] += v[q][e];
+        else store_f(C, c_dtype, o, v[q][e]);
+      }
+    }
+  };
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+
+  aim(t);
+  clear();
+  f32x4 v[PIECES];
   // A stage: its second operands come out of LDS under the first products; then the next stage goes in, the loads that
   // take its registers go out, and its first operands come back under the second products.
-  auto stage = [&](int s, int next_slot, bool next, bool more) __attribute__((always_inline)) {
-    get(1);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(0);
-    __builtin_amdgcn_sched_barrier(0);
-    if (next) {
-      put(next_slot, s + 1);
-      __builtin_amdgcn_sched_barrier(0);                // (the loads take the registers that have just been written out)
-      if (more) load(next_slot, s + 1 + D);
-      __builtin_amdgcn_sched_barrier(0);
-      get(0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(1);
-  };
-  auto begin = [&](auto count) __attribute__((always_inline)) {                        // stages there are, at least (what is known when compiling)
-    constexpr int R = decltype(count)::value;
-#pragma unroll
-    for (int u = 0; u < D && u < R; ++u) load(u, u);
-    put(0, 0);
-    if (R > D) load(0, D);
-    get(0);
-  };
-  auto finish = [&](int s0, auto count) __attribute__((always_inline)) {               // the last stages, without a condition between the loads
-    constexpr int R = decltype(count)::value;
-#pragma unroll
-    for (int i = 0; i < R; ++i) stage(s0 + i, (i + 1) % D, i + 1 < R, i + 1 + D < R);
-  };
-  // Straight code for the last 2 D stages: behind a branch that may have loaded the compiler waits for more than it needs.
-  if (steps > 2 * D) {
-    begin(Count<2 * D + 1>{});
-    int s0 = 0;
-    for (; steps - s0 > 2 * D; s0 += D)
-#pragma unroll
-      for (int u = 0; u < D; ++u) stage(s0 + u, (u + 1) % D, true, true);
-    each_count<2 * D>([&](auto r) __attribute__((always_inline)) {
-      if (steps - s0 == decltype(r)::value) finish(s0, r);
-    });
-  } else {
-    each_count<2 * D>([&](auto r) __attribute__((always_inline)) {
-      if (steps == decltype(r)::value) begin(r), finish(0, r);
-    });
-  }
-
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) lds[wave * SUM_F4 + (i * NT + j) * 64 + lane] = acc[i][j];
-  __syncthreads();
-  const bool wide = mode == 0 && c_dtype == APC_F32 && ldc % 4 == 0 && ((uintptr_t)C & 15u) == 0;   // 16-byte stores
-  for (int p = threadIdx.x; p < MT * NO * 64; p += 64 * SL) {
-    const int i = p / (NO * 64), j = p / 64 % NO, l = p % 64;
-    auto sum = [&](int band) __attribute__((always_inline)) {
-      const int at = (i * NT + band) * 64 + l;
-      f32x4 v = lds[at];
-#pragma unroll
-      for (int w = 1; w < SL; ++w) v += lds[w * SUM_F4 + at];
-      return v;
+  if constexpr (ON) {
+    // A block of these takes tile after tile.  Behind a tile's last stage its registers ask for the next tile's first one,
+    // which is there when the eight waves have met; a launch of several rounds then pays the way of the first loads (every
+    // wave's stage at once: 112 KB a unit), the block's start and the stores' way once and not every round.
+    int at_stage = 0, at_tile = t;                      // the stage that the next load is of, and its tile
+    auto asked = [&]() __attribute__((always_inline)) {
+      if (++at_stage == steps) {
+        at_stage = 0;
+        if (at_tile + stride < last) aim(at_tile += stride);         // (no tile left: a stage that nobody takes)
+      }
     };
-    f32x4 v = sum(j);
-    if constexpr (GLU) {
-      const f32x4 u = sum(NO + j);
+    auto first_in = [&]() __attribute__((always_inline)) {
+      put(0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(0, at_stage);
+      __builtin_amdgcn_sched_barrier(0);
+      asked();
+      get(0);
+    };
+    int row0 = m0, out0 = n0;                           // of the tile that is multiplied
+    if (steps > 0) load(0, 0), asked(), first_in();
+    while (true) {
+      if (steps > 0) {
+        for (int s = 0; s < steps - 1; ++s) {
+          get(1);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (v[e] / (1.0f + expf(-v[e]))) * u[e];
-    }
-    const int m = m0 + i * 16 + l % 16, n = n0 + j * 16 + (l / 16) * 4;
-    if (m >= M) continue;
-    if (wide && n + 4 <= N) {
-      *(f32x4*)((float*)C + (size_t)m * ldc + n) = v;
-      continue;
-    }
+          for (int u = 0; u < 2 * BANDS; ++u) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (n + e >= N) continue;
-      const size_t o = (size_t)m * ldc + n + e;
-      if (mode == 1) ((float*)C)[o] += v[e];
-      else store_f(C, c_dtype, o, v[e]);
+            for (int p = u * PRODUCTS / (2 * BANDS); p < (u + 1) * PRODUCTS / (2 * BANDS); ++p) multiply_one(0, p);
+            put_one(0, u / 2, u % 2);
+            load_one(0, at_stage, u / 2, u % 2);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          put_end(s + 1);
+          asked();
+          get(0);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(1);
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_waitcnt(0xc07f);           // LDS only
+        }
+        get(1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0);
+        multiply(1);
+      }
+      t += stride;
+      meet(v);
+      if (t < last) {
+        __syncthreads();                                // everyone has read the sums
+        clear();
+        if (steps > 0) first_in();
+      }
+      leave(v, row0, out0);
+      if (t >= last) break;
+      row0 = (t % tiles_m) * (16 * MT), out0 = (t / tiles_m) * (16 * NO);
     }
+  } else {
+    auto stage = [&](int s, int next_slot, bool next, bool more) __attribute__((always_inline)) {
+      get(1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (next) {
+        put(next_slot, s + 1);
+        __builtin_amdgcn_sched_barrier(0);                // (the loads take the registers that have just been written out)
+        if (more) load(next_slot, s + 1 + D);
+        __builtin_amdgcn_sched_barrier(0);
+        get(0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(1);
+    };
+    auto begin = [&](auto count) __attribute__((always_inline)) {                        // stages there are, at least (what is known when compiling)
+      constexpr int R = decltype(count)::value;
+#pragma unroll
+      for (int u = 0; u < D && u < R; ++u) load(u, u);
+      put(0, 0);
+      if (R > D) load(0, D);
+      get(0);
+    };
+    auto finish = [&](int s0, auto count) __attribute__((always_inline)) {               // the last stages, without a condition between the loads
+      constexpr int R = decltype(count)::value;
+#pragma unroll
+      for (int i = 0; i < R; ++i) stage(s0 + i, (i + 1) % D, i + 1 < R, i + 1 + D < R);
+    };
+    // Straight code for the last 2 D stages: behind a branch that may have loaded the compiler waits for more than it needs.
+    if (steps > 2 * D) {
+      begin(Count<2 * D + 1>{});
+      int s0 = 0;
+      for (; steps - s0 > 2 * D; s0 += D)
+#pragma unroll
+        for (int u = 0; u < D; ++u) stage(s0 + u, (u + 1) % D, true, true);
+      each_count<2 * D>([&](auto r) __attribute__((always_inline)) {
+        if (steps - s0 == decltype(r)::value) finish(s0, r);
+      });
+    } else {
+      each_count<2 * D>([&](auto r) __attribute__((always_inline)) {
+        if (steps == decltype(r)::value) begin(r), finish(0, r);
+      });
+    }
+    meet(v);
+    leave(v, m0, n0);
   }
 }
 
@@ -216,7 +310,9 @@ int launch_slices(const float* A, int lda, const float* W, int ldw, void* C, int
   const int tiles_m = ceil_div(M, 16 * MT);
   const long long tiles = (long long)tiles_m * ceil_div(N, 16 * (GLU ? NT / 2 : NT));
   if (tiles > (1 << 27)) return APC_ERR_BAD_ARG;
-  hipLaunchKernelGGL((gemm_f32_kernel<SL, MT, NT, D, ONCE, MIN_WAVES, GLU>), dim3(ceil_div((int)tiles, 8) * 8), dim3(64 * SL), 0,
+  int blocks = ceil_div((int)tiles, 8) * 8;
+  if (SL == SLICES && D == 1 && blocks > 256) blocks = 256;           // such a block has a compute unit to itself
+  hipLaunchKernelGGL((gemm_f32_kernel<SL, MT, NT, D, ONCE, MIN_WAVES, GLU>), dim3(blocks), dim3(64 * SL), 0,
                      stream, A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, tiles_m, (int)tiles);
   APC_LAUNCH_CHECK();
   return 0;
@@ -242,35 +338,43 @@ bool gemm_f32_takes(const void* A, int lda, const void* W, int ldw, int K) {
          ldw < (1 << 22);            // (64 rows fit a descriptor's 32-bit offsets)
 }
 
-// A tile of 16 mt x 16 nt and what a launch of its blocks costs: start and, for every 256 of them, round.
-struct TileCost { int mt, nt; bool shares; double start, round; };
+// A tile of 16 mt x 16 nt and what a launch of its blocks costs, in microseconds: once, and for every 256 of them (a round);
+// each a part that stays and a part that grows with K, as for K = 2,048.
+struct TileCost { int mt, nt; bool shares; double start, start_k, round, round_k; };
 template <int COUNT>
-static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, int outputs) {   // outputs: of 16 nt columns
+static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, double k_shares, double k_alone, int outputs) {   // outputs: of 16 nt columns
+  if (M <= 16) return 0;                                // (the other tiles multiply rows that are not there)
   int best = 0;
   double best_cost = 1e30;
   for (int i = 0; i < COUNT; ++i) {
     const TileCost& s = shapes[i];
     double rounds = (double)ceil_div(M, 16 * s.mt) * ceil_div(N, outputs * s.nt) / 256;
     if (!s.shares) rounds = ceil(rounds);
-    const double cost = s.start + s.round * (rounds > 1.0 ? rounds : 1.0);
+    const double k = (s.shares ? k_shares : k_alone) / 2048;
+    const double cost = s.start + s.start_k * k + (s.round + s.round_k * k) * (rounds > 1.0 ? rounds : 1.0);
     if (cost < best_cost) best = i, best_cost = cost;
   }
   return best;
 }
 
-// The tile: the least of these times (microseconds at K = 2,048; K stretches them alike) over the tiles' shapes.  A
-// block of the small tiles shares its compute unit with others, so their time grows with the blocks; the large ones have
-// a unit to themselves and go in whole rounds of 256.  Measured on 24 to 2,048 rows x 2,048 to 16,384 outputs, where the
-// choice is within a tenth of the best of the six: 2,048 outputs take 9.4 us up to 48 rows, 18 at 160 rows (48 x 32
-// tiles; 16 x 16: 25, 64 x 64: 41), 31 at 330 (48 x 64; 16 x 16: 43).  (The 64 x 64 tile keeps 48 registers of loads in
-// scratch memory and is the best from 512 rows x 2,048 outputs on all the same: 43 us against 50 and 53 of the next two,
-// 1,024 rows x 8,192 311 against 317.)
+// The tile: the least expected time.  A block of the small tiles shares its compute unit with others, so their time grows
+// with the blocks; the large ones have a unit to themselves and go in whole rounds of 256.  Fitted to 33 to 2,048 rows x
+// 2,048 and 3,072 outputs, K 256 to 8,192: the choice takes 1.01 of the best tile's time in the mean, 1.15 at worst.  At
+// K = 2,048, 2,048 outputs take 10.1 us at 33 rows (32 x 16 tiles; 32 x 32 13.1, 48 x 32 17.1), 13.3 at 100 (32 x 32;
+// 32 x 16: 15.6), 29.5 at 325 (48 x 64; 48 x 32: 31.8, 64 x 64: 38.2), 39 at 400 and 146 at 2,048 rows (64 x 64; 48 x 64:
+// 55, 159).
 // Up to K = 128 (see launch_slices) blocks of all tiles share their units.
-constexpr TileCost TILES[] = {{1, 1, true, 4.5, 5.0},   {2, 1, true, 4.0, 5.8},   {2, 2, false, 1.5, 13.0},
-                              {3, 2, false, 1.5, 15.5}, {3, 4, false, 1.5, 28.7}, {4, 4, false, 1.5, 39.0}};
-constexpr TileCost TILES_SHORT[] = {{1, 1, true, 3.6, 0.75}, {2, 1, true, 3.6, 0.95}, {2, 2, true, 4.1, 0.69},
-                                    {3, 2, true, 4.4, 0.93}};        // (48 x 64 and 64 x 64 are never the least)
-static int tile_of(int M, int N, int K) { return K <= 4 * STAGE ? least_cost(TILES_SHORT, M, N, 16) : least_cost(TILES, M, N, 16); }
+constexpr TileCost TILES[] = {{1, 1, true, 2.1, 0.5, 0.5, 4.7},    {2, 1, true, 2.1, 0.9, 0.5, 5.9},   {2, 2, false, 2.4, 0.5, 1.1, 9.0},
+                              {3, 2, false, 2.3, 0.4, 1.5, 12.7}, {3, 4, false, 2.4, 0.4, 2.6, 23.5}, {4, 4, false, 2.0, 0.6, 4.3, 30.7}};
+constexpr TileCost TILES_SHORT[] = {{1, 1, true, 3.6, 0.0, 0.75, 0.0}, {2, 1, true, 3.6, 0.0, 0.95, 0.0}, {2, 2, true, 4.1, 0.0, 0.69, 0.0},
+                                    {3, 2, true, 4.4, 0.0, 0.93, 0.0}};        // (48 x 64 and 64 x 64 are never the least)
+static int tile_of(int M, int N, int K) {
+  if (K <= 4 * STAGE) return least_cost(TILES_SHORT, M, N, K, K, 16);
+  // a K between two multiples of 256 leaves waves with a stage less than the others: 480 rows x 2,048 outputs at K = 256,
+  // 320, 512 take 11.4, 14.4, 16.6 us on 32 x 16 tiles and 12.6, 17.8, 18.9 on 48 x 64
+  const int over = SLICES * STAGE * ceil_div(K, SLICES * STAGE) - K;
+  return least_cost(TILES, M, N, K + 0.4 * over, K + 0.8 * over, 16);
+}
 
 // Rows of the tile, times 1,000, and its outputs.
 APC_EXPORT int apc_gemm_f32_tile(int M, int N, int K) {
@@ -304,10 +408,12 @@ APC_EXPORT int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int l
   return gemm_f32_takes(A, lda, W, ldw, K) && ((long long)F + 64) * ldw < (1LL << 29);   // byte offsets of 32 bits
 }
 
-constexpr TileCost GLU_TILES[] = {{1, 2, true, 4.5, 8.5}, {2, 2, false, 1.5, 13.0}, {3, 2, false, 1.5, 15.5},
-                                  {3, 4, false, 1.5, 28.7}, {4, 4, false, 1.5, 39.0}};
-constexpr TileCost GLU_TILES_SHORT[] = {{1, 2, true, 3.6, 0.95}, {2, 2, true, 4.1, 0.69}, {3, 2, true, 4.4, 0.93}};
-static int glu_tile_of(int M, int F, int K) { return K <= 4 * STAGE ? least_cost(GLU_TILES_SHORT, M, F, 8) : least_cost(GLU_TILES, M, F, 8); }
+// (33 to 2,048 rows x 4,096 and 8,192 outputs, K 256 to 2,048: never more than 1.03 of the best tile's time.  K = 2,048, 8,192
+// outputs: 325 rows 188 us on 48 x 32 tiles, 205 on 48 x 16, 211 on 64 x 32; 100 rows 76 on 64 x 32, 85 on 48 x 32.)
+constexpr TileCost GLU_TILES[] = {{1, 2, true, 2.5, 2.5, 0.7, 7.8}, {2, 2, false, 2.1, 4.8, 1.4, 8.9}, {3, 2, false, 2.6, 5.5, 1.7, 12.4},
+                                  {3, 4, false, 2.6, 4.8, 2.7, 22.9}, {4, 4, false, 3.1, 4.0, 3.6, 30.5}};
+constexpr TileCost GLU_TILES_SHORT[] = {{1, 2, true, 3.6, 0.0, 0.95, 0.0}, {2, 2, true, 4.1, 0.0, 0.69, 0.0}, {3, 2, true, 4.4, 0.0, 0.93, 0.0}};
+static int glu_tile_of(int M, int F, int K) { return K <= 4 * STAGE ? least_cost(GLU_TILES_SHORT, M, F, K, K, 8) : least_cost(GLU_TILES, M, F, K, K, 8); }
 
 // Rows of the tile, times 1,000, and its outputs (half of the columns it computes).
 APC_EXPORT int apc_swiglu_f32_tile(int M, int F, int K) {

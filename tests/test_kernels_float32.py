@@ -60,6 +60,19 @@ def test_product_against_64_bits_and_rows_alone(M, N, K):
     assert torch.equal(both, add + out)
 
 
+# more tiles than compute units: a block's second and third tile, with slices of no, one, two and several stages, tiles
+# that a block has one more of than its neighbour, and outputs that are added to
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(700, 4099, 132), (700, 4099, 256), (331, 6145, 300), (490, 3100, 580), (1030, 2045, 776)])
+def test_product_of_more_tiles_than_units(M, N, K):
+    test_product_against_64_bits_and_rows_alone(M, N, K)
+    a, w = gen(M, K, seed=3), gen(N, K, seed=4)
+    out, added = torch.empty(M, N, device=DEV), torch.ones(M, N, device=DEV)
+    ops().gemm_plain(a, w, out)
+    ops().gemm_plain(a, w, added, accumulate=True)
+    assert torch.equal(added, out + 1.0)
+
+
 @pytest.mark.gpu
 def test_product_of_views_reads_nothing_past_their_width():
     """Rows of a wider matrix whose other columns hold NaN, outputs into a wider matrix, bfloat16 outputs."""

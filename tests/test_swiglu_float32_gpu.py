@@ -35,6 +35,12 @@ def test_both_products_and_the_activation(M, F, K, pad):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,F,K", [(700, 9000, 132), (331, 9001, 256), (200, 8200, 520)])
+def test_both_products_of_more_tiles_than_units(M, F, K):
+    test_both_products_and_the_activation(M, F, K, 0)
+
+
+@pytest.mark.gpu
 def test_rows_that_are_no_pieces_of_16_bytes_are_left_alone():
     from allpaca_amd.kernels import ops
     h, w = gen(4, 63).to(DEV), gen(48, 63).to(DEV)
