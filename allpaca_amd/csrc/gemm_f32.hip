@@ -27,6 +27,7 @@
 namespace {
 
 constexpr int SLICES = 8, STAGE = 32;
+constexpr int NORM_K = 4096;            // the longest row that a product normalises by itself
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -43,19 +44,58 @@ __device__ __forceinline__ void each_count(F f) {        // f(1), .. f(N), known
   f(Count<N>{});
 }
 
+__device__ __forceinline__ float row_scale(float squares, int K, float eps) { return 1.0f / sqrtf(squares / (float)K + eps); }
+
+// H = A * G and R = 1 / sqrt(mean square + eps) of rows in front of an RMS norm, with the operations of the product's NORM
+// form: 32 lanes a row, a lane the quarter of a slice's 16 k that an operand's lane holds there.
+__global__ __launch_bounds__(64) void norm_rows_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ G, float eps,
+                                                           float* __restrict__ H, float* __restrict__ R, int M, int K) {
+  const int lane = threadIdx.x % 32, m = min((int)(blockIdx.x * 2 + threadIdx.x / 32), M - 1);   // (a last row twice: the same values)
+  const int slice = STAGE * ((K + STAGE * SLICES - 1) / (STAGE * SLICES)), k0 = lane / 4 * slice, end = min(K, k0 + slice);
+  const float* a = A + (size_t)m * lda;
+  float ss[2] = {0.f, 0.f};
+  for (int k = k0 + lane % 4 * 4; k < end; k += 128) {
+    f32x4 v[8], g[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = g[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k + 16 * u < end) v[u] = *(const f32x4*)(a + k + 16 * u), g[u] = *(const f32x4*)(G + k + 16 * u);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss[e % 2] = fmaf(v[u][e], v[u][e], ss[e % 2]), v[u][e] *= g[u][e];
+      if (k + 16 * u < end) *(f32x4*)(H + (size_t)m * K + k + 16 * u) = v[u];
+    }
+  }
+  float own = ss[0] + ss[1];
+  own += __shfl_xor(own, 1), own += __shfl_xor(own, 2);
+  float all = 0.f;
+#pragma unroll
+  for (int w = 0; w < SLICES; ++w) all += __shfl(own, w * 4, 32);
+  if (lane == 0) R[m] = row_scale(all, K, eps);
+}
+
 // MT x NT tiles of 16 rows x 16 outputs a block, D stages of loads ahead.
 // GLU: W is [2 N][K], rows of gates and then rows of values; a block's bands of W are NT / 2 of gates and the NT / 2 of
 // values that belong to them, and it writes silu(gate) * value.  A product is the same sum as without, so the result is
 // the bits of the product of 2 N outputs and the activation's own pass.
-template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU>
+// NORM: A is the row in front of an RMS norm of weight G.  Every block reads whole rows of A anyway (a wave its own k), so a
+// wave multiplies its operands by G, adds up the squares beside that, and the sums are scaled by the row's 1 / sqrt(mean
+// square + eps) where the waves meet.  The squares of a row are added in an order that depends on K alone, too.  For one row
+// tile only: with several, every block does it again for the same rows (325 rows x 8,192 outputs of SwiGLU 194 -> 205 us,
+// twice the norm's own launch), so norm_rows_f32_kernel does it once, with the same operations, and R has the rows' scales.
+template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU, bool NORM>
 __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
-    const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, void* __restrict__ C, int c_dtype,
-    int ldc, int M, int N, int K, int mode, int tiles_m, int tiles) {
+    const float* __restrict__ A, int lda, const float* __restrict__ G, float eps, const float* __restrict__ R,
+    const float* __restrict__ W, int ldw, void* __restrict__ C, int c_dtype, int ldc, int M, int N, int K, int mode, int tiles_m, int tiles) {
   constexpr int BANDS = MT + NT;
   constexpr bool ON = SL == SLICES && D == 1;                         // tile after tile (large tiles, a long K)
   constexpr int STAGE_F4 = BANDS * 128, SUM_F4 = MT * NT * 64;       // float4 a wave: its stage, and at the end its sums
   constexpr int WAVE_F4 = STAGE_F4 > SUM_F4 ? STAGE_F4 : SUM_F4;
   __shared__ f32x4 lds[SL * WAVE_F4];
+  __shared__ float squares[NORM ? SL * 16 * MT : 1];
+  __shared__ f32x4 gains[NORM ? NORM_K / 4 : 1];
   // The block ids that one XCD gets (every eighth) take a run of tiles, row tiles of the same outputs next to each other:
   // they share W in that XCD's L2.  A block goes on to the tile gridDim.x / 8 further in its run.
   const int per = (tiles + 7) / 8, first = (blockIdx.x % 8) * per, last = min(tiles, first + per), stride = gridDim.x / 8;
@@ -89,6 +129,22 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
     const int back = k0 + s * STAGE + lk >= K ? 4 * lk : 0;
     reg[slot][b][h] = b < NT ? load_f32x4<ONCE>(from_w, off[b][h] - back, at) : load_f32x4<false>(from_a, off[b][h] - back, at);
   };
+  float ss[NORM ? MT : 1][2];                           // squares of row lane % 16 of a band of A, of the k that this lane holds
+  // G goes into LDS behind the first stages' loads: in registers beside every stage in flight it cost the tiles of few rows
+  // their second block a unit.
+  f32x4 gain[NORM ? NORM_K / (256 * SL) : 1] = {};
+  if constexpr (NORM) {
+#pragma unroll
+    for (int q = 0; q < NORM_K / (256 * SL); ++q)
+      if (threadIdx.x + q * 64 * SL < K / 4) gain[q] = reinterpret_cast<const f32x4*>(G)[threadIdx.x + q * 64 * SL];
+  }
+  auto gains_in = [&]() __attribute__((always_inline)) {
+    if constexpr (NORM) {
+#pragma unroll
+      for (int q = 0; q < NORM_K / (256 * SL); ++q) gains[threadIdx.x + q * 64 * SL] = gain[q];
+      __syncthreads();
+    }
+  };
   auto load = [&](int slot, int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int b = 0; b < BANDS; ++b)
@@ -117,11 +173,23 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       for (int h = 0; h < 2; ++h) put_one(slot, b, h);
     put_end(s);
   };
-  f32x4 f[2][BANDS];                                    // operands of a stage's first and second 16 k
-  auto get = [&](int half) __attribute__((always_inline)) {
+  f32x4 f[2][BANDS], g[NORM ? 2 : 1];                   // operands of a stage's first and second 16 k, the gains of those
+  auto get = [&](int half, int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int b = 0; b < BANDS; ++b) f[half][b] = mine[b * 128 + get_at[half]];
+    if constexpr (NORM) g[half] = gains[(k0 + s * STAGE) / 4 + quarter + 4 * half];
     wave_lds_order();
+  };
+  auto normalise = [&](int half) __attribute__((always_inline)) {      // (zeros past the end of a row)
+    if constexpr (NORM) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          ss[i][e % 2] = fmaf(f[half][NT + i][e], f[half][NT + i][e], ss[i][e % 2]);
+          f[half][NT + i][e] *= g[half][e];
+        }
+    }
   };
   floatx4 acc[MT][NT];
   auto multiply_one = [&](int half, int u) __attribute__((always_inline)) {            // the u-th product of a half
@@ -130,16 +198,33 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
   };
   constexpr int PRODUCTS = 4 * MT * NT;
   auto multiply = [&](int half) __attribute__((always_inline)) {
+    normalise(half);
 #pragma unroll
     for (int u = 0; u < PRODUCTS; ++u) multiply_one(half, u);
   };
   // The sums of a tile's eight slices, of what this thread stores: its q-th piece of four outputs.
   constexpr int PIECES = (MT * NO + SL - 1) / SL;
+  float scale[PIECES];
+  auto load_scale = [&](int row0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < PIECES; ++q) {
+      const int p = threadIdx.x + q * 64 * SL, m = row0 + p / (NO * 64) * 16 + p % 16;
+      scale[q] = !NORM && R && p < MT * NO * 64 ? R[min(m, M - 1)] : 1.f;
+    }
+  };
   auto meet = [&](f32x4 (&v)[PIECES]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) lds[wave * WAVE_F4 + (i * NT + j) * 64 + lane] = acc[i][j];
+    if constexpr (NORM) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        float own = ss[i][0] + ss[i][1];
+        own += __shfl_xor(own, 16), own += __shfl_xor(own, 32);
+        if (quarter == 0) squares[wave * 16 * MT + i * 16 + row] = own;
+      }
+    }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < PIECES; ++q) {
@@ -153,9 +238,15 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
         for (int w = 1; w < SL; ++w) u += lds[w * WAVE_F4 + at];
         return u;
       };
-      v[q] = sum(j);
+      if constexpr (NORM) {
+        float all = 0.f;
+#pragma unroll
+        for (int w = 0; w < SL; ++w) all += squares[w * 16 * MT + i * 16 + l % 16];
+        scale[q] = row_scale(all, K, eps);
+      }
+      v[q] = sum(j) * scale[q];
       if constexpr (GLU) {
-        const f32x4 u = sum(NO + j);
+        const f32x4 u = sum(NO + j) * scale[q];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[q][e] = (v[q][e] / (1.0f + expf(-v[q][e]))) * u[e];
       }
@@ -186,6 +277,10 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (NORM) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) ss[i][0] = ss[i][1] = 0.f;
+    }
   };
 
   aim(t);
@@ -210,15 +305,19 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       load(0, at_stage);
       __builtin_amdgcn_sched_barrier(0);
       asked();
-      get(0);
+      get(0, 0);
     };
     int row0 = m0, out0 = n0;                           // of the tile that is multiplied
-    if (steps > 0) load(0, 0), asked(), first_in();
+    if (steps > 0) load(0, 0), asked();
+    gains_in();
+    if (steps > 0) first_in();
     while (true) {
+      load_scale(row0);
       if (steps > 0) {
         for (int s = 0; s < steps - 1; ++s) {
-          get(1);
+          get(1, s);
           __builtin_amdgcn_sched_barrier(0);
+          normalise(0);
 #pragma unroll
           for (int u = 0; u < 2 * BANDS; ++u) {
 #pragma unroll
@@ -229,13 +328,13 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
           }
           put_end(s + 1);
           asked();
-          get(0);
+          get(0, s + 1);
           __builtin_amdgcn_sched_barrier(0);
           multiply(1);
           __builtin_amdgcn_sched_barrier(0);
           __builtin_amdgcn_s_waitcnt(0xc07f);           // LDS only
         }
-        get(1);
+        get(1, steps - 1);
         __builtin_amdgcn_sched_barrier(0);
         multiply(0);
         multiply(1);
@@ -252,8 +351,9 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       row0 = (t % tiles_m) * (16 * MT), out0 = (t / tiles_m) * (16 * NO);
     }
   } else {
+    load_scale(m0);
     auto stage = [&](int s, int next_slot, bool next, bool more) __attribute__((always_inline)) {
-      get(1);
+      get(1, s);
       __builtin_amdgcn_sched_barrier(0);
       multiply(0);
       __builtin_amdgcn_sched_barrier(0);
@@ -262,7 +362,7 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
         __builtin_amdgcn_sched_barrier(0);                // (the loads take the registers that have just been written out)
         if (more) load(next_slot, s + 1 + D);
         __builtin_amdgcn_sched_barrier(0);
-        get(0);
+        get(0, s + 1);
       }
       __builtin_amdgcn_sched_barrier(0);
       multiply(1);
@@ -271,9 +371,10 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       constexpr int R = decltype(count)::value;
 #pragma unroll
       for (int u = 0; u < D && u < R; ++u) load(u, u);
+      gains_in();
       put(0, 0);
       if (R > D) load(0, D);
-      get(0);
+      get(0, 0);
     };
     auto finish = [&](int s0, auto count) __attribute__((always_inline)) {               // the last stages, without a condition between the loads
       constexpr int R = decltype(count)::value;
@@ -294,6 +395,7 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       each_count<2 * D>([&](auto r) __attribute__((always_inline)) {
         if (steps == decltype(r)::value) begin(r), finish(0, r);
       });
+      if (steps <= 0) gains_in();
     }
     meet(v);
     leave(v, m0, n0);
@@ -304,24 +406,27 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
 // its waves idle and 128 KiB of LDS taken.  2,048 rows x 16,384 outputs at K = 32, 64, 128: 200, 203, 216 us with eight
 // slices and stores of 4 bytes, 84, 101, 147 with the two or four there are, 53, 69, 125 with 16-byte stores beside (one
 // fma chain an output on the vector units: 70, 98, 150).
-template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU>
-int launch_slices(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
-           hipStream_t stream) {
+template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU, bool NORM>
+int launch_slices(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C,
+                  int c_dtype, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
   const int tiles_m = ceil_div(M, 16 * MT);
   const long long tiles = (long long)tiles_m * ceil_div(N, 16 * (GLU ? NT / 2 : NT));
   if (tiles > (1 << 27)) return APC_ERR_BAD_ARG;
   int blocks = ceil_div((int)tiles, 8) * 8;
   if (SL == SLICES && D == 1 && blocks > 256) blocks = 256;           // such a block has a compute unit to itself
-  hipLaunchKernelGGL((gemm_f32_kernel<SL, MT, NT, D, ONCE, MIN_WAVES, GLU>), dim3(blocks), dim3(64 * SL), 0,
-                     stream, A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, tiles_m, (int)tiles);
+  hipLaunchKernelGGL((gemm_f32_kernel<SL, MT, NT, D, ONCE, MIN_WAVES, GLU, NORM>), dim3(blocks), dim3(64 * SL), 0,
+                     stream, A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, tiles_m, (int)tiles);
   APC_LAUNCH_CHECK();
   return 0;
 }
 
 template <int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU = false>
-int launch(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
-           hipStream_t stream) {
-#define SL_GO(SL_) return launch_slices<SL_, MT, NT, D, ONCE, MIN_WAVES, GLU>(A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
+int launch(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C, int c_dtype,
+           int ldc, int M, int N, int K, int mode, hipStream_t stream) {
+  if constexpr (MT == 1 && ONCE)
+    if (G) return launch_slices<SLICES, MT, NT, D, ONCE, MIN_WAVES, GLU, true>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream);
+  if (G) return APC_ERR_UNSUPPORTED;
+#define SL_GO(SL_) return launch_slices<SL_, MT, NT, D, ONCE, MIN_WAVES, GLU, false>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
   if constexpr (MT * NT >= 4 && MT * NT <= 6) {         // (smaller tiles share their units with eight too; larger ones are not chosen)
     if (K <= 2 * STAGE) SL_GO(2);
     if (K <= 4 * STAGE) SL_GO(4);
@@ -382,13 +487,15 @@ APC_EXPORT int apc_gemm_f32_tile(int M, int N, int K) {
   return 16 * t.mt * 1000 + 16 * t.nt;
 }
 
-int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
-             hipStream_t stream) {
-#define GO(...) return launch<__VA_ARGS__>(A, lda, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
+// Few rows: two stages of loads ahead, not four.  4 rows x 2,048 outputs x K 2,048 7.1 -> 6.7 us, K 8,192 21.5 -> 18.8, 128,256
+// outputs 155 -> 150: the straight code of a stage count's every case is a third as long, and a launch finds it cold.
+static int product(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C,
+                   int c_dtype, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
+#define GO(...) return launch<__VA_ARGS__>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
   // (one row tile: W is read once, past the caches)
   switch (tile_of(M, N, K)) {
     case 0:
-      if (M <= 16) GO(1, 1, 4, true, 4);
+      if (M <= 16) GO(1, 1, 2, true, 4);
       GO(1, 1, 4, false, 4);
     case 1:
       if (M <= 32) GO(2, 1, 2, true, 2);
@@ -399,6 +506,38 @@ int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dt
     default: GO(4, 4, 1, false, 2);
   }
 #undef GO
+}
+
+int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dtype, int ldc, int M, int N, int K, int mode,
+             hipStream_t stream) {
+  return product(A, lda, nullptr, 0.f, nullptr, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream);
+}
+
+// C[M,N] = rmsnorm(A; G, eps) . W^T.  Up to 16 rows in one launch: 4 rows x 3,072 outputs x K 2,048 6.9 us without the norm, 7.6
+// with it, and the norm's own launch was 4.7; 6,144 x K 4,096 19.8 and 21.0.  More rows need room for M rows of K and their
+// scales: apc_gemm_norm_f32_workspace(M, K) floats.  A row's outputs do not depend on the rows beside it, nor on M.
+static bool norm_in_product(int M, int K) { return M <= 16 && K <= NORM_K; }
+APC_EXPORT long long apc_gemm_norm_f32_workspace(int M, int K) { return norm_in_product(M, K) ? 0 : (long long)M * (K + 1); }
+APC_EXPORT int apc_gemm_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int K) {
+  return gemm_f32_takes(A, lda, W, ldw, K) && G && ((uintptr_t)G & 15u) == 0;
+}
+static int norm_rows(const float* A, int lda, const float* G, float eps, float* ws, int M, int K, hipStream_t stream) {
+  if (!ws || ((uintptr_t)ws & 15u)) return APC_ERR_BAD_ARG;
+  hipLaunchKernelGGL(norm_rows_f32_kernel, dim3(ceil_div(M, 2)), dim3(64), 0, stream, A, lda, G, eps, ws, ws + (size_t)M * K, M, K);
+  APC_LAUNCH_CHECK();
+  return 0;
+}
+
+APC_EXPORT int apc_gemm_norm_f32(const void* A, int lda, const void* G, float eps, const void* W, int ldw, void* C, int ldc, int M,
+                                 int N, int K, void* ws, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || lda < K || ldw < K || ldc < N) return APC_ERR_BAD_ARG;
+  if (!apc_gemm_norm_f32_takes(A, lda, G, W, ldw, K)) return APC_ERR_UNSUPPORTED;
+  const float *a = (const float*)A, *g = (const float*)G, *w = (const float*)W;
+  if (norm_in_product(M, K)) return product(a, lda, g, eps, nullptr, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
+  float* h = (float*)ws;
+  if (const int rc = norm_rows(a, lda, g, eps, h, M, K, stream)) return rc;
+  return product(h, K, nullptr, 0.f, h + (size_t)M * K, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
 }
 
 // out[M,F] = silu(A . Wg^T) * (A . Wu^T), W = [Wg; Wu] of 2 F rows: the same sums as the product of 2 F outputs, without
@@ -421,12 +560,14 @@ APC_EXPORT int apc_swiglu_f32_tile(int M, int F, int K) {
   return 16 * t.mt * 1000 + 8 * t.nt;
 }
 
-APC_EXPORT int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, void* out, int ldo, int M, int F, int K,
-                              hipStream_t stream) {
+static int swiglu(const void* A, int lda, const void* G, float eps, const float* R, const void* W, int ldw, void* out, int ldo,
+                  int M, int F, int K, hipStream_t stream) {
   if (M <= 0 || F <= 0) return 0;
   if (K <= 0 || lda < K || ldw < K || ldo < F) return APC_ERR_BAD_ARG;
   if (!apc_swiglu_f32_takes(A, lda, W, ldw, F, K)) return APC_ERR_UNSUPPORTED;
-#define GO(...) return launch<__VA_ARGS__, true>((const float*)A, lda, (const float*)W, ldw, out, APC_F32, ldo, M, F, K, 0, stream)
+#define GO(...)                                                                                                             \
+  return launch<__VA_ARGS__, true>((const float*)A, lda, (const float*)G, eps, R, (const float*)W, ldw, out, APC_F32, ldo, M, F, K, \
+                                   0, stream)
   switch (glu_tile_of(M, F, K)) {
     case 0:
       if (M <= 16) GO(1, 2, 2, true, 4);
@@ -437,4 +578,26 @@ APC_EXPORT int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, vo
     default: GO(4, 4, 1, false, 2);
   }
 #undef GO
+}
+
+APC_EXPORT int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, void* out, int ldo, int M, int F, int K,
+                              hipStream_t stream) {
+  return swiglu(A, lda, nullptr, 0.f, nullptr, W, ldw, out, ldo, M, F, K, stream);
+}
+
+// The same of the normalised rows, out of the rows in front of the norm (4 rows x 8,192 outputs x K 2,048: 22.4 us without the
+// norm, 23.3 with it); the workspace is apc_gemm_norm_f32's.
+APC_EXPORT int apc_swiglu_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int F, int K) {
+  return apc_swiglu_f32_takes(A, lda, W, ldw, F, K) && G && ((uintptr_t)G & 15u) == 0;
+}
+
+APC_EXPORT int apc_swiglu_norm_f32(const void* A, int lda, const void* G, float eps, const void* W, int ldw, void* out, int ldo,
+                                   int M, int F, int K, void* ws, hipStream_t stream) {
+  if (M <= 0 || F <= 0) return 0;
+  if (K <= 0 || lda < K || ldw < K || ldo < F) return APC_ERR_BAD_ARG;
+  if (!apc_swiglu_norm_f32_takes(A, lda, G, W, ldw, F, K)) return APC_ERR_UNSUPPORTED;
+  if (norm_in_product(M, K)) return swiglu(A, lda, G, eps, nullptr, W, ldw, out, ldo, M, F, K, stream);
+  float* h = (float*)ws;
+  if (const int rc = norm_rows((const float*)A, lda, (const float*)G, eps, h, M, K, stream)) return rc;
+  return swiglu(h, K, nullptr, 0.f, h + (size_t)M * K, W, ldw, out, ldo, M, F, K, stream);
 }

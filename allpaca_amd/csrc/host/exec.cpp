@@ -342,7 +342,18 @@ int normed_tensor(Program& P, Normed& n) {
   return 0;
 }
 
+bool folds_f32(const Program& P, const Normed& n, const ApcMatrix& w, const Buf& out) {
+  return !n.pre && !n.have && P.run_dtype == APC_DT_F32 && !w.packed && w.dtype == APC_DT_F32 && out.dtype == APC_DT_F32 &&
+         w.K == P.x.cols && out.rows == P.x.rows;
+}
+
 int normed_linear(Program& P, Normed& n, const ApcMatrix& w, const Buf& out) {
+  if (folds_f32(P, n, w, out) && out.cols == w.N && apc_gemm_norm_f32_takes(P.x.p, P.x.ld, n.g, w.data, w.ld, w.K)) {
+    float* ws = P.floats((size_t)apc_gemm_norm_f32_workspace(P.x.rows, w.K));
+    LAUNCH(P, "gemm_norm_f32",
+           apc_gemm_norm_f32(P.x.p, P.x.ld, n.g, n.eps, w.data, w.ld, out.p, out.ld, P.x.rows, w.N, w.K, ws, P.stream));
+    return 0;
+  }
   if (n.pre && !n.have) {
     const int rc = linear_pre(P, *n.pre, w, out);
     if (rc) return rc < 0 ? rc : 0;
@@ -501,7 +512,7 @@ int run_layer(Program& P, const ApcLayer& L, const ApcPlanEntry& E, const Emit& 
   mid.eps = L.norm2_eps;
   Buf qkv = P.rows(T, (L.H + 2 * L.Hk) * L.d, P.run_dtype);
   bool fused = false;
-  if (E.writes && L.rot == L.d && L.rot > 0) {
+  if (E.writes && L.rot == L.d && L.rot > 0 && L.w_qkv.packed && !P.tun.force_plain) {
     int rc;
     if (h1.pre) {
       rc = qkv_rope(P, h1.pre->raw, h1.pre, L, qkv, E);
@@ -539,6 +550,14 @@ int run_layer(Program& P, const ApcLayer& L, const ApcPlanEntry& E, const Emit& 
     rc = swiglu_pre(P, *h2.pre, L, act);
     if (rc < 0) return rc;
     done = rc == 1;
+  }
+  if (!done && folds_f32(P, h2, L.w_gate, act) && L.w_gate.N == 2 * L.F &&
+      apc_swiglu_norm_f32_takes(P.x.p, P.x.ld, h2.g, L.w_gate.data, L.w_gate.ld, L.F, L.w_gate.K)) {
+    float* ws = P.floats((size_t)apc_gemm_norm_f32_workspace(T, L.w_gate.K));
+    LAUNCH(P, "swiglu_norm_f32",
+           apc_swiglu_norm_f32(P.x.p, P.x.ld, h2.g, h2.eps, L.w_gate.data, L.w_gate.ld, act.p, act.ld, T, L.F, L.w_gate.K, ws,
+                               P.stream));
+    done = true;
   }
   if (!done) {
     rc = normed_tensor(P, h2);

@@ -20,6 +20,13 @@ int apc_rope_kv_write(void* qkv, int dtype, int ld, int q_off, int k_off, int v_
 int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int ldw, int F, int K);
 int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, void* out, int ldo, int M, int F, int K,
                    hipStream_t stream);
+long long apc_gemm_norm_f32_workspace(int M, int K);
+int apc_gemm_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int K);
+int apc_gemm_norm_f32(const void* A, int lda, const void* G, float eps, const void* W, int ldw, void* C, int ldc, int M, int N,
+                      int K, void* ws, hipStream_t stream);
+int apc_swiglu_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int F, int K);
+int apc_swiglu_norm_f32(const void* A, int lda, const void* G, float eps, const void* W, int ldw, void* out, int ldo, int M,
+                        int F, int K, void* ws, hipStream_t stream);
 int apc_gemm_plain(const void* A, int a_dtype, int lda, const void* W, int w_dtype, int ldw, void* C, int c_dtype,
                    int ldc, int M, int N, int K, int mode, hipStream_t stream);
 int apc_paged_attention_plain(const void* q, int q_dtype, int ldq, int q_off, void* out, int out_dtype, int ldo,

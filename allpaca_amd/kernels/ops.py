@@ -322,6 +322,47 @@ def _swiglu_f32(h: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     return True
 
 
+def _norm_room(L, h: torch.Tensor) -> torch.Tensor:
+    return torch.empty(max(1, L.apc_gemm_norm_f32_workspace(h.shape[0], h.shape[1])), dtype=torch.float32, device=h.device)
+
+
+def _float32_gain(x: torch.Tensor, g: torch.Tensor) -> bool:
+    return g.dtype == torch.float32 and g.is_contiguous() and g.shape == (x.shape[1],)
+
+
+def linear_normed(x: torch.Tensor, g: torch.Tensor, eps: float, w, out: torch.Tensor) -> bool:
+    """out = rmsnorm(x; g, eps) . w^T of float32 operands without the norm's own kernel (few rows) or with one that leaves
+    the rows' scales to the product; False (nothing done) for operands it does not take."""
+    if isinstance(w, PackedWeight) or not (x.dtype == w.dtype == out.dtype == torch.float32 and _float32_gain(x, g)):
+        return False
+    _gpu(x, g, w, out)
+    ldx, ldw, ldo = _rows(x, "norm product x"), _rows(w, "norm product w"), _rows(out, "norm product out")
+    M, K = x.shape
+    N = w.shape[0]
+    L = _lib.load("plain")
+    if w.shape[1] != K or out.shape != (M, N) or not L.apc_gemm_norm_f32_takes(x.data_ptr(), ldx, g.data_ptr(), w.data_ptr(), ldw, K):
+        return False
+    _lib.check(L.apc_gemm_norm_f32(x.data_ptr(), ldx, g.data_ptr(), float(eps), w.data_ptr(), ldw, out.data_ptr(), ldo, M, N, K,
+                                   _norm_room(L, x).data_ptr(), _stream()), "gemm_norm_f32")
+    return True
+
+
+def swiglu_normed(x: torch.Tensor, g: torch.Tensor, eps: float, w, out: torch.Tensor) -> bool:
+    """`swiglu` of rmsnorm(x; g, eps), as `linear_normed` (w: [Wg; Wu] in float32)."""
+    if isinstance(w, tuple) or not (x.dtype == w.dtype == out.dtype == torch.float32 and _float32_gain(x, g)):
+        return False
+    _gpu(x, g, w, out)
+    ldx, ldw, ldo = _rows(x, "swiglu x"), _rows(w, "swiglu w"), _rows(out, "swiglu out")
+    T, F = out.shape
+    K = x.shape[1]
+    L = _lib.load("plain")
+    if x.shape[0] != T or w.shape != (2 * F, K) or not L.apc_swiglu_norm_f32_takes(x.data_ptr(), ldx, g.data_ptr(), w.data_ptr(), ldw, F, K):
+        return False
+    _lib.check(L.apc_swiglu_norm_f32(x.data_ptr(), ldx, g.data_ptr(), float(eps), w.data_ptr(), ldw, out.data_ptr(), ldo, T, F, K,
+                                     _norm_room(L, x).data_ptr(), _stream()), "swiglu_norm_f32")
+    return True
+
+
 def linear_pre(raw: torch.Tensor, ss: torch.Tensor, eps: float, w, out: torch.Tensor) -> bool:
     """The product of a normalised row from what `linear(..., emit=...)` left; False if there is no kernel for
     these sizes (nothing is done then)."""
@@ -331,13 +372,18 @@ def linear_pre(raw: torch.Tensor, ss: torch.Tensor, eps: float, w, out: torch.Te
     return False
 
 
+def qkv_rope_possible(w) -> bool:
+    """Whether `qkv_rope_write` has kernels for this weight at all."""
+    return isinstance(w, PackedWeight) and not FORCE_PLAIN
+
+
 def qkv_rope_write(a: torch.Tensor, pre, w, q_out: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int,
                    cos_sin: torch.Tensor, positions: torch.Tensor, row_seg: torch.Tensor, block_table: torch.Tensor,
                    cache: torch.Tensor, page_tokens: int) -> bool:
     """The product for q, k and v, the rotation of whole q and k heads and the write of k and v into the pages in
     one kernel (few rows; `pre` = (ss, eps) if `a` is a row that `linear(..., emit=...)` left, else None).  False if
     there is no such kernel for these sizes (nothing is done then)."""
-    if isinstance(w, PackedWeight) and not FORCE_PLAIN:
+    if qkv_rope_possible(w):
         from . import tuned
         return tuned.qkv_rope_bf16(a, pre, w, q_out, n_heads, n_kv_heads, head_dim, cos_sin, positions, row_seg,
                                    block_table, cache, page_tokens)

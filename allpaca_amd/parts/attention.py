@@ -64,7 +64,7 @@ class Attention(Mixer):
         rot, table = fused if fused is not None else (0, None)
         kv = cache.kv if cache.writes else None
         # few rows, whole heads rotated, an own cache: one kernel gives q, k, v, rotates and fills the pages
-        if (kv is not None and rot == self.d and h.product(
+        if (kv is not None and rot == self.d and ops.qkv_rope_possible(self.w_qkv) and h.product(
                 lambda a, pre: ops.qkv_rope_write(a, pre, self.w_qkv, qkv, self.H, self.Hk, self.d, table,
                                                   step.positions, step.row_seg, cache.block_table, kv,
                                                   cache.page_tokens))):

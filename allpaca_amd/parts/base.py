@@ -215,8 +215,13 @@ class NormedInput:
     def linear(self, w, out: torch.Tensor) -> None:
         from ..kernels import ops
         p = self.pre
+        if p is None and self._folds() and ops.linear_normed(self.x, *self.norm.rms_params(), w, out):
+            return
         if p is None or self._h is not None or not ops.linear_pre(p.raw, p.ss, p.eps, w, out):
             ops.linear(self.tensor(), w, out)
+
+    def _folds(self) -> bool:      # a float32 norm that nobody has asked for by itself: its product may do it
+        return self._h is None and self.dtype == torch.float32 and self.norm.rms_params() is not None
 
     def product(self, op) -> bool:
         """For a part with a fused first product of its own: `op(a, pre)` is called with the row that the product
@@ -230,6 +235,8 @@ class NormedInput:
     def swiglu(self, w_gate_up, out: torch.Tensor) -> None:
         from ..kernels import ops
         p = self.pre
+        if p is None and self._folds() and ops.swiglu_normed(self.x, *self.norm.rms_params(), w_gate_up, out):
+            return
         if p is None or self._h is not None or not ops.swiglu_pre(p.raw, p.ss, p.eps, w_gate_up, out):
             ops.swiglu(self.tensor(), w_gate_up, out)
 

@@ -151,3 +151,36 @@ def test_attention_against_64_bits_and_rows_alone(H, Hk, d, P, window):
         most = float((torch.einsum("hd,thd->ht", qr.abs(), k.abs()) / math.sqrt(d)).max())
         bound = (2 * (d + 2) * most + 2 * (p + 1 - first + 16) + 16) * U * float(v.abs().max())
         assert float((out[r].double().view(H, d) - want).abs().max()) <= bound
+
+
+# the norm in the product (up to 16 rows of up to 4,096) and in front of it: both against float64, a row of a batch against
+# the row alone bit for bit across that line, rows with more elements than they are used with, several tiles a block
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16, 4), (4, 70, 36), (16, 515, 256), (17, 130, 260), (8, 3072, 2048), (33, 100, 4096),
+                                   (5, 48, 4100), (331, 2045, 516), (700, 4099, 256), (20, 8200, 388)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_product_of_normalised_rows(M, N, K, gated):
+    o = ops()
+    x, g, w = gen(M, K + 4, seed=1)[:, :K] * 3.0, 1.0 + 0.1 * gen(K, seed=2), gen(N * (2 if gated else 1), K, seed=3) * 2 * K ** -0.5
+    x[M // 2] *= 1e-3
+    eps = 1e-5
+    fn = o.swiglu_normed if gated else o.linear_normed
+    out = torch.full((M, N + 4), 7.0, device=DEV)
+    assert fn(x, g, eps, w, out[:, :N])
+    assert (out[:, N:] == 7.0).all()
+    h = x.double() * torch.rsqrt(x.double().square().mean(1, keepdim=True) + eps) * g.double()
+    y = h @ w.double().T
+    # beside the product's own bound: the rounded x * g, the sum of squares, the root and the last product
+    bound = product_bound(h, w) + (K / 16 + 16) * U * (h.abs() @ w.double().abs().T)
+    if gated:
+        s, u = y[:, :N], y[:, N:]
+        want = torch.nn.functional.silu(s) * u
+        # silu' is at most 1.1; its own rounding and that of the product
+        bound = 1.1 * bound[:, :N] * u.abs() + bound[:, N:] * torch.nn.functional.silu(s).abs() + 1.1 * bound[:, :N] * bound[:, N:] + 8 * U * want.abs()
+    else:
+        want = y
+    assert ((out[:, :N].double() - want).abs() <= bound).all()
+    for r in sorted({0, M // 2, M - 1}):
+        alone = torch.empty(1, N, device=DEV)
+        assert fn(x[r:r + 1], g, eps, w, alone)
+        assert torch.equal(alone[0], out[r, :N])
