@@ -515,9 +515,9 @@ int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dt
 
 // C[M,N] = rmsnorm(A; G, eps) . W^T.  Up to 16 rows in one launch: 4 rows x 3,072 outputs x K 2,048 6.9 us without the norm, 7.6
 // with it, and the norm's own launch was 4.7; 6,144 x K 4,096 19.8 and 21.0.  More rows need room for M rows of K and their
-// scales: apc_gemm_norm_f32_workspace(M, K) floats.  A row's outputs do not depend on the rows beside it, nor on M.
+// scales: apc_gemm_norm_f32_kib(M, K) KiB.  A row's outputs do not depend on the rows beside it, nor on M.
 static bool norm_in_product(int M, int K) { return M <= 16 && K <= NORM_K; }
-APC_EXPORT long long apc_gemm_norm_f32_workspace(int M, int K) { return norm_in_product(M, K) ? 0 : (long long)M * (K + 1); }
+APC_EXPORT int apc_gemm_norm_f32_kib(int M, int K) { return norm_in_product(M, K) ? 0 : (int)(((long long)M * (K + 1) * 4 + 1023) / 1024); }
 APC_EXPORT int apc_gemm_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int K) {
   return gemm_f32_takes(A, lda, W, ldw, K) && G && ((uintptr_t)G & 15u) == 0;
 }

@@ -349,7 +349,7 @@ bool folds_f32(const Program& P, const Normed& n, const ApcMatrix& w, const Buf&
 
 int normed_linear(Program& P, Normed& n, const ApcMatrix& w, const Buf& out) {
   if (folds_f32(P, n, w, out) && out.cols == w.N && apc_gemm_norm_f32_takes(P.x.p, P.x.ld, n.g, w.data, w.ld, w.K)) {
-    float* ws = P.floats((size_t)apc_gemm_norm_f32_workspace(P.x.rows, w.K));
+    float* ws = P.floats((size_t)apc_gemm_norm_f32_kib(P.x.rows, w.K) * 256);
     LAUNCH(P, "gemm_norm_f32",
            apc_gemm_norm_f32(P.x.p, P.x.ld, n.g, n.eps, w.data, w.ld, out.p, out.ld, P.x.rows, w.N, w.K, ws, P.stream));
     return 0;
@@ -553,7 +553,7 @@ int run_layer(Program& P, const ApcLayer& L, const ApcPlanEntry& E, const Emit& 
   }
   if (!done && folds_f32(P, h2, L.w_gate, act) && L.w_gate.N == 2 * L.F &&
       apc_swiglu_norm_f32_takes(P.x.p, P.x.ld, h2.g, L.w_gate.data, L.w_gate.ld, L.F, L.w_gate.K)) {
-    float* ws = P.floats((size_t)apc_gemm_norm_f32_workspace(T, L.w_gate.K));
+    float* ws = P.floats((size_t)apc_gemm_norm_f32_kib(T, L.w_gate.K) * 256);
     LAUNCH(P, "swiglu_norm_f32",
            apc_swiglu_norm_f32(P.x.p, P.x.ld, h2.g, h2.eps, L.w_gate.data, L.w_gate.ld, act.p, act.ld, T, L.F, L.w_gate.K, ws,
                                P.stream));

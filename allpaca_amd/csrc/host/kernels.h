@@ -20,7 +20,7 @@ int apc_rope_kv_write(void* qkv, int dtype, int ld, int q_off, int k_off, int v_
 int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int ldw, int F, int K);
 int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, void* out, int ldo, int M, int F, int K,
                    hipStream_t stream);
-long long apc_gemm_norm_f32_workspace(int M, int K);
+int apc_gemm_norm_f32_kib(int M, int K);
 int apc_gemm_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int K);
 int apc_gemm_norm_f32(const void* A, int lda, const void* G, float eps, const void* W, int ldw, void* C, int ldc, int M, int N,
                       int K, void* ws, hipStream_t stream);

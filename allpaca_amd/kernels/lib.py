@@ -41,7 +41,7 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
         "apc_gemm_norm_f32": [P, I, P, F, P, I, P, I, I, I, I, P, P],
         "apc_swiglu_norm_f32_takes": [P, I, P, P, I, I, I],
         "apc_swiglu_norm_f32": [P, I, P, F, P, I, P, I, I, I, I, P, P],
-        "apc_gemm_norm_f32_workspace": [I, I],
+        "apc_gemm_norm_f32_kib": [I, I],
         "apc_paged_attention_plain": [P, I, I, I, P, I, I, I, I, I, I, P, I, I, P, I, P, P, I, F, P],
         "apc_conv_heads": [P, I, I, I, I, I, I, I, I, I, I, I, P, P, I, P, I, P, P, P, P, P, I, F, I, P, P, I, F, I, P, I, I, P, I, P, I, I, P],
         "apc_conv_state": [P, I, I, P, I, P, I, I, P, P, P, P],
@@ -145,7 +145,7 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
 # The host library's entry points take structures (declared in `kernels/host.py`, which fills this in) and some
 # return something other than an int.
 SIGNATURES["host"] = {}
-RESTYPES: Dict[str, object] = {"apc_gemm_norm_f32_workspace": ctypes.c_longlong}
+RESTYPES: Dict[str, object] = {}
 
 _loaded: Dict[str, "Library"] = {}
 
@@ -181,7 +181,7 @@ NOT_KERNELS = {"apc_delta_rule_bf16_takes", "apc_delta_rule_fact_size", "apc_del
                "apc_gated_recurrence_bf16_takes", "apc_latent_attention_takes", "apc_latent_rows_bf16_takes", "apc_selective_scan_bf16_takes", "apc_attention_masked_takes", "apc_rotary_pages_bf16_takes", "apc_routed_bf16_takes", "apc_routed_max_tiles", "apc_linear_attention_bf16_takes", "apc_conv_heads_bf16_takes", "apc_attention_decode_whole_fits", "apc_attention_decode_last_fits", "apc_attention_decode_even_workspace", "apc_attention_decode_even_region", "apc_attention_prefill_tile_rows",
                "apc_attention_prefill_wide_takes",
                "apc_gemm_direct_k_split", "apc_gemm_rows_takes", "apc_gemm_rows_qkv_takes", "apc_gemm_rows_emit_takes", "apc_gemm_direct_emit_parts", "apc_sample_rows_scratch_kib", "apc_swiglu_f32_takes", "apc_gemm_f32_tile",
-               "apc_swiglu_f32_tile", "apc_gemm_norm_f32_takes", "apc_swiglu_norm_f32_takes", "apc_gemm_norm_f32_workspace"}
+               "apc_swiglu_f32_tile", "apc_gemm_norm_f32_takes", "apc_swiglu_norm_f32_takes", "apc_gemm_norm_f32_kib"}
 
 
 class timing:

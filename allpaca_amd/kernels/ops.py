@@ -323,7 +323,7 @@ def _swiglu_f32(h: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
 
 
 def _norm_room(L, h: torch.Tensor) -> torch.Tensor:
-    return torch.empty(max(1, L.apc_gemm_norm_f32_workspace(h.shape[0], h.shape[1])), dtype=torch.float32, device=h.device)
+    return torch.empty(max(1, L.apc_gemm_norm_f32_kib(h.shape[0], h.shape[1]) * 256), dtype=torch.float32, device=h.device)
 
 
 def _float32_gain(x: torch.Tensor, g: torch.Tensor) -> bool:
