@@ -16,6 +16,7 @@
 #include "common.h"
 #include "no_alloc.h"
 #include <math.h>
+#include <string.h>
 #include <mutex>
 
 constexpr int SNT = 256;
@@ -289,7 +290,7 @@ APC_EXPORT int apc_argmax_rows_no_alloc(const float* logits, int ldl, int n_rows
 }
 
 // What a block's threads share while they choose one row's token
-struct SampleShared {
+struct alignas(16) SampleShared {
   float fsm[SNT / WAVE];
   uint32_t usm[SNT / WAVE];
   float bv[SNT / WAVE];
@@ -546,6 +547,8 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
 // reads 256 + 32 numbers of it, not all.
 // Few survivors (up to SMALL_MAX after top-k) are gathered and go through the reference's sequential arithmetic as
 // above.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 namespace {
 
 typedef unsigned long long u64;
@@ -595,6 +598,11 @@ struct SampleShape {
   int id_digits;           // ... by id alone
 };
 
+// The rows' options: on the device, or, of up to BY_VALUE rows, with the launch (no copy to the device in front of it).
+constexpr int BY_VALUE = 64;
+struct RowOptions { const float *temperature, *top_p, *uniform; const int* top_k; };
+struct RowValues { float temperature[BY_VALUE], top_p[BY_VALUE], uniform[BY_VALUE]; int top_k[BY_VALUE]; };
+
 struct SampleSpace {
   u64* fine;               // [ROTA][row][FINE]
   u64* coarse;             // [ROTA][row][COARSE]
@@ -606,6 +614,7 @@ struct SampleSpace {
   RowState* state;         // [launch + 1][row]
   uint32_t* few_key;       // [row][SMALL_MAX]
   int* few_id;
+  RowValues* options;      // where options that came with the first launch stand for the others
   size_t bytes;
 };
 
@@ -626,6 +635,7 @@ SampleSpace carve(void* base, int R) {
   s.state = (RowState*)take((N_SELECTS * MAX_DIGITS + 1) * r * sizeof(RowState));
   s.few_key = (uint32_t*)take(r * SMALL_MAX * 4);
   s.few_id = (int*)take(r * SMALL_MAX * 4);
+  s.options = (RowValues*)take(sizeof(RowValues));
   s.bytes = at;
   return s;
 }
@@ -774,8 +784,10 @@ __device__ __forceinline__ void settle(RowState& S, const SampleShape& sz, int s
   if (stage == ST_TOPK) S.n = (uint32_t)S.target;
 }
 
-__global__ __launch_bounds__(PNT) void sample_max_kernel(const float* __restrict__ logits, SampleShape sz,
-                                                         SampleSpace sp) {
+// RowValues: the rows' options came with this launch and are put where the later ones look for them.
+struct NoValues {};
+template <typename Values>
+__global__ __launch_bounds__(PNT) void sample_max_kernel(const float* __restrict__ logits, SampleShape sz, Values values, SampleSpace sp) {
   __shared__ float bv[PNT / WAVE], fv[PNT / WAVE];
   __shared__ int bi[PNT / WAVE];
   __shared__ uint32_t nv[PNT / WAVE];
@@ -784,7 +796,15 @@ __global__ __launch_bounds__(PNT) void sample_max_kernel(const float* __restrict
   for (int j = piece * PNT + threadIdx.x; j < FINE; j += sz.pieces * PNT) sp.fine[(size_t)row * FINE + j] = 0;
   if (piece == 0) {
     sp.coarse[(size_t)row * COARSE + threadIdx.x] = 0;
-    if (threadIdx.x == 0) sp.few_count[row] = 0u;
+    if (threadIdx.x == 0) {
+      sp.few_count[row] = 0u;
+      if constexpr (!__is_same(Values, NoValues)) {
+        sp.options->temperature[row] = values.temperature[row];
+        sp.options->top_p[row] = values.top_p[row];
+        sp.options->uniform[row] = values.uniform[row];
+        sp.options->top_k[row] = values.top_k[row];
+      }
+    }
   }
   const float* lg = logits + (size_t)row * sz.ldl;
   const int i0 = piece * sz.chunk, i1 = min(sz.V, i0 + sz.chunk);
@@ -962,7 +982,8 @@ __global__ __launch_bounds__(SNT) void sample_end_kernel(const float* __restrict
                                                          const float* __restrict__ temperature,
                                                          const int* __restrict__ top_k, const float* __restrict__ top_p,
                                                          const float* __restrict__ uniform, SampleSpace sp, int q,
-                                                         int last_stage, int last_digit, int* __restrict__ out) {
+                                                         int last_stage, int last_digit, int* __restrict__ out,
+                                                         int* __restrict__ out_host) {
   __shared__ EndShared sh;
   const int row = blockIdx.x, R = sz.R;
   const float tp = top_p[row], r = uniform[row];
@@ -971,9 +992,16 @@ __global__ __launch_bounds__(SNT) void sample_end_kernel(const float* __restrict
   settle<SNT>(S, sz, last_stage, last_digit, sp.fine + prev * FINE, sp.coarse + prev * COARSE,
               last_stage == ST_TOPP ? tp : r, sh.settle);
   if (S.phase == PH_DONE) {
-    if (threadIdx.x == 0) out[row] = S.result;
+    if (threadIdx.x == 0) {
+      out[row] = S.result;
+      if (out_host) out_host[row] = S.result;
+    }
     return;
   }
+  auto to_host = [&]() {                                // (one thread of the block has written out[row])
+    __syncthreads();
+    if (out_host && threadIdx.x == 0) out_host[row] = *(volatile int*)(out + row);
+  };
   __syncthreads();
   if (S.phase == PH_FEW) {
     const int cnt = (int)min(sp.few_count[row], (uint32_t)SMALL_MAX);
@@ -984,10 +1012,12 @@ __global__ __launch_bounds__(SNT) void sample_end_kernel(const float* __restrict
     __syncthreads();
     const bool use_top_p = tp >= 0.0f && tp < 1.0f && S.n > 1u;
     sample_few(sh.one, cnt, use_top_p, tp, r, out + row);
+    to_host();
     return;
   }
   // a row whose cut or draw the launches did not cover (the caller's word on its rows was wrong), or is not through
   sample_row_one_block(sh.one, logits + (size_t)row * sz.ldl, sz.V, temperature[row], top_k[row], tp, r, out + row);
+  to_host();
 }
 
 // ---- Rows that all keep at most SMALL_MAX candidates (0 < top-k <= 1,024), in two launches ----
@@ -996,9 +1026,9 @@ __global__ __launch_bounds__(SNT) void sample_end_kernel(const float* __restrict
 // reference's sequential arithmetic.  A threshold is found by radix descent over the same 64-bit sort key, 11
 // bits a pass, with the histogram in LDS.  What bounds it is latency: each launch is a handful of passes over values that
 // are in L2 after the first, each with two or three barriers; the descents above make five launches of it, each of which
-// begins with where the one before it left off.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 10 + 20 us (the descents:
-// 73 us in seven launches).  Of the 20 us, by clock readings inside the kernel: the pieces' results 2, their candidates 4,
-// the selection 5, sorting and exponentials 3, the sums in order 5.
+// begins with where the one before it left off.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 10 + 16 us (the descents:
+// 73 us in seven launches).  Of the 16 us, by clock readings inside the kernel: the pieces' results 2, their candidates 1.6,
+// the selection 4.3, sorting and exponentials 2, the sums in order 3 (7 when every value went from lane to lane).
 constexpr int FEW_SPARE = 128, FEW_STRIDE = SMALL_MAX + FEW_SPARE;
 constexpr int FEW_BITS = 11, FEW_BINS = 1 << FEW_BITS;
 
@@ -1096,14 +1126,13 @@ __device__ __forceinline__ void first_max(float& best, int& best_i, float ov, in
   if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
 }
 
-__global__ __launch_bounds__(PNT) void sample_few_pieces_kernel(const float* __restrict__ logits, SampleShape sz,
-                                                                const float* __restrict__ temperature,
-                                                                const int* __restrict__ top_k, FewSpace sp) {
+template <typename Options>
+__global__ __launch_bounds__(PNT) void sample_few_pieces_kernel(const float* __restrict__ logits, SampleShape sz, Options opt, FewSpace sp) {
   __shared__ FewShared sh;
   const int row = blockIdx.y, piece = blockIdx.x;
   const float* lg = logits + (size_t)row * sz.ldl;
-  const float t = fmaxf(temperature[row], 1e-5f);
-  const int tk = top_k[row];
+  const float temperature = opt.temperature[row], t = fmaxf(temperature, 1e-5f);
+  const int tk = opt.top_k[row];
   const int i0 = piece * sz.chunk, i1 = min(sz.V, i0 + sz.chunk);
   float best = -INFINITY;
   int best_i = 0x7fffffff;
@@ -1135,7 +1164,7 @@ __global__ __launch_bounds__(PNT) void sample_few_pieces_kernel(const float* __r
     sp.piece_arg[at] = best_i;
     sp.piece_finite[at] = nfin;
   }
-  if (tk <= 0 || tk > SMALL_MAX || temperature[row] <= 1e-5f) return;   // the last launch knows what to do with the row
+  if (tk <= 0 || tk > SMALL_MAX || temperature <= 1e-5f) return;   // the last launch knows what to do with the row
   auto each = [&](auto f) {
     for_piece(lg, sz.vec, i0, i1, [&](int i, float x) {
       if (finite_f(x)) f(sort_key(key_of(x / t), i, sz.id_bits, 0));
@@ -1152,25 +1181,34 @@ __global__ __launch_bounds__(PNT) void sample_few_pieces_kernel(const float* __r
   if (threadIdx.x == 0) sp.piece_count[at] = sh.count;
 }
 
-// a[0] + a[1] + .. of the first n values, one after the other (the order of the reference's sums), by one wave; `each`
-// gets lane i's running sum for value i.  (Loops of a few instructions: a block alone pays for every line of code it
-// brings in, and written out 64 times these sums took longer than all else.)
-template <typename Each>
-__device__ __forceinline__ float sum_in_order(const float* a, int n, Each&& each) {
+// run[i] = start + sign (a[0] + .. + a[i]) for the first n values, one after the other (the order of the reference's sums), by
+// one wave.  All lanes add the same values, sixteen out of LDS at a time and the next sixteen asked for meanwhile; there is room
+// behind n in both up to a multiple of 16.  (A value handed round from lane to lane costs 110 cycles, and code written out 64
+// times more than the sums, since a block alone brings in every line of it.)
+__device__ __forceinline__ void sums_in_order(const float* a, float* run, int n, float start, float sign) {
   const int lane = threadIdx.x % WAVE;
-  float acc = 0.f;
-  for (int i0 = 0; i0 < n; i0 += WAVE) {
-    const float mine = i0 + lane < n ? a[i0 + lane] : 0.f;
-    float run = 0.f;
-    const int m = min(WAVE, n - i0);
+  const f32x4* a4 = reinterpret_cast<const f32x4*>(a);
+  float acc = start;
+  f32x4 next[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) next[q] = a4[q];
 #pragma unroll 1
-    for (int l = 0; l < m; ++l) {
-      acc += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), l));
-      run = lane == l ? acc : run;
+  for (int i = 0; i < n; i += 16) {
+    f32x4 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = next[q];
+    const int then = min(i + 16, (n - 1) / 16 * 16) / 4;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) next[q] = a4[then + q];
+    float mine = 0.f;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      acc += sign * v[u / 4][u % 4];                     // (what stands behind n is added behind all that counts)
+      mine = lane == u ? acc : mine;
     }
-    if (each(i0 + lane, run)) break;
+    if (lane < 16) run[i + lane] = mine;
   }
-  return acc;
+  __builtin_amdgcn_wave_barrier();
 }
 
 constexpr int FEW_HELD = 6144;           // candidates of a row that are held in LDS (all of them up to top-k 64)
@@ -1179,15 +1217,20 @@ struct FewEnd {
   SampleShared one;
   u64 held[FEW_HELD];
   uint32_t from[MAX_PIECES + 1];         // where the candidates of a piece begin
+  float sums[SMALL_MAX];                 // running sums of the weights
 };
 
-__global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __restrict__ logits, SampleShape sz,
-                                                             const float* __restrict__ temperature,
-                                                             const int* __restrict__ top_k, const float* __restrict__ top_p,
-                                                             const float* __restrict__ uniform, FewSpace sp, int* __restrict__ out) {
+// `out_host` (may be null): host memory that the ids are written to as well.
+template <typename Options>
+__global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __restrict__ logits, SampleShape sz, Options opt, FewSpace sp,
+                                                             int* __restrict__ out, int* __restrict__ out_host) {
   __shared__ FewEnd sh;
-  const int row = blockIdx.x, tk = top_k[row];
-  const float T = temperature[row], tp = top_p[row];
+  const int row = blockIdx.x, tk = opt.top_k[row];
+  const float T = opt.temperature[row], tp = opt.top_p[row], uniform = opt.uniform[row];
+  auto leave = [&](int id) {
+    out[row] = id;
+    if (out_host) out_host[row] = id;
+  };
   float best = -INFINITY;
   int best_i = 0x7fffffff;
   uint32_t n = 0;
@@ -1204,7 +1247,7 @@ __global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __rest
     n += __shfl_xor(n, o, WAVE);
   }
   if (n == 0u || T <= 1e-5f) {
-    if (threadIdx.x == 0) out[row] = n == 0u || best_i == 0x7fffffff ? 0 : best_i;
+    if (threadIdx.x == 0) leave(n == 0u || best_i == 0x7fffffff ? 0 : best_i);
     return;
   }
   const bool cut = tk > 0 && n > (uint32_t)tk;
@@ -1212,7 +1255,9 @@ __global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __rest
   const bool use_top_p = tp >= 0.0f && tp < 1.0f && keep > 1u;
   if (tk <= 0 || tk > SMALL_MAX || !(cut || use_top_p)) {
     // the caller's word on the row was wrong, or fewer candidates than top-k keeps and no top-p: drawn in id order
-    sample_row_one_block(sh.one, logits + (size_t)row * sz.ldl, sz.V, T, tk, tp, uniform[row], out + row);
+    sample_row_one_block(sh.one, logits + (size_t)row * sz.ldl, sz.V, T, tk, tp, uniform, out + row);
+    __syncthreads();
+    if (out_host && threadIdx.x == 0) out_host[row] = *(volatile int*)(out + row);
     return;
   }
   if (wave == 0) {
@@ -1287,53 +1332,125 @@ __global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __rest
   for (int i = threadIdx.x; i < cnt; i += SNT) e[i] = expf(value_of(sh.one.s_key2[i]) - vmax);
   __syncthreads();
   if (wave != 0) return;
-  auto all = [](int, float) { return false; };
-  int m = cnt;
-  if (use_top_p) {
-    const float sum = sum_in_order(e, m, all);
-    if (sum == 0.f || !finite_f(sum)) {
-      const int some = (int)ceilf(tp * (float)m);
-      m = some < 1 ? 1 : (some > m ? m : some);
-    } else {
-      float* share = reinterpret_cast<float*>(sh.one.s_id);
-      for (int i = lane; i < cnt; i += WAVE) share[i] = e[i] / sum;
-      __builtin_amdgcn_wave_barrier();
-      int first = m - 1;
-      sum_in_order(share, cnt, [&](int i, float run) {
-        const unsigned long long hit = __ballot(i < cnt && run >= tp);
-        if (hit) first = i - lane + __ffsll(hit) - 1;
-        return hit != 0;
-      });
-      m = first + 1;
-    }
-  }
-  const float sum = sum_in_order(e, m, all);
-  float* share = reinterpret_cast<float*>(sh.one.s_id);
-  for (int i = lane; i < m; i += WAVE) share[i] = sum == 0.f ? 1.0f / (float)m : e[i] / sum;
-  __builtin_amdgcn_wave_barrier();
-  // r - p[0] - p[1] - ..: the first candidate at which nothing is left
-  int pick = m - 1;
-  float left = uniform[row];
-  for (int i0 = 0; i0 < m; i0 += WAVE) {
-    const float mine = i0 + lane < m ? share[i0 + lane] : 0.f;
-    float run = 0.f;
-    const int here = min(WAVE, m - i0);
+  // The weights' sum, the shares' sum up to top-p, and the uniform number less the shares of the m that are left: three times
+  // the same code (over values that differ), which a block fetches once.  The sum of the first m is one of the first pass's.
+  float* run = reinterpret_cast<float*>(sh.one.s_id);
+  float* share = reinterpret_cast<float*>(sh.select.hist);             // (picked has been sorted)
+  int m = cnt, pick = 0;
+  float sum = 0.f;
 #pragma unroll 1
-    for (int l = 0; l < here; ++l) {
-      left -= __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), l));
-      run = lane == l ? left : run;
+  for (int pass = 0; pass < 3; ++pass) {
+    if (pass == 1) {
+      if (!use_top_p) continue;
+      if (sum == 0.f || !finite_f(sum)) {
+        const int some = (int)ceilf(tp * (float)m);
+        m = some < 1 ? 1 : (some > m ? m : some);
+        sum = sh.sums[m - 1];
+        continue;
+      }
     }
-    const unsigned long long hit = __ballot(i0 + lane < m && run <= 0.f);
-    if (hit) {
-      pick = i0 + __ffsll(hit) - 1;
-      break;
+    for (int i = lane; i < m; i += WAVE) share[i] = pass == 0 ? e[i] : pass == 2 && sum == 0.f ? 1.0f / (float)m : e[i] / sum;
+    __builtin_amdgcn_wave_barrier();
+    float* to = pass == 0 ? sh.sums : run;
+    sums_in_order(share, to, m, pass == 2 ? uniform : 0.f, pass == 2 ? -1.f : 1.f);
+    if (pass == 0) {
+      sum = sh.sums[m - 1];
+      continue;
     }
+    // the first candidate at which top-p is reached, or at which nothing is left
+    int first = m - 1;
+    for (int i0 = 0; i0 < m; i0 += WAVE) {
+      const int i = i0 + lane;
+      const unsigned long long hit = __ballot(i < m && (pass == 1 ? run[i] >= tp : run[i] <= 0.f));
+      if (hit) {
+        first = i0 + __ffsll(hit) - 1;
+        break;
+      }
+    }
+    if (pass == 1) m = first + 1, sum = sh.sums[first];
+    else pick = first;
   }
-  if (lane == 0) out[row] = sh.one.s_id2[pick];
+  if (lane == 0) leave(sh.one.s_id2[pick]);
 }
 
 std::mutex pass_attr_lock;
 bool pass_attr_set[64];
+
+SampleShape shape_of(const float* logits, int ldl, int n_rows, int V) {
+  SampleShape sz;
+  sz.ldl = ldl;
+  sz.V = V;
+  sz.R = n_rows;
+  cut_row(n_rows, V, &sz.pieces, &sz.chunk);
+  sz.vec = ((uintptr_t)logits % 16 == 0 && ldl % 4 == 0) ? 1 : 0;
+  sz.id_bits = 1;
+  while (sz.id_bits < 31 && (1u << sz.id_bits) < (unsigned)V) ++sz.id_bits;
+  sz.key_digits = ceil_div(32 + sz.id_bits, DIGIT_BITS);
+  sz.id_digits = ceil_div(sz.id_bits, DIGIT_BITS);
+  return sz;
+}
+
+template <typename Options>
+int launch_few(const float* logits, const SampleShape& sz, const Options& opt, void* scratch, int* out, int* out_host, hipStream_t stream) {
+  const FewSpace fs = carve_few(scratch, sz.R);
+  hipLaunchKernelGGL(sample_few_pieces_kernel<Options>, dim3(sz.pieces, sz.R), dim3(PNT), 0, stream, logits, sz, opt, fs);
+  APC_LAUNCH_CHECK();
+  hipLaunchKernelGGL(sample_few_end_kernel<Options>, dim3(sz.R), dim3(SNT), 0, stream, logits, sz, opt, fs, out, out_host);
+  APC_LAUNCH_CHECK();
+  return 0;
+}
+
+int allow_pass_lds(int dev) {
+  std::lock_guard<std::mutex> hold(pass_attr_lock);
+  if (!pass_attr_set[dev]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)sample_pass_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)sizeof(PassShared));
+    if (e != hipSuccess) return (int)e;
+    pass_attr_set[dev] = true;
+  }
+  return 0;
+}
+
+// `values`: the options, if they are on the host (then `opt` is not looked at)
+int launch_descents(const float* logits, const SampleShape& sz, RowOptions opt, const RowValues* values, void* scratch, int* out,
+                    int* out_host, int cuts, hipStream_t stream) {
+  const SampleSpace sp = carve(scratch, sz.R);
+  const dim3 grid(sz.pieces, sz.R);
+  if (values) {
+    opt = RowOptions{sp.options->temperature, sp.options->top_p, sp.options->uniform, sp.options->top_k};
+    hipLaunchKernelGGL(sample_max_kernel<RowValues>, grid, dim3(PNT), 0, stream, logits, sz, *values, sp);
+  } else {
+    hipLaunchKernelGGL(sample_max_kernel<NoValues>, grid, dim3(PNT), 0, stream, logits, sz, NoValues{}, sp);
+  }
+  APC_LAUNCH_CHECK();
+  int q = 0, prev_stage = -1, prev_digit = -1;
+  for (int stage = 0; stage < N_SELECTS; ++stage) {
+    int digits = sz.key_digits;
+    if (stage == ST_TOPK && !(cuts & 1)) continue;
+    if (stage == ST_TOPP && !(cuts & 2)) continue;
+    if (stage == ST_DRAW) digits = (cuts & 3) ? sz.key_digits : sz.id_digits;
+    for (int digit = 0; digit < digits; ++digit) {
+      hipLaunchKernelGGL(sample_pass_kernel, grid, dim3(PNT), sizeof(PassShared), stream, logits, sz, opt.temperature,
+                         opt.top_k, opt.top_p, opt.uniform, sp, q, stage, digit, prev_stage, prev_digit);
+      APC_LAUNCH_CHECK();
+      ++q;
+      prev_stage = stage;
+      prev_digit = digit;
+    }
+  }
+  hipLaunchKernelGGL(sample_end_kernel, dim3(sz.R), dim3(SNT), 0, stream, logits, sz, opt.temperature, opt.top_k, opt.top_p,
+                     opt.uniform, sp, q, prev_stage, prev_digit, out, out_host);
+  APC_LAUNCH_CHECK();
+  return 0;
+}
+
+uint64_t splitmix64(uint64_t x) {
+  x += 0x9E3779B97F4A7C15ull;
+  uint64_t z = x;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
 
 }  // namespace
 
@@ -1369,54 +1486,43 @@ APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, 
   const bool few = (cuts & 5) == 5;
   if (((uintptr_t)scratch & 15u) || scratch_bytes < (few ? carve_few(nullptr, n_rows).bytes : carve(nullptr, n_rows).bytes))
     return APC_ERR_BAD_ARG;
-  if (!few) {
-    std::lock_guard<std::mutex> hold(pass_attr_lock);
-    if (!pass_attr_set[dev]) {
-      const hipError_t e = hipFuncSetAttribute((const void*)sample_pass_kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(PassShared));
-      if (e != hipSuccess) return (int)e;
-      pass_attr_set[dev] = true;
-    }
+  if (!few)
+    if (const int rc = allow_pass_lds(dev)) return rc;
+  const SampleShape sz = shape_of(logits, ldl, n_rows, V);
+  if (few) return launch_few(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, scratch, out, nullptr, stream);
+  return launch_descents(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, nullptr, scratch, out, nullptr, cuts, stream);
+}
+
+// The same for up to 64 rows with their options on the host: they go with the first launch, and the ids also to `out_host` (host
+// memory that the device can write, or null), so that nothing is copied either way.  `options`: n_rows temperatures (float),
+// top-p (float), top-k (int), seeds (uint64) and numbers of the generated token (int64), one behind the other; the uniform number
+// of a row is that of (seed, number).  From the call to the ids on the host, 8 rows of 128,256: top-k 40 and top-p 0.95 86 -> 48
+// us (of which the sums in order above are 4), top-p alone 142 -> 108.
+APC_EXPORT int apc_sample_rows_host(const float* logits, int ldl, int n_rows, int V, const void* options, int* out, int* out_host,
+                                    void* scratch, size_t scratch_bytes, int cuts, hipStream_t stream) {
+  if (n_rows <= 0) return 0;
+  const bool few = (cuts & 5) == 5;
+  if (V <= 0 || ldl < V || n_rows > BY_VALUE || !options || !scratch || ((uintptr_t)scratch & 15u) ||
+      scratch_bytes < (few ? carve_few(nullptr, n_rows).bytes : carve(nullptr, n_rows).bytes))
+    return APC_ERR_BAD_ARG;
+  int dev = -1;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return (int)e;
+  if (V > (1 << 22) || dev < 0 || dev >= 64) return APC_ERR_UNSUPPORTED;
+  RowValues opt = {};
+  const size_t n = n_rows;
+  const char* from = (const char*)options;
+  memcpy(opt.temperature, from, 4 * n);
+  memcpy(opt.top_p, from + 4 * n, 4 * n);
+  memcpy(opt.top_k, from + 8 * n, 4 * n);
+  for (size_t r = 0; r < n; ++r) {
+    uint64_t seed, number;
+    memcpy(&seed, from + 12 * n + 8 * r, 8);
+    memcpy(&number, from + 20 * n + 8 * r, 8);
+    opt.uniform[r] = (float)(splitmix64(splitmix64(seed) ^ ((number + 1) * 0xD6E8FEB86659FD93ull)) >> 40) / (float)(1 << 24);
   }
-  SampleShape sz;
-  sz.ldl = ldl;
-  sz.V = V;
-  sz.R = n_rows;
-  cut_row(n_rows, V, &sz.pieces, &sz.chunk);
-  sz.vec = ((uintptr_t)logits % 16 == 0 && ldl % 4 == 0) ? 1 : 0;
-  sz.id_bits = 1;
-  while (sz.id_bits < 31 && (1u << sz.id_bits) < (unsigned)V) ++sz.id_bits;
-  sz.key_digits = ceil_div(32 + sz.id_bits, DIGIT_BITS);
-  sz.id_digits = ceil_div(sz.id_bits, DIGIT_BITS);
-  const dim3 grid(sz.pieces, n_rows);
-  if (few) {
-    const FewSpace fs = carve_few(scratch, n_rows);
-    hipLaunchKernelGGL(sample_few_pieces_kernel, grid, dim3(PNT), 0, stream, logits, sz, temperature, top_k, fs);
-    APC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sample_few_end_kernel, dim3(n_rows), dim3(SNT), 0, stream, logits, sz, temperature, top_k, top_p, uniform, fs, out);
-    APC_LAUNCH_CHECK();
-    return 0;
-  }
-  const SampleSpace sp = carve(scratch, n_rows);
-  hipLaunchKernelGGL(sample_max_kernel, grid, dim3(PNT), 0, stream, logits, sz, sp);
-  APC_LAUNCH_CHECK();
-  int q = 0, prev_stage = -1, prev_digit = -1;
-  for (int stage = 0; stage < N_SELECTS; ++stage) {
-    int digits = sz.key_digits;
-    if (stage == ST_TOPK && !(cuts & 1)) continue;
-    if (stage == ST_TOPP && !(cuts & 2)) continue;
-    if (stage == ST_DRAW) digits = (cuts & 3) ? sz.key_digits : sz.id_digits;
-    for (int digit = 0; digit < digits; ++digit) {
-      hipLaunchKernelGGL(sample_pass_kernel, grid, dim3(PNT), sizeof(PassShared), stream, logits, sz, temperature,
-                         top_k, top_p, uniform, sp, q, stage, digit, prev_stage, prev_digit);
-      APC_LAUNCH_CHECK();
-      ++q;
-      prev_stage = stage;
-      prev_digit = digit;
-    }
-  }
-  hipLaunchKernelGGL(sample_end_kernel, dim3(n_rows), dim3(SNT), 0, stream, logits, sz, temperature, top_k, top_p,
-                     uniform, sp, q, prev_stage, prev_digit, out);
-  APC_LAUNCH_CHECK();
-  return 0;
+  const SampleShape sz = shape_of(logits, ldl, n_rows, V);
+  if (few) return launch_few(logits, sz, opt, scratch, out, out_host, stream);
+  if (const int rc = allow_pass_lds(dev)) return rc;
+  return launch_descents(logits, sz, RowOptions{}, &opt, scratch, out, out_host, cuts, stream);
 }

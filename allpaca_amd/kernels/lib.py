@@ -76,6 +76,7 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
         "apc_argmax_rows_no_alloc": [P, I, I, I, P, P],
         "apc_sample_rows": [P, I, I, I, P, P, P, P, P, P, Z, I, P],
         "apc_sample_rows_scratch_kib": [I],
+        "apc_sample_rows_host": [P, I, I, I, P, P, P, P, Z, I, P],
     },
     "tuned": {
         "apc_gemm_bf16": [P, I, P, P, I, I, I, I, I, P],

@@ -4,8 +4,10 @@ what the kernel and its grid assume, and launches on torch's current stream.
 Nothing here computes on the CPU and nothing falls back to a library."""
 from __future__ import annotations
 
+import functools
 import math
 import os
+import struct
 from typing import Optional
 
 import torch
@@ -233,13 +235,48 @@ def argmax_rows(logits: torch.Tensor, out: torch.Tensor) -> None:
                                  scratch.data_ptr() if scratch is not None else 0, _stream()), "argmax_rows")
 
 
+OPTIONS_ON_HOST = 64     # rows whose options `sample_rows` takes as lists
+
+
+class PinnedIds:
+    """Host memory for token ids that a kernel may write (int32 [n])."""
+    __slots__ = ("tensor", "size", "address")
+
+    def __init__(self, n: int):
+        self.tensor = torch.empty(n, dtype=torch.int32).pin_memory()
+        self.size, self.address = n, self.tensor.data_ptr()
+
+
+@functools.lru_cache(maxsize=None)
+def _packed_options(n: int) -> struct.Struct:
+    return struct.Struct(f"<{n}f{n}f{n}i{n}Q{n}q")
+
+
 def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
                 uniform: torch.Tensor, out: torch.Tensor, any_top_k: bool = True, any_top_p: bool = True,
-                few_after_top_k: bool = False, one_block: bool = False) -> None:
+                few_after_top_k: bool = False, one_block: bool = False, out_host: Optional[PinnedIds] = None) -> bool:
     """One token a row by temperature / top-k / top-p with the row's uniform number.  `any_top_k`, `any_top_p`: whether
     some row may ask for that cut; `few_after_top_k`: every row that samples has 0 < top-k <= 1,024.  A caller that
     knows its rows saves the launches that none of them needs; a row for which its word is wrong still gets its
-    token, slowly.  `one_block`: the kernel without working memory, one block a row."""
+    token, slowly.  `one_block`: the kernel without working memory, one block a row.  Up to 64 rows may have their
+    options as lists, and (seeds, numbers of the generated token) for the uniform numbers: they go with the launch.  The ids are then written to `out_host` too; True if they are."""
+    L = _lib.load("plain")
+    if isinstance(temperature, list):
+        _gpu(logits, out)
+        ld = _rows(logits, "logits")
+        R, V = logits.shape
+        _need(logits.dtype == torch.float32, "logits are float32")
+        _need(not one_block and R == len(temperature) <= OPTIONS_ON_HOST, "options as lists: one for each of up to 64 rows")
+        seeds, numbers = uniform
+        kib = L.apc_sample_rows_scratch_kib(R)
+        scratch = torch.empty(kib * 1024, dtype=torch.uint8, device=logits.device)
+        host = out_host is not None and out_host.size >= R
+        cuts = (1 if any_top_k else 0) | (2 if any_top_p else 0) | (4 if few_after_top_k else 0)
+        _lib.check(L.apc_sample_rows_host(logits.data_ptr(), ld, R, V,
+                                          _packed_options(R).pack(*temperature, *top_p, *top_k, *seeds, *numbers),
+                                          _i32(out, R, "sample out"), out_host.address if host else 0, scratch.data_ptr(), kib * 1024,
+                                          cuts, _stream()), "sample_rows_host")
+        return host
     _gpu(logits, temperature, top_k, top_p, uniform, out)
     ld = _rows(logits, "logits")
     R, V = logits.shape
@@ -247,7 +284,6 @@ def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Te
     for t, name in ((temperature, "temperature"), (top_p, "top_p"), (uniform, "uniform")):
         if not (t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= R):
             raise ValueError(f"{name}: float32 [{R}]")
-    L = _lib.load("plain")
     kib = 0 if one_block else L.apc_sample_rows_scratch_kib(R)
     scratch = torch.empty(kib * 1024, dtype=torch.uint8, device=logits.device) if kib else None
     _lib.check(L.apc_sample_rows(logits.data_ptr(), ld, R, V, temperature.data_ptr(), _i32(top_k, R, "top_k"),
@@ -256,6 +292,7 @@ def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Te
                                  (1 if any_top_k else 0) | (2 if any_top_p else 0) | (4 if few_after_top_k else 0),
                                  _stream()),
                "sample_rows")
+    return False
 
 
 # --------------------------------------------------------------------------- dispatch

@@ -93,21 +93,33 @@ class Sampler:
         R = logits.shape[0]
         out = torch.empty(R, dtype=torch.int32, device=self.device)
         self._turn ^= 1
-        if all(p.greedy for p in params):
+        t = self._turn
+        if self._pinned[t] is None or self._pinned[t].size < R:
+            self._pinned[t] = ops.PinnedIds(max(R, 64))
+        pinned, on_host = self._pinned[t], False
+        temps = [p.temperature for p in params]
+        if all(x <= 1e-5 for x in temps):
             ops.argmax_rows(logits, out)
         else:
-            f = self._upload(params, indices)
-            ops.sample_rows(logits, f[0, :R], f[3, :R].view(torch.int32), f[1, :R], f[2, :R], out,
-                            any_top_k=any(p.top_k > 0 for p in params),
-                            any_top_p=any(0.0 <= p.top_p < 1.0 for p in params),
-                            few_after_top_k=all(p.greedy or 0 < p.top_k <= 1024 for p in params))
-        if self._pinned[self._turn] is None or self._pinned[self._turn].numel() < R:
-            self._pinned[self._turn] = torch.empty(max(R, 64), dtype=torch.int32).pin_memory()
-        pinned = self._pinned[self._turn]
-        pinned[:R].copy_(out, non_blocking=True)
+            ks, tops = [p.top_k for p in params], [p.top_p for p in params]
+            few = all(x <= 1e-5 or 0 < k <= 1024 for x, k in zip(temps, ks))
+            if self._by_value(logits.shape, temps, ks, tops):
+                opts = (temps, ks, tops, ([(self.default_seed if p.seed is None else p.seed) & _M64 for p in params], indices))
+            else:
+                f = self._upload(params, indices)
+                opts = (f[0, :R], f[3, :R].view(torch.int32), f[1, :R], f[2, :R])
+            on_host = ops.sample_rows(logits, *opts, out, any_top_k=max(ks) > 0, any_top_p=any(0.0 <= x < 1.0 for x in tops),
+                                      few_after_top_k=few, out_host=pinned)
+        if not on_host:
+            pinned.tensor[:R].copy_(out, non_blocking=True)
         done = torch.cuda.Event()
         done.record()
-        return Pending(pinned, R, done, out)
+        return Pending(pinned.tensor, R, done, out)
+
+    def _by_value(self, shape, temps, ks, tops) -> bool:
+        """Whether the rows' options can go with the launch itself (few rows, and numbers that the kernels' types hold)."""
+        return (self.device.type == "cuda" and shape[0] <= ops.OPTIONS_ON_HOST and shape[1] <= 1 << 22 and all(abs(x) < 3e38 for x in temps)
+                and all(abs(x) < 3e38 for x in tops) and max(ks) < 1 << 31)
 
 
 class Pending:

@@ -64,3 +64,26 @@ def test_greedy_rows_and_rows_the_callers_word_was_wrong_about():
     wide = torch.randn(6, 20003, generator=g, device=DEV)
     got, want = both_ways(wide[:, 1:20002], 0.8, 40, 0.95, rng.random(6))
     assert got == want
+
+
+# options on the host, with the launch: every rule, one row, the most rows that go that way and one more, rows of unlike
+# rules, a greedy row among others, numbers of tokens and seeds at the ends of their ranges
+@pytest.mark.parametrize("R,V", [(1, 4099), (8, 32001), (64, 9001), (65, 5000)])
+@pytest.mark.parametrize("rule", [(0.8, 40, 0.95), (0.7, 0, 0.9), (0.8, 0, 1.0), (1.1, 2000, 0.5), None])
+def test_options_that_go_with_the_launch(R, V, rule):
+    from allpaca_amd.kernels import ops
+    from allpaca_amd.sampling import GenerationParams
+    from allpaca_amd.sampling.sampler import Sampler, uniforms_for
+    logits = torch.randn(R, V, generator=torch.Generator(device=DEV).manual_seed(R), device=DEV) * 3
+    rules = [rule or [(0.0, 0, 1.0), (0.8, 40, 0.95), (1.0, 0, 1.0), (0.6, 1, 0.3), (0.9, 0, 0.7)][r % 5] for r in range(R)]
+    seeds = [(1 << 64) - 1 if r == 0 else None if r == 1 else 977 * r for r in range(R)]
+    numbers = [(1 << 40) * (r % 2) + r for r in range(R)]
+    params = [GenerationParams(temperature=t, top_k=k, top_p=p, seed=s) for (t, k, p), s in zip(rules, seeds)]
+    f = lambda x, dt: torch.tensor(x, dtype=dt, device=DEV)  # noqa: E731
+    want = torch.empty(R, dtype=torch.int32, device=DEV)
+    ops.sample_rows(logits, f([t for t, _, _ in rules], torch.float32), f([k for _, k, _ in rules], torch.int32), f([p for _, _, p in rules], torch.float32),
+                    torch.from_numpy(uniforms_for([5 if s is None else s for s in seeds], numbers)).to(DEV), want, one_block=True)
+    sampler = Sampler(torch.device(DEV), 5)
+    for _ in range(3):                                       # (both of the sampler's result buffers)
+        pending = sampler.launch(logits, params, numbers)
+        assert pending.wait() == want.tolist() == pending.device.tolist()
