@@ -134,6 +134,129 @@ __global__ __launch_bounds__(256) void recurrence_states_kernel(float* __restric
   *st = s;
 }
 
+// ---- One row of every request (decoding): convolution, the gates' products and the recurrence in one launch ----
+// A block takes one of the parts and all rows (up to 16): the convolution of its channels, moving the requests' kept inputs on,
+// into LDS; a wave's bands of r's and i's logits on the matrix cores, their weights asked for at the very start; and where the
+// logits lie, four channels of a row a lane, the recurrence, whose state, y and constants were asked for at the start too.  The
+// operations are those of conv_channels_bf16x8_kernel, heads_gemm_few_kernel and gated_recurrence_kernel, in their order, so the
+// results are the same bits.  What bounds it is latency: three launches that do this took 5.8 + 3.5 + 3.7 us for 8 rows of 2,048
+// channels in 16 parts (1 MB of weights), this takes 7.0 (6.2 + 4.5 + 3.7 beside it); 25 steps of 8 requests 8.72 -> 8.48 ms.
+constexpr int STEP_ROWS = 16, STEP_W = 256, STEP_PAD = 8, STEP_WAVES = 8;
+__device__ __forceinline__ float sigmoid_exact(float z) { return 1.0f / (1.0f + expf(-z)); }
+__device__ __forceinline__ float gelu_tanh_exact(float z) {
+  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+}
+
+struct StepArgs {
+  const bf16_t *x, *y;             // [M][C] rows of strides ldx, ldy
+  int ldx, ldy;
+  const float *in_bias, *conv_w, *conv_b;
+  float* conv_state;               // [slot][taps - 1][C]
+  const bf16_t* W;                 // [parts][2 w / 16][w / 32] tiles
+  const float *zb, *rate, *yb;
+  float out_scale;
+  float* state;                    // [slot][C]
+  const int *row_seg, *conv_slots, *slots;
+  bf16_t* out;
+  int ldo, M, C, w;
+};
+
+template <int TAPS, int CHUNKS>    // CHUNKS: w / 32
+__global__ __launch_bounds__(STEP_WAVES * 64) void recurrent_step_kernel(StepArgs A) {
+  constexpr int w = CHUNKS * 32, BANDS = w / 16, TURNS = (BANDS + STEP_WAVES - 1) / STEP_WAVES;
+  __shared__ __attribute__((aligned(16))) bf16_t us[STEP_ROWS][w + STEP_PAD];
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, li = lane % 16, lc = lane / 16;
+  const int part = blockIdx.x, c0 = part * w, row = min(li, A.M - 1);
+  const bf16_t* wp = A.W + (size_t)part * 2 * BANDS * CHUNKS * 512 + lane * 8;
+  Frag fr[CHUNKS], fi[CHUNKS];
+  auto load_gates = [&](int band) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < CHUNKS; ++k) {
+      fr[k] = load_frag(wp + (size_t)(band * CHUNKS + k) * 512);
+      fi[k] = load_frag(wp + (size_t)((BANDS + band) * CHUNKS + k) * 512);
+    }
+  };
+  load_gates(min(wave, BANDS - 1));
+  const int slot = A.slots[A.row_seg[row]];
+
+  for (int p = threadIdx.x; p < A.M * (w / 8); p += STEP_WAVES * 64) {
+    const int r = p / (w / 8), c = c0 + p % (w / 8) * 8;
+    float* st = A.conv_state + (size_t)A.conv_slots[A.row_seg[r]] * (TAPS - 1) * A.C + c;
+    float u[TAPS][8], ib[8], b[8], wt[8][TAPS];
+    const uint4 v = *reinterpret_cast<const uint4*>(A.x + (size_t)r * A.ldx + c);
+#pragma unroll
+    for (int j = 0; j + 1 < TAPS; ++j) {
+      const float4 lo = *reinterpret_cast<const float4*>(st + (size_t)j * A.C), hi = *reinterpret_cast<const float4*>(st + (size_t)j * A.C + 4);
+      u[j][0] = lo.x; u[j][1] = lo.y; u[j][2] = lo.z; u[j][3] = lo.w;
+      u[j][4] = hi.x; u[j][5] = hi.y; u[j][6] = hi.z; u[j][7] = hi.w;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) wt[e][j] = A.conv_w[(size_t)(c + e) * TAPS + j];
+      b[e] = A.conv_b ? A.conv_b[c + e] : 0.f;
+      ib[e] = A.in_bias ? A.in_bias[c + e] : 0.f;
+    }
+    const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      u[TAPS - 1][2 * k] = __uint_as_float(q[k] << 16) + ib[2 * k];
+      u[TAPS - 1][2 * k + 1] = __uint_as_float(q[k] & 0xffff0000u) + ib[2 * k + 1];
+    }
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      acc[e] = 0.f;
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) acc[e] = fmaf(wt[e][j], u[j][e], acc[e]);     // oldest first
+      if (A.conv_b) acc[e] += b[e];
+    }
+    *reinterpret_cast<uint4*>(&us[r][p % (w / 8) * 8]) =
+        uint4{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]), pack_bf16x2(acc[4], acc[5]), pack_bf16x2(acc[6], acc[7])};
+#pragma unroll
+    for (int j = 1; j < TAPS; ++j) {
+      *reinterpret_cast<float4*>(st + (size_t)(j - 1) * A.C) = float4{u[j][0], u[j][1], u[j][2], u[j][3]};
+      *reinterpret_cast<float4*>(st + (size_t)(j - 1) * A.C + 4) = float4{u[j][4], u[j][5], u[j][6], u[j][7]};
+    }
+  }
+
+  for (int turn = 0; turn < TURNS; ++turn) {
+    const int band = wave + turn * STEP_WAVES;
+    const bool on = band < BANDS && li < A.M;
+    const int at = min(band, BANDS - 1) * 16 + lc * 4, c = c0 + at;     // this lane's first channel, in the part and in all
+    float* sp = A.state + (size_t)slot * A.C + c;
+    const float4 S4 = *reinterpret_cast<const float4*>(sp), k4 = *reinterpret_cast<const float4*>(A.rate + c);
+    const float4 br4 = *reinterpret_cast<const float4*>(A.zb + 2 * c0 + at), bi4 = *reinterpret_cast<const float4*>(A.zb + 2 * c0 + w + at);
+    const float4 by4 = A.yb ? *reinterpret_cast<const float4*>(A.yb + c) : float4{0.f, 0.f, 0.f, 0.f};
+    const uint2 y2 = *reinterpret_cast<const uint2*>(A.y + (size_t)row * A.ldy + c);
+    if (turn == 0) __syncthreads();                     // the convolution's rows are there
+    floatx4 zr = floatx4{0.f, 0.f, 0.f, 0.f}, zi = zr;
+#pragma unroll
+    for (int k = 0; k < CHUNKS; ++k) {
+      const Frag fa = *reinterpret_cast<const Frag*>(&us[li][k * 32 + lc * 8]);   // (rows past the last hold anything: columns of their own)
+      zr = mfma16(fr[k], fa, zr);
+      zi = mfma16(fi[k], fa, zi);
+    }
+    if (turn + 1 < TURNS) load_gates(min(band + STEP_WAVES, BANDS - 1));
+    if (!on) continue;
+    const float Sv[4] = {S4.x, S4.y, S4.z, S4.w}, kv[4] = {k4.x, k4.y, k4.z, k4.w}, br[4] = {br4.x, br4.y, br4.z, br4.w};
+    const float bi[4] = {bi4.x, bi4.y, bi4.z, bi4.w}, by[4] = {by4.x, by4.y, by4.z, by4.w};
+    const uint2 u2 = *reinterpret_cast<const uint2*>(&us[li][at]);
+    float S[4], o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t ub = e < 2 ? u2.x : u2.y, yw = e < 2 ? y2.x : y2.y;
+      const float uv = __uint_as_float(e % 2 ? ub & 0xffff0000u : ub << 16), yv = __uint_as_float(e % 2 ? yw & 0xffff0000u : yw << 16);
+      const float log_a = kv[e] * sigmoid_exact(zr[e] + br[e]);
+      const float in = sigmoid_exact(zi[e] + bi[e]) * uv;
+      S[e] = fmaf(expf(log_a), Sv[e], sqrtf(-expm1f(2.0f * log_a)) * in);
+      o[e] = S[e] * gelu_tanh_exact(yv + by[e]) * A.out_scale;
+    }
+    *reinterpret_cast<float4*>(sp) = float4{S[0], S[1], S[2], S[3]};
+    *reinterpret_cast<uint2*>(A.out + (size_t)li * A.ldo + c) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+  }
+}
+
 }  // namespace
 
 // 1 if the kernels take these sizes, else 0 (the caller then runs the kernel that walks row by row)
@@ -169,5 +292,42 @@ APC_EXPORT int apc_gated_recurrence_bf16(const void* u, int ldu, const float* z,
   APC_LAUNCH_CHECK();
   REC_LAUNCH(2);
 #undef REC_LAUNCH
+  return 0;
+}
+
+// 1 if one launch takes a step of M single rows with these sizes and strides
+APC_EXPORT int apc_recurrent_step_bf16_takes(int M, int C, int parts, int taps, int ldx, int ldy, int ldo) {
+  if (M < 1 || M > STEP_ROWS || C <= 0 || parts <= 0 || C % parts || taps < 2 || taps > 4) return 0;
+  const int w = C / parts;
+  return ((w == 32 || w == 64 || w == 128 || w == 256) && w <= STEP_W && ldx % 8 == 0 && ldy % 4 == 0 && ldo % 4 == 0) ? 1 : 0;
+}
+
+// row_seg: a row's segment, of which it is the only row; conv_slots, slots: the segments' places in conv_state and state
+APC_EXPORT int apc_recurrent_step_bf16(const void* x, int ldx, const void* y, int ldy, const float* in_bias, const float* conv_w,
+                                       const float* conv_b, int taps, float* conv_state, const void* W, const float* zb, int parts,
+                                       const float* rate, const float* yb, float out_scale, float* state, int M, int C,
+                                       const int* row_seg, const int* conv_slots, const int* slots, void* out, int ldo,
+                                       hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (!apc_recurrent_step_bf16_takes(M, C, parts, taps, ldx, ldy, ldo)) return APC_ERR_UNSUPPORTED;
+  if (!x || !y || !conv_w || !conv_state || !W || !zb || !rate || !state || !row_seg || !conv_slots || !slots || !out || ldx < C ||
+      ldy < C || ldo < C || (((uintptr_t)x | (uintptr_t)W | (uintptr_t)conv_state | (uintptr_t)state | (uintptr_t)zb | (uintptr_t)rate |
+      (uintptr_t)yb) & 15u) || (((uintptr_t)y | (uintptr_t)out) & 7u))
+    return APC_ERR_BAD_ARG;
+  const StepArgs A{(const bf16_t*)x, (const bf16_t*)y, ldx, ldy, in_bias, conv_w, conv_b, conv_state, (const bf16_t*)W, zb, rate, yb,
+                   out_scale, state, row_seg, conv_slots, slots, (bf16_t*)out, ldo, M, C, C / parts};
+#define STEP_LAUNCH(TAPS_, CHUNKS_) \
+  hipLaunchKernelGGL((recurrent_step_kernel<TAPS_, CHUNKS_>), dim3(parts), dim3(STEP_WAVES * 64), 0, stream, A)
+#define STEP_BY_W(TAPS_)                                                                                          \
+  switch (A.w) {                                                                                                  \
+    case 32: STEP_LAUNCH(TAPS_, 1); break;                                                                        \
+    case 64: STEP_LAUNCH(TAPS_, 2); break;                                                                        \
+    case 128: STEP_LAUNCH(TAPS_, 4); break;                                                                       \
+    default: STEP_LAUNCH(TAPS_, 8); break;                                                                        \
+  }
+  if (taps == 2) { STEP_BY_W(2) } else if (taps == 3) { STEP_BY_W(3) } else { STEP_BY_W(4) }
+#undef STEP_BY_W
+#undef STEP_LAUNCH
+  APC_LAUNCH_CHECK();
   return 0;
 }

@@ -1258,3 +1258,15 @@ def gated_recurrence(u: torch.Tensor, z: torch.Tensor, z_bias: torch.Tensor, blo
         int(blocks), _f32(rate, C, "rate"), y.data_ptr(), _code(y), _rows(y, "y"), _f32(y_bias, C, "y bias"),
         float(out_scale), state.data_ptr(), C, S, _i32(step.seg_row0, S, "seg_row0"), _i32(step.seg_rows, S, "seg_rows"),
         _i32(slots, S, "slots"), out.data_ptr(), _code(out), _rows(out, "out"), _stream()), "gated_recurrence")
+
+
+def recurrent_step(x: torch.Tensor, y: torch.Tensor, in_bias, conv_w: torch.Tensor, conv_b, conv_state: torch.Tensor, conv_slots: torch.Tensor,
+                   w_gates, z_bias: torch.Tensor, blocks: int, rate: torch.Tensor, y_bias, state: torch.Tensor, slots: torch.Tensor, step,
+                   out: torch.Tensor, out_scale: float = 1.0) -> bool:
+    """`conv_channels` of x, `heads_linear` of its rows with the gates' matrices and `gated_recurrence` of both with y, in
+    one launch for a step of few single rows; False (nothing done) where there is no such kernel."""
+    if isinstance(w_gates, torch.Tensor) or not getattr(step, "decode_only", False) or not _tuned_ok(x, y, out):
+        return False
+    from . import tuned
+    return tuned.recurrent_step_bf16(x, y, in_bias, conv_w, conv_b, conv_state, conv_slots, w_gates, z_bias, int(blocks), rate, y_bias,
+                                     state, slots, step, out, float(out_scale))

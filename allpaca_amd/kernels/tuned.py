@@ -850,6 +850,35 @@ def gated_recurrence_bf16(u, z, z_bias, blocks: int, rate, y, y_bias, state, ste
     return True
 
 
+def recurrent_step_bf16(x, y, in_bias, conv_w, conv_b, conv_state, conv_slots, w_gates, z_bias, blocks: int, rate, y_bias, state, slots,
+                        step, out, out_scale: float) -> bool:
+    """One row of every request through the convolution, the gates' products and the recurrence in one launch; False
+    (nothing done) for sizes that it does not take."""
+    L = _lib.load("tuned")
+    T, C = out.shape
+    taps = int(conv_w.shape[1])
+    ldx, ldy, ldo = _ops._rows(x, "conv input"), _ops._rows(y, "y"), _ops._rows(out, "out")
+    S = step.n_segs
+    if (conv_state is None or conv_slots is None or S != T or not L.apc_recurrent_step_bf16_takes(T, C, blocks, taps, ldx, ldy, ldo)
+            or not _aligned(x, conv_state, state, z_bias, rate, w_gates.data) or (y_bias is not None and not _aligned(y_bias))
+            or any(t.data_ptr() % 8 for t in (y, out))):
+        return False
+    w = C // blocks
+    _ops._gpu(x, y, conv_w, conv_state, w_gates.data, state, out)
+    _ops._need(x.shape[0] == T and x.shape[1] >= C and y.shape == (T, C), "recurrent step: x and y hold the channels of every row")
+    _ops._need(w_gates.H == blocks and w_gates.N == 2 * w and w_gates.K == w, "recurrent step: a matrix [2 w, w] for every part")
+    _ops._need(conv_w.shape[0] == C and conv_w.dtype == torch.float32 and conv_w.is_contiguous(), "recurrent step: float32 [channels, taps]")
+    _ops._need(conv_state.dtype == torch.float32 and conv_state.is_contiguous() and tuple(conv_state.shape[1:]) == (taps - 1, C)
+               and state.dtype == torch.float32 and state.is_contiguous() and tuple(state.shape[1:]) == (C,),
+               "recurrent step: states must be float32 [slots, taps - 1, channels] and [slots, channels]")
+    _lib.check(L.apc_recurrent_step_bf16(
+        x.data_ptr(), ldx, y.data_ptr(), ldy, _ops._f32(in_bias, C, "input bias"), conv_w.data_ptr(), _ops._f32(conv_b, C, "bias"), taps,
+        conv_state.data_ptr(), w_gates.data.data_ptr(), _ops._f32(z_bias, 2 * C, "gate biases"), blocks, _ops._f32(rate, C, "rate"),
+        _ops._f32(y_bias, C, "y bias"), out_scale, state.data_ptr(), T, C, _ops._i32(step.row_seg, T, "row_seg"),
+        _ops._i32(conv_slots, S, "slots"), _ops._i32(slots, S, "slots"), out.data_ptr(), ldo, _ops._stream()), "recurrent_step_bf16")
+    return True
+
+
 LINEAR_CHUNK_ROWS = 64
 
 

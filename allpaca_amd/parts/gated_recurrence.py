@@ -85,6 +85,10 @@ class GatedRecurrence(Mixer):
         if state is None or not state.writes:
             raise ValueError("a recurrent mixer needs a state of its own")
         T, dev, C = proj.shape[0], proj.device, self.C
+        if conv is not None and ops.recurrent_step(proj[:, C:2 * C], proj[:, :C], self.x_b, self.conv_w, self.conv_b, conv.state, conv.slots,
+                                                   self.w_gates, self.gates_b, self.B, self.rate, self.y_b, state.state, state.slots,
+                                                   step, out, scale):
+            return
         u = torch.empty((T, C), dtype=self.rt.dtype, device=dev)
         ops.conv_channels(proj[:, C:], C, self.conv_w, self.conv_b, conv.state if conv is not None else None, step,
                           conv.slots if conv is not None else None, "none", u, in_bias=self.x_b)

@@ -598,3 +598,38 @@ def test_command_line_and_replay_program(tmp_path):
             assert at == rows.shape[0]
         for k, toks in zip("abc", (a, b, c)):
             check(np.concatenate(got[k]), name, toks, dtype, f"replay {k}")
+
+
+# one row, the most rows and some between; parts of every width that is taken (one band a wave, fewer and more bands than
+# waves); two to four taps; with and without biases
+@pytest.mark.parametrize("M, C, parts, taps", [(1, 2048, 16, 4), (16, 256, 1, 4), (5, 96, 3, 2), (8, 512, 8, 3), (11, 1024, 4, 4), (3, 128, 1, 2)])
+@pytest.mark.parametrize("biases", [True, False])
+def test_a_recurrent_step_in_one_launch(M, C, parts, taps, biases):
+    """The same bits as the convolution, the gates' products and the recurrence one after the other, and the same states
+    behind them; other requests' states are left alone."""
+    from allpaca_amd.kernels import ops
+    rng = np.random.default_rng(C + M)
+    w, tdt = C // parts, torch.bfloat16
+    proj = dev(bf(rng.normal(size=(M, 2 * C + 8))), tdt)
+    gates = ops.prepare_heads(dev(bf(rng.normal(size=(parts, 2 * w, w)) / w ** 0.5), tdt), tdt, w, 2 * w)
+    x_b, y_b, conv_b = (dev(np.float32(rng.normal(size=C) * 0.5)) if biases else None for _ in range(3))
+    conv_w, zb = dev(np.float32(rng.normal(size=(C, taps)))), dev(np.float32(rng.normal(size=2 * C) * 0.5))
+    rate = dev(np.float32(-8.0 * P.softplus(rng.normal(size=C) * 3.0 - 4.0)))
+    slots = rng.permutation(M + 2)[:M].tolist()
+    step = make_step([(7, 1)] * M, [[1]] * M, slots)
+    conv, state = dev(np.float32(rng.normal(size=(M + 3, taps - 1, C)))), dev(np.float32(rng.normal(size=(M + 3, C))))
+    conv2, state2 = conv.clone(), state.clone()
+    out, want = (torch.full((M, C + 8), 9.0, dtype=tdt, device=DEV) for _ in range(2))
+    x, y, s = proj[:, C:2 * C], proj[:, :C], step.state_slots
+    assert step.decode_only
+    for _ in range(2):
+        assert ops.recurrent_step(x, y, x_b, conv_w, conv_b, conv, s, gates, zb, parts, rate, y_b, state, s, step, out[:, :C], 0.6)
+        u, z = torch.empty((M, C), dtype=tdt, device=DEV), torch.empty((M, 2 * C), dtype=torch.float32, device=DEV)
+        ops.conv_channels(x, C, conv_w, conv_b, conv2, step, s, "none", u, in_bias=x_b)
+        ops.heads_linear(u, w, gates, z, 2 * w)
+        ops.gated_recurrence(u, z, zb, parts, rate, y, y_b, state2, step, s, want[:, :C], 0.6)
+        assert torch.equal(out, want) and torch.equal(conv, conv2) and torch.equal(state, state2)
+    many = make_step([(7, 1)] * 17, [[1]] * 17, list(range(17)))
+    p17 = torch.zeros((17, 2 * C), dtype=tdt, device=DEV)
+    assert not ops.recurrent_step(p17[:, C:], p17[:, :C], x_b, conv_w, conv_b, conv, many.state_slots, gates, zb, parts, rate, y_b, state,
+                                  many.state_slots, many, torch.empty((17, C), dtype=tdt, device=DEV))
