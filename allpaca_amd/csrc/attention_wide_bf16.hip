@@ -325,6 +325,7 @@ __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kerne
   const int* bt = block_table + (size_t)row_seg[row0] * max_blocks;
   const int first = (window > 0 && pos0 - window + 1 > 0) ? pos0 - window + 1 : 0;
   const size_t page_stride = (size_t)2 * Hk * P * d;
+  const uint32_t page_bytes = (uint32_t)(page_stride * 2);   // (the launch has seen that this is all of it)
   // The keys of the block: those its rows see, or with the tile's keys cut into n_splits ranges of whole key tiles,
   // one of them: `last` is then the range's last key, the rows see nothing beyond it, and what the block leaves is a
   // partial result that attn_wide_merge_kernel adds to the other ranges'.
@@ -413,12 +414,17 @@ __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kerne
   const int voff = (lane % 32) * (P * 2) + (lane / 32) * 16 + (DT - 1) * 1024;
   const int vstep = 32 * P * 2 - 1024;  // load i: elements 32 i .. of a page row of 2 P bytes, 1 KiB further in LDS
   auto group_of = [&](int j) { return min(t_begin + j * KT + 16 * wave, last16); };  // first key of the wave's 16
-  auto page_of = [&](int j) { return __builtin_amdgcn_readfirstlane(bt[group_of(j) >> lgP]); };
+  auto page_of = [&](int j) { return __builtin_amdgcn_readfirstlane(bt[((uint32_t)group_of(j) >> lgP) & 0x1fffffffu]); };
   const bf16_t* k_head_low = k_head - (DT - 1) * 512;  // 3 KiB lower (1 KiB with two loads a tile)
   const bf16_t* v_head_low = v_head - (DT - 1) * 512;
+  // Scalar work stands in the wave's one stream of instructions like all else: a page's place is one 32 x 32 bit product, made
+  // for K's page and handed on to V a pass later, and the bases are kept as they are added (63 -> 39 scalar instructions a pass).
+  uint64_t k_low = (uint64_t)(uintptr_t)k_head_low, v_low = (uint64_t)(uintptr_t)v_head_low;
+  asm volatile("" : "+s"(k_low), "+s"(v_low));
+  auto place_of = [&](int page) { return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(page) * page_bytes; };
   // one of the 4 loads of a tile's K or V (to stand between other work)
-  auto k_load_piece = [&](int j, int page, int i) {
-    const BufferRsrc kr = make_rsrc(k_head_low + (size_t)__builtin_amdgcn_readfirstlane(page) * page_stride);
+  auto k_load_piece = [&](int j, uint64_t place, int i) {
+    const BufferRsrc kr = make_rsrc((const void*)(k_low + place));
     const int soff = (group_of(j) & (P - 1)) * (d * 2);
     const lds_ptr dst = (lds_ptr)(smem + (j % STG) * K_STAGE + (16 * wave) * ROW_BYTES);
     if (i == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, dst, 16, koff0, soff, 0, 0);
@@ -428,8 +434,8 @@ __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kerne
       if (i == 3) __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, dst, 16, koff3, soff, 3072, 0);
     }
   };
-  auto v_load_piece = [&](int j, int page, int i) {
-    const BufferRsrc vr = make_rsrc(v_head_low + (size_t)__builtin_amdgcn_readfirstlane(page) * page_stride);
+  auto v_load_piece = [&](int j, uint64_t place, int i) {
+    const BufferRsrc vr = make_rsrc((const void*)(v_low + place));
     const int soff = (group_of(j) & (P - 1)) * 2;
     const lds_ptr dst = (lds_ptr)(smem + V_BASE + (j % STG) * V_STAGE + wave * (DT * 1024));
     if (i == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, dst, 16, voff, soff, 0, 0);
@@ -703,6 +709,8 @@ __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kerne
       kpg = page_of(5);
     }
 
+    uint64_t v_place = 0;                     // of V's next page, in the passes that keep it
+
     // ---- a pass of the loop.  Before pass i: S1(i) raw in s1, P0(i) in p0, the fragments of K(i + 1) and V(i) in kfr
     // and vfr (on their way from LDS).  MASKED: some row may not see some key of tile i (row tile 1) or tile i + 1 (row
     // tile 0), or tile i + 1 has stale positions.
@@ -763,20 +771,22 @@ __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kerne
         const int tk = t0 + KT + kh * 32;
         const int stage_k = ((i + 2) % STG) * K_STAGE;
         const int va = lds0 + vaddr + ((i + 1) % STG) * V_STAGE;
+        const uint64_t k_place = MASKED ? 0 : place_of(kpg);
 #define SLOT_B_STEP(G)  /* a fragment's registers are free once the MFMA behind the one that read them has gone out; \
                            the direct loads of K(i + 5) and V(i + 4) go out one a step */                          \
   if constexpr (G < NG) {                                                                           \
     if (G == 0) mfma_set<NO_WAIT>(s1, kfr[G], qf[1][G]);                                            \
     else mfma_add<NO_WAIT>(s1, kfr[G], qf[1][G]);                                                   \
     if constexpr (G > 0) vfr[G - 1] = lds_frag<(G > 0 ? G - 1 : 0) * 1024>(va);                     \
-    if (!MASKED && G < DT) k_load_piece(i + 5, kpg, G);                                             \
-    if (!MASKED && G >= DT) v_load_piece(i + 4, vpg, G - DT);                                       \
+    if (!MASKED && G < DT) k_load_piece(i + 5, k_place, G);                                         \
+    if (!MASKED && G >= DT) v_load_piece(i + 4, v_place, G - DT);                                   \
     SOFT_STEPS(G, 0, s0, p0, st[0])                                                                 \
     __builtin_amdgcn_sched_barrier(0);                                                              \
     mfma_acc<NO_WAIT>(o[1][G % DT], vfr[G], p1[G / DT]);                                            \
     kfr[G] = k_frag(stage_k, G);                                                                    \
     if (!MASKED && G == NG - 1) {                                                                   \
       vpg = kpg;                                                                                    \
+      v_place = k_place;                                                                            \
       kpg = page_of(i + 6);                                                                         \
     }                                                                                               \
     SOFT_STEPS(G, 1, s0, p0, st[0])                                                                 \
@@ -810,6 +820,7 @@ __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kerne
       int i_end = i + 1;
       while (i_end < n_kt && all_seen(i_end)) ++i_end;
       st[0].sum = st[1].sum = 0.f;
+      v_place = place_of(vpg);
       for (; i < i_end; ++i) pass(std::integral_constant<int, SOFT_SEEN>{}, i);
       st[0].l += halves_sum(st[0].sum);
       st[1].l += halves_sum(st[1].sum);
@@ -960,7 +971,7 @@ __global__ __launch_bounds__(256) void attn_wide_merge_kernel(const float* __res
 }  // namespace
 
 bool attn_wide_takes(int d, int page_tokens) {
-  return (d == 128 || d == 64) && page_tokens >= 16 && (page_tokens & (page_tokens - 1)) == 0;
+  return (d == 128 || d == 64) && page_tokens >= 16 && page_tokens <= 32768 && (page_tokens & (page_tokens - 1)) == 0;
 }
 
 int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, int ldo, int H, int Hk,
@@ -968,7 +979,7 @@ int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, i
                              const int* positions, const int* row_seg, const int* tile_row0, const int* tile_rows,
                              int n_tiles, int window, float scale, int n_splits, int part_rows, float* parts,
                              int d, hipStream_t stream) {
-  if (!attn_wide_takes(d, page_tokens)) return APC_ERR_UNSUPPORTED;
+  if (!attn_wide_takes(d, page_tokens) || (long long)4 * Hk * page_tokens * d >= (1LL << 32)) return APC_ERR_UNSUPPORTED;
   if (n_splits < 1 || n_splits > 8 || (n_splits > 1 && (!parts || part_rows <= 0)) ||
       (long)n_tiles * H * n_splits > 0x7fffffffL)
     return APC_ERR_BAD_ARG;
