@@ -924,48 +924,59 @@ __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kerne
   plain_rows(std::integral_constant<int, 1>{});
 }
 
-// The ranges of keys of a row added up: out = sum_s w_s O_s / sum_s w_s with w_s = l_s 2^(m_s - max m).  A thread
-// takes four elements of a head of a row; blockIdx.y counts the blocks of 256 threads a row needs.
-__global__ __launch_bounds__(256) void attn_wide_merge_kernel(const float* __restrict__ parts, int n_splits, int part_rows,
-                                                              int H, const int* __restrict__ tile_row0,
+// The ranges of keys of a row added up: out = sum_s w_s O_s / sum_s w_s with w_s = l_s 2^(m_s - max m).  A thread takes eight
+// elements of a head of a row; blockIdx.y counts the blocks of 256 threads a row needs.  What bounds it is the way of the partial
+// rows, so a thread asks for all of them before it looks at any (with the number of ranges known only at run time it waited for
+// each range's reference in turn): 1,500 rows x 32 heads of 64, four ranges (49 MB) 21.1 -> 10.0 us.
+template <int SPLITS>
+__global__ __launch_bounds__(256) void attn_wide_merge_kernel(const float* __restrict__ parts, int part_rows, int H,
+                                                              const int* __restrict__ tile_row0,
                                                               const int* __restrict__ tile_rows, bf16_t* __restrict__ out,
                                                               int ldo, int d) {
   const int tile = blockIdx.x / ATTN_WIDE_ROWS, r = blockIdx.x % ATTN_WIDE_ROWS;
   const int hq = blockIdx.y * 256 + threadIdx.x;
-  if (r >= tile_rows[tile] || hq >= H * (d / 4)) return;
-  const int row = tile_row0[tile] + r;
-  const float* part_ml = parts + (size_t)n_splits * part_rows * H * d;
+  const int row0 = tile_row0[tile], rows = tile_rows[tile];
+  if (r >= rows || hq >= H * (d / 8)) return;
+  const float* part_ml = parts + (size_t)SPLITS * part_rows * H * d;
   const size_t plane = (size_t)part_rows * H;
-  const int h = hq / (d / 4), e = (hq % (d / 4)) * 4;
-  const size_t at = (size_t)row * H + h;
-  constexpr int MOST = 8;  // ranges (the launch code refuses more)
-  float ms[MOST], ls[MOST];
-  floatx4 os[MOST];
+  const int h = hq / (d / 8), e = (hq % (d / 8)) * 8;
+  const size_t at = (size_t)(row0 + r) * H + h;
+  float2 ml[SPLITS];
+  floatx4 os[SPLITS][2];
+#pragma unroll
+  for (int s = 0; s < SPLITS; ++s) {
+    ml[s] = *reinterpret_cast<const float2*>(part_ml + (s * plane + at) * 2);
+    os[s][0] = *reinterpret_cast<const floatx4*>(parts + (s * plane + at) * d + e);
+    os[s][1] = *reinterpret_cast<const floatx4*>(parts + (s * plane + at) * d + e + 4);
+  }
   float m = -INFINITY;
 #pragma unroll
-  for (int s = 0; s < MOST; ++s) {
-    if (s < n_splits) {
-      ms[s] = part_ml[(s * plane + at) * 2];
-      ls[s] = part_ml[(s * plane + at) * 2 + 1];
-      os[s] = *reinterpret_cast<const floatx4*>(parts + (s * plane + at) * d + e);
-      m = fmaxf(m, ms[s]);
-    }
-  }
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < SPLITS; ++s) m = fmaxf(m, ml[s].x);
+  floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   float sum = 0.f;
 #pragma unroll
-  for (int s = 0; s < MOST; ++s) {
-    if (s < n_splits && ms[s] != -INFINITY) {  // (a range that the row sees no key of has left no row)
-      const float w = ls[s] * exp2_neg(ms[s] - m);
-      acc += w * os[s];
+  for (int s = 0; s < SPLITS; ++s) {
+    if (ml[s].x != -INFINITY) {  // (a range that the row sees no key of has left no row)
+      const float w = ml[s].y * exp2_neg(ml[s].x - m);
+      acc[0] += w * os[s][0];
+      acc[1] += w * os[s][1];
       sum += w;
     }
   }
   const float inv = sum > 0.f ? 1.0f / sum : 0.f;
-  uint2 pk;
-  pk.x = pack_bf16x2(acc[0] * inv, acc[1] * inv);
-  pk.y = pack_bf16x2(acc[2] * inv, acc[3] * inv);
-  *reinterpret_cast<uint2*>(out + (size_t)row * ldo + (size_t)h * d + e) = pk;
+  Frag f;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    f.w[2 * q] = pack_bf16x2(acc[q][0] * inv, acc[q][1] * inv);
+    f.w[2 * q + 1] = pack_bf16x2(acc[q][2] * inv, acc[q][3] * inv);
+  }
+  bf16_t* to = out + (size_t)(row0 + r) * ldo + (size_t)h * d + e;
+  if (((uintptr_t)out | (uintptr_t)(ldo * 2)) % 16 == 0) {
+    *reinterpret_cast<Frag*>(to) = f;
+  } else {
+    reinterpret_cast<uint2*>(to)[0] = uint2{f.w[0], f.w[1]};
+    reinterpret_cast<uint2*>(to)[1] = uint2{f.w[2], f.w[3]};
+  }
 }
 
 }  // namespace
@@ -1013,9 +1024,13 @@ int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, i
                      n_tiles, window, scale, n_splits, part_rows, parts);
   APC_LAUNCH_CHECK();
   if (n_splits > 1) {
-    hipLaunchKernelGGL(attn_wide_merge_kernel, dim3(n_tiles * ATTN_WIDE_ROWS, ceil_div(H * (d / 4), 256)),
-                       dim3(256), 0, stream, parts, n_splits,
-                       part_rows, H, tile_row0, tile_rows, out, ldo, d);
+#define MERGE(S_)                                                                                                       \
+  case S_:                                                                                                              \
+    hipLaunchKernelGGL(attn_wide_merge_kernel<S_>, dim3(n_tiles * ATTN_WIDE_ROWS, ceil_div(H * (d / 8), 256)), dim3(256), \
+                       0, stream, parts, part_rows, H, tile_row0, tile_rows, out, ldo, d);                              \
+    break;
+    switch (n_splits) { MERGE(2) MERGE(3) MERGE(4) MERGE(5) MERGE(6) MERGE(7) MERGE(8) }
+#undef MERGE
     APC_LAUNCH_CHECK();
   }
   return 0;
