@@ -143,11 +143,13 @@ __global__ __launch_bounds__(NT) void rmsnorm_rows_f32_kernel(const float* __res
   const int r = blockIdx.x;
   const float4* src = reinterpret_cast<const float4*>(x + (size_t)(rows ? rows[r] : r) * ldx);
   const int n4 = dim / 4;
-  float4 v[VPT];
+  const float4* w4 = reinterpret_cast<const float4*>(w);
+  float4 v[VPT], gain[VPT];                     // (the weight asked for behind the sum's barrier was one more trip to memory)
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * NT;
     v[j] = i < n4 ? src[i] : float4{0.f, 0.f, 0.f, 0.f};
+    gain[j] = i < n4 ? w4[i] : float4{0.f, 0.f, 0.f, 0.f};
   }
   float ss = 0.f;
 #pragma unroll
@@ -159,12 +161,11 @@ __global__ __launch_bounds__(NT) void rmsnorm_rows_f32_kernel(const float* __res
   }
   ss = block_sum<NT>(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)dim + eps);
-  const float4* w4 = reinterpret_cast<const float4*>(w);
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * NT;
     if (i >= n4) continue;
-    const float4 g = w4[i];
+    const float4 g = gain[j];
     const float o0 = (v[j].x * inv) * g.x, o1 = (v[j].y * inv) * g.y, o2 = (v[j].z * inv) * g.z,
                 o3 = (v[j].w * inv) * g.w;
     const size_t at = (size_t)r * ldo + (size_t)i * 4;
