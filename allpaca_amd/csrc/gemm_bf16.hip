@@ -636,14 +636,13 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
   }
   bf16_t* page = rope.cache + (size_t)rope.block_table[(size_t)seg * rope.max_blocks + pos / rope.P] * page_elems;
   // (the row's few sums of x^2 in front of its slices: behind them they were another trip to memory)
-  float rstd = 1.f, few = 0.f;
+  float rstd = 1.f;
+  floatx4 few = floatx4{0.f, 0.f, 0.f, 0.f};
   const bool few_parts = PRE && norm.pre_parts <= WAVE;
-  if (few_parts && lane < norm.pre_parts) few = norm.pre_ss[(size_t)m * norm.pre_parts + lane];
+  if (few_parts) few = row_parts_ask(norm.pre_ss + (size_t)m * norm.pre_parts, norm.pre_parts, lane);
   floatx4 g = fin_sum(partials + (size_t)m * N, plane, k_split, n, N);
   if (few_parts) {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o /= 2) few += __shfl_xor(few, o, WAVE);
-    rstd = 1.0f / sqrtf(few / (float)K + norm.eps);
+    rstd = 1.0f / sqrtf(row_parts_few_sum<WAVE>(few) / (float)K + norm.eps);
   } else if (PRE) {
     rstd = fin_rstd(norm, m, lane, K);
   }

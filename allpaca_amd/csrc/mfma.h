@@ -54,6 +54,13 @@ __device__ __forceinline__ floatx16 mfma32(const Frag& a, const Frag& b, floatx1
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
 }
 
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float sum) {
+#pragma unroll
+  for (int o = LANES / 2; o > 0; o /= 2) sum += __shfl_xor(sum, o, WAVE);
+  return sum;
+}
+
 // The sum of a row's `parts` sums of x^2 over the LANES lanes side by side that share the row (every lane gets it; `j`: which
 // of them this is).  Eight loads of four values a lane are in flight: 256 parts of 64 rows read 8 values at a time by a
 // thread a row held the tiled product's first step up by 9 us, and one value at a time by eight lanes by 2-3.
@@ -80,10 +87,22 @@ __device__ __forceinline__ float row_parts_sum(const float* __restrict__ row, in
       for (int k = 0; k < 8; ++k) sum += v[k];
     }
   }
-#pragma unroll
-  for (int o = LANES / 2; o > 0; o /= 2) sum += __shfl_xor(sum, o, WAVE);
-  return sum;
+  return lanes_sum<LANES>(sum);
 }
+
+// The same for up to LANES parts in two halves, so that the loads can stand in front of others: what lane j asks for, and the
+// sum, which is row_parts_sum's to the bit.
+__device__ __forceinline__ floatx4 row_parts_ask(const float* __restrict__ row, int parts, int j) {
+  floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (parts % 4 == 0 && ((uintptr_t)row & 15u) == 0) {
+    if (j * 4 < parts) v = *reinterpret_cast<const floatx4*>(row + j * 4);
+  } else if (j < parts) {
+    v[0] = row[j];
+  }
+  return v;
+}
+template <int LANES>
+__device__ __forceinline__ float row_parts_few_sum(const floatx4& v) { return lanes_sum<LANES>((v[0] + v[1]) + (v[2] + v[3])); }
 
 __device__ __forceinline__ float silu_f(float g) { return g / (1.0f + __expf(-g)); }
 // An activation by code: 1 silu, 2 the square of max(z, 0), 3 gelu in its tanh form (tanh by one exponential, off by

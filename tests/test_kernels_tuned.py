@@ -662,6 +662,41 @@ def test_product_for_q_k_v_that_rotates_and_fills_the_pages_equals_the_kernels_o
     assert (results[0][1] != 0).sum() + (results[0][2] != 0).sum() == M * 2 * Hk * d   # every row wrote its k and v, once
 
 
+# parts: sums of x^2 a row, asked for ahead of the slices up to 64, four a lane or (no multiple of 4) one; off: floats in front of
+# the table of angles, which are then read one by one
+@pytest.mark.parametrize("M,H,Hk,d,K,parts,off", [(300, 4, 2, 256, 2048, 8, 0), (257, 24, 8, 128, 4096, 16, 0), (512, 4, 2, 128, 2304, 9, 1),
+                                                  (130, 6, 1, 64, 1024, 64, 2), (129, 8, 4, 64, 2048, 72, 0), (200, 4, 2, 128, 1024, 130, 3)])
+def test_q_k_and_v_are_scaled_as_any_product_behind_the_norm(M, H, Hk, d, K, parts, off):
+    """With angles of zero the finishing kernel of q, k and v leaves the bits that the product behind the norm leaves: the
+    same slices, the row's sums of x^2 added in the same order (v's blocks share a row among other lanes)."""
+    from allpaca_amd.kernels import ops
+    t, P_, eps = tuned(), 16, 2e-5
+    rng = np.random.default_rng(M + parts)
+    N = (H + 2 * Hk) * d
+    w, a = pack(gen(N, K, seed=3, dtype=BF).to(DEV)), gen(M, K, seed=1, dtype=BF, scale=2.0).to(DEV)
+    ss = torch.from_numpy(rng.uniform(0.5, 40.0, (M, parts)).astype(np.float32)).to(DEV)
+    blocks = -(-M // P_) + 1
+    flat = torch.zeros(blocks * P_ * d + off, device=DEV)
+    table = flat[off:].view(blocks * P_, 2, d // 2)
+    table[:, 0] = 1.0
+    pos, seg = torch.arange(M, dtype=torch.int32, device=DEV), torch.zeros(M, dtype=torch.int32, device=DEV)
+    bt = torch.from_numpy(rng.permutation(blocks).astype(np.int32)).view(1, -1).to(DEV)
+    cache = torch.zeros(blocks, 2, Hk, P_, d, dtype=BF, device=DEV)
+    q, want = torch.empty(M, N, dtype=BF, device=DEV), torch.empty(M, N, dtype=BF, device=DEV)
+    assert ops.qkv_rope_write(a, (ss, eps), w, q, H, Hk, d, table, pos, seg, bt, cache, P_)
+    assert t.gemm_pre_bf16(a, ss, eps, w, want)
+    page, slot = bt[0][pos.long() // P_].long(), pos.long() % P_
+    keys = cache[page, 0, :, slot].reshape(M, Hk * d)
+    values = cache[:, 1].reshape(blocks, Hk, d, P_)[page, :, :, slot].reshape(M, Hk * d)
+    assert torch.equal(q[:, :H * d], want[:, :H * d])
+    assert torch.equal(keys, want[:, H * d:(H + Hk) * d])
+    v = want[:, (H + Hk) * d:]
+    if parts % 4 == 0 and parts <= 64:
+        assert torch.equal(values, v)
+    else:      # two orders of at most 130 positive sums: 2^-18, which moves a rounding to bfloat16 by one unit at most
+        assert ((values.float() - v.float()).abs() <= 2.0 ** -7 * v.float().abs()).all()
+
+
 @pytest.mark.parametrize("M,H,Hk,d,K,P_,pre,off,rows", [
     # in one launch: two to four row groups, whole and not, heads of 32 to 256, 2 to 6 steps of K a wave
     (17, 6, 2, 64, 1088, 8, True, 0, True), (33, 3, 1, 32, 1024, 16, False, 0, True), (64, 4, 2, 256, 1024, 32, True, 0, True),
