@@ -179,6 +179,15 @@ def test_products_of_17_to_64_rows_in_one_launch_where_that_is_faster(kind, M, N
     assert host.load().apc_host_rule_rows_bands(M, N, K, kind) == bands
 
 
+def test_bands_of_gated_products_in_one_launch_do_not_depend_on_the_rows():
+    """Where a block begins in K depends on the bands it takes: they must not change with the rows beside a row."""
+    from allpaca_amd.kernels import host
+    rule = host.load().apc_host_rule_rows_bands
+    for N in (16, 320, 1024, 2560, 4080, 4096, 4112, 5120, 8192, 11008, 14336):
+        for K in (1024, 1536, 2048, 3072, 4096, 5440, 8192, 14336):
+            assert {rule(M, N, K, 1) for M in range(17, 65)} <= {0, 4 if N > 4096 else 2}, (N, K)
+
+
 def test_gated_products_and_the_sums_behind_a_norm_by_the_executors_rules():
     from allpaca_amd.kernels import host, tuned
     L = host.load()

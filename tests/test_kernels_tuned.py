@@ -662,6 +662,24 @@ def test_product_for_q_k_v_that_rotates_and_fills_the_pages_equals_the_kernels_o
     assert (results[0][1] != 0).sum() + (results[0][2] != 0).sum() == M * 2 * Hk * d   # every row wrote its k and v, once
 
 
+# two and four bands a block; walks of K in step and (from six steps a wave, or with four bands) from different places, waves
+# with unequal numbers of steps among them; two, three and four groups of 16 rows
+@pytest.mark.parametrize("F,K", [(2048, 1024), (4096, 2048), (1040, 3008), (4096, 3072), (5120, 1024), (8176, 1536), (8192, 3072)])
+def test_a_row_of_a_gated_product_of_17_to_64_rows_does_not_depend_on_the_others(F, K):
+    from allpaca_amd.kernels import lib
+    t, L = tuned(), lib.load("tuned")
+    a = gen(64, K, seed=1, dtype=BF).to(DEV)
+    wg, wu = pack(gen(F, K, seed=2, dtype=BF).to(DEV)), pack(gen(F, K, seed=3, dtype=BF).to(DEV))
+    outs = []
+    for M in (17, 33, 48, 64):
+        out = torch.empty(M, F, dtype=BF, device=DEV)
+        assert L.apc_gemm_rows_takes(3, a.data_ptr(), K, wg.data.data_ptr(), wu.data.data_ptr(), out.data_ptr(), F, M, F, K)
+        t.swiglu_bf16(a[:M], wg, wu, out)
+        outs.append(out)
+    for out in outs[:-1]:
+        assert torch.equal(out, outs[-1][:out.shape[0]])
+
+
 # parts: sums of x^2 a row, asked for ahead of the slices up to 64, four a lane or (no multiple of 4) one; off: floats in front of
 # the table of angles, which are then read one by one
 @pytest.mark.parametrize("M,H,Hk,d,K,parts,off", [(300, 4, 2, 256, 2048, 8, 0), (257, 24, 8, 128, 4096, 16, 0), (512, 4, 2, 128, 2304, 9, 1),
