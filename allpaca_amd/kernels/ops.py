@@ -4,6 +4,7 @@ what the kernel and its grid assume, and launches on torch's current stream.
 Nothing here computes on the CPU and nothing falls back to a library."""
 from __future__ import annotations
 
+import collections
 import functools
 import math
 import os
@@ -238,13 +239,35 @@ def argmax_rows(logits: torch.Tensor, out: torch.Tensor) -> None:
 OPTIONS_ON_HOST = 64     # rows whose options `sample_rows` takes as lists
 
 
+_still_written: collections.deque = collections.deque()   # (memory, events) of `PinnedIds` that are gone
+
+
 class PinnedIds:
-    """Host memory for token ids that a kernel may write (int32 [n])."""
-    __slots__ = ("tensor", "size", "address")
+    """Host memory for token ids that a kernel may write (int32 [n]).  The allocator of pinned memory does not know of a kernel
+    that got the address, and would hand the block on as soon as nobody holds it; so whoever launches such a kernel calls
+    `queued()` behind it, and a block that is dropped is kept until the kernels of every stream are through.  (Events are asked
+    only where new memory is pinned, not where an object happens to be collected: a stream may be recording a graph then.)"""
+    __slots__ = ("tensor", "size", "address", "events")
 
     def __init__(self, n: int):
+        self.events = {}                      # of the last kernel of each stream
+        for _ in range(len(_still_written)):
+            gone = _still_written.popleft()
+            if not all(e.query() for e in gone[1]):
+                _still_written.append(gone)
         self.tensor = torch.empty(n, dtype=torch.int32).pin_memory()
         self.size, self.address = n, self.tensor.data_ptr()
+
+    def queued(self) -> torch.cuda.Event:
+        """A kernel that writes here has been queued on the current stream: the event behind it."""
+        done = torch.cuda.Event()
+        done.record()
+        self.events[_stream()] = done
+        return done
+
+    def __del__(self, keep=_still_written.append):
+        if self.events:
+            keep((self.tensor, list(self.events.values())))
 
 
 @functools.lru_cache(maxsize=None)
@@ -254,12 +277,14 @@ def _packed_options(n: int) -> struct.Struct:
 
 def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
                 uniform: torch.Tensor, out: torch.Tensor, any_top_k: bool = True, any_top_p: bool = True,
-                few_after_top_k: bool = False, one_block: bool = False, out_host: Optional[PinnedIds] = None) -> bool:
+                few_after_top_k: bool = False, one_block: bool = False,
+                out_host: Optional[PinnedIds] = None) -> Optional[torch.cuda.Event]:
     """One token a row by temperature / top-k / top-p with the row's uniform number.  `any_top_k`, `any_top_p`: whether
     some row may ask for that cut; `few_after_top_k`: every row that samples has 0 < top-k <= 1,024.  A caller that
     knows its rows saves the launches that none of them needs; a row for which its word is wrong still gets its
     token, slowly.  `one_block`: the kernel without working memory, one block a row.  Up to 64 rows may have their
-    options as lists, and (seeds, numbers of the generated token) for the uniform numbers: they go with the launch.  The ids are then written to `out_host` too; True if they are."""
+    options as lists, and (seeds, numbers of the generated token) for the uniform numbers: they go with the launch.  The ids
+    are then written to `out_host` too: the event behind that, else None."""
     L = _lib.load("plain")
     if isinstance(temperature, list):
         _gpu(logits, out)
@@ -276,7 +301,7 @@ def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Te
                                           _packed_options(R).pack(*temperature, *top_p, *top_k, *seeds, *numbers),
                                           _i32(out, R, "sample out"), out_host.address if host else 0, scratch.data_ptr(), kib * 1024,
                                           cuts, _stream()), "sample_rows_host")
-        return host
+        return out_host.queued() if host else None
     _gpu(logits, temperature, top_k, top_p, uniform, out)
     ld = _rows(logits, "logits")
     R, V = logits.shape
@@ -292,7 +317,7 @@ def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Te
                                  (1 if any_top_k else 0) | (2 if any_top_p else 0) | (4 if few_after_top_k else 0),
                                  _stream()),
                "sample_rows")
-    return False
+    return None
 
 
 # --------------------------------------------------------------------------- dispatch

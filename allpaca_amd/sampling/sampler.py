@@ -96,7 +96,7 @@ class Sampler:
         t = self._turn
         if self._pinned[t] is None or self._pinned[t].size < R:
             self._pinned[t] = ops.PinnedIds(max(R, 64))
-        pinned, on_host = self._pinned[t], False
+        pinned, done = self._pinned[t], None
         temps = [p.temperature for p in params]
         if all(x <= 1e-5 for x in temps):
             ops.argmax_rows(logits, out)
@@ -108,12 +108,12 @@ class Sampler:
             else:
                 f = self._upload(params, indices)
                 opts = (f[0, :R], f[3, :R].view(torch.int32), f[1, :R], f[2, :R])
-            on_host = ops.sample_rows(logits, *opts, out, any_top_k=max(ks) > 0, any_top_p=any(0.0 <= x < 1.0 for x in tops),
-                                      few_after_top_k=few, out_host=pinned)
-        if not on_host:
+            done = ops.sample_rows(logits, *opts, out, any_top_k=max(ks) > 0, any_top_p=any(0.0 <= x < 1.0 for x in tops),
+                                   few_after_top_k=few, out_host=pinned)
+        if done is None:
             pinned.tensor[:R].copy_(out, non_blocking=True)
-        done = torch.cuda.Event()
-        done.record()
+            done = torch.cuda.Event()
+            done.record()
         return Pending(pinned.tensor, R, done, out)
 
     def _by_value(self, shape, temps, ks, tops) -> bool:

@@ -71,6 +71,51 @@ def test_what_the_sampler_tells_the_kernels(monkeypatch, rules, want):
     assert (seen["any_top_k"], seen["any_top_p"], seen["few_after_top_k"]) == want
 
 
+def test_memory_that_a_queued_kernel_writes_is_kept_until_it_has(monkeypatch):
+    """Token ids come back through pinned memory whose address a kernel gets.  Dropped with kernels queued, on two streams, the
+    block is given back only when both are through."""
+    import gc
+    import weakref
+
+    import torch
+    from allpaca_amd.kernels import lib, ops
+    kernels, through, stream = [], set(), [1]
+
+    class Event:
+        def record(self):
+            self.kernel = len(kernels) - 1
+
+        def query(self):
+            return self.kernel in through
+
+    L = SimpleNamespace(apc_sample_rows_scratch_kib=lambda n: 1, apc_sample_rows_host=lambda *a: kernels.append(a[6]) or 0)
+    monkeypatch.setattr(lib, "load", lambda name: L)
+    monkeypatch.setattr(ops, "_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream", lambda: stream[0])
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda self: self)
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    ids = ops.PinnedIds(64)
+    tensor, address = weakref.ref(ids.tensor), ids.address
+
+    def choose(on):
+        stream[0] = on
+        return ops.sample_rows(torch.zeros(2, 16), [0.8] * 2, [40] * 2, [0.9] * 2, ([1, 2], [0, 1]), torch.zeros(2, dtype=torch.int32), out_host=ids)
+
+    events = [choose(1), choose(2), choose(2)]
+    assert kernels == [address] * 3 and all(isinstance(e, Event) for e in events)
+    del ids
+    for done in ({2}, {0, 1}):
+        gc.collect()
+        through.clear()
+        through.update(done)
+        ops.PinnedIds(64)
+        assert tensor() is not None and tensor().data_ptr() == address
+    through.update({0, 2})
+    ops.PinnedIds(64)
+    gc.collect()
+    assert tensor() is None
+
+
 def test_entry_points_that_launch_nothing_are_not_timed_as_kernels():
     """A kernel's last argument is its stream; what has none answers a question about sizes."""
     from allpaca_amd.kernels import lib
