@@ -82,3 +82,11 @@ __device__ __forceinline__ float block_max(float v, float* smem) {
 }
 
 __host__ __device__ static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// Norms of whole rows: whether the weight is asked for ahead of the sum of squares.  With few rows it comes from behind the L2
+// and its way is a large part of the kernel; with many it is there, and the registers cost more.  Microseconds with the weight
+// behind / ahead, weights that no launch has just read: 8 rows of 2,048 rmsnorm_rows 2.78 / 2.53, rmsnorm_add 2.89 / 2.67, of 4,096
+// 3.46 / 3.08 and 3.62 / 3.32; 177 rows of 8,192 4.97 / 4.45 and 5.97 / 5.57, gated 8.83 / 8.36; 512 rows 5.85 / 5.74 and 8.60 /
+// 8.55, gated 10.2 / 10.7; 2,048 rows of 2,048 4.45 / 4.55 and 7.43 / 7.78; rows of 1,024 (a load a thread) 1.80 / 1.81 and
+// 1.92 / 2.03.
+static inline bool norm_weight_ahead(int n_rows, int dim) { return n_rows <= 256 && dim > 1024; }

@@ -130,10 +130,10 @@ __global__ void rmsnorm_rows_kernel(const void* __restrict__ x, int x_dtype, int
 }
 
 // The same for float32 rows whose width is a multiple of 4 and at most NT*4*VPT: every thread keeps its
-// elements in registers between the sum and the scaling, and all its loads are in flight together.
-// Which of the two kernels runs, and so the order of the additions, is fixed by the width and the
+// elements in registers between the sum and the scaling, and all its loads are in flight together (AHEAD: the weight's too,
+// see norm_weight_ahead).  Which of the two kernels runs, and so the order of the additions, is fixed by the width and the
 // alignment of the rows alone, never by the batch.
-template <int NT, int VPT>
+template <int NT, int VPT, bool AHEAD>
 __global__ __launch_bounds__(NT) void rmsnorm_rows_f32_kernel(const float* __restrict__ x, int ldx,
                                                               const int* __restrict__ rows,
                                                               const float* __restrict__ w, float eps,
@@ -144,12 +144,12 @@ __global__ __launch_bounds__(NT) void rmsnorm_rows_f32_kernel(const float* __res
   const float4* src = reinterpret_cast<const float4*>(x + (size_t)(rows ? rows[r] : r) * ldx);
   const int n4 = dim / 4;
   const float4* w4 = reinterpret_cast<const float4*>(w);
-  float4 v[VPT], gain[VPT];                     // (the weight asked for behind the sum's barrier was one more trip to memory)
+  float4 v[VPT], gain[VPT];
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * NT;
     v[j] = i < n4 ? src[i] : float4{0.f, 0.f, 0.f, 0.f};
-    gain[j] = i < n4 ? w4[i] : float4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (AHEAD) gain[j] = i < n4 ? w4[i] : float4{0.f, 0.f, 0.f, 0.f};
   }
   float ss = 0.f;
 #pragma unroll
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_rows_f32_kernel(const float* __res
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * NT;
     if (i >= n4) continue;
-    const float4 g = gain[j];
+    const float4 g = AHEAD ? gain[j] : w4[i];
     const float o0 = (v[j].x * inv) * g.x, o1 = (v[j].y * inv) * g.y, o2 = (v[j].z * inv) * g.z,
                 o3 = (v[j].w * inv) * g.w;
     const size_t at = (size_t)r * ldo + (size_t)i * 4;
@@ -188,13 +188,14 @@ APC_EXPORT int apc_rmsnorm_rows(const void* x, int x_dtype, int ldx, const int* 
                    ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)out % 16) == 0;
   if (vec) {
     const int n4 = dim / 4;
-#define RN_LAUNCH(VPT_)                                                                                             \
-  hipLaunchKernelGGL((rmsnorm_rows_f32_kernel<256, VPT_>), dim3(n_rows), dim3(256), 0, stream, (const float*)x, ldx, \
+#define RN_LAUNCH(VPT_, AHEAD_)                                                                                             \
+  hipLaunchKernelGGL((rmsnorm_rows_f32_kernel<256, VPT_, AHEAD_>), dim3(n_rows), dim3(256), 0, stream, (const float*)x, ldx, \
                      rows, w, eps, out, out_dtype, ldo, dim)
-    if (n4 <= 256) RN_LAUNCH(1);
-    else if (n4 <= 512) RN_LAUNCH(2);
-    else if (n4 <= 1024) RN_LAUNCH(4);
-    else RN_LAUNCH(8);
+    const bool ahead = norm_weight_ahead(n_rows, dim);
+    if (n4 <= 256) RN_LAUNCH(1, false);
+    else if (n4 <= 512) { if (ahead) RN_LAUNCH(2, true); else RN_LAUNCH(2, false); }
+    else if (n4 <= 1024) { if (ahead) RN_LAUNCH(4, true); else RN_LAUNCH(4, false); }
+    else { if (ahead) RN_LAUNCH(8, true); else RN_LAUNCH(8, false); }
 #undef RN_LAUNCH
   } else {
     hipLaunchKernelGGL(rmsnorm_rows_kernel<256>, dim3(n_rows), dim3(256), 0, stream, x, x_dtype, ldx, rows, w, eps,

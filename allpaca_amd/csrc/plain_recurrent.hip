@@ -52,11 +52,11 @@ __global__ __launch_bounds__(NT) void rmsnorm_add_kernel(const void* __restrict_
 }
 
 // The same for float32 rows whose width is a multiple of 4 and at most NT*4*VPT: every thread keeps its elements of
-// y in registers between the sum and the scaling, and all its loads are in flight together, the weight's too: asked for
-// behind the sum's barrier it was one more trip to memory (8 rows of 2,048: 3.54 -> 3.46 us, 177 rows 3.91 -> 3.72).
+// y in registers between the sum and the scaling, and all its loads are in flight together; with AHEAD (norm_weight_ahead) the
+// weight's too: asked for behind the sum's barrier it is one more trip to memory.
 // Which of the two kernels runs, and so the order of the additions, is fixed by the width and the alignment of the rows
 // alone.
-template <int NT, int VPT>
+template <int NT, int VPT, bool AHEAD>
 __global__ __launch_bounds__(NT) void rmsnorm_add_f4_kernel(const float* __restrict__ y, int ldy,
                                                             const float* __restrict__ w, float eps, float mult,
                                                             float* __restrict__ x, int ldx, void* __restrict__ copy,
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_add_f4_kernel(const float* __restr
     const int i = threadIdx.x + j * NT;
     v[j] = i < n4 ? src[i] : float4{0.f, 0.f, 0.f, 0.f};
     old[j] = i < n4 ? xr[i] : float4{0.f, 0.f, 0.f, 0.f};
-    gain[j] = i < n4 ? w4[i] : float4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (AHEAD) gain[j] = i < n4 ? w4[i] : float4{0.f, 0.f, 0.f, 0.f};
   }
   float ss = 0.f;
 #pragma unroll
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_add_f4_kernel(const float* __restr
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * NT;
     if (i >= n4) continue;
-    const float4 g = gain[j];
+    const float4 g = AHEAD ? gain[j] : w4[i];
     const float4 nx = float4{old[j].x + mult * ((v[j].x * inv) * g.x), old[j].y + mult * ((v[j].y * inv) * g.y),
                              old[j].z + mult * ((v[j].z * inv) * g.z), old[j].w + mult * ((v[j].w * inv) * g.w)};
     xr[i] = nx;
@@ -212,8 +212,8 @@ __global__ __launch_bounds__(64) void gated_groupnorm_kernel(const float* __rest
 }
 
 // The same on 16-byte accesses for groups whose size is a multiple of 4 and at most 1,024: L lanes (a power of two) a
-// group, several groups a wave, a lane's elements in registers between the sum and the scaling.  Weight and gate are asked
-// for with them, ahead of the sum (8 rows of 16 groups of 128: 3.76 -> 3.61 us).
+// group, several groups a wave, a lane's elements in registers between the sum and the scaling.  (Weight and gate asked for ahead
+// of the sum: 8 rows of 1,024 in groups of 128 2.62 -> 2.94 us, of 4,096 3.25 -> 3.34, 2,048 rows 6.5 -> 6.9.)
 __global__ __launch_bounds__(256) void gated_groupnorm_f4_kernel(const float* __restrict__ o, int ldo_in,
                                                                  const float* __restrict__ w, float eps,
                                                                  const void* __restrict__ gate, int gate_dtype, int ldg,
@@ -225,28 +225,12 @@ __global__ __launch_bounds__(256) void gated_groupnorm_f4_kernel(const float* __
   const long r = on ? g / per_row : 0;
   const int c0 = on ? (int)(g % per_row) * group : 0;
   constexpr int VPT = 4;
-  float4 v[VPT], gain[VPT], g4[VPT];
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const int i = (l + j * L) * 4;
-    const bool in = on && i < group;
-    v[j] = i < group ? *reinterpret_cast<const float4*>(o + r * ldo_in + c0 + i) : float4{0.f, 0.f, 0.f, 0.f};
-    gain[j] = in && w ? *reinterpret_cast<const float4*>(w + c0 + i) : float4{1.f, 1.f, 1.f, 1.f};
-    g4[j] = float4{0.f, 0.f, 0.f, 0.f};
-    if (in && gate) {
-      const size_t at = (size_t)r * ldg + c0 + i;
-      if (gate_dtype == APC_F32) {
-        g4[j] = *reinterpret_cast<const float4*>((const float*)gate + at);
-      } else {
-        const uint2 q = *reinterpret_cast<const uint2*>((const bf16_t*)gate + at);
-        g4[j] = float4{__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xffff0000u), __uint_as_float(q.y << 16),
-                       __uint_as_float(q.y & 0xffff0000u)};
-      }
-    }
-  }
+  float4 v[VPT];
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
+    const int i = (l + j * L) * 4;
+    v[j] = i < group ? *reinterpret_cast<const float4*>(o + r * ldo_in + c0 + i) : float4{0.f, 0.f, 0.f, 0.f};
     ss = fmaf(v[j].x, v[j].x, ss);
     ss = fmaf(v[j].y, v[j].y, ss);
     ss = fmaf(v[j].z, v[j].z, ss);
@@ -260,10 +244,20 @@ __global__ __launch_bounds__(256) void gated_groupnorm_f4_kernel(const float* __
     if (!on || i >= group) continue;
     float a[4] = {v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv};
     if (w) {
-      a[0] *= gain[j].x; a[1] *= gain[j].y; a[2] *= gain[j].z; a[3] *= gain[j].w;
+      const float4 ww = *reinterpret_cast<const float4*>(w + c0 + i);
+      a[0] *= ww.x; a[1] *= ww.y; a[2] *= ww.z; a[3] *= ww.w;
     }
     if (gate) {
-      const float z[4] = {g4[j].x, g4[j].y, g4[j].z, g4[j].w};
+      float z[4];
+      const size_t at = (size_t)r * ldg + c0 + i;
+      if (gate_dtype == APC_F32) {
+        const float4 q = *reinterpret_cast<const float4*>((const float*)gate + at);
+        z[0] = q.x; z[1] = q.y; z[2] = q.z; z[3] = q.w;
+      } else {
+        const uint2 q = *reinterpret_cast<const uint2*>((const bf16_t*)gate + at);
+        z[0] = __uint_as_float(q.x << 16); z[1] = __uint_as_float(q.x & 0xffff0000u);
+        z[2] = __uint_as_float(q.y << 16); z[3] = __uint_as_float(q.y & 0xffff0000u);
+      }
 #pragma unroll
       for (int x = 0; x < 4; ++x) a[x] *= gate_kind == 1 ? z[x] * sigmoid_f(z[x]) : sigmoid_f(z[x]);
     }
@@ -302,9 +296,9 @@ __global__ __launch_bounds__(NT) void gated_rmsnorm_kernel(const float* __restri
 }
 
 // The same for rows whose width is a multiple of 4 and at most NT * 4 * VPT, on 16-byte loads: a thread keeps its elements
-// between the sum and the scaling, and all its loads are in flight together.  Which of the two kernels runs is fixed by
-// the width and the alignment of the rows alone.
-template <int NT, int VPT>
+// between the sum and the scaling, and all its loads are in flight together (AHEAD: the weight's too, see norm_weight_ahead).
+// Which of the two kernels runs is fixed by the width and the alignment of the rows alone.
+template <int NT, int VPT, bool AHEAD>
 __global__ __launch_bounds__(NT) void gated_rmsnorm_f4_kernel(const float* __restrict__ o, int ldo_in,
                                                               const float* __restrict__ w, float eps,
                                                               const void* __restrict__ gate, int gate_dtype, int ldg,
@@ -316,7 +310,7 @@ __global__ __launch_bounds__(NT) void gated_rmsnorm_f4_kernel(const float* __res
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * NT;
     v[j] = i < n4 ? reinterpret_cast<const float4*>(o + (size_t)r * ldo_in)[i] : float4{0.f, 0.f, 0.f, 0.f};
-    gain[j] = i < n4 ? reinterpret_cast<const float4*>(w)[i] : float4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (AHEAD) gain[j] = i < n4 ? reinterpret_cast<const float4*>(w)[i] : float4{0.f, 0.f, 0.f, 0.f};
     g[j] = float4{0.f, 0.f, 0.f, 0.f};
     if (gate && i < n4) {
       const size_t at = (size_t)r * ldg + (size_t)i * 4;
@@ -343,7 +337,7 @@ __global__ __launch_bounds__(NT) void gated_rmsnorm_f4_kernel(const float* __res
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * NT;
     if (i >= n4) continue;
-    const float4 wv = gain[j];
+    const float4 wv = AHEAD ? gain[j] : reinterpret_cast<const float4*>(w)[i];
     float4 y = float4{(v[j].x * inv) * wv.x, (v[j].y * inv) * wv.y, (v[j].z * inv) * wv.z, (v[j].w * inv) * wv.w};
     if (gate) {
       y.x *= sigmoid_f(g[j].x);
@@ -409,13 +403,14 @@ APC_EXPORT int apc_rmsnorm_add(const void* y, int y_dtype, int ldy, const float*
                    ((uintptr_t)w % 16) == 0 && ((uintptr_t)copy % 16) == 0;
   if (vec) {
     const int n4 = dim / 4;
-#define RA_LAUNCH(VPT_)                                                                                          \
-  hipLaunchKernelGGL((rmsnorm_add_f4_kernel<256, VPT_>), dim3(n_rows), dim3(256), 0, stream, (const float*)y, ldy, \
+#define RA_LAUNCH(VPT_, AHEAD_)                                                                                          \
+  hipLaunchKernelGGL((rmsnorm_add_f4_kernel<256, VPT_, AHEAD_>), dim3(n_rows), dim3(256), 0, stream, (const float*)y, ldy, \
                      w, eps, mult, x, ldx, copy, copy_dtype, ldc, dim)
-    if (n4 <= 256) RA_LAUNCH(1);
-    else if (n4 <= 512) RA_LAUNCH(2);
-    else if (n4 <= 1024) RA_LAUNCH(4);
-    else RA_LAUNCH(8);
+    const bool ahead = norm_weight_ahead(n_rows, dim);
+    if (n4 <= 256) RA_LAUNCH(1, false);
+    else if (n4 <= 512) { if (ahead) RA_LAUNCH(2, true); else RA_LAUNCH(2, false); }
+    else if (n4 <= 1024) { if (ahead) RA_LAUNCH(4, true); else RA_LAUNCH(4, false); }
+    else { if (ahead) RA_LAUNCH(8, true); else RA_LAUNCH(8, false); }
 #undef RA_LAUNCH
   } else {
     hipLaunchKernelGGL(rmsnorm_add_kernel<256>, dim3(n_rows), dim3(256), 0, stream, y, y_dtype, ldy, w, eps, mult, x,
@@ -478,13 +473,14 @@ APC_EXPORT int apc_gated_rmsnorm(const float* o, int ldo_in, const float* w, flo
   }
   if (dim % 4 == 0 && dim <= 256 * 4 * 8 && ldo_in % 4 == 0 && ldo % 4 == 0 && aligned(o, APC_F32) && aligned(w, APC_F32) &&
       aligned(out, out_dtype) && (!gate || (ldg % 4 == 0 && aligned(gate, gate_dtype)))) {
-#define GATED_LAUNCH(VPT_)                                                                                               \
-  hipLaunchKernelGGL((gated_rmsnorm_f4_kernel<256, VPT_>), dim3(n_rows), dim3(256), 0, stream, o, ldo_in, w, eps, gate, \
+#define GATED_LAUNCH(VPT_, AHEAD_)                                                                                               \
+  hipLaunchKernelGGL((gated_rmsnorm_f4_kernel<256, VPT_, AHEAD_>), dim3(n_rows), dim3(256), 0, stream, o, ldo_in, w, eps, gate, \
                      gate_dtype, ldg, out, out_dtype, ldo, dim)
-    if (dim <= 1024) GATED_LAUNCH(1);
-    else if (dim <= 2048) GATED_LAUNCH(2);
-    else if (dim <= 4096) GATED_LAUNCH(4);
-    else GATED_LAUNCH(8);
+    const bool ahead = norm_weight_ahead(n_rows, dim);
+    if (dim <= 1024) GATED_LAUNCH(1, false);
+    else if (dim <= 2048) { if (ahead) GATED_LAUNCH(2, true); else GATED_LAUNCH(2, false); }
+    else if (dim <= 4096) { if (ahead) GATED_LAUNCH(4, true); else GATED_LAUNCH(4, false); }
+    else { if (ahead) GATED_LAUNCH(8, true); else GATED_LAUNCH(8, false); }
 #undef GATED_LAUNCH
     APC_LAUNCH_CHECK();
     return 0;

@@ -68,6 +68,30 @@ def test_rmsnorm(D):
     close(f64(sel), P.rms_norm(f64(x)[[6, 0]], f64(w), 1e-5), atol=1e-5, rtol=1e-5)
 
 
+# one load of the weight a thread, two, four and eight, the last of them not by every thread; the weight behind the sum (513 rows,
+# or up to 1,024 columns) and ahead of it (a row alone)
+@pytest.mark.parametrize("D", [1024, 1028, 2048, 2052, 4100, 8192])
+def test_norms_of_many_rows_are_those_of_a_row_alone(D):
+    o = ops()
+    x, res = gen(513, D, seed=D, scale=3.0).to(DEV), gen(513, D, seed=2).to(DEV)
+    w, gate = (1 + 0.1 * gen(D, seed=1)).to(DEV), gen(513, D, seed=3, dtype=torch.bfloat16).to(DEV)
+
+    def all_three(r0, r1):
+        out, gated, added = torch.empty(r1 - r0, D, device=DEV), torch.empty(r1 - r0, D, device=DEV), res[r0:r1].clone()
+        o.rmsnorm_rows(x[r0:r1], w, 1e-5, out)
+        o.gated_rmsnorm(x[r0:r1], w, 1e-5, gate[r0:r1], gated)
+        o.rmsnorm_add(x[r0:r1], w, 1e-5, 0.5, added)
+        return out, gated, added
+
+    many = all_three(0, 513)
+    h = P.rms_norm(f64(x), f64(w), 1e-5)
+    for got, want in zip(many, (h, h / (1.0 + np.exp(-f64(gate))), f64(res) + 0.5 * h)):
+        close(f64(got), want, atol=1e-5, rtol=1e-5)
+    for r in (0, 511, 512):
+        for got, alone in zip(many, all_three(r, r + 1)):
+            assert torch.equal(got[r], alone[0])
+
+
 def test_rmsnorm_reference_vector_and_zero():
     o = ops()
     x = torch.tensor([[3.0, 4.0], [0.0, 0.0]], device=DEV)
