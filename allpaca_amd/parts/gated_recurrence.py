@@ -20,6 +20,11 @@ from .base import MIXERS, FixedState, Mixer, Runtime, as_normed, to_device
 from .spec import ParamSpec
 
 RATE = -8.0      # log a at r = 1, in units of softplus(lam)
+# Widest part whose decoded rows go through convolution, gates and recurrence in one launch.  A part is one block there, which
+# reads all of its gates: 2 w^2 weights, 64 KB at 128.  Three launches / one, us, 1, 8 and 16 rows, four taps: 32 parts of 32
+# channels 8.3 / 5.9, 8.9 / 4.7, 9.1 / 5.0; 8 of 64 7.7 / 7.6, 8.2 / 5.0, 8.4 / 5.6; 16 of 128 10.1 / 8.0, 10.7 / 6.8, 11.0 / 8.4;
+# 8 of 256 10.3 / 11.4, 11.0 / 11.5, 11.4 / 15.2.
+ONE_LAUNCH_WIDTH = 128
 
 
 @MIXERS.register("gated_recurrence")
@@ -85,9 +90,9 @@ class GatedRecurrence(Mixer):
         if state is None or not state.writes:
             raise ValueError("a recurrent mixer needs a state of its own")
         T, dev, C = proj.shape[0], proj.device, self.C
-        if conv is not None and ops.recurrent_step(proj[:, C:2 * C], proj[:, :C], self.x_b, self.conv_w, self.conv_b, conv.state, conv.slots,
-                                                   self.w_gates, self.gates_b, self.B, self.rate, self.y_b, state.state, state.slots,
-                                                   step, out, scale):
+        if conv is not None and self.w <= ONE_LAUNCH_WIDTH and ops.recurrent_step(
+                proj[:, C:2 * C], proj[:, :C], self.x_b, self.conv_w, self.conv_b, conv.state, conv.slots, self.w_gates, self.gates_b,
+                self.B, self.rate, self.y_b, state.state, state.slots, step, out, scale):
             return
         u = torch.empty((T, C), dtype=self.rt.dtype, device=dev)
         ops.conv_channels(proj[:, C:], C, self.conv_w, self.conv_b, conv.state if conv is not None else None, step,

@@ -116,6 +116,24 @@ def test_memory_that_a_queued_kernel_writes_is_kept_until_it_has(monkeypatch):
     assert tensor() is None
 
 
+@pytest.mark.parametrize("parts,one", [(64, True), (32, True), (16, True), (8, False), (1, False)])
+def test_gated_recurrence_in_one_launch_for_parts_of_up_to_128_channels(monkeypatch, parts, one):
+    """A block reads all gates of a part: of 256 channels three launches are faster (parts of 32 to 2,048 channels here)."""
+    import torch
+    from allpaca_amd.kernels import ops
+    from allpaca_amd.parts.gated_recurrence import GatedRecurrence
+    C, went = 2048, []
+    monkeypatch.setattr(ops, "recurrent_step", lambda *a: went.append("one") or True)
+    for name in ("conv_channels", "heads_linear", "gated_recurrence"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, **kw: went.append(name))
+    mixer = SimpleNamespace(C=C, B=parts, w=C // parts, rt=SimpleNamespace(dtype=torch.bfloat16),
+                            **{n: None for n in ("x_b", "y_b", "conv_w", "conv_b", "w_gates", "gates_b", "rate")})
+    view = SimpleNamespace(writes=True, state=None, slots=None)
+    proj, out = torch.zeros(2, 2 * C, dtype=torch.bfloat16), torch.zeros(2, C, dtype=torch.bfloat16)
+    GatedRecurrence.core(mixer, proj, None, {"mixer": view, "mixer.state": view}, out)
+    assert went == (["one"] if one else ["conv_channels", "heads_linear", "gated_recurrence"])
+
+
 def test_entry_points_that_launch_nothing_are_not_timed_as_kernels():
     """A kernel's last argument is its stream; what has none answers a question about sizes."""
     from allpaca_amd.kernels import lib
