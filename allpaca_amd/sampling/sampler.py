@@ -103,7 +103,7 @@ class Sampler:
         else:
             ks, tops = [p.top_k for p in params], [p.top_p for p in params]
             few = all(x <= 1e-5 or 0 < k <= 1024 for x, k in zip(temps, ks))
-            if self._by_value(logits.shape, temps, ks, tops):
+            if self._by_value(logits.shape, temps, ks, tops, indices):
                 opts = (temps, ks, tops, ([(self.default_seed if p.seed is None else p.seed) & _M64 for p in params], indices))
             else:
                 f = self._upload(params, indices)
@@ -116,10 +116,13 @@ class Sampler:
             done.record()
         return Pending(pinned.tensor, R, done, out)
 
-    def _by_value(self, shape, temps, ks, tops) -> bool:
-        """Whether the rows' options can go with the launch itself (few rows, and numbers that the kernels' types hold)."""
-        return (self.device.type == "cuda" and shape[0] <= ops.OPTIONS_ON_HOST and shape[1] <= 1 << 22 and all(abs(x) < 3e38 for x in temps)
-                and all(abs(x) < 3e38 for x in tops) and max(ks) < 1 << 31)
+    def _by_value(self, shape, temps, ks, tops, indices) -> bool:
+        """Whether the rows' options can go with the launch itself: few rows, and numbers that the kernels' types hold as they
+        are (a top-k of 40.0, which the device copy takes as 40, goes that way)."""
+        return (self.device.type == "cuda" and len(temps) == shape[0] <= ops.OPTIONS_ON_HOST and shape[1] <= 1 << 22
+                and all(abs(x) < 3e38 for x in temps) and all(abs(x) < 3e38 for x in tops)
+                and all(type(k) is int and -(1 << 31) <= k < 1 << 31 for k in ks)
+                and all(type(n) is int and 0 <= n < 1 << 63 for n in indices))
 
 
 class Pending:

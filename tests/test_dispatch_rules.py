@@ -71,6 +71,22 @@ def test_what_the_sampler_tells_the_kernels(monkeypatch, rules, want):
     assert (seen["any_top_k"], seen["any_top_p"], seen["few_after_top_k"]) == want
 
 
+@pytest.mark.parametrize("rows,k,number,by_value", [
+    (2, 40, 7, True), (64, -1, 0, True), (65, 40, 7, False), (2, (1 << 31) - 1, (1 << 63) - 1, True),
+    # what only the copy to the device takes: floats, numbers beyond a signed 64-bit one; and what it refuses
+    (2, 40.0, 7, False), (2, 40, 7.0, False), (2, 40, 1 << 63, False), (2, 1 << 31, 7, False), (2, -(1 << 31) - 1, 7, False), (2, 40, -1, False)])
+def test_options_of_few_rows_go_with_the_launch_if_its_types_hold_them(rows, k, number, by_value):
+    import torch
+    from allpaca_amd.kernels import ops
+    from allpaca_amd.sampling.sampler import Sampler
+    s = Sampler(torch.device("cuda"), 0)
+    temps, tops, ks, numbers = [0.8] * rows, [0.95] * rows, [5] * (rows - 1) + [k], [3] * (rows - 1) + [number]
+    assert s._by_value((rows, 32000), temps, ks, tops, numbers) == by_value
+    assert not s._by_value((rows - 1, 32000), temps, ks, tops, numbers)          # (more options than rows)
+    if by_value:
+        ops._packed_options(rows).pack(*temps, *tops, *ks, *range(rows), *numbers)
+
+
 def test_memory_that_a_queued_kernel_writes_is_kept_until_it_has(monkeypatch):
     """Token ids come back through pinned memory whose address a kernel gets.  Dropped with kernels queued, on two streams, the
     block is given back only when both are through."""

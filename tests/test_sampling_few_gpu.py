@@ -87,3 +87,17 @@ def test_options_that_go_with_the_launch(R, V, rule):
     for _ in range(3):                                       # (both of the sampler's result buffers)
         pending = sampler.launch(logits, params, numbers)
         assert pending.wait() == want.tolist() == pending.device.tolist()
+
+
+def test_options_that_only_the_copy_to_the_device_takes():
+    """A top-k that is a float and numbers of tokens beyond a signed 64-bit one, beside the same choice with the launch."""
+    from allpaca_amd.sampling import GenerationParams
+    from allpaca_amd.sampling.sampler import Sampler
+    logits = torch.randn(3, 5000, generator=torch.Generator(device=DEV).manual_seed(3), device=DEV) * 3
+    params = lambda k: [GenerationParams(temperature=0.9, top_k=k, top_p=0.95, seed=r) for r in range(3)]  # noqa: E731
+    s = Sampler(torch.device(DEV), 5)
+    assert s.sample(logits, params(40.0), [4, 5, 6]) == s.sample(logits, params(40), [4, 5, 6])
+    assert s.sample(logits, params(40.7), [4.0, 5, 6]) == s.sample(logits, params(40), [4, 5, 6])
+    top = (1 << 64) - 2
+    ids = s.sample(logits, params(40), [top, 1 << 63, 0])
+    assert ids[2] == s.sample(logits, params(40), [1, 2, 0])[2] and all(0 <= t < 5000 for t in ids)
