@@ -1185,7 +1185,7 @@ APC_EXPORT int apc_attention_prefill_bf16(const void* q, int ldq, int q_off, voi
   // n_rows: the rows of all tiles together.  Tiles of 64 rows and more on average go to the kernel that takes 128 rows a
   // block; with many short ones (many small requests) half of its waves would have no rows (measured at 8B shapes: 17-32
   // rows a tile 2-4 % slower than the 64-row kernel, 16 rows over 128 keys 36 %; 33-128 rows a tile 1.2-1.35 times as fast).
-  if (attn_wide_takes(d, page_tokens) && (long)n_rows * 2 >= (long)n_tiles * TILE_ROWS)
+  if (attn_wide_takes(Hk, d, page_tokens) && (long)n_rows * 2 >= (long)n_tiles * TILE_ROWS)
     return launch_attn_prefill_wide((const bf16_t*)q, ldq, q_off, (bf16_t*)out, ldo, H, Hk, (const bf16_t*)cache,
                                     page_tokens, block_table, max_blocks, positions, row_seg, tile_row0, tile_rows,
                                     n_tiles, window, scale, n_splits < 1 ? 1 : n_splits, part_rows, parts, d, stream);
@@ -1334,8 +1334,8 @@ APC_EXPORT int apc_attention_decode_last_fits(int H, int Hk, int d, int n_parts)
 
 // 1 if apc_attention_prefill_bf16 sends a step of `n_tiles` tiles with `n_rows` rows in all to the kernel of 128-row
 // blocks (the only one that cuts a tile's keys into ranges and reads `parts`), else 0.
-APC_EXPORT int apc_attention_prefill_wide_takes(int d, int page_tokens, int n_tiles, int n_rows) {
-  return (n_tiles > 0 && attn_wide_takes(d, page_tokens) && (long)n_rows * 2 >= (long)n_tiles * TILE_ROWS) ? 1 : 0;
+APC_EXPORT int apc_attention_prefill_wide_takes(int Hk, int d, int page_tokens, int n_tiles, int n_rows) {
+  return (n_tiles > 0 && attn_wide_takes(Hk, d, page_tokens) && (long)n_rows * 2 >= (long)n_tiles * TILE_ROWS) ? 1 : 0;
 }
 
 // Rows of a tile of the prefill kernels: the caller cuts every segment of several rows into tiles of at most this many

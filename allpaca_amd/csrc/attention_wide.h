@@ -5,8 +5,9 @@
 
 constexpr int ATTN_WIDE_ROWS = 128;  // rows of a tile
 
-// True for the head sizes (128 and 64) and page sizes the kernel takes (pages of a power of two, at least 16 positions).
-bool attn_wide_takes(int d, int page_tokens);
+// True for the head sizes (128 and 64) and page sizes the kernel takes (pages of a power of two, 16 to 32,768 positions and less
+// than 4 GiB).
+bool attn_wide_takes(int Hk, int d, int page_tokens);
 // Arguments as apc_attention_prefill_bf16; tiles of up to ATTN_WIDE_ROWS rows.  n_splits > 1: the keys of every tile
 // are cut into that many ranges, a block each, and a second kernel adds the ranges; `parts` then has room for
 // n_splits * part_rows * H * (d + 2) floats, part_rows being at least the largest row index of a tile + 1.

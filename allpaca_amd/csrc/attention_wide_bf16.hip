@@ -981,8 +981,10 @@ __global__ __launch_bounds__(256) void attn_wide_merge_kernel(const float* __res
 
 }  // namespace
 
-bool attn_wide_takes(int d, int page_tokens) {
-  return (d == 128 || d == 64) && page_tokens >= 16 && page_tokens <= 32768 && (page_tokens & (page_tokens - 1)) == 0;
+// (a page of 2^32 bytes or more: its place is the product of two 32-bit numbers here)
+bool attn_wide_takes(int Hk, int d, int page_tokens) {
+  return (d == 128 || d == 64) && page_tokens >= 16 && page_tokens <= 32768 && (page_tokens & (page_tokens - 1)) == 0 &&
+         (long long)4 * Hk * page_tokens * d < (1LL << 32);
 }
 
 int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, int ldo, int H, int Hk,
@@ -990,7 +992,7 @@ int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, i
                              const int* positions, const int* row_seg, const int* tile_row0, const int* tile_rows,
                              int n_tiles, int window, float scale, int n_splits, int part_rows, float* parts,
                              int d, hipStream_t stream) {
-  if (!attn_wide_takes(d, page_tokens) || (long long)4 * Hk * page_tokens * d >= (1LL << 32)) return APC_ERR_UNSUPPORTED;
+  if (!attn_wide_takes(Hk, d, page_tokens)) return APC_ERR_UNSUPPORTED;
   if (n_splits < 1 || n_splits > 8 || (n_splits > 1 && (!parts || part_rows <= 0)) ||
       (long)n_tiles * H * n_splits > 0x7fffffffL)
     return APC_ERR_BAD_ARG;

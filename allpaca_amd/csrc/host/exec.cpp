@@ -427,7 +427,7 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
   const int* table = s.table[E.group];
   const int width = s.table_width[E.group];
   if (s.n_tiles) {
-    const bool wide = P.tun.wide_tiles && apc_attention_prefill_wide_takes(d, page, s.n_tiles, T - s.n_decode);
+    const bool wide = P.tun.wide_tiles && apc_attention_prefill_wide_takes(Hk, d, page, s.n_tiles, T - s.n_decode);
     const int splits = !wide ? 1
                        : d <= 64 || (long)s.n_tiles * H > CHIP_UNITS
                            ? key_splits_by_time(s.n_tiles, T - s.n_decode, H, d, s.prompt_passes, window, P.tun.key_splits_max)

@@ -98,5 +98,5 @@ int apc_attention_decode_even_workspace(int H, int Hk, int d);
 int apc_attention_decode_last_fits(int H, int Hk, int d, int n_parts);
 int apc_attention_decode_whole_fits(int H, int Hk, int d);
 int apc_attention_prefill_tile_rows();
-int apc_attention_prefill_wide_takes(int d, int page_tokens, int n_tiles, int n_rows);
+int apc_attention_prefill_wide_takes(int Hk, int d, int page_tokens, int n_tiles, int n_rows);
 }

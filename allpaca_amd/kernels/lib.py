@@ -137,7 +137,7 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
         "apc_attention_decode_last_fits": [I, I, I, I],
         "apc_attention_decode_whole_fits": [I, I, I],
         "apc_attention_prefill_tile_rows": [],
-        "apc_attention_prefill_wide_takes": [I, I, I, I],
+        "apc_attention_prefill_wide_takes": [I, I, I, I, I],
     },
     "bench": {
         "apc_probe_read": [P, Z, P, I, I, I, P],

@@ -623,7 +623,7 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
         step.decode_shapes.add(shape)
     if step.n_tiles:
         # (only the kernel of 128-row blocks cuts keys into ranges: no room is taken for the others)
-        wide = WIDE_TILES and L.apc_attention_prefill_wide_takes(head_dim, page_tokens, step.n_tiles, T - step.n_decode_rows)
+        wide = WIDE_TILES and L.apc_attention_prefill_wide_takes(n_kv_heads, head_dim, page_tokens, step.n_tiles, T - step.n_decode_rows)
         splits = _prompt_ranges(step, T - step.n_decode_rows, n_heads, head_dim, int(window)) if wide else 1
         parts = (torch.empty(splits * T * n_heads * (head_dim + 2), dtype=torch.float32, device=q.device)
                  if splits > 1 else None)

@@ -132,6 +132,14 @@ def test_memory_that_a_queued_kernel_writes_is_kept_until_it_has(monkeypatch):
     assert tensor() is None
 
 
+@pytest.mark.parametrize("Hk,d,page,takes", [(8, 128, 16, 1), (8, 64, 32768, 1), (255, 128, 32768, 1), (256, 128, 32768, 0), (511, 64, 32768, 1),
+                                             (512, 64, 32768, 0), (2048, 128, 4096, 0), (8, 128, 65536, 0), (8, 128, 8, 0), (8, 96, 16, 0), (8, 64, 48, 0)])
+def test_pages_that_the_attention_kernel_of_128_rows_takes(Hk, d, page, takes):
+    """The question that room for ranges of keys hangs on is the dispatch's own: a page of 4 GiB goes to the narrower kernels."""
+    from allpaca_amd.kernels import lib
+    assert lib.load("tuned").apc_attention_prefill_wide_takes(Hk, d, page, 2, 256) == takes
+
+
 @pytest.mark.parametrize("parts,one", [(64, True), (32, True), (16, True), (8, False), (1, False)])
 def test_gated_recurrence_in_one_launch_for_parts_of_up_to_128_channels(monkeypatch, parts, one):
     """A block reads all gates of a part: of 256 channels three launches are faster (parts of 32 to 2,048 channels here)."""
