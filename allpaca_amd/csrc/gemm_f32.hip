@@ -448,7 +448,6 @@ bool gemm_f32_takes(const void* A, int lda, const void* W, int ldw, int K) {
 struct TileCost { int mt, nt; bool shares; double start, start_k, round, round_k; };
 template <int COUNT>
 static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, double k_shares, double k_alone, int outputs) {   // outputs: of 16 nt columns
-  if (M <= 16) return 0;                                // (the other tiles multiply rows that are not there)
   int best = 0;
   double best_cost = 1e30;
   for (int i = 0; i < COUNT; ++i) {
@@ -468,13 +467,16 @@ static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, double k_sh
 // K = 2,048, 2,048 outputs take 10.1 us at 33 rows (32 x 16 tiles; 32 x 32 13.1, 48 x 32 17.1), 13.3 at 100 (32 x 32;
 // 32 x 16: 15.6), 29.5 at 325 (48 x 64; 48 x 32: 31.8, 64 x 64: 38.2), 39 at 400 and 146 at 2,048 rows (64 x 64; 48 x 64:
 // 55, 159).
-// Up to K = 128 (see launch_slices) blocks of all tiles share their units.
+// Up to K = 128 (see launch_slices) blocks of all tiles share their units, and with many outputs tiles that leave the empty
+// slices out are the better ones for few rows too: 16 rows x 128,256 outputs, 32 x 32 / 16 x 16 tiles, K = 32 10.4 / 19.6 us, 64
+// 13.1 / 22.6, 128 22.2 / 25.7; 32,768 outputs 4.5 / 6.7, 5.2 / 7.1.
 constexpr TileCost TILES[] = {{1, 1, true, 2.1, 0.5, 0.5, 4.7},    {2, 1, true, 2.1, 0.9, 0.5, 5.9},   {2, 2, false, 2.4, 0.5, 1.1, 9.0},
                               {3, 2, false, 2.3, 0.4, 1.5, 12.7}, {3, 4, false, 2.4, 0.4, 2.6, 23.5}, {4, 4, false, 2.0, 0.6, 4.3, 30.7}};
 constexpr TileCost TILES_SHORT[] = {{1, 1, true, 3.6, 0.0, 0.75, 0.0}, {2, 1, true, 3.6, 0.0, 0.95, 0.0}, {2, 2, true, 4.1, 0.0, 0.69, 0.0},
                                     {3, 2, true, 4.4, 0.0, 0.93, 0.0}};        // (48 x 64 and 64 x 64 are never the least)
 static int tile_of(int M, int N, int K) {
   if (K <= 4 * STAGE) return least_cost(TILES_SHORT, M, N, K, K, 16);
+  if (M <= 16) return 0;                                // (the other tiles multiply rows that are not there)
   // a K between two multiples of 256 leaves waves with a stage less than the others: 480 rows x 2,048 outputs at K = 256,
   // 320, 512 take 11.4, 14.4, 16.6 us on 32 x 16 tiles and 12.6, 17.8, 18.9 on 48 x 64
   const int over = SLICES * STAGE * ceil_div(K, SLICES * STAGE) - K;
@@ -516,8 +518,10 @@ int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dt
 // C[M,N] = rmsnorm(A; G, eps) . W^T.  Up to 16 rows in one launch: 4 rows x 3,072 outputs x K 2,048 6.9 us without the norm, 7.6
 // with it, and the norm's own launch was 4.7; 6,144 x K 4,096 19.8 and 21.0.  More rows need room for M rows of K and their
 // scales: apc_gemm_norm_f32_kib(M, K) KiB.  A row's outputs do not depend on the rows beside it, nor on M.
-static bool norm_in_product(int M, int K) { return M <= 16 && K <= NORM_K; }
-APC_EXPORT int apc_gemm_norm_f32_kib(int M, int K) { return norm_in_product(M, K) ? 0 : (int)(((long long)M * (K + 1) * 4 + 1023) / 1024); }
+static bool norm_in_product(int M, int K, int tile) { return M <= 16 && K <= NORM_K && tile == 0; }
+APC_EXPORT int apc_gemm_norm_f32_kib(int M, int K) {
+  return M <= 16 && K > 4 * STAGE && K <= NORM_K ? 0 : (int)(((long long)M * (K + 1) * 4 + 1023) / 1024);
+}
 APC_EXPORT int apc_gemm_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int K) {
   return gemm_f32_takes(A, lda, W, ldw, K) && G && ((uintptr_t)G & 15u) == 0;
 }
@@ -534,7 +538,7 @@ APC_EXPORT int apc_gemm_norm_f32(const void* A, int lda, const void* G, float ep
   if (K <= 0 || lda < K || ldw < K || ldc < N) return APC_ERR_BAD_ARG;
   if (!apc_gemm_norm_f32_takes(A, lda, G, W, ldw, K)) return APC_ERR_UNSUPPORTED;
   const float *a = (const float*)A, *g = (const float*)G, *w = (const float*)W;
-  if (norm_in_product(M, K)) return product(a, lda, g, eps, nullptr, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
+  if (norm_in_product(M, K, tile_of(M, N, K))) return product(a, lda, g, eps, nullptr, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
   float* h = (float*)ws;
   if (const int rc = norm_rows(a, lda, g, eps, h, M, K, stream)) return rc;
   return product(h, K, nullptr, 0.f, h + (size_t)M * K, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
@@ -552,7 +556,10 @@ APC_EXPORT int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int l
 constexpr TileCost GLU_TILES[] = {{1, 2, true, 2.5, 2.5, 0.7, 7.8}, {2, 2, false, 2.1, 4.8, 1.4, 8.9}, {3, 2, false, 2.6, 5.5, 1.7, 12.4},
                                   {3, 4, false, 2.6, 4.8, 2.7, 22.9}, {4, 4, false, 3.1, 4.0, 3.6, 30.5}};
 constexpr TileCost GLU_TILES_SHORT[] = {{1, 2, true, 3.6, 0.0, 0.95, 0.0}, {2, 2, true, 4.1, 0.0, 0.69, 0.0}, {3, 2, true, 4.4, 0.0, 0.93, 0.0}};
-static int glu_tile_of(int M, int F, int K) { return K <= 4 * STAGE ? least_cost(GLU_TILES_SHORT, M, F, K, K, 8) : least_cost(GLU_TILES, M, F, K, K, 8); }
+static int glu_tile_of(int M, int F, int K) {
+  if (K <= 4 * STAGE) return least_cost(GLU_TILES_SHORT, M, F, K, K, 8);
+  return M <= 16 ? 0 : least_cost(GLU_TILES, M, F, K, K, 8);
+}
 
 // Rows of the tile, times 1,000, and its outputs (half of the columns it computes).
 APC_EXPORT int apc_swiglu_f32_tile(int M, int F, int K) {
@@ -596,7 +603,7 @@ APC_EXPORT int apc_swiglu_norm_f32(const void* A, int lda, const void* G, float 
   if (M <= 0 || F <= 0) return 0;
   if (K <= 0 || lda < K || ldw < K || ldo < F) return APC_ERR_BAD_ARG;
   if (!apc_swiglu_norm_f32_takes(A, lda, G, W, ldw, F, K)) return APC_ERR_UNSUPPORTED;
-  if (norm_in_product(M, K)) return swiglu(A, lda, G, eps, nullptr, W, ldw, out, ldo, M, F, K, stream);
+  if (norm_in_product(M, K, glu_tile_of(M, F, K))) return swiglu(A, lda, G, eps, nullptr, W, ldw, out, ldo, M, F, K, stream);
   float* h = (float*)ws;
   if (const int rc = norm_rows((const float*)A, lda, (const float*)G, eps, h, M, K, stream)) return rc;
   return swiglu(h, K, nullptr, 0.f, h + (size_t)M * K, W, ldw, out, ldo, M, F, K, stream);

@@ -184,3 +184,28 @@ def test_product_of_normalised_rows(M, N, K, gated):
         alone = torch.empty(1, N, device=DEV)
         assert fn(x[r:r + 1], g, eps, w, alone)
         assert torch.equal(alone[0], out[r, :N])
+
+
+def test_tiles_of_few_rows():
+    """Up to 16 rows take the tile of 16 rows, but for many outputs of a K up to 128, where tiles that leave the empty slices
+    out are faster."""
+    from allpaca_amd.kernels import lib
+    L = lib.load("plain")
+    for M in (1, 9, 16):
+        for K in (32, 64, 128):
+            assert L.apc_gemm_f32_tile(M, 2048, K) == 16016 and L.apc_gemm_f32_tile(M, 128256, K) == 32032, (M, K)
+        for K in (132, 2048, 8192):
+            assert {L.apc_gemm_f32_tile(M, N, K) for N in (16, 2048, 128256)} == {16016}, (M, K)
+
+
+# few rows of a K up to 128: two and four slices, and 16 rows of eight, with the norm in the product and in front of it
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(16, 40003, 32), (3, 33000, 64), (9, 50010, 100), (1, 128256, 128), (40, 300, 128), (33, 100, 64)])
+def test_few_rows_of_a_short_k(M, N, K):
+    test_product_against_64_bits_and_rows_alone(M, N, K)
+    for gated in (False, True):
+        test_product_of_normalised_rows(M, N // 2 if gated else N, K, gated)
+    o, x, g, w = ops(), gen(M, K, seed=1), 1.0 + 0.1 * gen(K, seed=2), gen(N, K, seed=3)
+    many, few = torch.empty(M, N, device=DEV), torch.empty(M, 48, device=DEV)
+    assert o.linear_normed(x, g, 1e-5, w, many) and o.linear_normed(x, g, 1e-5, w[:48], few)
+    assert torch.equal(many[:, :48], few)                  # (48 outputs: the norm in the product up to 16 rows)
