@@ -80,17 +80,21 @@ __global__ __launch_bounds__(64) void norm_rows_f32_kernel(const float* __restri
 // GLU: W is [2 N][K], rows of gates and then rows of values; a block's bands of W are NT / 2 of gates and the NT / 2 of
 // values that belong to them, and it writes silu(gate) * value.  A product is the same sum as without, so the result is
 // the bits of the product of 2 N outputs and the activation's own pass.
-// NORM: A is the row in front of an RMS norm of weight G.  Every block reads whole rows of A anyway (a wave its own k), so a
+// NORMALISED: A is the row in front of an RMS norm of weight G.  Every block reads whole rows of A anyway (a wave its own k), so a
 // wave multiplies its operands by G, adds up the squares beside that, and the sums are scaled by the row's 1 / sqrt(mean
 // square + eps) where the waves meet.  The squares of a row are added in an order that depends on K alone, too.  For one row
 // tile only: with several, every block does it again for the same rows (325 rows x 8,192 outputs of SwiGLU 194 -> 205 us,
-// twice the norm's own launch), so norm_rows_f32_kernel does it once, with the same operations, and R has the rows' scales.
-template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU, bool NORM>
+// twice the norm's own launch), so norm_rows_f32_kernel does it once, with the same operations, and R has the rows' scales (SCALED; a form
+// of its own: with the scales' loads in front of every tile, behind a condition, the compiler waited there and where the waves
+// meet for all that was on its way).
+enum Rows { PLAIN, SCALED, NORMALISED };
+template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU, int ROWS, bool ON>
 __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
     const float* __restrict__ A, int lda, const float* __restrict__ G, float eps, const float* __restrict__ R,
     const float* __restrict__ W, int ldw, void* __restrict__ C, int c_dtype, int ldc, int M, int N, int K, int mode, int tiles_m, int tiles) {
   constexpr int BANDS = MT + NT;
-  constexpr bool ON = SL == SLICES && D == 1;                         // tile after tile (large tiles, a long K)
+  constexpr bool NORM = ROWS == NORMALISED;
+  static_assert(!(ON && NORM), "the norm is in the product of one row tile only");
   constexpr int STAGE_F4 = BANDS * 128, SUM_F4 = MT * NT * 64;       // float4 a wave: its stage, and at the end its sums
   constexpr int WAVE_F4 = STAGE_F4 > SUM_F4 ? STAGE_F4 : SUM_F4;
   __shared__ f32x4 lds[SL * WAVE_F4];
@@ -202,17 +206,9 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
 #pragma unroll
     for (int u = 0; u < PRODUCTS; ++u) multiply_one(half, u);
   };
-  // The sums of a tile's eight slices, of what this thread stores: its q-th piece of four outputs.
+  // The waves meet: their sums into LDS, then a thread adds the slices' sums of the pieces of four outputs that it stores.
   constexpr int PIECES = (MT * NO + SL - 1) / SL;
-  float scale[PIECES];
-  auto load_scale = [&](int row0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < PIECES; ++q) {
-      const int p = threadIdx.x + q * 64 * SL, m = row0 + p / (NO * 64) * 16 + p % 16;
-      scale[q] = !NORM && R && p < MT * NO * 64 ? R[min(m, M - 1)] : 1.f;
-    }
-  };
-  auto meet = [&](f32x4 (&v)[PIECES]) __attribute__((always_inline)) {
+  auto meet = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -226,52 +222,53 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       }
     }
     __syncthreads();
+  };
+  auto scale_of = [&](int q, int row0) __attribute__((always_inline)) {                // (SCALED)
+    return R[min(row0 + (int)(threadIdx.x + q * 64 * SL) / (NO * 64) * 16 + (int)threadIdx.x % 16, M - 1)];
+  };
+  auto piece = [&](int q, float scale) __attribute__((always_inline)) {
+    const int p = threadIdx.x + q * 64 * SL, i = p / (NO * 64), j = p / 64 % NO, l = p % 64;
+    auto sum = [&](int band) __attribute__((always_inline)) {
+      const int at = (i * NT + band) * 64 + l;
+      f32x4 u = lds[at];
 #pragma unroll
-    for (int q = 0; q < PIECES; ++q) {
-      const int p = threadIdx.x + q * 64 * SL;
-      if (p >= MT * NO * 64) continue;
-      const int i = p / (NO * 64), j = p / 64 % NO, l = p % 64;
-      auto sum = [&](int band) __attribute__((always_inline)) {
-        const int at = (i * NT + band) * 64 + l;
-        f32x4 u = lds[at];
+      for (int w = 1; w < SL; ++w) u += lds[w * WAVE_F4 + at];
+      return u;
+    };
+    if constexpr (NORM) {
+      float all = 0.f;
 #pragma unroll
-        for (int w = 1; w < SL; ++w) u += lds[w * WAVE_F4 + at];
-        return u;
-      };
-      if constexpr (NORM) {
-        float all = 0.f;
-#pragma unroll
-        for (int w = 0; w < SL; ++w) all += squares[w * 16 * MT + i * 16 + l % 16];
-        scale[q] = row_scale(all, K, eps);
-      }
-      v[q] = sum(j) * scale[q];
-      if constexpr (GLU) {
-        const f32x4 u = sum(NO + j) * scale[q];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[q][e] = (v[q][e] / (1.0f + expf(-v[q][e]))) * u[e];
-      }
+      for (int w = 0; w < SL; ++w) all += squares[w * 16 * MT + i * 16 + l % 16];
+      scale = row_scale(all, K, eps);
     }
+    f32x4 v = sum(j);
+    if constexpr (ROWS != PLAIN) v *= scale;
+    if constexpr (GLU) {
+      f32x4 u = sum(NO + j);
+      if constexpr (ROWS != PLAIN) u *= scale;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (v[e] / (1.0f + expf(-v[e]))) * u[e];
+    }
+    return v;
   };
   const bool wide = mode == 0 && c_dtype == APC_F32 && ldc % 4 == 0 && ((uintptr_t)C & 15u) == 0;   // 16-byte stores
-  auto leave = [&](const f32x4 (&v)[PIECES], int row0, int out0) __attribute__((always_inline)) {
+  auto leave = [&](int q, const f32x4& v, int row0, int out0) __attribute__((always_inline)) {
+    const int p = threadIdx.x + q * 64 * SL;
+    const int m = row0 + p / (NO * 64) * 16 + p % 16, n = out0 + p / 64 % NO * 16 + (p % 64 / 16) * 4;
+    if (m >= M) return;
+    if (wide && n + 4 <= N) {
+      *(f32x4*)((float*)C + (size_t)m * ldc + n) = v;
+      return;
+    }
 #pragma unroll
-    for (int q = 0; q < PIECES; ++q) {
-      const int p = threadIdx.x + q * 64 * SL;
-      const int m = row0 + p / (NO * 64) * 16 + p % 16, n = out0 + p / 64 % NO * 16 + (p % 64 / 16) * 4;
-      if (p >= MT * NO * 64 || m >= M) continue;
-      if (wide && n + 4 <= N) {
-        *(f32x4*)((float*)C + (size_t)m * ldc + n) = v[q];
-        continue;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (n + e >= N) continue;
-        const size_t o = (size_t)m * ldc + n + e;
-        if (mode == 1) ((float*)C)[o] += v[q][e];
-        else store_f(C, c_dtype, o, v[q][e]);
-      }
+    for (int e = 0; e < 4; ++e) {
+      if (n + e >= N) continue;
+      const size_t o = (size_t)m * ldc + n + e;
+      if (mode == 1) ((float*)C)[o] += v[e];
+      else store_f(C, c_dtype, o, v[e]);
     }
   };
+  auto has = [&](int q) __attribute__((always_inline)) { return (int)threadIdx.x + q * 64 * SL < MT * NO * 64; };
   auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -285,7 +282,6 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
 
   aim(t);
   clear();
-  f32x4 v[PIECES];
   // A stage: its second operands come out of LDS under the first products; then the next stage goes in, the loads that
   // take its registers go out, and its first operands come back under the second products.
   if constexpr (ON) {
@@ -308,16 +304,12 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       get(0, 0);
     };
     int row0 = m0, out0 = n0;                           // of the tile that is multiplied
-    if (steps > 0) load(0, 0), asked();
-    gains_in();
-    if (steps > 0) first_in();
+    if (steps > 0) load(0, 0), asked(), first_in();
     while (true) {
-      load_scale(row0);
       if (steps > 0) {
         for (int s = 0; s < steps - 1; ++s) {
           get(1, s);
           __builtin_amdgcn_sched_barrier(0);
-          normalise(0);
 #pragma unroll
           for (int u = 0; u < 2 * BANDS; ++u) {
 #pragma unroll
@@ -340,18 +332,27 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
         multiply(1);
       }
       t += stride;
-      meet(v);
+      f32x4 v[PIECES];
+      float scale[PIECES] = {};
+      if constexpr (ROWS == SCALED)
+#pragma unroll
+        for (int q = 0; q < PIECES; ++q) scale[q] = scale_of(q, row0);
+      meet();
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q)
+        if (has(q)) v[q] = piece(q, scale[q]);
       if (t < last) {
         __syncthreads();                                // everyone has read the sums
         clear();
         if (steps > 0) first_in();
       }
-      leave(v, row0, out0);
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q)
+        if (has(q)) leave(q, v[q], row0, out0);
       if (t >= last) break;
       row0 = (t % tiles_m) * (16 * MT), out0 = (t / tiles_m) * (16 * NO);
     }
   } else {
-    load_scale(m0);
     auto stage = [&](int s, int next_slot, bool next, bool more) __attribute__((always_inline)) {
       get(1, s);
       __builtin_amdgcn_sched_barrier(0);
@@ -397,8 +398,10 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       });
       if (steps <= 0) gains_in();
     }
-    meet(v);
-    leave(v, m0, n0);
+    meet();
+#pragma unroll
+    for (int q = 0; q < PIECES; ++q)
+      if (has(q)) leave(q, piece(q, ROWS == SCALED ? scale_of(q, m0) : 1.f), m0, n0);
   }
 }
 
@@ -406,15 +409,15 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
 // its waves idle and 128 KiB of LDS taken.  2,048 rows x 16,384 outputs at K = 32, 64, 128: 200, 203, 216 us with eight
 // slices and stores of 4 bytes, 84, 101, 147 with the two or four there are, 53, 69, 125 with 16-byte stores beside (one
 // fma chain an output on the vector units: 70, 98, 150).
-template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU, bool NORM>
+template <int SL, int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU, int ROWS, bool ON>
 int launch_slices(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C,
                   int c_dtype, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
   const int tiles_m = ceil_div(M, 16 * MT);
   const long long tiles = (long long)tiles_m * ceil_div(N, 16 * (GLU ? NT / 2 : NT));
   if (tiles > (1 << 27)) return APC_ERR_BAD_ARG;
   int blocks = ceil_div((int)tiles, 8) * 8;
-  if (SL == SLICES && D == 1 && blocks > 256) blocks = 256;           // such a block has a compute unit to itself
-  hipLaunchKernelGGL((gemm_f32_kernel<SL, MT, NT, D, ONCE, MIN_WAVES, GLU, NORM>), dim3(blocks), dim3(64 * SL), 0,
+  if (ON && blocks > 256) blocks = 256;                 // such a block has a compute unit to itself
+  hipLaunchKernelGGL((gemm_f32_kernel<SL, MT, NT, D, ONCE, MIN_WAVES, GLU, ROWS, ON>), dim3(blocks), dim3(64 * SL), 0,
                      stream, A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, tiles_m, (int)tiles);
   APC_LAUNCH_CHECK();
   return 0;
@@ -424,14 +427,25 @@ template <int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU = false>
 int launch(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C, int c_dtype,
            int ldc, int M, int N, int K, int mode, hipStream_t stream) {
   if constexpr (MT == 1 && ONCE)
-    if (G) return launch_slices<SLICES, MT, NT, D, ONCE, MIN_WAVES, GLU, true>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream);
+    if (G) return launch_slices<SLICES, MT, NT, D, ONCE, MIN_WAVES, GLU, NORMALISED, false>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream);
   if (G) return APC_ERR_UNSUPPORTED;
-#define SL_GO(SL_) return launch_slices<SL_, MT, NT, D, ONCE, MIN_WAVES, GLU, false>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
+#define SL_GO(SL_, ON_)                                                                                                             \
+  return R ? launch_slices<SL_, MT, NT, D, ONCE, MIN_WAVES, GLU, SCALED, ON_>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream) \
+           : launch_slices<SL_, MT, NT, D, ONCE, MIN_WAVES, GLU, PLAIN, ON_>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
   if constexpr (MT * NT >= 4 && MT * NT <= 6) {         // (smaller tiles share their units with eight too; larger ones are not chosen)
-    if (K <= 2 * STAGE) SL_GO(2);
-    if (K <= 4 * STAGE) SL_GO(4);
+    if (K <= 2 * STAGE) SL_GO(2, false);
+    if (K <= 4 * STAGE) SL_GO(4, false);
   }
-  SL_GO(SLICES);
+  // Which tiles' blocks go on to further tiles, with a stage's stores and loads between its products.  Time of the form that ends
+  // after its tile / of this one, mean over 17 to 2,048 rows x 64 to 32,768 outputs: 32 x 32 tiles (two blocks a unit without it)
+  // 0.87-0.95 at every K; 48 x 32 in one round of 256 blocks 0.91-0.99, in more 1.05-1.09 up to K = 1,024 and 1.00-1.03 beyond;
+  // 48 x 64 one round 0.92-0.98 up to K = 512, 1.02-1.04 beyond, more rounds 1.01-1.10; 64 x 64 0.84-0.97 up to K = 512, then one
+  // round 0.97 up to K = 1,024, else 1.00-1.02.  SwiGLU: 48 x 16 outputs 0.93-1.00, the others as their products.
+  if constexpr (MT * NT > 6 || (MT * NT == 6 && !GLU)) {
+    const bool rounds = (long long)ceil_div(M, 16 * MT) * ceil_div(N, 16 * (GLU ? NT / 2 : NT)) > 256;
+    if (MT * NT == 6 ? rounds : MT * NT == 12 ? rounds || K > 512 : K > (rounds ? 512 : 1024)) SL_GO(SLICES, true);
+  }
+  SL_GO(SLICES, false);
 #undef SL_GO
 }
 
@@ -443,44 +457,41 @@ bool gemm_f32_takes(const void* A, int lda, const void* W, int ldw, int K) {
          ldw < (1 << 22);            // (64 rows fit a descriptor's 32-bit offsets)
 }
 
-// A tile of 16 mt x 16 nt and what a launch of its blocks costs, in microseconds: once, and for every 256 of them (a round);
-// each a part that stays and a part that grows with K, as for K = 2,048.
-struct TileCost { int mt, nt; bool shares; double start, start_k, round, round_k; };
+// A tile of 16 mt x 16 nt and what a launch of its blocks costs, in microseconds: once, and for every 256 of them (a round); each
+// a part that stays and a part that grows with K, as for K = 2,048.  `part`: how far a last round that is not full takes less
+// (1: blocks share their units, their time grows with them).  `over`: what the columns up to the next multiple of 256 count (a K
+// between leaves waves with a stage less than the others).
+struct TileCost { int mt, nt; double start, start_k, round, round_k, over, part; };
 template <int COUNT>
-static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, double k_shares, double k_alone, int outputs) {   // outputs: of 16 nt columns
+static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, int K, int outputs) {   // outputs: of 16 nt columns
   int best = 0;
   double best_cost = 1e30;
   for (int i = 0; i < COUNT; ++i) {
     const TileCost& s = shapes[i];
-    double rounds = (double)ceil_div(M, 16 * s.mt) * ceil_div(N, outputs * s.nt) / 256;
-    if (!s.shares) rounds = ceil(rounds);
-    const double k = (s.shares ? k_shares : k_alone) / 2048;
-    const double cost = s.start + s.start_k * k + (s.round + s.round_k * k) * (rounds > 1.0 ? rounds : 1.0);
+    const double raw = (double)ceil_div(M, 16 * s.mt) * ceil_div(N, outputs * s.nt) / 256;
+    const double rounds = raw > 1.0 ? s.part * raw + (1.0 - s.part) * ceil(raw) : 1.0;
+    const double k = (K + s.over * (SLICES * STAGE * ceil_div(K, SLICES * STAGE) - K)) / 2048;
+    const double cost = s.start + s.start_k * k + (s.round + s.round_k * k) * rounds;
     if (cost < best_cost) best = i, best_cost = cost;
   }
   return best;
 }
 
-// The tile: the least expected time.  A block of the small tiles shares its compute unit with others, so their time grows
-// with the blocks; the large ones have a unit to themselves and go in whole rounds of 256.  Fitted to 33 to 2,048 rows x
-// 2,048 and 3,072 outputs, K 256 to 8,192: the choice takes 1.01 of the best tile's time in the mean, 1.15 at worst.  At
-// K = 2,048, 2,048 outputs take 10.1 us at 33 rows (32 x 16 tiles; 32 x 32 13.1, 48 x 32 17.1), 13.3 at 100 (32 x 32;
-// 32 x 16: 15.6), 29.5 at 325 (48 x 64; 48 x 32: 31.8, 64 x 64: 38.2), 39 at 400 and 146 at 2,048 rows (64 x 64; 48 x 64:
-// 55, 159).
-// Up to K = 128 (see launch_slices) blocks of all tiles share their units, and with many outputs tiles that leave the empty
-// slices out are the better ones for few rows too: 16 rows x 128,256 outputs, 32 x 32 / 16 x 16 tiles, K = 32 10.4 / 19.6 us, 64
-// 13.1 / 22.6, 128 22.2 / 25.7; 32,768 outputs 4.5 / 6.7, 5.2 / 7.1.
-constexpr TileCost TILES[] = {{1, 1, true, 2.1, 0.5, 0.5, 4.7},    {2, 1, true, 2.1, 0.9, 0.5, 5.9},   {2, 2, false, 2.4, 0.5, 1.1, 9.0},
-                              {3, 2, false, 2.3, 0.4, 1.5, 12.7}, {3, 4, false, 2.4, 0.4, 2.6, 23.5}, {4, 4, false, 2.0, 0.6, 4.3, 30.7}};
-constexpr TileCost TILES_SHORT[] = {{1, 1, true, 3.6, 0.0, 0.75, 0.0}, {2, 1, true, 3.6, 0.0, 0.95, 0.0}, {2, 2, true, 4.1, 0.0, 0.69, 0.0},
-                                    {3, 2, true, 4.4, 0.0, 0.93, 0.0}};        // (48 x 64 and 64 x 64 are never the least)
+// The tile: the least expected time.  Fitted to 2,233 products of 17 to 2,048 rows x 64 to 32,768 outputs, K 160 to 14,336, each on
+// all six tiles: the choice takes 1.008 of the best tile's time in the mean, more than 1.03 in 199 of them, 1.22 at worst (100
+// rows x 6,144 outputs, K = 512: 16.4 us, 13.4 on 64 x 64).  K = 2,048: 33 rows x 2,048 outputs 10.1 us (32 x 16 tiles; 32 x 32 13.1),
+// 325 rows 28.2 (48 x 64; 64 x 64 36.4), 2,048 rows 146 (64 x 64; 48 x 64 159); K = 256: 64 rows x 16,384 10.1 (64 x 64).
+// Up to K = 128 (see launch) blocks of all tiles share their units, and with many outputs tiles that leave the empty slices out
+// are the better ones for few rows too: 16 rows x 128,256 outputs, 32 x 32 / 16 x 16 tiles, K = 32 10.4 / 19.6 us, 64 13.1 / 22.6, 128
+// 22.2 / 25.7; 32,768 outputs 4.5 / 6.7, 5.2 / 7.1.
+constexpr TileCost TILES[] = {{1, 1, 0.45, 1.86, 1.48, 4.05, 0.4, 0.77},   {2, 1, 1.74, 1.19, 0.85, 5.6, 0.4, 0.07},
+                              {2, 2, 3.18, 0.71, 0.74, 9.07, 0.55, 0.11},  {3, 2, 1.98, 0.79, 1.37, 13.92, 0.55, 0.07},
+                              {3, 4, 2.43, 1.29, 2.41, 24.83, 0.55, 0.09}, {4, 4, 2.39, 0.61, 3.7, 33.4, 0.55, 0.18}};
+constexpr TileCost TILES_SHORT[] = {{1, 1, 3.6, 0.0, 0.75, 0.0, 0.0, 1.0}, {2, 1, 3.6, 0.0, 0.95, 0.0, 0.0, 1.0}, {2, 2, 4.1, 0.0, 0.69, 0.0, 0.0, 1.0},
+                                    {3, 2, 4.4, 0.0, 0.93, 0.0, 0.0, 1.0}};        // (48 x 64 and 64 x 64 are never the least)
 static int tile_of(int M, int N, int K) {
-  if (K <= 4 * STAGE) return least_cost(TILES_SHORT, M, N, K, K, 16);
-  if (M <= 16) return 0;                                // (the other tiles multiply rows that are not there)
-  // a K between two multiples of 256 leaves waves with a stage less than the others: 480 rows x 2,048 outputs at K = 256,
-  // 320, 512 take 11.4, 14.4, 16.6 us on 32 x 16 tiles and 12.6, 17.8, 18.9 on 48 x 64
-  const int over = SLICES * STAGE * ceil_div(K, SLICES * STAGE) - K;
-  return least_cost(TILES, M, N, K + 0.4 * over, K + 0.8 * over, 16);
+  if (K <= 4 * STAGE) return least_cost(TILES_SHORT, M, N, K, 16);
+  return M <= 16 ? 0 : least_cost(TILES, M, N, K, 16);   // (the other tiles multiply rows that are not there)
 }
 
 // Rows of the tile, times 1,000, and its outputs.
@@ -551,14 +562,15 @@ APC_EXPORT int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int l
   return gemm_f32_takes(A, lda, W, ldw, K) && ((long long)F + 64) * ldw < (1LL << 29);   // byte offsets of 32 bits
 }
 
-// (33 to 2,048 rows x 4,096 and 8,192 outputs, K 256 to 2,048: never more than 1.03 of the best tile's time.  K = 2,048, 8,192
-// outputs: 325 rows 188 us on 48 x 32 tiles, 205 on 48 x 16, 211 on 64 x 32; 100 rows 76 on 64 x 32, 85 on 48 x 32.)
-constexpr TileCost GLU_TILES[] = {{1, 2, true, 2.5, 2.5, 0.7, 7.8}, {2, 2, false, 2.1, 4.8, 1.4, 8.9}, {3, 2, false, 2.6, 5.5, 1.7, 12.4},
-                                  {3, 4, false, 2.6, 4.8, 2.7, 22.9}, {4, 4, false, 3.1, 4.0, 3.6, 30.5}};
-constexpr TileCost GLU_TILES_SHORT[] = {{1, 2, true, 3.6, 0.0, 0.95, 0.0}, {2, 2, true, 4.1, 0.0, 0.69, 0.0}, {3, 2, true, 4.4, 0.0, 0.93, 0.0}};
+// (1,801 gated products of 17 to 1,024 rows x 64 to 14,336 outputs, K 160 to 8,192: 1.004 of the best tile's time in the mean, 1.10
+// at worst.  K = 2,048, 8,192 outputs: 325 rows 187 us on 48 x 32 tiles, 205 on 48 x 16, 211 on 64 x 32; 100 rows 76 on 64 x 32, 85 on 48 x 32.)
+constexpr TileCost GLU_TILES[] = {{1, 2, 2.44, 2.65, 0.55, 5.34, 0.4, 0.16}, {2, 2, 3.03, 1.13, 0.83, 8.93, 0.55, 0.44},
+                                  {3, 2, 2.82, 0.89, 1.1, 14.48, 0.55, 0.39}, {3, 4, 2.49, 1.85, 2.2, 24.42, 0.55, 0.0},
+                                  {4, 4, 0.55, 1.13, 3.44, 32.83, 0.55, 0.0}};
+constexpr TileCost GLU_TILES_SHORT[] = {{1, 2, 3.6, 0.0, 0.95, 0.0, 0.0, 1.0}, {2, 2, 4.1, 0.0, 0.69, 0.0, 0.0, 1.0}, {3, 2, 4.4, 0.0, 0.93, 0.0, 0.0, 1.0}};
 static int glu_tile_of(int M, int F, int K) {
-  if (K <= 4 * STAGE) return least_cost(GLU_TILES_SHORT, M, F, K, K, 8);
-  return M <= 16 ? 0 : least_cost(GLU_TILES, M, F, K, K, 8);
+  if (K <= 4 * STAGE) return least_cost(GLU_TILES_SHORT, M, F, K, 8);
+  return M <= 16 ? 0 : least_cost(GLU_TILES, M, F, K, 8);
 }
 
 // Rows of the tile, times 1,000, and its outputs (half of the columns it computes).
