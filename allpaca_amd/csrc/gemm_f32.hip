@@ -46,8 +46,10 @@ __device__ __forceinline__ void each_count(F f) {        // f(1), .. f(N), known
 
 __device__ __forceinline__ float row_scale(float squares, int K, float eps) { return 1.0f / sqrtf(squares / (float)K + eps); }
 
-// H = A * G and R = 1 / sqrt(mean square + eps) of rows in front of an RMS norm, with the operations of the product's NORM
-// form: 32 lanes a row, a lane the quarter of a slice's 16 k that an operand's lane holds there.
+// H = A * G and R = 1 / sqrt(mean square + eps) of rows in front of an RMS norm, with the operations of the product's NORMALISED
+// form and in its order: the squares of a slice's k are added by four chains, one a quarter of every 16 k, as an operand's lanes
+// hold them there.  Two forms of the same bits.  Here the 32 lanes that add read the row themselves, two rows a wave: for rows so
+// many that they fill the chip, and short ones.
 __global__ __launch_bounds__(64) void norm_rows_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ G, float eps,
                                                            float* __restrict__ H, float* __restrict__ R, int M, int K) {
   const int lane = threadIdx.x % 32, m = min((int)(blockIdx.x * 2 + threadIdx.x / 32), M - 1);   // (a last row twice: the same values)
@@ -74,6 +76,65 @@ __global__ __launch_bounds__(64) void norm_rows_f32_kernel(const float* __restri
 #pragma unroll
   for (int w = 0; w < SLICES; ++w) all += __shfl(own, w * 4, 32);
   if (lane == 0) R[m] = row_scale(all, K, eps);
+}
+
+// Here a block takes a row: every thread has pieces of the eight slices, and they go through LDS to the 32 lanes of the first wave
+// that add.  Bound by the row's way: 32 lanes have an eighth of a long row's loads in flight at a time.
+constexpr int NORM_PASSES = 4, NORM_PITCH = 36;         // passes of 128 k of every slice; 16-byte pieces between slices (banks)
+__global__ __launch_bounds__(256) void norm_row_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ G, float eps,
+                                                            float* __restrict__ H, float* __restrict__ R, int M, int K) {
+  extern __shared__ f32x4 room[];                       // [group % 2][pass][slice][piece], what K needs of it
+  const int m = blockIdx.x, own = threadIdx.x / 32, at = threadIdx.x % 32;     // this thread's slice, its piece of a pass of it
+  const int slice = STAGE * ((K + STAGE * SLICES - 1) / (STAGE * SLICES));
+  const int passes = (slice + 127) / 128, groups = (passes + NORM_PASSES - 1) / NORM_PASSES;
+  const float* a = A + (size_t)m * lda;
+  f32x4 v[NORM_PASSES], g[NORM_PASSES];
+  auto column = [&](int group, int u, bool& in) __attribute__((always_inline)) {
+    const int o = (group * NORM_PASSES + u) * 128 + at * 4, k = own * slice + o;
+    in = o < slice && k < K;
+    return in ? k : 0;
+  };
+  auto load = [&](int group) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NORM_PASSES; ++u) {
+      bool in;
+      const int k = column(group, u, in);
+      v[u] = *(const f32x4*)(a + k), g[u] = *(const f32x4*)(G + k);
+    }
+  };
+  load(0);
+  float ss[2] = {0.f, 0.f};
+  for (int group = 0; group < groups; ++group) {
+#pragma unroll
+    for (int u = 0; u < NORM_PASSES; ++u) {
+      if (group * NORM_PASSES + u >= passes) break;
+      bool in;
+      const int k = column(group, u, in);
+      room[(((group % 2) * NORM_PASSES + u) * SLICES + own) * NORM_PITCH + at] = in ? v[u] : f32x4{0.f, 0.f, 0.f, 0.f};
+      if (in) *(f32x4*)(H + (size_t)m * K + k) = v[u] * g[u];
+    }
+    if (group + 1 < groups) load(group + 1);
+    __syncthreads();                                    // (the first wave reads one half while the others fill the other)
+    if (threadIdx.x < 32) {
+#pragma unroll 1
+      for (int u = 0; u < min(NORM_PASSES, passes - group * NORM_PASSES); ++u) {
+        f32x4 q[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) q[x] = room[(((group % 2) * NORM_PASSES + u) * SLICES + threadIdx.x / 4) * NORM_PITCH + threadIdx.x % 4 + 4 * x];
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ss[e % 2] = fmaf(q[x][e], q[x][e], ss[e % 2]);
+      }
+    }
+  }
+  if (threadIdx.x >= 32) return;
+  float sum = ss[0] + ss[1];
+  sum += __shfl_xor(sum, 1), sum += __shfl_xor(sum, 2);
+  float all = 0.f;
+#pragma unroll
+  for (int w = 0; w < SLICES; ++w) all += __shfl(sum, w * 4, 32);
+  if (threadIdx.x == 0) R[m] = row_scale(all, K, eps);
 }
 
 // MT x NT tiles of 16 rows x 16 outputs a block, D stages of loads ahead.
@@ -353,6 +414,10 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
       row0 = (t % tiles_m) * (16 * MT), out0 = (t / tiles_m) * (16 * NO);
     }
   } else {
+    float scale[PIECES] = {};
+    if constexpr (ROWS == SCALED)
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) scale[q] = scale_of(q, m0);
     auto stage = [&](int s, int next_slot, bool next, bool more) __attribute__((always_inline)) {
       get(1, s);
       __builtin_amdgcn_sched_barrier(0);
@@ -401,7 +466,7 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
     meet();
 #pragma unroll
     for (int q = 0; q < PIECES; ++q)
-      if (has(q)) leave(q, piece(q, ROWS == SCALED ? scale_of(q, m0) : 1.f), m0, n0);
+      if (has(q)) leave(q, piece(q, scale[q]), m0, n0);
   }
 }
 
@@ -529,16 +594,27 @@ int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dt
 // C[M,N] = rmsnorm(A; G, eps) . W^T.  Up to 16 rows in one launch: 4 rows x 3,072 outputs x K 2,048 6.9 us without the norm, 7.6
 // with it, and the norm's own launch was 4.7; 6,144 x K 4,096 19.8 and 21.0.  More rows need room for M rows of K and their
 // scales: apc_gemm_norm_f32_kib(M, K) KiB.  A row's outputs do not depend on the rows beside it, nor on M.
-static bool norm_in_product(int M, int K, int tile) { return M <= 16 && K <= NORM_K && tile == 0; }
+// With a short K and many outputs every block does the norm again for little else: 8 rows x 128,256 outputs, in the product / in
+// front of it, K = 256 44.1 / 32.2 us, 512 62.2 / 45.6, 1,024 90.9 / 80.1 (2,048 on: the other way), 32,768 outputs 13.1 / 12.1,
+// 18.1 / 16.1, 26.1 / 26.0, 14,336 outputs 9.9 / 10.3 at K = 512; SwiGLU at K = 512 of 32,768 outputs 28.1 / 28.3, of 128,256 95.0 / 89.1.
+static bool norm_in_product(int M, int N, int K, int tile, int most) { return M <= 16 && K <= NORM_K && (K > 1024 || N <= most) && tile == 0; }
 APC_EXPORT int apc_gemm_norm_f32_kib(int M, int K) {
-  return M <= 16 && K > 4 * STAGE && K <= NORM_K ? 0 : (int)(((long long)M * (K + 1) * 4 + 1023) / 1024);
+  return M <= 16 && K > 1024 && K <= NORM_K ? 0 : (int)(((long long)M * (K + 1) * 4 + 1023) / 1024);
 }
 APC_EXPORT int apc_gemm_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int K) {
   return gemm_f32_takes(A, lda, W, ldw, K) && G && ((uintptr_t)G & 15u) == 0;
 }
 static int norm_rows(const float* A, int lda, const float* G, float eps, float* ws, int M, int K, hipStream_t stream) {
   if (!ws || ((uintptr_t)ws & 15u)) return APC_ERR_BAD_ARG;
-  hipLaunchKernelGGL(norm_rows_f32_kernel, dim3(ceil_div(M, 2)), dim3(64), 0, stream, A, lda, G, eps, ws, ws + (size_t)M * K, M, K);
+  // Two rows a wave / a row a block, us: 17 rows of 512 2.3 / 2.4, of 2,048 2.8 / 2.6, of 4,096 3.9 / 3.1, of 8,192 6.2 / 4.4; 177 of
+  // 4,096 5.2 / 4.1; 330 of 2,048 4.1 / 4.1; 1,024 of 2,048 6.7 / 7.7, of 8,192 17.2 / 12.7; 2,048 of 1,024 6.3 / 8.4.
+  if (K > NORM_K || (M <= 512 && K > 512)) {
+    const int passes = ceil_div(STAGE * ceil_div(K, STAGE * SLICES), 128);
+    const int lds = (passes < 2 * NORM_PASSES ? passes : 2 * NORM_PASSES) * SLICES * NORM_PITCH * 16;
+    hipLaunchKernelGGL(norm_row_f32_kernel, dim3(M), dim3(256), lds, stream, A, lda, G, eps, ws, ws + (size_t)M * K, M, K);
+  } else {
+    hipLaunchKernelGGL(norm_rows_f32_kernel, dim3(ceil_div(M, 2)), dim3(64), 0, stream, A, lda, G, eps, ws, ws + (size_t)M * K, M, K);
+  }
   APC_LAUNCH_CHECK();
   return 0;
 }
@@ -549,7 +625,7 @@ APC_EXPORT int apc_gemm_norm_f32(const void* A, int lda, const void* G, float ep
   if (K <= 0 || lda < K || ldw < K || ldc < N) return APC_ERR_BAD_ARG;
   if (!apc_gemm_norm_f32_takes(A, lda, G, W, ldw, K)) return APC_ERR_UNSUPPORTED;
   const float *a = (const float*)A, *g = (const float*)G, *w = (const float*)W;
-  if (norm_in_product(M, K, tile_of(M, N, K))) return product(a, lda, g, eps, nullptr, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
+  if (norm_in_product(M, N, K, tile_of(M, N, K), 16384)) return product(a, lda, g, eps, nullptr, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
   float* h = (float*)ws;
   if (const int rc = norm_rows(a, lda, g, eps, h, M, K, stream)) return rc;
   return product(h, K, nullptr, 0.f, h + (size_t)M * K, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
@@ -615,7 +691,7 @@ APC_EXPORT int apc_swiglu_norm_f32(const void* A, int lda, const void* G, float 
   if (M <= 0 || F <= 0) return 0;
   if (K <= 0 || lda < K || ldw < K || ldo < F) return APC_ERR_BAD_ARG;
   if (!apc_swiglu_norm_f32_takes(A, lda, G, W, ldw, F, K)) return APC_ERR_UNSUPPORTED;
-  if (norm_in_product(M, K, glu_tile_of(M, F, K))) return swiglu(A, lda, G, eps, nullptr, W, ldw, out, ldo, M, F, K, stream);
+  if (norm_in_product(M, F, K, glu_tile_of(M, F, K), 32768)) return swiglu(A, lda, G, eps, nullptr, W, ldw, out, ldo, M, F, K, stream);
   float* h = (float*)ws;
   if (const int rc = norm_rows((const float*)A, lda, (const float*)G, eps, h, M, K, stream)) return rc;
   return swiglu(h, K, nullptr, 0.f, h + (size_t)M * K, W, ldw, out, ldo, M, F, K, stream);

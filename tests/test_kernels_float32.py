@@ -209,3 +209,23 @@ def test_few_rows_of_a_short_k(M, N, K):
     many, few = torch.empty(M, N, device=DEV), torch.empty(M, 48, device=DEV)
     assert o.linear_normed(x, g, 1e-5, w, many) and o.linear_normed(x, g, 1e-5, w[:48], few)
     assert torch.equal(many[:, :48], few)                  # (48 outputs: the norm in the product up to 16 rows)
+
+
+# where the norm stands: in the product, or in front of it (many outputs of a K up to 1,024) by two rows a wave or a row a block
+# (rows of more than 512 numbers; of more than 4,096 for however many rows), whose last pass of a slice is whole or not
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3, 32776, 300), (2, 16400, 1024), (16, 16384, 516), (1, 32776, 1028), (17, 40, 508), (17, 40, 516), (512, 40, 1156),
+                                   (513, 40, 1156), (600, 24, 4100), (3, 40, 8196), (40, 24, 16388)])
+def test_rows_behind_a_norm_in_every_form(M, N, K):
+    o, eps = ops(), 1e-5
+    x, g, w = gen(M, K, seed=1) * 2.0, 1.0 + 0.1 * gen(K, seed=2), gen(N, K, seed=3) * 2 * K ** -0.5
+    out, few = torch.empty(M, N, device=DEV), torch.empty(M, 24, device=DEV)
+    assert o.linear_normed(x, g, eps, w, out) and o.linear_normed(x, g, eps, w[:24].contiguous(), few)
+    h = x.double() * torch.rsqrt(x.double().square().mean(1, keepdim=True) + eps) * g.double()
+    bound = product_bound(h, w) + (K / 16 + 16) * U * (h.abs() @ w.double().abs().T)
+    assert ((out.double() - h @ w.double().T).abs() <= bound).all()
+    assert torch.equal(out[:, :24], few)
+    for r in sorted({0, M // 2, M - 1}):
+        alone = torch.empty(1, N, device=DEV)
+        assert o.linear_normed(x[r:r + 1], g, eps, w, alone)
+        assert torch.equal(alone[0], out[r])
