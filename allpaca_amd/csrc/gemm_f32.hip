@@ -488,6 +488,17 @@ int launch_slices(const float* A, int lda, const float* G, float eps, const floa
   return 0;
 }
 
+// Which tiles' blocks go on to further tiles, with a stage's stores and loads between its products.  Time of the form that ends
+// after its tile / of this one, mean over 17 to 2,048 rows x 64 to 32,768 outputs: 32 x 32 tiles (two blocks a unit without it)
+// 0.87-0.95 at every K; 48 x 32 in one round of 256 blocks 0.91-0.99, in more 1.05-1.09 up to K = 1,024 and 1.00-1.03 beyond;
+// 48 x 64 one round 0.92-0.98 up to K = 512, 1.02-1.04 beyond, more rounds 1.01-1.10; 64 x 64 0.84-0.97 up to K = 512, then one
+// round 0.97 up to K = 1,024, else 1.00-1.02.  SwiGLU: 48 x 16 outputs 0.93-1.00, the others as their products.
+bool goes_on(int mt, int nt, bool glu, int M, int N, int K) {
+  const bool rounds = (long long)ceil_div(M, 16 * mt) * ceil_div(N, 16 * (glu ? nt / 2 : nt)) > 256;
+  if (K <= 4 * STAGE || mt * nt < 6 || (mt * nt == 6 && glu)) return false;
+  return mt * nt == 6 ? rounds : mt * nt == 12 ? rounds || K > 512 : K > (rounds ? 512 : 1024);
+}
+
 template <int MT, int NT, int D, bool ONCE, int MIN_WAVES, bool GLU = false>
 int launch(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C, int c_dtype,
            int ldc, int M, int N, int K, int mode, hipStream_t stream) {
@@ -501,15 +512,8 @@ int launch(const float* A, int lda, const float* G, float eps, const float* R, c
     if (K <= 2 * STAGE) SL_GO(2, false);
     if (K <= 4 * STAGE) SL_GO(4, false);
   }
-  // Which tiles' blocks go on to further tiles, with a stage's stores and loads between its products.  Time of the form that ends
-  // after its tile / of this one, mean over 17 to 2,048 rows x 64 to 32,768 outputs: 32 x 32 tiles (two blocks a unit without it)
-  // 0.87-0.95 at every K; 48 x 32 in one round of 256 blocks 0.91-0.99, in more 1.05-1.09 up to K = 1,024 and 1.00-1.03 beyond;
-  // 48 x 64 one round 0.92-0.98 up to K = 512, 1.02-1.04 beyond, more rounds 1.01-1.10; 64 x 64 0.84-0.97 up to K = 512, then one
-  // round 0.97 up to K = 1,024, else 1.00-1.02.  SwiGLU: 48 x 16 outputs 0.93-1.00, the others as their products.
-  if constexpr (MT * NT > 6 || (MT * NT == 6 && !GLU)) {
-    const bool rounds = (long long)ceil_div(M, 16 * MT) * ceil_div(N, 16 * (GLU ? NT / 2 : NT)) > 256;
-    if (MT * NT == 6 ? rounds : MT * NT == 12 ? rounds || K > 512 : K > (rounds ? 512 : 1024)) SL_GO(SLICES, true);
-  }
+  if constexpr (MT * NT > 6 || (MT * NT == 6 && !GLU))
+    if (goes_on(MT, NT, GLU, M, N, K)) SL_GO(SLICES, true);
   SL_GO(SLICES, false);
 #undef SL_GO
 }
@@ -564,6 +568,13 @@ APC_EXPORT int apc_gemm_f32_tile(int M, int N, int K) {
   const TileCost& t = TILES[tile_of(M, N, K)];
   return 16 * t.mt * 1000 + 16 * t.nt;
 }
+
+// Tiles that a block of the product takes at most: 1 where it ends behind its tile.
+static int tiles_a_block(const TileCost& t, bool glu, int M, int N, int K) {
+  const int tiles = ceil_div(M, 16 * t.mt) * ceil_div(N, 16 * (glu ? t.nt / 2 : t.nt));
+  return goes_on(t.mt, t.nt, glu, M, N, K) ? ceil_div(ceil_div(tiles, 8), 32) : 1;
+}
+APC_EXPORT int apc_gemm_f32_tiles_a_block(int M, int N, int K) { return tiles_a_block(TILES[tile_of(M, N, K)], false, M, N, K); }
 
 // Few rows: two stages of loads ahead, not four.  4 rows x 2,048 outputs x K 2,048 7.1 -> 6.7 us, K 8,192 21.5 -> 18.8, 128,256
 // outputs 155 -> 150: the straight code of a stage count's every case is a third as long, and a launch finds it cold.
@@ -654,6 +665,8 @@ APC_EXPORT int apc_swiglu_f32_tile(int M, int F, int K) {
   const TileCost& t = GLU_TILES[glu_tile_of(M, F, K)];
   return 16 * t.mt * 1000 + 8 * t.nt;
 }
+
+APC_EXPORT int apc_swiglu_f32_tiles_a_block(int M, int F, int K) { return tiles_a_block(GLU_TILES[glu_tile_of(M, F, K)], true, M, F, K); }
 
 static int swiglu(const void* A, int lda, const void* G, float eps, const float* R, const void* W, int ldw, void* out, int ldo,
                   int M, int F, int K, hipStream_t stream) {

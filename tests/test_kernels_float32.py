@@ -60,10 +60,23 @@ def test_product_against_64_bits_and_rows_alone(M, N, K):
     assert torch.equal(both, add + out)
 
 
-# more tiles than compute units: a block's second and third tile, with slices of no, one, two and several stages, tiles
-# that a block has one more of than its neighbour, and outputs that are added to
+# more tiles than compute units, on every tile whose blocks go on: a block's second and third tile, with slices of no, one, two
+# and several stages, tiles that a block has one more of than its neighbour, and outputs that are added to
+MORE_TILES = [(700, 4099, 132), (700, 4099, 256), (331, 6145, 300), (720, 3100, 580), (1030, 2045, 776), (517, 2045, 132), (1047, 1001, 520),
+              (305, 6145, 520), (623, 3100, 776)]
+
+
+def test_the_sizes_of_more_tiles_than_units_make_blocks_go_on():
+    from allpaca_amd.kernels import lib
+    L = lib.load("plain")
+    assert all(L.apc_gemm_f32_tiles_a_block(*s) > 1 for s in MORE_TILES)
+    assert {L.apc_gemm_f32_tile(*s) for s in MORE_TILES} == {48032, 48064, 64064}
+    # (a row behind a norm among them: the form with the rows' scales goes on alike)
+    assert L.apc_gemm_f32_tiles_a_block(700, 4099, 256) > 1 and L.apc_gemm_f32_tiles_a_block(16, 128256, 2048) == 1
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(700, 4099, 132), (700, 4099, 256), (331, 6145, 300), (490, 3100, 580), (1030, 2045, 776)])
+@pytest.mark.parametrize("M,N,K", MORE_TILES)
 def test_product_of_more_tiles_than_units(M, N, K):
     test_product_against_64_bits_and_rows_alone(M, N, K)
     a, w = gen(M, K, seed=3), gen(N, K, seed=4)

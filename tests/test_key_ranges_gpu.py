@@ -59,3 +59,25 @@ def test_every_number_of_ranges(monkeypatch, d, window):
         run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500, 130, 77], rows_per_seg=[300, 129, 1], window=window, seed=s, ranges=s,
                       stale=float("nan"))
         run_attention(H=4, Hk=2, d=d, P_=16, lens=[1500], rows_per_seg=[256], window=window, seed=s, ranges=s, loud=(0, 1460, 40.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,d,off,pad", [(4, 64, 4, 4), (4, 128, 0, 4), (6, 64, 8, 8), (40, 64, 4, 12)])
+@pytest.mark.parametrize("ranges", [2, 5])
+def test_ranges_added_into_rows_off_16_bytes(monkeypatch, H, d, off, pad, ranges):
+    """The adding kernel stores 16 bytes where the output's place and its rows allow it, else 8: the same numbers."""
+    from allpaca_amd.engine.batch import Entry, pack_step
+    from test_kernels_tuned import DEV, tuned
+    t, Hk, P_, rows, before = tuned(), H // 2, 16, 200, 900
+    blocks = -(-(before + rows) // P_)
+    step = pack_step([Entry(0, [0] * rows)], [before], [0], [[list(range(1, blocks + 1))]], torch.device(DEV), [0])
+    gen = torch.Generator(device=DEV).manual_seed(H + d)
+    q = torch.randn(rows, H * d, generator=gen, device=DEV).bfloat16()
+    cache = torch.randn(blocks + 1, 2, Hk, P_, d, generator=gen, device=DEV).bfloat16()
+    monkeypatch.setattr(t, "_prompt_ranges", lambda *a: ranges)
+    want = torch.empty(rows, H * d, dtype=torch.bfloat16, device=DEV)
+    wide = torch.full((rows, off + H * d + pad), 9.0, dtype=torch.bfloat16, device=DEV)
+    for out in (want, wide[:, off:off + H * d]):
+        assert t.attention_bf16(q, 0, out, H, Hk, d, cache, P_, step.block_tables[0], step)
+    assert torch.equal(wide[:, off:off + H * d], want)
+    assert (wide[:, :off] == 9.0).all() and (wide[:, off + H * d:] == 9.0).all()

@@ -70,7 +70,7 @@ def test_greedy_rows_and_rows_the_callers_word_was_wrong_about():
 # rules, a greedy row among others, numbers of tokens and seeds at the ends of their ranges
 @pytest.mark.parametrize("R,V", [(1, 4099), (8, 32001), (64, 9001), (65, 5000)])
 @pytest.mark.parametrize("rule", [(0.8, 40, 0.95), (0.7, 0, 0.9), (0.8, 0, 1.0), (1.1, 2000, 0.5), None])
-def test_options_that_go_with_the_launch(R, V, rule):
+def test_options_that_go_with_the_launch(R, V, rule, monkeypatch):
     from allpaca_amd.kernels import ops
     from allpaca_amd.sampling import GenerationParams
     from allpaca_amd.sampling.sampler import Sampler, uniforms_for
@@ -83,10 +83,19 @@ def test_options_that_go_with_the_launch(R, V, rule):
     want = torch.empty(R, dtype=torch.int32, device=DEV)
     ops.sample_rows(logits, f([t for t, _, _ in rules], torch.float32), f([k for _, k, _ in rules], torch.int32), f([p for _, _, p in rules], torch.float32),
                     torch.from_numpy(uniforms_for([5 if s is None else s for s in seeds], numbers)).to(DEV), want, one_block=True)
-    sampler = Sampler(torch.device(DEV), 5)
+    sampler, sample_rows, went = Sampler(torch.device(DEV), 5), ops.sample_rows, []
+
+    def seen(logits, temperature, *a, **kw):
+        done = sample_rows(logits, temperature, *a, **kw)
+        went.append((isinstance(temperature, list), done is not None))
+        return done
+
+    monkeypatch.setattr(ops, "sample_rows", seen)
     for _ in range(3):                                       # (both of the sampler's result buffers)
         pending = sampler.launch(logits, params, numbers)
         assert pending.wait() == want.tolist() == pending.device.tolist()
+    by_value = R <= 64                                       # options with the launch, ids from the kernel to the host
+    assert went == ([] if rule is None and R == 1 else [(by_value, by_value)] * 3)       # (one greedy row: no sampling)
 
 
 def test_options_that_only_the_copy_to_the_device_takes():
@@ -101,3 +110,33 @@ def test_options_that_only_the_copy_to_the_device_takes():
     top = (1 << 64) - 2
     ids = s.sample(logits, params(40), [top, 1 << 63, 0])
     assert ids[2] == s.sample(logits, params(40), [1, 2, 0])[2] and all(0 <= t < 5000 for t in ids)
+
+
+def test_a_result_that_is_dropped_keeps_its_memory_until_the_kernel_is_through():
+    """The memory of a dropped result is nobody else's while the kernel that writes it is behind other work."""
+    from allpaca_amd.kernels import ops
+    from allpaca_amd.sampling import GenerationParams
+    from allpaca_amd.sampling.sampler import Sampler
+    torch.cuda.synchronize()
+    ops.PinnedIds(1)                                         # (what earlier tests left is taken back)
+    held = len(ops._still_written)
+    logits = torch.randn(4, 32000, device=DEV)
+    a = torch.randn(8192, 8192, device=DEV)
+    params = [GenerationParams(temperature=0.8, top_k=40, top_p=0.95, seed=r) for r in range(4)]
+    sampler = Sampler(torch.device(DEV), 5)
+    want = sampler.sample(logits, params, [0] * 4)           # (both buffers have been pinned and the kernels loaded)
+    assert sampler.sample(logits, params, [0] * 4) == want
+    for _ in range(8):
+        a @ a
+    pending = sampler.launch(logits, params, [0] * 4)
+    memory, device = pending.pinned, pending.device
+    addresses = {p.address for p in sampler._pinned}
+    del pending, sampler
+    assert len(ops._still_written) == held + 2 and {m.data_ptr() for m, _ in list(ops._still_written)[held:]} == addresses
+    del memory
+    new = torch.empty(64, dtype=torch.int32).pin_memory()
+    assert new.data_ptr() not in addresses
+    torch.cuda.synchronize()
+    assert device.tolist() == want and list(ops._still_written)[-1][1][-1].query()
+    ops.PinnedIds(1)
+    assert len(ops._still_written) == 0

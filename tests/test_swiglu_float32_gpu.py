@@ -34,8 +34,18 @@ def test_both_products_and_the_activation(M, F, K, pad):
     assert bool((out[:, F:] == 7.0).all())
 
 
+MORE_TILES = [(700, 9000, 132), (331, 9001, 256), (517, 2045, 388), (464, 2045, 520), (888, 1001, 580)]
+
+
+def test_the_sizes_of_more_tiles_than_units_make_blocks_go_on():
+    from allpaca_amd.kernels import lib
+    L = lib.load("plain")
+    assert all(L.apc_swiglu_f32_tiles_a_block(*s) > 1 for s in MORE_TILES)
+    assert {L.apc_swiglu_f32_tile(*s) for s in MORE_TILES} == {48032, 64032}
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,F,K", [(700, 9000, 132), (331, 9001, 256), (200, 8200, 520)])
+@pytest.mark.parametrize("M,F,K", MORE_TILES)
 def test_both_products_of_more_tiles_than_units(M, F, K):
     test_both_products_and_the_activation(M, F, K, 0)
 
