@@ -16,8 +16,7 @@
 // Bound by a fixed part of some 5 us (first loads, the waves' meeting, the store) and the activations' way: with the weights
 // beside them a compute unit gets 33-60 GB/s in all.  Times, and where the tiled kernel is the better one: gemm_rows_takes.
 // K must be a multiple of 64, from 1,024 on; N of 16.
-// The order of additions for an output depends on K alone, with SwiGLU on N and the output's column too (a gated product's
-// bands a block are a matter of N): in either case not on the rows beside it.
+// The order of additions for an output depends on K alone.
 // Reference counterpart: gemm_nt_bf16_tiled_kernel, hip/src/kernels.cpp:634 (no matrix cores there).
 #include "gemm_rows.h"
 #include "host/rules.h"
@@ -112,16 +111,12 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rows_gemm_kernel(const bf16_t* 
   };
 
   // this wave's steps, at least two (GEMM_ROWS_MIN_K); DEPTH loaded ahead, no branch around a load in the loop
-  const int steps = K / 64, lo = wave * steps / WAVES, n = (wave + 1) * steps / WAVES - lo;
-  // SwiGLU's blocks begin at different steps of a wave's range: in step they all ask the same lines of the activations of L2
-  // (64 rows, K 3,072 into 8,192 outputs 23.2 -> 21.6 us, K 2,048 16.7 -> 15.6; the other products 0-3 % slower that way).
-  // Two bands a block gain from six steps a wave on: 17 to 64 rows, 2,048 to 4,096 outputs, of the time in step K 1,024
-  // 1.06-1.13, 2,048 0.99-1.03, 3,072 0.98-1.00, 8,192 0.94-0.99; four bands K 1,024 0.95, 1,536 1.01, 2,048 0.96, 8,192 0.88.
-  const int turn = MODE == R_SWIGLU && (NB == 4 || n >= 6) ? (int)(blockIdx.x / 8 % (unsigned)n) : 0;
-  auto at = [&](int s) { const int u = min(s, n - 1) + turn; return lo + (u >= n ? u - n : u); };
+  const int steps = K / 64, lo = wave * steps / WAVES, n = (wave + 1) * steps / WAVES - lo, last = lo + n - 1;
+  // All blocks walk K in the same order: a SwiGLU whose blocks begin at different steps of a wave's range asks L2 for fewer equal
+  // lines at a time (64 rows, K 3,072 into 8,192 outputs 23.5 us in step, 22.3 so), but adds an output in its own order a block
   RowsSet<MT, NB> set[DEPTH];
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) load_step(set[d], at(d));
+  for (int d = 0; d < DEPTH; ++d) load_step(set[d], min(lo + d, last));
 
   // Behind the first loads: the rows' scale (8 threads a row), and what the finishing waves add to or rotate by
   if constexpr (PRE) {
@@ -166,7 +161,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rows_gemm_kernel(const bf16_t* 
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
       compute(set[d]);
-      load_step(set[d], at(t + d + DEPTH));
+      load_step(set[d], min(lo + t + d + DEPTH, last));
     }
   }
 #pragma unroll

@@ -267,7 +267,7 @@ def test_products_of_17_to_64_rows_in_one_launch_where_that_is_faster(kind, M, N
 
 
 def test_bands_of_gated_products_in_one_launch_do_not_depend_on_the_rows():
-    """Where a block begins in K depends on the bands it takes: they must not change with the rows beside a row."""
+    """Which block an output is in is a matter of N, not of the rows beside a row."""
     from allpaca_amd.kernels import host
     rule = host.load().apc_host_rule_rows_bands
     for N in (16, 320, 1024, 2560, 4080, 4096, 4112, 5120, 8192, 11008, 14336):

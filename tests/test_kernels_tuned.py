@@ -662,8 +662,7 @@ def test_product_for_q_k_v_that_rotates_and_fills_the_pages_equals_the_kernels_o
     assert (results[0][1] != 0).sum() + (results[0][2] != 0).sum() == M * 2 * Hk * d   # every row wrote its k and v, once
 
 
-# two and four bands a block; walks of K in step and (from six steps a wave, or with four bands) from different places, waves
-# with unequal numbers of steps among them; two, three and four groups of 16 rows
+# two and four bands a block, waves with unequal numbers of steps among them; two, three and four groups of 16 rows
 @pytest.mark.parametrize("F,K", [(2048, 1024), (4096, 2048), (1040, 3008), (4096, 3072), (5120, 1024), (8176, 1536), (8192, 3072)])
 def test_a_row_of_a_gated_product_of_17_to_64_rows_does_not_depend_on_the_others(F, K):
     from allpaca_amd.kernels import lib
@@ -678,6 +677,19 @@ def test_a_row_of_a_gated_product_of_17_to_64_rows_does_not_depend_on_the_others
         outs.append(out)
     for out in outs[:-1]:
         assert torch.equal(out, outs[-1][:out.shape[0]])
+
+
+@pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("F,K", [(4096, 3072), (8192, 1024), (8192, 3072)])
+def test_an_output_of_a_gated_product_of_17_to_64_rows_does_not_depend_on_its_block(M, F, K):
+    """The same 16 outputs in every band: all bands are equal, bit for bit."""
+    t = tuned()
+    a = gen(M, K, seed=1, dtype=BF).to(DEV)
+    wg, wu = (gen(16, K, seed=s, dtype=BF).to(DEV).repeat(F // 16, 1) for s in (2, 3))
+    out = torch.empty(M, F, dtype=BF, device=DEV)
+    t.swiglu_bf16(a, pack(wg), pack(wu), out)
+    out = out.view(M, F // 16, 16)
+    assert torch.equal(out, out[:, :1].expand_as(out))
 
 
 # parts: sums of x^2 a row, asked for ahead of the slices up to 64, four a lane or (no multiple of 4) one; off: floats in front of
