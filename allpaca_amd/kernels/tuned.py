@@ -1042,9 +1042,6 @@ def latent_rows_bf16(proj, ld, H, dn, dr, kv, ldkv, c_off, R, norm_w, eps, cos_s
 LATENT_BLOCKS = 256          # blocks that the keys of few rows are cut for (a block a compute unit at a latent of 512)
 LATENT_SPLITS_MAX = 128      # (the adding kernel takes up to 256; 128 was the fastest for one row over 32,768 keys)
 LATENT_DECODE_TILES = 2      # key tiles that a range of a decoded row's keys must keep
-# contexts up to which a decoded row's keys stay one range: 1 to 32 rows, 16 and 32 heads, latents of 128 to 512, two ranges and
-# the kernel that adds them / one, us: 192 keys 8.5-15.3 / 6.3-11.6, 256 keys 8.6-16.1 / 7.2-13.6, 384 keys 8.6-17.8 / 8.9-17.5
-LATENT_ONE_RANGE = 256
 LATENT_RANGE_TILES = 8       # key tiles (of 64) that a range of a prompt tile's keys must keep
 
 
@@ -1086,7 +1083,5 @@ def latent_attention_bf16(q, out, n_heads: int, rank: int, rot_dim: int, pages, 
         n = step.n_decode_rows
         blocks = n * -(-H // (64 if H > 32 else 32))
         splits = max(1, min(LATENT_BLOCKS // blocks, -(-step.max_decode_context // (64 * LATENT_DECODE_TILES)), LATENT_SPLITS_MAX))
-        if step.max_decode_context <= LATENT_ONE_RANGE:
-            splits = 1
         run(step.decode_rows, None, n, 1, splits, "latent_attention_bf16 (decoded rows)")
     return True

@@ -98,7 +98,7 @@ def test_ranges_of_keys_are_added(H, R, dr, blocks, monkeypatch):
 @pytest.mark.parametrize("longest", [191, 254, 255, 256])
 @pytest.mark.parametrize("H, R, dr", [(32, 512, 64), (5, 64, 16)])
 def test_decoded_rows_of_short_contexts(H, R, dr, longest):
-    """Contexts on either side of the one up to which a decoded row's keys stay one range."""
+    """Contexts of up to two ranges, on either side of their ends."""
     segs = [(longest, 1), (63, 1), (0, 1), (128, 1)]
     plant = [(0, 0, 0, 0), (0, 0, H - 1, longest), (1, 0, 0, 63), (3, 0, H - 1, 127)]
     check_latent_attention(H, R, dr, 16, segs, "bfloat16", longest, plant=plant)
