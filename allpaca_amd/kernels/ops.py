@@ -252,9 +252,16 @@ class PinnedIds:
     def __init__(self, n: int):
         self.events = {}                      # of the last kernel of each stream
         for _ in range(len(_still_written)):
-            gone = _still_written.popleft()
-            if not all(e.query() for e in gone[1]):
-                _still_written.append(gone)
+            try:
+                gone = _still_written.popleft()
+            except IndexError:                # another thread has taken the last one
+                break
+            through = False
+            try:
+                through = all(e.query() for e in gone[1])
+            finally:                          # (an event that cannot be asked keeps its memory)
+                if not through:
+                    _still_written.append(gone)
         self.tensor = torch.empty(n, dtype=torch.int32).pin_memory()
         self.size, self.address = n, self.tensor.data_ptr()
 

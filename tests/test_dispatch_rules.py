@@ -132,6 +132,34 @@ def test_memory_that_a_queued_kernel_writes_is_kept_until_it_has(monkeypatch):
     assert tensor() is None
 
 
+def test_memory_for_ids_is_pinned_by_threads_at_a_time_and_kept_by_an_event_that_raises(monkeypatch):
+    import collections
+    import torch
+    from allpaca_amd.kernels import ops
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda self: self)
+    waiting = collections.deque()
+    monkeypatch.setattr(ops, "_still_written", waiting)
+
+    class Emptied:                      # what a thread sees whose last entry another one has just taken
+        def __len__(self):
+            return 1
+
+        def popleft(self):
+            raise IndexError
+
+    def refuses():
+        raise RuntimeError("capturing")
+
+    monkeypatch.setattr(ops, "_still_written", Emptied())
+    assert ops.PinnedIds(4).size == 4
+    monkeypatch.setattr(ops, "_still_written", waiting)
+    entry = (torch.zeros(1), [SimpleNamespace(query=refuses)])
+    waiting.append(entry)
+    with pytest.raises(RuntimeError, match="capturing"):
+        ops.PinnedIds(4)
+    assert list(waiting) == [entry]
+
+
 @pytest.mark.parametrize("Hk,d,page,takes", [(8, 128, 16, 1), (8, 64, 32768, 1), (255, 128, 32768, 1), (256, 128, 32768, 0), (511, 64, 32768, 1),
                                              (512, 64, 32768, 0), (2048, 128, 4096, 0), (8, 128, 65536, 0), (8, 128, 8, 0), (8, 96, 16, 0), (8, 64, 48, 0)])
 def test_pages_that_the_attention_kernel_of_128_rows_takes(Hk, d, page, takes):
