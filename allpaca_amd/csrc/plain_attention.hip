@@ -291,6 +291,9 @@ void launch_f32(const AttArgs& A, hipStream_t stream) {
 // chunk's arithmetic stands between its loads, and what is then read four times comes out of L2.  The heads' sums are the
 // same.  32 heads on 8 kv heads, 4 rows at 101 to 907 keys: heads of 64 18.2 -> 16.2 us, of 128 34.3 -> 28.6; 8 rows at 900
 // keys 19.0 -> 16.9 and 49.2 -> 36.0; 16 rows at 900 keys would go from 23.9 to 34.2 and from 51.3 to 68.5.
+// Long contexts too, where the bytes go past the L2 of one XCD: it is the units that are few, not the bytes.  8 rows at 8,192
+// and 24,000 keys, each from pages that no launch has just read: heads of 64 191 -> 151 and 544 -> 426 us, of 128 460 -> 355 and
+// 1,337 -> 1,023.  Over 1 to 10 rows of 130 to 24,000 keys, groups of 2 to 8 heads, 0.72 to 1.05 of the time, 0.88 in the mean.
 template <int EL>
 void launch_heads(const AttArgs& A, hipStream_t stream) {
   const int group = A.H / A.Hk;

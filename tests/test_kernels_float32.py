@@ -76,7 +76,7 @@ def test_the_sizes_of_more_tiles_than_units_make_blocks_go_on():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", MORE_TILES)
+@pytest.mark.parametrize("M,N,K", MORE_TILES + [(490, 3100, 580)])
 def test_product_of_more_tiles_than_units(M, N, K):
     test_product_against_64_bits_and_rows_alone(M, N, K)
     a, w = gen(M, K, seed=3), gen(N, K, seed=4)

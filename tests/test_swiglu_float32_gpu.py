@@ -45,7 +45,7 @@ def test_the_sizes_of_more_tiles_than_units_make_blocks_go_on():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,F,K", MORE_TILES)
+@pytest.mark.parametrize("M,F,K", MORE_TILES + [(200, 8200, 520)])
 def test_both_products_of_more_tiles_than_units(M, F, K):
     test_both_products_and_the_activation(M, F, K, 0)
 
