@@ -15,12 +15,13 @@
 // What bounds it: with few rows the bytes of W, else the matrix cores' float32 rate (157 TFLOP/s, of which a library
 // product of 8,192^3 reaches 151 and a loop of these instructions 156).  Blocks of the large tiles go on to further tiles
 // with the next one's first loads on their way while the eight waves meet, and a stage's LDS stores and loads stand between
-// its first half's products: 325 rows x 8,192 outputs of SwiGLU 200 -> 187 us, x 2,048 outputs x K 2,048 32.2 -> 29.6, K
-// 8,192 104.9 -> 101 (108 TFLOP/s).  What is left there: the loads (without them, timing only, 14 % less: their way into the
+// its first half's products: 325 rows x 8,192 outputs of SwiGLU 202 -> 186 us, x 2,048 outputs x K 2,048 32.0 -> 30.6, K
+// 8,192 104 -> 99 (110 TFLOP/s).  What is left there: the loads (without them, timing only, 14 % less: their way into the
 // registers beside the products) and, for every tile, 3 us in which the waves meet.  Measured, microseconds (in brackets
 // the kernel of one fma chain an output on the vector units, which takes the other types): 4 rows x 2,048 outputs x K
-// 2,048 7.8; x 128,256 outputs 149 (7.1 TB/s); 325 rows x 16,384 outputs and SwiGLU 187 (about 1,600; 117 TFLOP/s); 2,048
-// rows x 2,048 outputs x K 8,192 519 (132 TFLOP/s).
+// 2,048 6.7; x 128,256 outputs 151 (7.0 TB/s); 325 rows x 8,192 outputs of SwiGLU 186 (about 1,600; 117 TFLOP/s); 2,048
+// rows x 2,048 outputs x K 8,192 512 (134 TFLOP/s).  All times in this file: launches of a graph one behind the other, weights
+// that no launch has just read; inside a step the same products take up to 1 us more.
 #include "mfma.h"
 #include <math.h>
 
@@ -554,7 +555,7 @@ static int least_cost(const TileCost (&shapes)[COUNT], int M, int N, int K, int 
 // The tile: the least expected time.  Fitted to 2,233 products of 17 to 2,048 rows x 64 to 32,768 outputs, K 160 to 14,336, each on
 // all six tiles: the choice takes 1.008 of the best tile's time in the mean, more than 1.03 in 199 of them, 1.22 at worst (100
 // rows x 6,144 outputs, K = 512: 16.4 us, 13.4 on 64 x 64).  K = 2,048: 33 rows x 2,048 outputs 10.1 us (32 x 16 tiles; 32 x 32 13.1),
-// 325 rows 28.2 (48 x 64; 64 x 64 36.4), 2,048 rows 146 (64 x 64; 48 x 64 159); K = 256: 64 rows x 16,384 10.1 (64 x 64).
+// 325 rows 30.6 (48 x 64), 2,048 rows 146 (64 x 64; 48 x 64 159); K = 256: 64 rows x 16,384 10.1 (64 x 64).
 // Up to K = 128 (see launch) blocks of all tiles share their units, and with many outputs tiles that leave the empty slices out
 // are the better ones for few rows too: 16 rows x 128,256 outputs, 32 x 32 / 16 x 16 tiles, K = 32 10.4 / 19.6 us, 64 13.1 / 22.6, 128
 // 22.2 / 25.7; 32,768 outputs 4.5 / 6.7, 5.2 / 7.1.
@@ -581,8 +582,8 @@ static int tiles_a_block(const TileCost& t, bool glu, int M, int N, int K) {
 }
 APC_EXPORT int apc_gemm_f32_tiles_a_block(int M, int N, int K) { return tiles_a_block(TILES[tile_of(M, N, K)], false, M, N, K); }
 
-// Few rows: two stages of loads ahead, not four.  4 rows x 2,048 outputs x K 2,048 7.1 -> 6.7 us, K 8,192 21.5 -> 18.8, 128,256
-// outputs 155 -> 150: the straight code of a stage count's every case is a third as long, and a launch finds it cold.
+// Few rows: two stages of loads ahead, not four.  4 rows x 2,048 outputs x K 2,048 7.2 -> 6.7 us, K 8,192 21.6 -> 19.3 (128,256
+// outputs, K 2,048: 150 and 151): the straight code of a stage count's every case is a third as long, and a launch finds it cold.
 static int product(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C,
                    int c_dtype, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
 #define GO(...) return launch<__VA_ARGS__>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
@@ -607,9 +608,10 @@ int gemm_f32(const float* A, int lda, const float* W, int ldw, void* C, int c_dt
   return product(A, lda, nullptr, 0.f, nullptr, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream);
 }
 
-// C[M,N] = rmsnorm(A; G, eps) . W^T.  Up to 16 rows in one launch: 4 rows x 3,072 outputs x K 2,048 6.9 us without the norm, 7.6
-// with it, and the norm's own launch was 4.7; 6,144 x K 4,096 19.8 and 21.0.  More rows need room for M rows of K and their
-// scales: apc_gemm_norm_f32_kib(M, K) KiB.  A row's outputs do not depend on the rows beside it, nor on M.
+// C[M,N] = rmsnorm(A; G, eps) . W^T.  Up to 16 rows in one launch: 4 rows x 3,072 outputs x K 2,048 7.1 us without the norm, 7.6
+// with it, and the norm's own launch was 4.7; 6,144 x K 4,096 21.6 and 21.0.  More rows need room for M rows of K and their
+// scales: apc_gemm_norm_f32_kib(M, K) KiB; they buy the bits of the few rows, not time (325 rows x 3,072 outputs 51 us, the norm's launch
+// and the product 5 and 46).  A row's outputs do not depend on the rows beside it, nor on M.
 // With a short K and many outputs every block does the norm again for little else: 8 rows x 128,256 outputs, in the product / in
 // front of it, K = 256 44.1 / 32.2 us, 512 62.2 / 45.6, 1,024 90.9 / 80.1 (2,048 on: the other way), 32,768 outputs 13.1 / 12.1,
 // 18.1 / 16.1, 26.1 / 26.0, 14,336 outputs 9.9 / 10.3 at K = 512; SwiGLU at K = 512 of 32,768 outputs 28.1 / 28.3, of 128,256 95.0 / 89.1.
@@ -648,14 +650,14 @@ APC_EXPORT int apc_gemm_norm_f32(const void* A, int lda, const void* G, float ep
 }
 
 // out[M,F] = silu(A . Wg^T) * (A . Wu^T), W = [Wg; Wu] of 2 F rows: the same sums as the product of 2 F outputs, without
-// the pass over them (4.8 us of a layer of 4 rows x 8,192, 7 of one of 340): both products and the activation take 23.0 us
-// with 4 rows of K = 2,048 and 208 with 340.
+// the pass over them (4.8 us of a layer of 4 rows x 8,192, 7 of one of 340): both products and the activation take 22.6 us
+// with 4 rows of K = 2,048 and 210 with 340.
 APC_EXPORT int apc_swiglu_f32_takes(const void* A, int lda, const void* W, int ldw, int F, int K) {
   return gemm_f32_takes(A, lda, W, ldw, K) && ((long long)F + 64) * ldw < (1LL << 29);   // byte offsets of 32 bits
 }
 
 // (1,801 gated products of 17 to 1,024 rows x 64 to 14,336 outputs, K 160 to 8,192: 1.004 of the best tile's time in the mean, 1.10
-// at worst.  K = 2,048, 8,192 outputs: 325 rows 187 us on 48 x 32 tiles, 205 on 48 x 16, 211 on 64 x 32; 100 rows 76 on 64 x 32, 85 on 48 x 32.)
+// at worst.  K = 2,048, 8,192 outputs: 325 rows 186 us on 48 x 32 tiles, 205 on 48 x 16, 211 on 64 x 32; 100 rows 76 on 64 x 32, 85 on 48 x 32.)
 constexpr TileCost GLU_TILES[] = {{1, 2, 2.44, 2.65, 0.55, 5.34, 0.4, 0.16}, {2, 2, 3.03, 1.13, 0.83, 8.93, 0.55, 0.44},
                                   {3, 2, 2.82, 0.89, 1.1, 14.48, 0.55, 0.39}, {3, 4, 2.49, 1.85, 2.2, 24.42, 0.55, 0.0},
                                   {4, 4, 0.55, 1.13, 3.44, 32.83, 0.55, 0.0}};
@@ -698,8 +700,8 @@ APC_EXPORT int apc_swiglu_f32(const void* A, int lda, const void* W, int ldw, vo
   return swiglu(A, lda, nullptr, 0.f, nullptr, W, ldw, out, ldo, M, F, K, stream);
 }
 
-// The same of the normalised rows, out of the rows in front of the norm (4 rows x 8,192 outputs x K 2,048: 22.4 us without the
-// norm, 23.3 with it); the workspace is apc_gemm_norm_f32's.
+// The same of the normalised rows, out of the rows in front of the norm (4 rows x 8,192 outputs x K 2,048: 22.6 us without the
+// norm, 23.8 with it); the workspace is apc_gemm_norm_f32's.
 APC_EXPORT int apc_swiglu_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int F, int K) {
   return apc_swiglu_f32_takes(A, lda, W, ldw, F, K) && G && ((uintptr_t)G & 15u) == 0;
 }

@@ -1026,9 +1026,10 @@ __global__ __launch_bounds__(SNT) void sample_end_kernel(const float* __restrict
 // reference's sequential arithmetic.  A threshold is found by radix descent over the same 64-bit sort key, 11
 // bits a pass, with the histogram in LDS.  What bounds it is latency: each launch is a handful of passes over values that
 // are in L2 after the first, each with two or three barriers; the descents above make five launches of it, each of which
-// begins with where the one before it left off.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 10 + 16 us (the descents:
-// 73 us in seven launches).  Of the 16 us, by clock readings inside the kernel: the pieces' results 2, their candidates 1.6,
-// the selection 4.3, sorting and exponentials 2, the sums in order 3 (7 when every value went from lane to lane).
+// begins with where the one before it left off.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 9.5 + 14.9 us (the descents:
+// 73 us in seven launches).  Of the 14.9 us, by clock readings inside the kernel: the pieces' results 2, their candidates 1.6,
+// the selection 4.3, sorting and exponentials 2, the sums in order 3 (7 when every value went from lane to lane); start and
+// end of the launch are not among them.
 constexpr int FEW_SPARE = 128, FEW_STRIDE = SMALL_MAX + FEW_SPARE;
 constexpr int FEW_BITS = 11, FEW_BINS = 1 << FEW_BITS;
 
@@ -1496,8 +1497,8 @@ APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, 
 // The same for up to 64 rows with their options on the host: they go with the first launch, and the ids also to `out_host` (host
 // memory that the device can write, or null), so that nothing is copied either way.  `options`: n_rows temperatures (float),
 // top-p (float), top-k (int), seeds (uint64) and numbers of the generated token (int64), one behind the other; the uniform number
-// of a row is that of (seed, number).  From the call to the ids on the host, 8 rows of 128,256: top-k 40 and top-p 0.95 86 -> 48
-// us (of which the sums in order above are 4), top-p alone 142 -> 108.
+// of a row is that of (seed, number).  From the call to the ids on the host, 8 rows of 128,256: top-k 40 and top-p 0.95 85 -> 48
+// us (of which the sums in order, 7 -> 3, are 4), top-p alone 142 -> 108.
 APC_EXPORT int apc_sample_rows_host(const float* logits, int ldl, int n_rows, int V, const void* options, int* out, int* out_host,
                                     void* scratch, size_t scratch_bytes, int cuts, hipStream_t stream) {
   if (n_rows <= 0) return 0;
