@@ -27,6 +27,7 @@
 #include "gemm_direct.h"
 #include "host/rules.h"
 #include "mfma.h"
+#include <algorithm>
 
 namespace {
 
@@ -92,7 +93,7 @@ __host__ __device__ constexpr int loads_behind_a() {
 template <int BMG, int NF, int MODE>
 __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                                             const bf16_t* __restrict__ W2, int chunks, void* __restrict__ C, int ldc,
-                                            int M, int N, int K, DirectPre pre = DirectPre{}) {
+                                            int M, int N, int K, int group_rows, DirectPre pre = DirectPre{}) {
   static_assert(R % 2 == 0, "ring slots are static over two stages");
   constexpr int NP = BMG / 2;  // direct loads of A a wave and stage (BMG * 2 fragments over 4 waves)
   constexpr int G = 2 * BMG;   // groups of NF MFMAs a stage: (chunk of 32 columns, row group)
@@ -107,18 +108,18 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
   constexpr int NB = 4 * NOUT * 16;                     // outputs of a block
   int mt, nt;
   {
-    // Consecutive block ids go to the 8 XCDs in turn (an L2 each).  The tiles are put in one order: groups of up to 16
-    // row tiles, inside a group column tile by column tile, row tile fastest; XCD x takes the x-th eighth of that
-    // order, so the blocks that run on an XCD at one time share a few panels of W, and every XCD gets the same number
-    // of tiles whatever the number of column tiles (20 column tiles of 12 rows each dealt out by whole columns gave
-    // four XCDs 36 tiles for their 32 compute units and the others 24: two rounds for 240 tiles).
+    // Consecutive block ids go to the 8 XCDs in turn (an L2 each).  The tiles are put in one order: groups of
+    // `group_rows` row tiles, inside a group column tile by column tile, row tile fastest; XCD x takes the x-th eighth of
+    // that order, so the blocks that run on an XCD at one time share a few panels of A and of W (see rows_together), and
+    // every XCD gets the same number of tiles whatever the number of column tiles (20 column tiles of 12 rows each dealt
+    // out by whole columns gave four XCDs 36 tiles for their 32 compute units and the others 24: two rounds for 240 tiles).
     const int MT = ceil_div(M, BMG * 16), NT = ceil_div(N, NB);
-    constexpr int GM = 16;
     const int per_xcd = ceil_div(MT * NT, 8);
     const int slot = bid / 8;
     const int t = (bid % 8) * per_xcd + slot;
     if (slot >= per_xcd || t >= MT * NT) return;
-    const int group = t / (GM * NT), first_m = group * GM, gsz = min(MT - first_m, GM), r = t - group * GM * NT;
+    const int group = t / (group_rows * NT), first_m = group * group_rows, gsz = min(MT - first_m, group_rows);
+    const int r = t - group * group_rows * NT;
     nt = r / gsz;
     mt = first_m + r % gsz;
   }
@@ -359,8 +360,8 @@ __global__ __launch_bounds__(256, 1) void gemm_direct_kernel(const bf16_t* __res
                                                              const bf16_t* __restrict__ W,
                                                              const bf16_t* __restrict__ W2, int chunks,
                                                              void* __restrict__ C, int ldc, int M, int N, int K,
-                                                             DirectPre pre) {
-  direct_tile<8, NF, MODE>(blockIdx.x, A, lda, W, W2, chunks, C, ldc, M, N, K, pre);
+                                                             int group_rows, DirectPre pre) {
+  direct_tile<8, NF, MODE>(blockIdx.x, A, lda, W, W2, chunks, C, ldc, M, N, K, group_rows, pre);
 }
 
 // K in `gridDim.y` slices of k_slice columns: slice s leaves its float32 sums in partials[s][M][N] (the tiled product's
@@ -369,10 +370,10 @@ template <int NF>
 __global__ __launch_bounds__(256, 1) void gemm_direct_slices_kernel(const bf16_t* __restrict__ A, int lda,
                                                                     const bf16_t* __restrict__ W, int chunks,
                                                                     float* __restrict__ partials, int M, int N,
-                                                                    int k_slice) {
+                                                                    int k_slice, int group_rows) {
   const int s = blockIdx.y;
   direct_tile<8, NF, D_STORE_F32>(blockIdx.x, A + (size_t)s * k_slice, lda, W + (size_t)s * (k_slice / 32) * 512, nullptr,
-                                  chunks, partials + (size_t)s * M * N, N, M, N, k_slice);
+                                  chunks, partials + (size_t)s * M * N, N, M, N, k_slice, group_rows);
 }
 
 // Which NF takes a shape: a launch runs ceil(blocks / 256) rounds of one block a compute unit, and a round of blocks
@@ -398,6 +399,26 @@ int pick_bands(int M, int N, bool swiglu, int k_split = 1, double* cost_out = nu
   return best;
 }
 
+// Row tiles that a launch puts in one group (see direct_tile).  The blocks of an XCD, up to 32 at a time, read every panel of A
+// (128 rows) and of W (`tile_rows_of_w` rows) that they share out of memory once; those bytes are fewest when the rows and
+// the columns of what runs together are about as many.  Groups of one size, the larger one where two are alike.  2,048 rows, groups
+// of 16 / of 8, us: 4,096 outputs, K 4,096 59.9 / 58.0, K 14,336 199 / 188, 6,144 outputs 81.3 / 79.5, SwiGLU of 12,288 outputs
+// 295 / 289; the order of the groups this gives is that of the times for 1,153 and 1,500 rows too (1,153 rows x 8,192 SwiGLU
+// outputs: 10 row tiles in one group 105.4, in two 106.1).
+int rows_together(int M, int N, int nb, int tile_rows_of_w) {
+  const int mt = ceil_div(M, 128);
+  const int here = std::min(32, ceil_div(mt * ceil_div(N, nb), 8));   // tiles that run on an XCD at one time
+  int best = mt;
+  long best_rows = 0;
+  for (int groups = 1; groups <= mt && groups <= 64; ++groups) {
+    const int r = ceil_div(mt, groups);
+    const long rows = std::min(r, here) * 128L + (long)ceil_div(here, r) * tile_rows_of_w;
+    if (!best_rows || rows < best_rows) best = r, best_rows = rows;
+    if (r == 1) break;
+  }
+  return best;
+}
+
 template <int NF, int MODE>
 int launch(const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C, int ldc, int M, int N, int K,
            hipStream_t stream, DirectPre pre) {
@@ -405,7 +426,7 @@ int launch(const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C,
   const long blocks = 8L * ceil_div((long)ceil_div(N, NB) * ceil_div(M, 128), 8L);
   if (blocks > 0x7fffffffL) return APC_ERR_BAD_ARG;
   hipLaunchKernelGGL((gemm_direct_kernel<NF, MODE>), dim3((unsigned)blocks), dim3(256), 0, stream, A, lda, W, W2,
-                     ceil_div(K, 32), C, ldc, M, N, K, pre);
+                     ceil_div(K, 32), C, ldc, M, N, K, rows_together(M, N, NB, 4 * NF * 16), pre);
   APC_LAUNCH_CHECK();
   return 0;
 }
@@ -462,9 +483,10 @@ int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* 
   const long blocks = 8L * ceil_div((long)ceil_div(N, nb) * ceil_div(M, 128), 8L);
   if (blocks > 0x7fffffffL) return APC_ERR_BAD_ARG;
   const dim3 grid((unsigned)blocks, (unsigned)k_split);
+  const int group_rows = rows_together(M, N, nb, nb);
 #define SLICES(NF_)                                                                                              \
   hipLaunchKernelGGL((gemm_direct_slices_kernel<NF_>), grid, dim3(256), 0, stream, A, lda, W, ceil_div(K, 32), partials, \
-                     M, N, k_slice)
+                     M, N, k_slice, group_rows)
   if (nf == 3) SLICES(3);
   else if (nf == 4) SLICES(4);
   else if (nf == 5) SLICES(5);

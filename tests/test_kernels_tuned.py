@@ -83,6 +83,17 @@ def test_gemm_bf16(M, N, K):
     check(f64(acc) - before, want, torch.float32)
 
 
+# row tiles of 128 in groups: 13 in 7 and 6, 12 in 6 and 6, 24 in three of 8, 27 in 7, 7, 7 and 6, 9 in 5 and 4, 17 in one with
+# more than a round of blocks an XCD
+@pytest.mark.parametrize("M,N", [(1560, 4096), (1500, 2048), (2950, 2052), (3330, 1028), (1030, 4096), (2060, 12292)])
+def test_gemm_bf16_of_row_tiles_in_groups(M, N):
+    t = tuned()
+    a, w = gen(M, 128, seed=4, dtype=BF).to(DEV), gen(N, 128, seed=5, dtype=BF).to(DEV)
+    out = torch.full((M, N), 7.0, dtype=torch.float32, device=DEV)
+    t.gemm_bf16(a, pack(w), out)
+    check(f64(out), f64(a) @ f64(w).T, torch.float32)
+
+
 def test_gemm_bf16_strided_views_and_padding_rows_untouched():
     t = tuned()
     big = gen(40, 200, seed=5, dtype=BF).to(DEV)
