@@ -538,6 +538,18 @@ struct KVRegs {
   Frag v[DP / 16];     // 32 positions of 16 value elements per tile
 };
 
+// Two loads of keys as they come, 8 keys x 64 elements each (lane: key lane % 8, 16 bytes (lane % 16 / 8) * 4 + lane / 16 of
+// the 128 of its line), into two operands of 16 keys x 32 elements: the lanes 8-15 of 16 of the first load change places with the
+// lanes 0-7 of the second.
+__device__ __forceinline__ void lines_to_operands(Frag& a, Frag& b) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const int x = (int)a.w[w], y = (int)b.w[w];
+    a.w[w] = (uint32_t)__builtin_amdgcn_update_dpp(x, y, 0x128, 0xf, 0xc, false);   // row_ror:8 into the lanes 8-15
+    b.w[w] = (uint32_t)__builtin_amdgcn_update_dpp(y, x, 0x128, 0xf, 0x3, false);   // and into the lanes 0-7
+  }
+}
+
 // Ways to the finished heads of a (row, kv head):
 //  DEC_PARTS  a block is 4 parts (ranges of KW keys) of the pair; its waves leave their results in `parts` and
 //             attn_merge_kernel, a second launch, finishes.  Kept for the sizes the other two do not take.
@@ -570,6 +582,13 @@ struct KVRegs {
 //             1 to 4 us.
 // The order of additions for a row depends on its position, KW and the number of parts only (DEC_EVEN: on the lengths of
 // the rows in front of it too).
+// LINES (heads of 64 and 128, pages of a power of two): a load of keys asks for 8 whole lines of 128 bytes instead of 16 half
+// ones, and 24 moves between the lanes of a row of 16 a 16 keys of a head of 128 make operands of two such loads; the page
+// of a group of 8 keys is one value for the wave, so places are scalar work and no look-up goes through LDS.  What bounds
+// the kernel beside its bytes is the chain to the first keys and what a unit's loads cost (half lines leave the L2 at a third of
+// the rate).  One layer, 32 heads over 8, without / with, us: heads of 128, 1 row x 387 keys 11.6 / 11.0, 8 x 2,048 19.4 / 18.4,
+// 64 x 100 13.5 / 10.3, 64 x 1,024 49.8 / 45.9, 64 rows of 90 to 2,100 (DEC_EVEN) 40.3 / 37.6; heads of 64, 1 x 387 8.8 / 8.2,
+// 8 x 2,048 12.7 / 12.3, 64 x 2,048 47.3 / 45.6; of 60 measured sizes none is slower.  The same bits.
 constexpr int NW = 4;  // waves of a block of the decode kernel
 constexpr int LAST_DIRECT = 8;  // up to so many blocks a pair the last one reads the others' results in one go
 enum { DEC_PARTS = 0, DEC_WHOLE = 1, DEC_LAST = 2, DEC_EVEN = 3 };
@@ -642,7 +661,7 @@ __host__ __device__ inline EvenRoom even_room(int G, int d, int waves, int tile)
   const long long place = (long long)waves * 2 * (d + 4), first = tile * place * (G < 16 ? G : 16);
   return {heads, d + 4, first, first + place * heads};
 }
-template <int DP, int MODE>
+template <int DP, int MODE, bool LINES>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
     const bf16_t* __restrict__ q, int ldq, int q_off, int H, int Hk, int d, const bf16_t* __restrict__ cache, int P,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ positions,
@@ -651,7 +670,8 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
   constexpr bool WHOLE = MODE == DEC_WHOLE, LAST = MODE == DEC_LAST, EVEN = MODE == DEC_EVEN;
   __shared__ __attribute__((aligned(16))) bf16_t Ps[NW * 16 * (32 + KPAD)];
   extern __shared__ __attribute__((aligned(16))) float meet[];  // WHOLE, LAST: [NW][heads of the tile][d + 2]
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  static_assert(!LINES || DP % 64 == 0, "whole lines of 64 elements");
+  const int lane = threadIdx.x % WAVE, wave = LINES ? __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) : threadIdx.x / WAVE;
   const int li = lane % 16, lc = lane / 16;
   const int G = H / Hk, gtiles = (G + 15) / 16;
   const int ri = blockIdx.x;
@@ -710,7 +730,27 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
   // position is read from that position instead (its score is masked), an element beyond d from element 0 or
   // d - 1 (the query is zero there; such output columns are not stored), so the loads of the next 32 keys can be
   // in flight while these are used.
+  const int lgP = LINES ? 31 - __builtin_clz(P) : 0;
   auto load_kv = [&](KVRegs<DP>& r, int kb) {
+    if constexpr (LINES) {
+      const int last8 = pos & ~7;          // the group of 8 keys with the row's own: what lies beyond is read from there
+      size_t at[4];                        // of the groups' keys 0 in the head's part of the cache
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const int g0 = min(kb + 8 * h, last8), rr = min(li % 8, pos - g0);
+        const int page = __builtin_amdgcn_readlane(my_page, (g0 >> lgP) - page0);
+        at[h] = (size_t)page * page_stride + head_off;
+        const bf16_t* krow = cache + at[h] + (size_t)(g0 & (P - 1)) * DP + (rr * DP + ((li / 8) * 4 + lc) * 8);
+        at[h] += v_off + (g0 & (P - 1));
+#pragma unroll
+        for (int kp = 0; kp < DP / 64; ++kp) r.k[h / 2][2 * kp + h % 2] = load_frag_once(krow + kp * 64);
+      }
+      const size_t mine = lc == 0 ? at[0] : lc == 1 ? at[1] : lc == 2 ? at[2] : at[3];
+      const bf16_t* vbase = cache + mine + (size_t)li * P;
+#pragma unroll
+      for (int dt = 0; dt < DP / 16; ++dt) r.v[dt] = load_frag_once(vbase + (size_t)dt * 16 * P);
+      return;
+    }
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
       const int t = min(kb + nt * 16 + li, pos);
@@ -744,6 +784,10 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
       s[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (LINES) {
+#pragma unroll
+        for (int kp = 0; kp < DP / 64; ++kp) lines_to_operands(r.k[nt][2 * kp], r.k[nt][2 * kp + 1]);
+      }
 #pragma unroll
       for (int ks = 0; ks < DP / 32; ++ks) s[nt] = mfma16(r.k[nt][ks], qf[ks], s[nt]);
     }
@@ -1224,6 +1268,11 @@ static bool last_fits(int G, int d, int n_parts) {
   return whole_fits(G, d) && (n_parts + NW - 1) / NW <= 2 * (d + 2);
 }
 
+// Whether the decode kernel asks for keys in whole lines (see lines_to_operands).
+static bool whole_lines(int d, int page_tokens) {
+  return (d == 64 || d == 128) && (page_tokens & (page_tokens - 1)) == 0;
+}
+
 // Three ways (see attn_decode_kernel), chosen by the operands:
 //   workspace null                every (row, kv head) is one block that finishes its heads itself
 //                                 (`apc_attention_decode_whole_fits` says whether it can; n_parts is not used);
@@ -1248,8 +1297,9 @@ APC_EXPORT int apc_attention_decode_bf16(const void* q, int ldq, int q_off, void
   const int G = H / Hk, gtiles = (G + 15) / 16;
   if (Hk * gtiles > 65535 || H > 65535) return APC_ERR_BAD_ARG;
   const size_t lds = (size_t)NW * (G < 16 ? G : 16) * (d + 2) * sizeof(float);
+  const bool lines = whole_lines(d, page_tokens);
 #define DEC_LAUNCH(DP_, MODE_, GRID_, LDS_, PARTS_, WS_, CTR_)                                                         \
-  hipLaunchKernelGGL((attn_decode_kernel<DP_, MODE_>), GRID_, dim3(NW * 64), LDS_, stream, (const bf16_t*)q, ldq, q_off, \
+  hipLaunchKernelGGL((lines ? attn_decode_kernel<DP_, MODE_, DP_ == 64 || DP_ == 128> : attn_decode_kernel<DP_, MODE_, false>), GRID_, dim3(NW * 64), LDS_, stream, (const bf16_t*)q, ldq, q_off, \
                      H, Hk, d, (const bf16_t*)cache, page_tokens, block_table, max_blocks, positions, row_seg, rows,   \
                      window, scale, keys_per_part, PARTS_, WS_, (bf16_t*)out, ldo, CTR_)
 #define DEC_BY_HEAD(MODE_, GRID_, LDS_, PARTS_, WS_, CTR_)            \
@@ -1318,6 +1368,7 @@ APC_EXPORT int apc_attention_decode_even_bf16(const void* q, int ldq, int q_off,
   if (tiles > 65535) return APC_ERR_BAD_ARG;
   if (ldo % 4 || ((uintptr_t)out & 7u)) return APC_ERR_UNSUPPORTED;  // outputs are stored 8 bytes at a time
   const int keys_per_part = 0;
+  const bool lines = whole_lines(d, page_tokens);
   dim3 grid(even_blocks(H, Hk), tiles);
   DEC_BY_HEAD(DEC_EVEN, grid, 0, n_rows, workspace, counters);
 #undef DEC_BY_HEAD

@@ -1086,6 +1086,16 @@ def test_attention_decode_of_many_rows_takes_the_one_block_kernel_by_itself():
         run_attention(H=16, Hk=8, d=64, P_=16, lens=lens, rows_per_seg=[1] * len(lens), seed=3, entry="apc_attention_decode_bf16")
 
 
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("P_", [8, 16, 24, 64])
+@pytest.mark.parametrize("d", [64, 128])
+def test_attention_decode_of_contexts_that_end_anywhere_in_a_group_of_keys(monkeypatch, d, P_, window, decode_path):
+    """Keys come 8 at a time in whole lines (heads of 64 and 128, pages of a power of two; by halves of lines otherwise): rows that
+    end at every place of a group, of a step of 32 keys and of a page, with what lies behind them far larger."""
+    lens = list(range(1, 71)) + [127, 128, 129, 255, 256, 257]
+    run_attention(H=6, Hk=2, d=d, P_=P_, lens=lens, rows_per_seg=[1] * len(lens), window=window, seed=d + P_, stale=300.0)
+
+
 def test_attention_finds_a_far_key_in_every_path(monkeypatch):
     t = tuned()
     from allpaca_amd.engine.batch import Entry, pack_step
