@@ -33,10 +33,12 @@ namespace {
 
 // D_..._PRE: A is a row that a product into the residual left for the RMS norm, and the sums are scaled by the row's
 // 1 / sqrt(mean of x^2 + eps).  D_ACC_EMIT: add into the residual and leave that row for the norm that reads it next.
+// D_QKV: the outputs are the heads of q, k and v; q and k are rotated, k and v go to the pages (see DirectRope).
 enum { D_STORE_BF16 = 0, D_STORE_F32 = 1, D_ACC_F32 = 2, D_SWIGLU = 3, D_SWIGLU_PRE = 4, D_ACC_EMIT = 5,
-       D_STORE_BF16_PRE = 6, D_STORE_ACT = 7 };
+       D_STORE_BF16_PRE = 6, D_STORE_ACT = 7, D_QKV = 8, D_QKV_PRE = 9 };
 __host__ __device__ constexpr bool is_swiglu(int mode) { return mode == D_SWIGLU || mode == D_SWIGLU_PRE; }
-__host__ __device__ constexpr bool is_pre(int mode) { return mode == D_SWIGLU_PRE || mode == D_STORE_BF16_PRE; }
+__host__ __device__ constexpr bool is_pre(int mode) { return mode == D_SWIGLU_PRE || mode == D_STORE_BF16_PRE || mode == D_QKV_PRE; }
+__host__ __device__ constexpr bool is_qkv(int mode) { return mode == D_QKV || mode == D_QKV_PRE; }
 
 // What goes with a norm folded into the product.  PRE: ss [M][parts] sums of x^2 of the rows (read), eps.
 // EMIT: g the norm's weight [N]; raw [M][ldr] takes bfloat16(x g); ss [M][parts] takes the sums of x^2 of the block's
@@ -50,6 +52,23 @@ struct DirectPre {
   int ldr;
   int part0;
   int act;           // D_STORE_ACT: the activation on the sums
+};
+
+// D_QKV: W is [(H + 2 Hk) d, K], heads in the order q, k, v, d 64 or 128.  The sums are rounded to bfloat16, q and k turned by
+// the row's position (pairs (e, e + d / 2)); q goes to C, k to cache[page][0][kv head][slot][:], v to cache[page][1][kv
+// head][:][slot], page = block_table[row_seg][pos / P], slot = pos % P.  A wave takes the bands of 16 outputs in pairs j, j + d / 32
+// of one head, the same j in all of its heads, so that a lane holds both elements of its pairs and one place of the angles' table
+// serves all heads of a row.  What it costs beside the store that it replaces is the trip for the angles, 1-2 us; what falls away
+// is a launch that reads and writes q, k and v (the two of them, us, K = the width, without / with): 2,048 rows into 6,144
+// outputs of an 8B model DQ0, 1,153 rows into 5,120 of a 3B model DQ1, 1,500 into 3,072 of a 1B model DQ2.
+struct DirectRope {
+  const float* cos_sin;     // [positions][2][d / 2]
+  const int* positions;     // [M]
+  const int* row_seg;       // [M]
+  const int* block_table;   // [segments][max_blocks]
+  int max_blocks;
+  bf16_t* cache;
+  int P, H, Hk, d;
 };
 
 constexpr int R = 4;           // ring slots of W fragments: loads run R - 1 steps of 32 columns ahead
@@ -93,7 +112,8 @@ __host__ __device__ constexpr int loads_behind_a() {
 template <int BMG, int NF, int MODE>
 __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                                             const bf16_t* __restrict__ W2, int chunks, void* __restrict__ C, int ldc,
-                                            int M, int N, int K, int group_rows, DirectPre pre = DirectPre{}) {
+                                            int M, int N, int K, int group_rows, DirectPre pre = DirectPre{},
+                                            DirectRope rope = DirectRope{}) {
   static_assert(R % 2 == 0, "ring slots are static over two stages");
   constexpr int NP = BMG / 2;  // direct loads of A a wave and stage (BMG * 2 fragments over 4 waves)
   constexpr int G = 2 * BMG;   // groups of NF MFMAs a stage: (chunk of 32 columns, row group)
@@ -126,13 +146,19 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
   const int m0 = mt * BMG * 16;
   const int bands = (N + 15) / 16;
   const int band0 = nt * (4 * NOUT) + wave * NOUT;  // first band of this wave
-  const int base_band = min(band0, bands - 1);
+  // (D_QKV: band f of this wave is half f % 2 of its pair f / 2)
+  const int qkv_j = rope.d == 128 ? wave : wave % 2;
+  const int qkv_head0 = is_qkv(MODE) ? nt * (NB / rope.d) + (rope.d == 128 ? 0 : wave / 2 * (NF / 2)) : 0;
+  const int base_band = is_qkv(MODE) ? nt * (NB / 16) : min(band0, bands - 1);
   const BufferRsrc abuf = make_rsrc(A + (size_t)m0 * lda);
   const BufferRsrc wbuf = make_rsrc(W + (size_t)base_band * chunks * 512);
   const BufferRsrc ubuf = make_rsrc((is_swiglu(MODE) ? W2 : W) + (size_t)base_band * chunks * 512);
   int woff[NF];  // SwiGLU: NOUT gate bands, then the same bands of up
 #pragma unroll
-  for (int f = 0; f < NF; ++f) woff[f] = (min(band0 + f % NOUT, bands - 1) - base_band) * chunks * 1024 + lane * 16;
+  for (int f = 0; f < NF; ++f) {
+    const int band = is_qkv(MODE) ? (qkv_head0 + f / 2) * (rope.d / 16) + qkv_j + f % 2 * (rope.d / 32) : band0 + f % NOUT;
+    woff[f] = (min(band, bands - 1) - base_band) * chunks * 1024 + lane * 16;
+  }
   // This wave's pieces of A in a stage, 8 rows x 64 columns each: lane -> (row lane / 8, 16 bytes lane % 8 ^ row), so that
   // an instruction asks for eight whole lines of 128 bytes
   int aoff[NP];
@@ -146,6 +172,13 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
 #pragma unroll
     for (int f = 0; f < NF; ++f) acc[a][f] = floatx4{0.f, 0.f, 0.f, 0.f};
 
+  // D_QKV: position and segment of a row of the block, a thread a row, asked for ahead of the first loads; the page
+  // is looked up behind the loop, beside the angles
+  int my_pos = 0, my_seg = 0;
+  if constexpr (is_qkv(MODE)) {
+    my_pos = rope.positions[min(m0 + tid % (BMG * 16), M - 1)];
+    my_seg = rope.row_seg[min(m0 + tid % (BMG * 16), M - 1)];
+  }
   const int ktiles = K / 64;
   auto a_piece = [&](int kt, int p) {  // piece p (0..NP-1) of this wave's share of stage kt
     load_to_lds(abuf, &As[kt % S][wave * NP + p][0], aoff[p], min(kt, ktiles - 1) * 128);
@@ -237,6 +270,73 @@ __device__ __forceinline__ void direct_tile(int bid, const bf16_t* __restrict__ 
     __syncthreads();
 #pragma unroll
     for (int a = 0; a < BMG; ++a) row_scale[a] = scales[a * 16 + mi];
+  }
+  if constexpr (is_qkv(MODE)) {
+    // [position, page, slot][BMG * 16], in the LDS that the stages have left (behind the scales; with an array of its own the
+    // compiler set waits between the loop's direct loads)
+    int(*row_at)[BMG * 16] = reinterpret_cast<int(*)[BMG * 16]>(&As[0][2][0]);
+    const int my_page = rope.block_table[(size_t)my_seg * rope.max_blocks + my_pos / rope.P];
+    __syncthreads();
+    if (tid < BMG * 16) {
+      row_at[0][tid] = my_pos;
+      row_at[2][tid] = my_pos % rope.P;
+    }
+    __syncthreads();
+    const int d = rope.d, half = d / 2, e = qkv_j * 16 + nq * 4;
+    const size_t page_stride = (size_t)2 * rope.Hk * rope.P * d;
+    floatx4 cs[BMG], sn[BMG];   // the angles of all row groups first: one trip
+#pragma unroll
+    for (int a = 0; a < BMG; ++a) {
+      const float* at = rope.cos_sin + (size_t)row_at[0][a * 16 + mi] * d + e;
+      cs[a] = *reinterpret_cast<const floatx4*>(at);
+      sn[a] = *reinterpret_cast<const floatx4*>(at + half);
+    }
+    if (tid < BMG * 16) row_at[1][tid] = my_page;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NF / 2; ++k) {
+      const int head = qkv_head0 + k;
+      if (head >= rope.H + 2 * rope.Hk) continue;
+#pragma unroll
+      for (int a = 0; a < BMG; ++a) {
+        const int m = m0 + a * 16 + mi;
+        if (m >= M) continue;
+        bf16_t lo[4], hi[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          lo[r] = float_to_bf16(is_pre(MODE) ? acc[a][2 * k][r] * row_scale[a] : acc[a][2 * k][r]);
+          hi[r] = float_to_bf16(is_pre(MODE) ? acc[a][2 * k + 1][r] * row_scale[a] : acc[a][2 * k + 1][r]);
+        }
+        const int slot = row_at[2][a * 16 + mi];
+        bf16_t* page = rope.cache + (size_t)row_at[1][a * 16 + mi] * page_stride;
+        if (head < rope.H + rope.Hk) {
+          float ya[4], yb[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float av = bf16_to_float(lo[r]), bv = bf16_to_float(hi[r]), c = cs[a][r], sv = sn[a][r];
+            ya[r] = av * c - bv * sv;
+            yb[r] = av * sv + bv * c;
+          }
+          bf16_t* dst = head < rope.H ? (bf16_t*)C + (size_t)m * ldc + (size_t)head * d
+                                      : page + ((size_t)(head - rope.H) * rope.P + slot) * d;
+          uint2 oa, ob;
+          oa.x = pack_bf16x2(ya[0], ya[1]);
+          oa.y = pack_bf16x2(ya[2], ya[3]);
+          ob.x = pack_bf16x2(yb[0], yb[1]);
+          ob.y = pack_bf16x2(yb[2], yb[3]);
+          *reinterpret_cast<uint2*>(dst + e) = oa;
+          *reinterpret_cast<uint2*>(dst + e + half) = ob;
+        } else {   // (16 lanes have 16 rows of one column: slots side by side where the rows are a prompt's)
+          bf16_t* col = page + ((size_t)(rope.Hk + head - rope.H - rope.Hk) * d + e) * rope.P + slot;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            col[(size_t)r * rope.P] = lo[r];
+            col[(size_t)(half + r) * rope.P] = hi[r];
+          }
+        }
+      }
+    }
+    return;
   }
   float emit_sq[BMG];
 #pragma unroll
@@ -364,6 +464,13 @@ __global__ __launch_bounds__(256, 1) void gemm_direct_kernel(const bf16_t* __res
   direct_tile<8, NF, MODE>(blockIdx.x, A, lda, W, W2, chunks, C, ldc, M, N, K, group_rows, pre);
 }
 
+template <int NF, int MODE>
+__global__ __launch_bounds__(256, 1) void gemm_direct_qkv_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+                                                                 int chunks, bf16_t* __restrict__ q_out, int ldq, int M, int N, int K,
+                                                                 int group_rows, DirectPre pre, DirectRope rope) {
+  direct_tile<8, NF, MODE>(blockIdx.x, A, lda, W, nullptr, chunks, q_out, ldq, M, N, K, group_rows, pre, rope);
+}
+
 // K in `gridDim.y` slices of k_slice columns: slice s leaves its float32 sums in partials[s][M][N] (the tiled product's
 // finishing kernel adds the slices in order and runs the epilogue).
 template <int NF>
@@ -444,7 +551,7 @@ int launch_mode(int nf, const bf16_t* A, int lda, const bf16_t* W, const bf16_t*
 }
 
 bool direct_takes(int mode, const void* A, int lda, const void* C, int ldc, int M, int N, int K) {
-  if (mode < 0 || mode > D_STORE_ACT || M <= 0 || K < 128 || K % 128 || N % 4 || ldc % 4) return false;
+  if (mode < 0 || mode > D_QKV_PRE || M <= 0 || K < 128 || K % 128 || N % 4 || ldc % 4) return false;
   if (((uintptr_t)A & 15u) || ((uintptr_t)C & 15u) || lda % 8) return false;
   // the lanes' byte offsets into the block's rows of A and the wave's bands of W are 32-bit
   if ((long)128 * lda * 2 >= 0x7fffffffL || (long)8 * ceil_div(K, 32) * 1024 >= 0x7fffffffL) return false;
@@ -524,13 +631,13 @@ int launch_columns(int nf, int mode, const bf16_t* A, int lda, const bf16_t* W, 
 // of 0.72 of the time).  3 time units for the second launch.
 struct ColumnPlan {
   int nf1, cols1, nf2;  // cols1 == 0: one launch
+  double cost;          // time units, see pick_bands
 };
 ColumnPlan plan_columns(int M, int N, bool swiglu) {
   double whole = 0.0;
   const int nf = pick_bands(M, N, swiglu, 1, &whole);
   const int mt = ceil_div(M, 128);
-  ColumnPlan plan{nf, 0, 0};
-  double best = whole;
+  ColumnPlan plan{nf, 0, 0, whole};
   if (mt <= 256) {
     for (int f : {3, 4, 5, 6, 8}) {
       if (swiglu && f % 2) continue;
@@ -540,7 +647,7 @@ ColumnPlan plan_columns(int M, int N, bool swiglu) {
       double rest = 0.0;
       const int rf = pick_bands(M, N - big_cols * nb, swiglu, 1, &rest);
       const double cost = (double)ceil_div((long)big_cols * mt, 256L) * round_cost(f) + rest + 3.0;
-      if (cost < 0.97 * best) best = cost, plan = ColumnPlan{f, big_cols * nb, rf};
+      if (cost < 0.97 * plan.cost) plan = ColumnPlan{f, big_cols * nb, rf, cost};
     }
   }
   return plan;
@@ -636,4 +743,74 @@ int launch_gemm_direct_emit(const bf16_t* A, int lda, const bf16_t* W, float* C,
   pre.ldr = ldr;
   pre.part0 = 0;
   return launch_direct(D_ACC_EMIT, A, lda, W, nullptr, C, ldc, M, N, K, stream, pre);
+}
+
+// The product for q, k and v that rotates and fills the pages (D_QKV).
+namespace {
+// Whole heads in pairs of bands want tiles of 4, 6 or 8 bands a wave.
+int qkv_bands(int M, int N, double* cost) {
+  int best = 0;
+  for (int nf : {4, 6, 8}) {
+    const double c = (double)ceil_div((long)ceil_div(M, 128) * ceil_div(N, 64 * nf), 256L) * round_cost(nf);
+    if (!best || c <= *cost) best = nf, *cost = c;
+  }
+  return best;
+}
+
+template <int MODE>
+int launch_qkv(const bf16_t* A, int lda, const bf16_t* W, bf16_t* q_out, int ldq, int M, int N, int K, DirectPre pre, DirectRope rope,
+               hipStream_t stream) {
+  double cost = 0.0;
+  const int nf = qkv_bands(M, N, &cost), nb = 64 * nf;
+  const long blocks = 8L * ceil_div((long)ceil_div(N, nb) * ceil_div(M, 128), 8L);
+  if (blocks > 0x7fffffffL) return APC_ERR_BAD_ARG;
+#define QKV(NF_)                                                                                                               \
+  hipLaunchKernelGGL((gemm_direct_qkv_kernel<NF_, MODE>), dim3((unsigned)blocks), dim3(256), 0, stream, A, lda, W, ceil_div(K, 32), \
+                     q_out, ldq, M, N, K, rows_together(M, N, nb, nb), pre, rope)
+  if (nf == 4) QKV(4);
+  else if (nf == 6) QKV(6);
+  else QKV(8);
+#undef QKV
+  APC_LAUNCH_CHECK();
+  return 0;
+}
+}  // namespace
+
+// Whether the next entry point takes these sizes and is expected to be faster than the product and the kernel that rotates and
+// fills the pages, one after the other: the tiles that it does not have (3 and 5 bands a wave, columns in two launches) against
+// that kernel's time (us, 7 and 0.42 a million outputs: 12.1, 10.2 and 9.4 measured for 2,048 x 6,144, 1,153 x 5,120 and 1,500 x
+// 3,072) less 1.5 for what the epilogue costs.
+APC_EXPORT int apc_gemm_direct_qkv_takes(const void* A, int lda, const void* q_out, int ldq, int M, int K, int H, int Hk, int d,
+                                         const void* cos_sin, const void* cache) {
+  if (M <= 0 || H <= 0 || Hk <= 0 || (d != 64 && d != 128) || lda < K || ldq < H * d) return 0;
+  const int N = (H + 2 * Hk) * d;
+  if (!enough_tiles(M, N, false) || !direct_takes(D_QKV, A, lda, q_out, ldq, M, N, K)) return 0;
+  if ((long)32 * ceil_div(K, 32) * 1024 >= 0x7fffffffL) return 0;   // a block's bands of W, 32-bit offsets from its first
+  if (((uintptr_t)cos_sin & 15u) || ((uintptr_t)cache & 7u)) return 0;
+  double fused = 0.0;
+  qkv_bands(M, N, &fused);
+  const double units = K / 4096.0, apart = plan_columns(M, N, false).cost * units + 7.0 + 0.42e-6 * M * N;
+  return fused * units + 1.5 < apart ? 1 : 0;
+}
+
+// q, k and v of M rows in one product, q and k rotated, k and v written into the paged cache (see DirectRope).  W: tiled layout of
+// [(H + 2 Hk) d, K]; q_out [M, ldq] takes the rotated q heads in its first H d columns.  With ss [M][ss_parts]: A is a row that a
+// product into the residual left, and the sums are scaled by 1 / sqrt(sum(ss[m]) / K + eps).
+APC_EXPORT int apc_gemm_direct_qkv_rope_bf16(const void* A, int lda, const float* ss, int ss_parts, float eps, const void* W,
+                                             void* q_out, int ldq, int M, int K, int H, int Hk, int d, const float* cos_sin,
+                                             const int* positions, const int* row_seg, const int* block_table, int max_blocks,
+                                             void* cache, int page_tokens, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (!W || !q_out || !cos_sin || !positions || !row_seg || !block_table || max_blocks <= 0 || !cache || page_tokens <= 0 ||
+      (ss && ss_parts <= 0))
+    return APC_ERR_BAD_ARG;
+  if (!apc_gemm_direct_qkv_takes(A, lda, q_out, ldq, M, K, H, Hk, d, cos_sin, cache) || ((uintptr_t)W & 15u)) return APC_ERR_UNSUPPORTED;
+  const DirectRope rope{cos_sin, positions, row_seg, block_table, max_blocks, (bf16_t*)cache, page_tokens, H, Hk, d};
+  DirectPre pre{};
+  pre.ss = const_cast<float*>(ss);
+  pre.parts = ss_parts;
+  pre.eps = eps;
+  const int N = (H + 2 * Hk) * d;
+  return ss ? launch_qkv<D_QKV_PRE>((const bf16_t*)A, lda, (const bf16_t*)W, (bf16_t*)q_out, ldq, M, N, K, pre, rope, stream)
+            : launch_qkv<D_QKV>((const bf16_t*)A, lda, (const bf16_t*)W, (bf16_t*)q_out, ldq, M, N, K, pre, rope, stream);
 }

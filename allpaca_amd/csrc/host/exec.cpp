@@ -373,10 +373,12 @@ int qkv_rope(Program& P, const Buf& a, const Emit* pre, const ApcLayer& L, const
   if (few && !(d % 32 == 0 && qkv.ld % 4 == 0 && ((uintptr_t)qkv.p & 7u) == 0)) return 0;
   const int ks = few ? 1 : tiled_k_split(M, N, K);
   const bool rows = !few && apc_gemm_rows_qkv_takes(a.p, a.ld, L.w_qkv.data, qkv.p, qkv.ld, M, K, H, Hk, d, L.cos_sin, E.kv);
-  if (!few && ((ks == 1 && !rows) || 256 % d || d % 2)) return 0;
+  const bool direct = !few && ks == 1 && !rows &&
+                      apc_gemm_direct_qkv_takes(a.p, a.ld, qkv.p, qkv.ld, M, K, H, Hk, d, L.cos_sin, E.kv) != 0;
+  if (!few && !direct && ((ks == 1 && !rows) || 256 % d || d % 2)) return 0;
   if (pre) {
     if (few && !pre_ok_skinny(*pre, K)) return 0;
-    if (!few && !(pre->ss_rows == M && pre->ss_cols >= 1 && pre->ss_cols <= ss_parts_max(M))) return 0;
+    if (direct ? !(pre->ss_rows == M && pre->ss_cols >= 1) : !few && !(pre->ss_rows == M && pre->ss_cols >= 1 && pre->ss_cols <= ss_parts_max(M))) return 0;
   }
   if (L.w_qkv.K != K || L.w_qkv.N != N || qkv.rows != M || qkv.cols < H * d) return -1;
   const ApcStep& s = P.step;
@@ -387,6 +389,13 @@ int qkv_rope(Program& P, const Buf& a, const Emit* pre, const ApcLayer& L, const
            apc_skinny_qkv_rope_bf16(a.p, a.ld, pre ? pre->ss : nullptr, pre ? (int)cdiv(K, 16) : 0, pre ? pre->eps : 0.f,
                                     L.w_qkv.data, qkv.p, qkv.ld, M, K, H, Hk, d, L.cos_sin, s.positions,
                                     s.row_seg, table, width, E.kv, E.page_tokens, P.stream));
+    return 1;
+  }
+  if (direct) {
+    LAUNCH(P, "gemm_direct_qkv_rope_bf16",
+           apc_gemm_direct_qkv_rope_bf16(a.p, a.ld, pre ? pre->ss : nullptr, pre ? pre->ss_cols : 0, pre ? pre->eps : 0.f,
+                                         L.w_qkv.data, qkv.p, qkv.ld, M, K, H, Hk, d, L.cos_sin, s.positions, s.row_seg, table,
+                                         width, E.kv, E.page_tokens, P.stream));
     return 1;
   }
   float* ws = rows ? nullptr : P.floats((size_t)ks * M * N);

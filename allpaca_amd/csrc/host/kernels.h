@@ -47,6 +47,11 @@ int apc_gemm_splitk_emit_bf16(const void* A, int lda, const void* W, void* C, in
 int apc_gemm_splitk_pre_bf16(const void* A, int lda, const float* ss, int ss_parts, float eps, const void* W,
                              const void* Wu, void* C, int ldc, int M, int N, int K, int mode, int k_split,
                              float* workspace, hipStream_t stream);
+int apc_gemm_direct_qkv_takes(const void* A, int lda, const void* q_out, int ldq, int M, int K, int H, int Hk, int d,
+                              const void* cos_sin, const void* cache);
+int apc_gemm_direct_qkv_rope_bf16(const void* A, int lda, const float* ss, int ss_parts, float eps, const void* W, void* q_out, int ldq,
+                                  int M, int K, int H, int Hk, int d, const float* cos_sin, const int* positions, const int* row_seg,
+                                  const int* block_table, int max_blocks, void* cache, int page_tokens, hipStream_t stream);
 int apc_gemm_splitk_qkv_rope_bf16(const void* A, int lda, const float* ss, int ss_parts, float eps, const void* W,
                                   void* q_out, int ldq, int M, int K, int H, int Hk, int d, const float* cos_sin,
                                   const int* positions, const int* row_seg, const int* block_table, int max_blocks,

@@ -334,7 +334,8 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
     """q, k, v in one product that also rotates q and k (whole heads) and writes k and v into the pages; rotated q
     goes to the first n_heads * head_dim columns of q_out.  Up to 16 rows: the streaming kernel (head size a
     multiple of 32); up to 64 the kernel that finishes in one launch, where that is faster; more rows: the tiled kernel
-    where it cuts K into slices, in its finishing kernel (256 a multiple of the head size).  `a`: the normalised rows, or with `pre` = (ss, eps) the row that
+    where it cuts K into slices, in its finishing kernel (256 a multiple of the head size), and the kernel whose weights go
+    straight into registers where that takes the product in one piece (heads of 64 and 128).  `a`: the normalised rows, or with `pre` = (ss, eps) the row that
     `gemm_emit_bf16` left.  False, with nothing done, for sizes neither takes."""
     _ops._gpu(a, w.data, q_out, cos_sin, positions, row_seg, block_table, cache)
     M, K = a.shape
@@ -349,7 +350,9 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
     rows = SKINNY_MAX_ROWS < M <= ROWS_MAX and _lib.load("tuned").apc_gemm_rows_qkv_takes(
         a.data_ptr(), a.stride(0), w.data.data_ptr(), q_out.data_ptr(), q_out.stride(0), M, K, H, Hk, d, cos_sin.data_ptr(),
         cache.data_ptr())
-    if not few and ((ks == 1 and not rows) or 256 % d or d % 2):
+    direct = not few and ks == 1 and not rows and _lib.load("tuned").apc_gemm_direct_qkv_takes(
+        a.data_ptr(), a.stride(0), q_out.data_ptr(), q_out.stride(0), M, K, H, Hk, d, cos_sin.data_ptr(), cache.data_ptr())
+    if not few and not direct and ((ks == 1 and not rows) or 256 % d or d % 2):
         return False
     ss, eps = None, 0.0
     if pre is not None:
@@ -357,7 +360,7 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
         if few and not _pre_ok(a, ss, K):
             return False
         if not few and not (ss.dtype == torch.float32 and ss.is_contiguous() and ss.dim() == 2 and ss.shape[0] == M
-                            and 1 <= ss.shape[1] <= _ss_parts_max(M)):
+                            and 1 <= ss.shape[1] and (direct or ss.shape[1] <= _ss_parts_max(M))):
             return False
     if not (w.K == K and w.N == N and q_out.shape[0] == M and q_out.shape[1] >= H * d):
         raise ValueError(f"qkv: a [{M}, {K}], w {w.shape}, {H}+2*{Hk} heads of {d}, q_out {tuple(q_out.shape)}")
@@ -375,6 +378,13 @@ def qkv_rope_bf16(a: torch.Tensor, pre, w: PackedWeight, q_out: torch.Tensor, n_
             q_out.data_ptr(), _ops._rows(q_out, "q_out"), M, K, H, Hk, d, cos_sin.data_ptr(),
             _ops._i32(positions, M, "positions"), _ops._i32(row_seg, M, "row_seg"), block_table.data_ptr(),
             block_table.shape[1], cache.data_ptr(), page_tokens, _ops._stream()), "skinny_qkv_rope_bf16")
+        return True
+    if direct:
+        _lib.check(L.apc_gemm_direct_qkv_rope_bf16(
+            a.data_ptr(), _ops._rows(a, "a"), ss_ptr, ss.shape[1] if ss is not None else 0, float(eps), w.data.data_ptr(),
+            q_out.data_ptr(), _ops._rows(q_out, "q_out"), M, K, H, Hk, d, cos_sin.data_ptr(),
+            _ops._i32(positions, M, "positions"), _ops._i32(row_seg, M, "row_seg"), block_table.data_ptr(),
+            block_table.shape[1], cache.data_ptr(), page_tokens, _ops._stream()), "gemm_direct_qkv_rope_bf16")
         return True
     ws = None if rows else torch.empty(ks * M * N, dtype=torch.float32, device=a.device)
     _lib.check(L.apc_gemm_splitk_qkv_rope_bf16(

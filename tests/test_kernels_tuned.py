@@ -673,6 +673,17 @@ def test_product_for_q_k_v_that_rotates_and_fills_the_pages_equals_the_kernels_o
     assert (results[0][1] != 0).sum() + (results[0][2] != 0).sum() == M * 2 * Hk * d   # every row wrote its k and v, once
 
 
+# tiles of 4, 6 and 8 bands a wave; a last row tile of 1, 6 and 92 rows, a last tile of columns with fewer heads than it has room
+# for; few rows into many columns; K in one and several passes
+@pytest.mark.parametrize("M,H,Hk,d,K,P_,pre", [(1024, 4, 2, 64, 128, 8, False), (1030, 5, 1, 128, 384, 16, True), (1153, 24, 8, 128, 256, 16, True),
+                                               (1500, 32, 8, 64, 256, 32, False), (2048, 32, 8, 128, 128, 16, True), (2048, 33, 3, 64, 256, 24, True),
+                                               (2048, 48, 8, 128, 128, 64, False), (140, 125, 2, 128, 128, 16, True)])
+def test_product_for_q_k_v_of_many_rows_that_rotates_and_fills_the_pages(M, H, Hk, d, K, P_, pre):
+    with tuned()._lib.timing() as launched:
+        test_product_for_q_k_v_that_rotates_and_fills_the_pages_equals_the_kernels_one_after_the_other(M, H, Hk, d, K, P_, pre)
+    assert "apc_gemm_direct_qkv_rope_bf16" in launched.totals()
+
+
 # two and four bands a block, waves with unequal numbers of steps among them; two, three and four groups of 16 rows
 @pytest.mark.parametrize("F,K", [(2048, 1024), (4096, 2048), (1040, 3008), (4096, 3072), (5120, 1024), (8176, 1536), (8192, 3072)])
 def test_a_row_of_a_gated_product_of_17_to_64_rows_does_not_depend_on_the_others(F, K):
