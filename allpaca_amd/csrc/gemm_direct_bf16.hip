@@ -60,7 +60,7 @@ struct DirectPre {
 // of one head, the same j in all of its heads, so that a lane holds both elements of its pairs and one place of the angles' table
 // serves all heads of a row.  What it costs beside the store that it replaces is the trip for the angles, 1-2 us; what falls away
 // is a launch that reads and writes q, k and v (the two of them, us, K = the width, without / with): 2,048 rows into 6,144
-// outputs of an 8B model DQ0, 1,153 rows into 5,120 of a 3B model DQ1, 1,500 into 3,072 of a 1B model DQ2.
+// outputs of an 8B model 83 + 12 / 86, 1,153 rows into 5,120 of a 3B model 42 + 10 / 46, 1,500 into 3,072 of a 1B model 28 + 9 / 33.
 struct DirectRope {
   const float* cos_sin;     // [positions][2][d / 2]
   const int* positions;     // [M]

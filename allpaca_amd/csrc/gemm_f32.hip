@@ -476,6 +476,194 @@ __global__ __launch_bounds__(64 * SL, MIN_WAVES) void gemm_f32_kernel(
   }
 }
 
+// What goes with the product for q, k and v (ROPE): W is [(H + 2 Hk) d, K], heads in the order q, k, v, d a multiple of 16.  A block
+// takes eight outputs j 8 .. of a head's first half and the same of its second, so that a lane of the first wave finds both elements of
+// four pairs (e, e + d / 2) in the sums.  Rotated q goes to C; k to cache[page][0][kv head][slot][:], v to cache[page][1][kv
+// head][:][slot], page = block_table[row_seg][pos / P], slot = pos % P.
+struct RopeF32 {
+  const float* cos_sin;     // [positions][2][d / 2]
+  const int* positions;     // [M]
+  const int* row_seg;       // [M]
+  const int* block_table;   // [segments][max_blocks]
+  int max_blocks;
+  float* cache;
+  int P, H, Hk, d;
+};
+
+// The product of up to 8 rows.  The same slices, the same sums to the bit as gemm_f32_kernel's; what differs is what a stage brings:
+// 8 rows of A, not 16 of which half are repeats, and 8 or 16 rows of W, so that 2,048 outputs have a block for every compute unit;
+// two stages are on their way in a loop whose last round asks again for the last stage instead of code for every remainder, and a
+// stage's operands come out of LDS under the products of the one before.  A residual is asked for ahead of the first weights.
+// What bounds it is a unit's eight waves' way from loads to products (as many stages as registers hold are no faster: 4 rows x
+// 2,048 outputs x K 2,048 7.6 us with two, 7.9 with four, 8.7 with eight).  gemm_f32_kernel / this one, us, launches of a graph one
+// behind the other over 67 to 840 MB of weights: 4 rows x 2,048 outputs x K 2,048 8.4 / 7.6, K 8,192 23.3 / 20.5, 1,024 x 4,096
+// 11.2 / 10.0, 576 x 576 5.8 / 5.2; bands of 16: 3,072 x 2,048 8.7 / 8.3, 4,096 x 4,096 15.1 / 14.0.
+template <int BAND, int D, bool NORM, bool ROPE>
+__global__ __launch_bounds__(64 * SLICES, 4) void gemm_f32_few_kernel(const float* __restrict__ A, int lda, const float* __restrict__ G,
+                                                                      float eps, const float* __restrict__ W, int ldw, void* __restrict__ C,
+                                                                      int c_dtype, int ldc, int M, int N, int K, int mode, RopeF32 rope) {
+  static_assert(!ROPE || BAND == 16, "two halves of eight");
+  static_assert(D % 2 == 0 && (BAND == 8 || BAND == 16), "two stages in LDS take turns");
+  constexpr int WL = BAND / 8, STAGE_F4 = 64 * (WL + 1);
+  __shared__ f32x4 lds[SLICES][2][STAGE_F4];
+  __shared__ float squares[NORM ? SLICES * 16 : 1];
+  __shared__ f32x4 gains[NORM ? NORM_K / 4 : 1];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+  const int slice = STAGE * ((K + STAGE * SLICES - 1) / (STAGE * SLICES)), k0 = wave * slice;
+  const int steps = (min(K, k0 + slice) - k0 + STAGE - 1) / STAGE;   // <= 0: no k left for this wave
+  const int lr = lane / 8, lk = (lane % 8) * 4, row = lane % 16, quarter = lane / 16;
+  const int head = ROPE ? blockIdx.x / (rope.d / 16) : 0, j = ROPE ? blockIdx.x % (rope.d / 16) : 0, half_head = rope.d / 2;
+  const int n0 = ROPE ? head * rope.d + j * 8 : blockIdx.x * BAND;
+  const BufferRsrc from_w = make_rsrc(W + (size_t)n0 * ldw), from_a = make_rsrc(A);
+  int off[WL + 1];
+#pragma unroll
+  for (int h = 0; h < WL; ++h) off[h] = 4 * ((ROPE ? h * half_head + lr : min(8 * h + lr, N - 1 - n0)) * ldw + lk);
+  off[WL] = 4 * (min(lr, M - 1) * lda + lk);
+  // the outputs that a lane of the first wave leaves: row `row`, n .. n + 3
+  const int n = n0 + quarter * 4;
+  const bool own = wave == 0 && row < M && quarter * 4 < (ROPE ? 8 : BAND);
+  const bool wide = c_dtype == APC_F32 && ldc % 4 == 0 && ((uintptr_t)C & 15u) == 0 && n + 4 <= N;   // 16 bytes
+  f32x4 before = {0.f, 0.f, 0.f, 0.f};
+  if (own && wide && mode == 1) before = *(const f32x4*)((const float*)C + (size_t)row * ldc + n);
+  int pos = 0, seg = 0, page = 0;                       // ROPE: asked for in front of the first weights, what hangs on them behind
+  f32x4 cs = {0.f, 0.f, 0.f, 0.f}, sn = {0.f, 0.f, 0.f, 0.f};
+  if (ROPE && own) pos = rope.positions[row], seg = rope.row_seg[row];
+  f32x4 reg[D][WL + 1];
+  auto load = [&](int slot, int s) __attribute__((always_inline)) {
+    s = min(s, steps - 1);
+    const int at = 4 * (k0 + s * STAGE), back = k0 + s * STAGE + lk >= K ? 4 * lk : 0;
+#pragma unroll
+    for (int h = 0; h < WL; ++h) reg[slot][h] = load_f32x4<true>(from_w, off[h] - back, at);
+    reg[slot][WL] = load_f32x4<false>(from_a, off[WL] - back, at);
+  };
+  const int put_at = lr * 8 + ((lane % 8) ^ lr);
+  auto put = [&](int slot, int s, int to) __attribute__((always_inline)) {
+    const bool end = k0 + min(s, steps - 1) * STAGE + lk >= K;       // (behind K: zeros)
+#pragma unroll
+    for (int h = 0; h <= WL; ++h) lds[wave][to][h * 64 + put_at] = end ? f32x4{0.f, 0.f, 0.f, 0.f} : reg[slot][h];
+    wave_lds_order();
+  };
+  f32x4 w[2][2], a[2][2], g[2][2];                      // [stage % 2][half]: operands, gains of the stage's 16 k
+  auto get = [&](int s, int from) __attribute__((always_inline)) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int piece = (quarter + 4 * half) ^ (row % 8);
+      w[from][half] = lds[wave][from][row % BAND * 8 + piece];
+      a[from][half] = lds[wave][from][WL * 64 + row % 8 * 8 + piece];
+      if constexpr (NORM) g[from][half] = gains[(k0 + min(s, steps - 1) * STAGE) / 4 + quarter + 4 * half];
+    }
+    wave_lds_order();
+  };
+  float ss[2] = {0.f, 0.f};
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int of) __attribute__((always_inline)) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if constexpr (NORM) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss[e % 2] = fmaf(a[of][half][e], a[of][half][e], ss[e % 2]), a[of][half][e] *= g[of][half][e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[of][half][e], a[of][half][e], acc, 0, 0, 0);
+    }
+  };
+  f32x4 gain[NORM ? NORM_K / (256 * SLICES) : 1] = {};
+  if constexpr (NORM) {
+#pragma unroll
+    for (int q = 0; q < NORM_K / (256 * SLICES); ++q)
+      if (threadIdx.x + q * 64 * SLICES < K / 4) gain[q] = reinterpret_cast<const f32x4*>(G)[threadIdx.x + q * 64 * SLICES];
+  }
+  if (steps > 0) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) load(u, u);
+  }
+  if (ROPE && own) {
+    const float* at = rope.cos_sin + (size_t)pos * rope.d + j * 8 + quarter * 4;
+    cs = *(const f32x4*)at, sn = *(const f32x4*)(at + half_head);
+    page = rope.block_table[(size_t)seg * rope.max_blocks + pos / rope.P];
+  }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int q = 0; q < NORM_K / (256 * SLICES); ++q) gains[threadIdx.x + q * 64 * SLICES] = gain[q];
+    __syncthreads();
+  }
+  if (steps > 0) {
+    put(0, 0, 0);
+    load(0, D);
+    get(0, 0);
+    for (int s0 = 0; s0 < steps; s0 += D) {
+#pragma unroll
+      for (int u = 0; u < D; ++u) {
+        put((u + 1) % D, s0 + u + 1, (u + 1) % 2);
+        load((u + 1) % D, s0 + u + 1 + D);
+        get(s0 + u + 1, (u + 1) % 2);
+        if (s0 + u < steps) multiply(u % 2);
+      }
+    }
+  }
+  lds[wave][0][lane] = acc;                             // the waves meet
+  if constexpr (NORM) {
+    float sq = ss[0] + ss[1];
+    sq += __shfl_xor(sq, 16), sq += __shfl_xor(sq, 32);
+    if (quarter == 0) squares[wave * 16 + row] = sq;
+  }
+  __syncthreads();
+  if (!own) return;
+  auto sum = [&](int l) __attribute__((always_inline)) {
+    f32x4 v = lds[0][0][l];
+#pragma unroll
+    for (int x = 1; x < SLICES; ++x) v += lds[x][0][l];
+    return v;
+  };
+  float scale = 1.f;
+  if constexpr (NORM) {
+    float all = 0.f;
+#pragma unroll
+    for (int x = 0; x < SLICES; ++x) all += squares[x * 16 + row];
+    scale = row_scale(all, K, eps);
+  }
+  f32x4 v = sum(lane);
+  if constexpr (NORM) v *= scale;
+  if constexpr (ROPE) {
+    f32x4 hi = sum(lane + 32);
+    if constexpr (NORM) hi *= scale;
+    const int e = j * 8 + quarter * 4, slot = pos % rope.P;
+    float* in_page = rope.cache + (size_t)page * ((size_t)2 * rope.Hk * rope.P * rope.d);
+    if (head < rope.H + rope.Hk) {
+      f32x4 ra, rb;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float fa = v[x], fb = hi[x], c = cs[x], s = sn[x];
+        ra[x] = fmaf(fa, c, -(fb * s));                 // (as the compiler makes it of rope_kv_write_kernel's text)
+        rb[x] = fmaf(fb, c, fa * s);
+      }
+      float* to = head < rope.H ? (float*)C + (size_t)row * ldc + (size_t)head * rope.d
+                                : in_page + ((size_t)(head - rope.H) * rope.P + slot) * rope.d;
+      *(f32x4*)(to + e) = ra;
+      *(f32x4*)(to + e + half_head) = rb;
+    } else {
+      float* to = in_page + ((size_t)(rope.Hk + head - rope.H - rope.Hk) * rope.d + e) * rope.P + slot;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        to[(size_t)x * rope.P] = v[x];
+        to[(size_t)(half_head + x) * rope.P] = hi[x];
+      }
+    }
+    return;
+  }
+  if (wide) {
+    *(f32x4*)((float*)C + (size_t)row * ldc + n) = mode == 1 ? before + v : v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (n + e >= N) continue;
+    const size_t o = (size_t)row * ldc + n + e;
+    if (mode == 1) ((float*)C)[o] += v[e];
+    else store_f(C, c_dtype, o, v[e]);
+  }
+}
+
 // Slices without k are left out: with all eight, a block of a large tile keeps its unit for 6 us whatever K is, most of
 // its waves idle and 128 KiB of LDS taken.  2,048 rows x 16,384 outputs at K = 32, 64, 128: 200, 203, 216 us with eight
 // slices and stores of 4 bytes, 84, 101, 147 with the two or four there are, 53, 69, 125 with 16-byte stores beside (one
@@ -586,6 +774,19 @@ APC_EXPORT int apc_gemm_f32_tiles_a_block(int M, int N, int K) { return tiles_a_
 // outputs, K 2,048: 150 and 151): the straight code of a stage count's every case is a third as long, and a launch finds it cold.
 static int product(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C,
                    int c_dtype, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
+  // Up to 8 rows (see gemm_f32_few_kernel): one round of blocks of 8 outputs, or of 16 with a K that pays.  4 rows, us, tiles / blocks of 8
+  // / of 16: 2,048 outputs at K = 576 5.9 / 5.5 / 5.7; 3,072 at K = 1,024 6.8 / 7.4 / 6.9, K = 4,096 13.3 / 16.0 / 12.1; 6,144 at
+  // K = 1,024 9.5 / 10.1 / 10.3, 8,192 47.5 / 47.4 / 51.2.
+  if (M <= 8 && !G && !R && K > 4 * STAGE && N <= 4096 && (N <= 2048 || K > 1024)) {
+#define FEW(BAND_)                                                                                                             \
+  hipLaunchKernelGGL((gemm_f32_few_kernel<BAND_, 2, false, false>), dim3(ceil_div(N, BAND_)), dim3(64 * SLICES), 0, stream, A, lda, \
+                     nullptr, 0.f, W, ldw, C, c_dtype, ldc, M, N, K, mode, RopeF32{})
+    if (N <= 2048) FEW(8);
+    else FEW(16);
+#undef FEW
+    APC_LAUNCH_CHECK();
+    return 0;
+  }
 #define GO(...) return launch<__VA_ARGS__>(A, lda, G, eps, R, W, ldw, C, c_dtype, ldc, M, N, K, mode, stream)
   // (one row tile: W is read once, past the caches)
   switch (tile_of(M, N, K)) {
@@ -647,6 +848,30 @@ APC_EXPORT int apc_gemm_norm_f32(const void* A, int lda, const void* G, float ep
   float* h = (float*)ws;
   if (const int rc = norm_rows(a, lda, g, eps, h, M, K, stream)) return rc;
   return product(h, K, nullptr, 0.f, h + (size_t)M * K, w, ldw, C, APC_F32, ldc, M, N, K, 0, stream);
+}
+
+// q, k and v of up to 8 rows in one launch with the norm in front, the rotation of whole q and k heads and the write of k and v into
+// the pages (see RopeF32); q_out [M, ldq] takes the rotated q heads in its first H d columns.  The sums are apc_gemm_norm_f32's.
+// 4 rows of a 1B model (3,072 outputs, K 2,048), inside a step: 8.4 + 4.6 -> 9.6 us.  Up to 8,192 outputs: from there on the tiles are
+// faster by what the launch costs.
+APC_EXPORT int apc_qkv_rope_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, const void* q_out, int ldq, int M,
+                                      int K, int H, int Hk, int d, const void* cos_sin, const void* cache) {
+  if (M <= 0 || M > 8 || H <= 0 || Hk <= 0 || d <= 0 || d % 16 || (H + 2 * Hk) * (long long)d > 8192) return 0;
+  if (K <= 4 * STAGE || K > NORM_K || lda < K || ldw < K || ldq < H * d || ldq % 4) return 0;
+  if ((((uintptr_t)q_out | (uintptr_t)cos_sin | (uintptr_t)cache) & 15u) || (d / 2 + 8LL) * ldw * 4 >= (1LL << 31)) return 0;
+  return apc_gemm_norm_f32_takes(A, lda, G, W, ldw, K);
+}
+APC_EXPORT int apc_qkv_rope_f32(const float* A, int lda, const float* G, float eps, const float* W, int ldw, float* q_out, int ldq, int M,
+                                int K, int H, int Hk, int d, const float* cos_sin, const int* positions, const int* row_seg,
+                                const int* block_table, int max_blocks, float* cache, int page_tokens, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (!positions || !row_seg || !block_table || max_blocks <= 0 || !cache || !cos_sin || page_tokens <= 0) return APC_ERR_BAD_ARG;
+  if (!apc_qkv_rope_f32_takes(A, lda, G, W, ldw, q_out, ldq, M, K, H, Hk, d, cos_sin, cache)) return APC_ERR_UNSUPPORTED;
+  const RopeF32 rope{cos_sin, positions, row_seg, block_table, max_blocks, cache, page_tokens, H, Hk, d};
+  hipLaunchKernelGGL((gemm_f32_few_kernel<16, 2, true, true>), dim3((H + 2 * Hk) * d / 16), dim3(64 * SLICES), 0, stream, A, lda, G, eps, W,
+                     ldw, q_out, APC_F32, ldq, M, (H + 2 * Hk) * d, K, 0, rope);
+  APC_LAUNCH_CHECK();
+  return 0;
 }
 
 // out[M,F] = silu(A . Wg^T) * (A . Wu^T), W = [Wg; Wu] of 2 F rows: the same sums as the product of 2 F outputs, without

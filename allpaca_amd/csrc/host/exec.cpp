@@ -406,6 +406,20 @@ int qkv_rope(Program& P, const Buf& a, const Emit* pre, const ApcLayer& L, const
   return 1;
 }
 
+// the same of float32 rows with the norm in front in the kernel, up to 8 rows; 1 done, 0 not taken
+int qkv_rope_f32(Program& P, const Normed& n, const ApcLayer& L, const Buf& qkv, const ApcPlanEntry& E) {
+  const int M = P.x.rows, K = P.x.cols, H = L.H, Hk = L.Hk, d = L.d;
+  if (!folds_f32(P, n, L.w_qkv, qkv) || E.kv_dtype != APC_DT_F32 || L.w_qkv.N != (H + 2 * Hk) * d || qkv.cols < H * d ||
+      !apc_qkv_rope_f32_takes(P.x.p, P.x.ld, n.g, L.w_qkv.data, L.w_qkv.ld, qkv.p, qkv.ld, M, K, H, Hk, d, L.cos_sin, E.kv))
+    return 0;
+  const ApcStep& s = P.step;
+  LAUNCH(P, "qkv_rope_f32",
+         apc_qkv_rope_f32((const float*)P.x.p, P.x.ld, n.g, n.eps, (const float*)L.w_qkv.data, L.w_qkv.ld, (float*)qkv.p, qkv.ld, M, K, H,
+                          Hk, d, L.cos_sin, s.positions, s.row_seg, s.table[E.group], s.table_width[E.group], (float*)E.kv,
+                          E.page_tokens, P.stream));
+  return 1;
+}
+
 int rope_kv_write(Program& P, const Buf& qkv, const ApcLayer& L, const ApcPlanEntry& E, bool write) {
   const int H = L.H, Hk = L.Hk, d = L.d, q_off = 0, k_off = H * d, v_off = (H + Hk) * d;
   const ApcStep& s = P.step;
@@ -530,6 +544,11 @@ int run_layer(Program& P, const ApcLayer& L, const ApcPlanEntry& E, const Emit& 
       if (rc) return rc;
       rc = qkv_rope(P, h1.h, nullptr, L, qkv, E);
     }
+    if (rc < 0) return rc;
+    fused = rc == 1;
+  }
+  if (!fused && E.writes && L.rot == L.d && L.rot > 0) {
+    const int rc = qkv_rope_f32(P, h1, L, qkv, E);
     if (rc < 0) return rc;
     fused = rc == 1;
   }

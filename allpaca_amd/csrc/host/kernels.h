@@ -24,6 +24,11 @@ int apc_gemm_norm_f32_kib(int M, int K);
 int apc_gemm_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int K);
 int apc_gemm_norm_f32(const void* A, int lda, const void* G, float eps, const void* W, int ldw, void* C, int ldc, int M, int N,
                       int K, void* ws, hipStream_t stream);
+int apc_qkv_rope_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, const void* q_out, int ldq, int M, int K, int H,
+                           int Hk, int d, const void* cos_sin, const void* cache);
+int apc_qkv_rope_f32(const float* A, int lda, const float* G, float eps, const float* W, int ldw, float* q_out, int ldq, int M, int K,
+                     int H, int Hk, int d, const float* cos_sin, const int* positions, const int* row_seg, const int* block_table,
+                     int max_blocks, float* cache, int page_tokens, hipStream_t stream);
 int apc_swiglu_norm_f32_takes(const void* A, int lda, const void* G, const void* W, int ldw, int F, int K);
 int apc_swiglu_norm_f32(const void* A, int lda, const void* G, float eps, const void* W, int ldw, void* out, int ldo, int M,
                         int F, int K, void* ws, hipStream_t stream);

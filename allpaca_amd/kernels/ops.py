@@ -416,6 +416,36 @@ def linear_normed(x: torch.Tensor, g: torch.Tensor, eps: float, w, out: torch.Te
     return True
 
 
+def qkv_rope_normed(x: torch.Tensor, g: torch.Tensor, eps: float, w, q_out: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int,
+                    cos_sin: torch.Tensor, positions: torch.Tensor, row_seg: torch.Tensor, block_table: torch.Tensor,
+                    cache: torch.Tensor, page_tokens: int) -> bool:
+    """q, k and v of rmsnorm(x; g, eps) in float32 in one kernel that also rotates whole q and k heads and writes k and v into the
+    pages (up to 8 rows); rotated q goes to the first columns of q_out.  False (nothing done) for operands it does not take."""
+    if isinstance(w, PackedWeight) or not (x.dtype == w.dtype == q_out.dtype == cache.dtype == torch.float32 and _float32_gain(x, g)):
+        return False
+    _gpu(x, g, w, q_out, cos_sin, positions, row_seg, block_table, cache)
+    ldx, ldw, ldq = _rows(x, "qkv x"), _rows(w, "qkv w"), _rows(q_out, "q_out")
+    M, K = x.shape
+    H, Hk, d = n_heads, n_kv_heads, head_dim
+    L = _lib.load("plain")
+    if not L.apc_qkv_rope_f32_takes(x.data_ptr(), ldx, g.data_ptr(), w.data_ptr(), ldw, q_out.data_ptr(), ldq, M, K, H, Hk, d,
+                                    cos_sin.data_ptr(), cache.data_ptr()):
+        return False
+    if not (w.shape == ((H + 2 * Hk) * d, K) and q_out.shape[0] == M and q_out.shape[1] >= H * d):
+        raise ValueError(f"qkv: x [{M}, {K}], w {tuple(w.shape)}, {H}+2*{Hk} heads of {d}, q_out {tuple(q_out.shape)}")
+    _need(cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and tuple(cos_sin.shape[1:]) == (2, d // 2),
+          "cos/sin table must be float32 [positions, 2, head_dim/2]")
+    if not (cache.dim() == 5 and cache.is_contiguous() and tuple(cache.shape[1:]) == (2, Hk, page_tokens, d)):
+        raise ValueError(f"cache must be [pages, 2, {Hk}, {page_tokens}, {d}], got {tuple(cache.shape)}")
+    _need(block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.is_contiguous(),
+          "block table must be contiguous int32 [segments, blocks]")
+    _lib.check(L.apc_qkv_rope_f32(x.data_ptr(), ldx, g.data_ptr(), float(eps), w.data_ptr(), ldw, q_out.data_ptr(), ldq, M, K, H, Hk, d,
+                                  cos_sin.data_ptr(), _i32(positions, M, "positions"), _i32(row_seg, M, "row_seg"),
+                                  block_table.data_ptr(), block_table.shape[1], cache.data_ptr(), page_tokens, _stream()),
+               "qkv_rope_f32")
+    return True
+
+
 def swiglu_normed(x: torch.Tensor, g: torch.Tensor, eps: float, w, out: torch.Tensor) -> bool:
     """`swiglu` of rmsnorm(x; g, eps), as `linear_normed` (w: [Wg; Wu] in float32)."""
     if isinstance(w, tuple) or not (x.dtype == w.dtype == out.dtype == torch.float32 and _float32_gain(x, g)):

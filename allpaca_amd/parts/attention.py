@@ -69,6 +69,9 @@ class Attention(Mixer):
                                                   step.positions, step.row_seg, cache.block_table, kv,
                                                   cache.page_tokens))):
             pass
+        elif kv is not None and rot == self.d and h.qkv_rope(self.w_qkv, qkv, self.H, self.Hk, self.d, table, step.positions,
+                                                             step.row_seg, cache.block_table, kv, cache.page_tokens):
+            pass
         else:
             h.linear(self.w_qkv, qkv)
             if self.position is not None and fused is None:

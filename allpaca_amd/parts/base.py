@@ -232,6 +232,11 @@ class NormedInput:
             return bool(op(p.raw, (p.ss, p.eps)))
         return bool(op(self.tensor(), None))
 
+    def qkv_rope(self, w, q_out: torch.Tensor, *args) -> bool:
+        """`ops.qkv_rope_normed` where the norm may be folded; False if nothing was done."""
+        from ..kernels import ops
+        return self.pre is None and self._folds() and ops.qkv_rope_normed(self.x, *self.norm.rms_params(), w, q_out, *args)
+
     def swiglu(self, w_gate_up, out: torch.Tensor) -> None:
         from ..kernels import ops
         p = self.pre

@@ -242,3 +242,59 @@ def test_rows_behind_a_norm_in_every_form(M, N, K):
         alone = torch.empty(1, N, device=DEV)
         assert o.linear_normed(x[r:r + 1], g, eps, w, alone)
         assert torch.equal(alone[0], out[r])
+
+
+# blocks of 8 outputs (up to 2,048) and of 16, last blocks that are not full; slices with no, one and several stages, a last stage cut by
+# K; outputs whose rows do not allow 16-byte stores
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(8, 132), (40, 14340), (515, 256), (2048, 2048), (2047, 388), (2049, 1028), (4090, 2052), (4096, 1056)])
+def test_up_to_8_rows_are_the_bits_of_more(N, K):
+    o = ops()
+    a, w = gen(12, K, seed=1), gen(N, K, seed=2)
+    many = torch.empty(12, N, device=DEV)
+    o.gemm_plain(a, w, many)
+    assert ((many.double() - a.double() @ w.double().T).abs() <= product_bound(a, w)).all()
+    for M in (1, 2, 5, 8):
+        for ld in (N, N + 3):
+            out = torch.full((M, ld), 7.0, device=DEV)
+            o.gemm_plain(a[:M], w, out[:, :N])
+            assert torch.equal(out[:, :N], many[:M]) and (out[:, N:] == 7.0).all()
+            o.gemm_plain(a[:M], w, out[:, :N], accumulate=True)
+            assert torch.equal(out[:, :N], many[:M] + many[:M]) and (out[:, N:] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,H,Hk,d,K,P", [(1, 32, 8, 64, 2048, 16), (4, 32, 8, 64, 2048, 16), (8, 4, 2, 128, 4096, 8), (5, 3, 1, 16, 132, 4),
+                                          (7, 6, 2, 80, 1000, 24), (3, 5, 5, 32, 260, 5)])
+def test_q_k_v_rotated_and_in_the_pages_are_the_bits_of_the_kernels_one_after_the_other(M, H, Hk, d, K, P):
+    o = ops()
+    rng = np.random.default_rng(M * 100 + d)
+    x, g, w = gen(M, K + 4, seed=1)[:, :K] * 3.0, 1.0 + 0.1 * gen(K, seed=2), gen((H + 2 * Hk) * d, K, seed=3)
+    blocks = 6
+    places = rng.permutation(3 * blocks * P)[:M]
+    seg = torch.tensor(places // (blocks * P), dtype=torch.int32, device=DEV)
+    pos = torch.tensor(places % (blocks * P), dtype=torch.int32, device=DEV)
+    table = torch.from_numpy(rng.permutation(3 * blocks).reshape(3, blocks).astype(np.int32)).to(DEV)
+    angles = torch.arange(blocks * P, dtype=torch.float64)[:, None] * 300.0 ** (-torch.arange(d // 2, dtype=torch.float64) / (d // 2))
+    cos_sin = torch.stack([angles.cos(), angles.sin()], 1).float().to(DEV)
+    got, want = (torch.full((M, (H + 2 * Hk) * d + 4), 7.0, device=DEV) for _ in range(2))
+    pages_got, pages_want = (torch.zeros(3 * blocks, 2, Hk, P, d, device=DEV) for _ in range(2))
+    assert o.qkv_rope_normed(x, g, 1e-5, w, got, H, Hk, d, cos_sin, pos, seg, table, pages_got, P)
+    assert o.linear_normed(x, g, 1e-5, w, want[:, :-4])
+    o.rope_kv_write(want, 0, H * d, (H + Hk) * d, H, Hk, d, d, cos_sin, pos, seg, table, pages_want, P)
+    assert torch.equal(got[:, :H * d], want[:, :H * d]) and torch.equal(pages_got, pages_want)
+    assert (got[:, H * d:] == 7.0).all()
+
+
+@pytest.mark.gpu
+def test_q_k_v_that_are_left_to_the_kernels_one_after_the_other():
+    o = ops()
+
+    def taken(M=4, H=4, Hk=2, d=32, K=256):
+        x, w = gen(M, K), gen((H + 2 * Hk) * d, K)
+        ints = [torch.zeros(n, dtype=torch.int32, device=DEV) for n in (M, M)]
+        return o.qkv_rope_normed(x, gen(K), 1e-5, w, torch.empty(M, (H + 2 * Hk) * d, device=DEV), H, Hk, d, torch.zeros(64, 2, d // 2, device=DEV),
+                                 *ints, torch.zeros(1, 4, dtype=torch.int32, device=DEV), torch.zeros(4, 2, Hk, 16, d, device=DEV), 16)
+
+    assert taken()
+    assert not taken(M=9) and not taken(d=24) and not taken(K=128) and not taken(K=4100) and not taken(H=300)
