@@ -16,6 +16,7 @@
 #include "common.h"
 #include "no_alloc.h"
 #include <math.h>
+#include <algorithm>
 #include <string.h>
 #include <mutex>
 
@@ -1212,6 +1213,57 @@ __device__ __forceinline__ void sums_in_order(const float* a, float* run, int n,
   __builtin_amdgcn_wave_barrier();
 }
 
+// The token among the cnt candidates in sh.s_key2 / sh.s_id2, in order: as `sample_few`, with the exponentials and quotients by
+// all threads and the sums in order by one wave.  share, sums: room for cnt floats and up to a multiple of 16 behind them.
+template <int NT, typename Leave>
+__device__ __forceinline__ void draw_in_order(SampleShared& sh, float* share, float* sums, int cnt, bool use_top_p, float tp, float uniform,
+                                              Leave&& leave) {
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  float* e = reinterpret_cast<float*>(sh.s_key);
+  const float vmax = value_of(sh.s_key2[0]);
+  for (int i = threadIdx.x; i < cnt; i += NT) e[i] = expf(value_of(sh.s_key2[i]) - vmax);
+  __syncthreads();
+  if (wave != 0) return;
+  // The weights' sum, the shares' sum up to top-p, and the uniform number less the shares of the m that are left: three times
+  // the same code (over values that differ), which a block fetches once.  The sum of the first m is one of the first pass's.
+  float* run = reinterpret_cast<float*>(sh.s_id);
+  int m = cnt, pick = 0;
+  float sum = 0.f;
+#pragma unroll 1
+  for (int pass = 0; pass < 3; ++pass) {
+    if (pass == 1) {
+      if (!use_top_p) continue;
+      if (sum == 0.f || !finite_f(sum)) {
+        const int some = (int)ceilf(tp * (float)m);
+        m = some < 1 ? 1 : (some > m ? m : some);
+        sum = sums[m - 1];
+        continue;
+      }
+    }
+    for (int i = lane; i < m; i += WAVE) share[i] = pass == 0 ? e[i] : pass == 2 && sum == 0.f ? 1.0f / (float)m : e[i] / sum;
+    __builtin_amdgcn_wave_barrier();
+    float* to = pass == 0 ? sums : run;
+    sums_in_order(share, to, m, pass == 2 ? uniform : 0.f, pass == 2 ? -1.f : 1.f);
+    if (pass == 0) {
+      sum = sums[m - 1];
+      continue;
+    }
+    // the first candidate at which top-p is reached, or at which nothing is left
+    int first = m - 1;
+    for (int i0 = 0; i0 < m; i0 += WAVE) {
+      const int i = i0 + lane;
+      const unsigned long long hit = __ballot(i < m && (pass == 1 ? run[i] >= tp : run[i] <= 0.f));
+      if (hit) {
+        first = i0 + __ffsll(hit) - 1;
+        break;
+      }
+    }
+    if (pass == 1) m = first + 1, sum = sums[first];
+    else pick = first;
+  }
+  if (lane == 0) leave(sh.s_id2[pick]);
+}
+
 constexpr int FEW_HELD = 6144;           // candidates of a row that are held in LDS (all of them up to top-k 64)
 struct FewEnd {
   FewShared select;
@@ -1317,7 +1369,6 @@ __global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __rest
     if (j < (uint32_t)SMALL_MAX) picked[j] = c;
   });
   __syncthreads();
-  // as `sample_few`, with the exponentials and quotients by all threads and the sums in order by one wave
   const int cnt = (int)keep;
   for (int e = threadIdx.x; e < cnt; e += SNT) {
     const u64 mine = picked[e];
@@ -1328,50 +1379,228 @@ __global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __rest
     sh.one.s_id2[rank] = id_of_sort_key(mine, sz.id_bits, 0);
   }
   __syncthreads();
-  float* e = reinterpret_cast<float*>(sh.one.s_key);
-  const float vmax = value_of(sh.one.s_key2[0]);
-  for (int i = threadIdx.x; i < cnt; i += SNT) e[i] = expf(value_of(sh.one.s_key2[i]) - vmax);
-  __syncthreads();
-  if (wave != 0) return;
-  // The weights' sum, the shares' sum up to top-p, and the uniform number less the shares of the m that are left: three times
-  // the same code (over values that differ), which a block fetches once.  The sum of the first m is one of the first pass's.
-  float* run = reinterpret_cast<float*>(sh.one.s_id);
-  float* share = reinterpret_cast<float*>(sh.select.hist);             // (picked has been sorted)
-  int m = cnt, pick = 0;
-  float sum = 0.f;
-#pragma unroll 1
-  for (int pass = 0; pass < 3; ++pass) {
-    if (pass == 1) {
-      if (!use_top_p) continue;
-      if (sum == 0.f || !finite_f(sum)) {
-        const int some = (int)ceilf(tp * (float)m);
-        m = some < 1 ? 1 : (some > m ? m : some);
-        sum = sh.sums[m - 1];
-        continue;
-      }
-    }
-    for (int i = lane; i < m; i += WAVE) share[i] = pass == 0 ? e[i] : pass == 2 && sum == 0.f ? 1.0f / (float)m : e[i] / sum;
-    __builtin_amdgcn_wave_barrier();
-    float* to = pass == 0 ? sh.sums : run;
-    sums_in_order(share, to, m, pass == 2 ? uniform : 0.f, pass == 2 ? -1.f : 1.f);
-    if (pass == 0) {
-      sum = sh.sums[m - 1];
-      continue;
-    }
-    // the first candidate at which top-p is reached, or at which nothing is left
-    int first = m - 1;
-    for (int i0 = 0; i0 < m; i0 += WAVE) {
-      const int i = i0 + lane;
-      const unsigned long long hit = __ballot(i < m && (pass == 1 ? run[i] >= tp : run[i] <= 0.f));
-      if (hit) {
-        first = i0 + __ffsll(hit) - 1;
-        break;
-      }
-    }
-    if (pass == 1) m = first + 1, sum = sh.sums[first];
-    else pick = first;
+  draw_in_order<SNT>(sh.one, reinterpret_cast<float*>(sh.select.hist), sh.sums, cnt, use_top_p, tp, uniform, leave);   // (picked has been sorted)
+}
+
+// ---- The same, with a bound that the largest values of groups give ----
+// Of a row's groups of values, at least k have a largest value at or above the k-th largest of these; so the row's k largest
+// stand at or above it too, and only in groups whose largest does.  The first launch reads the row once and leaves every
+// wave's largest value; the second finds the bound among at most BOUND_SET of them (waves, or four waves together), reads again
+// the few groups that reach it (for k of 40 some 45 of 512, of 256 values each) and puts what it finds in order by counting who
+// stands above whom.  A row whose large values lie close together (all in one group, or all equal) has more than HEAD_HELD
+// there: their threshold is found by the radix descent, over those groups.
+// What bounds it is latency: the first launch is one pass where the pair above makes three, the second has some 45 groups' values to
+// look at instead of 1,300 to 5,000 candidates.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 9.9 + 15.0 -> 4.5 + 12.5 us (with
+// 256 threads in the second 17.9), from the call to the ids 47.5 -> 39.7.  The host has to know the rows' top-k, and a large
+// one (above 85, or fewer with many rows) keeps the pair above.
+constexpr int BOUND_SET = 256, HEAD_HELD = 512, HEAD_WAVES = PNT / WAVE;
+struct HeadSpace {
+  float* piece_best;       // [row][pieces] ...
+  int* piece_arg;
+  uint32_t* piece_finite;
+  uint32_t* wave_key;      // [row][pieces][HEAD_WAVES] key of the largest finite value, 0: none
+};
+// (in carve_few's memory: the candidates' place holds the waves' keys)
+HeadSpace head_space(const FewSpace& fs) { return HeadSpace{fs.piece_best, fs.piece_arg, fs.piece_finite, fs.key}; }
+
+__global__ __launch_bounds__(PNT) void sample_head_pieces_kernel(const float* __restrict__ logits, SampleShape sz, HeadSpace sp) {
+  __shared__ float bv[HEAD_WAVES];
+  __shared__ int bi[HEAD_WAVES];
+  __shared__ uint32_t nv[HEAD_WAVES];
+  const int row = blockIdx.y, piece = blockIdx.x, wave = threadIdx.x / WAVE;
+  const float* lg = logits + (size_t)row * sz.ldl;
+  const int i0 = piece * sz.chunk, i1 = min(sz.V, i0 + sz.chunk);
+  float best = -INFINITY;
+  int best_i = 0x7fffffff;
+  uint32_t nfin = 0, top = 0;
+  for_piece(lg, sz.vec, i0, i1, [&](int i, float v) {
+    if (v > best) { best = v; best_i = i; }
+    if (finite_f(v)) ++nfin, top = max(top, key_of(v));
+  });
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) {
+    first_max(best, best_i, __shfl_xor(best, o, WAVE), __shfl_xor(best_i, o, WAVE));
+    nfin += __shfl_xor(nfin, o, WAVE);
+    top = max(top, (uint32_t)__shfl_xor((int)top, o, WAVE));
   }
-  if (lane == 0) leave(sh.one.s_id2[pick]);
+  const size_t at = (size_t)row * sz.pieces + piece;
+  if (threadIdx.x % WAVE == 0) {
+    bv[wave] = best;
+    bi[wave] = best_i;
+    nv[wave] = nfin;
+    sp.wave_key[at * HEAD_WAVES + wave] = top;
+  }
+  __syncthreads();
+  if (threadIdx.x >= HEAD_WAVES) return;
+  best = bv[threadIdx.x], best_i = bi[threadIdx.x], nfin = nv[threadIdx.x];
+#pragma unroll
+  for (int o = HEAD_WAVES / 2; o > 0; o >>= 1) {
+    first_max(best, best_i, __shfl_xor(best, o, HEAD_WAVES), __shfl_xor(best_i, o, HEAD_WAVES));
+    nfin += __shfl_xor(nfin, o, HEAD_WAVES);
+  }
+  if (threadIdx.x == 0) {
+    sp.piece_best[at] = best;
+    sp.piece_arg[at] = best_i;
+    sp.piece_finite[at] = nfin;
+  }
+}
+
+// Whether the two kernels above and below take rows cut like this that keep up to `most` candidates: half as many groups again to
+// bound them with (fewer leave a bound that many values reach).
+__host__ __device__ int bound_set(const SampleShape& sz) {
+  const int waves = sz.pieces * HEAD_WAVES;
+  return waves <= BOUND_SET ? waves : waves / 4;
+}
+bool head_takes(const SampleShape& sz, int most) { return most * 3 <= bound_set(sz) * 2; }
+
+struct HeadEnd {
+  FewShared select;
+  SampleShared one;
+  uint32_t bound[BOUND_SET];
+  u64 held[HEAD_HELD];
+  int group[MAX_PIECES * HEAD_WAVES];
+  int groups;
+  uint32_t least;
+  float sums[HEAD_HELD];                 // running sums of the weights
+};
+
+template <typename Options>
+__global__ __launch_bounds__(PNT) void sample_head_end_kernel(const float* __restrict__ logits, SampleShape sz, Options opt, HeadSpace sp,
+                                                              int* __restrict__ out, int* __restrict__ out_host) {
+  __shared__ HeadEnd sh;
+  const int row = blockIdx.x, tk = opt.top_k[row];
+  const float T = opt.temperature[row], t = fmaxf(T, 1e-5f), tp = opt.top_p[row], uniform = opt.uniform[row];
+  const float* lg = logits + (size_t)row * sz.ldl;
+  auto leave = [&](int id) {
+    out[row] = id;
+    if (out_host) out_host[row] = id;
+  };
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int waves = sz.pieces * HEAD_WAVES;
+  const uint32_t* wave_key = sp.wave_key + (size_t)row * waves;
+  auto scaled = [&](uint32_t key) { return key ? key_of(value_of(key) / t) : 0u; };
+  static_assert(MAX_PIECES * HEAD_WAVES <= PNT, "a thread looks at one wave's key");
+  const uint32_t mine = (int)threadIdx.x < waves ? wave_key[threadIdx.x] : 0u;
+  const bool fours = waves > BOUND_SET;
+  uint32_t own = 0;                                     // this thread's of the set
+  if (!fours) own = mine;
+  else if ((int)threadIdx.x < waves / 4) {
+    const uint4 q = reinterpret_cast<const uint4*>(wave_key)[threadIdx.x];
+    own = max(max(q.x, q.y), max(q.z, q.w));
+  }
+  float best = -INFINITY;
+  int best_i = 0x7fffffff;
+  uint32_t n = 0;
+  if (lane < sz.pieces) {                               // every wave for itself, a piece a lane
+    const size_t at = (size_t)row * sz.pieces + lane;
+    best = sp.piece_best[at];
+    best_i = sp.piece_arg[at];
+    n = sp.piece_finite[at];
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) {
+    first_max(best, best_i, __shfl_xor(best, o, WAVE), __shfl_xor(best_i, o, WAVE));
+    n += __shfl_xor(n, o, WAVE);
+  }
+  if (n == 0u || T <= 1e-5f) {
+    if (threadIdx.x == 0) leave(n == 0u || best_i == 0x7fffffff ? 0 : best_i);
+    return;
+  }
+  const bool cut = tk > 0 && n > (uint32_t)tk;
+  const uint32_t keep = cut ? (uint32_t)tk : n;
+  const bool use_top_p = tp >= 0.0f && tp < 1.0f && keep > 1u;
+  const int set = bound_set(sz);
+  if (tk <= 0 || tk * 3 > set * 2 || !(cut || use_top_p)) {
+    // the caller's word on the row was wrong, or fewer candidates than top-k keeps and no top-p: drawn in id order
+    if (threadIdx.x >= SNT) return;                     // (whole waves: a barrier does not wait for those that have ended)
+    sample_row_one_block(sh.one, lg, sz.V, T, tk, tp, uniform, out + row);
+    __syncthreads();
+    if (out_host && threadIdx.x == 0) out_host[row] = *(volatile int*)(out + row);
+    return;
+  }
+  // the bound: the keep-th largest of the set.  The lowest byte says who is who, so no two are alike, and is then left out
+  const uint32_t tag = BOUND_SET - 1 - threadIdx.x, who = (scaled(own) & ~(uint32_t)(BOUND_SET - 1)) | tag;
+  if ((int)threadIdx.x < BOUND_SET) sh.bound[threadIdx.x] = (int)threadIdx.x < set ? who : 0u;
+  if (threadIdx.x == 0) sh.groups = 0, sh.least = 0u, sh.select.count = 0;
+  __syncthreads();
+  if (cut) {
+    if ((int)threadIdx.x < set) {
+      int above = 0;
+      const uint4* others = reinterpret_cast<const uint4*>(sh.bound);
+#pragma unroll 8
+      for (int q = 0; q < (set + 3) / 4; ++q) {
+        const uint4 o = others[q];
+        above += (o.x > who) + (o.y > who) + (o.z > who) + (o.w > who);
+      }
+      if (above == (int)keep - 1) sh.least = who & ~(uint32_t)(BOUND_SET - 1);
+    }
+    __syncthreads();
+  }
+  const uint32_t least = max(sh.least, 1u);
+  if (scaled(mine) >= least) sh.group[atomicAdd(&sh.groups, 1)] = threadIdx.x;
+  __syncthreads();
+  // f(sort key) for every finite value of these groups: a wave takes four rounds of a group at a time
+  const int per = sz.vec ? 4 * PNT : PNT, rounds = ceil_div(sz.chunk, per), items = sh.groups * rounds;
+  auto each = [&](auto f) {
+    for (int q = wave * 4; q < items; q += PNT / WAVE * 4) {
+      float x[4][4];
+      int at[4], end[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int item = min(q + u, items - 1), g = sh.group[item / rounds], piece = g / HEAD_WAVES, i0 = piece * sz.chunk;
+        end[u] = q + u < items ? min(sz.V, i0 + sz.chunk) : 0;
+        at[u] = i0 + item % rounds * per + (g % HEAD_WAVES * WAVE + lane) * (sz.vec ? 4 : 1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[u][e] = INFINITY;
+        if (sz.vec) {
+          if (at[u] + 3 < end[u]) {
+            const float4 v = *reinterpret_cast<const float4*>(lg + at[u]);
+            x[u][0] = v.x, x[u][1] = v.y, x[u][2] = v.z, x[u][3] = v.w;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (at[u] + e < end[u]) x[u][e] = lg[at[u] + e];
+          }
+        } else if (at[u] < end[u]) {
+          x[u][0] = lg[at[u]];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (finite_f(x[u][e])) f(sort_key(key_of(x[u][e] / t), at[u] + e, sz.id_bits, 0));
+    }
+  };
+  auto gather = [&](u64 from) {
+    each([&](u64 c) {
+      if (c < from) return;
+      const uint32_t j = atomicAdd(&sh.select.count, 1u);
+      if (j < (uint32_t)HEAD_HELD) sh.held[j] = c;
+    });
+    __syncthreads();
+  };
+  gather((u64)least << 32);
+  if (sh.select.count > (uint32_t)HEAD_HELD) {          // (the same for all threads)
+    const u64 from = few_threshold<PNT>(sh.select, keep, keep, 32 + sz.id_bits, each);
+    __syncthreads();
+    if (threadIdx.x == 0) sh.select.count = 0;
+    __syncthreads();
+    gather(from);
+  }
+  const int found = (int)sh.select.count;
+  for (int e = threadIdx.x; e < found; e += PNT) {
+    const u64 c = sh.held[e];
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < found; ++j) rank += sh.held[j] > c ? 1 : 0;
+    if (rank < (int)keep) {
+      sh.one.s_key2[rank] = (uint32_t)(c >> 32);
+      sh.one.s_id2[rank] = id_of_sort_key(c, sz.id_bits, 0);
+    }
+  }
+  __syncthreads();
+  draw_in_order<PNT>(sh.one, reinterpret_cast<float*>(sh.select.hist), sh.sums, (int)keep, use_top_p, tp, uniform, leave);
 }
 
 std::mutex pass_attr_lock;
@@ -1391,9 +1620,18 @@ SampleShape shape_of(const float* logits, int ldl, int n_rows, int V) {
   return sz;
 }
 
+// `most`: the largest top-k of the rows that sample, where the host knows it (else 0)
 template <typename Options>
-int launch_few(const float* logits, const SampleShape& sz, const Options& opt, void* scratch, int* out, int* out_host, hipStream_t stream) {
+int launch_few(const float* logits, const SampleShape& sz, const Options& opt, void* scratch, int* out, int* out_host, int most,
+               hipStream_t stream) {
   const FewSpace fs = carve_few(scratch, sz.R);
+  if (most > 0 && head_takes(sz, most)) {
+    hipLaunchKernelGGL(sample_head_pieces_kernel, dim3(sz.pieces, sz.R), dim3(PNT), 0, stream, logits, sz, head_space(fs));
+    APC_LAUNCH_CHECK();
+    hipLaunchKernelGGL(sample_head_end_kernel<Options>, dim3(sz.R), dim3(PNT), 0, stream, logits, sz, opt, head_space(fs), out, out_host);
+    APC_LAUNCH_CHECK();
+    return 0;
+  }
   hipLaunchKernelGGL(sample_few_pieces_kernel<Options>, dim3(sz.pieces, sz.R), dim3(PNT), 0, stream, logits, sz, opt, fs);
   APC_LAUNCH_CHECK();
   hipLaunchKernelGGL(sample_few_end_kernel<Options>, dim3(sz.R), dim3(SNT), 0, stream, logits, sz, opt, fs, out, out_host);
@@ -1490,7 +1728,7 @@ APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, 
   if (!few)
     if (const int rc = allow_pass_lds(dev)) return rc;
   const SampleShape sz = shape_of(logits, ldl, n_rows, V);
-  if (few) return launch_few(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, scratch, out, nullptr, stream);
+  if (few) return launch_few(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, scratch, out, nullptr, 0, stream);
   return launch_descents(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, nullptr, scratch, out, nullptr, cuts, stream);
 }
 
@@ -1523,7 +1761,12 @@ APC_EXPORT int apc_sample_rows_host(const float* logits, int ldl, int n_rows, in
     opt.uniform[r] = (float)(splitmix64(splitmix64(seed) ^ ((number + 1) * 0xD6E8FEB86659FD93ull)) >> 40) / (float)(1 << 24);
   }
   const SampleShape sz = shape_of(logits, ldl, n_rows, V);
-  if (few) return launch_few(logits, sz, opt, scratch, out, out_host, stream);
+  if (few) {
+    int most = 0;                                        // (greedy rows may ask for any)
+    for (int r = 0; r < n_rows; ++r)
+      if (opt.temperature[r] > 1e-5f) most = std::max(most, opt.top_k[r]);
+    return launch_few(logits, sz, opt, scratch, out, out_host, most, stream);
+  }
   if (const int rc = allow_pass_lds(dev)) return rc;
   return launch_descents(logits, sz, RowOptions{}, &opt, scratch, out, out_host, cuts, stream);
 }

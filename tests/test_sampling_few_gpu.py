@@ -140,3 +140,51 @@ def test_a_result_that_is_dropped_keeps_its_memory_until_the_kernel_is_through()
     assert device.tolist() == want and list(ops._still_written)[-1][1][-1].query()
     ops.PinnedIds(1)
     assert len(ops._still_written) == 0
+
+
+def with_the_launch(logits, temperature, top_k, top_p):
+    """(ids by options that go with the launch, ids of the kernel of one block a row)"""
+    from allpaca_amd.kernels import ops
+    from allpaca_amd.sampling.sampler import uniforms_for
+    R = logits.shape[0]
+    temps, ks, tops = ([x] * R if np.isscalar(x) else list(x) for x in (temperature, top_k, top_p))
+    seeds, numbers = [31 * r + top_k if np.isscalar(top_k) else r for r in range(R)], list(range(R))
+    f = lambda x, dt: torch.tensor(x, dtype=dt, device=DEV)  # noqa: E731
+    got, want = (torch.full((R,), -7, dtype=torch.int32, device=DEV) for _ in range(2))
+    ops.sample_rows(logits, temps, ks, tops, (seeds, numbers), got, few_after_top_k=True)
+    ops.sample_rows(logits, f(temps, torch.float32), f(ks, torch.int32), f(tops, torch.float32),
+                    torch.from_numpy(uniforms_for(seeds, numbers)).to(DEV), want, one_block=True)
+    return got.tolist(), want.tolist()
+
+
+# the bound from waves' largest values: sets of 48 to 256 waves and of fours of waves; the largest top-k that they take and the next; pieces of
+# several rounds (64 rows) and a ragged last one; rows that start off 16 bytes
+@pytest.mark.parametrize("V,R", [(12289, 3), (32001, 8), (65536, 1), (128256, 16), (128255, 8), (60001, 64)])
+def test_top_k_bounded_by_the_largest_values_of_groups(V, R):
+    logits = torch.randn(R, V + 3, generator=torch.Generator(device=DEV).manual_seed(V), device=DEV) * 3
+    for view in (logits[:, :V], logits[:, 1:V + 1]):
+        for top_k in (1, 31, 32, 40, 85, 86):
+            got, want = with_the_launch(view, 0.8, top_k, 0.95)
+            assert got == want, top_k
+
+
+@pytest.mark.parametrize("V", [20000, 70001])
+def test_groups_of_unlike_and_of_like_values(V):
+    """All large values in one group, equal values, values in order, few that are finite: more than the block holds stand at the bound."""
+    rng = np.random.default_rng(3)
+    rows = [np.full(V, 1.5), np.round(rng.normal(size=V)), np.sort(rng.normal(size=V)), -np.sort(rng.normal(size=V)), np.full(V, -np.inf),
+            np.full(V, np.nan), rng.normal(size=V), np.where(np.arange(V) % 2, 0.0, -0.0), rng.normal(size=V) * 1e-38, rng.normal(size=V) * 1e38,
+            np.full(V, -np.inf), np.full(V, -np.inf), rng.normal(size=V)]
+    rows[1][::3] = -0.0
+    rows[3][700:] = -np.inf
+    rows[6][[3, 77]] = np.inf
+    rows[10][[5, V - 1]] = 2.0, 2.0
+    rows[11][np.arange(0, V, V // 30)] = rng.normal(size=np.arange(0, V, V // 30).size)
+    rows[12][4096:4096 + 900] += 20.0                        # 900 values far above all others
+    logits = torch.tensor(np.stack(rows), dtype=torch.float32, device=DEV)
+    for top_k in (1, 40):
+        for top_p in (0.3, 0.95, 1.0):
+            got, want = with_the_launch(logits, 0.7, top_k, top_p)
+            assert got == want, (top_k, top_p)
+    got, want = with_the_launch(logits, [0.7, 0.0, 1e-6] * 4 + [1.5], [40, 7, 0] * 4 + [3], [0.9, 1.0, 0.5] * 4 + [0.4])
+    assert got == want
