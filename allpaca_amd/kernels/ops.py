@@ -1293,6 +1293,36 @@ def delta_rule(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, n_heads: 
                                 _stream()), "delta_rule")
 
 
+def delta_step(x: torch.Tensor, q_off: int, k_off: int, v_off: int, n_heads: int, n_kv_heads: int, key_dim: int, value_dim: int,
+               a_off: int, b_off: int, g_off: int, conv_w: torch.Tensor, conv_state: Optional[torch.Tensor],
+               conv_slots: Optional[torch.Tensor], A: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor, slots: torch.Tensor,
+               norm_w: torch.Tensor, eps: float, step, out: torch.Tensor) -> bool:
+    """For a step of single rows, in one launch: `conv_channels` (silu) of x's columns up to v_off + heads * value_dim, `delta_rule` of what
+    that gives with the logits at a_off and b_off, and `gated_rmsnorm` of a head's output (group value_dim, the gate at g_off through
+    silu) into `out`, x's type.  False (nothing done) for sizes that it does not take."""
+    H, G, dk, dv = int(n_heads), int(n_kv_heads), int(key_dim), int(value_dim)
+    T, taps = x.shape[0], int(conv_w.shape[1])
+    L = _lib.load("plain")
+    if (not getattr(step, "decode_only", False) or step.n_segs != T or x.dtype not in (torch.float32, torch.bfloat16) or out.dtype != x.dtype
+            or (taps > 1 and (conv_state is None or conv_slots is None))
+            or not L.apc_delta_step_takes(H, G, dk, dv, taps, state.data_ptr())):
+        return False
+    _gpu(x, conv_w, conv_state, conv_slots, A, dt_bias, state, slots, norm_w, out)
+    ldx, ldo, C = _rows(x, "rows"), _rows(out, "delta step out"), v_off + H * dv
+    _need(max(C, a_off + H, b_off + H, g_off + H * dv, q_off + G * dk, k_off + G * dk) <= x.shape[1], "delta step: columns exceed the row")
+    _need(conv_w.shape[0] == C and conv_w.dtype == torch.float32 and conv_w.is_contiguous(), "delta step: weights must be float32 [channels, taps]")
+    _need(taps == 1 or (conv_state.dtype == torch.float32 and conv_state.is_contiguous() and tuple(conv_state.shape[1:]) == (taps - 1, C)),
+          f"delta step: inputs kept must be float32 [slots, {taps - 1}, {C}]")
+    _need(out.shape == (T, H * dv) and state.dtype == torch.float32 and state.is_contiguous() and tuple(state.shape[1:]) == (H, dk, dv),
+          f"delta step: out [rows, heads * value_dim], state float32 [slots, {H}, {dk}, {dv}]")
+    _lib.check(L.apc_delta_step(
+        x.data_ptr(), _code(x), ldx, q_off, k_off, v_off, H, G, dk, dv, a_off, b_off, g_off, conv_w.data_ptr(), taps,
+        conv_state.data_ptr() if taps > 1 else 0, _f32(A, H, "A"), _f32(dt_bias, H, "dt bias"), float(dk) ** -0.5, state.data_ptr(),
+        _f32(norm_w, H * dv, "norm weight"), float(eps), T, _i32(step.row_seg, T, "row_seg"),
+        _i32(conv_slots, T, "slots") if taps > 1 else 0, _i32(slots, T, "slots"), out.data_ptr(), ldo, _stream()), "delta_step")
+    return True
+
+
 def gated_recurrence(u: torch.Tensor, z: torch.Tensor, z_bias: torch.Tensor, blocks: int, rate: torch.Tensor,
                      y: torch.Tensor, y_bias: Optional[torch.Tensor], state: torch.Tensor, step, slots: torch.Tensor,
                      out: torch.Tensor, out_scale: float = 1.0) -> None:

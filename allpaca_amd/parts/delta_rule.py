@@ -91,14 +91,22 @@ class GatedDeltaRule(Mixer):
         T, dev, dt, N = h.shape[0], h.device, self.rt.dtype, self.H * self.dv
         proj = torch.empty((T, self.width), dtype=dt, device=dev)
         ops.linear(h, self.w_in, proj)
+        a = torch.empty((T, N), dtype=dt, device=dev)
+        if not ops.delta_step(proj, self.q_off, self.k_off, self.v_off, self.H, self.G, self.dk, self.dv, self.a_off, self.a_off + self.H,
+                              self.g_off, self.conv_w, conv.state if conv is not None else None, conv.slots if conv is not None else None,
+                              self.A, self.dt_bias, state.state, state.slots, self.norm_w, self.eps, step, a):
+            self._apart(proj, step, state, conv, a)
+        out = torch.empty((T, self.D), dtype=torch.float32, device=dev)
+        ops.linear(a, self.w_o, out)
+        return out
+
+    def _apart(self, proj, step, state, conv, a) -> None:
+        """Convolutions, rule and gated norm one after the other."""
+        T, dev, dt, N = proj.shape[0], proj.device, self.rt.dtype, self.H * self.dv
         act = torch.empty((T, self.channels), dtype=dt, device=dev)
         ops.conv_channels(proj, self.channels, self.conv_w, None, conv.state if conv is not None else None, step,
                           conv.slots if conv is not None else None, "silu", act)
         o = torch.empty((T, N), dtype=torch.float32, device=dev)
         ops.delta_rule(act, self.q_off, self.k_off, self.v_off, self.H, self.G, self.dk, self.dv, proj, self.a_off,
                        self.a_off + self.H, self.A, self.dt_bias, state.state, step, state.slots, o)
-        a = torch.empty((T, N), dtype=dt, device=dev)
         ops.gated_rmsnorm(o, self.norm_w, self.eps, proj[:, self.g_off:self.g_off + N], a, group=self.dv, gate_act="silu")
-        out = torch.empty((T, self.D), dtype=torch.float32, device=dev)
-        ops.linear(a, self.w_o, out)
-        return out

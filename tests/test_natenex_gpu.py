@@ -633,3 +633,42 @@ def test_a_recurrent_step_in_one_launch(M, C, parts, taps, biases):
     p17 = torch.zeros((17, 2 * C), dtype=tdt, device=DEV)
     assert not ops.recurrent_step(p17[:, C:], p17[:, :C], x_b, conv_w, conv_b, conv, many.state_slots, gates, zb, parts, rate, y_b, state,
                                   many.state_slots, many, torch.empty((17, C), dtype=tdt, device=DEV))
+
+
+# one to four value heads a key head (three of them: threads that are no power of two); keys of 6 to 128, values of 8 to 64; one to eight taps
+@pytest.mark.parametrize("M, H, G, dk, dv, taps", [(8, 32, 16, 64, 64, 4), (1, 3, 1, 6, 8, 3), (16, 4, 4, 128, 48, 2), (5, 4, 1, 32, 64, 1), (3, 8, 4, 72, 20, 8),
+                                                   (70, 6, 2, 40, 32, 4)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_delta_step_in_one_launch(M, H, G, dk, dv, taps, dtype):
+    """The same bits as the convolutions, the rule and the gated norm one after the other, and the same states behind them; other
+    requests' states are left alone."""
+    from allpaca_amd.kernels import ops
+    rng = np.random.default_rng(H * 100 + dk + dv)
+    tdt = DTYPES[dtype]
+    C, N = 2 * G * dk + H * dv, H * dv
+    g_off = -(-C // 8) * 8
+    a_off = -(-(g_off + N) // 8) * 8
+    width = -(-(a_off + 2 * H) // 8) * 8
+    conv_w = dev(np.float32(rng.normal(size=(C, taps)) * 0.4))
+    A, bias = dev(np.float32(np.exp(rng.normal(size=H)))), dev(np.float32(rng.normal(size=H) - 1.0))
+    norm_w = dev(np.float32(1.0 + 0.1 * rng.normal(size=N)))
+    slots = rng.permutation(M + 2)[:M].tolist()
+    step = make_step([(7, 1)] * M, [[1]] * M, slots)
+    s = step.state_slots
+    conv = dev(np.float32(rng.normal(size=(M + 3, taps - 1, C)))) if taps > 1 else None
+    state = dev(np.float32(rng.normal(size=(M + 3, H, dk, dv))))
+    conv2, state2 = conv.clone() if taps > 1 else None, state.clone()
+    out, want = (torch.full((M, N + 8), 9.0, dtype=tdt, device=DEV) for _ in range(2))
+    for _ in range(2):
+        proj = dev(bf(rng.normal(size=(M, width))), tdt)
+        assert ops.delta_step(proj, 0, G * dk, 2 * G * dk, H, G, dk, dv, a_off, a_off + H, g_off, conv_w, conv, s, A, bias, state, s, norm_w,
+                              1e-6, step, out[:, :N])
+        act, o = torch.empty((M, C), dtype=tdt, device=DEV), torch.empty((M, N), dtype=torch.float32, device=DEV)
+        ops.conv_channels(proj, C, conv_w, None, conv2, step, s if taps > 1 else None, "silu", act)
+        ops.delta_rule(act, 0, G * dk, 2 * G * dk, H, G, dk, dv, proj, a_off, a_off + H, A, bias, state2, step, s, o)
+        ops.gated_rmsnorm(o, norm_w, 1e-6, proj[:, g_off:g_off + N], want[:, :N], group=dv, gate_act="silu")
+        assert torch.equal(out, want) and torch.equal(state, state2) and (taps == 1 or torch.equal(conv, conv2))
+    two = make_step([(7, 2)] * M, [[1]] * M, slots)
+    p2 = torch.zeros((2 * M, width), dtype=tdt, device=DEV)
+    assert not ops.delta_step(p2, 0, G * dk, 2 * G * dk, H, G, dk, dv, a_off, a_off + H, g_off, conv_w, conv, s, A, bias, state, s, norm_w,
+                              1e-6, two, torch.empty((2 * M, N), dtype=tdt, device=DEV))
