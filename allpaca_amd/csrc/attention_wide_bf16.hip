@@ -68,6 +68,7 @@
 // bits with two blocks a compute unit.)
 // Formula: crates/allpaca-cpu/src/kernels.rs:293-356.  Reference kernel (contiguous K/V, no matrix cores):
 // attention_qtile_kernel hip/src/kernels.cpp:2203.
+#include "attention_decode.h"
 #include "attention_wide.h"
 #include "mfma.h"
 #include <math.h>
@@ -281,14 +282,35 @@ __device__ __forceinline__ void soft_any(int h, floatx16& s, Frag (&pf)[2], Soft
 
 // WIN: the rows see a window of keys (without one, a row's first key is key 0, which costs no register)
 // HD: the head size, 128 or 64 (half the MFMAs a pass for the same softmax)
-template <int HD, bool WIN>
+// DEC: DEC_LAST or DEC_WHOLE: a step's prompt rows and decoded rows in one launch (NO_DECODE: prompt rows alone).  The first
+// `wide_blocks` blocks are the prompt rows', the others those of attn_decode_kernel; each leaves the bits it leaves in a launch of its
+// own.  Decoded rows are latency, some 15 us for a few megabytes, and a portion of a prompt hardly ever fills its last round of blocks
+// (504 rows x 32 heads of 128: 128 blocks on 256 compute units), so one goes beside the other: these rows over 2,048 keys, 8 decoded
+// ones of 700 to 2,047 beside them, 39.2 + 15.0 -> 39.9 us a layer.
+constexpr int NO_DECODE = -1;
+template <int HD, bool WIN, int DEC>
 __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kernel(
     const bf16_t* __restrict__ q, int ldq, int q_off, bf16_t* __restrict__ out, int ldo, int H, int Hk,
     const bf16_t* __restrict__ cache, int lgP, const int* __restrict__ block_table, int max_blocks,
     const int* __restrict__ positions, const int* __restrict__ row_seg, const int* __restrict__ tile_row0,
     const int* __restrict__ tile_rows, int n_tiles, int window_arg, float scale, int n_splits, int part_rows,
-    float* __restrict__ parts) {
+    float* __restrict__ parts,
+    int wide_blocks, int page_tokens, AttnDecodeRows dec) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  if constexpr (DEC != NO_DECODE) {
+    if ((int)blockIdx.x >= wide_blocks) {
+      constexpr int MEET = attn_decode::DEC_P_ELEMS * 2 + 16;   // (is_last lies behind P)
+      static_assert(MEET % 16 == 0 && MEET + attn_decode::NW * 16 * (HD + 2) * 4 <= lds_request(HD), "what a block's waves meet in");
+      const int pairs = Hk * ceil_div(H / Hk, 16), id = (int)blockIdx.x - wide_blocks;
+      const attn_decode::DecodeAt blk{id % dec.n, id / dec.n % pairs, id / dec.n / pairs, dec.n, pairs,
+                                      DEC == attn_decode::DEC_WHOLE ? 1 : ceil_div(dec.n_parts, attn_decode::NW)};
+      attn_decode::attn_decode_block<HD, DEC, true>(
+          blk, reinterpret_cast<bf16_t*>(smem), reinterpret_cast<float*>(smem + MEET),
+          reinterpret_cast<int*>(smem + attn_decode::DEC_P_ELEMS * 2), q, ldq, q_off, H, Hk, HD, cache, page_tokens, block_table,
+          max_blocks, positions, row_seg, dec.rows, WIN ? window_arg : 0, scale, 0, dec.n_parts, dec.workspace, out, ldo, dec.counters);
+      return;
+    }
+  }
   const int window = WIN ? window_arg : 0;
   constexpr int d = HD;
   constexpr int DT = d / 32;                 // tiles of 32 elements of a head; also a wave's direct loads per K or V tile
@@ -991,7 +1013,7 @@ int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, i
                              const bf16_t* cache, int page_tokens, const int* block_table, int max_blocks,
                              const int* positions, const int* row_seg, const int* tile_row0, const int* tile_rows,
                              int n_tiles, int window, float scale, int n_splits, int part_rows, float* parts,
-                             int d, hipStream_t stream) {
+                             int d, hipStream_t stream, const AttnDecodeRows* dec) {
   if (!attn_wide_takes(Hk, d, page_tokens)) return APC_ERR_UNSUPPORTED;
   if (n_splits < 1 || n_splits > 8 || (n_splits > 1 && (!parts || part_rows <= 0)) ||
       (long)n_tiles * H * n_splits > 0x7fffffffL)
@@ -1001,29 +1023,55 @@ int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, i
   while ((1 << lgP) < page_tokens) ++lgP;
   static bool configured[64] = {};
   static std::mutex configured_lock;
-  const auto kernel = d == 128 ? (window > 0 ? attn_prefill_wide_kernel<128, true> : attn_prefill_wide_kernel<128, false>)
-                               : (window > 0 ? attn_prefill_wide_kernel<64, true> : attn_prefill_wide_kernel<64, false>);
   const int lds = lds_request(d);
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return (int)e;
   if (dev < 0 || dev >= 64) return APC_ERR_UNSUPPORTED;
+#define WIDE_ARGS                                                                                                             \
+  q, ldq, q_off, out, ldo, H, Hk, cache, lgP, block_table, max_blocks, positions, row_seg, tile_row0, tile_rows, n_tiles, window, scale, \
+      n_splits, part_rows, parts
+#define WIDE_INSTANCES(DO_) DO_(128, true) DO_(128, false) DO_(64, true) DO_(64, false)
   {  // more LDS than a kernel gets without asking: once per device
     std::lock_guard<std::mutex> hold(configured_lock);
     if (!configured[dev]) {
-      const std::pair<const void*, int> instances[] = {
-          {(const void*)attn_prefill_wide_kernel<128, true>, 128}, {(const void*)attn_prefill_wide_kernel<128, false>, 128},
-          {(const void*)attn_prefill_wide_kernel<64, true>, 64}, {(const void*)attn_prefill_wide_kernel<64, false>, 64}};
-      for (const auto& [f, hd] : instances) {
-        e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_request(hd));
-        if (e != hipSuccess) return (int)e;
-      }
+#define ALLOW(HD_, WIN_)                                                                             \
+  for (const void* f : {(const void*)attn_prefill_wide_kernel<HD_, WIN_, NO_DECODE>,                 \
+                        (const void*)attn_prefill_wide_kernel<HD_, WIN_, attn_decode::DEC_LAST>,     \
+                        (const void*)attn_prefill_wide_kernel<HD_, WIN_, attn_decode::DEC_WHOLE>}) { \
+    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_request(HD_));        \
+    if (e != hipSuccess) return (int)e;                                                              \
+  }
+      WIDE_INSTANCES(ALLOW)
+#undef ALLOW
       configured[dev] = true;
     }
   }
-  hipLaunchKernelGGL(kernel, dim3(n_tiles * H * n_splits), dim3(256), lds, stream, q, ldq,
-                     q_off, out, ldo, H, Hk, cache, lgP, block_table, max_blocks, positions, row_seg, tile_row0, tile_rows,
-                     n_tiles, window, scale, n_splits, part_rows, parts);
+  const long blocks = (long)n_tiles * H * n_splits;
+  if (dec) {
+    const bool last = dec->workspace != nullptr;
+    const long all = blocks + (long)dec->n * Hk * ceil_div(H / Hk, 16) * (last ? ceil_div(dec->n_parts, attn_decode::NW) : 1);
+    if (all > 0x7fffffffL) return APC_ERR_BAD_ARG;
+    const auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)all), dim3(256), lds, stream, WIDE_ARGS, (int)blocks, page_tokens, *dec);
+    };
+#define MIXED(HD_, WIN_)                                                                       \
+  if (d == HD_ && (window > 0) == WIN_) {                                                      \
+    if (last) launch(attn_prefill_wide_kernel<HD_, WIN_, attn_decode::DEC_LAST>);              \
+    else launch(attn_prefill_wide_kernel<HD_, WIN_, attn_decode::DEC_WHOLE>);                  \
+  }
+    WIDE_INSTANCES(MIXED)
+#undef MIXED
+  } else {
+#define WIDE(HD_, WIN_)                                                                                                   \
+  if (d == HD_ && (window > 0) == WIN_)                                                                                   \
+    hipLaunchKernelGGL((attn_prefill_wide_kernel<HD_, WIN_, NO_DECODE>), dim3((unsigned)blocks), dim3(256), lds, stream, WIDE_ARGS, \
+                       (int)blocks, page_tokens, AttnDecodeRows{});
+    WIDE_INSTANCES(WIDE)
+#undef WIDE
+  }
+#undef WIDE_ARGS
+#undef WIDE_INSTANCES
   APC_LAUNCH_CHECK();
   if (n_splits > 1) {
 #define MERGE(S_)                                                                                                       \

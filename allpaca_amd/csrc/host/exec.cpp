@@ -449,6 +449,21 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
   const float sc = L.scale != 0.f ? L.scale : 1.0f / std::sqrt((float)d);
   const int* table = s.table[E.group];
   const int width = s.table_width[E.group];
+  // how the decoded rows' keys are shared out
+  const int n = s.n_decode;
+  const int span = window ? std::min(s.max_decode_context, window) : s.max_decode_context;
+  const int* rows = s.all_rows_decode ? nullptr : s.decode_rows;
+  const long pairs = (long)n * Hk * cdiv(H / Hk, 16);
+  const int n_parts = n ? decode_parts(pairs, span) : 0;
+  const bool pair_fits = apc_attention_decode_whole_fits(H, Hk, d);
+  const bool even = n && decode_even(pairs, span, pair_fits, P.tun.even_min_pairs, P.tun.even_min_span) &&
+                    (!pair_fits || even_pays(s.decode_steps, s.decode_longest, n, (int)(pairs / n), window)) && pairs <= P.pair_capacity &&
+                    out.ld % 4 == 0 && ((uintptr_t)out.p & 7u) == 0;
+  // (rows so short that one block's waves take a pair's ranges need no partial results either)
+  const bool whole = n && !even && (pairs >= P.tun.whole_min_pairs || n_parts <= WHOLE_WAVES) && pair_fits;
+  const bool last = n && !even && !whole && P.tun.last_block_merges && pairs <= P.pair_capacity &&
+                    apc_attention_decode_last_fits(H, Hk, d, n_parts);
+  const size_t last_floats = last ? (size_t)n * H * cdiv(n_parts, WHOLE_WAVES) * (d + 2) : 0;
   if (s.n_tiles) {
     const bool wide = P.tun.wide_tiles && apc_attention_prefill_wide_takes(Hk, d, page, s.n_tiles, T - s.n_decode);
     const int splits = !wide ? 1
@@ -457,51 +472,38 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
                            : key_splits(s.n_tiles, H, s.max_prompt_keys, window, P.tun.key_splits_max,
                                         std::max(1, P.tun.key_range_min));
     float* parts = splits > 1 ? P.floats((size_t)splits * T * H * (d + 2)) : nullptr;
+    // (rows dealt out evenly fill the chip by themselves)
+    if (wide && (whole || last) && apc_attention_mixed_takes(H, Hk, d, page, s.n_tiles, T - n, n, n_parts, last)) {
+      float* ws = last ? P.floats(last_floats) : nullptr;
+      LAUNCH(P, "attention_mixed_bf16",
+             apc_attention_mixed_bf16(q.p, q.ld, 0, out.p, out.ld, H, Hk, d, E.kv, page, table, width, s.positions, s.row_seg, s.tile_row0,
+                                      s.tile_rows, s.n_tiles, T - n, window, sc, splits, T, parts, rows, n, n_parts, ws,
+                                      last ? P.pair_counters : nullptr, P.stream));
+      return 1;
+    }
     LAUNCH(P, "attention_prefill_bf16",
            apc_attention_prefill_bf16(q.p, q.ld, 0, out.p, out.ld, H, Hk, d, E.kv, page, table, width,
                                       s.positions, s.row_seg, s.tile_row0, s.tile_rows,
                                       s.n_tiles, P.tun.wide_tiles ? T - s.n_decode : 0, window, sc, splits, T, parts,
                                       P.stream));
   }
-  if (s.n_decode) {
-    const int n = s.n_decode;
-    const int span = window ? std::min(s.max_decode_context, window) : s.max_decode_context;
-    const int* rows = s.all_rows_decode ? nullptr : s.decode_rows;
-    const long pairs = (long)n * Hk * cdiv(H / Hk, 16);
-    const int n_parts = decode_parts(pairs, span);
-    const bool pair_fits = apc_attention_decode_whole_fits(H, Hk, d);
-    if (decode_even(pairs, span, pair_fits, P.tun.even_min_pairs, P.tun.even_min_span) &&
-        (!pair_fits || even_pays(s.decode_steps, s.decode_longest, n, (int)(pairs / n), window)) && pairs <= P.pair_capacity &&
-        out.ld % 4 == 0 && ((uintptr_t)out.p & 7u) == 0) {
-      float* ws = P.floats((size_t)apc_attention_decode_even_workspace(H, Hk, d));
-      LAUNCH(P, "attention_decode_bf16 (even shares)",
-             apc_attention_decode_even_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width, s.positions,
-                                            s.row_seg, rows, window, sc, ws, P.pair_counters, P.stream));
-      return 1;
-    }
-    // (rows so short that one block's waves take a pair's ranges need no partial results either)
-    if ((pairs >= P.tun.whole_min_pairs || n_parts <= WHOLE_WAVES) && pair_fits) {
-      // no length of the ranges: every row's own keys, one range a wave of its block
-      LAUNCH(P, "attention_decode_bf16 (whole)",
-             apc_attention_decode_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width,
-                                       s.positions, s.row_seg, rows, window, sc, 0, 0, nullptr, nullptr,
-                                       P.stream));
-      return 1;
-    }
-    const int kw = 0;  // every row's own keys in n_parts ranges
-    if (P.tun.last_block_merges && pairs <= P.pair_capacity && apc_attention_decode_last_fits(H, Hk, d, n_parts)) {
-      const int nz = (int)cdiv(n_parts, WHOLE_WAVES);
-      float* ws = P.floats((size_t)n * H * nz * (d + 2));
-      LAUNCH(P, "attention_decode_bf16 (last block merges)",
-             apc_attention_decode_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width,
-                                       s.positions, s.row_seg, rows, window, sc, kw, n_parts, ws,
-                                       P.pair_counters, P.stream));
-      return 1;
-    }
-    float* ws = P.floats((size_t)n * H * n_parts * (d + 2));
-    LAUNCH(P, "attention_decode_bf16",
+  if (even) {
+    float* ws = P.floats((size_t)apc_attention_decode_even_workspace(H, Hk, d));
+    LAUNCH(P, "attention_decode_bf16 (even shares)",
+           apc_attention_decode_even_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width, s.positions,
+                                          s.row_seg, rows, window, sc, ws, P.pair_counters, P.stream));
+  } else if (whole) {
+    // no length of the ranges: every row's own keys, one range a wave of its block
+    LAUNCH(P, "attention_decode_bf16 (whole)",
            apc_attention_decode_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width,
-                                     s.positions, s.row_seg, rows, window, sc, kw, n_parts, ws, nullptr,
+                                     s.positions, s.row_seg, rows, window, sc, 0, 0, nullptr, nullptr,
+                                     P.stream));
+  } else if (n) {
+    const int kw = 0;  // every row's own keys in n_parts ranges
+    float* ws = P.floats(last ? last_floats : (size_t)n * H * n_parts * (d + 2));
+    LAUNCH(P, last ? "attention_decode_bf16 (last block merges)" : "attention_decode_bf16",
+           apc_attention_decode_bf16(q.p, q.ld, 0, out.p, out.ld, n, H, Hk, d, E.kv, page, table, width,
+                                     s.positions, s.row_seg, rows, window, sc, kw, n_parts, ws, last ? P.pair_counters : nullptr,
                                      P.stream));
   }
   return 1;

@@ -96,6 +96,12 @@ int apc_attention_prefill_bf16(const void* q, int ldq, int q_off, void* out, int
                                const int* positions, const int* row_seg, const int* tile_row0, const int* tile_rows,
                                int n_tiles, int n_rows, int window, float scale, int n_splits, int part_rows,
                                float* parts, hipStream_t stream);
+int apc_attention_mixed_takes(int H, int Hk, int d, int page_tokens, int n_tiles, int n_rows, int n_decode, int n_parts, int last);
+int apc_attention_mixed_bf16(const void* q, int ldq, int q_off, void* out, int ldo, int H, int Hk, int d, const void* cache,
+                             int page_tokens, const int* block_table, int max_blocks, const int* positions, const int* row_seg,
+                             const int* tile_row0, const int* tile_rows, int n_tiles, int n_rows, int window, float scale, int n_splits,
+                             int part_rows, float* parts, const int* rows, int n_decode, int n_parts, float* workspace, int* counters,
+                             hipStream_t stream);
 int apc_attention_decode_bf16(const void* q, int ldq, int q_off, void* out, int ldo, int n_rows, int H, int Hk, int d,
                               const void* cache, int page_tokens, const int* block_table, int max_blocks,
                               const int* positions, const int* row_seg, const int* rows, int window, float scale,
