@@ -401,10 +401,15 @@ __global__ __launch_bounds__(WPB * 64, sk_waves(MG, MODE, NB, WPB, PRE)) void sk
 }
 
 // bands per block and waves per block: enough blocks and waves to keep HBM busy, never more waves than K
-// can feed with whole steps or LDS can hold
-static void pick_shape(int N, int K, bool swiglu, int* nb, int* wpb) {
+// can feed with whole steps or LDS can hold.  The waves, and with them the order of additions, do not depend on M.
+// Of many bands a block takes two, one set of activations for both.  A K of 4,096, 8,192, .. puts a wave's two streams a power of
+// two of 128 KiB and more apart, where they come at 6 TB/s instead of 7; one band a block then, while the activations are few.
+// 128,256 outputs, one band / two, us: K 4,096 with 1, 8, 16 rows 155, 158, 188 / 177, 178, 182, K 8,192 305, 310, 368 / 345, 346,
+// 354; 32,768 outputs, K 4,096, 8 rows 40 / 50; K 2,048, 8 rows 80 / 81, K 5,120 196 / 189, K 12,288 467 / 462.
+static void pick_shape(int M, int N, int K, bool swiglu, int* nb, int* wpb) {
   const int bands = ceil_div(N, 16), chunks = ceil_div(K, 32);
-  *nb = (!swiglu && bands >= 2048) ? 2 : 1;
+  const bool streams_collide = chunks >= 128 && (chunks & (chunks - 1)) == 0;
+  *nb = (!swiglu && bands >= 2048) && !(streams_collide && M <= 8) ? 2 : 1;
   const int blocks = ceil_div(bands, *nb);
   const int sets = swiglu ? 2 : *nb;
   int w = 4;
@@ -418,7 +423,7 @@ template <int MODE, bool PRE, bool EMIT>
 static int launch_skinny(const bf16_t* A, int lda, const bf16_t* W, const bf16_t* W2, void* C, int ldc, int M, int N,
                          int K, SkNorm norm, hipStream_t stream, SkRope rope = SkRope{}) {
   int nb, wpb;
-  pick_shape(MODE == SK_QKV_ROPE ? N / 2 : N, K, MODE == SK_SWIGLU || MODE == SK_QKV_ROPE, &nb, &wpb);
+  pick_shape(M, MODE == SK_QKV_ROPE ? N / 2 : N, K, MODE == SK_SWIGLU || MODE == SK_QKV_ROPE, &nb, &wpb);
   const int chunks = ceil_div(K, 32), bands = ceil_div(N, 16);
   if ((MODE == SK_SWIGLU || MODE == SK_QKV_ROPE) && wpb > 8) wpb = 8;
   if (PRE && norm.ld_ss > 4 * 4 * wpb * SS_LOADS) return APC_ERR_UNSUPPORTED;

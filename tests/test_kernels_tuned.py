@@ -157,6 +157,21 @@ def test_skinny_rows_together_equal_each_row_alone():
         assert torch.equal(some, tog[3:8])
 
 
+@pytest.mark.parametrize("N", [32768, 32780, 32784])
+def test_skinny_rows_over_many_columns_do_not_depend_on_the_bands_of_a_block(N):
+    """K of 4,096: up to 8 rows take a band of 16 outputs a block, more rows two (the last block's second one may be missing)."""
+    t = tuned()
+    a, w = gen(16, 4096, seed=1, dtype=BF).to(DEV), gen(N, 4096, seed=2, dtype=BF).to(DEV)
+    packed = pack(w)
+    outs = {}
+    for M in (1, 8, 9, 16):
+        outs[M] = torch.full((M, N), 7.0, device=DEV)
+        t.gemm_bf16(a[:M], packed, outs[M])
+    check(f64(outs[8]), f64(a[:8]) @ f64(w).T, torch.float32)
+    for M, out in outs.items():
+        assert torch.equal(out, outs[16][:M])
+
+
 def bf16_round(a):
     """float64 array rounded to bfloat16 (nearest even), as float64."""
     return f64(torch.from_numpy(np.asarray(a, np.float32)).to(BF))
