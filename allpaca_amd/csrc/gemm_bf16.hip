@@ -686,6 +686,8 @@ __global__ __launch_bounds__(256) void gemm_finish_qkv_rope_kernel(const float* 
 // How many slices of K the product of many rows (gemm_direct_bf16.hip) wants for this shape: 1, or 2 when narrow
 // tiles would be needed to fill the chip otherwise.  The caller brings the workspace for apc_gemm_splitk_bf16.
 APC_EXPORT int apc_gemm_direct_k_split(int M, int N, int K) { return gemm_direct_k_split(M, N, K); }
+// the same of apc_gemm_direct_emit_bf16
+APC_EXPORT int apc_gemm_direct_emit_k_split(int M, int N, int K) { return gemm_direct_emit_k_split(M, N, K); }
 
 // residual += A . W^T for more than 1,024 rows, leaving the row for the RMS norm (weight g) that reads the residual
 // next: raw [M][N] bfloat16 and ss [M][parts] (see gemm_direct.h).  apc_gemm_direct_emit_parts: the parts these sizes

@@ -30,7 +30,7 @@ int launch_gemm_direct_pre(int mode, const bf16_t* A, int lda, const float* ss, 
 // The product into the float32 residual C that also leaves the row for the RMS norm that reads the residual next:
 // raw [M][ldr] = bfloat16(C g) and ss [M][parts] = sums of C^2 over parts of the columns.  gemm_direct_emit_parts says
 // how many parts these sizes give (0: not taken; which depends on whether K goes in slices and on the tiles chosen);
-// workspace: room for gemm_direct_k_split(M, N, K) * M * N floats where that is more than 1.
+// workspace: room for gemm_direct_emit_k_split(M, N, K) * M * N floats where that is more than 1.
 int gemm_direct_emit_parts(const void* A, int lda, const void* C, int ldc, int M, int N, int K);
 int launch_gemm_direct_emit(const bf16_t* A, int lda, const bf16_t* W, float* C, int ldc, int M, int N, int K,
                             const float* g, bf16_t* raw, int ldr, float* ss, int ss_parts, float* workspace,
@@ -38,5 +38,6 @@ int launch_gemm_direct_emit(const bf16_t* A, int lda, const bf16_t* W, float* C,
 // Slices of K that a product of M rows into N columns should be cut into (1: none).  With more than one:
 // launch_gemm_direct_slices leaves float32 sums in partials[slice][M][N], K a multiple of k_split * 128.
 int gemm_direct_k_split(int M, int N, int K);
+int gemm_direct_emit_k_split(int M, int N, int K);   // of launch_gemm_direct_emit
 int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* partials, int M, int N, int K,
                               int k_split, hipStream_t stream);

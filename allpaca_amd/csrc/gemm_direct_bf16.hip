@@ -565,15 +565,24 @@ bool direct_takes(int mode, const void* A, int lda, const void* C, int ldc, int 
 // wide tiles (8 bands) a full round: down of an 8B model (K = 14,336) 276 -> 207 us plus the kernel that adds the
 // slices.  Time units as in pick_bands, per 4,096 columns of K; the adding kernel about 22 units per 2,048 x 4,096
 // outputs and slice pair, and a launch 3.
-int gemm_direct_k_split(int M, int N, int K) {
-  if (M < GEMM_DIRECT_MIN_ROWS || K % 256 || N % 4 || K < 4096) return 1;
+namespace {
+bool halves_pay(int M, int N, int K, int min_k, double add_units, double launch, double worth) {
+  if (M < GEMM_DIRECT_MIN_ROWS || K % 256 || N % 4 || K < min_k) return false;
   double whole = 0.0, halves = 0.0;
   pick_bands(M, N, false, 1, &whole);
   pick_bands(M, N, false, 2, &halves);
   const double k_units = K / 4096.0;
-  const double add = 22.0 * ((double)M * N / (2048.0 * 4096.0)) + 3.0;
-  return halves * k_units / 2 + add < 0.92 * whole * k_units ? 2 : 1;
+  const double add = add_units * ((double)M * N / (2048.0 * 4096.0)) + launch;
+  return halves * k_units / 2 + add < worth * whole * k_units;
 }
+}  // namespace
+int gemm_direct_k_split(int M, int N, int K) { return halves_pay(M, N, K, 4096, 22.0, 3.0, 0.92) ? 2 : 1; }
+// A product into the residual that leaves the next norm's row has an epilogue of some 4 us in one piece, which the adding kernel has
+// for nothing, so halves pay sooner.  us, K in one piece / two slices: 2,048 x 2,048 (K) 1,025 rows 32.9 / 25.1, 1,300 31.5 / 25.3,
+// 1,700 32.0 / 30.5, 2,048 32.8 / 34.5; 3,072 x 3,072 1,025 rows 40.9 / 36.0, 1,153 39.5 / 36.7, 1,300 39.9 / 41.7; 4,096 columns,
+// K 14,336, 1,500 rows 193 / 182.  Of 70 sizes (1,025 to 2,048 rows, 1,024 to 4,096 columns, K 2,048 to 14,336) what is chosen takes
+// 1.002 of the better one's time in the mean and 1.05 at worst (with the rule above 1.02 and 1.31).
+int gemm_direct_emit_k_split(int M, int N, int K) { return halves_pay(M, N, K, 2048, 18.0, 1.0, 0.93) ? 2 : 1; }
 
 int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* partials, int M, int N, int K,
                               int k_split, hipStream_t stream) {
@@ -714,7 +723,7 @@ int launch_gemm_direct_pre(int mode, const bf16_t* A, int lda, const float* ss, 
 
 int gemm_direct_emit_parts(const void* A, int lda, const void* C, int ldc, int M, int N, int K) {
   if (M < GEMM_DIRECT_MIN_ROWS || !direct_takes(D_ACC_EMIT, A, lda, C, ldc, M, N, K) || M > 65535) return 0;
-  if (gemm_direct_k_split(M, N, K) > 1) return ceil_div(N, 1024);
+  if (gemm_direct_emit_k_split(M, N, K) > 1) return ceil_div(N, 1024);
   return column_tiles(plan_columns(M, N, false), N, false);
 }
 
@@ -725,7 +734,7 @@ int launch_gemm_direct_emit(const bf16_t* A, int lda, const bf16_t* W, float* C,
   if (!parts || parts != ss_parts || !g || !raw || !ss || ldr < N || ldr % 4 || ((uintptr_t)raw & 7u) ||
       ((uintptr_t)g & 15u))
     return APC_ERR_UNSUPPORTED;
-  const int k_split = gemm_direct_k_split(M, N, K);
+  const int k_split = gemm_direct_emit_k_split(M, N, K);
   if (k_split > 1) {
     if (!workspace) return APC_ERR_BAD_ARG;
     const int e = launch_gemm_direct_slices(A, lda, W, workspace, M, N, K, k_split, stream);

@@ -181,7 +181,7 @@ int gemm_emit_bf16(Program& P, const Buf& a, const ApcMatrix& w, const Buf& resi
     emit.ss = (float*)P.emit_take(emit, sizeof(float) * (size_t)M * parts);
     emit.ss_rows = M;
     emit.ss_cols = parts;
-    const int ks = apc_gemm_direct_k_split(M, N, K);
+    const int ks = apc_gemm_direct_emit_k_split(M, N, K);
     float* ws = ks > 1 ? P.floats((size_t)ks * M * N) : nullptr;
     LAUNCH(P, "gemm_direct_emit_bf16",
            apc_gemm_direct_emit_bf16(a.p, a.ld, w.data, (float*)residual.p, residual.ld, M, N, K, emit.g, emit.raw.p, N,

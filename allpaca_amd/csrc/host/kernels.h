@@ -70,6 +70,7 @@ int apc_gemm_rows_emit_takes(const void* A, int lda, const void* W, const float*
 int apc_gemm_rows_emit_bf16(const void* A, int lda, const void* W, float* residual, int ldc, int M, int N, int K,
                             const float* g, void* raw, int ldr, float* ss, hipStream_t stream);
 int apc_gemm_direct_k_split(int M, int N, int K);
+int apc_gemm_direct_emit_k_split(int M, int N, int K);
 int apc_gemm_direct_emit_parts(const void* A, int lda, const void* residual, int ldc, int M, int N, int K);
 int apc_gemm_direct_emit_bf16(const void* A, int lda, const void* W, float* residual, int ldc, int M, int N, int K,
                               const float* g, void* raw, int ldr, float* ss, int parts, float* workspace,

@@ -242,7 +242,7 @@ def gemm_emit_bf16(a: torch.Tensor, w: PackedWeight, residual: torch.Tensor, g: 
             return None
         raw = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
         ss = torch.empty((M, parts), dtype=torch.float32, device=a.device)
-        ks = L.apc_gemm_direct_k_split(M, N, K)
+        ks = L.apc_gemm_direct_emit_k_split(M, N, K)
         ws = torch.empty(ks * M * N, dtype=torch.float32, device=a.device) if ks > 1 else None
         _lib.check(L.apc_gemm_direct_emit_bf16(a.data_ptr(), lda, w.data.data_ptr(), residual.data_ptr(), ldc, M, N, K,
                                                g.data_ptr(), raw.data_ptr(), N, ss.data_ptr(), parts,

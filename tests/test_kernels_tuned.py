@@ -359,6 +359,25 @@ def test_product_into_the_residual_leaves_the_next_norms_row_with_more_than_1024
     check(f64(out), P.silu(f64(raw) @ f64(w3[:F]).T * rstd) * (f64(raw) @ f64(w3[F:]).T * rstd), BF)
 
 
+@pytest.mark.parametrize("M,D,K,slices", [(1025, 2048, 2048, 2), (1153, 3072, 3072, 2), (1031, 1028, 2304, 2), (2048, 2048, 2048, 1),
+                                          (1025, 2048, 1792, 1)])
+def test_short_k_into_the_residual_in_one_piece_or_two(M, D, K, slices):
+    """K of 2,048 and more in two slices where that is expected to be faster; a last row tile of 1 and 7 rows."""
+    from allpaca_amd.kernels import lib
+    t = tuned()
+    assert lib.load("tuned").apc_gemm_direct_emit_k_split(M, D, K) == slices
+    assert lib.load("tuned").apc_gemm_direct_k_split(M, D, K) == 1
+    a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(D, K, seed=2, dtype=BF).to(DEV)
+    res, g = gen(M, D, seed=3, scale=2.0).to(DEV), (1 + 0.2 * gen(D, seed=4)).to(DEV)
+    x, raw_want, _ = emit_reference(a, w, f64(res), g)
+    raw, ss = t.gemm_emit_bf16(a, pack(w), res, g)
+    check(f64(res), x, torch.float32)
+    assert (ss.shape[1] == -(-D // 1024)) == (slices == 2)
+    assert np.allclose(f64(ss).sum(axis=1), (x ** 2).sum(axis=1), rtol=1e-5)
+    d = np.abs(f64(raw) - raw_want)
+    assert (d <= 2.0 ** -7 * np.abs(raw_want) + 1.5e-5 * np.abs(x).max()).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(40, 200, 1208), (64, 6144, 4096), (100, 96, 520), (128, 130, 2048),
                                    # K in one piece (enough tiles without slices): 224 and 192 tiles; a last row tile of 44
                                    (64, 28672, 520), (300, 8192, 264), (300, 2048, 1288),
