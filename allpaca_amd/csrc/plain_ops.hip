@@ -264,15 +264,19 @@ APC_EXPORT int apc_silu_mul(const void* gu, int in_dtype, int ldg, void* out, in
 //   values  cache[page][1][kv_head][i][slot]      (an element's slots lie together: the
 //           value product sums over positions, and matrix cores want that axis contiguous)
 // With cache == nullptr only the rotation is done (k in place as well).
+// TW threads a head, 256 / TW heads of a row a block: the work is a few trips, and a block a head spent longer on being dealt out
+// than on them.  325 rows of 48 heads of 64 in float32: 7.5 -> 6.5 us.
 // ---------------------------------------------------------------------------
-__global__ void rope_kv_write_kernel(void* __restrict__ qkv, int dtype, int ld, int q_off, int k_off, int v_off,
+template <int TW>
+__global__ __launch_bounds__(256) void rope_kv_write_kernel(void* __restrict__ qkv, int dtype, int ld, int q_off, int k_off, int v_off,
                                      int H, int Hk, int d, int rot, const float* __restrict__ cos_sin,
                                      const int* __restrict__ positions, const int* __restrict__ row_seg,
                                      const int* __restrict__ block_table, int max_blocks, void* __restrict__ cache,
                                      int cache_dtype, int P) {
   const int t = blockIdx.x;
-  const int slot_head = blockIdx.y;  // [0,H): q   [H,H+Hk): k   [H+Hk,H+2Hk): v
-  const int pos = positions[t];
+  const int slot_head = blockIdx.y * (256 / TW) + threadIdx.x / TW;  // [0,H): q   [H,H+Hk): k   [H+Hk,H+2Hk): v
+  if (slot_head >= H + 2 * Hk) return;
+  const int me = threadIdx.x % TW, pos = positions[t];
   const int half = rot / 2;
   size_t src;
   int kind, head;
@@ -288,12 +292,12 @@ __global__ void rope_kv_write_kernel(void* __restrict__ qkv, int dtype, int ld, 
   }
   if (kind == 2) {
     if (!cache) return;
-    for (int i = threadIdx.x; i < d; i += blockDim.x)
+    for (int i = me; i < d; i += TW)
       store_f(cache, cache_dtype, dst + (size_t)i * P, load_f(qkv, dtype, src + i));
     return;
   }
   const float* cs = cos_sin + (size_t)pos * rot;  // [2][half]
-  for (int i = threadIdx.x; i < half; i += blockDim.x) {
+  for (int i = me; i < half; i += TW) {
     const float a = load_f(qkv, dtype, src + i), b = load_f(qkv, dtype, src + i + half);
     const float c = cs[i], s = cs[half + i];
     const float ra = a * c - b * s, rb = a * s + b * c;
@@ -306,7 +310,7 @@ __global__ void rope_kv_write_kernel(void* __restrict__ qkv, int dtype, int ld, 
     }
   }
   if (kind == 1 && cache)  // the part of a head beyond the rotated width is copied
-    for (int i = rot + threadIdx.x; i < d; i += blockDim.x)
+    for (int i = rot + me; i < d; i += TW)
       store_f(cache, cache_dtype, dst + i, load_f(qkv, dtype, src + i));
 }
 
@@ -318,9 +322,12 @@ APC_EXPORT int apc_rope_kv_write(void* qkv, int dtype, int ld, int q_off, int k_
   if (H < 0 || Hk < 0 || d <= 0 || rot < 0 || rot > d || (rot & 1) || (rot > 0 && !cos_sin)) return APC_ERR_BAD_ARG;
   if (cache && (page_tokens <= 0 || !block_table || !row_seg || max_blocks <= 0)) return APC_ERR_BAD_ARG;
   if (H + 2 * Hk > 65535 || H + 2 * Hk == 0) return APC_ERR_BAD_ARG;
-  hipLaunchKernelGGL(rope_kv_write_kernel, dim3(n_tok, H + 2 * Hk), dim3(64), 0, stream, qkv, dtype, ld, q_off, k_off,
-                     v_off, H, Hk, d, rot, cos_sin, positions, row_seg, block_table, max_blocks, cache, cache_dtype,
-                     page_tokens);
+#define ROPE_KV(TW_)                                                                                                              \
+  hipLaunchKernelGGL(rope_kv_write_kernel<TW_>, dim3(n_tok, ceil_div(H + 2 * Hk, 256 / TW_)), dim3(256), 0, stream, qkv, dtype, ld, q_off, \
+                     k_off, v_off, H, Hk, d, rot, cos_sin, positions, row_seg, block_table, max_blocks, cache, cache_dtype, page_tokens)
+  if (d <= 64) ROPE_KV(32);
+  else ROPE_KV(64);
+#undef ROPE_KV
   APC_LAUNCH_CHECK();
   return 0;
 }
