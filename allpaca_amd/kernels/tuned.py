@@ -607,7 +607,8 @@ def attention_bf16(q: torch.Tensor, q_off: int, out: torch.Tensor, n_heads: int,
                    cache: torch.Tensor, page_tokens: int, block_table: torch.Tensor, step, window: int = 0,
                    scale: Optional[float] = None) -> bool:
     """Attention of a whole step: single-row segments on the split-key decode kernel, longer segments on the
-    tiled prefill kernel.  Returns False (nothing done) if the sizes are not ones these kernels take."""
+    tiled prefill kernel (the compiled executor runs both in one launch, `apc_attention_mixed_bf16`, where the sizes allow it: the
+    same bits).  Returns False (nothing done) if the sizes are not ones these kernels take."""
     _ops._gpu(q, out, cache, block_table)
     ldq, ldo = _ops._rows(q, "attention q"), _ops._rows(out, "attention out")
     T = q.shape[0]
