@@ -9,6 +9,7 @@ per-user folder under the system's temporary directory).  A library is rebuilt
 when the text of its sources or the flags change."""
 from __future__ import annotations
 
+import glob
 import hashlib
 import os
 import shutil
@@ -32,8 +33,6 @@ LIBS: Dict[str, List[str]] = {
     "bench": ["probe.hip"],
     "host": ["host/exec.cpp", "host/cache.cpp", "host/pack.cpp", "host/sched.cpp"],
 }
-HEADERS = ["common.h", "mfma.h", "gemm_wide.h", "gemm_direct.h", "gemm_rows.h", "attention_wide.h", "no_alloc.h",
-           "host/host.h", "host/kernels.h", "host/rules.h", "host/cache.h"]
 # libraries a library is linked against (built first; found at run time beside it)
 NEEDS: Dict[str, List[str]] = {"host": ["plain", "tuned"]}
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wno-unused-value", "-Wno-unused-result"]
@@ -105,7 +104,8 @@ def source_hash(name: str) -> str:
     h.update(" ".join(sorted(ACC_REGISTER_SOURCES)).encode())
     for dep in NEEDS.get(name, []):
         h.update(source_hash(dep).encode())
-    for path in _sources(name) + [os.path.join(CSRC, f) for f in HEADERS]:
+    # every header, whichever sources include it: one that is left out here leaves the built library in use after an edit
+    for path in _sources(name) + sorted(glob.glob(os.path.join(CSRC, "**", "*.h"), recursive=True)):
         if os.path.isfile(path):
             h.update(os.path.basename(path).encode())
             with open(path, "rb") as f:

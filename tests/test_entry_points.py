@@ -3,6 +3,7 @@ that is passed as an int would lose its upper half."""
 import glob
 import os
 import re
+import shutil
 
 import pytest
 
@@ -36,3 +37,28 @@ def test_argument_types_are_those_of_the_sources(library):
     for name, args in lib.SIGNATURES[library].items():
         assert name in SOURCES, name
         assert args == SOURCES[name], (name, [a.__name__ for a in args], [a.__name__ for a in SOURCES[name]])
+
+
+def test_a_library_is_built_again_after_an_edit_of_any_file_that_its_sources_include(tmp_path, monkeypatch):
+    root = str(tmp_path / "csrc")
+    shutil.copytree(build.CSRC, root)
+    monkeypatch.setattr(build, "CSRC", root)
+
+    def reached(path, seen):
+        with open(path) as f:
+            for name in re.findall(r'^#include "([^"]+)"', f.read(), re.M):
+                at = next(p for p in (os.path.join(os.path.dirname(path), name), os.path.join(root, name)) if os.path.isfile(p))
+                if at not in seen:
+                    seen.add(at)
+                    reached(at, seen)
+        return seen
+
+    for library, sources in build.LIBS.items():
+        files = {os.path.join(root, s) for s in sources}
+        for s in list(files):
+            reached(s, files)
+        for path in sorted(files):
+            before = build.source_hash(library)
+            with open(path, "a") as f:
+                f.write("// edited\n")
+            assert build.source_hash(library) != before, (library, os.path.relpath(path, root))
