@@ -1075,14 +1075,16 @@ struct alignas(8) FewShared {
 
 // The largest threshold c (a sort key with zeros below some digit) at which at least k and at most `most` >= k of the
 // values stand at or above it; `each(f)` calls f(sort key) for the values of the block's NT threads.  Fewer than k values:
-// 0.  With most == k the answer is exact: sort keys are all different.
-template <int NT, typename Each>
-__device__ __forceinline__ u64 few_threshold(FewShared& sh, uint32_t k, uint32_t most, int key_bits, Each&& each) {
+// 0.  With most == k the answer is exact: sort keys are all different.  A caller that knows k values whose bits from `hi` (32 or
+// more) on are `prefix`, and none above them, says so.  ALIKE: a wave's values are often of one bin (in order, or equal), where an
+// add a lane takes its turn (90,000 of them some 90 us): the lanes of the first one's bin add as one.
+template <int NT, bool ALIKE = false, typename Each>
+__device__ __forceinline__ u64 few_threshold(FewShared& sh, uint32_t k, uint32_t most, int key_bits, Each&& each, u64 prefix = 0,
+                                             int hi = 64) {
   constexpr int PER = FEW_BINS / NT;
-  u64 prefix = 0;
   uint32_t above = 0;                                   // values above the prefix's range
-  for (int hi = 64;;) {
-    const int lo = hi - FEW_BITS;                       // (ends at 9 or before: an id has at most 22 bits, see apc_sample_rows)
+  for (;;) {
+    const int lo = hi - FEW_BITS;                       // (0 or more: an id has at most 22 bits, see apc_sample_rows)
     __syncthreads();
 #pragma unroll
     for (int g = 0; g < PER; ++g) sh.hist[threadIdx.x + g * NT] = 0;
@@ -1090,7 +1092,17 @@ __device__ __forceinline__ u64 few_threshold(FewShared& sh, uint32_t k, uint32_t
     __syncthreads();
     each([&](u64 c) {
       if (hi < 64 && (c >> hi) != (prefix >> hi)) return;
-      atomicAdd(&sh.hist[(uint32_t)(c >> lo) & (FEW_BINS - 1)], 1u);
+      const uint32_t bin = (uint32_t)(c >> lo) & (FEW_BINS - 1);
+      uint32_t n = 1;
+      if constexpr (ALIKE) {
+        const uint32_t first = __builtin_amdgcn_readfirstlane(bin);
+        const u64 same = __ballot(bin == first);
+        if (bin == first) {
+          if ((int)(threadIdx.x % WAVE) != __ffsll(same) - 1) return;
+          n = (uint32_t)__popcll(same);
+        }
+      }
+      atomicAdd(&sh.hist[bin], n);
     });
     __syncthreads();
     // threads in descending order of the bins
@@ -1388,11 +1400,16 @@ __global__ __launch_bounds__(SNT) void sample_few_end_kernel(const float* __rest
 // wave's largest value; the second finds the bound among at most BOUND_SET of them (waves, or four waves together), reads again
 // the few groups that reach it (for k of 40 some 45 of 512, of 256 values each) and puts what it finds in order by counting who
 // stands above whom.  A row whose large values lie close together (all in one group, or all equal) has more than HEAD_HELD
-// there: their threshold is found by the radix descent, over those groups.
+// there: of all waves by their largest value (of equal ones the earlier pieces') only those that fewer than k others come in front
+// of can hold one of the k largest, some k of them, and the radix descent over these stops at a few values more than k.
 // What bounds it is latency: the first launch is one pass where the pair above makes three, the second has some 45 groups' values to
-// look at instead of 1,300 to 5,000 candidates.  8 rows of 128,256 logits, top-k 40, top-p 0.95: 9.9 + 15.0 -> 4.5 + 12.5 us (with
-// 256 threads in the second 17.9), from the call to the ids 47.5 -> 39.7.  The host has to know the rows' top-k, and a large
-// one (above 85, or fewer with many rows) keeps the pair above.
+// look at instead of 1,300 to 5,000 candidates, and divides only those by the temperature that may stand at the bound.  Both launches,
+// rows of 128,256 random logits, top-p 0.95, pair above / this one, us: 8 rows top-k 8 19.4 / 14.1, 40 25.2 / 16.2, 85 30.2 / 22.5; 64
+// rows 38.6 / 17.6, 44.6 / 23.1, 54.0 / 33.2; from the call to the ids, 8 rows of top-k 40, 47.5 / 39.7 (without the divisions that are
+// spared).  8 rows of equal values, top-k 40, 43.9 / 40.3 (476 with a descent over all of the row); where the large values are some
+// thousand neighbours, which logits are not, the pair above stays ahead: in descending order 28.2 / 31.7, top-k 85 32.2 / 42.4.
+// The host has to know the rows' top-k, and one of more than two thirds of the set keeps the pair above: 85 of 128 fours of waves (up to
+// 16 rows of 128,256), 170 of 256 waves (17 to 32 rows of 65,536, 32 of 128,256).
 constexpr int BOUND_SET = 256, HEAD_HELD = 512, HEAD_WAVES = PNT / WAVE;
 struct HeadSpace {
   float* piece_best;       // [row][pieces] ...
@@ -1453,6 +1470,14 @@ __host__ __device__ int bound_set(const SampleShape& sz) {
 }
 bool head_takes(const SampleShape& sz, int most) { return most * 3 <= bound_set(sz) * 2; }
 
+// A value below this one, divided by t, has a key below `key` (rounded either way; spares the division for most values).
+__device__ __forceinline__ float floor_of(uint32_t key, float t) {
+  constexpr float MOST = 3.402823466e+38f;
+  if (key < key_of(-MOST)) return -INFINITY;
+  const float v = fminf(fminf(value_of(key), MOST) * t, MOST);
+  return v - fabsf(v) * 1e-6f - 1e-37f;
+}
+
 struct HeadEnd {
   FewShared select;
   SampleShared one;
@@ -1460,12 +1485,11 @@ struct HeadEnd {
   u64 held[HEAD_HELD];
   int group[MAX_PIECES * HEAD_WAVES];
   int groups;
-  uint32_t least;
+  uint32_t least, most;
   float sums[HEAD_HELD];                 // running sums of the weights
 };
 
-template <typename Options>
-__global__ __launch_bounds__(PNT) void sample_head_end_kernel(const float* __restrict__ logits, SampleShape sz, Options opt, HeadSpace sp,
+__global__ __launch_bounds__(PNT) void sample_head_end_kernel(const float* __restrict__ logits, SampleShape sz, RowValues opt, HeadSpace sp,
                                                               int* __restrict__ out, int* __restrict__ out_host) {
   __shared__ HeadEnd sh;
   const int row = blockIdx.x, tk = opt.top_k[row];
@@ -1537,12 +1561,16 @@ __global__ __launch_bounds__(PNT) void sample_head_end_kernel(const float* __res
     __syncthreads();
   }
   const uint32_t least = max(sh.least, 1u);
-  if (scaled(mine) >= least) sh.group[atomicAdd(&sh.groups, 1)] = threadIdx.x;
+  const int listed = scaled(mine) >= least ? atomicAdd(&sh.groups, 1) : -1;
+  if (listed >= 0) sh.group[listed] = threadIdx.x;
   __syncthreads();
-  // f(sort key) for every finite value of these groups: a wave takes four rounds of a group at a time
-  const int per = sz.vec ? 4 * PNT : PNT, rounds = ceil_div(sz.chunk, per), items = sh.groups * rounds;
+  // f(sort key) for the finite values of these groups that may stand at the bound: a wave takes four rounds of a group at a time
+  const int per = sz.vec ? 4 * PNT : PNT, rounds = ceil_div(sz.chunk, per);
+  int items = sh.groups * rounds;
+  float floor = floor_of(least, t);
   auto each = [&](auto f) {
     for (int q = wave * 4; q < items; q += PNT / WAVE * 4) {
+      if (*(volatile uint32_t*)&sh.select.count > (uint32_t)HEAD_HELD) break;   // (more than there is room for: see below)
       float x[4][4];
       int at[4], end[4];
 #pragma unroll
@@ -1569,7 +1597,7 @@ __global__ __launch_bounds__(PNT) void sample_head_end_kernel(const float* __res
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (finite_f(x[u][e])) f(sort_key(key_of(x[u][e] / t), at[u] + e, sz.id_bits, 0));
+          if (x[u][e] >= floor && finite_f(x[u][e])) f(sort_key(key_of(x[u][e] / t), at[u] + e, sz.id_bits, 0));
     }
   };
   auto gather = [&](u64 from) {
@@ -1582,10 +1610,35 @@ __global__ __launch_bounds__(PNT) void sample_head_end_kernel(const float* __res
   };
   gather((u64)least << 32);
   if (sh.select.count > (uint32_t)HEAD_HELD) {          // (the same for all threads)
-    const u64 from = few_threshold<PNT>(sh.select, keep, keep, 32 + sz.id_bits, each);
+    // The waves that fewer than `keep` others come in front of; another one's values stand behind `keep` others.
+    u64* order = reinterpret_cast<u64*>(sh.select.hist);
+    static_assert(MAX_PIECES * HEAD_WAVES * sizeof(u64) <= sizeof(sh.select.hist), "room for all waves");
+    const u64 me = (u64)scaled(mine) << 32 | (MAX_PIECES - threadIdx.x / HEAD_WAVES);
+    const int n_listed = sh.groups;
+    if (listed >= 0) order[listed] = me;
     __syncthreads();
-    if (threadIdx.x == 0) sh.select.count = 0;
+    if (threadIdx.x == 0) sh.groups = 0, sh.select.count = 0, sh.least = 0xffffffffu, sh.most = 0;
+    uint32_t front = 0;
+    if (listed >= 0) {
+#pragma unroll 8
+      for (int q = 0; q < n_listed; ++q) front += order[q] > me;
+    }
     __syncthreads();
+    if (listed >= 0 && front < keep) {
+      sh.group[atomicAdd(&sh.groups, 1)] = threadIdx.x;
+      atomicMin(&sh.least, (uint32_t)(me >> 32));
+      atomicMax(&sh.most, (uint32_t)(me >> 32));
+    }
+    __syncthreads();
+    items = sh.groups * rounds;
+    // Where there are `keep` such waves, `keep` values stand between the least and the largest of their keys: the bits that these two
+    // have in common need no pass.
+    const uint32_t low = sh.groups >= (int)keep ? sh.least : 1u;
+    const int hi = low == sh.most ? 32 : 64 - __clz((int)(low ^ sh.most));
+    const u64 prefix = hi < 64 ? (u64)sh.most << 32 >> hi << hi : 0;
+    floor = floor_of(low, t);
+    const u64 from = few_threshold<PNT, true>(sh.select, keep, keep + FEW_SPARE, 32 + sz.id_bits, each, prefix, hi);
+    floor = floor_of((uint32_t)(from >> 32), t);
     gather(from);
   }
   const int found = (int)sh.select.count;
@@ -1620,21 +1673,21 @@ SampleShape shape_of(const float* logits, int ldl, int n_rows, int V) {
   return sz;
 }
 
-// `most`: the largest top-k of the rows that sample, where the host knows it (else 0)
 template <typename Options>
-int launch_few(const float* logits, const SampleShape& sz, const Options& opt, void* scratch, int* out, int* out_host, int most,
-               hipStream_t stream) {
+int launch_few(const float* logits, const SampleShape& sz, const Options& opt, void* scratch, int* out, int* out_host, hipStream_t stream) {
   const FewSpace fs = carve_few(scratch, sz.R);
-  if (most > 0 && head_takes(sz, most)) {
-    hipLaunchKernelGGL(sample_head_pieces_kernel, dim3(sz.pieces, sz.R), dim3(PNT), 0, stream, logits, sz, head_space(fs));
-    APC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sample_head_end_kernel<Options>, dim3(sz.R), dim3(PNT), 0, stream, logits, sz, opt, head_space(fs), out, out_host);
-    APC_LAUNCH_CHECK();
-    return 0;
-  }
   hipLaunchKernelGGL(sample_few_pieces_kernel<Options>, dim3(sz.pieces, sz.R), dim3(PNT), 0, stream, logits, sz, opt, fs);
   APC_LAUNCH_CHECK();
   hipLaunchKernelGGL(sample_few_end_kernel<Options>, dim3(sz.R), dim3(SNT), 0, stream, logits, sz, opt, fs, out, out_host);
+  APC_LAUNCH_CHECK();
+  return 0;
+}
+
+int launch_head(const float* logits, const SampleShape& sz, const RowValues& opt, void* scratch, int* out, int* out_host, hipStream_t stream) {
+  const HeadSpace sp = head_space(carve_few(scratch, sz.R));
+  hipLaunchKernelGGL(sample_head_pieces_kernel, dim3(sz.pieces, sz.R), dim3(PNT), 0, stream, logits, sz, sp);
+  APC_LAUNCH_CHECK();
+  hipLaunchKernelGGL(sample_head_end_kernel, dim3(sz.R), dim3(PNT), 0, stream, logits, sz, opt, sp, out, out_host);
   APC_LAUNCH_CHECK();
   return 0;
 }
@@ -1728,8 +1781,14 @@ APC_EXPORT int apc_sample_rows(const float* logits, int ldl, int n_rows, int V, 
   if (!few)
     if (const int rc = allow_pass_lds(dev)) return rc;
   const SampleShape sz = shape_of(logits, ldl, n_rows, V);
-  if (few) return launch_few(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, scratch, out, nullptr, 0, stream);
+  if (few) return launch_few(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, scratch, out, nullptr, stream);
   return launch_descents(logits, sz, RowOptions{temperature, top_p, uniform, top_k}, nullptr, scratch, out, nullptr, cuts, stream);
+}
+
+// 1 if the entry point below bounds the rows' values by the largest ones of groups (sample_head_end_kernel) where no row that samples
+// has a larger top-k than `most`, all of them between 1 and 1,024.
+APC_EXPORT int apc_sample_rows_bounded(int n_rows, int V, int most) {
+  return n_rows > 0 && n_rows <= BY_VALUE && V > 0 && V <= (1 << 22) && most > 0 && head_takes(shape_of(nullptr, V, n_rows, V), most) ? 1 : 0;
 }
 
 // The same for up to 64 rows with their options on the host: they go with the first launch, and the ids also to `out_host` (host
@@ -1765,7 +1824,8 @@ APC_EXPORT int apc_sample_rows_host(const float* logits, int ldl, int n_rows, in
     int most = 0;                                        // (greedy rows may ask for any)
     for (int r = 0; r < n_rows; ++r)
       if (opt.temperature[r] > 1e-5f) most = std::max(most, opt.top_k[r]);
-    return launch_few(logits, sz, opt, scratch, out, out_host, most, stream);
+    return most > 0 && head_takes(sz, most) ? launch_head(logits, sz, opt, scratch, out, out_host, stream)
+                                            : launch_few(logits, sz, opt, scratch, out, out_host, stream);
   }
   if (const int rc = allow_pass_lds(dev)) return rc;
   return launch_descents(logits, sz, RowOptions{}, &opt, scratch, out, out_host, cuts, stream);

@@ -188,3 +188,55 @@ def test_groups_of_unlike_and_of_like_values(V):
             assert got == want, (top_k, top_p)
     got, want = with_the_launch(logits, [0.7, 0.0, 1e-6] * 4 + [1.5], [40, 7, 0] * 4 + [3], [0.9, 1.0, 0.5] * 4 + [0.4])
     assert got == want
+
+
+@pytest.mark.parametrize("V,R,most", [(12289, 3, 42), (32001, 8, 85), (65536, 1, 170), (128256, 16, 85), (128255, 8, 85), (60001, 64, 85), (128256, 32, 170), (128256, 24, 58)])
+def test_top_k_up_to_which_rows_are_bounded_by_groups(V, R, most):
+    """Which pair of launches a call takes, and the same tokens at the largest top-k of either."""
+    from allpaca_amd.kernels import lib
+    L = lib.load("plain")
+    assert L.apc_sample_rows_bounded(R, V, most) == 1 and L.apc_sample_rows_bounded(R, V, most + 1) == 0
+    assert L.apc_sample_rows_bounded(R, V, 0) == 0 and L.apc_sample_rows_bounded(65, V, 1) == 0
+    logits = torch.randn(R, V, generator=torch.Generator(device=DEV).manual_seed(R), device=DEV) * 3
+    logits[0] = logits[0].sort(descending=True).values       # large values side by side: more than the block holds
+    logits[R // 2, :900] += 25.0
+    logits[-1] = logits[-1].round() / 2
+    for top_k in (most // 2, most, most + 1):
+        got, want = with_the_launch(logits, 0.8, top_k, 0.95)
+        assert got == want, top_k
+
+
+@pytest.mark.parametrize("temperature", [1.1e-5, 0.5, 3.0, 1e4])
+def test_bounds_at_the_ends_of_float32(temperature):
+    """Quotients that overflow (all infinite, told apart by their ids), that vanish, and values next to the bound."""
+    rng = np.random.default_rng(7)
+    V = 40000
+    near = np.float32(2.0) + np.float32(2.0 ** -22) * rng.integers(0, 40, size=V).astype(np.float32)      # neighbours that a division may round together
+    rows = [rng.normal(size=V) * 1e38, rng.normal(size=V) * 1e34, -np.abs(rng.normal(size=V)) * 3e38, rng.normal(size=V) * 1e-44, rng.normal(size=V) * 1e-36, near, -near,
+            np.where(rng.random(V) < 0.01, 3.4028e38, rng.normal(size=V))]
+    logits = torch.tensor(np.clip(np.stack(rows), -3.4028234e38, 3.4028234e38), dtype=torch.float32, device=DEV)
+    for top_k in (1, 40, 85):
+        got, want = with_the_launch(logits, temperature, top_k, 0.9)
+        assert got == want, top_k
+
+
+def test_rows_of_equal_values_take_no_multiple_of_random_ones():
+    """A row with more values at the bound than a block holds: some 2.5 times as long as random logits, and not 30."""
+    from allpaca_amd.kernels import ops
+    out = torch.zeros(8, dtype=torch.int32, device=DEV)
+
+    def us(logits):
+        least = 1e9
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                ops.sample_rows(logits, [0.8] * 8, [40] * 8, [0.95] * 8, (list(range(8)), [0] * 8), out, few_after_top_k=True)
+            b.record()
+            b.synchronize()
+            least = min(least, a.elapsed_time(b) * 100.0)
+        return least
+
+    random = us(torch.randn(8, 128256, device=DEV) * 3)
+    for like in (torch.zeros(8, 128256, device=DEV), torch.full((8, 128256), -1.7, device=DEV)):
+        assert us(like) < 8 * random
