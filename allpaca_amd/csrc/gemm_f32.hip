@@ -491,13 +491,11 @@ struct RopeF32 {
 };
 
 // The product of up to 8 rows.  The same slices, the same sums to the bit as gemm_f32_kernel's; what differs is what a stage brings:
-// 8 rows of A, not 16 of which half are repeats, and 8 or 16 rows of W, so that 2,048 outputs have a block for every compute unit;
+// 8 rows of A, not 16 of which half are repeats, and 8 rows of W (16 with ROPE), so that 2,048 outputs have a block for every unit;
 // two stages are on their way in a loop whose last round asks again for the last stage instead of code for every remainder, and a
 // stage's operands come out of LDS under the products of the one before.  A residual is asked for ahead of the first weights.
 // What bounds it is a unit's eight waves' way from loads to products (as many stages as registers hold are no faster: 4 rows x
-// 2,048 outputs x K 2,048 7.6 us with two, 7.9 with four, 8.7 with eight).  gemm_f32_kernel / this one, us, launches of a graph one
-// behind the other over 67 to 840 MB of weights: 4 rows x 2,048 outputs x K 2,048 8.4 / 7.6, K 8,192 23.3 / 20.5, 1,024 x 4,096
-// 11.2 / 10.0, 576 x 576 5.8 / 5.2; bands of 16: 3,072 x 2,048 8.7 / 8.3, 4,096 x 4,096 15.1 / 14.0.
+// 2,048 outputs x K 2,048 7.6 us with two, 7.9 with four, 8.7 with eight).  apc_gemm_f32_few says where it is taken, with both sides' times.
 template <int BAND, int D, bool NORM, bool ROPE>
 __global__ __launch_bounds__(64 * SLICES, 4) void gemm_f32_few_kernel(const float* __restrict__ A, int lda, const float* __restrict__ G,
                                                                       float eps, const float* __restrict__ W, int ldw, void* __restrict__ C,
@@ -770,20 +768,23 @@ static int tiles_a_block(const TileCost& t, bool glu, int M, int N, int K) {
 }
 APC_EXPORT int apc_gemm_f32_tiles_a_block(int M, int N, int K) { return tiles_a_block(TILES[tile_of(M, N, K)], false, M, N, K); }
 
+// Whether a product without a norm goes to gemm_f32_few_kernel: up to 8 rows, one round of blocks of 8 outputs, and a short K only
+// where the sums are added to what is there, which is then asked for early.  Launches of a graph over 0.5 GB of weights, tiles / blocks
+// of 8 outputs, us, 4 rows (1 and 8 rows within 5 % of it), stored: 2,048 outputs x K 2,048 6.6 / 6.4, K 8,192 19.7 / 18.3, 1,024 x
+// 4,096 9.6 / 9.0, but 2,048 x 256 3.4 / 3.6, x 1,024 4.7 / 4.9; added: 2,048 x 256 3.8 / 3.8, x 2,048 7.1 / 6.7, x 8,192 20.3 / 18.5, 1,024
+// x 4,096 10.1 / 9.1, 576 x 576 4.7 / 4.3.  Beyond 2,048 outputs blocks of 16 lost, stored: 3,072 x 2,048 7.0 / 7.4, 4,096 x 1,028 6.5 /
+// 7.6, 4,096 x 4,096 13.1 / 13.5 (added: 13.4 / 13.5).
+APC_EXPORT int apc_gemm_f32_few(int M, int N, int K, int mode) {
+  return M > 0 && M <= 8 && N > 0 && N <= 2048 && K > (mode == 1 ? 4 * STAGE : 1024) ? 1 : 0;
+}
+
 // Few rows: two stages of loads ahead, not four.  4 rows x 2,048 outputs x K 2,048 7.2 -> 6.7 us, K 8,192 21.6 -> 19.3 (128,256
 // outputs, K 2,048: 150 and 151): the straight code of a stage count's every case is a third as long, and a launch finds it cold.
 static int product(const float* A, int lda, const float* G, float eps, const float* R, const float* W, int ldw, void* C,
                    int c_dtype, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
-  // Up to 8 rows (see gemm_f32_few_kernel): one round of blocks of 8 outputs, or of 16 with a K that pays.  4 rows, us, tiles / blocks of 8
-  // / of 16: 2,048 outputs at K = 576 5.9 / 5.5 / 5.7; 3,072 at K = 1,024 6.8 / 7.4 / 6.9, K = 4,096 13.3 / 16.0 / 12.1; 6,144 at
-  // K = 1,024 9.5 / 10.1 / 10.3, 8,192 47.5 / 47.4 / 51.2.
-  if (M <= 8 && !G && !R && K > 4 * STAGE && N <= 4096 && (N <= 2048 || K > 1024)) {
-#define FEW(BAND_)                                                                                                             \
-  hipLaunchKernelGGL((gemm_f32_few_kernel<BAND_, 2, false, false>), dim3(ceil_div(N, BAND_)), dim3(64 * SLICES), 0, stream, A, lda, \
-                     nullptr, 0.f, W, ldw, C, c_dtype, ldc, M, N, K, mode, RopeF32{})
-    if (N <= 2048) FEW(8);
-    else FEW(16);
-#undef FEW
+  if (!G && !R && apc_gemm_f32_few(M, N, K, mode)) {
+    hipLaunchKernelGGL((gemm_f32_few_kernel<8, 2, false, false>), dim3(ceil_div(N, 8)), dim3(64 * SLICES), 0, stream, A, lda, nullptr, 0.f,
+                       W, ldw, C, c_dtype, ldc, M, N, K, mode, RopeF32{});
     APC_LAUNCH_CHECK();
     return 0;
   }

@@ -34,6 +34,7 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
         "apc_cast": [P, I, P, I, Z, P],
         "apc_gemm_plain": [P, I, I, P, I, I, P, I, I, I, I, I, I, P],
         "apc_gemm_f32_tile": [I, I, I],
+        "apc_gemm_f32_few": [I, I, I, I],
         "apc_swiglu_f32_tile": [I, I, I],
         "apc_gemm_f32_tiles_a_block": [I, I, I],
         "apc_swiglu_f32_tiles_a_block": [I, I, I],
@@ -195,7 +196,7 @@ _timer = None
 NOT_KERNELS = {"apc_delta_rule_bf16_takes", "apc_delta_rule_fact_size", "apc_delta_rule_coef_size",
                "apc_gated_recurrence_bf16_takes", "apc_recurrent_step_bf16_takes", "apc_delta_step_takes", "apc_latent_attention_takes", "apc_latent_rows_bf16_takes", "apc_selective_scan_bf16_takes", "apc_attention_masked_takes", "apc_rotary_pages_bf16_takes", "apc_routed_bf16_takes", "apc_routed_max_tiles", "apc_linear_attention_bf16_takes", "apc_conv_heads_bf16_takes", "apc_attention_decode_whole_fits", "apc_attention_decode_last_fits", "apc_attention_decode_even_workspace", "apc_attention_decode_even_region", "apc_attention_prefill_tile_rows",
                "apc_attention_prefill_wide_takes", "apc_attention_mixed_takes",
-               "apc_gemm_direct_k_split", "apc_gemm_direct_emit_k_split", "apc_gemm_rows_takes", "apc_gemm_rows_qkv_takes", "apc_gemm_direct_qkv_takes", "apc_gemm_rows_emit_takes", "apc_gemm_direct_emit_parts", "apc_sample_rows_scratch_kib", "apc_sample_rows_bounded", "apc_swiglu_f32_takes", "apc_gemm_f32_tile",
+               "apc_gemm_direct_k_split", "apc_gemm_direct_emit_k_split", "apc_gemm_rows_takes", "apc_gemm_rows_qkv_takes", "apc_gemm_direct_qkv_takes", "apc_gemm_rows_emit_takes", "apc_gemm_direct_emit_parts", "apc_sample_rows_scratch_kib", "apc_sample_rows_bounded", "apc_swiglu_f32_takes", "apc_gemm_f32_tile", "apc_gemm_f32_few",
                "apc_swiglu_f32_tile", "apc_gemm_f32_tiles_a_block", "apc_swiglu_f32_tiles_a_block", "apc_gemm_norm_f32_takes", "apc_qkv_rope_f32_takes", "apc_swiglu_norm_f32_takes", "apc_gemm_norm_f32_kib"}
 
 

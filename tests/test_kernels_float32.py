@@ -244,10 +244,10 @@ def test_rows_behind_a_norm_in_every_form(M, N, K):
         assert torch.equal(alone[0], out[r])
 
 
-# blocks of 8 outputs (up to 2,048) and of 16, last blocks that are not full; slices with no, one and several stages, a last stage cut by
-# K; outputs whose rows do not allow 16-byte stores
+# blocks of 8 outputs (up to 2,048) and tiles beyond, last blocks that are not full; slices with no, one and several stages, a last stage cut
+# by K; outputs whose rows do not allow 16-byte stores
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,K", [(8, 132), (40, 14340), (515, 256), (2048, 2048), (2047, 388), (2049, 1028), (4090, 2052), (4096, 1056)])
+@pytest.mark.parametrize("N,K", [(8, 132), (40, 14340), (515, 256), (2048, 2048), (2047, 388), (2049, 1028), (4090, 2052), (4096, 1056), (1001, 132), (2040, 1024)])
 def test_up_to_8_rows_are_the_bits_of_more(N, K):
     o = ops()
     a, w = gen(12, K, seed=1), gen(N, K, seed=2)
@@ -261,6 +261,14 @@ def test_up_to_8_rows_are_the_bits_of_more(N, K):
             assert torch.equal(out[:, :N], many[:M]) and (out[:, N:] == 7.0).all()
             o.gemm_plain(a[:M], w, out[:, :N], accumulate=True)
             assert torch.equal(out[:, :N], many[:M] + many[:M]) and (out[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,N,K,stored,added", [(1, 2048, 1028, 1, 1), (8, 2048, 2048, 1, 1), (8, 8, 14336, 1, 1), (4, 2048, 1024, 0, 1), (4, 576, 132, 0, 1),
+                                                (4, 576, 128, 0, 0), (9, 2048, 2048, 0, 0), (4, 2049, 2048, 0, 0), (4, 4096, 4096, 0, 0)])
+def test_products_that_the_kernel_of_up_to_8_rows_takes(M, N, K, stored, added):
+    from allpaca_amd.kernels import lib
+    few = lib.load("plain").apc_gemm_f32_few
+    assert (few(M, N, K, 0), few(M, N, K, 1)) == (stored, added)
 
 
 @pytest.mark.gpu
