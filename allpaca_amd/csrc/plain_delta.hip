@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void delta_rule_kernel(
 // that use it, four waves each: it owns those channels of the convolutions' state, which it moves on.  The operations are those of
 // conv_channels_kernel, delta_rule_kernel and gated_groupnorm_f4_kernel, in their order: the same bits.  What bounds it is
 // latency, the trips to a request's slot, its inputs and its matrix; the matrix is asked for at the start.  8 rows, 32 heads of 64
-// over 16, four taps, inside a step: 5.3 + 6.7 + 3.9 -> 9.1 us.
+// over 16, four taps, inside a step: 4.6 + 6.4 + 3.4 -> 9.1 us (apc_delta_step_takes has other sizes).
 // ---------------------------------------------------------------------------
 struct DeltaStep {
   const void* x;                   // [rows][ldx]: q, k and v in front of the convolutions, logits of a and b, the gate
@@ -333,12 +333,14 @@ APC_EXPORT int apc_delta_rule(const void* rows, int dtype, int ld, int q_off, in
   return 0;
 }
 
-// Whether apc_delta_step takes these sizes (of q/k heads with up to 4 value heads; heads of up to 64 values, a multiple of 4).
-APC_EXPORT int apc_delta_step_takes(int H, int G, int dk, int dv, int taps, const void* state) {
-  return H > 0 && G > 0 && H % G == 0 && H / G <= STEP_HEADS && G <= 65535 && dk > 0 && dk <= 128 && dv > 0 && dv <= 64 && dv % 4 == 0 &&
-                 taps > 0 && taps <= STEP_TAPS && ((uintptr_t)state & 15u) == 0
-             ? 1
-             : 0;
+// Whether apc_delta_step takes these sizes (of q/k heads with up to 4 value heads; heads of up to 64 values, a multiple of 4), and so many
+// rows: what it saves is two launches and the trips between them, and once the chip is full a block of up to 16 waves that meet three
+// times is slower than the three kernels' small ones.  Three launches / one, us, bfloat16 rows, four taps: 32 heads of 64 over 16, 1 row
+// 13.6 / 9.1, 8 13.7 / 9.4, 32 20.7 / 15.7, 64 28.1 / 26.9, 128 50.6 / 53.5, 256 85.6 / 94.2; over 8, 32 rows 20.6 / 16.2, 64 27.6 / 28.7,
+// 256 84.6 / 109; 48 heads over 16, 16 rows 18.7 / 13.8, 64 41.5 / 48.2; 64 heads over 16, keys of 128, 16 rows 26.4 / 20.7, 64 80.6 / 87.2.
+APC_EXPORT int apc_delta_step_takes(int H, int G, int dk, int dv, int taps, const void* state, int n_rows) {
+  if (H <= 0 || G <= 0 || H % G || H / G > STEP_HEADS || G > 65535 || dk <= 0 || dk > 128 || dv <= 0 || dv > 64 || dv % 4) return 0;
+  return taps > 0 && taps <= STEP_TAPS && ((uintptr_t)state & 15u) == 0 && (long)n_rows * H <= (H / G <= 2 ? 2048 : 1024) ? 1 : 0;
 }
 
 // One row of every request (see DeltaStep): row r is of segment row_seg[r], whose slots are conv_slots[.] and slots[.]; no two
@@ -348,7 +350,7 @@ APC_EXPORT int apc_delta_step(const void* x, int dtype, int ldx, int q_off, int 
                               float q_scale, float* state, const float* norm_w, float eps, int n_rows, const int* row_seg,
                               const int* conv_slots, const int* slots, void* out, int ldo, hipStream_t stream) {
   if (n_rows <= 0) return 0;
-  if (!apc_delta_step_takes(H, G, dk, dv, taps, state)) return APC_ERR_UNSUPPORTED;
+  if (!apc_delta_step_takes(H, G, dk, dv, taps, state, n_rows)) return APC_ERR_UNSUPPORTED;
   if (!x || !conv_w || (taps > 1 && (!conv_state || !conv_slots)) || !A || !dt_bias || !state || !norm_w || !row_seg || !slots || !out ||
       ldo < H * dv || ldx < v_off + H * dv || ldx < q_off + G * dk || ldx < k_off + G * dk || ldx < a_off + H || ldx < b_off + H ||
       ldx < g_off + H * dv || (dtype != APC_BF16 && dtype != APC_F32))

@@ -76,7 +76,7 @@ SIGNATURES: Dict[str, Dict[str, list]] = {
         "apc_weighted_pair": [P, I, P, I, F, P, I, F, I, I, P],
         "apc_routed_down": [P, I, P, I, I, I, I, P, P, I, P, I, I, P, I, I, I, P],
         "apc_delta_rule": [P, I, I, I, I, I, I, I, I, I, P, I, I, I, I, P, P, F, P, I, P, P, P, P, I, P],
-        "apc_delta_step_takes": [I, I, I, I, I, P],
+        "apc_delta_step_takes": [I, I, I, I, I, P, I],
         "apc_delta_step": [P, I, I, I, I, I, I, I, I, I, I, I, I, P, I, P, P, P, F, P, P, F, I, P, P, P, P, I, P],
         "apc_gated_recurrence": [P, I, I, P, I, P, I, P, P, I, I, P, F, P, I, I, P, P, P, P, I, I, P],
         "apc_argmax_rows": [P, I, I, I, P, P, P],

@@ -1299,13 +1299,13 @@ def delta_step(x: torch.Tensor, q_off: int, k_off: int, v_off: int, n_heads: int
                norm_w: torch.Tensor, eps: float, step, out: torch.Tensor) -> bool:
     """For a step of single rows, in one launch: `conv_channels` (silu) of x's columns up to v_off + heads * value_dim, `delta_rule` of what
     that gives with the logits at a_off and b_off, and `gated_rmsnorm` of a head's output (group value_dim, the gate at g_off through
-    silu) into `out`, x's type.  False (nothing done) for sizes that it does not take."""
+    silu) into `out`, x's type.  False (nothing done) for sizes that it does not take, or rows so many that the three are faster."""
     H, G, dk, dv = int(n_heads), int(n_kv_heads), int(key_dim), int(value_dim)
     T, taps = x.shape[0], int(conv_w.shape[1])
     L = _lib.load("plain")
     if (not getattr(step, "decode_only", False) or step.n_segs != T or x.dtype not in (torch.float32, torch.bfloat16) or out.dtype != x.dtype
             or (taps > 1 and (conv_state is None or conv_slots is None))
-            or not L.apc_delta_step_takes(H, G, dk, dv, taps, state.data_ptr())):
+            or not L.apc_delta_step_takes(H, G, dk, dv, taps, state.data_ptr(), T)):
         return False
     _gpu(x, conv_w, conv_state, conv_slots, A, dt_bias, state, slots, norm_w, out)
     ldx, ldo, C = _rows(x, "rows"), _rows(out, "delta step out"), v_off + H * dv

@@ -320,3 +320,11 @@ def test_the_expected_times_of_a_size_are_worked_out_once(monkeypatch):
     want = tuned._tiled_k_split(517, 4100, 4224)
     monkeypatch.setattr(tuned, "_direct_slices_us", lambda *a: pytest.fail("worked out again"))
     assert tuned._tiled_k_split(517, 4100, 4224) == want
+
+
+@pytest.mark.parametrize("H,G,dk,dv,rows", [(32, 16, 64, 64, 64), (32, 32, 64, 64, 64), (32, 8, 64, 64, 32), (48, 16, 64, 64, 21), (64, 16, 128, 64, 16), (4, 1, 64, 64, 256)])
+def test_single_rows_of_the_delta_rule_in_one_launch_while_the_chip_is_not_full(H, G, dk, dv, rows):
+    from allpaca_amd.kernels import lib
+    takes = lib.load("plain").apc_delta_step_takes
+    assert takes(H, G, dk, dv, 4, 0, 1) and takes(H, G, dk, dv, 4, 0, rows) and not takes(H, G, dk, dv, 4, 0, rows + 1)
+    assert not takes(H, G, dk, dv, 9, 0, 1) and not takes(H, G, dk, dv, 4, 8, 1) and not takes(5 * G, G, dk, dv, 4, 0, 1) and not takes(H, G, dk, 68, 4, 0, 1)
