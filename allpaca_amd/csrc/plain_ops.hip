@@ -264,17 +264,19 @@ APC_EXPORT int apc_silu_mul(const void* gu, int in_dtype, int ldg, void* out, in
 //   values  cache[page][1][kv_head][i][slot]      (an element's slots lie together: the
 //           value product sums over positions, and matrix cores want that axis contiguous)
 // With cache == nullptr only the rotation is done (k in place as well).
-// TW threads a head, 256 / TW heads of a row a block: the work is a few trips, and a block a head spent longer on being dealt out
-// than on them.  325 rows of 48 heads of 64 in float32: 7.5 -> 6.5 us.
+// TW threads a head, HEADS heads of a row a block.  The work is a few trips, and with many rows a block a head spends longer on being
+// dealt out than on them; with few, a block's own start counts.  Rows x heads: a head / several heads a block, us, float32, 48 heads of 64:
+// 1 row 2.52 / 2.65, 8 2.71 / 2.92, 32 3.08 / 3.04, 325 7.5 / 5.6, 2,048 29 / 18; 40 heads of 128: 8 rows 2.89 / 2.98, 64 3.68 / 3.62, 325 8.6 /
+// 8.0; 6 heads of 16: 100 rows 2.75 / 2.94, 325 3.03 / 3.02.
 // ---------------------------------------------------------------------------
-template <int TW>
-__global__ __launch_bounds__(256) void rope_kv_write_kernel(void* __restrict__ qkv, int dtype, int ld, int q_off, int k_off, int v_off,
+template <int TW, int HEADS>
+__global__ __launch_bounds__(TW * HEADS) void rope_kv_write_kernel(void* __restrict__ qkv, int dtype, int ld, int q_off, int k_off, int v_off,
                                      int H, int Hk, int d, int rot, const float* __restrict__ cos_sin,
                                      const int* __restrict__ positions, const int* __restrict__ row_seg,
                                      const int* __restrict__ block_table, int max_blocks, void* __restrict__ cache,
                                      int cache_dtype, int P) {
   const int t = blockIdx.x;
-  const int slot_head = blockIdx.y * (256 / TW) + threadIdx.x / TW;  // [0,H): q   [H,H+Hk): k   [H+Hk,H+2Hk): v
+  const int slot_head = blockIdx.y * HEADS + threadIdx.x / TW;  // [0,H): q   [H,H+Hk): k   [H+Hk,H+2Hk): v
   if (slot_head >= H + 2 * Hk) return;
   const int me = threadIdx.x % TW, pos = positions[t];
   const int half = rot / 2;
@@ -322,11 +324,12 @@ APC_EXPORT int apc_rope_kv_write(void* qkv, int dtype, int ld, int q_off, int k_
   if (H < 0 || Hk < 0 || d <= 0 || rot < 0 || rot > d || (rot & 1) || (rot > 0 && !cos_sin)) return APC_ERR_BAD_ARG;
   if (cache && (page_tokens <= 0 || !block_table || !row_seg || max_blocks <= 0)) return APC_ERR_BAD_ARG;
   if (H + 2 * Hk > 65535 || H + 2 * Hk == 0) return APC_ERR_BAD_ARG;
-#define ROPE_KV(TW_)                                                                                                              \
-  hipLaunchKernelGGL(rope_kv_write_kernel<TW_>, dim3(n_tok, ceil_div(H + 2 * Hk, 256 / TW_)), dim3(256), 0, stream, qkv, dtype, ld, q_off, \
-                     k_off, v_off, H, Hk, d, rot, cos_sin, positions, row_seg, block_table, max_blocks, cache, cache_dtype, page_tokens)
-  if (d <= 64) ROPE_KV(32);
-  else ROPE_KV(64);
+#define ROPE_KV(TW_, HEADS_)                                                                                                          \
+  hipLaunchKernelGGL((rope_kv_write_kernel<TW_, HEADS_>), dim3(n_tok, ceil_div(H + 2 * Hk, HEADS_)), dim3(TW_ * HEADS_), 0, stream, qkv, dtype, \
+                     ld, q_off, k_off, v_off, H, Hk, d, rot, cos_sin, positions, row_seg, block_table, max_blocks, cache, cache_dtype, page_tokens)
+  if ((long)n_tok * (H + 2 * Hk) < 2048) ROPE_KV(64, 1);
+  else if (d <= 64) ROPE_KV(32, 8);
+  else ROPE_KV(64, 4);
 #undef ROPE_KV
   APC_LAUNCH_CHECK();
   return 0;

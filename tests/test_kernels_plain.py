@@ -457,3 +457,30 @@ def test_sample_rows_frequencies():
     p /= p.sum()
     chi2 = ((counts - n * p) ** 2 / (n * p)).sum()
     assert chi2 < 31.26  # 11 degrees of freedom, p = 0.001
+
+
+# heads of up to 64 (eight a block) and above (four), last blocks of a row that are not full; 2,048 (row, head) pairs and the next
+@pytest.mark.parametrize("H,Hk,d,rot,rows", [(6, 1, 16, 16, 256), (5, 2, 48, 16, 300), (9, 3, 64, 64, 137), (3, 1, 80, 40, 410), (6, 2, 128, 128, 300)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rope_kv_write_of_many_rows_is_that_of_few(H, Hk, d, rot, rows, dtype):
+    from allpaca_amd.kernels import lib
+    o, P_ = ops(), 8
+    width, pages = (H + 2 * Hk) * d, -(-rows // P_)
+    table = gen(rows, 2, rot // 2, seed=1).to(DEV)
+    x = gen(rows, width + 4, seed=2, dtype=dtype).to(DEV)
+    pos = torch.randperm(rows, generator=torch.Generator().manual_seed(3)).to(torch.int32).to(DEV)
+    seg, bt = torch.zeros(rows, dtype=torch.int32, device=DEV), torch.randperm(pages, generator=torch.Generator().manual_seed(4)).to(torch.int32)[None].to(DEV)
+    code, L = 1 if dtype == torch.bfloat16 else 0, lib.load("plain")
+
+    def run(chunk, paged):
+        y, cache = x.clone(), torch.zeros(pages, 2, Hk, P_, d, dtype=dtype, device=DEV)
+        for r in range(0, rows, chunk):
+            n = min(chunk, rows - r)
+            lib.check(L.apc_rope_kv_write(y[r:].data_ptr(), code, y.stride(0), 0, H * d, (H + Hk) * d, n, H, Hk, d, rot, table.data_ptr(), pos[r:].data_ptr(),
+                                          seg[r:].data_ptr(), bt.data_ptr(), pages, cache.data_ptr() if paged else 0, code, P_, o._stream()), "rope")
+        return y, cache
+
+    assert rows * (H + 2 * Hk) >= 2048 > 100 * (H + 2 * Hk)
+    for paged in (True, False):
+        for got, want in zip(run(rows, paged), run(100, paged)):
+            assert torch.equal(got, want)
