@@ -786,9 +786,10 @@ int launch_qkv(const bf16_t* A, int lda, const bf16_t* W, bf16_t* q_out, int ldq
 }  // namespace
 
 // Whether the next entry point takes these sizes and is expected to be faster than the product and the kernel that rotates and
-// fills the pages, one after the other: the tiles that it does not have (3 and 5 bands a wave, columns in two launches) against
-// that kernel's time (us, 7 and 0.42 a million outputs: 12.1, 10.2 and 9.4 measured for 2,048 x 6,144, 1,153 x 5,120 and 1,500 x
-// 3,072) less 1.5 for what the epilogue costs.
+// fills the pages, one after the other: that kernel less what the epilogue costs, 0.9 us a million outputs, against the tiles that this
+// product does not have (3 and 5 bands a wave, columns in two launches; 0.73 us a time unit of pick_bands).  Fitted to 361 sizes (24
+// pairs of heads and widths, 129 to 4,096 rows): what is chosen takes 0.941 of the time of one after the other in the mean and 1.015 at worst
+// (the better of the two 0.941, always together 0.952 and 1.11: 1,153 rows into 1,280 outputs, K 2,048 25.9 / 28.5 us).
 APC_EXPORT int apc_gemm_direct_qkv_takes(const void* A, int lda, const void* q_out, int ldq, int M, int K, int H, int Hk, int d,
                                          const void* cos_sin, const void* cache) {
   if (M <= 0 || H <= 0 || Hk <= 0 || (d != 64 && d != 128) || lda < K || ldq < H * d) return 0;
@@ -798,8 +799,7 @@ APC_EXPORT int apc_gemm_direct_qkv_takes(const void* A, int lda, const void* q_o
   if (((uintptr_t)cos_sin & 15u) || ((uintptr_t)cache & 7u)) return 0;
   double fused = 0.0;
   qkv_bands(M, N, &fused);
-  const double units = K / 4096.0, apart = plan_columns(M, N, false).cost * units + 7.0 + 0.42e-6 * M * N;
-  return fused * units + 1.5 < apart ? 1 : 0;
+  return 0.73 * (fused - plan_columns(M, N, false).cost) * (K / 4096.0) < 0.9e-6 * M * N ? 1 : 0;
 }
 
 // q, k and v of M rows in one product, q and k rotated, k and v written into the paged cache (see DirectRope).  W: tiled layout of

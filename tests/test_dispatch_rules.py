@@ -328,3 +328,13 @@ def test_single_rows_of_the_delta_rule_in_one_launch_while_the_chip_is_not_full(
     takes = lib.load("plain").apc_delta_step_takes
     assert takes(H, G, dk, dv, 4, 0, 1) and takes(H, G, dk, dv, 4, 0, rows) and not takes(H, G, dk, dv, 4, 0, rows + 1)
     assert not takes(H, G, dk, dv, 9, 0, 1) and not takes(H, G, dk, dv, 4, 8, 1) and not takes(5 * G, G, dk, dv, 4, 0, 1) and not takes(H, G, dk, 68, 4, 0, 1)
+
+
+@pytest.mark.parametrize("M,H,Hk,d,K,together", [
+    (2048, 32, 8, 128, 4096, 1), (1153, 24, 8, 128, 3072, 1), (1500, 32, 8, 64, 2048, 1), (2048, 16, 8, 128, 1024, 1), (1024, 4, 2, 64, 128, 1),
+    # few columns in one round of blocks: tiles of 3 bands a wave, which the product that rotates does not have, end sooner
+    (1025, 8, 1, 128, 2048, 0), (2048, 16, 2, 64, 2048, 0), (1300, 8, 2, 128, 2048, 0), (1025, 16, 2, 128, 2048, 0), (1025, 14, 2, 64, 896, 0),
+    (64, 32, 8, 128, 4096, 0), (2048, 32, 8, 96, 4096, 0), (2048, 32, 8, 128, 4100, 0)])
+def test_q_k_v_of_many_rows_rotated_by_the_product_where_that_is_faster(M, H, Hk, d, K, together):
+    from allpaca_amd.kernels import lib
+    assert lib.load("tuned").apc_gemm_direct_qkv_takes(0, K, 0, (H + 2 * Hk) * d, M, K, H, Hk, d, 0, 0) == together
