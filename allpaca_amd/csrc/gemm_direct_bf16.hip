@@ -578,11 +578,16 @@ bool halves_pay(int M, int N, int K, int min_k, double add_units, double launch,
 }  // namespace
 int gemm_direct_k_split(int M, int N, int K) { return halves_pay(M, N, K, 4096, 22.0, 3.0, 0.92) ? 2 : 1; }
 // A product into the residual that leaves the next norm's row has an epilogue of some 4 us in one piece, which the adding kernel has
-// for nothing, so halves pay sooner.  us, K in one piece / two slices: 2,048 x 2,048 (K) 1,025 rows 32.9 / 25.1, 1,300 31.5 / 25.3,
-// 1,700 32.0 / 30.5, 2,048 32.8 / 34.5; 3,072 x 3,072 1,025 rows 40.9 / 36.0, 1,153 39.5 / 36.7, 1,300 39.9 / 41.7; 4,096 columns,
-// K 14,336, 1,500 rows 193 / 182.  Of 70 sizes (1,025 to 2,048 rows, 1,024 to 4,096 columns, K 2,048 to 14,336) what is chosen takes
-// 1.002 of the better one's time in the mean and 1.05 at worst (with the rule above 1.02 and 1.31).
-int gemm_direct_emit_k_split(int M, int N, int K) { return halves_pay(M, N, K, 2048, 18.0, 1.0, 0.93) ? 2 : 1; }
+// for nothing, so halves pay sooner, and from K = 2,048 on; between 4,096 and 12,288 by less than the units say (the product of a short K
+// is mostly epilogue, that of a long one has no part of it to lose).  us, K in one piece / two slices: 2,048 x 2,048 (K) 1,025 rows 32.9 / 25.1,
+// 1,300 31.5 / 25.3, 1,700 32.0 / 30.5, 2,048 32.8 / 34.5; 3,072 x 3,072 1,025 rows 40.9 / 36.0, 1,153 39.5 / 36.7, 1,300 39.9 / 41.7; 4,096 x
+// 4,096 1,025 rows 48.5 / 49.7; 4,096 columns, K 8,192, 1,153 rows 88.1 / 91.9, K 14,336, 1,500 rows 193 / 182.  Against the rule above, over
+// 310 sizes (1,025 to 4,096 rows, 1,024 to 8,192 columns, K 2,048 to 14,336) where the two could differ, what is chosen takes 0.863 of the
+// time in the mean and 1.013 at worst (the better of the two 0.859).
+int gemm_direct_emit_k_split(int M, int N, int K) {
+  const double worth = K >= 4096 && K < 12288 ? 0.86 : 0.93;
+  return gemm_direct_k_split(M, N, K) > 1 || halves_pay(M, N, K, 2048, 18.0, 1.0, worth) ? 2 : 1;
+}
 
 int launch_gemm_direct_slices(const bf16_t* A, int lda, const bf16_t* W, float* partials, int M, int N, int K,
                               int k_split, hipStream_t stream) {

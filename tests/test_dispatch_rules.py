@@ -338,3 +338,17 @@ def test_single_rows_of_the_delta_rule_in_one_launch_while_the_chip_is_not_full(
 def test_q_k_v_of_many_rows_rotated_by_the_product_where_that_is_faster(M, H, Hk, d, K, together):
     from allpaca_amd.kernels import lib
     assert lib.load("tuned").apc_gemm_direct_qkv_takes(0, K, 0, (H + 2 * Hk) * d, M, K, H, Hk, d, 0, 0) == together
+
+
+@pytest.mark.parametrize("M,N,K,slices", [
+    # a short K, columns so few that tiles of 3 bands would be needed to fill the chip
+    (1025, 2048, 2048, 2), (1153, 3072, 3072, 2), (1300, 1024, 2048, 2),
+    # a longer K: the slices' way through memory (48.5 / 49.7, 88 / 92, 139 / 146, 87 / 90, 51 / 54 us)
+    (1025, 4096, 4096, 1), (1153, 4096, 8192, 1), (1153, 5120, 11008, 1), (2400, 2048, 8192, 1), (3000, 1536, 4096, 1), (2048, 2048, 2048, 1),
+    # what products that leave no row take in slices
+    (1153, 3072, 8192, 2), (1025, 1024, 4096, 2), (2048, 2048, 8192, 2), (1023, 2048, 8192, 1), (1025, 2048, 2200, 1),
+    (1500, 4096, 14336, 2)])
+def test_slices_of_k_of_products_into_the_residual_of_more_than_1024_rows(M, N, K, slices):
+    from allpaca_amd.kernels import lib
+    L = lib.load("tuned")
+    assert L.apc_gemm_direct_emit_k_split(M, N, K) == slices >= L.apc_gemm_direct_k_split(M, N, K)
