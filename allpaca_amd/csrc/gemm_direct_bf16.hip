@@ -508,22 +508,22 @@ int pick_bands(int M, int N, bool swiglu, int k_split = 1, double* cost_out = nu
 
 // Row tiles that a launch puts in one group (see direct_tile).  The blocks of an XCD, up to 32 at a time, read every panel of A
 // (128 rows) and of W (`tile_rows_of_w` rows) that they share out of memory once; those bytes are fewest when the rows and
-// the columns of what runs together are about as many.  Groups of one size, the larger one where two are alike.  2,048 rows, groups
-// of 16 / of 8, us: 4,096 outputs, K 4,096 59.9 / 58.0, K 14,336 199 / 188, 6,144 outputs 81.3 / 79.5, SwiGLU of 12,288 outputs
-// 295 / 289; the order of the groups this gives is that of the times for 1,153 and 1,500 rows too (1,153 rows x 8,192 SwiGLU
-// outputs: 10 row tiles in one group 105.4, in two 106.1).
+// the columns of what runs together are about as many.  Groups of one size, the larger one where two are alike; of more than 16 row tiles
+// groups of 8, which divide the 32, where no other size saves more than 6 % (8,192 rows x 14,336 SwiGLU outputs, K 4,096, groups of 16 / 11 /
+// 8: 1,375 / 1,411 / 1,369 us).  2,048 rows, groups of 16 / of 8, us: 4,096 outputs, K 4,096 59.9 / 58.0, K 14,336 199 / 188, 6,144 outputs
+// 81.3 / 79.5, SwiGLU of 12,288 outputs 295 / 289.  Over 12 products each at 1,025 to 2,048 rows, 2,049 to 4,096 and 5,000 to 16,384 the time
+// is 0.991, 0.987 and 0.986 of that with groups of 16 in the mean and 1.009, 1.016 and 1.011 at worst.
 int rows_together(int M, int N, int nb, int tile_rows_of_w) {
   const int mt = ceil_div(M, 128);
   const int here = std::min(32, ceil_div(mt * ceil_div(N, nb), 8));   // tiles that run on an XCD at one time
+  const auto rows_read = [&](int r) { return std::min(r, here) * 128L + (long)ceil_div(here, r) * tile_rows_of_w; };
   int best = mt;
-  long best_rows = 0;
-  for (int groups = 1; groups <= mt && groups <= 64; ++groups) {
+  for (int groups = 2; groups <= mt && groups <= 64; ++groups) {
     const int r = ceil_div(mt, groups);
-    const long rows = std::min(r, here) * 128L + (long)ceil_div(here, r) * tile_rows_of_w;
-    if (!best_rows || rows < best_rows) best = r, best_rows = rows;
+    if (rows_read(r) < rows_read(best)) best = r;
     if (r == 1) break;
   }
-  return best;
+  return mt > 16 && rows_read(8) * 100 <= rows_read(best) * 106 ? 8 : best;
 }
 
 template <int NF, int MODE>

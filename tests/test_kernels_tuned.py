@@ -83,9 +83,9 @@ def test_gemm_bf16(M, N, K):
     check(f64(acc) - before, want, torch.float32)
 
 
-# row tiles of 128 in groups: 13 in 7 and 6, 12 in 6 and 6, 24 in three of 8, 27 in 7, 7, 7 and 6, 9 in 5 and 4, 17 in one with
-# more than a round of blocks an XCD
-@pytest.mark.parametrize("M,N", [(1560, 4096), (1500, 2048), (2950, 2052), (3330, 1028), (1030, 4096), (2060, 12292)])
+# row tiles of 128 in groups: 13 in 7 and 6, 12 in 6 and 6, 24 in three of 8, 27 in three of 8 and one of 3, 9 in 5 and 4, 17 in two of 8 and
+# one of 1, with more than a round of blocks an XCD; 33 and 65 with one row tile behind groups of 8
+@pytest.mark.parametrize("M,N", [(1560, 4096), (1500, 2048), (2950, 2052), (3330, 1028), (1030, 4096), (2060, 12292), (4100, 2048), (8200, 1540)])
 def test_gemm_bf16_of_row_tiles_in_groups(M, N):
     t = tuned()
     a, w = gen(M, 128, seed=4, dtype=BF).to(DEV), gen(N, 128, seed=5, dtype=BF).to(DEV)
