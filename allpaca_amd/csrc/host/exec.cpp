@@ -473,7 +473,8 @@ int attention_bf16(Program& P, const Buf& q, const Buf& out, const ApcLayer& L, 
                                         std::max(1, P.tun.key_range_min));
     float* parts = splits > 1 ? P.floats((size_t)splits * T * H * (d + 2)) : nullptr;
     // (rows dealt out evenly fill the chip by themselves)
-    if (wide && (whole || last) && apc_attention_mixed_takes(H, Hk, d, page, s.n_tiles, T - n, n, n_parts, last)) {
+    if (wide && (whole || last) && decode_beside_tiles((long)s.n_tiles * H * splits, d, pairs, last) &&
+        apc_attention_mixed_takes(H, Hk, d, page, s.n_tiles, T - n, n, n_parts, last)) {
       float* ws = last ? P.floats(last_floats) : nullptr;
       LAUNCH(P, "attention_mixed_bf16",
              apc_attention_mixed_bf16(q.p, q.ld, 0, out.p, out.ld, H, Hk, d, E.kv, page, table, width, s.positions, s.row_seg, s.tile_row0,
@@ -798,6 +799,9 @@ APC_HOST_EXPORT int apc_host_rule_even_pays(long long steps, int longest, int n_
 }
 APC_HOST_EXPORT int apc_host_rule_decode_even(long long pairs, int span, int pair_fits, int min_pairs, int min_span) {
   return apc_rules::decode_even((long)pairs, span, pair_fits != 0, min_pairs, min_span);
+}
+APC_HOST_EXPORT int apc_host_rule_decode_beside_tiles(long long tile_blocks, int d, long long pairs, int last) {
+  return apc_rules::decode_beside_tiles((long)tile_blocks, d, (long)pairs, last != 0);
 }
 APC_HOST_EXPORT int apc_host_rule_key_splits(int n_tiles, int n_heads, int keys, int window, int splits_max,
                                              int range_min) {

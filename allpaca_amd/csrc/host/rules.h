@@ -164,6 +164,19 @@ inline bool even_pays(long long steps, int longest, int n_rows, int tiles, int w
   return 7.3 + std::max(share, 8.3) + 0.05 * (n_rows / 64.0) < whole;
 }
 
+// Whether a step's decoded rows go into the launch of its tiles of prompt rows (attn_prefill_wide_kernel), behind them.  There a
+// decode block has a unit of its own where two share one in a launch of their own (heads of 128; two and four with heads of 64), which
+// matters once they are many, and where the tiles fill whole rounds a round of them only waits.  tile_blocks: the tiles' blocks; pairs:
+// (row, kv head) pairs with a block each, or `last`: blocks for ranges of their keys, a round of the chip at most.  One layer, two launches /
+// one, us, 32 heads over 8 of 128: 504 rows behind 1,544 beside 32 rows of 1,000 keys 63 / 41, 128 of 1,000 125 / 107, 256 of 100 68 / 60;
+// 1,024 rows (a whole round) beside 8 of 2,000 (last) 45 / 42, 32 of 2,000 72 / 75, 64 112 / 117, 256 of 100 55 / 65; 70 rows beside 64 of 1,000
+// 59 / 53, 256 of 100 40 / 44.  Over 1,976 steps (70 to 1,900 prompt rows beside 1 to 256, five pairs of heads) what is chosen takes 0.797 of
+// the two launches' time in the mean and 1.008 at worst (always one 0.792 and 1.17, the better of the two 0.791).
+inline bool decode_beside_tiles(long tile_blocks, int d, long pairs, bool last) {
+  const long round = CHIP_UNITS * (d <= 64 ? 2 : 1), free = (round - tile_blocks % round) % round;
+  return last || pairs < CHIP_UNITS || (pairs <= 1024 && free * 16 > round);
+}
+
 // ranges of keys that the 128-row attention kernel cuts every tile of a step into; `keys`: of the longest prompt
 inline int key_splits(int n_tiles, int n_heads, int keys, int window, int splits_max, int range_min) {
   const long blocks = (long)n_tiles * n_heads;

@@ -81,6 +81,7 @@ _lib.SIGNATURES["host"].update({
     "apc_host_rule_decode_parts": [c_longlong, I],
     "apc_host_rule_even_pays": [c_longlong, I, I, I, I],
     "apc_host_rule_decode_even": [c_longlong, I, I, I, I],
+    "apc_host_rule_decode_beside_tiles": [c_longlong, I, c_longlong, I],
     "apc_host_rule_key_splits": [I, I, I, I, I, I],
     "apc_host_rule_key_splits_by_time": [I, I, I, I, c_longlong, I, I],
     # ---- the cache manager's books

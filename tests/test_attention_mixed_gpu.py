@@ -71,3 +71,53 @@ def test_sizes_that_take_two_launches():
     assert not L.apc_attention_mixed_takes(32, 8, 128, 16, 4, 255, 8, 16, 1)        # tiles mostly empty
     assert not L.apc_attention_mixed_takes(32, 8, 128, 16, 0, 0, 8, 16, 1)          # no prompt
     assert not L.apc_attention_mixed_takes(32, 8, 128, 16, 4, 504, 0, 16, 1)        # nothing decoded
+
+
+# rows of the prompt's portion, decoded rows and their contexts; heads and their size, window; which launches the executor issues
+@pytest.mark.parametrize("portion,contexts,H,Hk,d,window,launches", [
+    (200, [300, 20, 700], 8, 2, 128, None, ["attention_mixed_bf16"]),                        # ranges of keys, the last block adds
+    (200, [300, 20, 700], 8, 2, 64, None, ["attention_mixed_bf16"]),
+    (130, [33, 100, 250], 8, 2, 64, None, ["attention_mixed_bf16"]),                          # a block a pair
+    (65, [500, 90], 8, 4, 128, 100, ["attention_mixed_bf16"]),                                # a window
+    (300, [500, 90, 610], 16, 2, 64, 70, ["attention_mixed_bf16"]),
+    (40, [300, 700], 8, 2, 128, None, ["attention_prefill_bf16", "attention_decode_bf16 (last block merges)"]),   # no tile half full
+    (1024, [40 + i for i in range(33)], 32, 8, 128, None, ["attention_prefill_bf16", "attention_decode_bf16 (whole)"]),   # whole rounds of tiles
+    (800, [40 + i for i in range(33)], 32, 8, 128, None, ["attention_mixed_bf16"]),
+])
+def test_the_executor_gives_the_python_walks_bits_and_issues_the_launches(monkeypatch, portion, contexts, H, Hk, d, window, launches):
+    from allpaca_amd.engine.batch import Entry
+    from allpaca_amd.engine.runner import ModelRunner
+    from allpaca_amd.models import DecoderModel, describe_model
+    from allpaca_amd.parts import Runtime
+    import helpers
+    cfg = dict(helpers.TINY_B, hidden_size=256, num_attention_heads=H, num_key_value_heads=Hk, head_dim=d, intermediate_size=512, num_hidden_layers=2,
+               vocab_size=500, max_position_embeddings=4096, rope_scaling=None)
+    rng = np.random.default_rng(portion)
+    toks = [rng.integers(0, 500, size=n).tolist() for n in [portion + 77] + contexts]
+    got = []
+    for python_walk in (True, False):
+        if python_walk:
+            monkeypatch.setenv("ALLPACA_AMD_PYTHON_WALK", "1")
+        else:
+            monkeypatch.delenv("ALLPACA_AMD_PYTHON_WALK", raising=False)
+        _, _, spec = describe_model(cfg)
+        if window:
+            for block in spec.blocks:
+                block.parts["mixer"].params["window"] = window
+        model = DecoderModel(spec)
+        g = torch.Generator(device=DEV).manual_seed(1)
+        tensors = {name: torch.randn(ps.shape, generator=g, device=DEV, dtype=BF).mul_(0.1) for name, ps in model.param_specs().items()}
+        model.bind(tensors, Runtime(torch.device(DEV), BF, 4096))
+        runner = ModelRunner(model, 16, 64 + sum(-(-len(t) // 16) + 1 for t in toks), len(toks))
+        assert (runner.native is None) == python_walk
+        for i, t in enumerate(toks):
+            runner.admit(i)
+            runner.step([Entry(i, t[:77] if i == 0 else t[:-1], [])])
+        if not python_walk:
+            runner.native.timing(True)
+        got.append(runner.step([Entry(0, toks[0][77:], [portion - 1])] + [Entry(i, t[-1:], [0]) for i, t in enumerate(toks) if i]).cpu())
+        if not python_walk:
+            issued = [name for name, _ in runner.native.timing_report() if name.startswith("attention")]
+            runner.native.timing(False)
+            assert issued == launches * 2
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)

@@ -352,3 +352,13 @@ def test_slices_of_k_of_products_into_the_residual_of_more_than_1024_rows(M, N, 
     from allpaca_amd.kernels import lib
     L = lib.load("tuned")
     assert L.apc_gemm_direct_emit_k_split(M, N, K) == slices >= L.apc_gemm_direct_k_split(M, N, K)
+
+
+@pytest.mark.parametrize("tiles,heads,splits,d,pairs,last,one", [
+    (4, 32, 1, 128, 64, 1, 1), (8, 32, 1, 128, 128, 1, 1), (8, 32, 1, 128, 128, 0, 1),           # a round of decode blocks at most
+    (4, 32, 1, 128, 512, 0, 1), (12, 32, 1, 128, 1024, 0, 1), (4, 32, 1, 64, 1024, 0, 1),        # more, where the tiles leave units free
+    (8, 32, 1, 128, 512, 0, 0), (4, 32, 2, 128, 256, 0, 0), (8, 32, 2, 64, 256, 0, 0),           # tiles that fill whole rounds
+    (15, 32, 1, 128, 512, 0, 1), (4, 32, 1, 128, 2048, 0, 0), (1, 32, 1, 128, 2048, 0, 0), (4, 32, 1, 64, 2048, 0, 0)])
+def test_decoded_rows_in_the_launch_of_the_prompt_rows_where_that_is_faster(tiles, heads, splits, d, pairs, last, one):
+    from allpaca_amd.kernels import host
+    assert host.load().apc_host_rule_decode_beside_tiles(tiles * heads * splits, d, pairs, last) == one
