@@ -88,9 +88,11 @@ __device__ __forceinline__ void lines_to_operands(Frag& a, Frag& b) {
 // ones, and 24 moves between the lanes of a row of 16 a 16 keys of a head of 128 make operands of two such loads; the page
 // of a group of 8 keys is one value for the wave, so places are scalar work and no look-up goes through LDS.  What bounds
 // the kernel beside its bytes is the chain to the first keys and what a unit's loads cost (half lines leave the L2 at a third of
-// the rate).  One layer, 32 heads over 8, without / with, us: heads of 128, 1 row x 387 keys 11.6 / 11.0, 8 x 2,048 19.4 / 18.4,
-// 64 x 100 13.5 / 10.3, 64 x 1,024 49.8 / 45.9, 64 rows of 90 to 2,100 (DEC_EVEN) 40.3 / 37.6; heads of 64, 1 x 387 8.8 / 8.2,
-// 8 x 2,048 12.7 / 12.3, 64 x 2,048 47.3 / 45.6; of 60 measured sizes none is slower.  The same bits.
+// the rate).  One layer, 32 heads over 8, without / with, us: heads of 128, 1 row x 387 keys 10.8 / 10.1, 8 x 2,048 18.0 / 17.1,
+// 64 x 100 12.5 / 9.5, 64 x 1,000 50.2 / 46.0, 64 rows of 90 to 2,100 (DEC_EVEN) 39.3 / 36.1; heads of 64, 1 x 387 8.0 / 7.4, 8 x 2,048
+// 11.8 / 11.3, 64 x 2,048 47.9 / 46.7.  Of 1,791 sizes (1 to 256 rows of 1 to 8,192 keys, six pairs of heads), 0.94 in the mean, rows of up
+// to 31 keys are 0.1 us slower, and 384 to 768 (row, kv head) pairs of heads of 64 with up to 64 keys 0.2 of 5 us: three and four blocks
+// fit on a unit instead of three, and are not spread as evenly.  The same bits.
 constexpr int NW = 4;  // waves of a block of the decode kernel
 constexpr int LAST_DIRECT = 8;  // up to so many blocks a pair the last one reads the others' results in one go
 enum { DEC_PARTS = 0, DEC_WHOLE = 1, DEC_LAST = 2, DEC_EVEN = 3 };
@@ -340,8 +342,8 @@ __device__ __forceinline__ void attn_decode_block(
   };
 
   auto run_range = [&](int k_lo, int k_hi) {
-    page0 = k_lo / P;
-    my_page = bt[min(page0 + lane, pos / P)];
+    page0 = LINES ? k_lo >> lgP : k_lo / P;
+    my_page = bt[min(page0 + lane, LINES ? pos >> lgP : pos / P)];
     const int nsteps = (k_hi - k_lo + 31) / 32;
     KVRegs<DP> ra, rb;
     load_kv(ra, k_lo);
