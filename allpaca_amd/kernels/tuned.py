@@ -462,11 +462,13 @@ def _even_pays(steps: int, longest: int, n_rows: int, tiles: int, window: int) -
     of either in units of a wave's step of 32 keys.  Shares: a wave's share, a few units for the pieces' way through memory,
     and a look at all rows.  A block a pair: the same work, or the longest row's chain over four waves, slowed by the blocks
     that share its compute unit.  Fitted to 774 launches (1 to 32 kv heads of 64 to 256, 8 to 512 rows of equal, spread and
-    single long lengths), where the choice is on average 0.5 % over the better of the two; shares alone are 2.1 %, a block a
-    pair alone 50 %.  Microseconds a layer, block a pair / shares, 8 kv heads of 128: 32 rows of 1,100 keys 26.1 / 31.8, of
-    2,048 44.2 / 50.2, of 1,000 to 2,048 39.9 / 40.1, of 90 to 2,100 33.2 / 25.6; 64 rows of 1,100 49.1 / 53.8, of 2,048
-    85.7 / 87.5, of 1,000 to 2,048 75.1 / 71.4, of 90 to 2,100 63.5 / 37.9, one of 8,000 beside 63 of 100 120 / 30; 128 rows of
-    2,048 169 / 166.  32 kv heads of 128: 8 rows of 2,048 43.2 / 47.9, of 90 to 2,100 24.7 / 25.6, 16 rows of those 57 / 30."""
+    single long lengths) of the kernels before keys came in whole lines, when the choice was on average 0.5 % over the better
+    of the two.  Since then both are faster, a block a pair by more where two share a unit: of 684 launches (1 to 16 kv heads and
+    32) the choice is 0.9 % over the better one in the mean and 18 % at worst (512 rows of 500 to 1,500 keys on one kv head 49 / 58
+    us); shares alone are 2.9 %, a block a pair alone 37 %.  Microseconds a layer, block a pair / shares, 8 kv heads of 128: 32 rows
+    of 1,100 keys 27.1 / 32.5, of 2,048 46.1 / 52.6, of 1,000 to 2,048 37.3 / 40.2, of 90 to 2,100 28.5 / 23.5; 64 rows of 1,100 50.5 /
+    56.2, of 2,048 90.0 / 94.0, of 1,000 to 2,048 74.8 / 74.2, of 90 to 2,100 53.7 / 36.6, one of 8,000 beside 63 of 100 168 / 27; 128
+    rows of 2,048 169.7 / 169.0.  32 kv heads of 128: 8 rows of 2,048 45.5 / 51.4, of 90 to 2,100 23.0 / 22.9, 16 rows of those 46 / 31."""
     if window:
         most = window // 32 + 1
         longest, steps = min(longest, most), min(steps, n_rows * most)
