@@ -1187,3 +1187,24 @@ def test_attention_decode_many_launches_leave_the_counters_at_zero():
     for dev_counters in t._counters.values():
         for c in dev_counters:
             assert int(c.abs().max()) == 0
+
+
+@pytest.mark.parametrize("M,N,K", [(1025, 2048, 2048), (1153, 3072, 3072), (1300, 1024, 2304), (1500, 4096, 14336)])
+def test_slices_of_k_into_the_residual_are_no_further_from_64_bits_than_k_in_one_piece(M, N, K):
+    """Two sums of K / 2 products added in float32 against one of K (measured: 0.69 to 0.70 of its error), and the row's sum of squares, its
+    parts added in float32 as the next product does, against that of the same row in parts of 192 (0.6 to 0.87)."""
+    from allpaca_amd.kernels import lib
+    t, L = tuned(), lib.load("tuned")
+    assert (L.apc_gemm_direct_emit_k_split(M, N, K), L.apc_gemm_direct_k_split(M, N, K)) == (2, 1)
+    a, w = gen(M, K, seed=1, dtype=BF).to(DEV), gen(N, K, seed=2, dtype=BF, scale=0.02).to(DEV)
+    res, g = gen(M, N, seed=3).to(DEV), (1 + 0.2 * gen(N, seed=4)).to(DEV)
+    want = res.double() + a.double() @ w.double().T
+    packed, whole = pack(w), res.clone()
+    t.gemm_bf16(a, packed, whole, accumulate=True)
+    _, ss = t.gemm_emit_bf16(a, packed, res, g)
+    assert (res.double() - want).norm() <= (whole.double() - want).norm()
+    total = torch.zeros(M, device=DEV)
+    for part in ss.T:
+        total = total + part
+    squares = want.square().sum(1)
+    assert ((total.double() - squares) / squares).norm() / M ** 0.5 <= 7e-8     # (6e-8 with parts of 192: half a unit in the last place)
