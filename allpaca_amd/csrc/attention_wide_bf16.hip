@@ -288,25 +288,34 @@ __device__ __forceinline__ void soft_any(int h, floatx16& s, Frag (&pf)[2], Soft
 // (504 rows x 32 heads of 128: 128 blocks on 256 compute units), so one goes beside the other: these rows over 2,048 keys, 8 decoded
 // ones of 700 to 2,047 beside them, 39.2 + 15.0 -> 39.9 us a layer.
 constexpr int NO_DECODE = -1;
+// Arguments of their own: without decoded rows the kernel takes none of them, and its instances hold the same instructions as a kernel that
+// knows nothing of such rows (taken by all, 64-wide heads with a window were 0.2-0.3 us slower: 21 of 130 sizes by 1.0-1.8 %, now 11).
+struct WithDecode {
+  int wide_blocks, page_tokens;
+  AttnDecodeRows rows;
+};
+struct WithoutDecode {};
+template <int DEC>
+using Beside = std::conditional_t<DEC == NO_DECODE, WithoutDecode, WithDecode>;
 template <int HD, bool WIN, int DEC>
 __global__ __launch_bounds__(256, HD == 64 ? 2 : 1) void attn_prefill_wide_kernel(
     const bf16_t* __restrict__ q, int ldq, int q_off, bf16_t* __restrict__ out, int ldo, int H, int Hk,
     const bf16_t* __restrict__ cache, int lgP, const int* __restrict__ block_table, int max_blocks,
     const int* __restrict__ positions, const int* __restrict__ row_seg, const int* __restrict__ tile_row0,
     const int* __restrict__ tile_rows, int n_tiles, int window_arg, float scale, int n_splits, int part_rows,
-    float* __restrict__ parts,
-    int wide_blocks, int page_tokens, AttnDecodeRows dec) {
+    float* __restrict__ parts, Beside<DEC> beside) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   if constexpr (DEC != NO_DECODE) {
-    if ((int)blockIdx.x >= wide_blocks) {
+    if ((int)blockIdx.x >= beside.wide_blocks) {
+      const AttnDecodeRows dec = beside.rows;
       constexpr int MEET = attn_decode::DEC_P_ELEMS * 2 + 16;   // (is_last lies behind P)
       static_assert(MEET % 16 == 0 && MEET + attn_decode::NW * 16 * (HD + 2) * 4 <= lds_request(HD), "what a block's waves meet in");
-      const int pairs = Hk * ceil_div(H / Hk, 16), id = (int)blockIdx.x - wide_blocks;
+      const int pairs = Hk * ceil_div(H / Hk, 16), id = (int)blockIdx.x - beside.wide_blocks;
       const attn_decode::DecodeAt blk{id % dec.n, id / dec.n % pairs, id / dec.n / pairs, dec.n, pairs,
                                       DEC == attn_decode::DEC_WHOLE ? 1 : ceil_div(dec.n_parts, attn_decode::NW)};
       attn_decode::attn_decode_block<HD, DEC, true>(
           blk, reinterpret_cast<bf16_t*>(smem), reinterpret_cast<float*>(smem + MEET),
-          reinterpret_cast<int*>(smem + attn_decode::DEC_P_ELEMS * 2), q, ldq, q_off, H, Hk, HD, cache, page_tokens, block_table,
+          reinterpret_cast<int*>(smem + attn_decode::DEC_P_ELEMS * 2), q, ldq, q_off, H, Hk, HD, cache, beside.page_tokens, block_table,
           max_blocks, positions, row_seg, dec.rows, WIN ? window_arg : 0, scale, 0, dec.n_parts, dec.workspace, out, ldo, dec.counters);
       return;
     }
@@ -1053,7 +1062,7 @@ int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, i
     const long all = blocks + (long)dec->n * Hk * ceil_div(H / Hk, 16) * (last ? ceil_div(dec->n_parts, attn_decode::NW) : 1);
     if (all > 0x7fffffffL) return APC_ERR_BAD_ARG;
     const auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3((unsigned)all), dim3(256), lds, stream, WIDE_ARGS, (int)blocks, page_tokens, *dec);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)all), dim3(256), lds, stream, WIDE_ARGS, WithDecode{(int)blocks, page_tokens, *dec});
     };
 #define MIXED(HD_, WIN_)                                                                       \
   if (d == HD_ && (window > 0) == WIN_) {                                                      \
@@ -1066,7 +1075,7 @@ int launch_attn_prefill_wide(const bf16_t* q, int ldq, int q_off, bf16_t* out, i
 #define WIDE(HD_, WIN_)                                                                                                   \
   if (d == HD_ && (window > 0) == WIN_)                                                                                   \
     hipLaunchKernelGGL((attn_prefill_wide_kernel<HD_, WIN_, NO_DECODE>), dim3((unsigned)blocks), dim3(256), lds, stream, WIDE_ARGS, \
-                       (int)blocks, page_tokens, AttnDecodeRows{});
+                       WithoutDecode{});
     WIDE_INSTANCES(WIDE)
 #undef WIDE
   }
